@@ -4,7 +4,7 @@
 //   s = softmax(z) over the experts and the identity experts behind them, or sigmoid(z)
 //   c = s + correction                   (decides, does not weigh)
 //   groups of neighbours are ranked by their largest c, only the best `keep` of them take part
-//   the `top` largest c are chosen; weight = s * scale, of an expert's output, or of its input: then the product's rows are
+//   the `top` largest c are chosen; weight = s * scale (divided by the chosen ones' sum, if asked), of an expert's output, or of its input: then the product's rows are
 //   multiplied with it in front of the activation
 //
 // Steps of few tokens run the experts straight from the choices (experts_skinny_kernel: every chosen expert's weights
@@ -104,7 +104,8 @@ template <int Q>
 __global__ __launch_bounds__(256) void router_select_kernel(const float* __restrict__ z, int64_t ldz, int sigmoid,
                                                             const float* __restrict__ correction,
                                                             int* __restrict__ expert, float* __restrict__ weight, int T,
-                                                            int N, int groups, int keep, int top, float scale) {
+                                                            int N, int groups, int keep, int top, int normalize,
+                                                            float scale) {
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (t >= T) return;
   float s[Q], c[Q];
@@ -185,6 +186,12 @@ __global__ __launch_bounds__(256) void router_select_kernel(const float* __restr
         if (before[q] >= keep) c[q] = -INFINITY;
     }
     ranks(rank);
+    if (normalize) {
+      float mine = 0.f;
+#pragma unroll
+      for (int q = 0; q < Q; ++q) mine += lane + 64 * q < N && rank[q] < top ? s[q] : 0.f;
+      scale /= wave_sum(mine);
+    }
 #pragma unroll
     for (int q = 0; q < Q; ++q)
       if (lane + 64 * q < N && rank[q] < top) {
@@ -220,6 +227,10 @@ __global__ __launch_bounds__(256) void router_select_kernel(const float* __restr
       if (g >= groups || !((kept >> g) & 1)) c[q] = -INFINITY;
     }
   }
+  int rank[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) rank[q] = top;
+  float mine = 0.f;
   for (int j = 0; j < top; ++j) {
     float v = -INFINITY;
     int e = lane;
@@ -230,18 +241,21 @@ __global__ __launch_bounds__(256) void router_select_kernel(const float* __restr
         e = lane + 64 * q;
       }
     wave_argmax(v, e);
-    float w = 0.f;
 #pragma unroll
     for (int q = 0; q < Q; ++q)
       if (e == lane + 64 * q) {
         c[q] = -INFINITY;
-        w = s[q] * scale;
+        rank[q] = j;
+        mine += s[q];
       }
-    if (lane == (e & 63)) {
-      expert[(int64_t)t * top + j] = e;
-      weight[(int64_t)t * top + j] = w;
-    }
   }
+  if (normalize) scale /= wave_sum(mine);
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (rank[q] < top) {
+      expert[(int64_t)t * top + rank[q]] = lane + 64 * q;
+      weight[(int64_t)t * top + rank[q]] = s[q] * scale;
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -542,16 +556,17 @@ HDS_EXPORT int hds_router_logits(const void* x, int64_t ldx, const void* w, floa
 }
 
 // N = experts + identities <= 1024, in `groups` <= 64 equal groups of which `keep` take part; sigmoid: scores are sigmoid(z),
-// not softmax(z); correction may be null
+// not softmax(z); correction may be null; normalize: a token's chosen scores are divided by their sum
 HDS_EXPORT int hds_router_select(const float* z, int64_t ldz, int sigmoid, const float* correction, int* expert, float* weight,
-                                 int T, int N, int groups, int keep, int top, float scale, hipStream_t st) {
+                                 int T, int N, int groups, int keep, int top, int normalize, float scale,
+                                 hipStream_t st) {
   if (T <= 0) return 0;
   if (N < 1 || N > 1024 || ldz < N || groups < 1 || groups > 64 || N % groups || keep < 1 || keep > groups || top < 1 ||
       top > keep * (N / groups))
     return hipErrorInvalidValue;
 #define HDS_RS(Q)                                                                                                   \
   hipLaunchKernelGGL(router_select_kernel<Q>, dim3((T + 3) / 4), dim3(256), 0, st, z, ldz, sigmoid, correction, expert, \
-                     weight, T, N, groups, keep, top, scale)
+                     weight, T, N, groups, keep, top, normalize, scale)
   if (N <= 64) HDS_RS(1); else if (N <= 128) HDS_RS(2); else if (N <= 256) HDS_RS(4); else if (N <= 512) HDS_RS(8);
   else HDS_RS(16);
 #undef HDS_RS

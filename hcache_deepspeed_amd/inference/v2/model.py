@@ -51,6 +51,7 @@ class _Layer:
 
     def __init__(self):
         self.w = {}
+        self.routed = None  # an expert layer's weights as the routed expert kernels read them
 
     def __getitem__(self, k):
         return self.w.get(k)
@@ -135,6 +136,9 @@ class RaggedTransformer:
                          ("down.w", self.down_lin)):
             if w.get(key) is not None:
                 w[key] = mod.transform_param(w[key])
+        if w.get("w13") is not None:
+            shared = None if w.get("shared.w13") is None else (w["shared.w13"], w["shared.w2"], w["shared_gate.w"])
+            L.routed = self.moe_mod.lay_out(w["router.w"], w["w13"], w["w2"], shared)
 
     # ------------------------------------------------------------------------------------------
     # weights: canonical dict (arch.convert_*) -> this rank's shards
@@ -280,7 +284,9 @@ class RaggedTransformer:
         return self.down_lin(self.up_lin(x, L["up.w"], L["up.b"]), L["down.w"], L["down.b"])
 
     def _moe(self, L, x):
-        out = self.moe_mod(x, L["router.w"], L["w13"], L["w2"])
+        out = self.moe_mod(x, L["router.w"], L["w13"], L["w2"], L.routed)
+        if L.routed is not None:
+            return out
         if L["shared.w13"] is not None:
             s = F.linear(glu(F.linear(x, L["shared.w13"]), self._act_name()), L["shared.w2"])
             gate = torch.sigmoid(F.linear(x.float(), L["shared_gate.w"].float())).to(s.dtype)
@@ -331,11 +337,14 @@ class RaggedTransformer:
 
     # ------------------------------------------------------------------------------------------
     def decode_graph_eligible(self, batch, capture_latents):
-        """A decode-only ragged batch (one new token per sequence) of a dense model without tensor parallelism:
-        its whole forward depends on the batch size alone, so it replays from a HIP graph captured per size. With
+        """A decode-only ragged batch (one new token per sequence) of a dense model, or of one whose experts run on the
+        routed expert kernels, without tensor parallelism: its whole forward depends on the batch size alone, so it
+        replays from a HIP graph captured per size (Qwen2-MoE layout of width 2048, 4 layers, 4 sequences: 2,930 us a step
+        with torch routing and without a graph, 520 us with both). With
         ``capture_latents`` the graph also stores every layer's latent into a device ring (``_LatentRing``)."""
         if (self.device.type != "cuda" or (capture_latents and not self.decode_graph_latents) or self.tp != 1
-                or self.spec.moe is not None or self.decode_graph_max_batch <= 0):
+                or self.decode_graph_max_batch <= 0
+                or (self.spec.moe is not None and any(L["w13"] is not None and L.routed is None for L in self.layers))):
             return False
         S = batch.current_sequences
         return (batch.logits_of_last_tokens and 0 < S <= self.decode_graph_max_batch and batch.current_tokens == S

@@ -15,7 +15,7 @@ import torch.nn.functional as F
 from .... import comm as dist
 from ....ops.activations import bias_act, glu, glu_rows
 from ....ops.delta_rule import DeltaShape, delta_rule, make_delta_plan, step_ok
-from ....ops.experts import PAD, routed_experts
+from ....ops.experts import PAD, RouterShape, routed_experts
 from ....ops.gated_scan import gated_scan, recur_step, recur_step_ok
 from ....ops.gemv import glu_gemv
 from ....ops.grouped_gemm import moe_ffn_dropless
@@ -174,7 +174,9 @@ class QuantizedIntLinear(DSLinearBase):
 # ---------------------------------------------------------------------------------------------------------------
 @DSMoERegistry.register_module
 class GroupedGemmMoE(DSMoEBase):
-    """Top-k MoE without token dropping. GPU bf16: sync-free routing + two HIP grouped GEMMs over the
+    """Top-k MoE without token dropping. GPU bf16 with a SiLU gate: the routed expert kernels (ops/experts.py: router,
+    choice, experts straight from the choices up to 64 tokens and sorted by expert beyond, gated sum with the shared
+    expert), 7 to 9 launches a layer without the host. Other activations: torch routing and two grouped GEMMs over the
     expert-contiguous rows; elsewhere: capacity slots + batched expert GEMMs."""
 
     @staticmethod
@@ -185,10 +187,31 @@ class GroupedGemmMoE(DSMoEBase):
     def supports_config(c):
         return c.activation.endswith("_glu") and 1 <= c.top_k <= c.n_experts
 
-    def forward(self, x, router_w, w13, w2):
+    def lay_out(self, router_w, w13, w2, shared=None):
+        """The layer's weights for the routed expert kernels, or None where those do not apply. ``shared``: (gate and up
+        rows, down, gate row) of the shared expert; its gate is scored with the experts."""
+        c = self._config
+        E, H, I = w2.shape
+        ws13, ws2, gate = shared if shared is not None else (None, None, None)
+        mats = [t for t in (router_w, w13, w2, ws13, ws2, gate) if t is not None]
+        if not (c.activation == "silu_glu" and E <= 1024 and H % PAD == 0 and I % PAD == 0 and w13.is_cuda
+                and all(t.dtype == torch.bfloat16 and t.is_contiguous() for t in mats)
+                and (ws2 is None or ws2.shape[1] % PAD == 0)):
+            return None
+        return {"router.w": router_w if gate is None else torch.cat([router_w, gate]), "router.c": None, "w13": w13,
+                "w2": w2, "ws13": ws13, "ws2": ws2}
+
+    def forward(self, x, router_w, w13, w2, laid=None):
+        """``laid``: the weights from ``lay_out``, the shared expert among them; its part is then in the result."""
         c = self._config
         act = c.activation[:-4]
         T, H = x.shape
+        grad = torch.is_grad_enabled() and any(t.requires_grad for t in (x, router_w, w13, w2))
+        if laid is None and x.dtype == torch.bfloat16 and not grad:
+            laid = self.lay_out(router_w, w13, w2)
+        if laid is not None and T:
+            shape = RouterShape(w2.shape[0], top=c.top_k, normalize=bool(c.normalize_scores) and c.top_k > 1)
+            return sum_experts(x, routed_experts(x, laid, shape), x.dtype)
         logits = F.linear(x.float(), router_w.float())
         if x.is_cuda and x.dtype == torch.bfloat16 and H % 128 == 0 and w2.shape[2] % 128 == 0:
             expert, pos, w, counts = topk_assign(logits, c.top_k, normalize=c.normalize_scores)

@@ -30,6 +30,7 @@ class RouterShape:
     scale: float = 1.0
     score: str = "softmax"     # or "sigmoid"
     weigh_input: bool = False  # the weights multiply what the experts read instead of what they return
+    normalize: bool = False    # a token's weights are divided by their sum
 
     @property
     def outputs(self):
@@ -80,7 +81,7 @@ def route(z, correction, shape):
         native.check(
             native.kernels().hds_router_select(z.data_ptr(), z.stride(0), int(shape.score == "sigmoid"),
                                                native.ptr(correction), expert.data_ptr(), weight.data_ptr(), T, n, shape.groups, shape.keep, shape.top,
-                                               float(shape.scale), native.stream()), "router_select")
+                                               int(shape.normalize), float(shape.scale), native.stream()), "router_select")
         return expert, weight
     s = torch.sigmoid(z[:, :n]) if shape.score == "sigmoid" else torch.softmax(z[:, :n], -1)
     c = s if correction is None else s + correction
@@ -90,7 +91,10 @@ def route(z, correction, shape):
         drop = torch.ones(T, shape.groups, dtype=torch.bool).scatter_(1, best, False)
         c = by_group.masked_fill(drop[..., None], float("-inf")).view(T, n)
     expert = c.topk(shape.top, -1).indices
-    return expert.to(torch.int32), s.gather(1, expert) * shape.scale
+    weight = s.gather(1, expert)
+    if shape.normalize:
+        weight = weight / weight.sum(-1, keepdim=True)
+    return expert.to(torch.int32), weight * shape.scale
 
 
 def _shared_product(x, w):

@@ -43,7 +43,7 @@ _KERNEL_SIGS = {
     "hds_experts_norm": "i" + "ppp" + "l" + "pp" + "pl" + "ppp" + "pl" + "pl" + "iiiii" + "f" + "s",
     "hds_embed_rows": "i" + "pp" + "f" + "pp" + "l" + "iii" + "s",
     "hds_router_logits": "pl" + "p" + "pl" + "iii" + "s",
-    "hds_router_select": "pl" + "i" + "ppp" + "iiiii" + "f" + "s",
+    "hds_router_select": "pl" + "i" + "ppp" + "iiiiii" + "f" + "s",
     "hds_expert_sort": "p" + "iii" + "ppppp" + "i" + "ppp" + "i" + "s",
     "hds_experts_skinny_max": "",
     "hds_experts_skinny": "i" + "pl" + "p" + "pl" + "p" + "iiiii" + "pl" + "p" + "pl" + "iii" + "i" + "f" + "p" + "s",

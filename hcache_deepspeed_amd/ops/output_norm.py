@@ -75,7 +75,8 @@ def residual_norm(x, delta, gain, eps, dtype, pad=1):
 
 
 def sum_experts(x, parts, dtype):
-    """The sum of an ExpertSum as a [T, W] matrix of ``dtype`` (x: the residual, which identity choices return)."""
+    """The sum of an ExpertSum as a [T, W] matrix of ``dtype`` (x: the residual, which identity choices return; only its
+    shape counts without any)."""
     out = torch.empty(x.shape, dtype=dtype, device=x.device)
     if native.use_native(x):
         _experts_norm(x, None, 0, None, out, parts, 0.0)

@@ -129,3 +129,62 @@ def test_quantized_engine_gpu(mode, tol):
     want = full[[39, 40, 41, 42]]
     err = (torch.stack(outs) - want).norm() / want.norm()
     assert err < tol, float(err)
+
+
+def _moe_reference(x, rw, w13, w2, top, normalize, shared=None):
+    """In float64; the choices and weights too."""
+    x, rw, w13, w2 = (t.double() for t in (x, rw, w13, w2))
+    p = torch.softmax(x @ rw.t(), -1)
+    weight, chosen = p.topk(top, -1)
+    if normalize:
+        weight = weight / weight.sum(-1, keepdim=True)
+    out = torch.zeros_like(x)
+    for e in range(rw.shape[0]):
+        t, j = (chosen == e).nonzero(as_tuple=True)
+        g, u = (x[t] @ w13[e].t()).chunk(2, -1)
+        out.index_add_(0, t, weight[t, j, None] * ((torch.nn.functional.silu(g) * u) @ w2[e].t()))
+    if shared is not None:
+        s13, s2, gate = (t.double() for t in shared)
+        g, u = (x @ s13.t()).chunk(2, -1)
+        out += torch.sigmoid(x @ gate.t()) * ((torch.nn.functional.silu(g) * u) @ s2.t())
+    return out, weight, chosen
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,top,normalize,has_shared", [
+    (1, 8, 2, True, False), (16, 64, 6, False, True), (64, 8, 2, True, True), (64, 200, 33, True, False),
+    (65, 8, 1, True, False), (300, 64, 4, False, True), (700, 130, 3, True, False)])
+def test_routed_moe_module_gpu(T, E, top, normalize, has_shared):
+    """Both sides of the line between the products straight from the choices (64 tokens, 2,048 choices) and the sorted
+    ones; one, two and four router entries a lane. Inputs are integers / 4, so that router logits are exact and
+    no choice depends on rounding; what is left is bf16: the hidden rows, the experts' outputs and the result, each 2^-9."""
+    H, I, S = 256, 128, 384
+    g = torch.Generator().manual_seed(T)
+    dev = torch.device("cuda")
+    x = (torch.randint(-8, 9, (T, H), generator=g) / 4).bfloat16().to(dev)
+    rw = (torch.randint(-8, 9, (E, H), generator=g) / 64).bfloat16().to(dev)
+    mat = lambda *s: (torch.randn(*s, generator=g) * s[-1]**-0.5).bfloat16().to(dev)  # noqa: E731
+    w13, w2 = mat(E, 2 * I, H), mat(E, H, I)
+    shared = (mat(2 * S, H), mat(H, S), mat(1, H)) if has_shared else None
+    moe = instantiate_moe(DSMoEConfig(H, I, E, top, "silu_glu", normalize))
+    laid = moe.lay_out(rw, w13, w2, shared)
+    assert laid is not None
+    y = moe(x, rw, w13, w2, laid)
+    want, weight, _ = _moe_reference(x, rw, w13, w2, top, normalize and top > 1, shared)
+    assert (y.double() - want).norm() / want.norm() < 3 * 2**-8
+    if not has_shared:
+        assert torch.equal(y, moe(x, rw, w13, w2))  # laid out on the way
+    from hcache_deepspeed_amd.ops.experts import RouterShape, route
+    z = x.float() @ rw.float().t()
+    expert, got = route(z, None, RouterShape(E, top=top, normalize=normalize and top > 1))
+    # 32-bit exponentials and one division
+    assert torch.allclose(got.double(), weight, rtol=1e-5, atol=1e-9)
+    assert torch.equal(z.gather(1, expert.long()), z.topk(top, -1).values)
+
+
+def test_route_normalizes():
+    from hcache_deepspeed_amd.ops.experts import RouterShape, route
+    z = torch.randn(5, 12, generator=torch.Generator().manual_seed(0))
+    _, w = route(z, None, RouterShape(12, top=3, normalize=True, scale=2.0))
+    p = torch.softmax(z, -1).topk(3, -1).values
+    assert torch.allclose(w, 2.0 * p / p.sum(-1, keepdim=True))
