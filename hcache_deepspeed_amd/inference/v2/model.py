@@ -355,7 +355,7 @@ class RaggedTransformer:
         """Replay the decode step for ``batch.current_sequences`` sequences: the step's token ids and packed
         metadata (same layout as ``RaggedBatchWrapper.finalize``) are copied into the graph's static buffers, the
         graph replays every layer's kernels with one launch, and the logits are copied out. The first step of a
-        batch size runs the forward eagerly once (it writes the same KV the replay writes) and captures it.
+        batch size runs the forward eagerly over the same buffers, for a size may come once; the second captures it.
 
         ``capture_latents``: the graph also stores each layer's latent rows into a device ring slot (HCache during
         decode, reference llama_v2/model.py:211-218 captures in every forward); returns ``(logits, latents)`` with
@@ -372,12 +372,17 @@ class RaggedTransformer:
         g.ids.copy_(batch.input_ids, non_blocking=True)
         g.meta.copy_(batch._dev_meta[:n], non_blocking=True)
         view = g.ring.begin_step() if g.ring is not None else None
-        if g.graph is None:
-            g.capture(self)
-        g.graph.replay()
+        if not g.seen:
+            g.seen = True
+            out = g.forward(self)
+        else:
+            if g.graph is None:
+                g.capture(self)
+            g.graph.replay()
+            out = g.out.clone()
         if g.ring is not None:
             g.ring.end_step()
-        return g.out.clone(), view
+        return out, view
 
     def latent_rings(self):
         return [g.ring for g in self._decode_graphs.values() if g.ring is not None]
@@ -710,6 +715,11 @@ class _LatentRing:
         return any(self.filled[h] > self.drained[h] for h in (0, 1))
 
 
+# Free device memory below which a capture first takes back what the caching allocator holds: a decode step's activations
+# are tens of MB
+_CAPTURE_ROOM = 2 << 30
+
+
 class _DecodeGraph:
     """Static inputs, captured graph and output of one decode batch size (RaggedTransformer.forward_decode_graph),
     with its latent ring when the graph captures HCache latents."""
@@ -749,37 +759,52 @@ class _DecodeGraph:
         sb.seq_meta_host = None
         sb.tables_host = None
         self.batch = sb
+        self.seen = False
         self.graph = None
         self.out = None
+
+    def forward(self, model):
+        """The step over the static inputs, launch by launch; its latents go to the ring's slot, which moves on."""
+        cap = self.ring is not None
+        out, _ = model.forward(self.batch, capture_latents=cap, sink=self.ring.sink if cap else None)
+        if cap:
+            self.ring.advance()
+        return out
 
     def capture(self, model):
         cur = torch.cuda.current_stream()
         side = torch.cuda.Stream()
         side.wait_stream(cur)
         cap = self.ring is not None
-        sink = self.ring.sink if cap else None
         with torch.cuda.stream(side):
             # warm-up: hipBLASLt / GEMV handles, KV (idempotent; recurrent state is put back); its latents go to the
             # slot the replay rewrites
             snap = model.save_state(self.batch)
-            model.forward(self.batch, capture_latents=cap, sink=sink)
+            model.forward(self.batch, capture_latents=cap, sink=self.ring.sink if cap else None)
             model.load_state(self.batch, snap)
         cur.wait_stream(side)
         if model._graph_pool is None:
             model._graph_pool = torch.cuda.graph_pool_handle()
+        if torch.cuda.mem_get_info(model.device)[0] < _CAPTURE_ROOM:
+            torch.cuda.empty_cache()  # the caching allocator cannot give blocks back while a stream captures
+        torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph()
-        # no Python GC while capturing: a collection that frees another engine's CUDAGraph calls hipGraphDestroy, which
-        # is not permitted while a stream captures (the capture and the process abort)
+        # No Python GC while capturing: a collection that frees another engine's CUDAGraph calls hipGraphDestroy, which
+        # is not permitted while a stream captures (the capture and the process abort). Switching it off is enough: a
+        # collection ahead of it takes 23 ms of the first step of every batch size, torch.cuda.graph's own preparation
+        # (another collection of the allocator's blocks) 5 - 7 ms, the capture itself 1.5 ms (4 layers)
         import gc
         was_enabled = gc.isenabled()
-        gc.collect()
         gc.disable()
         try:
-            with torch.cuda.graph(g, pool=model._graph_pool):
-                self.out, _ = model.forward(self.batch, capture_latents=cap, sink=sink)
-                if cap:
-                    self.ring.advance()
+            with torch.cuda.stream(side):
+                g.capture_begin(pool=model._graph_pool)
+                try:
+                    self.out = self.forward(model)
+                finally:
+                    g.capture_end()
         finally:
             if was_enabled:
                 gc.enable()
+        cur.wait_stream(side)
         self.graph = g

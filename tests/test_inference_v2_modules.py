@@ -188,3 +188,40 @@ def test_route_normalizes():
     _, w = route(z, None, RouterShape(12, top=3, normalize=True, scale=2.0))
     p = torch.softmax(z, -1).topk(3, -1).values
     assert torch.allclose(w, 2.0 * p / p.sum(-1, keepdim=True))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shared,normalize", [(True, False), (False, True)])
+def test_moe_decode_graph_matches_eager_gpu(shared, normalize):
+    """A batch size's first step runs eagerly over the graph's buffers, the second captures, later ones replay: each gives
+    the logits of an engine without graphs, bit for bit (the same kernels)."""
+    from hcache_deepspeed_amd.inference.v2.arch import ArchSpec
+    from hcache_deepspeed_amd.inference.v2.engine import InferenceEngineV2, RaggedInferenceEngineConfig
+    H, E, I, S, V = 256, 8, 128, 384, 211
+    g = torch.Generator().manual_seed(0)
+    dev = torch.device("cuda")
+    mat = lambda *s: (torch.randn(*s, generator=g) * s[-1]**-0.5).bfloat16().to(dev)  # noqa: E731
+    one = torch.ones(H, dtype=torch.bfloat16, device=dev)
+    layers = []
+    for _ in range(2):
+        L = {"ln1.w": one, "ln2.w": one, "qkv.w": mat(4 * 128, H), "o.w": mat(H, 256), "router.w": mat(E, H),
+             "w13": mat(E, 2 * I, H), "w2": mat(E, H, I)}
+        if shared:
+            L.update({"shared.w13": mat(2 * S, H), "shared.w2": mat(H, S), "shared_gate.w": mat(1, H)})
+        layers.append(L)
+    w = {"embed": mat(V, H) * 16, "final.w": one, "lm_head.w": mat(V, H), "layers": layers}
+    spec = ArchSpec("qwen2_moe", V, H, 2, 2, 1, 128, I, max_position_embeddings=512,
+                    moe=dict(num_experts=E, top_k=2, normalize=normalize, shared=shared))
+    conf = RaggedInferenceEngineConfig.from_dict(dict(dtype="bf16", state_manager=dict(max_context=512)))
+    engs = {k: InferenceEngineV2(spec, w, conf, device=dev, num_kv_blocks=32) for k in ("graph", "eager")}
+    engs["eager"]._model.decode_graph_max_batch = 0
+    prompts = [torch.randint(0, V, (n, ), generator=g) for n in (40, 65, 7)]
+    for e in engs.values():
+        e.put([1, 2, 3], prompts, capture_latents=False)
+    for step in range(8):
+        uids = [1, 2, 3] if step % 2 else [1, 3]
+        toks = [torch.randint(0, V, (1, ), generator=g) for _ in uids]
+        out = {k: e.put(uids, toks, capture_latents=False)[0] for k, e in engs.items()}
+        assert torch.equal(out["graph"], out["eager"]), step
+    assert set(engs["graph"]._model._decode_graphs) == {(2, False), (3, False)}
+    assert all(x.graph is not None for x in engs["graph"]._model._decode_graphs.values())
