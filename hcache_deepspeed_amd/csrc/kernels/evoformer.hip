@@ -1,16 +1,23 @@
-// Evoformer attention forward with MSA-mask and pair biases (DS4Sci_EvoformerAttention), gfx950.
+// Evoformer attention with MSA-mask and pair biases (DS4Sci_EvoformerAttention), forward and backward, gfx950.
 //
-// Reference parity: csrc/deepspeed4science/evoformer_attn (CUTLASS memory-efficient attention with bias, SURVEY.md
-// §2.10 N16 / §2.11 K24). Not a translation: one wave64 owns 32 queries of one (b, n, h) and streams the keys in
-// 32-row tiles through v_mfma_f32_32x32x16_bf16 with the FlashAttention orientation of attn_common.h:
-//   S^T = K . Q^T puts the QUERY on the lane, so the online-softmax statistics are lane-local (one cross-half
-//   shuffle), and the S^T accumulator is directly the B operand of O^T = V^T . P^T (acc_to_b) — no LDS round trip.
-// Evoformer heads are small (D = 32 or 64, L ~ 256-1024), so the operands come straight from global memory /
-// L2 as 16-byte rows (Q, K) and coalesced per-key rows (V^T: lanes = 32 consecutive d of one key); the grid is
-// (B*N*H, query tiles), tens of thousands of waves for MSA row attention. Biases (same dtype as Q) are added in
-// fp32 before the softmax: bias1[b, n, key] (mask, broadcast over heads/queries), bias2[b, h, q, key] (pair bias,
-// broadcast over the N rows). The kernel also writes the natural-log LSE per query for the memory-efficient
-// backward (ops/deepspeed4science/evoformer_attn.py recomputes P from it chunk by chunk).
+// Reference parity: csrc/deepspeed4science/evoformer_attn (CUTLASS memory-efficient attention with bias). Not a
+// translation.
+//
+// q, k, v [B, N, L, H, D]; bias1 [B, N, 1, 1, L] (mask), bias2 [B, 1, H, L, L] (pair bias, shared by the N rows), both in
+// bf16 or both in fp32 and added in fp32. The sequences are short (16 to 400 positions), the heads small (32, 64), the
+// rows many: the products are a few GFLOP and the inputs a few tens of MB, so the kernels are bound by the vector
+// instructions between the products (exponential, bias, conversion: about 12 a score) and by how the operands get there.
+//   * forward and dQ: a wave holds 32 queries of one (b, n, h), the workgroup stages its keys and values in LDS once
+//     (LDS-DMA, 32 KB a chunk, so that several workgroups share a CU). S^T = K Q^T puts the query on the lane: softmax
+//     statistics are lane-local and the S^T accumulator is the B operand of the next product (acc_to_b); V^T and K^T
+//     come out of the row-major tiles by transposing LDS reads. dQ also makes rowsum(dO * O), which the others read.
+//   * dK / dV: the same with 32 keys on the lanes and queries and output gradients in LDS.
+//   * pair-bias gradient: the sum of dS over the N rows stays in registers. A wave owns 32 queries x 64 keys of one
+//     (b, h) and walks over a chunk of the rows, recomputing the two products that dS needs; chunks are added by a second
+//     kernel that also rounds. No atomics, the same result every time.
+// Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): forward 53 us, dQ 58, dK / dV 124, pair gradient 78 + 5
+// (before: one wave a workgroup with operands from global memory and 2-byte reads of V 169 us; the FlashAttention
+// backward kernels with 32-bit atomics into the pair gradient 271 + 1,585 us).
 #include "attn_common.h"
 
 using namespace hds;
@@ -18,131 +25,559 @@ using namespace hds::attn;
 
 namespace {
 
-template <typename T>
-__device__ __forceinline__ float ld(const T* p) { return to_f(*p); }
+constexpr float kLog2e = 1.4426950408889634f;
 
-template <int D, typename T>
-__global__ __launch_bounds__(64) void evo_fwd_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k,
-                                                     const bf16* __restrict__ v, const T* __restrict__ b1,
-                                                     const T* __restrict__ b2, bf16* __restrict__ o,
-                                                     float* __restrict__ lse, int N, int L, int H, float scale) {
-  const int lane = threadIdx.x;
-  const int hf = lane >> 5, j = lane & 31;
-  const int q0 = blockIdx.y * 32;
-  const int bnh = blockIdx.x;  // (b * N + n) * H + h
-  const int h = bnh % H, bn = bnh / H, b = bn / N;
-  const int64_t tok = (int64_t)H * D;  // stride between tokens
-  const bf16* qb = q + (int64_t)bn * L * tok + (int64_t)h * D;
-  const bf16* kb = k + (int64_t)bn * L * tok + (int64_t)h * D;
-  const bf16* vb = v + (int64_t)bn * L * tok + (int64_t)h * D;
-  const int myq = q0 + j;
-  const int qc = myq < L ? myq : L - 1;
-  constexpr float kLog2e = 1.4426950408889634f;
-  const float c = scale * kLog2e;
+// ---------------------------------------------------------------------------------------------------------------
+// LDS tiles: rows of 2 D bytes whose 16-byte chunks are XOR-swizzled by the row, so that 16 lanes reading 16 rows at one
+// chunk (ds_read_b128), and 16 lanes reading 32 bytes of 4 rows (ds_read_b64_tr_b16), meet every bank once
+// ---------------------------------------------------------------------------------------------------------------
+template <int D>
+struct Tile {
+  static constexpr int RB = 2 * D, CH = D / 8;       // bytes, chunks of a row
+  static constexpr int ROWS = 8192 / D;              // rows of a chunk: 16 KB a matrix
+  static constexpr int KS = D / 16, DT = D / 32;     // steps of a contraction over D, 32-column blocks
+  static __device__ __forceinline__ int mix(int row) {
+    if constexpr (D == 32) return (row >> 2) & 3;
+    if constexpr (D == 64) return ((row & 2)) | ((row & 4)) | ((row >> 3) & 1);
+    return swz(row);
+  }
+  static __device__ __forceinline__ int off(int row, int ch) { return row * RB + 16 * (ch ^ mix(row)); }
 
-  bf16x8 qf[D / 16];
+  // rows row0 .. row0 + 32 nt - 1 of a matrix [L, ld] to LDS (rows past the end: the last one)
+  static __device__ __forceinline__ void stage(char* lds, const bf16* m, int64_t ld, int row0, int nt, int L, int nw) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    constexpr int PER = 1024 / RB;  // rows of one wave instruction
+    for (int i = w; i < nt * 32 / PER; i += nw) {
+      const int row = i * PER + lane / CH;
+      const int ch = (lane % CH) ^ mix(row);
+      const bf16* src = m + (int64_t)min(row0 + row, L - 1) * ld + 8 * ch;
+      __builtin_amdgcn_global_load_lds((gbl_void*)src, (lds_void*)(lds + i * 1024), 16, 0, 0);
+    }
+  }
+  // rows row0 + (lane & 31), elements 16 ks + 8 (lane >> 5) .. + 7
+  static __device__ __forceinline__ bf16x8 rows(const char* lds, int row0, int ks) {
+    const int lane = threadIdx.x & 63;
+    return *reinterpret_cast<const bf16x8*>(lds + off(row0 + (lane & 31), 2 * ks + (lane >> 5)));
+  }
+  // the transposed tile: column 32 dt + (lane & 31), rows row0 + 16 s + .. in the order of acc_to_b
+  static __device__ __forceinline__ bf16x8 cols(const char* lds, int row0, int s, int dt) {
+    const int lane = threadIdx.x & 63;
+    const int g = lane >> 4, i = lane & 15, q = i >> 2, p = i & 3;
+    const int row = row0 + 16 * s + 4 * (g >> 1) + q;
+    const int ch = 4 * dt + 2 * (g & 1) + (p >> 1);
+    const char* a0 = lds + off(row, ch) + 8 * (p & 1);
+    const char* a1 = lds + off(row + 8, ch) + 8 * (p & 1);
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(a0));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(a1));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+};
+
+// ---------------------------------------------------------------------------------------------------------------
+// biases
+// ---------------------------------------------------------------------------------------------------------------
+template <typename TB>
+struct __attribute__((packed, aligned(sizeof(TB)))) Four {  // L may be odd: rows are aligned to their element only
+  TB v[4];
+};
+
+// b[r] += row[k0 + acc_row(r, hf)]; TAIL: places past the end are read at the end
+template <bool TAIL, typename TB>
+__device__ __forceinline__ void add_row(const TB* row, int k0, int hf, int L, float (&b)[16]) {
 #pragma unroll
-  for (int ks = 0; ks < D / 16; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(qb + qc * tok + 16 * ks + 8 * hf);
-
-  f32x16 acc[D / 32];
+  for (int g = 0; g < 4; ++g) {
+    const int k = k0 + 8 * g + 4 * hf;
+    if constexpr (TAIL) {
 #pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt) acc[dt] = f32x16{};
+      for (int t = 0; t < 4; ++t) b[4 * g + t] += to_f(row[min(k + t, L - 1)]);
+    } else {
+      const Four<TB> f = *reinterpret_cast<const Four<TB>*>(row + k);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) b[4 * g + t] += to_f(f.v[t]);
+    }
+  }
+}
+
+struct EvoParams {
+  const bf16 *q, *k, *v, *o, *dout;
+  const void *b1, *b2;  // [B N, L], [B, H, L, L], or null
+  bf16 *out, *dq, *dk, *dv;
+  float *lse, *delta;   // [B N, H, L]: natural log of the softmax normaliser; rowsum(dO * O)
+  float* db1;           // [B N, L] or null
+  float* part;          // [chunks, B, H, L, L]
+  int B, N, L, H;
+  float scale;
+};
+
+// Workgroups of one row n next to each other on one XCD: neighbouring heads share cache lines, q blocks share k and v
+__device__ __forceinline__ int xcd_id() {
+  const int n = gridDim.x, i = blockIdx.x, q = n / 8, r = n % 8, x = i % 8;
+  return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + i / 8;
+}
+
+struct Place {
+  int blk, h, bn, b;
+  int64_t ld, base;  // between tokens; of (b, n, 0, h, 0)
+};
+template <int D>
+__device__ __forceinline__ Place place(const EvoParams& p, int blocks) {
+  Place a;
+  int id = xcd_id();
+  a.blk = id % blocks;
+  id /= blocks;
+  a.h = id % p.H;
+  a.bn = id / p.H;
+  a.b = a.bn / p.N;
+  a.ld = (int64_t)p.H * D;
+  a.base = (int64_t)a.bn * p.L * a.ld + (int64_t)a.h * D;
+  return a;
+}
+
+// fragments of row `row` (each lane's own), 16 ks + 8 hf .. + 7
+template <int D>
+__device__ __forceinline__ void load_frags(const bf16* m, int64_t ld, int row, bf16x8 (&f)[D / 16]) {
+  const bf16* r = m + (int64_t)row * ld + 8 * ((threadIdx.x & 63) >> 5);
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks) f[ks] = *reinterpret_cast<const bf16x8*>(r + 16 * ks);
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// forward
+// ---------------------------------------------------------------------------------------------------------------
+template <int D, typename TB>
+__global__ __launch_bounds__(512) void evo_fwd_kernel(EvoParams p, int blocks) {
+  using T = Tile<D>;
+  __shared__ __attribute__((aligned(1024))) char smem[2 * 16384];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int hf = lane >> 5, j = lane & 31, L = p.L;
+  const Place a = place<D>(p, blocks);
+  const int q0 = 32 * (a.blk * nw + w), myq = q0 + j, qc = min(myq, L - 1);
+  const bool live = q0 < L;
+  const float c = p.scale * kLog2e;
+  bf16x8 qf[T::KS];
+  load_frags<D>(p.q + a.base, a.ld, qc, qf);
+  f32x16 acc[T::DT];
+#pragma unroll
+  for (int dt = 0; dt < T::DT; ++dt) acc[dt] = f32x16{};
   float m = -INFINITY, l = 0.f;
-  const T* b1r = b1 ? b1 + (int64_t)bn * L : nullptr;
-  const T* b2r = b2 ? b2 + ((int64_t)(b * H + h) * L + qc) * L : nullptr;
+  const TB* b1 = p.b1 != nullptr ? (const TB*)p.b1 + (int64_t)a.bn * L : nullptr;
+  const TB* b2 = p.b2 != nullptr ? (const TB*)p.b2 + ((int64_t)(a.b * p.H + a.h) * L + qc) * L : nullptr;
 
-  for (int k0 = 0; k0 < L; k0 += 32) {
-    // S^T tile: rows = keys k0 + acc_row(r, hf), column = this lane's query
-    const int kr = min(k0 + j, L - 1);
+  auto tile = [&](const char* sk, const char* sv, int t0, int k0, auto tail) {
+    constexpr bool TAIL = decltype(tail)::value;
+    float bias[16] = {};
+    if (b1 != nullptr) add_row<TAIL>(b1, k0, hf, L, bias);
+    if (b2 != nullptr) add_row<TAIL>(b2, k0, hf, L, bias);
     f32x16 s = f32x16{};
 #pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks)
-      s = mfma(*reinterpret_cast<const bf16x8*>(kb + kr * tok + 16 * ks + 8 * hf), qf[ks], s);
-    float tmax = -INFINITY;
+    for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(sk, t0, ks), qf[ks], s);
+    float top = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int key = k0 + acc_row(r, hf);
-      float x = s[r] * c;
-      if (key < L) {
-        if (b1r) x += ld(b1r + key) * kLog2e;
-        if (b2r) x += ld(b2r + key) * kLog2e;
-      } else {
-        x = -INFINITY;
-      }
-      s[r] = x;
-      tmax = fmaxf(tmax, x);
+      s[r] = s[r] * c + bias[r] * kLog2e;
+      if (TAIL && k0 + acc_row(r, hf) >= L) s[r] = -INFINITY;
+      top = fmaxf(top, s[r]);
     }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float mnew = fmaxf(m, tmax);
-    const float alpha = (m == -INFINITY) ? 0.f : fast_exp2(m - mnew);
-    m = mnew;
-    float rs = 0.f;
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    const float mn = fmaxf(m, top);
+    const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - mn);
+    m = mn;
+    float sum = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const float e = fast_exp2(s[r] - m);
-      s[r] = e;
-      rs += e;
+      s[r] = fast_exp2(s[r] - mn);
+      sum += s[r];
     }
-    rs += __shfl_xor(rs, 32, 64);
-    l = l * alpha + rs;
-#pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt) acc[dt] *= alpha;
+    l = l * alpha + sum;  // of this lane's keys; both halves are added at the end
     const bf16x8 pb[2] = {acc_to_b<0>(s), acc_to_b<1>(s)};
-    // A operand = V^T: lane row d = 32*dt + j, element e of half hf <-> key 16*st + 8*(e>>2) + 4*hf + (e&3)
 #pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
+    for (int dt = 0; dt < T::DT; ++dt) {
+      acc[dt] *= alpha;
 #pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        bf16x8 va;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int key = min(k0 + 16 * st + 8 * (e >> 2) + 4 * hf + (e & 3), L - 1);
-          va[e] = vb[key * tok + 32 * dt + j];
-        }
-        acc[dt] = mfma(va, pb[st], acc[dt]);
-      }
-  }
+      for (int st = 0; st < 2; ++st) acc[dt] = mfma(T::cols(sv, t0, st, dt), pb[st], acc[dt]);
+    }
+  };
 
+  for (int c0 = 0; c0 < L; c0 += T::ROWS) {
+    const int nt = (min(T::ROWS, L - c0) + 31) / 32;
+    if (c0 > 0) __syncthreads();
+    T::stage(smem, p.k + a.base, a.ld, c0, nt, L, nw);
+    T::stage(smem + 16384, p.v + a.base, a.ld, c0, nt, L, nw);
+    __syncthreads();
+    if (!live) continue;
+    for (int t = 0; t < nt; ++t) {
+      const int k0 = c0 + 32 * t;
+      if (k0 + 32 <= L) tile(smem, smem + 16384, 32 * t, k0, std::false_type{});
+      else tile(smem, smem + 16384, 32 * t, k0, std::true_type{});
+    }
+  }
+  if (!live) return;
+  l += __shfl_xor(l, 32, 64);
   if (myq < L) {
     const float inv = l > 0.f ? 1.f / l : 0.f;
-    bf16* orow = o + (int64_t)bn * L * tok + (int64_t)myq * tok + (int64_t)h * D;
+    bf16* row = p.out + a.base + (int64_t)myq * a.ld;
 #pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt)
+    for (int dt = 0; dt < T::DT; ++dt) store_row_block<D>(row, acc[dt], dt, hf, inv);
+    if (hf == 0) p.lse[((int64_t)a.bn * p.H + a.h) * L + myq] = (m + log2f(l)) / kLog2e;
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// dQ, and rowsum(dO * O)
+// ---------------------------------------------------------------------------------------------------------------
+template <int D, typename TB>
+__global__ __launch_bounds__(512) void evo_dq_kernel(EvoParams p, int blocks) {
+  using T = Tile<D>;
+  __shared__ __attribute__((aligned(1024))) char smem[2 * 16384];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int hf = lane >> 5, j = lane & 31, L = p.L;
+  const Place a = place<D>(p, blocks);
+  const int q0 = 32 * (a.blk * nw + w), myq = q0 + j, qc = min(myq, L - 1);
+  const bool live = q0 < L;
+  const float c = p.scale * kLog2e;
+  bf16x8 qf[T::KS], df[T::KS];
+  load_frags<D>(p.q + a.base, a.ld, qc, qf);
+  load_frags<D>(p.dout + a.base, a.ld, qc, df);
+  const int64_t stat = ((int64_t)a.bn * p.H + a.h) * L;
+  float delta = 0.f;
+  {
+    bf16x8 of[T::KS];
+    load_frags<D>(p.o + a.base, a.ld, qc, of);
+#pragma unroll
+    for (int ks = 0; ks < T::KS; ++ks)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) delta += (float)of[ks][e] * (float)df[ks][e];
+    delta += __shfl_xor(delta, 32, 64);
+    if (live && myq < L && hf == 0) p.delta[stat + myq] = delta;
+  }
+  const float lse2 = p.lse[stat + qc] * kLog2e;
+  f32x16 acc[T::DT];
+#pragma unroll
+  for (int dt = 0; dt < T::DT; ++dt) acc[dt] = f32x16{};
+  const TB* b1 = p.b1 != nullptr ? (const TB*)p.b1 + (int64_t)a.bn * L : nullptr;
+  const TB* b2 = p.b2 != nullptr ? (const TB*)p.b2 + ((int64_t)(a.b * p.H + a.h) * L + qc) * L : nullptr;
+
+  auto tile = [&](const char* sk, const char* sv, int t0, int k0, auto tail) {
+    constexpr bool TAIL = decltype(tail)::value;
+    float bias[16] = {};
+    if (b1 != nullptr) add_row<TAIL>(b1, k0, hf, L, bias);
+    if (b2 != nullptr) add_row<TAIL>(b2, k0, hf, L, bias);
+    f32x16 s = f32x16{}, d = f32x16{};
+#pragma unroll
+    for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(sk, t0, ks), qf[ks], s);
+#pragma unroll
+    for (int ks = 0; ks < T::KS; ++ks) d = mfma(T::rows(sv, t0, ks), df[ks], d);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float pr = fast_exp2(s[r] * c + (bias[r] * kLog2e - lse2));
+      s[r] = pr * (d[r] - delta);
+      if (TAIL && k0 + acc_row(r, hf) >= L) s[r] = 0.f;
+    }
+    const bf16x8 sb[2] = {acc_to_b<0>(s), acc_to_b<1>(s)};
+#pragma unroll
+    for (int dt = 0; dt < T::DT; ++dt)
+#pragma unroll
+      for (int st = 0; st < 2; ++st) acc[dt] = mfma(T::cols(sk, t0, st, dt), sb[st], acc[dt]);
+  };
+
+  for (int c0 = 0; c0 < L; c0 += T::ROWS) {
+    const int nt = (min(T::ROWS, L - c0) + 31) / 32;
+    if (c0 > 0) __syncthreads();
+    T::stage(smem, p.k + a.base, a.ld, c0, nt, L, nw);
+    T::stage(smem + 16384, p.v + a.base, a.ld, c0, nt, L, nw);
+    __syncthreads();
+    if (!live) continue;
+    for (int t = 0; t < nt; ++t) {
+      const int k0 = c0 + 32 * t;
+      if (k0 + 32 <= L) tile(smem, smem + 16384, 32 * t, k0, std::false_type{});
+      else tile(smem, smem + 16384, 32 * t, k0, std::true_type{});
+    }
+  }
+  if (live && myq < L) {
+    bf16* row = p.dq + a.base + (int64_t)myq * a.ld;
+#pragma unroll
+    for (int dt = 0; dt < T::DT; ++dt) store_row_block<D>(row, acc[dt], dt, hf, p.scale);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// dK, dV and the mask's gradient
+// ---------------------------------------------------------------------------------------------------------------
+template <int D, typename TB>
+__global__ __launch_bounds__(512) void evo_dkdv_kernel(EvoParams p, int blocks) {
+  using T = Tile<D>;
+  __shared__ __attribute__((aligned(1024))) char smem[2 * 16384];
+  __shared__ __attribute__((aligned(16))) float s_lse[T::ROWS], s_delta[T::ROWS];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int hf = lane >> 5, j = lane & 31, L = p.L;
+  const Place a = place<D>(p, blocks);
+  const int k0 = 32 * (a.blk * nw + w), myk = k0 + j, kc = min(myk, L - 1);
+  const bool live = k0 < L;
+  const float c = p.scale * kLog2e;
+  bf16x8 kf[T::KS], vf[T::KS];
+  load_frags<D>(p.k + a.base, a.ld, kc, kf);
+  load_frags<D>(p.v + a.base, a.ld, kc, vf);
+  const int64_t stat = ((int64_t)a.bn * p.H + a.h) * L;
+  const float mask = p.b1 != nullptr ? to_f(((const TB*)p.b1)[(int64_t)a.bn * L + kc]) : 0.f;
+  const TB* b2 = p.b2 != nullptr ? (const TB*)p.b2 + (int64_t)(a.b * p.H + a.h) * L * L + kc : nullptr;
+  f32x16 dk[T::DT], dv[T::DT];
+#pragma unroll
+  for (int dt = 0; dt < T::DT; ++dt) dk[dt] = dv[dt] = f32x16{};
+  float db1 = 0.f;
+
+  for (int c0 = 0; c0 < L; c0 += T::ROWS) {
+    const int nt = (min(T::ROWS, L - c0) + 31) / 32;
+    if (c0 > 0) __syncthreads();
+    T::stage(smem, p.q + a.base, a.ld, c0, nt, L, nw);
+    T::stage(smem + 16384, p.dout + a.base, a.ld, c0, nt, L, nw);
+    for (int i = threadIdx.x; i < 32 * nt; i += blockDim.x) {
+      const bool ok = c0 + i < L;  // queries past the end: a probability of zero
+      s_lse[i] = ok ? p.lse[stat + c0 + i] * kLog2e : INFINITY;
+      s_delta[i] = ok ? p.delta[stat + c0 + i] : 0.f;
+    }
+    __syncthreads();
+    if (!live) continue;
+    for (int t = 0; t < nt; ++t) {
+      float bias[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int qr = min(c0 + 32 * t + acc_row(r, hf), L - 1);
+        bias[r] = b2 != nullptr ? to_f(b2[(int64_t)qr * L]) + mask : mask;
+      }
+      f32x16 s = f32x16{}, d = f32x16{};
+#pragma unroll
+      for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(smem, 32 * t, ks), kf[ks], s);
+#pragma unroll
+      for (int ks = 0; ks < T::KS; ++ks) d = mfma(T::rows(smem + 16384, 32 * t, ks), vf[ks], d);
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        bf16x4 v4;
+        const f32x4 ls = *reinterpret_cast<const f32x4*>(&s_lse[32 * t + 8 * g + 4 * hf]);
+        const f32x4 de = *reinterpret_cast<const f32x4*>(&s_delta[32 * t + 8 * g + 4 * hf]);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) v4[t] = (bf16)(acc[dt][4 * g + t] * inv);
-        *reinterpret_cast<bf16x4*>(orow + 32 * dt + acc_row(4 * g, hf)) = v4;
+        for (int i = 0; i < 4; ++i) {
+          const int r = 4 * g + i;
+          const float pr = fast_exp2(s[r] * c + (bias[r] * kLog2e - ls[i]));
+          s[r] = pr;
+          d[r] = pr * (d[r] - de[i]);
+          db1 += d[r];
+        }
       }
-    if (hf == 0) lse[(int64_t)bnh * L + myq] = (m + log2f(l)) / kLog2e;
+      const bf16x8 pb[2] = {acc_to_b<0>(s), acc_to_b<1>(s)}, sb[2] = {acc_to_b<0>(d), acc_to_b<1>(d)};
+#pragma unroll
+      for (int dt = 0; dt < T::DT; ++dt)
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+          dv[dt] = mfma(T::cols(smem + 16384, 32 * t, st, dt), pb[st], dv[dt]);
+          dk[dt] = mfma(T::cols(smem, 32 * t, st, dt), sb[st], dk[dt]);
+        }
+    }
   }
+  if (!live) return;
+  db1 += __shfl_xor(db1, 32, 64);
+  if (myk < L) {
+    const int64_t row = a.base + (int64_t)myk * a.ld;
+#pragma unroll
+    for (int dt = 0; dt < T::DT; ++dt) {
+      store_row_block<D>(p.dk + row, dk[dt], dt, hf, p.scale);
+      store_row_block<D>(p.dv + row, dv[dt], dt, hf, 1.f);
+    }
+    if (p.db1 != nullptr && hf == 0) unsafeAtomicAdd(p.db1 + (int64_t)a.bn * L + myk, db1);
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// gradient of the pair bias: sum of dS over the rows
+// ---------------------------------------------------------------------------------------------------------------
+constexpr int kPairTiles = 2;  // of 32 keys: a wave's 32 sums and 32 biases a lane leave room for four waves a SIMD
+
+template <int D, typename TB>
+__global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblocks, int kblocks, int rows_per) {
+  using T = Tile<D>;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int hf = lane >> 5, j = lane & 31, L = p.L;
+  int id = blockIdx.x;
+  const int qb = id % qblocks;
+  id /= qblocks;
+  const int kb = id % kblocks;
+  id /= kblocks;
+  const int h = id % p.H;
+  id /= p.H;
+  const int b = id % p.B, chunk = id / p.B;
+  const int q0 = 32 * (qb * nw + w), myq = q0 + j, qc = min(myq, L - 1);
+  if (q0 >= L) return;
+  const int n0 = chunk * rows_per, n1 = min(p.N, n0 + rows_per);
+  const float c = p.scale * kLog2e;
+  const int64_t ld = (int64_t)p.H * D;
+  float bias[kPairTiles][16];
+  int kr[kPairTiles];
+  f32x16 sum[kPairTiles];
+#pragma unroll
+  for (int t = 0; t < kPairTiles; ++t) {
+    const int k0 = 32 * (kb * kPairTiles + t);
+    kr[t] = min(k0 + j, L - 1);
+    sum[t] = f32x16{};
+#pragma unroll
+    for (int r = 0; r < 16; ++r) bias[t][r] = 0.f;
+    add_row<true>((const TB*)p.b2 + ((int64_t)(b * p.H + h) * L + qc) * L, k0, hf, L, bias[t]);
+  }
+#pragma unroll 1
+  for (int n = n0; n < n1; ++n) {
+    const int64_t bn = (int64_t)b * p.N + n, base = bn * L * ld + (int64_t)h * D, stat = (bn * p.H + h) * L;
+    bf16x8 qf[T::KS], df[T::KS], kf[kPairTiles][T::KS], vf[kPairTiles][T::KS];
+    load_frags<D>(p.q + base, ld, qc, qf);
+    load_frags<D>(p.dout + base, ld, qc, df);
+#pragma unroll
+    for (int t = 0; t < kPairTiles; ++t) {
+      load_frags<D>(p.k + base, ld, kr[t], kf[t]);
+      load_frags<D>(p.v + base, ld, kr[t], vf[t]);
+    }
+    const float lse2 = p.lse[stat + qc] * kLog2e, delta = p.delta[stat + qc];
+#pragma unroll
+    for (int t = 0; t < kPairTiles; ++t) {
+      const int k0 = 32 * (kb * kPairTiles + t);
+      float all[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) all[r] = bias[t][r];
+      if (p.b1 != nullptr) {
+        const TB* b1 = (const TB*)p.b1 + bn * L;
+        if (k0 + 32 <= L) add_row<false>(b1, k0, hf, L, all);
+        else add_row<true>(b1, k0, hf, L, all);
+      }
+      f32x16 s = f32x16{}, d = f32x16{};
+#pragma unroll
+      for (int ks = 0; ks < T::KS; ++ks) s = mfma(kf[t][ks], qf[ks], s);
+#pragma unroll
+      for (int ks = 0; ks < T::KS; ++ks) d = mfma(vf[t][ks], df[ks], d);
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        sum[t][r] += fast_exp2(s[r] * c + (all[r] * kLog2e - lse2)) * (d[r] - delta);
+    }
+  }
+  if (myq >= L) return;
+  float* out = p.part + (((int64_t)chunk * p.B + b) * p.H + h) * L * L + (int64_t)myq * L;
+#pragma unroll
+  for (int t = 0; t < kPairTiles; ++t)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int k = 32 * (kb * kPairTiles + t) + 8 * g + 4 * hf;
+      if (L % 4 == 0 && k < L) {
+        *reinterpret_cast<f32x4*>(out + k) = f32x4{sum[t][4 * g], sum[t][4 * g + 1], sum[t][4 * g + 2], sum[t][4 * g + 3]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (k + i < L) out[k + i] = sum[t][4 * g + i];
+      }
+    }
+}
+
+template <typename TB>
+__global__ __launch_bounds__(256) void evo_pair_sum_kernel(const float* __restrict__ part, TB* __restrict__ out,
+                                                           int64_t n, int chunks) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  if (n % 4 == 0) {
+    f32x4 s = *reinterpret_cast<const f32x4*>(part + i);
+#pragma unroll 4
+    for (int c = 1; c < chunks; ++c) s += *reinterpret_cast<const f32x4*>(part + c * n + i);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) out[i + t] = from_f<TB>(s[t]);
+    return;
+  }
+  for (int t = 0; t < 4 && i + t < n; ++t) {
+    float s = 0.f;
+    for (int c = 0; c < chunks; ++c) s += part[c * n + i + t];
+    out[i + t] = from_f<TB>(s);
+  }
+}
+
+bool bad_shape(int bias_dtype, int B, int N, int L, int H, int D) {
+  const int64_t blocks = (int64_t)B * N * H * ((L + 31) / 32);
+  return (D != 32 && D != 64 && D != 128) || (bias_dtype != kBF16 && bias_dtype != kF32) || blocks > 0x7fffffff;
+}
+
+// Waves of a workgroup: 32 positions each, at most 256 of them (a row's operands are then staged once), evenly spread
+int waves_of(int L) {
+  const int tiles = (L + 31) / 32, blocks = (tiles + 7) / 8;
+  return (tiles + blocks - 1) / blocks;
 }
 
 }  // namespace
 
-// q/k/v/o [B, N, L, H, D] bf16; b1 [B, N, 1, 1, L] or null; b2 [B, 1, H, L, L] or null (bias dtype: 1 = bf16,
-// 0 = fp32); lse [B, N, H, L] fp32 (natural log of the softmax normaliser of the scaled+biased scores).
+#define HDS_EVO_ALL(CALL)                                                                                           \
+  if (bias_dtype == kBF16) {                                                                                        \
+    if (D == 32) CALL(32, bf16); else if (D == 64) CALL(64, bf16); else CALL(128, bf16);                            \
+  } else {                                                                                                          \
+    if (D == 32) CALL(32, float); else if (D == 64) CALL(64, float); else CALL(128, float);                         \
+  }
+
+// q/k/v/o [B, N, L, H, D] bf16, 16-byte aligned; b1 [B, N, 1, 1, L] or null; b2 [B, 1, H, L, L] or null (bias dtype: 1 =
+// bf16, 0 = fp32); lse [B, N, H, L] fp32 (natural log of the softmax normaliser of the scaled + biased scores).
 HDS_EXPORT int hds_evoformer_fwd(const void* q, const void* k, const void* v, const void* b1, const void* b2,
                                  int bias_dtype, void* o, float* lse, int B, int N, int L, int H, int D, float scale,
                                  hipStream_t st) {
   if (B <= 0 || N <= 0 || L <= 0 || H <= 0) return 0;
-  if (D != 32 && D != 64 && D != 128) return hipErrorInvalidValue;
-  if ((L + 31) / 32 > 65535) return hipErrorInvalidValue;
-  const dim3 grid(B * N * H, (L + 31) / 32);
+  if (bad_shape(bias_dtype, B, N, L, H, D)) return hipErrorInvalidValue;
+  EvoParams p{};
+  p.q = (const bf16*)q; p.k = (const bf16*)k; p.v = (const bf16*)v; p.b1 = b1; p.b2 = b2; p.out = (bf16*)o; p.lse = lse;
+  p.B = B; p.N = N; p.L = L; p.H = H; p.scale = scale;
+  const int nw = waves_of(L), blocks = (L + 32 * nw - 1) / (32 * nw);
 #define HDS_EVO(DD, TT)                                                                                             \
-  hipLaunchKernelGGL((evo_fwd_kernel<DD, TT>), grid, dim3(64), 0, st, (const bf16*)q, (const bf16*)k,             \
-                     (const bf16*)v, (const TT*)b1, (const TT*)b2, (bf16*)o, lse, N, L, H, scale)
-#define HDS_EVO_D(TT)                                                                                               \
-  if (D == 32) HDS_EVO(32, TT); else if (D == 64) HDS_EVO(64, TT); else HDS_EVO(128, TT);
-  if (bias_dtype == kBF16) {
-    HDS_EVO_D(bf16)
-  } else if (bias_dtype == kF32) {
-    HDS_EVO_D(float)
-  } else {
-    return hipErrorInvalidValue;
-  }
-#undef HDS_EVO_D
+  hipLaunchKernelGGL((evo_fwd_kernel<DD, TT>), dim3(blocks * H * B * N), dim3(64 * nw), 0, st, p, blocks)
+  HDS_EVO_ALL(HDS_EVO)
 #undef HDS_EVO
+  return hipGetLastError();
+}
+
+// Chunks of rows that the pair bias' gradient is summed in, and so the floats of scratch it wants: chunks * B * H * L * L.
+// A wave walks over its chunk alone, so there are as many as fill the chip twice over, of at least four rows.
+HDS_EXPORT int hds_evoformer_pair_chunks(int B, int N, int L, int H) {
+  if (B <= 0 || N <= 0 || L <= 0 || H <= 0) return 0;
+  const int64_t waves = (int64_t)B * H * ((L + 31) / 32) * ((L + 32 * kPairTiles - 1) / (32 * kPairTiles));
+  int64_t chunks = (2 * 4 * 256 + waves - 1) / waves;
+  const int64_t most = (N + 3) / 4;
+  if (chunks > most) chunks = most;
+  const int per = (int)((N + chunks - 1) / chunks);
+  return (N + per - 1) / per;
+}
+
+// Gradients of the forward above from its result and lse. delta [B, N, H, L] fp32 scratch. db1 [B, N, L] fp32, zeroed, or
+// null; db2 [B, H, L, L] of the biases' dtype, or null; part: see hds_evoformer_pair_chunks (with db2).
+HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, const void* o, const float* lse,
+                                 const void* dout, void* dq, void* dk, void* dv, float* delta, const void* b1,
+                                 const void* b2, int bias_dtype, float* db1, void* db2, float* part, int B, int N, int L,
+                                 int H, int D, float scale, hipStream_t st) {
+  if (B <= 0 || N <= 0 || L <= 0 || H <= 0) return 0;
+  if (bad_shape(bias_dtype, B, N, L, H, D) || (db2 != nullptr && (b2 == nullptr || part == nullptr)))
+    return hipErrorInvalidValue;
+  EvoParams p{};
+  p.q = (const bf16*)q; p.k = (const bf16*)k; p.v = (const bf16*)v; p.o = (const bf16*)o; p.dout = (const bf16*)dout;
+  p.b1 = b1; p.b2 = b2; p.dq = (bf16*)dq; p.dk = (bf16*)dk; p.dv = (bf16*)dv; p.lse = (float*)lse; p.delta = delta;
+  p.db1 = db1; p.part = part; p.B = B; p.N = N; p.L = L; p.H = H; p.scale = scale;
+  const int nw = waves_of(L), blocks = (L + 32 * nw - 1) / (32 * nw);
+  const dim3 grid(blocks * H * B * N), threads(64 * nw);
+#define HDS_EVO(DD, TT)                                                                                             \
+  do {                                                                                                              \
+    hipLaunchKernelGGL((evo_dq_kernel<DD, TT>), grid, threads, 0, st, p, blocks);                                   \
+    hipLaunchKernelGGL((evo_dkdv_kernel<DD, TT>), grid, threads, 0, st, p, blocks);                                 \
+  } while (0)
+  HDS_EVO_ALL(HDS_EVO)
+#undef HDS_EVO
+  if (db2 != nullptr) {
+    const int chunks = hds_evoformer_pair_chunks(B, N, L, H), per = (N + chunks - 1) / chunks;
+    const int tiles = (L + 31) / 32, w4 = (tiles + (tiles + 3) / 4 - 1) / ((tiles + 3) / 4), qblocks = (L + 32 * w4 - 1) / (32 * w4);
+    const int kblocks = (L + 32 * kPairTiles - 1) / (32 * kPairTiles);
+    const int64_t n = (int64_t)B * H * L * L, grid2 = (int64_t)chunks * B * H * kblocks * qblocks;
+    if (grid2 > 0x7fffffff || (n + 1023) / 1024 > 0x7fffffff) return hipErrorInvalidValue;
+#define HDS_EVO(DD, TT)                                                                                             \
+  hipLaunchKernelGGL((evo_dpair_kernel<DD, TT>), dim3(grid2), dim3(64 * w4), 0, st, p, qblocks, kblocks, per)
+    HDS_EVO_ALL(HDS_EVO)
+#undef HDS_EVO
+    if (bias_dtype == kBF16)
+      hipLaunchKernelGGL(evo_pair_sum_kernel<bf16>, dim3((n + 1023) / 1024), dim3(256), 0, st, part, (bf16*)db2, n,
+                         chunks);
+    else
+      hipLaunchKernelGGL(evo_pair_sum_kernel<float>, dim3((n + 1023) / 1024), dim3(256), 0, st, part, (float*)db2, n,
+                         chunks);
+  }
   return hipGetLastError();
 }

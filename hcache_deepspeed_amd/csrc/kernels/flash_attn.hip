@@ -885,7 +885,7 @@ __device__ __forceinline__ void stage_full8(char* tile, const bf16* tile_base, c
 // PIPE: LDS operand reads issued two MFMAs ahead of their use as inline asm with counted lgkmcnt waits (a ring of
 // three fragments), instead of the compiler's load -> lgkmcnt(0) -> MFMA per product, which exposes the LDS latency
 // of every read (the MFMA pipe sat idle ~2/3 of the time: PMC 37 % MFMA busy).
-template <int D, int PRIO, bool EVO = false, int PIPE = 0>
+template <int D, int PRIO, int PIPE = 0>
 __global__ __launch_bounds__(512) void attn_bwd_dkdv_split_kernel(AttnParams p) {
   constexpr int BK = 128;
   constexpr int KS = Dim<D>::KS, DT = Dim<D>::DT;
@@ -1052,17 +1052,13 @@ __global__ __launch_bounds__(512) void attn_bwd_dkdv_split_kernel(AttnParams p) 
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int r = 4 * r4 + j;
-          float x = PIPE >= 2 ? sacc[r] * c - l4[j] : sacc[r] * c - l4[j] * kLog2e;  // PIPE 2: lse2 staged
-          if constexpr (EVO) x += evo_bias(p, b, hk, qt * BN + qr0 + j, myk) * kLog2e;
-          float pr = fast_exp2(x);
-          if constexpr (EVO) {
-            if (masked(p, qt * BN + qr0 + j, myk, len)) pr = 0.f;
-          }
+          const float x = PIPE >= 2 ? sacc[r] * c - l4[j] : sacc[r] * c - l4[j] * kLog2e;  // PIPE 2: lse2 staged
+          const float pr = fast_exp2(x);
           sacc[r] = pr;
           dpacc[r] = pr * (dpacc[r] - d4[j]);
         }
       }
-      if (!EVO && need_mask) {  // wave-uniform branch: interior tiles run no mask VALU at all
+      if (need_mask) {  // wave-uniform branch: interior tiles run no mask VALU at all
 #pragma unroll
         for (int r = 0; r < 16; ++r)
           if (outside(qt * BN + 32 * qh + acc_row(r, h), qlo, qhi)) sacc[r] = dpacc[r] = 0.f;
@@ -1150,7 +1146,7 @@ __global__ __launch_bounds__(512) void attn_bwd_dkdv_split_kernel(AttnParams p) 
 // PIPE: as in the dK/dV kernel -- LDS operand reads two MFMAs ahead as inline asm with counted waits, so neither
 // the per-read LDS latency nor the compiler's vmcnt(0) in front of the transposed-read builtin (which waits for
 // the NEXT tile's LDS-DMA in the middle of every iteration) stalls the MFMA pipe.
-template <int D, int NW, int PRIO, bool EVO = false, int PIPE = 0>
+template <int D, int NW, int PRIO, int PIPE = 0>
 __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(AttnParams p) {
   constexpr int BM = 32 * NW;
   constexpr int KS = Dim<D>::KS, DT = Dim<D>::DT, TL = Dim<D>::TILE;
@@ -1247,7 +1243,7 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(AttnParams p) {
     if (p.window > 0 && k0 + BN - 1 <= wq_lo - p.window) skip = true;
     if (!skip) {
       f32x16 s[2], dp[2];
-      if constexpr (PIPE != 0 && D == 128 && !EVO) {
+      if constexpr (PIPE != 0 && D == 128) {
         // j = 16 t + 8 which + ks: which 0 -> S (K rows x Q), 1 -> dP (V rows x dO)
         s[0] = s[1] = dp[0] = dp[1] = f32x16{};
         bf16x8 fa[3];
@@ -1294,45 +1290,16 @@ __global__ __launch_bounds__(64 * NW) void attn_bwd_dq_kernel(AttnParams p) {
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = k0 + 32 * t + acc_row(r, h);
-          float x = s[t][r] * c - lse2;
-          if constexpr (EVO) x += evo_bias(p, b, hq, myq, key) * kLog2e;
-          float pr = fast_exp2(x);
-          if constexpr (EVO) {
-            const bool off = masked(p, myq, key, len);
-            if (off) pr = 0.f;
-            s[t][r] = pr * (dp[t][r] - dlt);  // dS^T
-            // pair-bias gradient, summed over the N rows of the MSA (float atomics into [B][H][L][L])
-            if (p.db2 && !off)
-              atomicAdd(p.db2 + ((int64_t)((b / p.evo_n) * p.hq + hq) * len + myq) * len + key, s[t][r]);
-          } else {
-            s[t][r] = pr * (dp[t][r] - dlt);  // dS^T
-          }
-        }
-      if (!EVO && need_mask) {  // wave-uniform branch: interior tiles run no mask VALU at all
+        for (int r = 0; r < 16; ++r) s[t][r] = fast_exp2(s[t][r] * c - lse2) * (dp[t][r] - dlt);  // dS^T
+      if (need_mask) {  // wave-uniform branch: interior tiles run no mask VALU at all
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int r = 0; r < 16; ++r)
             if (outside(k0 + 32 * t + acc_row(r, h), klo, khi)) s[t][r] = 0.f;
       }
-      if constexpr (EVO) {
-        if (p.db1) {  // mask-bias gradient: sum over this wave's 32 queries, then over heads by atomics
-#pragma unroll
-          for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              float v = s[t][r];
-#pragma unroll
-              for (int off = 1; off < 32; off <<= 1) v += __shfl_xor(v, off, 64);
-              const int key = k0 + 32 * t + acc_row(r, h);
-              if ((lane & 31) == 0 && key < len) atomicAdd(p.db1 + (int64_t)b * len + key, v);
-            }
-        }
-      }
       const bf16x8 sb[4] = {acc_to_b<0>(s[0]), acc_to_b<1>(s[0]), acc_to_b<0>(s[1]), acc_to_b<1>(s[1])};
-      if constexpr (PIPE != 0 && D == 128 && !EVO) {
+      if constexpr (PIPE != 0 && D == 128) {
         bf16x8 ft[3];
         const uint32_t b0 = (uint32_t)(uintptr_t)Kt + ty0, b1 = (uint32_t)(uintptr_t)Kt + ty1;
         auto ldt = [&](int j) {
@@ -1408,10 +1375,6 @@ AttnParams make_params(const void* q, const void* k, const void* v, void* o, flo
   p.scale = scale;
   p.causal = causal;
   p.window = window;
-  p.b1 = p.b2 = nullptr;
-  p.bias_f32 = 0;
-  p.db1 = p.db2 = nullptr;
-  p.evo_n = 1;
   return p;
 }
 
@@ -1524,9 +1487,9 @@ int launch_bwd(const AttnParams& p, int batch, int max_len, int total_tokens, in
     if (g_dkdv_nw == 8) {
       const dim3 grid((max_len + 127) / 128, hkv, batch);
       if (g_bwd_pipe == 2 && D == 128 && p.lse2)
-        hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, 1, false, 2>), grid, dim3(512), 0, st, p);
+        hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, 1, 2>), grid, dim3(512), 0, st, p);
       else if (g_bwd_pipe && D == 128)
-        hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, 1, false, 1>), grid, dim3(512), 0, st, p);
+        hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, 1, 1>), grid, dim3(512), 0, st, p);
       else if (g_bwd_prio)
         hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, 1>), grid, dim3(512), 0, st, p);
       else
@@ -1561,9 +1524,9 @@ int launch_bwd(const AttnParams& p, int batch, int max_len, int total_tokens, in
     if (!done && g_dq_nw == 8) {
       const dim3 grid((max_len + 255) / 256, hq, batch);
       if (g_bwd_pipe == 2 && D == 128)
-        hipLaunchKernelGGL((attn_bwd_dq_kernel<D, 8, 1, false, 2>), grid, dim3(512), 0, st, p);
+        hipLaunchKernelGGL((attn_bwd_dq_kernel<D, 8, 1, 2>), grid, dim3(512), 0, st, p);
       else if (g_bwd_pipe && D == 128)
-        hipLaunchKernelGGL((attn_bwd_dq_kernel<D, 8, 1, false, 1>), grid, dim3(512), 0, st, p);
+        hipLaunchKernelGGL((attn_bwd_dq_kernel<D, 8, 1, 1>), grid, dim3(512), 0, st, p);
       else if (g_bwd_prio)
         hipLaunchKernelGGL((attn_bwd_dq_kernel<D, 8, 1>), grid, dim3(512), 0, st, p);
       else
@@ -1621,42 +1584,4 @@ HDS_EXPORT int hds_attn_bwd(const void* q, const void* k, const void* v, const v
   HDS_ATTN_DIMS(HDS_CASE)
 #undef HDS_CASE
   return hipErrorInvalidValue;
-}
-
-// Evoformer attention backward (DS4Sci_EvoformerAttention): q/k/v/o/dout/dq/dk/dv [B, N, L, H, D] contiguous,
-// lse / delta in this file's [H][B*N*L] layout, biases b1 [B, N, 1, 1, L] and b2 [B, 1, H, L, L] (bf16 or fp32,
-// either may be null), fp32 gradient accumulators db1 [B*N, L] / db2 [B, H, L, L] (zeroed by the caller; null
-// when not wanted). Runs the FlashAttention backward kernels with the biases folded into P.
-HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, const void* o, const float* lse,
-                                 const void* dout, void* dq, void* dk, void* dv, float* delta, const void* b1,
-                                 const void* b2, int bias_f32, float* db1, float* db2, int B, int N, int L, int H,
-                                 int D, float scale, hipStream_t st) {
-  if (!(D == 32 || D == 64 || D == 128) || B <= 0 || N <= 0 || L <= 0 || H <= 0) return hipErrorInvalidValue;
-  int64_t strides[8];
-  for (int i = 0; i < 8; ++i) strides[i] = (int64_t)H * D;
-  const int batch = B * N, total = B * N * L;
-  AttnParams p = make_params(q, k, v, (void*)o, (float*)lse, dout, dq, dk, dv, delta, strides, nullptr, nullptr,
-                             batch, L, total, H, H, scale, 0, 0);
-  p.b1 = b1;
-  p.b2 = b2;
-  p.bias_f32 = bias_f32;
-  p.db1 = db1;
-  p.db2 = db2;
-  p.evo_n = N;
-  const int64_t rows = (int64_t)total * H;
-  switch (D) {
-#define HDS_EVO(d)                                                                                              \
-  case d:                                                                                                       \
-    hipLaunchKernelGGL(attn_bwd_delta_kernel<d>, dim3((rows + 15) / 16), dim3(256), 0, st, p);                 \
-    hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<d, 1, true>), dim3((L + 127) / 128, H, batch), dim3(512), 0, \
-                       st, p);                                                                                  \
-    hipLaunchKernelGGL((attn_bwd_dq_kernel<d, 8, 1, true>), dim3((L + 255) / 256, H, batch), dim3(512), 0, st, \
-                       p);                                                                                      \
-    break;
-    HDS_EVO(32)
-    HDS_EVO(64)
-    HDS_EVO(128)
-#undef HDS_EVO
-  }
-  return hipGetLastError();
 }

@@ -42,29 +42,7 @@ struct AttnParams {
   float scale;
   int causal;
   int window;  // >0: sliding window (keys in (q - window, q])
-  // Evoformer (EVO kernels only): additive biases and their gradients, batch = B * evo_n sequences of seq_len
-  const void* b1;  // [B*N][L]        (bf16 or fp32, bias_f32)
-  const void* b2;  // [B][H][L][L]
-  int bias_f32;
-  float* db1;      // [B*N][L]  fp32, accumulated
-  float* db2;      // [B][H][L][L] fp32, accumulated
-  int evo_n;
 };
-
-__device__ __forceinline__ float ld_bias(const AttnParams& p, const void* base, int64_t i) {
-  return p.bias_f32 ? reinterpret_cast<const float*>(base)[i] : (float)reinterpret_cast<const bf16*>(base)[i];
-}
-
-// Evoformer pair / mask bias of (sequence bn, head h, query q, key) (indices clamped; masked() zeroes padding)
-__device__ __forceinline__ float evo_bias(const AttnParams& p, int bn, int h, int q, int key) {
-  const int L = p.seq_len;
-  q = q < L ? q : L - 1;
-  key = key < L ? key : L - 1;
-  float x = 0.f;
-  if (p.b1) x += ld_bias(p, p.b1, (int64_t)bn * L + key);
-  if (p.b2) x += ld_bias(p, p.b2, ((int64_t)((bn / p.evo_n) * p.hq + h) * L + q) * L + key);
-  return x;
-}
 
 __device__ __forceinline__ void seq_bounds(const AttnParams& p, int b, int& start, int& len) {
   if (p.cu_seqlens) {

@@ -62,3 +62,46 @@ def test_evoformer_backward_runs_hip_kernels(cuda, monkeypatch):
     q, k, v = (torch.randn(1, 2, 64, 2, 32, device=cuda, dtype=torch.bfloat16, requires_grad=True) for _ in range(3))
     DS4Sci_EvoformerAttention(q, k, v, []).sum().backward()
     assert called and q.grad is not None and torch.isfinite(q.grad.float()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,N,L,H,D,which,bias_dtype", [
+    (1, 1, 1, 1, 32, "both", torch.bfloat16), (1, 3, 31, 2, 64, "both", torch.bfloat16),
+    (2, 5, 33, 3, 32, "both", torch.float32), (1, 2, 64, 2, 128, "mask", torch.bfloat16),
+    (1, 9, 193, 4, 32, "pair", torch.bfloat16), (1, 2, 257, 1, 64, "both", torch.bfloat16),
+    (1, 33, 300, 2, 32, "both", torch.bfloat16), (1, 70, 40, 4, 64, "pair", torch.float32),
+    (1, 2, 545, 2, 128, "both", torch.bfloat16), (2, 130, 17, 4, 32, "both", torch.bfloat16)])
+def test_evoformer_edges_hip(cuda, B, N, L, H, D, which, bias_dtype):
+    """Tails of the 32-position tiles, odd rows of the pair bias, one and several LDS chunks, one and several chunks of
+    the rows in the pair gradient; masked keys at -1e9 and at minus infinity. Against float64; p, ds and the results are
+    rounded to bf16 (2^-9 each), the sums to 32 bits."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    q, k, v, do = (rnd(B, N, L, H, D).bfloat16() for _ in range(4))
+    b1 = b2 = None
+    if which != "pair":
+        gone = torch.rand(B, N, 1, 1, L, device="cuda", generator=g) < 0.2
+        gone[..., 0] = False
+        low = torch.full_like(gone, -1e9, dtype=bias_dtype)
+        low[:, ::2] = float("-inf")
+        b1 = torch.where(gone, low, torch.zeros((), dtype=bias_dtype, device="cuda"))
+    if which != "mask":
+        b2 = rnd(B, 1, H, L, L).to(bias_dtype)
+    leaves = [t.requires_grad_() for t in (q, k, v, b2) if t is not None]
+    out = DS4Sci_EvoformerAttention(q, k, v, [b1, b2])
+    got = [out] + list(torch.autograd.grad(out, leaves, do))
+    exact = [t.detach().double().requires_grad_() for t in leaves]
+    qh, kh, vh = (t.transpose(-2, -3) for t in exact[:3])
+    s = torch.matmul(qh, kh.transpose(-1, -2)) / math.sqrt(D)
+    if b1 is not None:
+        s = s + b1.double()
+    if b2 is not None:
+        s = s + exact[3]
+    ref = torch.matmul(torch.softmax(s, -1), vh).transpose(-2, -3)
+    want = [ref] + list(torch.autograd.grad(ref, exact, do.double()))
+    for x, y in zip(got, want):
+        assert torch.isfinite(x).all()
+        assert (x.double() - y).norm() <= 4 * 2**-8 * y.norm() + 1e-6
+    if b2 is not None:  # no atomics in these gradients
+        again = torch.autograd.grad(DS4Sci_EvoformerAttention(q, k, v, [b1, b2]), leaves, do)
+        assert all(torch.equal(x, y) for x, y in zip(got[1:], again))
