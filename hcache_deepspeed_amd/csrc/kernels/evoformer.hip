@@ -6,7 +6,7 @@
 // q, k, v [B, N, L, H, D]; bias1 [B, N, 1, 1, L] (mask), bias2 [B, 1, H, L, L] (pair bias, shared by the N rows), both in
 // bf16 or both in fp32 and added in fp32. The sequences are short (16 to 400 positions), the heads small (32, 64), the
 // rows many: the products are a few GFLOP and the inputs a few tens of MB, so the kernels are bound by the vector
-// instructions between the products (exponential, bias, conversion: about 12 a score) and by how the operands get there.
+// instructions between the products (exponential, differences, conversion) and by how the operands get there.
 //   * forward and dQ: a wave holds 32 queries of one (b, n, h), the workgroup stages its keys and values in LDS once
 //     (LDS-DMA, 32 KB a chunk, so that several workgroups share a CU). S^T = K Q^T puts the query on the lane: softmax
 //     statistics are lane-local and the S^T accumulator is the B operand of the next product (acc_to_b); V^T and K^T
@@ -15,7 +15,7 @@
 //   * pair-bias gradient: the sum of dS over the N rows stays in registers. A wave owns 32 queries x 64 keys of one
 //     (b, h) and walks over a chunk of the rows, recomputing the two products that dS needs; chunks are added by a second
 //     kernel that also rounds. No atomics, the same result every time.
-// Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): forward 53 us, dQ 58, dK / dV 124, pair gradient 78 + 5
+// Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): forward 42 us, dQ 51, dK / dV 51, pair gradient 59 + 5
 // (before: one wave a workgroup with operands from global memory and 2-byte reads of V 169 us; the FlashAttention
 // backward kernels with 32-bit atomics into the pair gradient 271 + 1,585 us).
 #include "attn_common.h"
@@ -31,6 +31,10 @@ constexpr float kLog2e = 1.4426950408889634f;
 // LDS tiles: rows of 2 D bytes whose 16-byte chunks are XOR-swizzled by the row, so that 16 lanes reading 16 rows at one
 // chunk (ds_read_b128), and 16 lanes reading 32 bytes of 4 rows (ds_read_b64_tr_b16), meet every bank once
 // ---------------------------------------------------------------------------------------------------------------
+// most waves of a workgroup: the 128-wide accumulators want more than the 256 registers that eight leave each
+template <int D>
+constexpr int kWaves = D == 128 ? 4 : 8;
+
 template <int D>
 struct Tile {
   static constexpr int RB = 2 * D, CH = D / 8;       // bytes, chunks of a row
@@ -76,27 +80,188 @@ struct Tile {
 // ---------------------------------------------------------------------------------------------------------------
 // biases
 // ---------------------------------------------------------------------------------------------------------------
-template <typename TB>
-struct __attribute__((packed, aligned(sizeof(TB)))) Four {  // L may be odd: rows are aligned to their element only
-  TB v[4];
+// They are added to the raw scores, divided by the scale: x = scale * log2(e) * (q . k + bias / scale). bf16 biases go
+// through the matrix cores, which have room: a pair bias tile times the matrix (1 / scale) I, a mask as an outer product
+// with 1 / scale. 1 / scale is cut into bf16 pieces (one for D = 64, three otherwise, which make up all 24 bits), so
+// that the products are exact. That takes two 16-byte loads a lane and no vector instruction a score, where unpacking
+// and adding took four, and two-byte loads where keys are on the lanes (forward 53 -> 42 us, dQ 58 -> 51, dK / dV
+// 124 -> 51, pair gradient 78 -> 59). Zeros of I meet other keys of the same query only: minus
+// infinity is made the lowest finite value first, which 1 / scale > 1 takes back to minus infinity. fp32 biases are
+// added by vector instructions.
+struct __attribute__((packed, aligned(2))) Eight {  // L may be odd: rows are aligned to their element only
+  u32x4 v;
+};
+struct __attribute__((packed, aligned(4))) Four {
+  f32x4 v;
 };
 
-// b[r] += row[k0 + acc_row(r, hf)]; TAIL: places past the end are read at the end
-template <bool TAIL, typename TB>
-__device__ __forceinline__ void add_row(const TB* row, int k0, int hf, int L, float (&b)[16]) {
+template <int D>
+struct Inverse {  // 1 / scale in bf16 pieces, rounded towards zero: all of one sign
+  static constexpr int N = D == 64 ? 1 : 3;
+  bf16 v[N];
+  __device__ __forceinline__ explicit Inverse(float scale) {
+    float r = 1.f / scale;
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int k = k0 + 8 * g + 4 * hf;
-    if constexpr (TAIL) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) b[4 * g + t] += to_f(row[min(k + t, L - 1)]);
-    } else {
-      const Four<TB> f = *reinterpret_cast<const Four<TB>*>(row + k);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) b[4 * g + t] += to_f(f.v[t]);
+    for (int i = 0; i < N; ++i) {
+      const float t = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xffff0000u);
+      v[i] = (bf16)t;
+      r -= t;
     }
   }
+};
+
+// Fragments of (1 / scale) I, either operand: row or column lane & 31, elements 16 ks + 8 hf ..
+template <int D>
+struct Diagonal {
+  bf16x8 f[Inverse<D>::N][2];
+  __device__ __forceinline__ explicit Diagonal(const Inverse<D>& inv) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < Inverse<D>::N; ++i)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[i][ks][e] = 16 * ks + 8 * (lane >> 5) + e == (lane & 31) ? inv.v[i] : (bf16)0.f;
+  }
+};
+
+constexpr uint32_t kLowest = 0xff7fff7fu;  // two bf16
+
+__device__ __forceinline__ u32x4 finite(u32x4 v) {  // minus infinity (and negative NaN) to the lowest finite value
+  typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+  const u16x8 low = __builtin_bit_cast(u16x8, u32x4{kLowest, kLowest, kLowest, kLowest});
+  return __builtin_bit_cast(u32x4, __builtin_elementwise_min(__builtin_bit_cast(u16x8, v), low));
 }
+
+// elements k .. k + 7 of a row of L; TAIL: past the end the lowest value
+template <bool TAIL>
+__device__ __forceinline__ u32x4 load_eight(const bf16* row, int k, int L) {
+  if constexpr (!TAIL) return reinterpret_cast<const Eight*>(row + k)->v;
+  typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+  u16x8 r;
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    r[e] = k + e < L ? __builtin_bit_cast(uint16_t, row[min(k + e, L - 1)]) : (uint16_t)kLowest;
+  return __builtin_bit_cast(u32x4, r);
+}
+
+// a mask value per lane (row or column lane & 31) against 1 / scale on the other side
+template <int D>
+__device__ __forceinline__ bf16x8 spread(bf16 v) {
+  bf16x8 f{};
+  if ((threadIdx.x & 63) < 32) {
+#pragma unroll
+    for (int i = 0; i < Inverse<D>::N; ++i) f[i] = v;
+  }
+  return f;
+}
+template <int D>
+__device__ __forceinline__ bf16x8 pieces(const Inverse<D>& inv) {
+  bf16x8 f{};
+  if ((threadIdx.x & 63) < 32) {
+#pragma unroll
+    for (int i = 0; i < Inverse<D>::N; ++i) f[i] = inv.v[i];
+  }
+  return f;
+}
+
+// Biases of a wave's tiles with keys down the rows of S^T and a query on each lane
+template <int D, typename TB>
+struct QueryBias;
+
+template <int D>
+struct QueryBias<D, bf16> {
+  const bf16 *b1, *b2;  // the row of (b, n), the row of (b, h, query)
+  Diagonal<D> eye;
+  bf16x8 inv;
+  u32x4 seen;  // largest bit patterns met: above 0xff80 is a negative NaN, which finite() hides
+  __device__ __forceinline__ QueryBias(const bf16* m, const bf16* pair, float scale)
+      : b1(m), b2(pair), eye(Inverse<D>(scale)), inv(pieces<D>(Inverse<D>(scale))), seen{} {}
+  template <bool TAIL>
+  __device__ __forceinline__ void load_pair(int k0, int L, u32x4 (&f)[2]) const {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) f[ks] = load_eight<TAIL>(b2, k0 + 16 * ks + 8 * ((threadIdx.x & 63) >> 5), L);
+  }
+  __device__ __forceinline__ f32x16 add_pair(const u32x4 (&f)[2], f32x16 s) const {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < Inverse<D>::N; ++i) s = mfma(eye.f[i][ks], __builtin_bit_cast(bf16x8, finite(f[ks])), s);
+    return s;
+  }
+  template <bool TAIL>
+  __device__ __forceinline__ f32x16 add_mask(int k0, int L, f32x16 s) const {
+    if (TAIL || b1 != nullptr) {
+      const int k = k0 + (threadIdx.x & 31);
+      bf16 v = b1 != nullptr ? b1[TAIL ? min(k, L - 1) : k] : (bf16)0.f;
+      if (TAIL && k >= L) v = __builtin_bit_cast(bf16, (uint16_t)kLowest);
+      s = mfma(spread<D>(v), inv, s);
+    }
+    return s;
+  }
+  template <bool TAIL, bool WATCH = false>
+  __device__ __forceinline__ f32x16 add(int k0, int hf, int L, f32x16 s) {
+    s = add_mask<TAIL>(k0, L, s);
+    if (b2 != nullptr) {
+      u32x4 f[2];
+      load_pair<TAIL>(k0, L, f);
+      if constexpr (WATCH) {
+        typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+          seen = __builtin_bit_cast(u32x4, __builtin_elementwise_max(__builtin_bit_cast(u16x8, seen),
+                                                                     __builtin_bit_cast(u16x8, f[ks])));
+      }
+      s = add_pair(f, s);
+    }
+    return s;
+  }
+  __device__ __forceinline__ bool nan() const {
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bad |= (seen[i] & 0xffffu) > 0xff80u || (seen[i] >> 16) > 0xff80u;
+    return bad;
+  }
+};
+
+template <int D>
+struct QueryBias<D, float> {
+  const float *b1, *b2;
+  float r;
+  __device__ __forceinline__ QueryBias(const float* m, const float* pair, float scale) : b1(m), b2(pair), r(1.f / scale) {}
+  template <bool TAIL>
+  static __device__ __forceinline__ void row(const float* b, int k0, int hf, int L, float r, f32x16& s) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int k = k0 + 8 * g + 4 * hf;
+      f32x4 f;
+      if constexpr (TAIL) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) f[t] = b[min(k + t, L - 1)];
+      } else {
+        f = reinterpret_cast<const Four*>(b + k)->v;
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) s[4 * g + t] += f[t] * r;
+    }
+  }
+  template <bool TAIL>
+  __device__ __forceinline__ f32x16 mask_end(int k0, int hf, int L, f32x16 s) const {
+    if constexpr (TAIL) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (k0 + acc_row(i, hf) >= L) s[i] = -INFINITY;
+    }
+    return s;
+  }
+  template <bool TAIL, bool WATCH = false>
+  __device__ __forceinline__ f32x16 add(int k0, int hf, int L, f32x16 s) {
+    if (b1 != nullptr) row<TAIL>(b1, k0, hf, L, r, s);
+    if (b2 != nullptr) row<TAIL>(b2, k0, hf, L, r, s);
+    return mask_end<TAIL>(k0, hf, L, s);
+  }
+  __device__ __forceinline__ bool nan() const { return false; }
+};
 
 struct EvoParams {
   const bf16 *q, *k, *v, *o, *dout;
@@ -145,7 +310,7 @@ __device__ __forceinline__ void load_frags(const bf16* m, int64_t ld, int row, b
 // forward
 // ---------------------------------------------------------------------------------------------------------------
 template <int D, typename TB>
-__global__ __launch_bounds__(512) void evo_fwd_kernel(EvoParams p, int blocks) {
+__global__ __launch_bounds__(64 * kWaves<D>) void evo_fwd_kernel(EvoParams p, int blocks) {
   using T = Tile<D>;
   __shared__ __attribute__((aligned(1024))) char smem[2 * 16384];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -159,33 +324,28 @@ __global__ __launch_bounds__(512) void evo_fwd_kernel(EvoParams p, int blocks) {
   f32x16 acc[T::DT];
 #pragma unroll
   for (int dt = 0; dt < T::DT; ++dt) acc[dt] = f32x16{};
-  float m = -INFINITY, l = 0.f;
-  const TB* b1 = p.b1 != nullptr ? (const TB*)p.b1 + (int64_t)a.bn * L : nullptr;
-  const TB* b2 = p.b2 != nullptr ? (const TB*)p.b2 + ((int64_t)(a.b * p.H + a.h) * L + qc) * L : nullptr;
+  float m = -INFINITY, l = 0.f;  // largest raw score, sum of the exponentials
+  QueryBias<D, TB> bias(p.b1 != nullptr ? (const TB*)p.b1 + (int64_t)a.bn * L : nullptr,
+                        p.b2 != nullptr ? (const TB*)p.b2 + ((int64_t)(a.b * p.H + a.h) * L + qc) * L : nullptr, p.scale);
 
   auto tile = [&](const char* sk, const char* sv, int t0, int k0, auto tail) {
     constexpr bool TAIL = decltype(tail)::value;
-    float bias[16] = {};
-    if (b1 != nullptr) add_row<TAIL>(b1, k0, hf, L, bias);
-    if (b2 != nullptr) add_row<TAIL>(b2, k0, hf, L, bias);
     f32x16 s = f32x16{};
 #pragma unroll
     for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(sk, t0, ks), qf[ks], s);
-    float top = -INFINITY;
+    s = bias.template add<TAIL, true>(k0, hf, L, s);
+    float top = s[0];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] = s[r] * c + bias[r] * kLog2e;
-      if (TAIL && k0 + acc_row(r, hf) >= L) s[r] = -INFINITY;
-      top = fmaxf(top, s[r]);
-    }
+    for (int r = 1; r < 15; r += 2) top = fmaxf(fmaxf(top, s[r]), s[r + 1]);
+    top = fmaxf(top, s[15]);
     top = fmaxf(top, __shfl_xor(top, 32, 64));
     const float mn = fmaxf(m, top);
-    const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - mn);
+    const float alpha = m == -INFINITY ? 0.f : fast_exp2((m - mn) * c);
     m = mn;
     float sum = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = fast_exp2(s[r] - mn);
+      s[r] = fast_exp2((s[r] - mn) * c);  // (not s c - mn c: a row whose keys all have a mask of -1e9 or below)
       sum += s[r];
     }
     l = l * alpha + sum;  // of this lane's keys; both halves are added at the end
@@ -212,13 +372,14 @@ __global__ __launch_bounds__(512) void evo_fwd_kernel(EvoParams p, int blocks) {
     }
   }
   if (!live) return;
+  if (bias.nan()) l = __builtin_nanf("");
   l += __shfl_xor(l, 32, 64);
   if (myq < L) {
-    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const float inv = l == 0.f ? 0.f : 1.f / l;
     bf16* row = p.out + a.base + (int64_t)myq * a.ld;
 #pragma unroll
     for (int dt = 0; dt < T::DT; ++dt) store_row_block<D>(row, acc[dt], dt, hf, inv);
-    if (hf == 0) p.lse[((int64_t)a.bn * p.H + a.h) * L + myq] = (m + log2f(l)) / kLog2e;
+    if (hf == 0) p.lse[((int64_t)a.bn * p.H + a.h) * L + myq] = (m * c + log2f(l)) / kLog2e;
   }
 }
 
@@ -226,7 +387,7 @@ __global__ __launch_bounds__(512) void evo_fwd_kernel(EvoParams p, int blocks) {
 // dQ, and rowsum(dO * O)
 // ---------------------------------------------------------------------------------------------------------------
 template <int D, typename TB>
-__global__ __launch_bounds__(512) void evo_dq_kernel(EvoParams p, int blocks) {
+__global__ __launch_bounds__(64 * kWaves<D>) void evo_dq_kernel(EvoParams p, int blocks) {
   using T = Tile<D>;
   __shared__ __attribute__((aligned(1024))) char smem[2 * 16384];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -250,27 +411,24 @@ __global__ __launch_bounds__(512) void evo_dq_kernel(EvoParams p, int blocks) {
     delta += __shfl_xor(delta, 32, 64);
     if (live && myq < L && hf == 0) p.delta[stat + myq] = delta;
   }
-  const float lse2 = p.lse[stat + qc] * kLog2e;
+  const float lse_raw = p.lse[stat + qc] / p.scale;
   f32x16 acc[T::DT];
 #pragma unroll
   for (int dt = 0; dt < T::DT; ++dt) acc[dt] = f32x16{};
-  const TB* b1 = p.b1 != nullptr ? (const TB*)p.b1 + (int64_t)a.bn * L : nullptr;
-  const TB* b2 = p.b2 != nullptr ? (const TB*)p.b2 + ((int64_t)(a.b * p.H + a.h) * L + qc) * L : nullptr;
+  QueryBias<D, TB> bias(p.b1 != nullptr ? (const TB*)p.b1 + (int64_t)a.bn * L : nullptr,
+                        p.b2 != nullptr ? (const TB*)p.b2 + ((int64_t)(a.b * p.H + a.h) * L + qc) * L : nullptr, p.scale);
 
   auto tile = [&](const char* sk, const char* sv, int t0, int k0, auto tail) {
     constexpr bool TAIL = decltype(tail)::value;
-    float bias[16] = {};
-    if (b1 != nullptr) add_row<TAIL>(b1, k0, hf, L, bias);
-    if (b2 != nullptr) add_row<TAIL>(b2, k0, hf, L, bias);
     f32x16 s = f32x16{}, d = f32x16{};
 #pragma unroll
     for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(sk, t0, ks), qf[ks], s);
+    s = bias.template add<TAIL>(k0, hf, L, s);
 #pragma unroll
     for (int ks = 0; ks < T::KS; ++ks) d = mfma(T::rows(sv, t0, ks), df[ks], d);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const float pr = fast_exp2(s[r] * c + (bias[r] * kLog2e - lse2));
-      s[r] = pr * (d[r] - delta);
+      s[r] = fast_exp2((s[r] - lse_raw) * c) * (d[r] - delta);
       if (TAIL && k0 + acc_row(r, hf) >= L) s[r] = 0.f;
     }
     const bf16x8 sb[2] = {acc_to_b<0>(s), acc_to_b<1>(s)};
@@ -303,8 +461,8 @@ __global__ __launch_bounds__(512) void evo_dq_kernel(EvoParams p, int blocks) {
 // ---------------------------------------------------------------------------------------------------------------
 // dK, dV and the mask's gradient
 // ---------------------------------------------------------------------------------------------------------------
-template <int D, typename TB>
-__global__ __launch_bounds__(512) void evo_dkdv_kernel(EvoParams p, int blocks) {
+template <int D, typename TB, bool MASK>
+__global__ __launch_bounds__(64 * kWaves<D>) void evo_dkdv_kernel(EvoParams p, int blocks) {
   using T = Tile<D>;
   __shared__ __attribute__((aligned(1024))) char smem[2 * 16384];
   __shared__ __attribute__((aligned(16))) float s_lse[T::ROWS], s_delta[T::ROWS];
@@ -318,8 +476,12 @@ __global__ __launch_bounds__(512) void evo_dkdv_kernel(EvoParams p, int blocks) 
   load_frags<D>(p.k + a.base, a.ld, kc, kf);
   load_frags<D>(p.v + a.base, a.ld, kc, vf);
   const int64_t stat = ((int64_t)a.bn * p.H + a.h) * L;
-  const float mask = p.b1 != nullptr ? to_f(((const TB*)p.b1)[(int64_t)a.bn * L + kc]) : 0.f;
-  const TB* b2 = p.b2 != nullptr ? (const TB*)p.b2 + (int64_t)(a.b * p.H + a.h) * L * L + kc : nullptr;
+  const TB mask = p.b1 != nullptr ? ((const TB*)p.b1)[(int64_t)a.bn * L + kc] : (TB)0.f;
+  const TB* b2 = p.b2 != nullptr ? (const TB*)p.b2 + (int64_t)(a.b * p.H + a.h) * L * L : nullptr;
+  const Inverse<D> inv(p.scale);
+  const Diagonal<D> eye(inv);
+  const bf16x8 one = pieces<D>(inv), maskf = spread<D>((bf16)to_f(mask));
+  const bool full = k0 + 32 <= L;
   f32x16 dk[T::DT], dv[T::DT];
 #pragma unroll
   for (int dt = 0; dt < T::DT; ++dt) dk[dt] = dv[dt] = f32x16{};
@@ -332,21 +494,35 @@ __global__ __launch_bounds__(512) void evo_dkdv_kernel(EvoParams p, int blocks) 
     T::stage(smem + 16384, p.dout + a.base, a.ld, c0, nt, L, nw);
     for (int i = threadIdx.x; i < 32 * nt; i += blockDim.x) {
       const bool ok = c0 + i < L;  // queries past the end: a probability of zero
-      s_lse[i] = ok ? p.lse[stat + c0 + i] * kLog2e : INFINITY;
+      s_lse[i] = ok ? p.lse[stat + c0 + i] / p.scale : INFINITY;
       s_delta[i] = ok ? p.delta[stat + c0 + i] : 0.f;
     }
     __syncthreads();
     if (!live) continue;
     for (int t = 0; t < nt; ++t) {
-      float bias[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int qr = min(c0 + 32 * t + acc_row(r, hf), L - 1);
-        bias[r] = b2 != nullptr ? to_f(b2[(int64_t)qr * L]) + mask : mask;
-      }
       f32x16 s = f32x16{}, d = f32x16{};
 #pragma unroll
       for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(smem, 32 * t, ks), kf[ks], s);
+      if constexpr (sizeof(TB) == 2) {  // queries down the rows: the pair bias is the left operand, its keys contract
+        if (p.b1 != nullptr) s = mfma(one, maskf, s);
+        if (b2 != nullptr) {
+          const bf16* row = (const bf16*)b2 + (int64_t)min(c0 + 32 * t + j, L - 1) * L;
+          u32x4 f[2];
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks)
+            f[ks] = full ? load_eight<false>(row, k0 + 16 * ks + 8 * hf, L) : load_eight<true>(row, k0 + 16 * ks + 8 * hf, L);
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int i = 0; i < Inverse<D>::N; ++i) s = mfma(__builtin_bit_cast(bf16x8, finite(f[ks])), eye.f[i][ks], s);
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int qr = min(c0 + 32 * t + acc_row(r, hf), L - 1);
+          s[r] += (b2 != nullptr ? to_f(b2[(int64_t)qr * L + kc]) + to_f(mask) : to_f(mask)) / p.scale;
+        }
+      }
 #pragma unroll
       for (int ks = 0; ks < T::KS; ++ks) d = mfma(T::rows(smem + 16384, 32 * t, ks), vf[ks], d);
 #pragma unroll
@@ -356,10 +532,10 @@ __global__ __launch_bounds__(512) void evo_dkdv_kernel(EvoParams p, int blocks) 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int r = 4 * g + i;
-          const float pr = fast_exp2(s[r] * c + (bias[r] * kLog2e - ls[i]));
+          const float pr = fast_exp2((s[r] - ls[i]) * c);
           s[r] = pr;
           d[r] = pr * (d[r] - de[i]);
-          db1 += d[r];
+          if (MASK) db1 += d[r];
         }
       }
       const bf16x8 pb[2] = {acc_to_b<0>(s), acc_to_b<1>(s)}, sb[2] = {acc_to_b<0>(d), acc_to_b<1>(d)};
@@ -381,7 +557,7 @@ __global__ __launch_bounds__(512) void evo_dkdv_kernel(EvoParams p, int blocks) 
       store_row_block<D>(p.dk + row, dk[dt], dt, hf, p.scale);
       store_row_block<D>(p.dv + row, dv[dt], dt, hf, 1.f);
     }
-    if (p.db1 != nullptr && hf == 0) unsafeAtomicAdd(p.db1 + (int64_t)a.bn * L + myk, db1);
+    if (MASK && hf == 0) unsafeAtomicAdd(p.db1 + (int64_t)a.bn * L + myk, db1);
   }
 }
 
@@ -408,51 +584,46 @@ __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblo
   const int n0 = chunk * rows_per, n1 = min(p.N, n0 + rows_per);
   const float c = p.scale * kLog2e;
   const int64_t ld = (int64_t)p.H * D;
-  float bias[kPairTiles][16];
-  int kr[kPairTiles];
+  QueryBias<D, TB> bias(nullptr, (const TB*)p.b2 + ((int64_t)(b * p.H + h) * L + qc) * L, p.scale);
+  const int kk0 = 32 * kb * kPairTiles;
   f32x16 sum[kPairTiles];
 #pragma unroll
-  for (int t = 0; t < kPairTiles; ++t) {
-    const int k0 = 32 * (kb * kPairTiles + t);
-    kr[t] = min(k0 + j, L - 1);
-    sum[t] = f32x16{};
+  for (int t = 0; t < kPairTiles; ++t) sum[t] = f32x16{};
+
+  auto walk = [&](auto tail) {
+    constexpr bool TAIL = decltype(tail)::value;
+    u32x4 pair[kPairTiles][2];
+    if constexpr (sizeof(TB) == 2) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) bias[t][r] = 0.f;
-    add_row<true>((const TB*)p.b2 + ((int64_t)(b * p.H + h) * L + qc) * L, k0, hf, L, bias[t]);
-  }
+      for (int t = 0; t < kPairTiles; ++t) bias.template load_pair<TAIL>(kk0 + 32 * t, L, pair[t]);
+    }
 #pragma unroll 1
-  for (int n = n0; n < n1; ++n) {
-    const int64_t bn = (int64_t)b * p.N + n, base = bn * L * ld + (int64_t)h * D, stat = (bn * p.H + h) * L;
-    bf16x8 qf[T::KS], df[T::KS], kf[kPairTiles][T::KS], vf[kPairTiles][T::KS];
-    load_frags<D>(p.q + base, ld, qc, qf);
-    load_frags<D>(p.dout + base, ld, qc, df);
+    for (int n = n0; n < n1; ++n) {
+      const int64_t bn = (int64_t)b * p.N + n, base = bn * L * ld + (int64_t)h * D, stat = (bn * p.H + h) * L;
+      bf16x8 qf[T::KS], df[T::KS];
+      load_frags<D>(p.q + base, ld, qc, qf);
+      load_frags<D>(p.dout + base, ld, qc, df);
+      const float lse_raw = p.lse[stat + qc] / p.scale, delta = p.delta[stat + qc];
+      if (p.b1 != nullptr) bias.b1 = (const TB*)p.b1 + bn * L;
 #pragma unroll
-    for (int t = 0; t < kPairTiles; ++t) {
-      load_frags<D>(p.k + base, ld, kr[t], kf[t]);
-      load_frags<D>(p.v + base, ld, kr[t], vf[t]);
-    }
-    const float lse2 = p.lse[stat + qc] * kLog2e, delta = p.delta[stat + qc];
+      for (int t = 0; t < kPairTiles; ++t) {
+        const int k0 = kk0 + 32 * t, kr = TAIL ? min(k0 + j, L - 1) : k0 + j;
+        bf16x8 kf[T::KS], vf[T::KS];
+        load_frags<D>(p.k + base, ld, kr, kf);
+        load_frags<D>(p.v + base, ld, kr, vf);
+        f32x16 s = f32x16{}, d = f32x16{};
 #pragma unroll
-    for (int t = 0; t < kPairTiles; ++t) {
-      const int k0 = 32 * (kb * kPairTiles + t);
-      float all[16];
+        for (int ks = 0; ks < T::KS; ++ks) s = mfma(kf[ks], qf[ks], s);
+        if constexpr (sizeof(TB) == 2) s = bias.add_pair(pair[t], bias.template add_mask<TAIL>(k0, L, s));
+        else s = bias.template add<TAIL>(k0, hf, L, s);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) all[r] = bias[t][r];
-      if (p.b1 != nullptr) {
-        const TB* b1 = (const TB*)p.b1 + bn * L;
-        if (k0 + 32 <= L) add_row<false>(b1, k0, hf, L, all);
-        else add_row<true>(b1, k0, hf, L, all);
+        for (int ks = 0; ks < T::KS; ++ks) d = mfma(vf[ks], df[ks], d);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[t][r] += fast_exp2((s[r] - lse_raw) * c) * (d[r] - delta);
       }
-      f32x16 s = f32x16{}, d = f32x16{};
-#pragma unroll
-      for (int ks = 0; ks < T::KS; ++ks) s = mfma(kf[t][ks], qf[ks], s);
-#pragma unroll
-      for (int ks = 0; ks < T::KS; ++ks) d = mfma(vf[t][ks], df[ks], d);
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-        sum[t][r] += fast_exp2(s[r] * c + (all[r] * kLog2e - lse2)) * (d[r] - delta);
     }
-  }
+  };
+  if (kk0 + 32 * kPairTiles <= L) walk(std::false_type{}); else walk(std::true_type{});
   if (myq >= L) return;
   float* out = p.part + (((int64_t)chunk * p.B + b) * p.H + h) * L * L + (int64_t)myq * L;
 #pragma unroll
@@ -496,8 +667,8 @@ bool bad_shape(int bias_dtype, int B, int N, int L, int H, int D) {
 }
 
 // Waves of a workgroup: 32 positions each, at most 256 of them (a row's operands are then staged once), evenly spread
-int waves_of(int L) {
-  const int tiles = (L + 31) / 32, blocks = (tiles + 7) / 8;
+int waves_of(int L, int most) {
+  const int tiles = (L + 31) / 32, blocks = (tiles + most - 1) / most;
   return (tiles + blocks - 1) / blocks;
 }
 
@@ -520,7 +691,7 @@ HDS_EXPORT int hds_evoformer_fwd(const void* q, const void* k, const void* v, co
   EvoParams p{};
   p.q = (const bf16*)q; p.k = (const bf16*)k; p.v = (const bf16*)v; p.b1 = b1; p.b2 = b2; p.out = (bf16*)o; p.lse = lse;
   p.B = B; p.N = N; p.L = L; p.H = H; p.scale = scale;
-  const int nw = waves_of(L), blocks = (L + 32 * nw - 1) / (32 * nw);
+  const int nw = waves_of(L, D == 128 ? kWaves<128> : kWaves<32>), blocks = (L + 32 * nw - 1) / (32 * nw);
 #define HDS_EVO(DD, TT)                                                                                             \
   hipLaunchKernelGGL((evo_fwd_kernel<DD, TT>), dim3(blocks * H * B * N), dim3(64 * nw), 0, st, p, blocks)
   HDS_EVO_ALL(HDS_EVO)
@@ -553,18 +724,21 @@ HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, co
   p.q = (const bf16*)q; p.k = (const bf16*)k; p.v = (const bf16*)v; p.o = (const bf16*)o; p.dout = (const bf16*)dout;
   p.b1 = b1; p.b2 = b2; p.dq = (bf16*)dq; p.dk = (bf16*)dk; p.dv = (bf16*)dv; p.lse = (float*)lse; p.delta = delta;
   p.db1 = db1; p.part = part; p.B = B; p.N = N; p.L = L; p.H = H; p.scale = scale;
-  const int nw = waves_of(L), blocks = (L + 32 * nw - 1) / (32 * nw);
+  const int nw = waves_of(L, D == 128 ? kWaves<128> : kWaves<32>), blocks = (L + 32 * nw - 1) / (32 * nw);
   const dim3 grid(blocks * H * B * N), threads(64 * nw);
 #define HDS_EVO(DD, TT)                                                                                             \
   do {                                                                                                              \
     hipLaunchKernelGGL((evo_dq_kernel<DD, TT>), grid, threads, 0, st, p, blocks);                                   \
-    hipLaunchKernelGGL((evo_dkdv_kernel<DD, TT>), grid, threads, 0, st, p, blocks);                                 \
+    if (db1 != nullptr)                                                                                             \
+      hipLaunchKernelGGL((evo_dkdv_kernel<DD, TT, true>), grid, threads, 0, st, p, blocks);                         \
+    else                                                                                                            \
+      hipLaunchKernelGGL((evo_dkdv_kernel<DD, TT, false>), grid, threads, 0, st, p, blocks);                        \
   } while (0)
   HDS_EVO_ALL(HDS_EVO)
 #undef HDS_EVO
   if (db2 != nullptr) {
     const int chunks = hds_evoformer_pair_chunks(B, N, L, H), per = (N + chunks - 1) / chunks;
-    const int tiles = (L + 31) / 32, w4 = (tiles + (tiles + 3) / 4 - 1) / ((tiles + 3) / 4), qblocks = (L + 32 * w4 - 1) / (32 * w4);
+    const int w4 = waves_of(L, 4), qblocks = (L + 32 * w4 - 1) / (32 * w4);
     const int kblocks = (L + 32 * kPairTiles - 1) / (32 * kPairTiles);
     const int64_t n = (int64_t)B * H * L * L, grid2 = (int64_t)chunks * B * H * kblocks * qblocks;
     if (grid2 > 0x7fffffff || (n + 1023) / 1024 > 0x7fffffff) return hipErrorInvalidValue;
