@@ -222,6 +222,139 @@ __global__ __launch_bounds__(256) void wmix_reduce_kernel(const float* __restric
   *reinterpret_cast<bf16x4*>(C + i) = o;
 }
 
+// ---------------------------------------------------------------------------------------------------------------
+// Few rows (decode): a stream of packed weights
+// ---------------------------------------------------------------------------------------------------------------
+// A workgroup owns 16 NT weight rows, its NW waves take runs of 512 k in turn. In a run a lane holds 32 consecutive k
+// of a weight row for each of four chunks of 128 (24 bytes fp6, 32 int8, 16 int4: all loads of the run are in flight
+// together), and mfma_f32_16x16x32_bf16 contracts elements 8 j .. 8 j + 7 of the four lane groups with the same k of up
+// to 16 MT rows of A. The operand is the weight's CODE, which bf16 holds exactly; the group's scale multiplies the 32-bit
+// sum of each group (every chunk lies in one group), so no weight is rounded. fp6 codes become bf16 in one instruction
+// for 32 of them. Measured at 8 rows, [28672, 4096] / [4096, 14336]: fp6 38 / 22 us (92 / 46 MB; the GEMV that decodes and
+// multiplies on the VALU 112 / 77), int8 39 / 20 us (121 / 61 MB; the tile kernel above 45 / 28), int4 29 / 16 us (41 /
+// 29). A third of the time at 8 rows goes to reading A again from L2 in every workgroup.
+typedef uint32_t u32x6 __attribute__((ext_vector_type(6)));
+typedef __bf16 bf16x32 __attribute__((ext_vector_type(32)));
+
+template <int FMT, int E>
+__device__ __forceinline__ void codes(const WRaw<FMT>& r, bf16x8 (&f)[4]) {
+  if constexpr (FMT == kFp6) {
+    const u32x6 q = {r.a.x, r.a.y, r.b.x, r.b.y, r.c.x, r.c.y};
+    bf16x32 v;
+    if constexpr (E == 3) v = __builtin_amdgcn_cvt_scalef32_pk32_bf16_bf6(q, 1.f);  // "bf6" is e3m2
+    else v = __builtin_amdgcn_cvt_scalef32_pk32_bf16_fp6(q, 1.f);
+    f[0] = __builtin_shufflevector(v, v, 0, 1, 2, 3, 4, 5, 6, 7);
+    f[1] = __builtin_shufflevector(v, v, 8, 9, 10, 11, 12, 13, 14, 15);
+    f[2] = __builtin_shufflevector(v, v, 16, 17, 18, 19, 20, 21, 22, 23);
+    f[3] = __builtin_shufflevector(v, v, 24, 25, 26, 27, 28, 29, 30, 31);
+  } else if constexpr (FMT == kInt8) {
+    const uint32_t dw[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t u = dw[i] ^ 0x80808080u;  // unsigned bytes, 128 too large
+#pragma unroll
+      for (int t = 0; t < 4; ++t) f[i >> 1][4 * (i & 1) + t] = (bf16)((float)((u >> (8 * t)) & 0xff) - 128.f);
+    }
+  } else {
+    const uint32_t dw[4] = {r.a.x, r.a.y, r.a.z, r.a.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t lo = (dw[i] & 0x0f0f0f0fu) ^ 0x08080808u, hi = ((dw[i] >> 4) & 0x0f0f0f0fu) ^ 0x08080808u;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        f[i][2 * t] = (bf16)((float)((lo >> (8 * t)) & 0xff) - 8.f);
+        f[i][2 * t + 1] = (bf16)((float)((hi >> (8 * t)) & 0xff) - 8.f);
+      }
+    }
+  }
+}
+
+// MW: waves a SIMD that the registers have to leave room for
+template <int FMT, int E, int NT, int MT, int NW, int MW>
+__global__ __launch_bounds__(64 * NW, MW) void wmix_skinny_kernel(const bf16* __restrict__ A,
+                                                                  const uint8_t* __restrict__ W,
+                                                                  const float* __restrict__ scales,
+                                                                  const bf16* __restrict__ bias, bf16* __restrict__ C,
+                                                                  int M, int N, int K, int G) {
+  __shared__ f32x4 red[NW - 1][NT][MT][64];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * 16 * NT, groups = K / G;
+  f32x4 acc[NT][MT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{};
+  const bf16* xp[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) xp[m] = A + (int64_t)min(16 * m + r, M - 1) * K + 32 * g;
+
+  for (int run = wid; run * 512 < K; run += NW) {
+    WRaw<FMT> raw[4][NT];
+    f32x4 sc[NT][4];  // of the lane's four sums, chunks 0 .. 3
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int k = min(512 * run + 128 * c, K - 128);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) raw[c][t] = load_w<FMT>(W, min(n0 + 16 * t + r, N - 1), K, k + 32 * g);
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float* s = scales + (int64_t)min(n0 + 16 * t + 4 * g + i, N - 1) * groups;
+        if (G == 128 && groups % 4 == 0) {
+          sc[t][i] = *reinterpret_cast<const f32x4*>(s + 4 * run);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) sc[t][i][c] = s[min(512 * run + 128 * c, K - 128) / G];
+        }
+      }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int k = 512 * run + 128 * c;
+      if (k >= K) break;  // wave-uniform
+      bf16x8 x[MT][4];
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[m][j] = *reinterpret_cast<const bf16x8*>(xp[m] + k + 8 * j);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        bf16x8 f[4];
+        codes<FMT, E>(raw[c][t], f);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          f32x4 s{};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[j], x[m][j], s, 0, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[t][m][i] += s[i] * sc[t][i][c];
+        }
+      }
+    }
+  }
+  if (wid > 0) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) red[wid - 1][t][m][lane] = acc[t][m];
+  }
+  __syncthreads();
+  if (wid > 0) return;
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+#pragma unroll
+      for (int v = 0; v < NW - 1; ++v) acc[t][m] += red[v][t][m][lane];
+      const int row = 16 * m + r, n = n0 + 16 * t + 4 * g;
+      if (row >= M) continue;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (n + i < N) C[(int64_t)row * N + n + i] = (bf16)(acc[t][m][i] + (bias ? (float)bias[n + i] : 0.f));
+    }
+}
+
 int pick_mb(int M) { return M <= 32 ? 1 : 2; }
 // weight fragments per wave: 1 at small M (more workgroups in flight for the weight stream), 4 once the A chunk
 // re-reads and the per-fragment MFMA chain matter (measured, profiles/wmix_bench_r2.log)
@@ -279,5 +412,34 @@ HDS_EXPORT int hds_wmix_gemm(const void* A, const void* W, const float* scales, 
   const int64_t MN = (int64_t)M * N;
   hipLaunchKernelGGL(wmix_reduce_kernel, dim3((unsigned)((MN / 4 + 255) / 256)), dim3(256), 0, st, ws,
                      (const bf16*)bias, (bf16*)C, M, N, splits);
+  return hipGetLastError();
+}
+
+// The same product for few rows as a stream of packed weights (wmix_skinny_kernel): 1 <= M <= 16, fp6 up to 32. K and G
+// multiples of 128, A 16-byte aligned.
+HDS_EXPORT int hds_wmix_skinny(const void* A, const void* W, const float* scales, const void* bias, void* C, int M, int N,
+                               int K, int G, int fmt, int ebits, hipStream_t st) {
+  if (M < 1 || M > (fmt == 2 ? 32 : 16) || N < 1 || K < 128 || K % 128 || G < 128 || G % 128 || K % G)
+    return hipErrorInvalidValue;
+  auto launch = [&](auto kern, int rows, int waves) {
+    hipLaunchKernelGGL(kern, dim3((N + rows - 1) / rows), dim3(64 * waves), 0, st, (const bf16*)A, (const uint8_t*)W,
+                       scales, (const bf16*)bias, (bf16*)C, M, N, K, G);
+  };
+  // From nine rows on two tiles of weight rows share what is read of A ([28672, 4096], 16 rows: fp6 48 -> 41 us), where
+  // enough workgroups remain. Short sums on many rows: four waves a workgroup (fp6, 8 rows 40 -> 38 us), otherwise eight
+  // ([4096, 14336] 27 -> 22 us).
+#define HDS_WS(F, E)                                                                                       \
+  do {                                                                                                     \
+    if (M > 8 && M <= 16 && N >= 32 * 512) launch(wmix_skinny_kernel<F, E, 2, 1, 4, 3>, 32, 4);            \
+    else if (M <= 16 && K <= 4096 && N >= 16 * 384) launch(wmix_skinny_kernel<F, E, 1, 1, 4, 1>, 16, 4);   \
+    else if (M <= 16) launch(wmix_skinny_kernel<F, E, 1, 1, 8, 1>, 16, 8);                                 \
+    else if constexpr (F == kFp6) launch(wmix_skinny_kernel<F, E, 1, 2, 8, 1>, 16, 8);                     \
+  } while (0)
+  if (fmt == 0) HDS_WS(kInt8, 0);
+  else if (fmt == 1) HDS_WS(kInt4, 0);
+  else if (fmt == 2 && ebits == 3) HDS_WS(kFp6, 3);
+  else if (fmt == 2 && ebits == 2) HDS_WS(kFp6, 2);
+  else return hipErrorInvalidValue;
+#undef HDS_WS
   return hipGetLastError();
 }

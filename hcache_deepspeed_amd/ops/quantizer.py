@@ -170,15 +170,39 @@ def wmix_gemm(x2, q_weight, scales, out_features, in_features, group_size, fmt, 
     return y
 
 
+def _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, fmt, ebits=3, bias=None):
+    """The packed-weight stream for few rows (csrc/kernels/wmix_gemm.hip ``wmix_skinny_kernel``), or None where it does not
+    apply. It wins up to 16 rows, with fp6 up to 32 ([28672, 4096], 24 rows: fp6 57 us against the tile kernel's 78, int8
+    61 against 50), with int8 from the second row on (one row: 36.5 us against the GEMV's 34.7, two 36.5 against 39)."""
+    M = x2.shape[0]
+    if (_needs_grad(x2) or not native.use_native(x2) or x2.dtype != torch.bfloat16 or in_features % 128
+            or group_size % 128 or not (fmt == "int8") < M <= (32 if fmt == "fp6" else 16)):
+        return None
+    x2 = x2.contiguous()
+    if x2.data_ptr() % 16:
+        return None
+    if bias is not None:
+        bias = bias.to(torch.bfloat16).contiguous()
+    y = torch.empty(M, out_features, dtype=torch.bfloat16, device=x2.device)
+    native.check(native.kernels().hds_wmix_skinny(x2.data_ptr(), q_weight.data_ptr(), scales.data_ptr(),
+                                                  native.ptr(bias), y.data_ptr(), M, out_features, in_features,
+                                                  group_size, {"int8": 0, "int4": 1, "fp6": 2}[fmt], int(ebits),
+                                                  native.stream()), "wmix_skinny")
+    return y
+
+
 def int_linear(x, q_weight, scales, out_features, in_features, group_size, bits=8, bias=None):
     """y = x @ dequant(W)^T for a symmetric group-quantized int8/int4 weight [out, in] (groups along ``in``).
 
-    Decode-sized inputs (<= 2 rows by default, ``HDS_INT_GEMV_MAX_M``) run the fused HIP GEMV (csrc/kernels/quant.hip
-    ``int_gemv_kernel``) that reads the packed weight straight from HBM (1.5-2.3x faster than the bf16 GEMM at one
-    row, profiles/int_gemv_bench_r1.log); larger batches dequantize once to bf16 and use the matrix cores."""
+    Up to 16 rows stream the packed weight through the matrix cores (``_wmix_skinny``, groups of a multiple of 128; one row
+    of int8 and other groups up to 2 rows, ``HDS_INT_GEMV_MAX_M``: the HIP GEMV of csrc/kernels/quant.hip); batches of up to 64 rows run the
+    tile kernel on packed weights, larger ones dequantize once to bf16."""
     lead = x.shape[:-1]
     x2 = x.reshape(-1, in_features)
     M = x2.shape[0]
+    y = _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, f"int{bits}", bias=bias)
+    if y is not None:
+        return y.view(*lead, out_features)
     if not _needs_grad(x2) and native.use_native(x2) and 0 < M <= _INT_GEMV_MAX_M and x2.dtype == torch.bfloat16 and in_features % 16 == 0 \
             and group_size % 16 == 0:
         x2 = x2.contiguous()
@@ -420,11 +444,15 @@ def dequantize_minifloat(q, scales, group_size=512, q_bits=6, mantissa_bits=2, d
 def fp6_linear(x, q_weight, scales, out_features, in_features, group_size, mantissa_bits=2):
     """y = x @ dequant(W)^T for an FP6-packed weight [out, in] (row-major, groups along ``in``).
 
-    Decode-sized inputs (<= 8 rows) run the fused HIP GEMV that reads 6-bit weights straight from HBM; larger
-    batches dequantize the weight once to bf16 and use the matrix cores (hipBLASLt)."""
+    Up to 32 rows stream the packed weight through the matrix cores (``_wmix_skinny``, groups of a multiple of 128; other
+    groups: the HIP GEMV of csrc/kernels/fpq.hip up to 8 rows); batches of up to 64 rows run the tile kernel on packed
+    weights, larger ones dequantize once to bf16 and use hipBLASLt."""
     lead = x.shape[:-1]
     x2 = x.reshape(-1, in_features)
     M = x2.shape[0]
+    y = _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, "fp6", 5 - mantissa_bits)
+    if y is not None:
+        return y.view(*lead, out_features)
     if not _needs_grad(x2) and native.use_native(x2) and M <= 8 and x2.dtype == torch.bfloat16 \
             and in_features % 16 == 0 \
             and group_size % 16 == 0:

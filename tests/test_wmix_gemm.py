@@ -54,3 +54,32 @@ def test_wmix_split_k_deterministic():
     assert torch.equal(a, b)
     ref = x.float() @ Q.dequantize(q, s, None, 128, 8, True, torch.float32).view(512, 14336).t()
     assert (a.float() - ref).abs().max().item() <= 1e-2 * ref.abs().max().item()
+
+
+@pytest.mark.parametrize("fmt", ["int8", "int4", "fp6_e3m2", "fp6_e2m3"])
+@pytest.mark.parametrize("M,N,K,G", [(1, 16, 128, 128), (8, 1000, 640, 128), (9, 16390, 512, 256), (16, 6160, 4224, 128),
+                                     (17, 250, 1024, 1024), (32, 48, 14336, 128), (5, 40, 1024, 64)])
+def test_few_rows_keep_the_weights_exact(fmt, M, N, K, G):
+    """The stream of packed weights: tails of the rows and of the 512-wide runs, one and two tiles of weight rows, four and
+    eight waves, scales read by four and one by one; groups of 64 take the older kernels. The codes are exact and the
+    scales 32-bit, so what is left are 32-bit sums (K terms) and the result's rounding."""
+    torch.manual_seed(K + M)
+    x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(N, K, device="cuda", dtype=torch.bfloat16) * 0.05
+    if fmt.startswith("int"):
+        bits = int(fmt[3:])
+        q, s, _ = Q.quantize(w.reshape(-1), G, bits, True)
+        wd = Q.dequantize(q, s, None, G, bits, True, torch.float32).view(N, K).double()
+        bias = torch.randn(N, device="cuda", dtype=torch.bfloat16)
+        y = Q.int_linear(x, q, s, N, K, G, bits=bits, bias=bias)
+        ref = x.double() @ wd.t() + bias.double()
+        stream = G % 128 == 0 and (bits == 8) < M <= 16
+    else:
+        mb = 2 if fmt.endswith("e3m2") else 3
+        q, s = Q.quantize_minifloat(w.reshape(-1), G, 6, mb)
+        wd = Q.dequantize_minifloat(q, s, G, 6, mb, torch.float32).view(N, K).double()
+        y = Q.fp6_linear(x, q, s, N, K, G, mb)
+        ref = x.double() @ wd.t()
+        stream = G % 128 == 0
+    bound = 2**-8 * ref.abs() + 1e-5 * (x.double().abs() @ wd.abs().t()) if stream else 0.02 * ref.abs().max()
+    assert ((y.double() - ref).abs() <= bound).all()
