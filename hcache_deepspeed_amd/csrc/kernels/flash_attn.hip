@@ -34,6 +34,7 @@ using namespace hds;
 using namespace hds::attn;
 
 // variant 9 lives in its own translation unit (flash_attn_w64.hip: built with the VGPR-form MFMA selection)
+int hds_attn_fwd_w64_paged_launch(const void* params, size_t params_bytes, int n, int hq, hipStream_t st);
 int hds_attn_fwd_w64_launch(const void* params, size_t params_bytes, int batch, int max_len, int hq, int mode,
                             hipStream_t st);
 // one-wave-per-SIMD dQ (flash_attn_bwd_w64.hip)
@@ -1345,7 +1346,7 @@ AttnParams make_params(const void* q, const void* k, const void* v, void* o, flo
                        void* dk, void* dv, float* delta, const int64_t* strides, const int* cu_seqlens,
                        const int* seq_lens, int batch, int seq_len, int total_tokens, int hq, int hkv, float scale,
                        int causal, int window) {
-  AttnParams p;
+  AttnParams p{};
   p.q = (const bf16*)q;
   p.k = (const bf16*)k;
   p.v = (const bf16*)v;
@@ -1584,4 +1585,26 @@ HDS_EXPORT int hds_attn_bwd(const void* q, const void* k, const void* v, const v
   HDS_ATTN_DIMS(HDS_CASE)
 #undef HDS_CASE
   return hipErrorInvalidValue;
+}
+
+// Causal attention of new tokens over the paged cache [blocks, block_size, 2, hkv, 128], head size 128, bf16. blocks: device
+// int32 [n_blocks][2], sequence and first of 256 new tokens; seq_meta: device int32 [sequences][3], first row of q, new
+// tokens, earlier tokens. q and o: [tokens, hq, 128] with token strides sq, so. block_size % 64 == 0, less than 2^31 slots.
+HDS_EXPORT int hds_paged_prefill(const void* q, int64_t sq, const void* cache, void* o, int64_t so, const int* blocks,
+                                 int n_blocks, const int* seq_meta, const int* block_tables, int max_blocks,
+                                 int block_size, int hq, int hkv, float scale, int window, hipStream_t st) {
+  if (n_blocks <= 0) return 0;
+  if (hq < 1 || hkv < 1 || hq % hkv || sq % 8 || so % 8 || block_size < 64 || block_size % 64 || max_blocks < 1 ||
+      window < 0 || (int64_t)n_blocks * hq > 0x7fffffff || (int64_t)64 * 2 * hkv * 128 * 2 > 0x7fffffff)
+    return hipErrorInvalidValue;
+  const int64_t slot = (int64_t)2 * hkv * 128;
+  const int64_t strides[8] = {sq, slot, slot, so, 0, 0, 0, 0};
+  AttnParams p = make_params(q, cache, (const bf16*)cache + (int64_t)hkv * 128, o, nullptr, nullptr, nullptr, nullptr,
+                             nullptr, nullptr, strides, nullptr, nullptr, 0, 0, 0, hq, hkv, scale, 1, window);
+  p.blocks = blocks;
+  p.meta = seq_meta;
+  p.tables = block_tables;
+  p.max_blocks = max_blocks;
+  p.block_size = block_size;
+  return hds_attn_fwd_w64_paged_launch(&p, sizeof(p), n_blocks, hq, st);
 }

@@ -42,6 +42,11 @@ struct AttnParams {
   float scale;
   int causal;
   int window;  // >0: sliding window (keys in (q - window, q])
+  // paged forward: [n][2] sequence, first new token; [sequences][3] first row, new tokens, earlier tokens; block tables
+  const int* blocks;
+  const int* meta;
+  const int* tables;
+  int max_blocks, block_size;
 };
 
 __device__ __forceinline__ void seq_bounds(const AttnParams& p, int b, int& start, int& len) {

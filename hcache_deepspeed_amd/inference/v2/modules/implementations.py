@@ -29,7 +29,7 @@ from ....ops.norm import layer_norm, rms_norm
 from ....ops.output_norm import (PairSum, embed_rows, padded, residual_norm, rms_rows, sandwich_norm, softcap_,
                                  stream_norm, sum_experts)
 from ....ops.paged import (HeadShape, head_attention, head_blocks_ok, kv_rope_scatter, make_head_plan,
-                           paged_attention)
+                           paged_attention, paged_attention_portions, portions_ok)
 from ....ops.quantizer import fp6_linear, int_linear, quantize, quantize_minifloat
 from ....ops.rope import rope_tables
 from .interfaces import (DSEmbeddingBase, DSEmbeddingRegistry, DSExpertLayerBase, DSExpertLayerRegistry, DSGatedMLPBase,
@@ -73,6 +73,10 @@ class DSDenseBlockedAttention(DSSelfAttentionBase):
         nq, nkv, D = c.n_heads_q, c.n_heads_kv, c.head_size
         kv_rope_scatter(qkv, cache, batch.tok_seq, batch.tok_pos, batch.block_tables, cos, sin, nq, nkv,
                         do_rope=c.positional_embedding_type != "none" and cos is not None, rotary_dim=c.rotary_dim)
+        portions = getattr(batch, "portions", None)
+        if portions is not None and portions_ok(qkv[:, :nq], cache, nq, nkv):
+            return paged_attention_portions(qkv[:, :nq], cache, *portions, batch, nq, nkv, c.scale_factor,
+                                            c.sliding_window).reshape(T, nq * D)
         o = paged_attention(qkv[:, :nq], cache, batch.atoms, batch.n_atoms, batch.seq_meta, batch.block_tables, nq,
                             nkv, c.scale_factor, c.sliding_window, batch.seq_meta_host, batch.tables_host,
                             decode=T == batch.current_sequences)

@@ -311,6 +311,7 @@ class RaggedBatchWrapper:
         import ctypes
         import numpy as np
         from ...ops import native
+        from ...ops.paged import make_portions
         S, T = len(self._seqs), self.current_tokens
         mb = self.max_blocks
         n_new = np.fromiter((nn for (_, nn, _) in self.seq_meta_host), dtype=np.int32, count=S)
@@ -326,8 +327,11 @@ class RaggedBatchWrapper:
         need = ctypes.c_int64(0)
         lib.hds_ragged_meta_build(P(n_new), P(seen), S, P(flat), P(off), mb, n_q, n_kv, rpa, None, 0,
                                   ctypes.byref(need))
-        # after the builder's part: the sequences' state slots, then explicit logits rows
-        extra = [seq.tracking_id for seq in self._seqs] + (self._logit_rows or [])
+        # after the builder's part: the sequences' state slots, explicit logits rows, the division of a step that is not
+        # single tokens only
+        mixed = any(nn != 1 for (_, nn, _) in self.seq_meta_host)
+        toks, blocks = make_portions(self.seq_meta_host) if mixed else ([], [])
+        extra = [seq.tracking_id for seq in self._seqs] + (self._logit_rows or []) + blocks + toks
         si, host = self._pinned_slot(int(need.value) + len(extra))
         A = lib.hds_ragged_meta_build(P(n_new), P(seen), S, P(flat), P(off), mb, n_q, n_kv, rpa,
                                       ctypes.c_void_p(host.data_ptr()), host.numel(), ctypes.byref(need))
@@ -372,6 +376,10 @@ class RaggedBatchWrapper:
         self.carry = {}
         if self._logit_rows is not None:
             self.last_token_idx = take(len(self._logit_rows), (-1, ))
+        self.portions = None
+        if mixed:
+            blocks = take(len(blocks), (-1, 2)) if blocks else None
+            self.portions = (take(len(toks), (-1, )) if toks else None, blocks)
         self.tables_host = host[4 * S + 2 * T:4 * S + 2 * T + S * mb].view(S, mb).clone() if S else \
             torch.zeros(1, mb, dtype=torch.int32)
         if S == 0:  # keep 1-row shapes for empty batches (kernels never run on them)

@@ -119,6 +119,7 @@ _KERNEL_SIGS = {
     "hds_skinny_set_unroll": "i",
     "hds_wmix_splits": "iii",
     "hds_wmix_supported": "iiii",
+    "hds_paged_prefill": "pl" + "p" + "pl" + "pi" + "pp" + "iiii" + "f" + "i" + "s",
     "hds_wmix_skinny": "ppppp" + "iiiiii" + "s",
     "hds_wmix_gemm": "pppppp" + "iiiiii" + "s",
     "hds_token_gather": "i" + "ppp" + "iiii" + "s",

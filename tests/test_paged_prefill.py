@@ -1,0 +1,110 @@
+"""Attention of steps that mix single tokens and portions of prompts over the paged cache: the prefill kernel
+(csrc/kernels/flash_attn_w64.hip over block tables) and the division of a step, against float64 over the same tables."""
+import math
+import types
+
+import pytest
+import torch
+
+from hcache_deepspeed_amd.ops.paged import DECODE_MAX, make_portions, paged_attention_portions, portions_ok
+
+D = 128
+
+
+def test_portions_cover_every_token_once():
+    metas, q0 = [], 0
+    for n, seen in [(1, 50), (700, 0), (DECODE_MAX, 9), (DECODE_MAX + 1, 1000), (0, 3), (256, 7), (257, 0)]:
+        metas.append((q0, n, seen))
+        q0 += n
+    toks, flat = make_portions(metas)
+    blocks = list(zip(flat[::2], flat[1::2]))
+    rows = set(toks)
+    for s, r in blocks:
+        own = range(metas[s][0] + r, metas[s][0] + min(r + 256, metas[s][1]))
+        assert len(own) and not rows & set(own)
+        rows |= set(own)
+    assert rows == set(range(q0)) and len(toks) == 1 + DECODE_MAX
+    last = [metas[s][2] + min(r + 256, metas[s][1]) for s, r in blocks]
+    assert last == sorted(last, reverse=True)
+
+
+def _setup(lens, seen, hkv, bs, device, g):
+    need = [-(-(n + s) // bs) for n, s in zip(lens, seen)]
+    width = max(need) + 1
+    perm = torch.randperm(sum(need) + 3, generator=g)
+    tab = torch.zeros(len(lens), width, dtype=torch.int32)
+    k = 0
+    for i, m in enumerate(need):
+        tab[i, :m] = perm[k:k + m].int()
+        k += m
+    cache = torch.randn(sum(need) + 3, bs, 2, hkv, D, generator=g).bfloat16().to(device)
+    metas, q0 = [], 0
+    for n, s in zip(lens, seen):
+        metas.append((q0, n, s))
+        q0 += n
+    seq = torch.tensor([i for i, n in enumerate(lens) for _ in range(n)], dtype=torch.int32)
+    pos = torch.tensor([s + j for n, s in zip(lens, seen) for j in range(n)], dtype=torch.int32)
+    batch = types.SimpleNamespace(seq_meta=torch.tensor(metas, dtype=torch.int32).to(device), tok_seq=seq.to(device),
+                                  tok_pos=pos.to(device), block_tables=tab.to(device))
+    return cache, tab, metas, q0, batch
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,seen,hq,hkv,bs,window", [
+    ([9], [0], 8, 2, 64, 0), ([64, 1, 65], [0, 700, 63], 16, 4, 64, 0), ([256, 8, 257], [1, 130, 64], 4, 4, 128, 0),
+    ([300, 1, 1], [5000, 4500, 3], 8, 1, 64, 0), ([1100], [0], 6, 2, 192, 0), ([513, 20], [100, 900], 32, 8, 64, 200),
+    ([40], [4090], 8, 8, 64, 64), ([2, 3], [500, 17], 8, 2, 64, 0), ([4400], [0], 2, 1, 64, 0)])
+def test_portions_match_float64(lens, seen, hq, hkv, bs, window):
+    """Tails of the 64-key tiles and of the 256-token workgroups, a portion behind a long context (more than 64 tiles, the
+    run of cache slots that a wave holds at a time), windows, blocks of several tiles, head counts that are no multiple of
+    8. p is rounded to bf16 against a 32-bit sum and the result to bf16: 2^-8 of the norm twice, with room for two more."""
+    g = torch.Generator().manual_seed(sum(lens) + hq)
+    dev = torch.device("cuda")
+    cache, tab, metas, T, batch = _setup(lens, seen, hkv, bs, dev, g)
+    qkv = torch.randn(T, hq + 2 * hkv, D, generator=g).bfloat16().to(dev)
+    q = qkv[:, :hq]
+    assert portions_ok(q, cache, hq, hkv)
+    toks, blocks = make_portions(metas)
+    toks = torch.tensor(toks, dtype=torch.int32, device=dev) if toks else None
+    blocks = torch.tensor(blocks, dtype=torch.int32, device=dev).view(-1, 2) if blocks else None
+    scale = 1 / math.sqrt(D)
+    o = paged_attention_portions(q, cache, toks, blocks, batch, hq, hkv, scale, window)
+    for i, (q0, n, s) in enumerate(metas):
+        at = torch.arange(s + n)
+        rows = cache[tab[i, at // bs].long().to(dev), (at % bs).to(dev)].double()
+        k, v = (rows[:, j].repeat_interleave(hq // hkv, 1).transpose(0, 1) for j in (0, 1))
+        sc = q[q0:q0 + n].double().transpose(0, 1) @ k.transpose(1, 2) * scale
+        mine = (s + torch.arange(n))[:, None]
+        hide = at[None] > mine
+        if window:
+            hide |= at[None] <= mine - window
+        want = (torch.softmax(sc.masked_fill(hide.to(dev), float("-inf")), -1) @ v).transpose(0, 1)
+        got = o[q0:q0 + n].double()
+        assert (got - want).norm() <= 4 * 2**-8 * want.norm(), i
+        worst = (got - want).norm(dim=-1) / want.norm(dim=-1)  # no single row off either
+        assert worst.max() < 0.03, (i, worst.max())
+
+
+@pytest.mark.gpu
+def test_engine_steps_in_pieces_match_whole_prompts():
+    """A prompt taken in pieces beside decoding sequences gives the logits of the prompt taken whole."""
+    from hcache_deepspeed_amd.inference.v2.engine import build_engine_from_model
+    from hcache_deepspeed_amd.models.llama import LlamaForCausalLM, tiny
+    torch.manual_seed(0)
+    m = LlamaForCausalLM(tiny(vocab_size=211)).eval()
+    conf = dict(dtype="bf16", state_manager={"max_context": 1024, "kv_block_size": 64, "max_ragged_batch_size": 1024})
+    g = torch.Generator().manual_seed(3)
+    prompt, other = (torch.randint(0, 211, (n, ), generator=g) for n in (700, 90))
+    step = [torch.randint(0, 211, (1, ), generator=g) for _ in range(3)]
+    dev = torch.device("cuda")
+    eng = build_engine_from_model(m, conf, device=dev, num_kv_blocks=40)
+    eng.put([1], [other], capture_latents=False)
+    got = [eng.put([1, 2], [t, p], capture_latents=False)[0].float() for t, p in zip(step, prompt.split(256))]
+    ref = build_engine_from_model(m, conf, device=dev, num_kv_blocks=40)
+    ref.put([1], [other], capture_latents=False)
+    for i, t in enumerate(step):
+        a = ref.put([1], [t], capture_latents=False)[0].float()
+        b = ref.put([2], [prompt[:256 * (i + 1)]], capture_latents=False)[0].float()
+        ref.flush(2)
+        want = torch.cat([a, b])
+        assert (got[i] - want).norm() < 2e-2 * want.norm()
