@@ -27,17 +27,34 @@ constexpr int kRowsPerBlock = 4;  // 4 waves per block, one row each per iterati
 // ---------------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------------
+// pick (may be null): output row i is made from rows pick[i] of x and res, of which there are n_in; negative ones count from
+// the end, and a row outside them gives NaN. A serving step normalises only the rows whose logits are wanted: gathering
+// them first took four launches (two index conversions, two gathers; 18 us of a 490 us decode step of 16 sequences).
+struct PickedRow {
+  int row;
+  bool ok;
+};
+__device__ __forceinline__ PickedRow picked_row(const int* pick, int row, int n_in) {
+  if (pick == nullptr) return {row, true};
+  int r = pick[row];
+  if (r < 0) r += n_in;
+  const bool ok = r >= 0 && r < n_in;
+  return {ok ? r : 0, ok};
+}
+
 template <typename T, typename WT, int NV, bool LN>
 __global__ __launch_bounds__(256) void norm_fwd_kernel(const T* __restrict__ x, const T* __restrict__ res,
                                                        T* __restrict__ res_out, const WT* __restrict__ w,
                                                        const WT* __restrict__ b, T* __restrict__ y,
                                                        float* __restrict__ stat_mean, float* __restrict__ stat_rstd,
-                                                       int rows, int cols, float eps) {
+                                                       int rows, int cols, float eps, const int* __restrict__ pick,
+                                                       int n_in) {
   const int lane = threadIdx.x & 63;
   const int wid = threadIdx.x >> 6;
   const int row = blockIdx.x * kRowsPerBlock + wid;
   if (row >= rows) return;
-  const T* xr = x + (int64_t)row * cols;
+  const PickedRow in = picked_row(pick, row, n_in);
+  const T* xr = x + (int64_t)in.row * cols;
   float v[NV][8];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -45,7 +62,7 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const T* __restrict__ x, 
     Vec8<T>::load(xr + c, v[i]);
   }
   if (res != nullptr) {
-    const T* rr = res + (int64_t)row * cols;
+    const T* rr = res + (int64_t)in.row * cols;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int c = (i * 64 + lane) * 8;
@@ -77,7 +94,7 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const T* __restrict__ x, 
       const float d = v[i][j] - mean;
       ss += d * d;
     }
-  const float rstd = rsqrtf(wave_sum(ss) / (float)cols + eps);
+  const float rstd = in.ok ? rsqrtf(wave_sum(ss) / (float)cols + eps) : NAN;
   T* yr = y + (int64_t)row * cols;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -107,12 +124,14 @@ __global__ __launch_bounds__(256) void norm_fwd_generic(const T* __restrict__ x,
                                                         T* __restrict__ res_out, const WT* __restrict__ w,
                                                         const WT* __restrict__ b, T* __restrict__ y,
                                                         float* __restrict__ stat_mean, float* __restrict__ stat_rstd,
-                                                        int rows, int cols, float eps) {
+                                                        int rows, int cols, float eps, const int* __restrict__ pick,
+                                                        int n_in) {
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
   if (row >= rows) return;
-  const T* xr = x + (int64_t)row * cols;
-  const T* rr = res ? res + (int64_t)row * cols : nullptr;
+  const PickedRow in = picked_row(pick, row, n_in);
+  const T* xr = x + (int64_t)in.row * cols;
+  const T* rr = res ? res + (int64_t)in.row * cols : nullptr;
   T* ro = res_out ? res_out + (int64_t)row * cols : nullptr;
   float s = 0.f, ss = 0.f;
   for (int c = lane * 8; c < cols; c += 512) {
@@ -135,7 +154,7 @@ __global__ __launch_bounds__(256) void norm_fwd_generic(const T* __restrict__ x,
   ss = wave_sum(ss);
   const float mean = LN ? s / cols : 0.f;
   const float var = LN ? fmaxf(ss / cols - mean * mean, 0.f) : ss / cols;
-  const float rstd = rsqrtf(var + eps);
+  const float rstd = in.ok ? rsqrtf(var + eps) : NAN;
   T* yr = y + (int64_t)row * cols;
   for (int c = lane * 8; c < cols; c += 512) {
     float v[8], wv[8], o[8];
@@ -334,11 +353,12 @@ __global__ __launch_bounds__(256) void reduce_parts_kernel(const float* __restri
 
 template <typename T, typename WT, bool LN>
 hipError_t launch_fwd(const void* x, const void* res, void* res_out, const void* w, const void* b, void* y,
-                      float* mean, float* rstd, int rows, int cols, float eps, hipStream_t st) {
+                      float* mean, float* rstd, int rows, int cols, float eps, const int* pick, int n_in,
+                      hipStream_t st) {
   dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock), block(256);
   auto args = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, block, 0, st, (const T*)x, (const T*)res, (T*)res_out, (const WT*)w,
-                       (const WT*)b, (T*)y, mean, rstd, rows, cols, eps);
+                       (const WT*)b, (T*)y, mean, rstd, rows, cols, eps, pick, n_in);
   };
   switch (cols) {
     case 512: args(norm_fwd_kernel<T, WT, 1, LN>); break;
@@ -395,10 +415,11 @@ hipError_t launch_bwd(const void* dy, const void* h, const void* dres, const voi
 
 HDS_EXPORT int hds_norm_fwd(int is_ln, int dtype, int wdtype, const void* x, const void* res, void* res_out,
                             const void* w, const void* b, void* y, float* mean, float* rstd, int rows, int cols,
-                            float eps, hipStream_t st) {
-  if (cols % 8) return hipErrorInvalidValue;
-  if (is_ln) HDS_DISPATCH2(dtype, wdtype, true, launch_fwd, x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, st);
-  HDS_DISPATCH2(dtype, wdtype, false, launch_fwd, x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, st);
+                            float eps, const int* pick, int n_in, hipStream_t st) {
+  if (cols % 8 || (pick != nullptr && n_in < 1)) return hipErrorInvalidValue;
+  if (is_ln)
+    HDS_DISPATCH2(dtype, wdtype, true, launch_fwd, x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, pick, n_in, st);
+  HDS_DISPATCH2(dtype, wdtype, false, launch_fwd, x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, pick, n_in, st);
 }
 
 static int g_norm_bwd_max_parts = 512;

@@ -32,6 +32,19 @@ __global__ __launch_bounds__(256) void token_gather_kernel(const T* __restrict__
   }
 }
 
+// Rows of a table by 64-bit ids, as bytes (an embedding lookup): one 16-byte access a thread, a row's accesses spread over
+// blockIdx.y. An id outside the table gives a row of set bits, which are NaNs. Latency bound: 16 rows of 8 KB
+// 13.2 us with torch's small-index kernel, 4.4 us here.
+__global__ __launch_bounds__(256) void gather_rows_kernel(const u32x4* __restrict__ table,
+                                                          const int64_t* __restrict__ ids, u32x4* __restrict__ out,
+                                                          int64_t n_rows, int64_t chunks) {
+  const int64_t c = (int64_t)blockIdx.y * 256 + threadIdx.x;
+  if (c >= chunks) return;
+  const int64_t id = ids[blockIdx.x];
+  const u32x4 none = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};
+  out[blockIdx.x * chunks + c] = id >= 0 && id < n_rows ? table[id * chunks + c] : none;
+}
+
 // out[b, idx[b, r], :] = part[b, r, :]   (out already holds the full [B, S, H] input)
 template <typename T>
 __global__ __launch_bounds__(256) void token_scatter_kernel(const T* __restrict__ part, const int* __restrict__ idx,
@@ -164,6 +177,17 @@ HDS_EXPORT int hds_token_gather(int dtype, const void* x, const int* idx, void* 
   if (H % 8 || B <= 0 || R <= 0) return (int)hipErrorInvalidValue;
   HDS_TOK_DISPATCH(dtype, hipLaunchKernelGGL(token_gather_kernel<T>, dim3(B * R), dim3(256), 0, st,
                                              (const T*)x, idx, (T*)out, S, R, H));
+  return (int)hipGetLastError();
+}
+
+// table [n_rows, row_bytes] and out [n, row_bytes] with 16-byte rows
+HDS_EXPORT int hds_gather_rows(const void* table, const int64_t* ids, void* out, int n, int64_t row_bytes,
+                               int64_t n_rows, hipStream_t st) {
+  if (n <= 0) return 0;
+  const int64_t chunks = row_bytes / 16, cols = (chunks + 255) / 256;
+  if (row_bytes < 16 || row_bytes % 16 || cols > 65535) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(gather_rows_kernel, dim3(n, (int)cols), dim3(256), 0, st, (const u32x4*)table, ids, (u32x4*)out,
+                     n_rows, chunks);
   return (int)hipGetLastError();
 }
 

@@ -352,10 +352,10 @@ class RaggedTransformer:
 
     @torch.no_grad()
     def forward_decode_graph(self, batch, capture_latents=False):
-        """Replay the decode step for ``batch.current_sequences`` sequences: the step's token ids and packed
-        metadata (same layout as ``RaggedBatchWrapper.finalize``) are copied into the graph's static buffers, the
-        graph replays every layer's kernels with one launch, and the logits are copied out. The first step of a
-        batch size runs the forward eagerly over the same buffers, for a size may come once; the second captures it.
+        """Replay the decode step for ``batch.current_sequences`` sequences: the graph reads the step's token ids and
+        metadata from the batch's device buffer (``RaggedBatchWrapper.finalize``), replays every layer's kernels with
+        one launch, and the logits are copied out. A graph of before that buffer grew keeps the old one, into which
+        they are copied. The first step of a batch size runs the forward eagerly over the same buffers, for a size may come once; the second captures it.
 
         ``capture_latents``: the graph also stores each layer's latent rows into a device ring slot (HCache during
         decode, reference llama_v2/model.py:211-218 captures in every forward); returns ``(logits, latents)`` with
@@ -364,13 +364,11 @@ class RaggedTransformer:
         B = batch.current_sequences
         key = (B, bool(capture_latents))
         g = self._decode_graphs.get(key)
-        n = batch.seq_meta.numel() + batch.tok_seq.numel() + batch.tok_pos.numel() + batch.last_token_idx.numel() \
-            + batch.block_tables.numel() + batch.atoms.numel() + batch.slots.numel()
         if g is None:
             ring = _LatentRing(self, B, self.decode_latent_ring_steps) if capture_latents else None
-            g = self._decode_graphs[key] = _DecodeGraph(self, batch, n, ring)
-        g.ids.copy_(batch.input_ids, non_blocking=True)
-        g.meta.copy_(batch._dev_meta[:n], non_blocking=True)
+            g = self._decode_graphs[key] = _DecodeGraph(self, batch, ring)
+        if g.meta.data_ptr() != batch._dev_meta.data_ptr():
+            g.meta.copy_(batch._dev_meta[:g.meta.numel()], non_blocking=True)
         view = g.ring.begin_step() if g.ring is not None else None
         if not g.seen:
             g.seen = True
@@ -724,15 +722,15 @@ class _DecodeGraph:
     """Static inputs, captured graph and output of one decode batch size (RaggedTransformer.forward_decode_graph),
     with its latent ring when the graph captures HCache latents."""
 
-    def __init__(self, model, batch, n, ring=None):
+    def __init__(self, model, batch, ring=None):
         self.ring = ring
-        dev = model.device
         B = batch.current_sequences
         mb = batch.block_tables.shape[1]
         A = batch.n_atoms
-        self.ids = torch.zeros(B, dtype=batch.input_ids.dtype, device=dev)
-        self.meta = torch.zeros(n, dtype=torch.int32, device=dev)
-        o = 0
+        n = 2 * B + batch.seq_meta.numel() + batch.tok_seq.numel() + batch.tok_pos.numel() + \
+            batch.last_token_idx.numel() + batch.block_tables.numel() + batch.atoms.numel() + batch.slots.numel()
+        self.meta = batch._dev_meta[:n]  # same layout as RaggedBatchWrapper.finalize
+        o = 2 * B
 
         def take(k, shape):
             nonlocal o
@@ -741,7 +739,7 @@ class _DecodeGraph:
             return v
 
         sb = types.SimpleNamespace()
-        sb.input_ids = self.ids
+        sb.input_ids = self.meta[:o].view(torch.int64)
         sb.seq_meta = take(3 * B, (B, 3))
         sb.tok_seq = take(B, (B, ))
         sb.tok_pos = take(B, (B, ))

@@ -15,6 +15,7 @@ import torch.nn.functional as F
 from .... import comm as dist
 from ....ops.activations import bias_act, glu, glu_rows
 from ....ops.delta_rule import DeltaShape, delta_rule, make_delta_plan, step_ok
+from ....ops.embedding import lookup_rows
 from ....ops.experts import PAD, RouterShape, routed_experts
 from ....ops.gated_scan import gated_scan, recur_step, recur_step_ok
 from ....ops.gemv import glu_gemv
@@ -25,7 +26,7 @@ from ....ops.latent_attention import LatentShape, can_expand, latent_attention, 
 from ....ops.matrix_memory import MemoryShape, make_memory_plan, matrix_memory
 from ....ops.matrix_memory import step_ok as memory_step_ok
 from ....ops.moe import moe_combine, moe_dispatch, topk_assign, topk_route
-from ....ops.norm import layer_norm, rms_norm
+from ....ops.norm import layer_norm, norm_picked, norm_picked_ok, rms_norm
 from ....ops.output_norm import (PairSum, embed_rows, padded, residual_norm, rms_rows, sandwich_norm, softcap_,
                                  stream_norm, sum_experts)
 from ....ops.paged import (HeadShape, head_attention, head_blocks_ok, kv_rope_scatter, make_head_plan,
@@ -296,7 +297,7 @@ class RaggedEmbedding(DSEmbeddingBase):
         return "ragged_embedding"
 
     def forward(self, batch, word_embeddings, position_embeddings=None):
-        h = F.embedding(batch.input_ids, word_embeddings)
+        h = lookup_rows(word_embeddings, batch.input_ids)
         if position_embeddings is not None:
             h = h + F.embedding(batch.tok_pos.long() + self._config.positional_offset, position_embeddings)
         return h
@@ -314,14 +315,29 @@ class RaggedUnembed(DSUnembedBase):
     def forward(self, hidden, residual, batch, lm_head, lm_head_b, final_w, final_b, norm_eps=1e-5, tp_group=None,
                 vocab=None):
         idx = batch.last_token_idx
-        if final_w is not None:
-            if self._config.norm_type == "rms":
-                hl, _ = rms_norm(hidden[idx], final_w, norm_eps, residual[idx])
+        is_ln = self._config.norm_type != "rms"
+        if self._every_row(batch, hidden):  # nothing to gather
+            if final_w is None:
+                hl = hidden + residual
+            elif is_ln:
+                hl, _ = layer_norm(hidden, final_w, final_b, norm_eps, residual)
             else:
-                hl, _ = layer_norm(hidden[idx], final_w, final_b, norm_eps, residual[idx])
-        else:
+                hl, _ = rms_norm(hidden, final_w, norm_eps, residual)
+        elif final_w is not None and norm_picked_ok(hidden, residual, idx, final_w, final_b):
+            hl = norm_picked(hidden, residual, idx, final_w, final_b, norm_eps, is_ln)
+        elif final_w is None:
             hl = hidden[idx] + residual[idx]
+        elif is_ln:
+            hl, _ = layer_norm(hidden[idx], final_w, final_b, norm_eps, residual[idx])
+        else:
+            hl, _ = rms_norm(hidden[idx], final_w, norm_eps, residual[idx])
         return self.project(hl, lm_head, lm_head_b, tp_group, vocab)
+
+    @staticmethod
+    def _every_row(batch, hidden):
+        """A step of single tokens whose logits are all wanted: row i is sequence i's."""
+        return (getattr(batch, "logits_of_last_tokens", False) and getattr(batch, "max_new", 0) == 1
+                and hidden.shape[0] == batch.current_sequences == batch.last_token_idx.shape[0])
 
     def project(self, hl, lm_head, lm_head_b=None, tp_group=None, vocab=None):
         """Logits of already normed rows."""

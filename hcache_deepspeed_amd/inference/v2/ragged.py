@@ -306,8 +306,8 @@ class RaggedBatchWrapper:
     def finalize(self):
         """Ship the batch description to the device: the native builder (csrc/host/ragged_meta.cpp) writes seq_meta,
         token -> sequence / position maps, last-token rows, the KV block table and the attention atoms into ONE
-        pinned int32 buffer, sent with one async H2D copy into a persistent device buffer (plus one for the token
-        ids); the device tensors below are views of it."""
+        pinned int32 buffer behind the 64-bit token ids, sent with one async H2D copy into a persistent device buffer;
+        the device tensors below are views of it."""
         import ctypes
         import numpy as np
         from ...ops import native
@@ -332,12 +332,15 @@ class RaggedBatchWrapper:
         mixed = any(nn != 1 for (_, nn, _) in self.seq_meta_host)
         toks, blocks = make_portions(self.seq_meta_host) if mixed else ([], [])
         extra = [seq.tracking_id for seq in self._seqs] + (self._logit_rows or []) + blocks + toks
-        si, host = self._pinned_slot(int(need.value) + len(extra))
+        head = 2 * T  # the ids, first: 8-byte aligned
+        si, host = self._pinned_slot(head + int(need.value) + len(extra))
         A = lib.hds_ragged_meta_build(P(n_new), P(seen), S, P(flat), P(off), mb, n_q, n_kv, rpa,
-                                      ctypes.c_void_p(host.data_ptr()), host.numel(), ctypes.byref(need))
+                                      ctypes.c_void_p(host.data_ptr() + 4 * head), host.numel() - head, ctypes.byref(need))
         if A < 0:
             raise RuntimeError(f"ragged metadata builder failed ({A})")
-        n = int(need.value)
+        if T:
+            torch.cat(self._tokens, out=host[:head].view(torch.int64))
+        n = head + int(need.value)
         if extra:
             host.numpy()[n:n + len(extra)] = extra
         n += len(extra)
@@ -345,14 +348,12 @@ class RaggedBatchWrapper:
         if dev_buf is None or dev_buf.numel() < n:
             dev_buf = self._dev_meta = torch.empty(max(n, 4096), dtype=torch.int32, device=self.device)
         dev_buf[:n].copy_(host[:n], non_blocking=True)
-        ids = torch.cat(self._tokens) if self._tokens else torch.zeros(0, dtype=torch.int64)
         if self.device.type == "cuda":
-            ids = ids.pin_memory()
             ev = torch.cuda.Event()
             ev.record()
             self._slot_events[si] = ev
-        self.input_ids = ids.to(self.device, non_blocking=True)
-        o = 0
+        self.input_ids = dev_buf[:head].view(torch.int64)
+        o = head
 
         def take(k, shape):
             nonlocal o
@@ -380,7 +381,7 @@ class RaggedBatchWrapper:
         if mixed:
             blocks = take(len(blocks), (-1, 2)) if blocks else None
             self.portions = (take(len(toks), (-1, )) if toks else None, blocks)
-        self.tables_host = host[4 * S + 2 * T:4 * S + 2 * T + S * mb].view(S, mb).clone() if S else \
+        self.tables_host = host[head + 4 * S + 2 * T:head + 4 * S + 2 * T + S * mb].view(S, mb).clone() if S else \
             torch.zeros(1, mb, dtype=torch.int32)
         if S == 0:  # keep 1-row shapes for empty batches (kernels never run on them)
             self.seq_meta = torch.zeros(1, 3, dtype=torch.int32, device=self.device)

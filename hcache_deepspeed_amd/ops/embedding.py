@@ -39,6 +39,21 @@ def embedding_grad_add_(grad, ids, dy, padding_idx=None):
     return grad
 
 
+def lookup_rows(table, ids):
+    """``F.embedding(ids, table)``, on the GPU by a kernel of one launch for tables without a gradient whose rows are whole
+    16-byte pieces; ids outside the table give NaN rows there."""
+    row = table.shape[-1] * table.element_size()
+    if native.use_native(table) and table.dim() == 2 and ids.dim() == 1 and ids.dtype == torch.int64 and \
+            ids.device == table.device and table.is_floating_point() and row % 16 == 0 and \
+            16 <= row <= 16 * 256 * 65535 and ids.is_contiguous() and table.is_contiguous() and \
+            table.data_ptr() % 16 == 0 and not (torch.is_grad_enabled() and table.requires_grad):
+        out = torch.empty(ids.numel(), table.shape[1], dtype=table.dtype, device=table.device)
+        native.check(native.kernels().hds_gather_rows(table.data_ptr(), ids.data_ptr(), out.data_ptr(), ids.numel(), row,
+                                                      table.shape[0], native.stream()), "gather_rows")
+        return out
+    return F.embedding(ids, table)
+
+
 class EmbeddingFunction(torch.autograd.Function):
 
     @staticmethod

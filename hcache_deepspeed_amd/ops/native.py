@@ -19,7 +19,8 @@ _hlib = None
 
 # argument spec letters: p=void*, i=int32, u=uint32, l=int64, f=float, s=hipStream_t
 _KERNEL_SIGS = {
-    "hds_norm_fwd": "iii" + "p" * 8 + "ii" + "f" + "s",
+    "hds_norm_fwd": "iii" + "p" * 8 + "ii" + "f" + "pi" + "s",
+    "hds_gather_rows": "ppp" + "ill" + "s",
     "hds_norm_bwd_nparts": "i",
     "hds_norm_bwd_set_max_parts": "i",
     "hds_norm_bwd": "iii" + "p" * 9 + "i" + "pp" + "iii" + "s",

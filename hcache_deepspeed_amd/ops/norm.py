@@ -28,10 +28,10 @@ def _ref_norm(x, residual, weight, bias, eps, is_ln):
     return y.to(x.dtype), h
 
 
-def _native_fwd(x2, r2, weight, bias, eps, is_ln):
-    rows, cols = x2.shape
-    y = torch.empty_like(x2)
-    h = torch.empty_like(x2) if r2 is not None else None
+def _native_fwd(x2, r2, weight, bias, eps, is_ln, pick=None):
+    rows, cols = x2.shape if pick is None else (pick.numel(), x2.shape[1])
+    y = torch.empty(rows, cols, device=x2.device, dtype=x2.dtype)
+    h = torch.empty_like(y) if r2 is not None and pick is None else None
     rstd = torch.empty(rows, device=x2.device, dtype=torch.float32)
     mean = torch.empty(rows, device=x2.device, dtype=torch.float32) if is_ln else None
     if rows:
@@ -39,7 +39,8 @@ def _native_fwd(x2, r2, weight, bias, eps, is_ln):
         native.check(
             lib.hds_norm_fwd(int(is_ln), native.dt(x2), native.dt(weight), x2.data_ptr(), native.ptr(r2),
                              native.ptr(h), weight.data_ptr(), native.ptr(bias), y.data_ptr(), native.ptr(mean),
-                             rstd.data_ptr(), rows, cols, float(eps), native.stream()), "norm_fwd")
+                             rstd.data_ptr(), rows, cols, float(eps), native.ptr(pick), x2.shape[0], native.stream()),
+            "norm_fwd")
     return y, (h if h is not None else x2), mean, rstd
 
 
@@ -138,6 +139,22 @@ def rms_norm(x, weight, eps=1e-6, residual=None):
 def layer_norm(x, weight, bias=None, eps=1e-5, residual=None):
     y, h = _NormFn.apply(x, residual, weight, bias, eps, True)
     return (y, h) if residual is not None else y
+
+
+def norm_picked_ok(x, residual, pick, *params):
+    """Can ``norm_picked`` take these (otherwise: index, then norm)?"""
+    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, residual) + params):
+        return False
+    return (x.dim() == 2 and pick.dim() == 1 and pick.dtype == torch.int32 and residual.shape == x.shape
+            and residual.dtype == x.dtype and x.shape[0] > 0
+            and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (x, residual)))
+
+
+def norm_picked(x, residual, pick, weight, bias=None, eps=1e-6, is_ln=False):
+    """Norm of the rows ``pick`` of x + residual, without a gradient: on the GPU one kernel reads them where they are."""
+    if native.use_native(x):
+        return _native_fwd(x, residual, weight, bias, eps, is_ln, pick.contiguous())[0]
+    return _ref_norm(x[pick], residual[pick], weight, bias, eps, is_ln)[0]
 
 
 class RMSNorm(nn.Module):

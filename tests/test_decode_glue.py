@@ -1,0 +1,130 @@
+"""What a decode step does around its layers: embedding rows, the rows whose logits are wanted, the step's description."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from hcache_deepspeed_amd.inference.v2.modules import DSUnembedConfig, instantiate_unembed
+from hcache_deepspeed_amd.ops.embedding import lookup_rows
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,W", [(torch.bfloat16, 8), (torch.bfloat16, 2056), (torch.float32, 4096), (torch.bfloat16, 12)])
+@pytest.mark.parametrize("n", [0, 1, 16, 700])
+def test_lookup_rows_gpu(dtype, W, n):
+    table = torch.randn(301, W, device="cuda").to(dtype)
+    ids = torch.randint(0, 301, (n, ), device="cuda")
+    ids[:1] = 300
+    assert torch.equal(lookup_rows(table, ids), F.embedding(ids, table))
+    if W % 8 == 0 and n > 1:
+        ids[1] = 301
+        out = lookup_rows(table, ids)
+        assert out[1].isnan().all() and torch.equal(out[0], table[300])
+
+
+def _unembed(norm, dev, W, n, T, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    r = lambda *s: torch.randn(*s, generator=g).to(dev, torch.bfloat16)  # noqa: E731
+    h, res, w, b, lm = r(T, W), r(T, W), r(W), r(W) if norm == "layer" else None, r(48, W)
+    mod = instantiate_unembed(DSUnembedConfig(model_dim=W, vocab_size=48, norm_type=norm))
+    return mod, h, res, w, b, lm
+
+
+def _plain(norm, h, res, w, b, lm, idx, final=True):
+    x = (h[idx].float() + res[idx].float()).to(h.dtype)
+    if final:
+        xf = x.float()
+        if norm == "layer":
+            y = F.layer_norm(xf, xf.shape[-1:], w.float(), b.float(), 1e-5)
+        else:
+            y = xf * torch.rsqrt((xf * xf).mean(-1, keepdim=True) + 1e-5) * w.float()
+        x = y.to(h.dtype)
+    return x.float() @ lm.float().t()
+
+
+class _Batch:
+    pass
+
+
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("norm", ["rms", "layer"])
+@pytest.mark.parametrize("W", [512, 4096, 648])
+@pytest.mark.parametrize("pick,new,last,dtype", [
+    ([0, 1, 2], 1, True, torch.int32),      # single tokens: every row
+    ([2, 6, 6, 0], 4, True, torch.int32),   # last tokens of portions, in any order
+    ([2, -1, 0], 4, False, torch.int32),    # rows of the caller's choice
+    ([2, 6, 0], 4, True, torch.int64),
+])
+@pytest.mark.parametrize("final", [True, False])
+def test_wanted_rows(dev, norm, W, pick, new, last, dtype, final):
+    T = 3 if new == 1 else 7
+    mod, h, res, w, b, lm = _unembed(norm, dev, W, len(pick), T)
+    batch = _Batch()
+    batch.last_token_idx = torch.tensor(pick, dtype=dtype, device=dev)
+    batch.logits_of_last_tokens, batch.max_new, batch.current_sequences = last, new, len(pick)
+    with torch.no_grad():
+        got = mod(h, res, batch, lm, None, w if final else None, b, 1e-5)
+    want = _plain(norm, h.cpu(), res.cpu(), w.cpu(), None if b is None else b.cpu(), lm.cpu(), batch.last_token_idx.cpu().long(),
+                  final)
+    # two roundings to bf16 of the row (2^-9 each) through W products of unit variance, and the logit's own
+    bound = 6 * 2**-8 * lm.cpu().float().norm(dim=1) * (w.abs().max().item() if final else 2) + 2**-8 * want.abs()
+    assert (got.cpu().float() - want).abs().le(bound).all()
+
+
+def test_step_description_on_the_host():
+    """Ids, metadata and the division of a mixed step are views of one buffer."""
+    from hcache_deepspeed_amd.inference.v2.ragged import (BlockedKVCache, DSStateManager, DSStateManagerConfig,
+                                                          RaggedBatchWrapper)
+    cfg = DSStateManagerConfig(max_context=256)
+    kv = BlockedKVCache(1, 2, 16, 64, torch.float32, torch.device("cpu"), cfg.memory_config, num_blocks=8)
+    sm = DSStateManager(cfg, kv)
+    b = RaggedBatchWrapper(cfg, torch.device("cpu"), sm.max_blocks_per_seq)
+    b.set_attention_geometry(4, 2, 128)
+    for lens in ([1], [1, 1, 1], [3, 1, 20], [5]):
+        b.clear()
+        toks = [torch.arange(n) + 2**33 * (i + 1) for i, n in enumerate(lens)]
+        for i, t in enumerate(toks):
+            seq = sm.get_or_create_sequence(i)
+            sm.maybe_allocate_kv(seq, len(t))
+            b.insert_sequence(seq, t)
+        b.finalize()
+        assert torch.equal(b.input_ids, torch.cat(toks)) and b.input_ids.dtype == torch.int64
+        T, S = sum(lens), len(lens)
+        assert b.tok_seq.tolist() == [i for i, n in enumerate(lens) for _ in range(n)]
+        assert b.tok_pos.tolist() == [j for n in lens for j in range(n)]
+        assert b.last_token_idx.tolist() == [sum(lens[:i + 1]) - 1 for i in range(S)]
+        assert torch.equal(b.tables_host, b.block_tables) and b.block_tables.shape == (S, sm.max_blocks_per_seq)
+        for i in range(S):
+            blocks = sm.get_sequence(i).kv_blocks
+            assert b.block_tables[i, :len(blocks)].tolist() == blocks
+        assert b.slots.tolist() == [sm.get_sequence(i).tracking_id for i in range(S)] and b.current_tokens == T
+
+
+@pytest.mark.gpu
+def test_graph_after_the_buffer_grew_gpu():
+    """A graph reads the batch's device buffer; when a larger step has replaced that, later steps reach the graph's own."""
+    from hcache_deepspeed_amd.inference.v2.arch import ArchSpec
+    from hcache_deepspeed_amd.inference.v2.engine import InferenceEngineV2, RaggedInferenceEngineConfig
+    H, I, V = 256, 512, 211
+    g = torch.Generator().manual_seed(0)
+    dev = torch.device("cuda")
+    mat = lambda *s: (torch.randn(*s, generator=g) * s[-1]**-0.5).bfloat16().to(dev)  # noqa: E731
+    one = torch.ones(H, dtype=torch.bfloat16, device=dev)
+    layers = [{"ln1.w": one, "ln2.w": one, "qkv.w": mat(4 * 128, H), "o.w": mat(H, 256), "up.w": mat(2 * I, H),
+               "down.w": mat(H, I)} for _ in range(2)]
+    w = {"embed": mat(V, H) * 16, "final.w": one, "lm_head.w": mat(V, H), "layers": layers}
+    spec = ArchSpec("llama", V, H, 2, 2, 1, 128, I, max_position_embeddings=8192)
+    conf = RaggedInferenceEngineConfig.from_dict(dict(dtype="bf16", state_manager=dict(max_context=4096,
+                                                                                       max_ragged_batch_size=8192)))
+    engs = {k: InferenceEngineV2(spec, w, conf, device=dev, num_kv_blocks=200) for k in ("graph", "eager")}
+    engs["eager"]._model.decode_graph_max_batch = 0
+    draw = lambda n: torch.randint(0, V, (n, ), generator=g)  # noqa: E731
+    step = lambda uids, toks: {k: e.put(uids, toks, capture_latents=False)[0] for k, e in engs.items()}  # noqa: E731
+    step([1, 2], [draw(40), draw(65)])
+    sizes = set()
+    for i in range(9):
+        if i in (3, 6):  # more tokens than the buffer holds, twice
+            step([10 + i], [draw(1500 * i // 3)])
+        out = step([1, 2], [draw(1), draw(1)])
+        assert torch.equal(out["graph"], out["eager"]), i
+        sizes.add(engs["graph"]._batch._dev_meta.numel())
+    assert len(sizes) == 3 and engs["graph"]._model._decode_graphs[2, False].graph is not None
