@@ -258,69 +258,178 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(const bf16* __restrict_
 // Skinny GEMM for 2..16 token rows on the matrix cores: y[M, N] = x[M, K] . W[N, K]^T (+ bias).
 // The VALU GEMV above spends 4 dot2 instructions per 16-B weight chunk PER ROW, so from a few rows on it is VALU-bound
 // (o projection at M = 8: 1.7 TB/s) and hipBLASLt's small-M tiles stream at 3.5-3.7 TB/s. Here one
-// mfma_f32_16x16x32_bf16 contracts a 16-column x 32-k weight tile with all (up to 16) token rows at once, so the
-// kernel is a pure weight stream: A = W rows (lane l: row n0 + (l & 15), k = 8 (l >> 4) .. +8, one 16-B load), B = x^T
-// (lane l: token l & 15, same k; zero past M), C: token = l & 15, column n0 + 4 (l >> 4) + reg. A workgroup owns 16
-// output columns; its 4 waves split K four ways with 8 weight loads per lane in flight, and the partial tiles are
-// summed through LDS.
+// mfma_f32_16x16x32_bf16 contracts a 16-row x 32-k weight tile with all (up to 16) token rows at once, so the
+// kernels are pure weight streams: A = W rows (lane l: row l & 15, k = 8 (l >> 4) .. +8), B = x^T
+// (lane l: token l & 15, same k), C: token = l & 15, weight row 4 (l >> 4) + reg. A workgroup owns 16
+// weight rows; its waves share K, and the partial tiles are summed through LDS.
+// GLU: W is [gate; up] of 2 N rows, a tile is 8 gate rows and the 8 up rows that belong to them, so that there are as many
+// workgroups as without (a tile of 16 + 16 rows left half of the chip's slots empty and lost against the separate
+// kernel), and y = bf16(act(bf16(gate)) * bf16(up)).
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <int U, bool GATHER>
-__global__ __launch_bounds__(256) void skinny_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
-                                                          const bf16* __restrict__ bias, bf16* __restrict__ y, int M,
-                                                          int N, int K, int64_t ldx, int64_t ldy, Gather gather) {
-  __shared__ f32x4 red[3][64];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int n0 = blockIdx.x * 16;
-  const int row = min(n0 + (lane & 15), N - 1);  // tail columns re-read column N-1 (not stored)
-  const int tok = lane & 15;
-  const int kq = K >> 2;  // this wave's quarter of K (K % 128 == 0)
-  const int kb = wid * kq + 8 * (lane >> 4);
-  const bf16* wp = w + (int64_t)row * K + kb;
-  const bf16* xp = x + (int64_t)min(tok, M - 1) * ldx + kb;
-  const bool tok_ok = tok < M;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  int k = 0;
-  for (; k + 32 * U <= kq; k += 32 * U) {
-    bf16x8_t a[U], b[U];
+struct SkinnyOut {
+  const bf16* bias;
+  bf16* y;
+  int M, N;
+  int64_t ldy;
+  int act;  // GLU
+};
+
+// W's row r (of 16) of the workgroup's tile; rows past the end re-read the last one (not stored)
+template <bool GLU>
+__device__ __forceinline__ int64_t skinny_row(int r, int N) {
+  if constexpr (GLU) {
+    const int n = min((int)blockIdx.x * 8 + (r & 7), N - 1);
+    return r < 8 ? n : (int64_t)N + n;
+  }
+  return min((int)blockIdx.x * 16 + r, N - 1);
+}
+
+template <bool GATHER, bool GLU>
+__device__ __forceinline__ void skinny_store(const SkinnyOut& o, const Gather& gather, f32x4 acc, int lane) {
+  const int tok = lane & 15, g = lane >> 4;
+  if constexpr (GLU) {  // lanes of the upper half hold the up rows of those 32 below
+    const int n0 = blockIdx.x * 8 + 4 * (g & 1);
 #pragma unroll
-    for (int u = 0; u < U; ++u) a[u] = *reinterpret_cast<const bf16x8_t*>(wp + k + 32 * u);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      b[u] = *reinterpret_cast<const bf16x8_t*>(xp + k + 32 * u);
-      if (!tok_ok) b[u] = bf16x8_t{};
+    for (int r = 0; r < 4; ++r) {
+      const int n = n0 + r;
+      float v = acc[r];
+      if (o.bias != nullptr && n < o.N) v += (float)o.bias[lane < 32 ? n : o.N + n];
+      const float up = __shfl_down(v, 32, 64);
+      if (lane < 32 && tok < o.M && n < o.N)
+        o.y[(int64_t)tok * o.ldy + n] = (bf16)(gate_f((float)(bf16)v, o.act) * (float)(bf16)up);
     }
+  } else if (tok < o.M) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u], acc, 0, 0, 0);
-  }
-  for (; k < kq; k += 32) {
-    const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(wp + k);
-    bf16x8_t b = *reinterpret_cast<const bf16x8_t*>(xp + k);
-    if (!tok_ok) b = bf16x8_t{};
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-  }
-  if (wid > 0) red[wid - 1][lane] = acc;
-  __syncthreads();
-  if (wid == 0) {
-#pragma unroll
-    for (int v = 0; v < 3; ++v) acc += red[v][lane];
-    if (tok_ok) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = n0 + 4 * (lane >> 4) + r;
-        if (n < N) {
-          float v = acc[r];
-          if (bias) v += (float)bias[n];
-          if constexpr (GATHER) v = gather(v, tok, n);
-          y[(int64_t)tok * ldy + n] = (bf16)v;
-        }
+    for (int r = 0; r < 4; ++r) {
+      const int n = blockIdx.x * 16 + 4 * g + r;
+      if (n < o.N) {
+        float v = acc[r];
+        if (o.bias != nullptr) v += (float)o.bias[n];
+        if constexpr (GATHER) v = gather(v, tok, n);
+        o.y[(int64_t)tok * o.ldy + n] = (bf16)v;
       }
     }
   }
 }
 
+// Up to 4 tokens: weights straight into the operand's registers, 16-B pieces of 16 rows a load. Four waves take turns at
+// 32 U columns (at K below that times four, a quarter each): [4096, 14336] at 3 rows 25.0 us with a quarter of K a wave, 22.1
+// in turns.
+template <int U, bool GATHER, bool GLU>
+__global__ __launch_bounds__(256) void skinny_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, int K,
+                                                          int64_t ldx, SkinnyOut o, Gather gather) {
+  __shared__ f32x4 red[3][64];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int part = min(32 * U, K >> 2);  // K % 128 == 0
+  const bf16* wp = w + skinny_row<GLU>(lane & 15, o.N) * K + 8 * (lane >> 4);
+  const bf16* xp = x + (int64_t)min(lane & 15, o.M - 1) * ldx + 8 * (lane >> 4);  // (columns past M are not stored)
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int k0 = wid * part; k0 < K; k0 += 4 * part) {
+    const int k1 = min(k0 + part, K);
+    if (k1 - k0 == 32 * U) {
+      bf16x8_t a[U], b[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) a[u] = *reinterpret_cast<const bf16x8_t*>(wp + k0 + 32 * u);
+#pragma unroll
+      for (int u = 0; u < U; ++u) b[u] = *reinterpret_cast<const bf16x8_t*>(xp + k0 + 32 * u);
+      __builtin_amdgcn_sched_barrier(0);  // all loads first: the compiler moves some behind the first products
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u], acc, 0, 0, 0);
+    } else {
+      for (int k = k0; k < k1; k += 32)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(wp + k),
+                                                      *reinterpret_cast<const bf16x8_t*>(xp + k), acc, 0, 0, 0);
+    }
+  }
+  if (wid > 0) red[wid - 1][lane] = acc;
+  __syncthreads();
+  if (wid > 0) return;
+#pragma unroll
+  for (int v = 0; v < 3; ++v) acc += red[v][lane];
+  skinny_store<GATHER, GLU>(o, gather, acc, lane);
+}
+
+// 5 to 16 tokens. The tokens are then as many bytes of loads as the weights, served by the L2, and what bounds the kernel
+// above is how many cache lines a CU can have on the way: its loads ask for half a line of 16 weight rows each. Here a load
+// takes whole lines (8 rows of 64 columns), which pass through the wave's own piece of LDS into the operand's layout
+// (16-B pieces, placed by row ^ piece so that the reads spread over the banks); a wave has 128 columns in flight and there
+// are up to 32 waves a CU to overlap them. 16 rows, the kernel above -> this one: [28672, 4096] 60 -> 48.0 us (4.9 TB/s),
+// [4096, 14336] 29.8 -> 26.5, [6144, 4096] 17.6 -> 13.5, [32000, 4096] 66 -> 53 (library 57); 7 rows: 45.6 -> 40.1, 26.1 -> 23.8,
+// 14.1 -> 12.2, 50.6 -> 44.7; at 3 rows the kernel above is ahead at K = 2048 ([16384, 2048] 13.4 against 15.7) and level
+// elsewhere. Two tiles a workgroup halve the tokens' loads but were slower (54 to 59 us), the DMA into LDS is level.
+template <int NW, bool GATHER, bool GLU>
+__global__ __launch_bounds__(64 * NW) void skinny_lines_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
+                                                               int K, int64_t ldx, SkinnyOut o, Gather gather) {
+  __shared__ __attribute__((aligned(16))) char buf[NW][4096];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int wr = lane >> 3, wz = lane & 7, rr = lane & 15, rp = lane >> 4;
+  const bf16* w0 = w + skinny_row<GLU>(wr, o.N) * K + 8 * wz;
+  const bf16* w1 = w + skinny_row<GLU>(8 + wr, o.N) * K + 8 * wz;
+  const bf16* xp = x + (int64_t)min(rr, o.M - 1) * ldx + 8 * rp;  // (columns past M are not stored)
+  char* mine = buf[wid];
+  char* put = mine + wr * 128 + (wz ^ wr) * 16;
+  const char* get0 = mine + rr * 128 + (rp ^ (rr & 7)) * 16;
+  const char* get1 = mine + rr * 128 + ((rp + 4) ^ (rr & 7)) * 16;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int k = 128 * wid; k < K; k += 128 * NW) {  // K % 128 == 0
+    bf16x8_t a[2][2], b[4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      a[u][0] = *reinterpret_cast<const bf16x8_t*>(w0 + k + 64 * u);
+      a[u][1] = *reinterpret_cast<const bf16x8_t*>(w1 + k + 64 * u);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) b[u] = *reinterpret_cast<const bf16x8_t*>(xp + k + 32 * u);
+    __builtin_amdgcn_sched_barrier(0);  // (the last of them waited for by itself: 54 us instead of 48 at [28672, 4096])
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      *reinterpret_cast<bf16x8_t*>(put + u * 2048) = a[u][0];
+      *reinterpret_cast<bf16x8_t*>(put + u * 2048 + 1024) = a[u][1];
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const bf16x8_t p0 = *reinterpret_cast<const bf16x8_t*>(get0 + u * 2048);
+      const bf16x8_t p1 = *reinterpret_cast<const bf16x8_t*>(get1 + u * 2048);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p0, b[2 * u], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p1, b[2 * u + 1], acc, 0, 0, 0);
+    }
+  }
+  reinterpret_cast<f32x4*>(mine)[lane] = acc;
+  __syncthreads();
+  if (wid > 0) return;
+#pragma unroll
+  for (int v = 1; v < NW; ++v) acc += reinterpret_cast<const f32x4*>(buf[v])[lane];
+  skinny_store<GATHER, GLU>(o, gather, acc, lane);
+}
+
 int g_skinny_u = 16;
+
+// Waves a workgroup: four where there are at least two workgroups a CU of whole K walks ([6144, 4096] 13.7 us against 14.7
+// with eight, [28672, 4096] 48.6 / 50.4), eight where those are few ([4096, 14336] 26.6 against 27.9, [2048, 8192] 13.0 / 14.0)
+// or short ([16384, 2048] 17.9 / 19.0), and at up to 8 rows, whose tokens take fewer loads ([28672, 4096], 7 rows: 40.1 / 41.7).
+template <bool GATHER, bool GLU>
+int launch_skinny(const void* x, const void* w, int K, int64_t ldx, const SkinnyOut& o, const Gather& gather,
+                  hipStream_t st) {
+  const int per = GLU ? 8 : 16, tiles = (o.N + per - 1) / per;
+#define HDS_SK(T, ...) \
+  hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(T), 0, st, (const bf16*)x, (const bf16*)w, K, ldx, o, gather)
+  if (o.M > 4 || K < 2048) {  // (a wave of the other kernel wants 16 loads a turn)
+    if (o.M > 8 && tiles > 256 && K >= 4096)
+      HDS_SK(256, skinny_lines_kernel<4, GATHER, GLU>);
+    else
+      HDS_SK(512, skinny_lines_kernel<8, GATHER, GLU>);
+  } else if (g_skinny_u == 32 && K % 1024 == 0) {
+    HDS_SK(256, skinny_mfma_kernel<32, GATHER, GLU>);
+  } else if (g_skinny_u >= 16) {
+    HDS_SK(256, skinny_mfma_kernel<16, GATHER, GLU>);
+  } else {
+    HDS_SK(256, skinny_mfma_kernel<8, GATHER, GLU>);
+  }
+#undef HDS_SK
+  return hipGetLastError();
+}
 
 // ---------------------------------------------------------------------------------------------------------------
 // One decode step of the gated recurrence (gated_scan.hip) with its projection: a wave owns one channel j and streams
@@ -419,23 +528,17 @@ HDS_EXPORT int hds_gemv_recur_bf16(const void* x, const void* w, const float* ba
   return hipGetLastError();
 }
 
-// Skinny matrix-core GEMM (skinny_mfma_kernel): 1 <= M <= 16, K % 128 == 0, 16-B aligned rows
+// Skinny matrix-core GEMM: 1 <= M <= 16, K % 128 == 0, 16-B aligned rows. glu: 0, or 1 + activation code (0 silu, 1
+// gelu_tanh, 2 relu) for w = [gate; up] of 2 N rows
 HDS_EXPORT int hds_skinny_gemm_bf16(const void* x, const void* w, const void* bias, void* y, int M, int N, int K,
-                                    int64_t ldx, int64_t ldy, hipStream_t st) {
-  if (M < 1 || M > 16 || N < 1 || K < 128 || K % 128 || ldx % 8) return hipErrorInvalidValue;
-  if (g_skinny_u == 32 && (K >> 2) % 1024 == 0)
-    hipLaunchKernelGGL((skinny_mfma_kernel<32, false>), dim3((N + 15) / 16), dim3(256), 0, st, (const bf16*)x,
-                       (const bf16*)w, (const bf16*)bias, (bf16*)y, M, N, K, ldx, ldy, Gather{});
-  else if (g_skinny_u >= 16)
-    hipLaunchKernelGGL((skinny_mfma_kernel<16, false>), dim3((N + 15) / 16), dim3(256), 0, st, (const bf16*)x,
-                       (const bf16*)w, (const bf16*)bias, (bf16*)y, M, N, K, ldx, ldy, Gather{});
-  else
-    hipLaunchKernelGGL((skinny_mfma_kernel<8, false>), dim3((N + 15) / 16), dim3(256), 0, st, (const bf16*)x,
-                       (const bf16*)w, (const bf16*)bias, (bf16*)y, M, N, K, ldx, ldy, Gather{});
-  return hipGetLastError();
+                                    int64_t ldx, int64_t ldy, int glu, hipStream_t st) {
+  if (M < 1 || M > 16 || N < 1 || K < 128 || K % 128 || ldx % 8 || glu < 0 || glu > 3) return hipErrorInvalidValue;
+  const SkinnyOut o{(const bf16*)bias, (bf16*)y, M, N, ldy, glu - 1};
+  return glu ? launch_skinny<false, true>(x, w, K, ldx, o, Gather{}, st)
+             : launch_skinny<false, false>(x, w, K, ldx, o, Gather{}, st);
 }
 
-// weight loads per lane in flight in the skinny GEMM (8, 16 or 32); returns the previous value
+// weight loads per lane in flight in the skinny GEMM of up to 4 rows (8, 16 or 32); returns the previous value
 HDS_EXPORT int hds_skinny_set_unroll(int u) {
   const int prev = g_skinny_u;
   g_skinny_u = u >= 32 ? 32 : (u >= 16 ? 16 : 8);
@@ -510,7 +613,6 @@ HDS_EXPORT int hds_gather_gemv_bf16(const void* x, const void* w, const void* ta
     hipLaunchKernelGGL((gemv_bf16_kernel<1, 1, true>), dim3((N + 3) / 4), dim3(256), 0, st, (const bf16*)x,
                        (const bf16*)w, (const bf16*)nullptr, (bf16*)y, M, N, K, ldx, ldy, gather);
   else
-    hipLaunchKernelGGL((skinny_mfma_kernel<16, true>), dim3((N + 15) / 16), dim3(256), 0, st, (const bf16*)x,
-                       (const bf16*)w, (const bf16*)nullptr, (bf16*)y, M, N, K, ldx, ldy, gather);
+    return launch_skinny<true, false>(x, w, K, ldx, SkinnyOut{nullptr, (bf16*)y, M, N, ldy, 0}, gather, st);
   return hipGetLastError();
 }

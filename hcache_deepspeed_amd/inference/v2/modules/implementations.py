@@ -18,7 +18,7 @@ from ....ops.delta_rule import DeltaShape, delta_rule, make_delta_plan, step_ok
 from ....ops.embedding import lookup_rows
 from ....ops.experts import PAD, RouterShape, routed_experts
 from ....ops.gated_scan import gated_scan, recur_step, recur_step_ok
-from ....ops.gemv import glu_gemv
+from ....ops.gemv import glu_gemv, glu_linear, linear  # decode-sized steps on the HIP kernels
 from ....ops.grouped_gemm import moe_ffn_dropless
 from ....ops.head_prep import HeadPrep
 from ....ops.input_norm import input_norm
@@ -98,9 +98,11 @@ class BlasFPLinear(DSLinearBase):
 
     def forward(self, x, w, b=None):
         a = self._config.activation
-        from ....ops.gemv import linear  # decode-sized ragged batches (<= 8 tokens) on the HIP GEMV
-        if a == "identity" or a.endswith("_glu"):
-            return _act_tail(linear(x, w, b), None, a)
+        if a.endswith("_glu"):
+            y = glu_linear(x, w, b, a[:-4])
+            return _act_tail(linear(x, w, b), None, a) if y is None else y
+        if a == "identity":
+            return linear(x, w, b)
         return bias_act(linear(x, w), b, a)
 
 
@@ -341,7 +343,7 @@ class RaggedUnembed(DSUnembedBase):
 
     def project(self, hl, lm_head, lm_head_b=None, tp_group=None, vocab=None):
         """Logits of already normed rows."""
-        logits = F.linear(hl, lm_head, lm_head_b)
+        logits = linear(hl, lm_head, lm_head_b)
         tp = dist.get_world_size(tp_group) if tp_group is not None else 1
         if tp > 1:
             parts = [torch.empty_like(logits) for _ in range(tp)]

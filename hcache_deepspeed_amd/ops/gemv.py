@@ -67,8 +67,24 @@ def skinny(x2, w, b=None):
     N = w.shape[0]
     y = torch.empty(M, N, dtype=x2.dtype, device=x2.device)
     native.check(native.kernels().hds_skinny_gemm_bf16(x2.data_ptr(), w.data_ptr(), native.ptr(b), y.data_ptr(), M, N,
-                                                       K, x2.stride(0), N, native.stream()), "skinny_gemm_bf16")
+                                                       K, x2.stride(0), N, 0, native.stream()), "skinny_gemm_bf16")
     return y
+
+
+def glu_linear(x, w, b, act):
+    """act(x . gate^T) * (x . up^T) for ``w`` = [gate; up] (and ``b``) in one kernel, for 2..16 rows of the skinny GEMM; None
+    for anything else. The projections are rounded to bf16 first, as the separate kernels store them."""
+    if act not in _GATHER_ACTS or not (x.dim() >= 1 and x.is_cuda and torch.is_tensor(w)):
+        return None
+    x2 = x.reshape(-1, x.shape[-1])
+    if not skinny_ok(x2, w, b) or w.shape[0] % 2:
+        return None
+    (M, K), N = x2.shape, w.shape[0] // 2
+    y = torch.empty(M, N, dtype=x2.dtype, device=x2.device)
+    native.check(native.kernels().hds_skinny_gemm_bf16(x2.data_ptr(), w.data_ptr(), native.ptr(b), y.data_ptr(), M, N,
+                                                       K, x2.stride(0), N, 1 + _GATHER_ACTS[act], native.stream()),
+                 "skinny_gemm_bf16")
+    return y.view(*x.shape[:-1], N)
 
 
 def linear(x, w, b=None):

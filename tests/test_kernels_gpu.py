@@ -792,6 +792,34 @@ def test_skinny_gemm_matches_fp32(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("act", [None, "silu", "gelu_tanh", "relu"])
+@pytest.mark.parametrize("M", [2, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(7, 128), (1000, 640), (16, 2048), (4104, 2176), (24, 4224), (4112, 4096)])
+def test_skinny_gemm_edges(act, M, N, K):
+    """Both skinny kernels and their gated form against 64 bits: tiles with a remainder, K shorter than a workgroup's waves
+    take and no multiple of it. 32-bit sums of K products, then one rounding; gated: the projections rounded first."""
+    from hcache_deepspeed_amd.ops.gemv import glu_linear, skinny
+    g = torch.Generator(device="cuda").manual_seed(M * 13 + N)
+    rows = N if act is None else 2 * N
+    w = (torch.randn(rows, K, device="cuda", generator=g) * K**-0.5).to(torch.bfloat16)
+    x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
+    b = torch.randn(rows, device="cuda", generator=g).to(torch.bfloat16) if M % 2 else None
+    ref = x.double() @ w.double().t() + (0 if b is None else b.double())
+    sums = 2**-24 * K**0.5 * 8 * (x.double().abs() @ w.double().abs().t())
+    if act is None:
+        y, bound = skinny(x, w, b), 2**-8 * ref.abs() + sums
+    else:
+        y = glu_linear(x, w, b, act)
+        gate, up = ref[:, :N], ref[:, N:]
+        f = {"silu": torch.nn.functional.silu, "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh"),
+             "relu": torch.relu}[act]
+        ref = f(gate) * up
+        # each factor within half a unit of the last place and its sum's error; |act'| <= 1.13
+        bound = 2**-8 * (1.13 * gate.abs() * up.abs() + 2 * ref.abs()) + 1.13 * (sums[:, :N] * up.abs() + sums[:, N:] * gate.abs())
+    assert y.shape == ref.shape and ((y.double() - ref).abs() <= bound + 1e-6).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,glu,res", [(1, 6144, 4096, False, True), (1, 14336, 4096, True, True),
                                            (3, 4100, 4096, False, False), (8, 1000, 1032, True, True),
                                            (5, 8192, 512, True, False)])
