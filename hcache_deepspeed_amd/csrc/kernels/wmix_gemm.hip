@@ -231,7 +231,7 @@ __global__ __launch_bounds__(256) void wmix_reduce_kernel(const float* __restric
 // to 16 MT rows of A. The operand is the weight's CODE, which bf16 holds exactly; the group's scale multiplies the 32-bit
 // sum of each group (every chunk lies in one group), so no weight is rounded. fp6 codes become bf16 in one instruction
 // for 32 of them. Measured at 8 rows, [28672, 4096] / [4096, 14336]: fp6 38 / 22 us (92 / 46 MB; the GEMV that decodes and
-// multiplies on the VALU 112 / 77), int8 39 / 20 us (121 / 61 MB; the tile kernel above 45 / 28), int4 29 / 16 us (41 /
+// multiplies on the VALU 112 / 77; 27 us with A resident, below), int8 39 / 20 us (121 / 61 MB; the tile kernel above 45 / 28), int4 29 / 16 us (41 /
 // 29). A third of the time at 8 rows goes to reading A again from L2 in every workgroup.
 typedef uint32_t u32x6 __attribute__((ext_vector_type(6)));
 typedef __bf16 bf16x32 __attribute__((ext_vector_type(32)));
@@ -269,16 +269,53 @@ __device__ __forceinline__ void codes(const WRaw<FMT>& r, bf16x8 (&f)[4]) {
   }
 }
 
+// GLU: W is [gate; up] of 2 N rows, a tile of 16 weight rows holds 8 gate rows and their 8 up rows (as many workgroups as
+// without), and the result is bf16(act(bf16(gate)) * bf16(up)) [M, N].
+template <bool GLU>
+__device__ __forceinline__ int wmix_row(int tile, int r, int N) {
+  if constexpr (GLU) {
+    const int n = min(tile * 8 + (r & 7), N - 1);
+    return r < 8 ? n : N + n;
+  }
+  return min(tile * 16 + r, N - 1);
+}
+
+__device__ __forceinline__ float wmix_act(float v, int act) {  // codes of act.hip
+  if (act == 2) return fmaxf(v, 0.f);
+  if (act == 1) return 0.5f * v * (1.f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
+  return v * __builtin_amdgcn_rcpf(1.f + __expf(-v));
+}
+
+// a tile's sums: lane = A row r | 16 g, weight rows 4 g .. 4 g + 3
+template <bool GLU>
+__device__ __forceinline__ void wmix_store(f32x4 s, int tile, int row, int g, int lane, const bf16* bias, bf16* C, int M,
+                                           int N, int act) {
+  if constexpr (GLU) {  // lanes of the upper half hold the up rows of those 32 below
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int n = tile * 8 + 4 * (g & 1) + i;
+      const float up = __shfl_down(s[i], 32, 64);
+      if (lane < 32 && row < M && n < N) C[(int64_t)row * N + n] = (bf16)(wmix_act((float)(bf16)s[i], act) * (float)(bf16)up);
+    }
+  } else if (row < M) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int n = tile * 16 + 4 * g + i;
+      if (n < N) C[(int64_t)row * N + n] = (bf16)(s[i] + (bias ? (float)bias[n] : 0.f));
+    }
+  }
+}
+
 // MW: waves a SIMD that the registers have to leave room for
-template <int FMT, int E, int NT, int MT, int NW, int MW>
+template <int FMT, int E, int NT, int MT, int NW, int MW, bool GLU>
 __global__ __launch_bounds__(64 * NW, MW) void wmix_skinny_kernel(const bf16* __restrict__ A,
                                                                   const uint8_t* __restrict__ W,
                                                                   const float* __restrict__ scales,
                                                                   const bf16* __restrict__ bias, bf16* __restrict__ C,
-                                                                  int M, int N, int K, int G) {
+                                                                  int M, int N, int K, int G, int act) {
   __shared__ f32x4 red[NW - 1][NT][MT][64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * 16 * NT, groups = K / G;
+  const int tile0 = blockIdx.x * NT, groups = K / G;
   f32x4 acc[NT][MT];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -295,13 +332,13 @@ __global__ __launch_bounds__(64 * NW, MW) void wmix_skinny_kernel(const bf16* __
     for (int c = 0; c < 4; ++c) {
       const int k = min(512 * run + 128 * c, K - 128);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) raw[c][t] = load_w<FMT>(W, min(n0 + 16 * t + r, N - 1), K, k + 32 * g);
+      for (int t = 0; t < NT; ++t) raw[c][t] = load_w<FMT>(W, wmix_row<GLU>(tile0 + t, r, N), K, k + 32 * g);
     }
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float* s = scales + (int64_t)min(n0 + 16 * t + 4 * g + i, N - 1) * groups;
+        const float* s = scales + (int64_t)wmix_row<GLU>(tile0 + t, 4 * g + i, N) * groups;
         if (G == 128 && groups % 4 == 0) {
           sc[t][i] = *reinterpret_cast<const f32x4*>(s + 4 * run);
         } else {
@@ -347,12 +384,107 @@ __global__ __launch_bounds__(64 * NW, MW) void wmix_skinny_kernel(const bf16* __
     for (int m = 0; m < MT; ++m) {
 #pragma unroll
       for (int v = 0; v < NW - 1; ++v) acc[t][m] += red[v][t][m][lane];
-      const int row = 16 * m + r, n = n0 + 16 * t + 4 * g;
-      if (row >= M) continue;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (n + i < N) C[(int64_t)row * N + n + i] = (bf16)(acc[t][m][i] + (bias ? (float)bias[n + i] : 0.f));
+      wmix_store<GLU>(acc[t][m], tile0 + t, 16 * m + r, g, lane, bias, C, M, N, act);
     }
+}
+
+// The same for fp6 and many weight rows, with A resident. At 8 rows A is more bytes of loads than the packed weights (2
+// against 0.75 a code), and every workgroup above loads all of it: [28672, 4096] 37.4 us, 2.5 TB/s. Here a workgroup of 16
+// waves stays on its CU: A lies in LDS in the order of the products (MP = its rows rounded up to 4, 8 or 16), RW waves
+// share a tile's K in runs of 512, and while a tile's sums are reduced the other waves' next runs are on their way. 2 / 8 /
+// 16 rows: 30.3 / 37.6 / 40.3 -> 25.2 / 26.6 / 28.9 us (3.5 TB/s). int8 and int4 are bound by turning codes into bf16 and
+// gain nothing (8 rows: 38.8 -> 37.8, 27.9 -> 30.2).
+constexpr int kResWaves = 16;
+constexpr int kResTiles = 1024;
+
+template <int FMT, int E, int RW, bool GLU>
+__global__ __launch_bounds__(64 * kResWaves) void wmix_resident_kernel(const bf16* __restrict__ A,
+                                                                       const uint8_t* __restrict__ W,
+                                                                       const float* __restrict__ scales,
+                                                                       const bf16* __restrict__ bias,
+                                                                       bf16* __restrict__ C, int M, int N, int K, int G,
+                                                                       int act, int tiles, int MP) {
+  extern __shared__ __attribute__((aligned(16))) char sm[];  // A: K * MP * 2, sums: [2][waves][64] of 16 bytes
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  constexpr int TG = kResWaves / RW;
+  const int tg = wid / RW, w = wid % RW;
+  const int runs = (K + 511) / 512, groups = K / G;
+  f32x4* red = reinterpret_cast<f32x4*>(sm + (int64_t)K * MP * 2);
+  const int t0 = blockIdx.x * TG, dt = gridDim.x * TG;
+  const int rounds = (tiles - t0 + dt - 1) / dt;  // the same for all waves: every round has one barrier
+  WRaw<FMT> raw[4];
+  f32x4 sc[4];
+  int lt = t0 + tg, lrun = w;  // the wave's next run to load
+  auto load = [&]() {
+    if (lt >= tiles || lrun >= runs) return;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      raw[c] = load_w<FMT>(W, wmix_row<GLU>(lt, r, N), K, min(512 * lrun + 128 * c, K - 128) + 32 * g);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* s = scales + (int64_t)wmix_row<GLU>(lt, 4 * g + i, N) * groups;
+      if (G == 128 && groups % 4 == 0) {
+        sc[i] = *reinterpret_cast<const f32x4*>(s + 4 * lrun);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) sc[i][c] = s[min(512 * lrun + 128 * c, K - 128) / G];
+      }
+    }
+    lrun += RW;
+    if (lrun >= runs) {
+      lrun = w;
+      lt += dt;
+    }
+  };
+  load();
+  // piece p of A: row p % MP, 8 columns of lane group (p / MP) % 4 for product (p / 4 MP) % 4 of 128-chunk p / 16 MP
+  for (int i = wid; i < K * MP / 512; i += kResWaves) {
+    const int p = 64 * i + lane, k = 128 * (p / (16 * MP)) + 32 * ((p / MP) & 3) + 8 * ((p / (4 * MP)) & 3);
+    __builtin_amdgcn_global_load_lds(
+        (const __attribute__((address_space(1))) void*)(A + (int64_t)min(p % MP, M - 1) * K + k),
+        (__attribute__((address_space(3))) void*)(sm + i * 1024), 16, 0, 0);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  __syncthreads();
+  const char* xs = sm + (g * MP + (r & (MP - 1))) * 16;
+  for (int round = 0, t = t0 + tg; round < rounds; ++round, t += dt) {
+    f32x4 acc{};
+    if (t < tiles) {
+      for (int run = w; run < runs; run += RW) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          if (512 * run + 128 * c >= K) break;  // wave-uniform
+          bf16x8 f[4];
+          codes<FMT, E>(raw[c], f);
+          f32x4 s{};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const bf16x8 x = *reinterpret_cast<const bf16x8*>(xs + (16 * (4 * run + c) + 4 * j) * MP * 16);
+            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[j], x, s, 0, 0, 0);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[i] += s[i] * sc[i][c];
+        }
+        load();
+      }
+    }
+    f32x4* rb = red + (round & 1) * kResWaves * 64;
+    rb[wid * 64 + lane] = acc;
+    __syncthreads();
+    if (t < tiles && w == round % RW) {
+      f32x4 s = rb[tg * RW * 64 + lane];
+#pragma unroll
+      for (int v = 1; v < RW; ++v) s += rb[(tg * RW + v) * 64 + lane];
+      wmix_store<GLU>(s, t, r, g, lane, bias, C, M, N, act);
+    }
+  }
+}
+
+// rows of A the resident kernel makes room for, and its LDS (0: it does not take the size)
+int resident_rows(int M) { return M <= 4 ? 4 : (M <= 8 ? 8 : 16); }
+size_t resident_bytes(int M, int K) {
+  const size_t b = (size_t)K * resident_rows(M) * 2 + 2 * kResWaves * 1024;
+  return M <= 16 && b <= 160 * 1024 ? b : 0;
 }
 
 int pick_mb(int M) { return M <= 32 ? 1 : 2; }
@@ -415,31 +547,58 @@ HDS_EXPORT int hds_wmix_gemm(const void* A, const void* W, const float* scales, 
   return hipGetLastError();
 }
 
-// The same product for few rows as a stream of packed weights (wmix_skinny_kernel): 1 <= M <= 16, fp6 up to 32. K and G
-// multiples of 128, A 16-byte aligned.
+// The same product for few rows as a stream of packed weights (wmix_skinny_kernel, wmix_resident_kernel): 1 <= M <= 16, fp6
+// up to 32. K and G multiples of 128, A 16-byte aligned. glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu) for
+// W = [gate; up] of 2 N rows (M <= 16, no bias).
 HDS_EXPORT int hds_wmix_skinny(const void* A, const void* W, const float* scales, const void* bias, void* C, int M, int N,
-                               int K, int G, int fmt, int ebits, hipStream_t st) {
-  if (M < 1 || M > (fmt == 2 ? 32 : 16) || N < 1 || K < 128 || K % 128 || G < 128 || G % 128 || K % G)
+                               int K, int G, int fmt, int ebits, int glu, hipStream_t st) {
+  if (M < 1 || M > (fmt == 2 && !glu ? 32 : 16) || N < 1 || K < 128 || K % 128 || G < 128 || G % 128 || K % G || glu < 0 ||
+      glu > 3 || (glu && bias) || (glu && N > (1 << 29)))
     return hipErrorInvalidValue;
-  auto launch = [&](auto kern, int rows, int waves) {
-    hipLaunchKernelGGL(kern, dim3((N + rows - 1) / rows), dim3(64 * waves), 0, st, (const bf16*)A, (const uint8_t*)W,
-                       scales, (const bf16*)bias, (bf16*)C, M, N, K, G);
+  const int tiles = (N + (glu ? 7 : 15)) / (glu ? 8 : 16);
+  auto launch = [&](auto kern, int nt, int waves) {
+    hipLaunchKernelGGL(kern, dim3((tiles + nt - 1) / nt), dim3(64 * waves), 0, st, (const bf16*)A, (const uint8_t*)W,
+                       scales, (const bf16*)bias, (bf16*)C, M, N, K, G, glu - 1);
+    return hipGetLastError();
   };
+  auto resident = [&](auto kern, int rw) {
+    const int wg = (tiles + kResWaves / rw - 1) / (kResWaves / rw);
+    const size_t lds = resident_bytes(M, K);
+    const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kern, dim3(wg < 256 ? wg : 256), dim3(64 * kResWaves), lds, st, (const bf16*)A, (const uint8_t*)W,
+                       scales, (const bf16*)bias, (bf16*)C, M, N, K, G, glu - 1, tiles, resident_rows(M));
+    return hipGetLastError();
+  };
+  // A resident from four tiles a CU on, where it fits: [16384, 4096], 8 rows 20.8 -> 16.8 us, [32768, 2048] 21.2 -> 15.8,
+  // [27648, 5120] 53 -> 33, [16384, 7168] 37.5 -> 25.6; at [12288, 4096] 2 / 8 / 16 rows 13.8 / 16.2 / 21.0 -> 15.0 / 16.3
+  // / 18.5, at [8192, 4096] level: the last round of tiles and the way of A into LDS.
+  const bool res = fmt == 2 && resident_bytes(M, K) != 0 && tiles >= kResTiles;
   // From nine rows on two tiles of weight rows share what is read of A ([28672, 4096], 16 rows: fp6 48 -> 41 us), where
-  // enough workgroups remain. Short sums on many rows: four waves a workgroup (fp6, 8 rows 40 -> 38 us), otherwise eight
-  // ([4096, 14336] 27 -> 22 us).
-#define HDS_WS(F, E)                                                                                       \
-  do {                                                                                                     \
-    if (M > 8 && M <= 16 && N >= 32 * 512) launch(wmix_skinny_kernel<F, E, 2, 1, 4, 3>, 32, 4);            \
-    else if (M <= 16 && K <= 4096 && N >= 16 * 384) launch(wmix_skinny_kernel<F, E, 1, 1, 4, 1>, 16, 4);   \
-    else if (M <= 16) launch(wmix_skinny_kernel<F, E, 1, 1, 8, 1>, 16, 8);                                 \
-    else if constexpr (F == kFp6) launch(wmix_skinny_kernel<F, E, 1, 2, 8, 1>, 16, 8);                     \
+  // enough workgroups remain. Short sums on many rows: four waves a workgroup, otherwise eight ([4096, 14336] fp6, 8 rows 27
+  // -> 22 us).
+#define HDS_WS(F, E, GL)                                                                                            \
+  do {                                                                                                              \
+    if constexpr (F == kFp6) {                                                                                      \
+      if (res && (K + 511) / 512 % 8 == 0) return resident(wmix_resident_kernel<F, E, 8, GL>, 8);                   \
+      if (res) return resident(wmix_resident_kernel<F, E, 4, GL>, 4);                                               \
+    }                                                                                                               \
+    if (M > 8 && M <= 16 && tiles >= 2 * 512) return launch(wmix_skinny_kernel<F, E, 2, 1, 4, 3, GL>, 2, 4);        \
+    if (M <= 16 && K <= 4096 && tiles >= 384) return launch(wmix_skinny_kernel<F, E, 1, 1, 4, 1, GL>, 1, 4);        \
+    if (M <= 16) return launch(wmix_skinny_kernel<F, E, 1, 1, 8, 1, GL>, 1, 8);                                     \
+    if constexpr (F == kFp6 && !GL) return launch(wmix_skinny_kernel<F, E, 1, 2, 8, 1, false>, 1, 8);               \
+    return hipErrorInvalidValue;                                                                                    \
   } while (0)
-  if (fmt == 0) HDS_WS(kInt8, 0);
-  else if (fmt == 1) HDS_WS(kInt4, 0);
-  else if (fmt == 2 && ebits == 3) HDS_WS(kFp6, 3);
-  else if (fmt == 2 && ebits == 2) HDS_WS(kFp6, 2);
-  else return hipErrorInvalidValue;
+#define HDS_WSG(F, E)          \
+  do {                         \
+    if (glu) HDS_WS(F, E, true); \
+    HDS_WS(F, E, false);       \
+  } while (0)
+  if (fmt == 0) HDS_WSG(kInt8, 0);
+  if (fmt == 1) HDS_WSG(kInt4, 0);
+  if (fmt == 2 && ebits == 3) HDS_WSG(kFp6, 3);
+  if (fmt == 2 && ebits == 2) HDS_WSG(kFp6, 2);
+#undef HDS_WSG
 #undef HDS_WS
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }

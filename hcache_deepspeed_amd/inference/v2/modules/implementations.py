@@ -31,7 +31,7 @@ from ....ops.output_norm import (PairSum, embed_rows, padded, residual_norm, rms
                                  stream_norm, sum_experts)
 from ....ops.paged import (HeadShape, head_attention, head_blocks_ok, kv_rope_scatter, make_head_plan,
                            paged_attention, paged_attention_portions, portions_ok)
-from ....ops.quantizer import fp6_linear, int_linear, quantize, quantize_minifloat
+from ....ops.quantizer import fp6_linear, int_linear, packed_glu, quantize, quantize_minifloat
 from ....ops.rope import rope_tables
 from .interfaces import (DSEmbeddingBase, DSEmbeddingRegistry, DSExpertLayerBase, DSExpertLayerRegistry, DSGatedMLPBase,
                          DSGatedMLPRegistry, DSInputNormBase, DSInputNormRegistry, DSLinearBase, DSLinearRegistry,
@@ -118,6 +118,13 @@ class _PackedWeight:
         return self.q.numel() * self.q.element_size() + self.scales.numel() * 4
 
 
+def _packed_glu(c, x, w, b, fmt):
+    """A gated projection of few rows with its activation in one kernel, or None."""
+    if b is not None or not c.activation.endswith("_glu"):
+        return None
+    return packed_glu(x, w.q, w.scales, w.out_features // 2, w.in_features, w.group_size, fmt, c.activation[:-4])
+
+
 def _group(c, in_features):
     g = c.group_size
     while in_features % g:
@@ -146,6 +153,9 @@ class QuantizedWf6Af16Linear(DSLinearBase):
         return _PackedWeight(q, s, out_f, in_f, g)
 
     def forward(self, x, w, b=None):
+        y = _packed_glu(self._config, x, w, b, "fp6")
+        if y is not None:
+            return y
         y = fp6_linear(x, w.q, w.scales, w.out_features, w.in_features, w.group_size, 2)
         return _act_tail(y, b, self._config.activation)
 
@@ -174,6 +184,9 @@ class QuantizedIntLinear(DSLinearBase):
         return _PackedWeight(q, s, out_f, in_f, g)
 
     def forward(self, x, w, b=None):
+        y = _packed_glu(self._config, x, w, b, self._config.quantization_mode)
+        if y is not None:
+            return y
         y = int_linear(x, w.q, w.scales, w.out_features, w.in_features, w.group_size, self._bits())
         return _act_tail(y, b, self._config.activation)
 

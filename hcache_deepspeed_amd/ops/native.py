@@ -121,7 +121,7 @@ _KERNEL_SIGS = {
     "hds_wmix_splits": "iii",
     "hds_wmix_supported": "iiii",
     "hds_paged_prefill": "pl" + "p" + "pl" + "pi" + "pp" + "iiii" + "f" + "i" + "s",
-    "hds_wmix_skinny": "ppppp" + "iiiiii" + "s",
+    "hds_wmix_skinny": "ppppp" + "iiiiiii" + "s",
     "hds_wmix_gemm": "pppppp" + "iiiiii" + "s",
     "hds_token_gather": "i" + "ppp" + "iiii" + "s",
     "hds_token_scatter": "i" + "ppp" + "iiii" + "s",

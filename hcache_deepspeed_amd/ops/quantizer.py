@@ -170,13 +170,13 @@ def wmix_gemm(x2, q_weight, scales, out_features, in_features, group_size, fmt, 
     return y
 
 
-def _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, fmt, ebits=3, bias=None):
+def _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, fmt, ebits=3, bias=None, glu=0):
     """The packed-weight stream for few rows (csrc/kernels/wmix_gemm.hip ``wmix_skinny_kernel``), or None where it does not
     apply. It wins up to 16 rows, with fp6 up to 32 ([28672, 4096], 24 rows: fp6 57 us against the tile kernel's 78, int8
     61 against 50), with int8 from the second row on (one row: 36.5 us against the GEMV's 34.7, two 36.5 against 39)."""
     M = x2.shape[0]
     if (_needs_grad(x2) or not native.use_native(x2) or x2.dtype != torch.bfloat16 or in_features % 128
-            or group_size % 128 or not (fmt == "int8") < M <= (32 if fmt == "fp6" else 16)):
+            or group_size % 128 or not (fmt == "int8") < M <= (32 if fmt == "fp6" and not glu else 16)):
         return None
     x2 = x2.contiguous()
     if x2.data_ptr() % 16:
@@ -186,9 +186,22 @@ def _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, fm
     y = torch.empty(M, out_features, dtype=torch.bfloat16, device=x2.device)
     native.check(native.kernels().hds_wmix_skinny(x2.data_ptr(), q_weight.data_ptr(), scales.data_ptr(),
                                                   native.ptr(bias), y.data_ptr(), M, out_features, in_features,
-                                                  group_size, {"int8": 0, "int4": 1, "fp6": 2}[fmt], int(ebits),
+                                                  group_size, {"int8": 0, "int4": 1, "fp6": 2}[fmt], int(ebits), int(glu),
                                                   native.stream()), "wmix_skinny")
     return y
+
+
+_GLU_ACTS = {"silu": 1, "gelu_tanh": 2, "relu": 3}
+
+
+def packed_glu(x, q_weight, scales, out_features, in_features, group_size, fmt, act, ebits=3):
+    """act(x . gate^T) * (x . up^T) for a packed [gate; up] of ``out_features`` rows each in one kernel (few rows); None where
+    the packed-weight stream does not apply. The projections are rounded to bf16 first, as the separate kernels store them."""
+    if act not in _GLU_ACTS:
+        return None
+    y = _wmix_skinny(x.reshape(-1, in_features), q_weight, scales, out_features, in_features, group_size, fmt, ebits,
+                     glu=_GLU_ACTS[act])
+    return None if y is None else y.view(*x.shape[:-1], out_features)
 
 
 def int_linear(x, q_weight, scales, out_features, in_features, group_size, bits=8, bias=None):

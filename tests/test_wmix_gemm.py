@@ -58,10 +58,12 @@ def test_wmix_split_k_deterministic():
 
 @pytest.mark.parametrize("fmt", ["int8", "int4", "fp6_e3m2", "fp6_e2m3"])
 @pytest.mark.parametrize("M,N,K,G", [(1, 16, 128, 128), (8, 1000, 640, 128), (9, 16390, 512, 256), (16, 6160, 4224, 128),
-                                     (17, 250, 1024, 1024), (32, 48, 14336, 128), (5, 40, 1024, 64)])
+                                     (17, 250, 1024, 1024), (32, 48, 14336, 128), (5, 40, 1024, 64),
+                                     (3, 16380, 640, 128), (8, 16384, 4224, 128), (16, 16390, 4096, 512), (5, 33000, 2048, 128)])
 def test_few_rows_keep_the_weights_exact(fmt, M, N, K, G):
     """The stream of packed weights: tails of the rows and of the 512-wide runs, one and two tiles of weight rows, four and
-    eight waves, scales read by four and one by one; groups of 64 take the older kernels. The codes are exact and the
+    eight waves, scales read by four and one by one, rows resident (from 16,384 weight rows of fp6 on) with one to three
+    rounds of tiles; groups of 64 take the older kernels. The codes are exact and the
     scales 32-bit, so what is left are 32-bit sums (K terms) and the result's rounding."""
     torch.manual_seed(K + M)
     x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
@@ -82,4 +84,31 @@ def test_few_rows_keep_the_weights_exact(fmt, M, N, K, G):
         ref = x.double() @ wd.t()
         stream = G % 128 == 0
     bound = 2**-8 * ref.abs() + 1e-5 * (x.double().abs() @ wd.abs().t()) if stream else 0.02 * ref.abs().max()
+    assert ((y.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("fmt", ["int8", "int4", "fp6"])
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu"])
+@pytest.mark.parametrize("M,N,K,G", [(2, 7, 128, 128), (8, 1000, 640, 128), (16, 4104, 4224, 128), (9, 8200, 4096, 128),
+                                     (5, 8189, 1024, 256)])
+def test_gated_projection_of_packed_weights(fmt, act, M, N, K, G):
+    """act(x . gate^T) * (x . up^T) in one kernel: remainders of a tile's 8 rows, one and two tiles, rows resident."""
+    torch.manual_seed(K + M)
+    x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(2 * N, K, device="cuda", dtype=torch.bfloat16) * K**-0.5
+    if fmt == "fp6":
+        q, s = Q.quantize_minifloat(w.reshape(-1), G, 6, 2)
+        wd = Q.dequantize_minifloat(q, s, G, 6, 2, torch.float32)
+    else:
+        q, s, _ = Q.quantize(w.reshape(-1), G, int(fmt[3:]), True)
+        wd = Q.dequantize(q, s, None, G, int(fmt[3:]), True, torch.float32)
+    wd = wd.view(2 * N, K).double()
+    y = Q.packed_glu(x, q, s, N, K, G, fmt, act)
+    gate, up = (x.double() @ wd.t()).split(N, 1)
+    f = {"silu": torch.nn.functional.silu, "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh"),
+         "relu": torch.relu}[act]
+    ref = f(gate) * up
+    eg, eu = (1e-5 * (x.double().abs() @ wd.abs().t())).split(N, 1)
+    # each factor within half a unit of the last place and its sum's error; |act'| <= 1.13
+    bound = 2**-8 * (1.13 * gate.abs() * up.abs() + 2 * ref.abs()) + 1.13 * (eg * up.abs() + eu * gate.abs()) + 1e-6
     assert ((y.double() - ref).abs() <= bound).all()
