@@ -498,6 +498,7 @@ struct PagedDecodeParams {
   // (token, kv head) to finish merges the splits itself (no combine launch) and resets its counter to 0, so a
   // HIP-graph replay finds it zeroed again.
   int* counters;
+  int tiles;  // the matrix-core kernel: splits are runs of whole tiles of 32 positions
 };
 
 struct DecodeToken {
@@ -511,16 +512,32 @@ __device__ __forceinline__ DecodeToken decode_token(const PagedDecodeParams<T>& 
   return {t, p.tok_seq[t], p.tok_pos[t]};
 }
 
-// this split's keys: an equal share of what the token sees, counted without the gap between the kept keys and the others
+// this split's keys: an equal share of what the token sees, counted without the gap between the kept keys and the others,
+// but no less than one turn of a workgroup: of the launched splits only the first `used` have keys then, and only those
+// are merged
+constexpr int kDecKeys = 64;
+
 struct DecodeKeys {
-  int j0, j1, keep, gap;
+  int j0, j1, keep, gap, used;
   __device__ __forceinline__ int pos(int j) const { return j < keep ? j : j + gap; }
 };
 template <typename T>
 __device__ __forceinline__ DecodeKeys decode_keys(const PagedDecodeParams<T>& p, int pos, int split) {
   const int gap = max(first_key(pos, p.window, p.chunk) - p.keep, 0), n = pos + 1 - gap;
-  const int per = (n + p.splits - 1) / p.splits;
-  return {split * per, min(n, split * per + per), p.keep, gap};
+  const int per = max((n + p.splits - 1) / p.splits, min(n, kDecKeys));
+  return {split * per, min(n, split * per + per), p.keep, gap, (n + per - 1) / per};
+}
+
+// the same in tiles of 32 positions, [a, b) of them for this split
+constexpr int kDecTiles = 4;
+struct DecodeTiles {
+  int a, b, lo, used;
+};
+template <typename T>
+__device__ __forceinline__ DecodeTiles decode_tiles(const PagedDecodeParams<T>& p, int pos, int split) {
+  const int lo = first_key(pos, p.window, 0), first = lo >> 5, n = (pos >> 5) - first + 1;
+  const int per = max((n + p.splits - 1) / p.splits, kDecTiles);
+  return {first + split * per, first + min(n, split * per + per), lo, (n + per - 1) / per};
 }
 
 // factor of head h's weighted value sum whose softmax so far has maximum m and denominator l
@@ -543,12 +560,13 @@ __device__ __forceinline__ float decode_gate(const PagedDecodeParams<T>& p, int 
 }
 
 template <typename T>
-__device__ __forceinline__ void decode_merge_splits(const PagedDecodeParams<T>& p, int b, int h, int d, int row) {
+__device__ __forceinline__ void decode_merge_splits(const PagedDecodeParams<T>& p, int b, int h, int d, int row,
+                                                    int used) {
   const float* pm = p.part_ml + ((int64_t)b * p.hq + h) * p.splits * 2;
   float mm = -INFINITY;
-  for (int s = 0; s < p.splits; ++s) mm = fmaxf(mm, pm[2 * s]);
+  for (int s = 0; s < used; ++s) mm = fmaxf(mm, pm[2 * s]);
   float ll = 0.f, oo = 0.f;
-  for (int s = 0; s < p.splits; ++s) {
+  for (int s = 0; s < used; ++s) {
     const float a = mm == -INFINITY ? 0.f : __expf(pm[2 * s] - mm);
     ll += pm[2 * s + 1] * a;
     oo += p.part_o[(((int64_t)b * p.hq + h) * p.splits + s) * p.dv + d] * a;
@@ -578,6 +596,7 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(PagedDecodeParams<bf1
   const int kl = lane / LPK, c = lane % LPK;
   const DecodeToken tk = decode_token(p, b);
   const DecodeKeys keys = decode_keys(p, tk.pos, split);
+  if (split >= keys.used && p.counters == nullptr) return;  // (nothing is read of it; with counters it has to be counted)
   const int j0 = keys.j0, j1 = keys.j1;
   const PageTable pages(p.block_tables + (int64_t)tk.seq * p.max_blocks, p.block_size, p.max_blocks);
   const int64_t kv_row = (int64_t)p.hkv * (p.dk + p.dv);
@@ -722,8 +741,218 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(PagedDecodeParams<bf1
     __syncthreads();
     if (!s_last) return;
     __threadfence();
-    for (int t = threadIdx.x; t < gn * p.dv; t += 256) decode_merge_splits(p, b, h0 + t / p.dv, t % p.dv, tk.row);
+    for (int t = threadIdx.x; t < gn * p.dv; t += 256) decode_merge_splits(p, b, h0 + t / p.dv, t % p.dv, tk.row, keys.used);
     if (threadIdx.x == 0) p.counters[b * p.hkv + hk] = 0;
+  }
+}
+
+// The same on the matrix cores, for heads of 128 and up to 16 query heads a key head. The kernel above spends about 30
+// vector instructions a (key, query head), two heads' worth of a key's loads, and ends at 3.3 TB/s however its registers and
+// splits are chosen. Here a wave takes 32 positions at a time: K and V rows are loaded whole (16 KB in flight a wave
+// beside the tile it works on), pass through the wave's piece of LDS, and
+//   S^T [32 keys, heads] = K Q^T,   O^T [128, heads] += V^T P^T
+// in mfma_f32_16x16x32_bf16: the column (lane & 15) is the query head in both, so that a score's place in S^T is its place
+// in the P^T operand and rescaling is one factor a lane. P keeps its 32 bits: it enters as the exact sum of three bf16
+// pieces. Tiles are aligned to 32 positions, so one lies in one block (block_size % 32 == 0).
+// ROPE: q, k and v of the token are taken as the projection wrote them. q is rotated on the way into the operand, the
+// split that holds the token's own position rotates k, puts k and v into its tile and appends them to the cache: no
+// launch of its own for that.
+// Measured with the merge, the vector kernel and its merge -> this: 16 sequences of up to 4,000 keys, 32 / 8 heads, 54.0 ->
+// 47.4 us (168 MB; 4 TB/s without the merge), up to 2,000 33.5 -> 28.3; 32 of up to 500 22.6 -> 17.3; one of 1,000, 16 / 4
+// heads, 13.9 -> 8.5, and the rotation's own launch (4 us) saved. More or smaller splits are level or slower (1,024 and
+// 2,048 workgroups: 46.4 and 45.3 us there, but 8 sequences of 1,000 keys 12.3 -> 15.4 and 22.5).
+struct DecodeRope {
+  bf16* cache;
+  const float* cos;  // [pos][rot / 2], null: k is appended as it is
+  const float* sin;
+  int rot;  // 128 or 64
+};
+
+__device__ __forceinline__ void rotate8(bf16x8& a, bf16x8& b, const float* c, const float* s) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float x = (float)a[e], y = (float)b[e];
+    a[e] = (bf16)(x * c[e] - y * s[e]);
+    b[e] = (bf16)(y * c[e] + x * s[e]);
+  }
+}
+
+template <bool ROPE>
+__global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(PagedDecodeParams<bf16> p, DecodeRope rope) {
+  constexpr int D = 128, kTile = 32 * 256;
+  __shared__ __attribute__((aligned(1024))) char smem[4][2 * kTile];
+  __shared__ float s_m[4][16], s_l[4][16];
+  const int split = blockIdx.x, hk = blockIdx.y, b = blockIdx.z, G = p.hq / p.hkv;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, hd = lane & 15, g = lane >> 4;
+  const DecodeToken tk = decode_token(p, b);
+  const DecodeTiles tiles = decode_tiles(p, tk.pos, split);
+  if (split >= tiles.used) return;
+  const int* table = p.block_tables + (int64_t)tk.seq * p.max_blocks;
+  const int64_t kv_row = (int64_t)p.hkv * 2 * D;
+  char* kt = smem[w];
+  char* vt = kt + kTile;
+
+  bf16x8 kr[8], vr[8];
+  auto fetch = [&](int T) {
+    const int pos = 32 * T, blk = __builtin_amdgcn_readfirstlane(table[pos / p.block_size]);
+    const bf16* base = p.cache + ((int64_t)blk * p.block_size + pos % p.block_size) * kv_row + hk * D + 8 * hd;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      kr[i] = *reinterpret_cast<const bf16x8*>(base + (4 * i + g) * kv_row);
+      vr[i] = *reinterpret_cast<const bf16x8*>(base + (4 * i + g) * kv_row + p.hkv * D);
+    }
+  };
+  int T = tiles.a + w;
+  if (T < tiles.b) fetch(T);
+
+  const bf16* row = p.q + (int64_t)tk.row * p.sq;
+  bf16x8 qf[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+    qf[s] = *reinterpret_cast<const bf16x8*>(row + (hk * G + min(hd, G - 1)) * D + 32 * s + 8 * g);
+  if constexpr (ROPE) {
+    if (rope.cos != nullptr) {
+      const float* c = rope.cos + (int64_t)tk.pos * (rope.rot / 2) + 8 * g;
+      const float* s = rope.sin + (int64_t)tk.pos * (rope.rot / 2) + 8 * g;
+      if (rope.rot == 128) {
+        rotate8(qf[0], qf[2], c, s);
+        rotate8(qf[1], qf[3], c + 32, s + 32);
+      } else {
+        rotate8(qf[0], qf[1], c, s);
+      }
+    }
+  }
+
+  float m = -INFINITY, l = 0.f;
+  f32x4 o[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) o[t] = f32x4{};
+  // transposed reads of V: a lane's address is a 4-column piece of rows 4 g .. 4 g + 3 (16 further in the second half)
+  const int vq = hd >> 2, vp = hd & 3;
+  for (; T < tiles.b; T += 4) {
+    const bool edge = 32 * T < tiles.lo || 32 * T + 31 > tk.pos;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 4 * i + g, key = 32 * T + r;
+      if (edge && (key < tiles.lo || key > tk.pos)) vr[i] = bf16x8{};  // whatever lies there, its weight is zero
+      *reinterpret_cast<bf16x8*>(kt + tile_off(r, hd)) = kr[i];
+      *reinterpret_cast<bf16x8*>(vt + tile_off(r, hd)) = vr[i];
+    }
+    if constexpr (ROPE) {
+      if (tk.pos >> 5 == T && lane < 16) {
+        const bf16* kn = row + (p.hq + hk) * D;
+        bf16x8 k = *reinterpret_cast<const bf16x8*>(kn + 8 * lane);
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(kn + p.hkv * D + 8 * lane);
+        const int half = rope.rot / 16;  // lanes from a column to its partner
+        if (rope.cos != nullptr && lane < 2 * half) {
+          const bool first = lane < half;
+          bf16x8 other = *reinterpret_cast<const bf16x8*>(kn + 8 * (first ? lane + half : lane - half));
+          const int64_t at = (int64_t)tk.pos * (rope.rot / 2) + 8 * (first ? lane : lane - half);
+          if (first) rotate8(k, other, rope.cos + at, rope.sin + at);
+          else rotate8(other, k, rope.cos + at, rope.sin + at);
+        }
+        const int r = tk.pos & 31, blk = table[tk.pos / p.block_size];
+        *reinterpret_cast<bf16x8*>(kt + tile_off(r, lane)) = k;
+        *reinterpret_cast<bf16x8*>(vt + tile_off(r, lane)) = v;
+        bf16* dst = rope.cache + ((int64_t)blk * p.block_size + tk.pos % p.block_size) * kv_row + hk * D + 8 * lane;
+        *reinterpret_cast<bf16x8*>(dst) = k;
+        *reinterpret_cast<bf16x8*>(dst + p.hkv * D) = v;
+      }
+    }
+    if (T + 4 < tiles.b) fetch(T + 4);
+    __builtin_amdgcn_sched_barrier(0);
+    float sc[8];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      f32x4 a{};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            *reinterpret_cast<const bf16x8*>(kt + tile_off(16 * u + hd, 4 * s + g)), qf[s], a, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int key = 32 * T + 16 * u + 4 * g + r;
+        sc[4 * u + r] = edge && (key < tiles.lo || key > tk.pos) ? -INFINITY : a[r] * p.scale;
+      }
+    }
+    float mn = m;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mn = fmaxf(mn, sc[i]);
+    mn = fmaxf(mn, __shfl_xor(mn, 16, 64));
+    mn = fmaxf(mn, __shfl_xor(mn, 32, 64));
+    const bool none = mn == -INFINITY;
+    const float alpha = none ? 1.f : __expf(m - mn);
+    m = mn;
+    l *= alpha;
+    bf16x8 p0, p1, p2;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float e = none ? 0.f : __expf(sc[i] - mn);
+      l += e;
+      p0[i] = (bf16)e;
+      const float e1 = e - (float)p0[i];
+      p1[i] = (bf16)e1;
+      p2[i] = (bf16)(e1 - (float)p1[i]);
+    }
+    if (__any(alpha != 1.f)) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) o[t] *= alpha;
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const int ch = 2 * t + (vp >> 1), r0 = 4 * g + vq;
+      const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+          (__attribute__((address_space(3))) bf16x4*)(vt + tile_off(r0, ch) + 8 * (vp & 1)));
+      const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+          (__attribute__((address_space(3))) bf16x4*)(vt + tile_off(r0 + 16, ch) + 8 * (vp & 1)));
+      const bf16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, p0, o[t], 0, 0, 0);
+      o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, p1, o[t], 0, 0, 0);
+      o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, p2, o[t], 0, 0, 0);
+    }
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  // the waves' results: [head][128] floats in each one's piece, in the place of its tiles
+  constexpr int kLd = D + 4;
+  static_assert(16 * kLd * 4 <= 2 * kTile, "LDS");
+  float* mine = reinterpret_cast<float*>(kt);
+  asm volatile("" ::: "memory");  // (behind the last reads of the tiles)
+  if (hd < G) {
+#pragma unroll
+    for (int t = 0; t < 8; ++t) *reinterpret_cast<f32x4*>(mine + hd * kLd + 16 * t + 4 * g) = o[t];
+  }
+  if (lane < 16) {
+    s_m[w][lane] = m;
+    s_l[w][lane] = l;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < G * (D / 4); i += 256) {
+    const int h = i / (D / 4), c = 4 * (i % (D / 4));
+    const float mm = fmaxf(fmaxf(s_m[0][h], s_m[1][h]), fmaxf(s_m[2][h], s_m[3][h]));
+    float ll = 0.f;
+    f32x4 acc{};
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const float a = mm == -INFINITY ? 0.f : __expf(s_m[v][h] - mm);
+      ll += s_l[v][h] * a;
+      acc += *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(smem[v]) + h * kLd + c) * a;
+    }
+    const int head = hk * G + h;
+    if (p.splits == 1) {
+      const float f = decode_factor(p, tk.row, head, mm, ll);
+      bf16x4 out;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[e] = (bf16)(acc[e] * f * decode_gate(p, tk.row, head, c + e));
+      *reinterpret_cast<bf16x4*>(p.o + (int64_t)tk.row * p.so + (int64_t)head * D + c) = out;
+    } else {
+      const int64_t pi = ((int64_t)b * p.hq + head) * p.splits + split;
+      *reinterpret_cast<f32x4*>(p.part_o + pi * D + c) = acc;
+      if (c == 0) {
+        p.part_ml[2 * pi] = mm;
+        p.part_ml[2 * pi + 1] = ll;
+      }
+    }
   }
 }
 
@@ -741,6 +970,7 @@ __global__ __launch_bounds__(256) void paged_plain_kernel(PagedDecodeParams<T> p
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const DecodeToken tk = decode_token(p, b);
   const DecodeKeys keys = decode_keys(p, tk.pos, split);
+  if (split >= keys.used) return;
   const int j0 = keys.j0, j1 = keys.j1;
   const PageTable pages(p.block_tables + (int64_t)tk.seq * p.max_blocks, p.block_size, p.max_blocks);
   const int64_t kv_row = (int64_t)p.hkv * (p.dk + p.dv);
@@ -790,53 +1020,74 @@ __global__ __launch_bounds__(256) void paged_plain_kernel(PagedDecodeParams<T> p
   }
 }
 
-// One workgroup per (token, q head): the split maxima / sums are loaded once, one per thread, into LDS
-// (one memory round trip instead of a dependent walk over the splits), then every thread merges its output column
-// over the splits from partial-o values it requested before the barrier (splits <= 64 <= threads).
-template <typename T>
+// One workgroup per (token, q head). Bound by its chain of round trips, so there is one: every wave reads all splits'
+// statistics, one per lane, beside its share of the partial sums (V columns a thread, the thread groups taking turns at the
+// splits), and only the splits that had keys are read (one sequence, 64 splits of which 16 are used: 8.3 -> 4.8 us).
+template <typename T, int V>
 __global__ __launch_bounds__(256) void paged_decode_combine_kernel(PagedDecodeParams<T> p) {
-  __shared__ float s_m[64], s_l[64];
-  const int bh = blockIdx.x, b = bh / p.hq, h = bh % p.hq;
-  const int d0 = threadIdx.x, dl = min(d0, p.dv - 1);
-  // every load is issued before the barrier: the partial-o column (its addresses need no split stat) and the output
-  // row overlap the stats' round trip instead of following it
+  __shared__ float s_a[64], s_acc[256 * V];
+  const int bh = blockIdx.x, b = bh / p.hq, h = bh % p.hq, lane = threadIdx.x & 63;
+  const DecodeToken tk = decode_token(p, b);
+  const int used = p.tiles ? decode_tiles(p, tk.pos, 0).used : decode_keys(p, tk.pos, 0).used;
+  const int cols = p.dv / V;
+  int L = 1;  // threads across a row: a power of two
+  while (L < cols && L < 256) L *= 2;
+  const int groups = 256 / L, grp = threadIdx.x / L, c0 = threadIdx.x % L;
   const float* po = p.part_o + (int64_t)bh * p.splits * p.dv;
-  float pov[64];
-#pragma unroll
-  for (int s = 0; s < 64; ++s) pov[s] = s < p.splits ? po[(int64_t)s * p.dv + dl] : 0.f;
-  const int row = decode_token(p, b).row;
-  const float gate0 = decode_gate(p, row, h, dl);
   const float* pm = p.part_ml + (int64_t)bh * p.splits * 2;
-  if (d0 < p.splits) {
-    s_m[d0] = pm[2 * d0];
-    s_l[d0] = pm[2 * d0 + 1];
-  }
-  __syncthreads();
-  float mm = -INFINITY;
-  for (int s = 0; s < p.splits; ++s) mm = fmaxf(mm, s_m[s]);
-  float ll = 0.f, oo = 0.f;
+  const float m = lane < used ? pm[2 * lane] : -INFINITY, l = lane < used ? pm[2 * lane + 1] : 0.f;
+  constexpr int U = 8;
+  float v[U][V];  // the first turns' values, on their way with the statistics
 #pragma unroll
-  for (int s = 0; s < 64; ++s) {
-    if (s < p.splits) {
-      const float a = mm == -INFINITY ? 0.f : __expf(s_m[s] - mm);
-      ll += s_l[s] * a;
-      oo += pov[s] * a;
-    }
+  for (int u = 0; u < U; ++u) {
+    const int s = grp + u * groups;
+    if (s < used && c0 < cols) VecN<float, V>::load(po + (int64_t)s * p.dv + c0 * V, v[u]);
   }
-  const float f = decode_factor(p, row, h, mm, ll);
-  T* op = p.o + (int64_t)row * p.so + (int64_t)h * p.dv;
-  if (d0 < p.dv) op[d0] = from_f<T>(oo * f * gate0);
-  for (int d = d0 + blockDim.x; d < p.dv; d += blockDim.x) {  // heads wider than the workgroup
-    oo = 0.f;
-    for (int s = 0; s < p.splits; ++s) oo += po[(int64_t)s * p.dv + d] * (mm == -INFINITY ? 0.f : __expf(s_m[s] - mm));
-    op[d] = from_f<T>(oo * f * decode_gate(p, row, h, d));
+  const float mm = wave_max(m);
+  const float a = mm == -INFINITY ? 0.f : __expf(m - mm);
+  const float ll = wave_sum(l * a);
+  if (threadIdx.x < 64) s_a[lane] = a;
+  __syncthreads();
+  const float f = decode_factor(p, tk.row, h, mm, ll);
+  T* op = p.o + (int64_t)tk.row * p.so + (int64_t)h * p.dv;
+  for (int c = c0; c - c0 < cols; c += L) {
+    float acc[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] = 0.f;
+    const bool on = c < cols;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int s = grp + u * groups;
+      if (s >= used || !on) break;
+      if (c != c0) VecN<float, V>::load(po + (int64_t)s * p.dv + c * V, v[u]);
+#pragma unroll
+      for (int i = 0; i < V; ++i) acc[i] += v[u][i] * s_a[s];
+    }
+    for (int s = grp + U * groups; s < used && on; s += groups) {
+      VecN<float, V>::load(po + (int64_t)s * p.dv + c * V, v[0]);
+#pragma unroll
+      for (int i = 0; i < V; ++i) acc[i] += v[0][i] * s_a[s];
+    }
+    if (groups > 1) {
+#pragma unroll
+      for (int i = 0; i < V; ++i) s_acc[threadIdx.x * V + i] = acc[i];
+      __syncthreads();
+      if (grp == 0)
+        for (int k = 1; k < groups; ++k)
+#pragma unroll
+          for (int i = 0; i < V; ++i) acc[i] += s_acc[(k * L + c0) * V + i];
+    }
+    if (grp == 0 && on) {
+#pragma unroll
+      for (int i = 0; i < V; ++i) op[c * V + i] = from_f<T>(acc[i] * f * decode_gate(p, tk.row, h, c * V + i));
+    }
   }
 }
 
 template <typename T>
 void launch_combine(const PagedDecodeParams<T>& p, int n, hipStream_t st) {
-  const int threads = p.dv >= 256 ? 256 : (p.dv + 63) / 64 * 64;
-  hipLaunchKernelGGL(paged_decode_combine_kernel<T>, dim3(n * p.hq), dim3(threads), 0, st, p);
+  if (p.dv % 4 == 0) hipLaunchKernelGGL((paged_decode_combine_kernel<T, 4>), dim3(n * p.hq), dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((paged_decode_combine_kernel<T, 1>), dim3(n * p.hq), dim3(256), 0, st, p);
 }
 
 template <int LPK>
@@ -847,6 +1098,20 @@ int launch_decode(const PagedDecodeParams<bf16>& p, int n, hipStream_t st) {
   if (G == 1) HDS_DEC(1); else if (G == 2) HDS_DEC(2); else if (G <= 4) HDS_DEC(4); else HDS_DEC(8);
 #undef HDS_DEC
   if (p.splits > 1 && p.counters == nullptr) launch_combine(p, n, st);
+  return hipGetLastError();
+}
+
+// tokens of plain heads of 128: the matrix-core kernel
+bool decode_mfma_ok(const PagedDecodeParams<bf16>& p) {
+  return p.dk == 128 && p.dv == 128 && p.hq / p.hkv <= 16 && p.block_size % 32 == 0 && p.chunk == 0 && p.keep == 0 &&
+         p.softcap == 0.f && p.counters == nullptr && p.sq % 8 == 0 && p.so % 4 == 0 && p.hkv <= 65535;
+}
+
+template <bool ROPE>
+int launch_decode_mfma(PagedDecodeParams<bf16> p, const DecodeRope& rope, int n, hipStream_t st) {
+  p.tiles = 1;
+  hipLaunchKernelGGL((paged_decode_mfma_kernel<ROPE>), dim3(p.splits, p.hkv, n), dim3(256), 0, st, p, rope);
+  if (p.splits > 1) launch_combine(p, n, st);
   return hipGetLastError();
 }
 
@@ -991,12 +1256,12 @@ HDS_EXPORT int hds_paged_decode(int dtype, int plain, const void* q, int64_t sq,
     return launch_plain(PagedDecodeParams<float>{(const float*)q, sq, (const float*)cache, (float*)o, so, part_o,
                                                  part_ml, seq_meta, toks, tok_seq, tok_pos, block_tables, max_blocks,
                                                  block_size, hq, hkv, dk, dv, splits, scale, window, chunk, keep, softcap,
-                                                 sink, (const float*)gate, sg, gw, nullptr}, n, st);
+                                                 sink, (const float*)gate, sg, gw, nullptr, 0}, n, st);
   }
   if (dtype != kBF16) return hipErrorInvalidValue;
   PagedDecodeParams<bf16> p{(const bf16*)q, sq, (const bf16*)cache, (bf16*)o, so, part_o, part_ml, seq_meta, toks,
                             tok_seq, tok_pos, block_tables, max_blocks, block_size, hq, hkv, dk, dv, splits, scale,
-                            window, chunk, keep, softcap, sink, (const bf16*)gate, sg, gw, counters};
+                            window, chunk, keep, softcap, sink, (const bf16*)gate, sg, gw, counters, 0};
   if (plain) {
     p.counters = nullptr;
     return launch_plain(p, n, st);
@@ -1004,9 +1269,29 @@ HDS_EXPORT int hds_paged_decode(int dtype, int plain, const void* q, int64_t sq,
   if (!hds_paged_decode_supported(dk, dv) || sq % 8 || so % 8 || hkv > 65535 / kDecGMax ||
       (counters != nullptr && hq / hkv > kDecGMax))
     return hipErrorInvalidValue;
+  if (decode_mfma_ok(p)) return launch_decode_mfma<false>(p, DecodeRope{}, n, st);
   const int d = dk > dv ? dk : dv;
   if (d <= 32) return launch_decode<4>(p, n, st);
   if (d <= 64) return launch_decode<8>(p, n, st);
   if (d <= 128) return launch_decode<16>(p, n, st);
   return launch_decode<32>(p, n, st);
+}
+
+// A step of n single tokens, one of each sequence, from its projection: qkv [n, hq + 2 hkv, 128] with token stride sq is
+// rotated (cos / sin [pos][rot / 2], rot 128 or 64; null: not rotated), its keys and values are appended to the cache, and o
+// [n, hq, 128] attends to them and all earlier ones. 16-byte aligned rows, block_size % 32 == 0, at most 16 query heads a
+// key head.
+HDS_EXPORT int hds_paged_decode_qkv(const void* qkv, int64_t sq, void* cache, void* o, int64_t so, float* part_o,
+                                    float* part_ml, const int* seq_meta, const int* block_tables, int max_blocks,
+                                    int block_size, int n, int hq, int hkv, int splits, float scale, int window,
+                                    const float* cos_t, const float* sin_t, int rot, hipStream_t st) {
+  if (n <= 0) return 0;
+  if (hq < 1 || hkv < 1 || hq % hkv || splits < 1 || splits > 64 || n > 65535 || window < 0 || seq_meta == nullptr ||
+      (cos_t == nullptr) != (sin_t == nullptr) || (rot != 128 && rot != 64) || (splits > 1 && (!part_o || !part_ml)))
+    return hipErrorInvalidValue;
+  PagedDecodeParams<bf16> p{(const bf16*)qkv, sq, (const bf16*)cache, (bf16*)o, so, part_o, part_ml, seq_meta, nullptr,
+                            nullptr, nullptr, block_tables, max_blocks, block_size, hq, hkv, 128, 128, splits, scale,
+                            window, 0, 0, 0.f, nullptr, nullptr, 0, 1, nullptr, 0};
+  if (!decode_mfma_ok(p)) return hipErrorInvalidValue;
+  return launch_decode_mfma<true>(p, DecodeRope{(bf16*)cache, cos_t, sin_t, rot}, n, st);
 }

@@ -29,8 +29,8 @@ from ....ops.moe import moe_combine, moe_dispatch, topk_assign, topk_route
 from ....ops.norm import layer_norm, norm_picked, norm_picked_ok, rms_norm
 from ....ops.output_norm import (PairSum, embed_rows, padded, residual_norm, rms_rows, sandwich_norm, softcap_,
                                  stream_norm, sum_experts)
-from ....ops.paged import (HeadShape, head_attention, head_blocks_ok, kv_rope_scatter, make_head_plan,
-                           paged_attention, paged_attention_portions, portions_ok)
+from ....ops.paged import (HeadShape, decode_qkv_ok, head_attention, head_blocks_ok, kv_rope_scatter, make_head_plan,
+                           paged_attention, paged_attention_portions, paged_decode_qkv, portions_ok)
 from ....ops.quantizer import fp6_linear, int_linear, packed_glu, quantize, quantize_minifloat
 from ....ops.rope import rope_tables
 from .interfaces import (DSEmbeddingBase, DSEmbeddingRegistry, DSExpertLayerBase, DSExpertLayerRegistry, DSGatedMLPBase,
@@ -72,8 +72,14 @@ class DSDenseBlockedAttention(DSSelfAttentionBase):
         c = self._config
         T = qkv.shape[0]
         nq, nkv, D = c.n_heads_q, c.n_heads_kv, c.head_size
+        rope = c.positional_embedding_type != "none" and cos is not None
+        if T == batch.current_sequences and getattr(batch, "max_new", 0) == 1 and \
+                decode_qkv_ok(qkv, cache, nq, nkv, cos if rope else None, sin if rope else None, c.rotary_dim):
+            return paged_decode_qkv(qkv, cache, batch.seq_meta, batch.block_tables, nq, nkv, c.scale_factor,
+                                    c.sliding_window, cos if rope else None, sin if rope else None,
+                                    c.rotary_dim).reshape(T, nq * D)
         kv_rope_scatter(qkv, cache, batch.tok_seq, batch.tok_pos, batch.block_tables, cos, sin, nq, nkv,
-                        do_rope=c.positional_embedding_type != "none" and cos is not None, rotary_dim=c.rotary_dim)
+                        do_rope=rope, rotary_dim=c.rotary_dim)
         portions = getattr(batch, "portions", None)
         if portions is not None and portions_ok(qkv[:, :nq], cache, nq, nkv):
             return paged_attention_portions(qkv[:, :nq], cache, *portions, batch, nq, nkv, c.scale_factor,

@@ -159,6 +159,42 @@ def paged_attention(q, cache, atoms, n_atoms, seq_meta, block_tables, n_q, n_kv,
     return o
 
 
+def decode_qkv_ok(qkv, cache, n_q, n_kv, cos, sin, rotary_dim=0):
+    """Does ``paged_decode_qkv`` take this projection [T, n_q + 2 n_kv, D], cache and rotation?"""
+    if not (native.use_native(qkv) and qkv.dtype == torch.bfloat16 and cache.dtype == qkv.dtype and cache.dim() == 5):
+        return False
+    rot = rotary_dim or 128
+    rope_ok = cos is None or (rot in (64, 128) and all(
+        t.dtype == torch.float32 and t.is_contiguous() and t.shape[1] == rot // 2 and t.data_ptr() % 16 == 0
+        for t in (cos, sin)))
+    return (rope_ok and not _MERGE_IN_KERNEL and qkv.shape[2] == 128 and n_q % n_kv == 0 and n_q // n_kv <= 16
+            and qkv.shape[1] == n_q + 2 * n_kv and qkv.stride(2) == 1 and qkv.stride(1) == 128 and qkv.stride(0) % 8 == 0
+            and qkv.data_ptr() % 16 == 0 and cache.is_contiguous() and cache.shape[1] % 32 == 0
+            and tuple(cache.shape[2:]) == (2, n_kv, 128) and cache.data_ptr() % 16 == 0)
+
+
+def paged_decode_qkv(qkv, cache, seq_meta, block_tables, n_q, n_kv, scale, window, cos, sin, rotary_dim=0):
+    """A step of one new token per sequence from its projection: ``kv_rope_scatter`` and ``paged_attention(decode=True)`` in
+    one kernel (and the merge of the key splits). ``cos`` None: no rotation. Returns o [T, n_q, 128]."""
+    T, bs = qkv.shape[0], cache.shape[1]
+    o = torch.empty(T, n_q, 128, device=qkv.device, dtype=qkv.dtype)
+    if T == 0:
+        return o
+    lib, keys = native.kernels(), block_tables.shape[1] * bs
+    splits = lib.hds_paged_decode_splits(T, n_kv, min(keys, window) if window else keys)
+    part_o = part_ml = None
+    if splits > 1:
+        part_o = torch.empty(T * n_q * splits * 128, device=qkv.device, dtype=torch.float32)
+        part_ml = torch.empty(T * n_q * splits * 2, device=qkv.device, dtype=torch.float32)
+    native.check(
+        lib.hds_paged_decode_qkv(qkv.data_ptr(), qkv.stride(0), cache.data_ptr(), o.data_ptr(), n_q * 128,
+                                 native.ptr(part_o), native.ptr(part_ml), seq_meta.data_ptr(), block_tables.data_ptr(),
+                                 block_tables.shape[1], bs, T, n_q, n_kv, splits, float(scale), int(window),
+                                 native.ptr(cos), native.ptr(sin), 128 if cos is None else (rotary_dim or 128),
+                                 native.stream()), "paged_decode_qkv")
+    return o
+
+
 # new tokens of a workgroup of the prefill kernel
 PREFILL_ROWS = 256
 
