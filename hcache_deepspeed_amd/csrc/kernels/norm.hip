@@ -7,8 +7,8 @@
 // forward AND backward exist for both norms, because the training engine uses them.
 //
 // Design (MI355X-first):
-//   * one wave64 per row; the row lives in registers (NV 16-byte vectors per lane,
-//     NV = H/512 for bf16), so x is read from HBM exactly once in forward;
+//   * one to four waves per row (backward: one); the row lives in registers (NV = H/512 16-byte vectors per lane and row,
+//     shared by the row's waves), so x is read from HBM exactly once in forward;
 //   * residual add + norm + store of the new residual happen in one pass
 //     (pre-norm transformer: h = x + r; y = norm(h)) -- one read of x and r,
 //     one write of h and y, instead of three kernels;
@@ -42,77 +42,103 @@ __device__ __forceinline__ PickedRow picked_row(const int* pick, int row, int n_
   return {ok ? r : 0, ok};
 }
 
-template <typename T, typename WT, int NV, bool LN>
+// sum over a row's WPR waves; every wave of the workgroup comes here the same number of times
+template <int WPR>
+__device__ __forceinline__ float row_sum(float v, float* red) {
+  v = wave_sum(v);
+  if constexpr (WPR == 1) return v;
+  const int wid = threadIdx.x >> 6;
+  red[wid] = v;  // (all lanes the same)
+  __syncthreads();
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < WPR; ++k) s += red[wid / WPR * WPR + k];
+  return s;
+}
+
+// WPR waves take a row: four where its vectors divide, else two. One wave a row leaves the latencies of a whole row's loads and
+// stores to it. With a residual, one wave a row -> WPR: 16 rows of 2048 / 4096 / 8192 2.6 / 3.4 / 5.1 -> 2.1 / 2.4 / 2.7 us, 1,024
+// rows 4.0 / 6.4 / 11.2 -> 3.6 / 5.5 / 10.9, 16,384 rows 40.6 / 99 / 196 -> 38.5 / 91 / 181 (at 8,192 rows of up to 2048 3 %
+// behind).
+template <typename T, typename WT, int NV, bool LN, int WPR>
 __global__ __launch_bounds__(256) void norm_fwd_kernel(const T* __restrict__ x, const T* __restrict__ res,
                                                        T* __restrict__ res_out, const WT* __restrict__ w,
                                                        const WT* __restrict__ b, T* __restrict__ y,
                                                        float* __restrict__ stat_mean, float* __restrict__ stat_rstd,
                                                        int rows, int cols, float eps, const int* __restrict__ pick,
                                                        int n_in) {
+  static_assert(NV % WPR == 0, "whole vectors a wave");
+  constexpr int V = NV / WPR;
+  __shared__ float red[2][4];
   const int lane = threadIdx.x & 63;
   const int wid = threadIdx.x >> 6;
-  const int row = blockIdx.x * kRowsPerBlock + wid;
-  if (row >= rows) return;
+  const int row_at = blockIdx.x * (kRowsPerBlock / WPR) + wid / WPR;
+  if (WPR == 1 && row_at >= rows) return;
+  const bool live = row_at < rows;  // (the waves of a workgroup stay together for the sums)
+  const int row = live ? row_at : rows - 1;
+  const int c0 = (wid % WPR * V * 64 + lane) * 8;
   const PickedRow in = picked_row(pick, row, n_in);
   const T* xr = x + (int64_t)in.row * cols;
-  float v[NV][8];
+  float v[V][8], wv[V][8];
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int c = (i * 64 + lane) * 8;
-    Vec8<T>::load(xr + c, v[i]);
-  }
+  for (int i = 0; i < V; ++i) Vec8<T>::load(xr + c0 + i * 512, v[i]);
   if (res != nullptr) {
     const T* rr = res + (int64_t)in.row * cols;
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int c = (i * 64 + lane) * 8;
+    for (int i = 0; i < V; ++i) {
       float r[8];
-      Vec8<T>::load(rr + c, r);
+      Vec8<T>::load(rr + c0 + i * 512, r);
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[i][j] = to_f(from_f<T>(v[i][j] + r[j]));  // round like the unfused add
     }
-    if (res_out != nullptr) {
+    if (res_out != nullptr && live) {
       T* ro = res_out + (int64_t)row * cols;
 #pragma unroll
-      for (int i = 0; i < NV; ++i) Vec8<T>::store(ro + (i * 64 + lane) * 8, v[i]);
+      for (int i = 0; i < V; ++i) Vec8<T>::store(ro + c0 + i * 512, v[i]);
     }
+  }
+  if constexpr (WPR > 1) {  // in front of the barriers; with whole rows a wave the registers are worth more
+#pragma unroll
+    for (int i = 0; i < V; ++i) Vec8<WT>::load(w + c0 + i * 512, wv[i]);
   }
   float mean = 0.f;
   if constexpr (LN) {
     float s = 0.f;
 #pragma unroll
-    for (int i = 0; i < NV; ++i)
+    for (int i = 0; i < V; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) s += v[i][j];
-    mean = wave_sum(s) / (float)cols;
+    mean = row_sum<WPR>(s, red[0]) / (float)cols;
   }
   float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < NV; ++i)
+  for (int i = 0; i < V; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const float d = v[i][j] - mean;
       ss += d * d;
     }
-  const float rstd = in.ok ? rsqrtf(wave_sum(ss) / (float)cols + eps) : NAN;
+  const float sum = row_sum<WPR>(ss, red[1]);
+  const float rstd = in.ok ? rsqrtf(sum / (float)cols + eps) : NAN;
+  if (WPR > 1 && !live) return;
   T* yr = y + (int64_t)row * cols;
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int c = (i * 64 + lane) * 8;
-    float wv[8], o[8];
-    Vec8<WT>::load(w + c, wv);
+  for (int i = 0; i < V; ++i) {
+    const int c = c0 + i * 512;
+    float o[8];
+    if constexpr (WPR == 1) Vec8<WT>::load(w + c, wv[i]);
     if constexpr (LN) {
       float bv[8];
       if (b != nullptr) Vec8<WT>::load(b + c, bv);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = (v[i][j] - mean) * rstd * wv[j] + (b != nullptr ? bv[j] : 0.f);
+      for (int j = 0; j < 8; ++j) o[j] = (v[i][j] - mean) * rstd * wv[i][j] + (b != nullptr ? bv[j] : 0.f);
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = v[i][j] * rstd * wv[j];
+      for (int j = 0; j < 8; ++j) o[j] = v[i][j] * rstd * wv[i][j];
     }
     Vec8<T>::store(yr + c, o);
   }
-  if (lane == 0) {
+  if (lane == 0 && wid % WPR == 0) {
     stat_rstd[row] = rstd;
     if constexpr (LN) stat_mean[row] = mean;
   }
@@ -355,21 +381,20 @@ template <typename T, typename WT, bool LN>
 hipError_t launch_fwd(const void* x, const void* res, void* res_out, const void* w, const void* b, void* y,
                       float* mean, float* rstd, int rows, int cols, float eps, const int* pick, int n_in,
                       hipStream_t st) {
-  dim3 grid((rows + kRowsPerBlock - 1) / kRowsPerBlock), block(256);
-  auto args = [&](auto kern) {
-    hipLaunchKernelGGL(kern, grid, block, 0, st, (const T*)x, (const T*)res, (T*)res_out, (const WT*)w,
-                       (const WT*)b, (T*)y, mean, rstd, rows, cols, eps, pick, n_in);
+  auto args = [&](auto kern, int wpr) {
+    hipLaunchKernelGGL(kern, dim3((rows * wpr + kRowsPerBlock - 1) / kRowsPerBlock), dim3(256), 0, st, (const T*)x,
+                       (const T*)res, (T*)res_out, (const WT*)w, (const WT*)b, (T*)y, mean, rstd, rows, cols, eps, pick, n_in);
   };
   switch (cols) {
-    case 512: args(norm_fwd_kernel<T, WT, 1, LN>); break;
-    case 1024: args(norm_fwd_kernel<T, WT, 2, LN>); break;
-    case 2048: args(norm_fwd_kernel<T, WT, 4, LN>); break;
-    case 3072: args(norm_fwd_kernel<T, WT, 6, LN>); break;
-    case 4096: args(norm_fwd_kernel<T, WT, 8, LN>); break;
-    case 5120: args(norm_fwd_kernel<T, WT, 10, LN>); break;
-    case 6144: args(norm_fwd_kernel<T, WT, 12, LN>); break;
-    case 8192: args(norm_fwd_kernel<T, WT, 16, LN>); break;
-    default: args(norm_fwd_generic<T, WT, LN>); break;
+    case 512: args(norm_fwd_kernel<T, WT, 1, LN, 1>, 1); break;
+    case 1024: args(norm_fwd_kernel<T, WT, 2, LN, 2>, 2); break;
+    case 2048: args(norm_fwd_kernel<T, WT, 4, LN, 4>, 4); break;
+    case 3072: args(norm_fwd_kernel<T, WT, 6, LN, 2>, 2); break;
+    case 4096: args(norm_fwd_kernel<T, WT, 8, LN, 4>, 4); break;
+    case 5120: args(norm_fwd_kernel<T, WT, 10, LN, 2>, 2); break;
+    case 6144: args(norm_fwd_kernel<T, WT, 12, LN, 4>, 4); break;
+    case 8192: args(norm_fwd_kernel<T, WT, 16, LN, 4>, 4); break;
+    default: args(norm_fwd_generic<T, WT, LN>, 1); break;
   }
   return hipGetLastError();
 }

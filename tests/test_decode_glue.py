@@ -128,3 +128,29 @@ def test_graph_after_the_buffer_grew_gpu():
         assert torch.equal(out["graph"], out["eager"]), i
         sizes.add(engs["graph"]._batch._dev_meta.numel())
     assert len(sizes) == 3 and engs["graph"]._model._decode_graphs[2, False].graph is not None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("W", [512, 1024, 2048, 3072, 4096, 5120, 6144, 8192, 648])
+@pytest.mark.parametrize("rows", [1, 2, 3, 5, 130])
+@pytest.mark.parametrize("is_ln,res,dtype,wdtype", [(False, True, torch.bfloat16, torch.bfloat16),
+                                                    (True, True, torch.float32, torch.float32),
+                                                    (True, False, torch.bfloat16, torch.float32)])
+def test_norm_rows_over_waves_gpu(W, rows, is_ln, res, dtype, wdtype):
+    """Rows shared by one, two and four waves, workgroups with a row too many, against 64 bits."""
+    from hcache_deepspeed_amd.ops.norm import layer_norm, rms_norm
+    g = torch.Generator(device="cuda").manual_seed(W + rows)
+    x, r = (torch.randn(rows, W, device="cuda", generator=g).to(dtype) for _ in range(2))
+    w, b = (torch.randn(W, device="cuda", generator=g).to(wdtype) for _ in range(2))
+    r = r if res else None
+    y = layer_norm(x, w, b, 1e-5, r) if is_ln else rms_norm(x, w, 1e-5, r)
+    y, h = y if res else (y, x)
+    want_h = (x.float() + r.float()).to(dtype) if res else x
+    assert torch.equal(h, want_h)
+    hd = want_h.double()
+    m = hd.mean(-1, keepdim=True) if is_ln else 0.0
+    want = (hd - m) * torch.rsqrt(((hd - m)**2).mean(-1, keepdim=True) + 1e-5) * w.double() + (b.double() if is_ln else 0.0)
+    # 32-bit sums of W squares, then one rounding of a product and a sum
+    last = 2**-8 if dtype == torch.bfloat16 else 2**-22
+    mag = want.abs() + (2 * b.double().abs() if is_ln else 0.0)
+    assert ((y.double() - want).abs() <= (last + 2**-19) * mag + 1e-6).all()
