@@ -151,7 +151,7 @@ def routed_experts(x, w, shape, identity=True, act="silu", limit=0.0):
                                        native.ptr(ws), native.ptr(sd), Ns, T, Ns, Ks, code, limit,
                                        native.ptr(weigh_in), st), "experts_skinny")
         return parts
-    tm = lib.hds_experts_gemm_tile(n, out_w, E) if fast else 64
+    tm = lib.hds_experts_gemm_tile() if fast else 64
     max_tiles = n // tm + min(E, n) + 1
     buf = torch.empty(E + 1 + 2 * n + 2 * max_tiles + 1, dtype=torch.int32, device=dev)
     offs, row, token, tile_e, tile_m, n_tiles = buf.split([E + 1, n, n, max_tiles, max_tiles, 1])
@@ -167,9 +167,9 @@ def routed_experts(x, w, shape, identity=True, act="silu", limit=0.0):
         h = torch.empty(n, inter, dtype=x.dtype, device=dev)
         native.check(
             lib.hds_experts_gemm(x.data_ptr(), x.stride(0), token.data_ptr(), T, w13.data_ptr(), h.data_ptr(), inter,
-                                 *plan, tm, n, inter, K, E, 1, code, limit, native.ptr(row_weight), st), "experts_gemm")
+                                 *plan, n, inter, K, E, 1, code, limit, native.ptr(row_weight), st), "experts_gemm")
         native.check(
-            lib.hds_experts_gemm(h.data_ptr(), inter, None, 0, w2.data_ptr(), parts.y.data_ptr(), out_w, *plan, tm, n,
+            lib.hds_experts_gemm(h.data_ptr(), inter, None, 0, w2.data_ptr(), parts.y.data_ptr(), out_w, *plan, n,
                                  out_w, inter, E, 0, 0, 0.0, None, st), "experts_gemm")
     else:
         gu = torch.empty(n, 2 * inter, dtype=x.dtype, device=dev)

@@ -94,3 +94,48 @@ def test_dropless_moe_hip(cuda):
     out = moe_ffn_dropless(x, ex, pos, w, counts, w13, w2, lambda h: glu(h, "silu"))
     ref = _bmm_moe(x.float().cpu(), logits.cpu(), k, w13.float().cpu(), w2.float().cpu())
     torch.testing.assert_close(out.float().cpu(), ref, atol=3e-2, rtol=3e-2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts", [[1], [0, 64, 65, 0, 1, 128], [129, 192, 193, 3], [255, 256, 257, 0], [700, 20, 513],
+                                    [1100, 1030]])
+@pytest.mark.parametrize("N,K", [(128, 128), (384, 256), (256, 1152)])
+@pytest.mark.parametrize("gather,glu", [(False, False), (True, True), (True, False), (False, True)])
+def test_experts_gemm_hip(cuda, counts, N, K, gather, glu):
+    """The serving products over a ready tile list: one to four blocks of 64 rows a tile, several tiles an expert, empty
+    experts, more tile slots than tiles, 256 x 256 tiles from 512 rows an expert on (the last counts; N % 256 == 0)."""
+    from hcache_deepspeed_amd.ops import native
+    lib = native.kernels()
+    E, T, tm = len(counts), sum(counts), lib.hds_experts_gemm_tile()
+    g = torch.Generator(device="cuda").manual_seed(T + N + K)
+    n_src = T + 5 if gather else T
+    x = torch.randn(n_src, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
+    w = (torch.randn(E, (2 if glu else 1) * N, K, device="cuda", generator=g) * K**-0.5).to(torch.bfloat16)
+    src = torch.randint(0, n_src, (T, ), device="cuda", generator=g).to(torch.int32) if gather else None
+    weight = torch.rand(T, device="cuda", generator=g) if glu else None
+    offs = [0]
+    tiles = []
+    for e, c in enumerate(counts):
+        offs.append(offs[-1] + c)
+        tiles += [(e, m) for m in range(0, c, tm)]
+    slots = T // tm + min(E, T) + 1
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")  # noqa: E731
+    pad = [(0, 0)] * (slots - len(tiles))
+    te, tmm = (i32([t[j] for t in tiles + pad]) for j in (0, 1))
+    nt, of = i32([len(tiles)]), i32(offs)
+    y = torch.full((T, N + 8), float("nan"), device="cuda", dtype=torch.bfloat16)
+    native.check(
+        lib.hds_experts_gemm(x.data_ptr(), x.stride(0), native.ptr(src), n_src, w.data_ptr(), y.data_ptr(), N + 8,
+                             of.data_ptr(), te.data_ptr(), tmm.data_ptr(), nt.data_ptr(), slots, T, N, K, E, int(glu), 0,
+                             0.0, native.ptr(weight), native.stream()), "experts_gemm")
+    rows = (x if src is None else x[src.long()]).double()
+    z = torch.cat([rows[offs[e]:offs[e + 1]] @ w[e].double().t() for e in range(E)])
+    mag = torch.cat([rows[offs[e]:offs[e + 1]].abs() @ w[e].double().abs().t() for e in range(E)]) * (2**-24 * 8 * K**0.5)
+    if glu:
+        f = weight.double()[:, None]
+        gate, up = z[:, :N] * f, z[:, N:] * f
+        ref = torch.nn.functional.silu(gate) * up
+        bound = 2**-8 * ref.abs() + 1.13 * f * (mag[:, :N] * up.abs() + mag[:, N:] * gate.abs()) + 1e-5 * ref.abs() + 1e-6
+    else:
+        ref, bound = z, 2**-8 * z.abs() + mag
+    assert ((y[:, :N].double() - ref).abs() <= bound).all() and y[:, N:].isnan().all()
