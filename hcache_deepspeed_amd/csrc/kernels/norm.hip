@@ -7,7 +7,7 @@
 // forward AND backward exist for both norms, because the training engine uses them.
 //
 // Design (MI355X-first):
-//   * one to four waves per row (backward: one); the row lives in registers (NV = H/512 16-byte vectors per lane and row,
+//   * one wave64 per row (two or four for few rows); the row lives in registers (NV = H/512 16-byte vectors per lane,
 //     shared by the row's waves), so x is read from HBM exactly once in forward;
 //   * residual add + norm + store of the new residual happen in one pass
 //     (pre-norm transformer: h = x + r; y = norm(h)) -- one read of x and r,
@@ -23,6 +23,7 @@ using namespace hds;
 namespace {
 
 constexpr int kRowsPerBlock = 4;  // 4 waves per block, one row each per iteration
+constexpr int kFewRows = 64;
 
 // ---------------------------------------------------------------------------------
 // forward
@@ -56,10 +57,8 @@ __device__ __forceinline__ float row_sum(float v, float* red) {
   return s;
 }
 
-// WPR waves take a row: four where its vectors divide, else two. One wave a row leaves the latencies of a whole row's loads and
-// stores to it. With a residual, one wave a row -> WPR: 16 rows of 2048 / 4096 / 8192 2.6 / 3.4 / 5.1 -> 2.1 / 2.4 / 2.7 us, 1,024
-// rows 4.0 / 6.4 / 11.2 -> 3.6 / 5.5 / 10.9, 16,384 rows 40.6 / 99 / 196 -> 38.5 / 91 / 181 (at 8,192 rows of up to 2048 3 %
-// behind).
+// WPR waves take a row. The few rows of a decode step would leave the latencies of a whole row's loads and stores to one wave
+// each: with a residual, 16 rows of 2048 / 4096 / 8192 2.6 / 3.4 / 5.1 us, with four waves a row 2.1 / 2.4 / 2.7.
 template <typename T, typename WT, int NV, bool LN, int WPR>
 __global__ __launch_bounds__(256) void norm_fwd_kernel(const T* __restrict__ x, const T* __restrict__ res,
                                                        T* __restrict__ res_out, const WT* __restrict__ w,
@@ -385,17 +384,25 @@ hipError_t launch_fwd(const void* x, const void* res, void* res_out, const void*
     hipLaunchKernelGGL(kern, dim3((rows * wpr + kRowsPerBlock - 1) / kRowsPerBlock), dim3(256), 0, st, (const T*)x,
                        (const T*)res, (T*)res_out, (const WT*)w, (const WT*)b, (T*)y, mean, rstd, rows, cols, eps, pick, n_in);
   };
+  // Several waves a row up to 64 rows (1,024 rows 4.0 / 6.4 / 11.2 -> 3.6 / 5.5 / 10.9 us, 8,192 19.9 / 42 / 103 -> 20.5 / 39 /
+  // 93): longer steps, the training ones among them, keep the sums of one wave in their order.
+#define HDS_NF(COLS, NV, WPR)                                              \
+  case COLS:                                                               \
+    if (rows <= kFewRows) args(norm_fwd_kernel<T, WT, NV, LN, WPR>, WPR);  \
+    else args(norm_fwd_kernel<T, WT, NV, LN, 1>, 1);                       \
+    break
   switch (cols) {
     case 512: args(norm_fwd_kernel<T, WT, 1, LN, 1>, 1); break;
-    case 1024: args(norm_fwd_kernel<T, WT, 2, LN, 2>, 2); break;
-    case 2048: args(norm_fwd_kernel<T, WT, 4, LN, 4>, 4); break;
-    case 3072: args(norm_fwd_kernel<T, WT, 6, LN, 2>, 2); break;
-    case 4096: args(norm_fwd_kernel<T, WT, 8, LN, 4>, 4); break;
-    case 5120: args(norm_fwd_kernel<T, WT, 10, LN, 2>, 2); break;
-    case 6144: args(norm_fwd_kernel<T, WT, 12, LN, 4>, 4); break;
-    case 8192: args(norm_fwd_kernel<T, WT, 16, LN, 4>, 4); break;
+    HDS_NF(1024, 2, 2);
+    HDS_NF(2048, 4, 4);
+    HDS_NF(3072, 6, 2);
+    HDS_NF(4096, 8, 4);
+    HDS_NF(5120, 10, 2);
+    HDS_NF(6144, 12, 4);
+    HDS_NF(8192, 16, 4);
     default: args(norm_fwd_generic<T, WT, LN>, 1); break;
   }
+#undef HDS_NF
   return hipGetLastError();
 }
 
