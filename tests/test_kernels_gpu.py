@@ -792,6 +792,26 @@ def test_skinny_gemm_matches_fp32(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 5, 128, 132, 2047, 2500])
+@pytest.mark.parametrize("W", [512, 648, 2048])
+@pytest.mark.parametrize("is_ln", [False, True])
+def test_norm_weight_grad_parts(rows, W, is_ln):
+    """One to 512 partial rows (one, a thread's turn, more), columns that do not fill a workgroup, against 64 bits."""
+    from hcache_deepspeed_amd.ops.norm import layer_norm, rms_norm
+    g = torch.Generator(device="cuda").manual_seed(rows + W)
+    x, dy = (torch.randn(rows, W, device="cuda", generator=g) for _ in range(2))
+    w, b = (torch.randn(W, device="cuda", generator=g).requires_grad_() for _ in range(2))
+    y = layer_norm(x, w, b) if is_ln else rms_norm(x, w, 1e-5)
+    y.backward(dy)
+    xd = x.double()
+    m = xd.mean(-1, keepdim=True) if is_ln else 0.0
+    xh = (xd - m) * torch.rsqrt(((xd - m)**2).mean(-1, keepdim=True) + 1e-5)
+    for got, terms in ((w.grad, dy.double() * xh), (b.grad if is_ln else None, dy.double())):
+        if got is not None:  # 32-bit products and sums over the rows
+            assert ((got.double() - terms.sum(0)).abs() <= (2**-24 * (rows**0.5 + 16) * 4) * terms.abs().sum(0) + 1e-6).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("act", [None, "silu", "gelu_tanh", "relu"])
 @pytest.mark.parametrize("M", [2, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("N,K", [(7, 128), (1000, 640), (16, 2048), (4104, 2176), (24, 4224), (4112, 4096)])
