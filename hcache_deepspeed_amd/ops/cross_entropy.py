@@ -108,6 +108,18 @@ def _addmm_f32_(acc, a, b):
     acc.add_(_mm_f32(a, b))
 
 
+def _scaled_grad_(out, dw, scale, accumulate):
+    """out = (out +) dw * scale; dw float32, scale a float32 scalar tensor."""
+    if native.use_native(dw) and out.device == dw.device == scale.device and out.is_contiguous() and dw.is_contiguous() \
+            and out.shape == dw.shape and out.dtype in (torch.bfloat16, torch.float16, torch.float32) \
+            and dw.dtype == torch.float32 and out.data_ptr() % 16 == 0 and dw.data_ptr() % 16 == 0:
+        native.check(native.kernels().hds_scaled_grad(native.dt(out), dw.data_ptr(), scale.data_ptr(), out.data_ptr(),
+                                                      dw.numel(), int(accumulate), native.stream()), "scaled_grad")
+        return out
+    g = dw * scale
+    return out.add_(g) if accumulate else out.copy_(g)
+
+
 class _FusedLinearCEFn(torch.autograd.Function):
 
     @staticmethod
@@ -173,14 +185,14 @@ class _FusedLinearCEFn(torch.autograd.Function):
         gh = (dh * dsum.to(dh.dtype)) if dh is not None else None
         gw = None
         if dw is not None:
-            dw.mul_(dsum.float())
             from ..runtime.zero.linear import write_weight_grad
+            scale = dsum.float()
 
             def put(out, accumulate):  # fp32 accumulator -> the bf16 gradient buffer (one pass)
-                out.add_(dw) if accumulate else out.copy_(dw)
+                _scaled_grad_(out, dw, scale, accumulate)
 
             if not write_weight_grad(ctx.weight, put):
-                gw = dw.to(ctx.wdtype)
+                gw = _scaled_grad_(torch.empty(dw.shape, dtype=ctx.wdtype, device=dw.device), dw, scale, False)
         return gh, gw, None, None, None, None
 
 

@@ -78,6 +78,7 @@ _KERNEL_SIGS = {
     "hds_lamb_multi": "ii" + "pp" + "i" + "p" + "f" * 10 + "pp" + "s",
     "hds_sumsq": "iplpps",
     "hds_clip_coef": "pffpps",
+    "hds_scaled_grad": "i" + "ppp" + "l" + "i" + "s",
     "hds_xent": "i" + "pppp" + "l" + "i" + "l" + "i" + "f" + "i" + "f" + "s",
     "hds_attn_fwd": "p" * 8 + "i" * 7 + "f" + "ii" + "s",
     "hds_attn_bwd": "p" * 13 + "i" * 7 + "f" + "ii" + "s",

@@ -792,6 +792,30 @@ def test_skinny_gemm_matches_fp32(M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("shape,offset", [((1, 1), 0), ((3, 5), 0), ((7, 2056), 8), ((7, 2056), 3), ((4100, 4099), 0)])
+def test_scaled_weight_grad(dtype, accumulate, shape, offset):
+    """The 32-bit LM-head gradient, scaled, into its buffer: bit for bit what scaling and then copying gives (an addition is
+    fused: one rounding of the sum), tails and buffers that are not 16-byte aligned included; the 32-bit one stays as it is."""
+    from hcache_deepspeed_amd.ops.cross_entropy import _scaled_grad_
+    g = torch.Generator(device="cuda").manual_seed(1)
+    n = shape[0] * shape[1]
+    dw = torch.randn(shape, device="cuda", generator=g)
+    kept = dw.clone()
+    out = torch.randn(n + offset, device="cuda", generator=g).to(dtype)[offset:].view(shape)
+    scale = torch.tensor(0.3, device="cuda")
+    exact = dw.double() * scale.double() + (out.double() if accumulate else 0)
+    want = (dw * scale).to(dtype)
+    got = _scaled_grad_(out, dw, scale, accumulate)
+    assert got is out and torch.equal(dw, kept)
+    if not accumulate:
+        assert torch.equal(got, want)
+    half = {torch.bfloat16: 2**-8, torch.float16: 2**-11, torch.float32: 2**-23}[dtype]
+    assert ((got.double() - exact).abs() <= half * exact.abs() + 2**-23 * dw.double().abs() + 2**-24).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rows", [1, 5, 128, 132, 2047, 2500])
 @pytest.mark.parametrize("W", [512, 648, 2048])
 @pytest.mark.parametrize("is_ln", [False, True])
