@@ -300,6 +300,10 @@ def ptr(t):
 
 
 def stream(device=None):
+    """The current stream's handle, asked for at every launch: without the Stream object that ``current_stream`` makes (2.8 us
+    against 0.35 us a call)."""
+    if device is None:
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     return torch.cuda.current_stream(device).cuda_stream
 
 
