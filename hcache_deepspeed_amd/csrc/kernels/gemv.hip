@@ -40,10 +40,10 @@ struct Gather {
   }
 };
 
-template <int MAXM, int R, bool GATHER>
+template <int MAXM, int R>
 __global__ __launch_bounds__(256) void gemv_bf16_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                                         const bf16* __restrict__ bias, bf16* __restrict__ y, int M,
-                                                        int N, int K, int64_t ldx, int64_t ldy, Gather gather) {
+                                                        int N, int K, int64_t ldx, int64_t ldy) {
   const int lane = threadIdx.x & 63;
   const int n0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * R;
   if (n0 >= N) return;
@@ -94,7 +94,6 @@ __global__ __launch_bounds__(256) void gemv_bf16_kernel(const bf16* __restrict__
         float v = wave_sum(acc[r][m]);
         if (lane == 0) {
           if (bias) v += (float)bias[n0 + r];
-          if constexpr (GATHER) v = gather(v, m, n0 + r);
           y[m * ldy + n0 + r] = (bf16)v;
         }
       }
@@ -252,6 +251,126 @@ __global__ __launch_bounds__(256) void gemv_fused_kernel(const bf16* __restrict_
         }
       }
     }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// One row. A wave of the kernels above walks whole weight rows, two pieces at a time: at N = 2048 that is 2 KB on the way a wave
+// and a chain of K / 1024 round trips. Here a workgroup of four waves owns two columns (with GLU their gate and up rows) and
+// the waves take turns at pieces of 512 U along K, so that a wave has all rows' pieces on the way and a chain a quarter as
+// long; the sums meet in LDS once. The pre-norm works as above: its scale is one factor of the finished sums, the squares are
+// summed beside them. Measured before -> now: [2 x 5632, 2048] with norm and GLU 13.1 -> 10.7 us, [3072, 2048] with norm 6.4
+// -> 5.4, [2048, 5632] 6.6 -> 6.0, [2 x 14336, 4096] 45.7 -> 38.6 (6.1 TB/s), [4096, 4096] 8.5 -> 7.4, LM heads [32000, 2048]
+// 27.3 -> 22.4 and [32000, 4096] 47.8 -> 40.6. Four or eight columns a workgroup are level or slower (11.6 and 12.9 us at the
+// first), eight waves too.
+struct OneRow {
+  const bf16* h;      // [K]
+  const bf16* res;    // [K] or null
+  const bf16* gamma;  // [K]: NORM
+  float eps;
+  const bf16* w;
+  const bf16* bias;   // [N] or null
+  bf16* y;            // [N]
+  bf16* r_out;        // [K] or null: h + res
+  bf16* x_out;        // [K] or null: the normed row
+  int N, K, act;
+  float limit;
+};
+
+template <int U, bool NORM, bool GLU, bool GATHER>
+__global__ __launch_bounds__(256) void gemv_row_kernel(OneRow p, Gather gather) {
+  constexpr int R = 2, RR = GLU ? 2 * R : R, S = 4 * 512;
+  __shared__ float red[4][RR + 1];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, n0 = blockIdx.x * R;
+  const bf16* wr[RR];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int n = min(n0 + r, p.N - 1);  // a tail column re-reads column N - 1 (not stored)
+    wr[r] = p.w + (int64_t)n * p.K;
+    if constexpr (GLU) wr[R + r] = p.w + ((int64_t)p.N + n) * p.K;
+  }
+  float acc[RR], ss = 0.f;
+#pragma unroll
+  for (int r = 0; r < RR; ++r) acc[r] = 0.f;
+  for (int k0 = 512 * wid + 8 * lane; k0 < p.K; k0 += S * U) {
+    bf16x8 a[U][RR], x[U], g[U], q[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + u * S < p.K ? k0 + u * S : k0;
+#pragma unroll
+      for (int r = 0; r < RR; ++r) a[u][r] = *reinterpret_cast<const bf16x8*>(wr[r] + k);
+      x[u] = *reinterpret_cast<const bf16x8*>(p.h + k);
+      if constexpr (NORM) {
+        g[u] = *reinterpret_cast<const bf16x8*>(p.gamma + k);
+        if (p.res != nullptr) q[u] = *reinterpret_cast<const bf16x8*>(p.res + k);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u > 0 && k0 + u * S >= p.K) break;
+      bf16x8 o = x[u];
+      if constexpr (NORM) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          float v = (float)x[u][j];
+          if (p.res != nullptr) v = (float)(bf16)(v + (float)q[u][j]);  // round like the unfused add
+          ss += v * v;
+          o[j] = (bf16)(v * (float)g[u][j]);
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < RR; ++r) acc[r] = dot8(o, a[u][r], acc[r]);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RR; ++r) {
+    acc[r] = wave_sum(acc[r]);
+    if (lane == 0) red[wid][r] = acc[r];
+  }
+  if constexpr (NORM) {
+    ss = wave_sum(ss);
+    if (lane == 0) red[wid][RR] = ss;
+  }
+  __syncthreads();
+  auto total = [&](int r) { return red[0][r] + red[1][r] + red[2][r] + red[3][r]; };
+  const float rstd = NORM ? rsqrtf(total(RR) / (float)p.K + p.eps) : 1.f;
+  if ((int)threadIdx.x < R && n0 + (int)threadIdx.x < p.N) {
+    const int n = n0 + threadIdx.x;
+    float v = rstd * total(threadIdx.x);
+    if constexpr (GLU) {
+      const float u = rstd * total(R + threadIdx.x);
+      p.y[n] = (bf16)gated_f((float)(bf16)v, (float)(bf16)u, p.act, p.limit);
+    } else {
+      if (p.bias != nullptr) v += (float)p.bias[n];
+      if constexpr (GATHER) v = gather(v, 0, n);
+      p.y[n] = (bf16)v;
+    }
+  }
+  if (NORM && blockIdx.x == 0 && (p.r_out != nullptr || p.x_out != nullptr)) {
+    for (int c = threadIdx.x * 8; c < p.K; c += 2048) {
+      const bf16x8 r = load_r(p.h, p.res, 0, c);
+      if (p.r_out != nullptr && p.res != nullptr) *reinterpret_cast<bf16x8*>(p.r_out + c) = r;
+      if (p.x_out != nullptr) {
+        const bf16x8 g = *reinterpret_cast<const bf16x8*>(p.gamma + c);
+        bf16x8 o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = (bf16)((float)r[j] * rstd * (float)g[j]);
+        *reinterpret_cast<bf16x8*>(p.x_out + c) = o;
+      }
+    }
+  }
+}
+
+// Two pieces a wave on the way where K has them for all waves and N leaves several rounds of workgroups ([2 x 14336, 4096] 41.9
+// us with one piece, 38.6 with two; [6144, 4096] 12.0 / 12.3, [2 x 5632, 2048] 10.7 / 13.8).
+template <bool NORM, bool GLU, bool GATHER>
+int launch_row(const OneRow& p, const Gather& gather, hipStream_t st) {
+  const dim3 grid((p.N + 1) / 2);
+  if (p.K >= 4096 && p.N >= 12288)
+    hipLaunchKernelGGL((gemv_row_kernel<2, NORM, GLU, GATHER>), grid, dim3(256), 0, st, p, gather);
+  else
+    hipLaunchKernelGGL((gemv_row_kernel<1, NORM, GLU, GATHER>), grid, dim3(256), 0, st, p, gather);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -555,13 +674,19 @@ HDS_EXPORT int hds_gemv_fused_bf16(const void* h, const void* res, const void* g
   if (M < 1 || M > 8 || N < 1 || K < 8 || K % 8 || ldh % 8 || glu < 0 || glu > 6 || glu == 4 || glu == 5) return hipErrorInvalidValue;
   const int act = glu - 1;
   if (gamma == nullptr && (r_out != nullptr || x_out != nullptr || res != nullptr)) return hipErrorInvalidValue;
+  if (M == 1) {
+    const OneRow p{(const bf16*)h, (const bf16*)res, (const bf16*)gamma, eps, (const bf16*)w, nullptr, (bf16*)y,
+                   (bf16*)r_out, (bf16*)x_out, N, K, act, limit};
+    if (gamma != nullptr) return glu ? launch_row<true, true, false>(p, Gather{}, st) : launch_row<true, false, false>(p, Gather{}, st);
+    return glu ? launch_row<false, true, false>(p, Gather{}, st) : hipErrorInvalidValue;  // plain GEMV: hds_gemv_bf16
+  }
   const int R = N >= 8192 ? (glu ? 2 : 4) : (N >= 4096 ? 2 : 1);
 #define HDS_GF(MM, RR, NN, GG)                                                                                   \
   hipLaunchKernelGGL((gemv_fused_kernel<MM, RR, NN, GG>), dim3((N + 4 * RR - 1) / (4 * RR)), dim3(256), 0, st,  \
                      (const bf16*)h, (const bf16*)res, (const bf16*)gamma, eps, (const bf16*)w, (bf16*)y,      \
                      (bf16*)r_out, (bf16*)x_out, act, limit, M, N, K, ldh, ldy)
 #define HDS_GFM(RR, NN, GG)                                                                                    \
-  if (M == 1) HDS_GF(1, RR, NN, GG); else if (M <= 2) HDS_GF(2, RR, NN, GG);                                   \
+  if (M <= 2) HDS_GF(2, RR, NN, GG);                                                                           \
   else if (M <= 4) HDS_GF(4, RR, NN, GG); else HDS_GF(8, RR, NN, GG);
 #define HDS_GFR(NN, GG)                                                                                        \
   if (R == 4) { HDS_GFM(4, NN, GG) } else if (R == 2) { HDS_GFM(2, NN, GG) } else { HDS_GFM(1, NN, GG) }
@@ -582,12 +707,15 @@ HDS_EXPORT int hds_gemv_bf16_supported(int M, int N, int K) { return M >= 1 && M
 HDS_EXPORT int hds_gemv_bf16(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, int64_t ldx,
                              int64_t ldy, hipStream_t st) {
   if (!hds_gemv_bf16_supported(M, N, K) || ldx % 8) return hipErrorInvalidValue;
+  if (M == 1)
+    return launch_row<false, false, false>(OneRow{(const bf16*)x, nullptr, nullptr, 0.f, (const bf16*)w, (const bf16*)bias,
+                                                  (bf16*)y, nullptr, nullptr, N, K, 0, 0.f}, Gather{}, st);
   // R = 4 rows per wave while that still leaves >= 2 waves per SIMD on 256 CUs, else 2 / 1 (parallelism)
 #define HDS_GV(MM, RR)                                                                                        \
-  hipLaunchKernelGGL((gemv_bf16_kernel<MM, RR, false>), dim3((N + 4 * RR - 1) / (4 * RR)), dim3(256), 0, st, \
-                     (const bf16*)x, (const bf16*)w, (const bf16*)bias, (bf16*)y, M, N, K, ldx, ldy, Gather{})
+  hipLaunchKernelGGL((gemv_bf16_kernel<MM, RR>), dim3((N + 4 * RR - 1) / (4 * RR)), dim3(256), 0, st, (const bf16*)x, \
+                     (const bf16*)w, (const bf16*)bias, (bf16*)y, M, N, K, ldx, ldy)
 #define HDS_GVM(RR)                                                                                           \
-  if (M == 1) HDS_GV(1, RR); else if (M <= 2) HDS_GV(2, RR); else if (M <= 4) HDS_GV(4, RR); else HDS_GV(8, RR);
+  if (M <= 2) HDS_GV(2, RR); else if (M <= 4) HDS_GV(4, RR); else HDS_GV(8, RR);
   if (N >= 8192) {
     HDS_GVM(4)
   } else if (N >= 4096) {
@@ -610,8 +738,8 @@ HDS_EXPORT int hds_gather_gemv_bf16(const void* x, const void* w, const void* ta
     return hipErrorInvalidValue;
   const Gather gather{(const bf16*)table, ldt, ids, vocab, act};
   if (M == 1)
-    hipLaunchKernelGGL((gemv_bf16_kernel<1, 1, true>), dim3((N + 3) / 4), dim3(256), 0, st, (const bf16*)x,
-                       (const bf16*)w, (const bf16*)nullptr, (bf16*)y, M, N, K, ldx, ldy, gather);
+    return launch_row<false, false, true>(OneRow{(const bf16*)x, nullptr, nullptr, 0.f, (const bf16*)w, nullptr, (bf16*)y,
+                                                 nullptr, nullptr, N, K, 0, 0.f}, gather, st);
   else
     return launch_skinny<true, false>(x, w, K, ldx, SkinnyOut{nullptr, (bf16*)y, M, N, ldy, 0}, gather, st);
   return hipGetLastError();

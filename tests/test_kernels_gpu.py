@@ -836,6 +836,47 @@ def test_norm_weight_grad_parts(rows, W, is_ln):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N", [1, 2, 7, 300, 12289])
+@pytest.mark.parametrize("K", [8, 512, 520, 2048, 2056, 4096, 4104, 8200])
+@pytest.mark.parametrize("kind", ["plain", "norm", "norm_res", "norm_glu", "glu"])
+def test_one_row_edges(N, K, kind):
+    """The kernel of one row against 64 bits: pieces for some of the waves only, one and two pieces a turn, an odd last
+    column; the new residual bit for bit, the normed row to its rounding."""
+    from hcache_deepspeed_amd.ops.gemv import fused_gemv, gemv, glu_gemv
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    glu = kind.endswith("glu")
+    w = (torch.randn(N * (1 + glu), K, device="cuda", generator=g) * K**-0.5).to(torch.bfloat16)
+    h, r, gm = (torch.randn(n, K, device="cuda", generator=g).to(torch.bfloat16) for n in (1, 1, 1))
+    gamma = gm[0]
+    x, scale = h.double(), 1.0
+    if kind.startswith("norm"):
+        res = r if kind != "norm" else None
+        row = h if res is None else (h.float() + r.float()).to(torch.bfloat16)
+        y, got_r, got_x = fused_gemv(h, w, res, gamma, 1e-5, glu=glu, want_x=True)
+        assert torch.equal(got_r, row)
+        scale = torch.rsqrt((row.double()**2).mean() + 1e-5)
+        xn = row.double() * scale * gamma.double()
+        assert ((got_x.double() - xn).abs() <= (2**-8 + 2**-18) * xn.abs() + 1e-30).all()
+        x = (row.float() * gamma.float()).to(torch.bfloat16).double()
+    elif glu:
+        y = torch.empty(1, N, device="cuda", dtype=torch.bfloat16)
+        assert glu_gemv(h, w, "silu", y)
+    else:
+        b = torch.randn(N, device="cuda", generator=g).to(torch.bfloat16)
+        y = gemv(h, w, b)
+    z = x @ w.double().t() * scale
+    mag = (x.abs() @ w.double().abs().t()) * scale * (2**-24 * (K**0.5 + 16) * 4) + 2**-20 * z.abs()
+    if glu:
+        gate, up = z[:, :N], z[:, N:]
+        ref = torch.nn.functional.silu(gate) * up
+        bound = 2**-8 * (1.13 * gate.abs() * up.abs() + 2 * ref.abs()) + 1.13 * (mag[:, :N] * up.abs() + mag[:, N:] * gate.abs())
+    else:
+        ref = z + b.double() if kind == "plain" else z
+        bound = 2**-8 * ref.abs() + mag
+    assert ((y.double() - ref).abs() <= bound + 1e-6).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("act", [None, "silu", "gelu_tanh", "relu"])
 @pytest.mark.parametrize("M", [2, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("N,K", [(7, 128), (1000, 640), (16, 2048), (4104, 2176), (24, 4224), (4112, 4096)])
