@@ -30,7 +30,8 @@ from ....ops.norm import layer_norm, norm_picked, norm_picked_ok, rms_norm
 from ....ops.output_norm import (PairSum, embed_rows, padded, residual_norm, rms_rows, sandwich_norm, softcap_,
                                  stream_norm, sum_experts)
 from ....ops.paged import (HeadShape, decode_qkv_ok, head_attention, head_blocks_ok, kv_rope_scatter, make_head_plan,
-                           paged_attention, paged_attention_portions, paged_decode_qkv, portions_ok)
+                           paged_attention, paged_decode_qkv)
+from ....ops.paged_prefill import paged_attention_portions, portions_ok
 from ....ops.quantizer import fp6_linear, int_linear, packed_glu, quantize, quantize_minifloat
 from ....ops.rope import rope_tables
 from .interfaces import (DSEmbeddingBase, DSEmbeddingRegistry, DSExpertLayerBase, DSExpertLayerRegistry, DSGatedMLPBase,

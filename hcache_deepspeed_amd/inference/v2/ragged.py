@@ -311,7 +311,7 @@ class RaggedBatchWrapper:
         import ctypes
         import numpy as np
         from ...ops import native
-        from ...ops.paged import make_portions
+        from ...ops.paged_prefill import make_portions
         S, T = len(self._seqs), self.current_tokens
         mb = self.max_blocks
         n_new = np.fromiter((nn for (_, nn, _) in self.seq_meta_host), dtype=np.int32, count=S)

@@ -6,7 +6,8 @@ import types
 import pytest
 import torch
 
-from hcache_deepspeed_amd.ops.paged import DECODE_MAX, make_portions, paged_attention_portions, portions_ok
+from hcache_deepspeed_amd.ops.paged import DECODE_MAX
+from hcache_deepspeed_amd.ops.paged_prefill import make_portions, paged_attention_portions, portions_ok
 
 D = 128
 
