@@ -72,3 +72,40 @@ def test_decode_splits_and_merge(D, nq, nkv, lens, mb):
     got = paged_attention(qkv[:, :nq], cache, None, 0, meta, tables, nq, nkv, scale, decode=True)
     ref = _exact(qkv[:, :nq], cache, tables, lens, nq, nkv, scale, 0)
     assert ((got.double() - ref).abs() <= 2**-8 * ref.abs() + 2e-4).all()
+
+
+@pytest.mark.parametrize("sink", [False, True])
+@pytest.mark.parametrize("gate_width", [0, 1, 128])
+@pytest.mark.parametrize("window", [0, 50])
+@pytest.mark.parametrize("rows", [False, True])
+@pytest.mark.parametrize("splits", [1, 7])
+def test_matrix_core_kernel_against_the_plain_one(sink, gate_width, window, rows, splits):
+    """Every option that the rule for the matrix-core kernel lets through, on both kernels of the same entry point: a sink, a
+    gate a head or an element, a window, one token of each sequence or chosen rows of a step, strided rows."""
+    from hcache_deepspeed_amd.ops import native
+    lib, nq, nkv, D, bs, mb = native.kernels(), 12, 3, 128, 64, 8
+    lens = [1, 40, 64, 333, 500]
+    cache, tables, meta, qkv = _setup(lens, nq, nkv, D, bs, mb, seed=2)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    seq = torch.arange(len(lens), dtype=torch.int32, device="cuda")
+    pos = meta[:, 2].contiguous()
+    kv_rope_scatter(qkv, cache, seq, pos, tables, None, None, nq, nkv, do_rope=False)
+    toks = torch.tensor([4, 0, 3], dtype=torch.int32, device="cuda") if rows else None
+    n = 3 if rows else len(lens)
+    sinks = torch.randn(nq, device="cuda", generator=g) if sink else None
+    gate = torch.randn(len(lens), max(1, nq * gate_width) + 8, device="cuda", generator=g).to(torch.bfloat16) if gate_width else None
+    out = []
+    for plain in (0, 1):
+        o = torch.zeros(len(lens), nq * D + 8, device="cuda", dtype=torch.bfloat16)
+        po = torch.empty(n * nq * splits * D, device="cuda")
+        pm = torch.empty(n * nq * splits * 2, device="cuda")
+        native.check(
+            lib.hds_paged_decode(native.dt(qkv), plain, qkv.data_ptr(), qkv.stride(0), cache.data_ptr(), o.data_ptr(),
+                                 o.stride(0), po.data_ptr(), pm.data_ptr(), None if rows else meta.data_ptr(),
+                                 native.ptr(toks), seq.data_ptr(), pos.data_ptr(), tables.data_ptr(), mb, bs, n, nq, nkv, D,
+                                 D, splits, 0.09, window, 0, 0, 0.0, native.ptr(sinks), native.ptr(gate),
+                                 0 if gate is None else gate.stride(0), max(1, gate_width), None, native.stream()), "decode")
+        out.append(o.float())
+    a, b = out
+    # both sum in 32 bits and round once
+    assert ((a - b).abs() <= 2**-7 * b.abs() + 2e-4).all() and a.abs().sum() > 0
