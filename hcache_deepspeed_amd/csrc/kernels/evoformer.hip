@@ -341,11 +341,12 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_fwd_kernel(EvoParams p, in
     top = fmaxf(top, __shfl_xor(top, 32, 64));
     const float mn = fmaxf(m, top);
     const float alpha = m == -INFINITY ? 0.f : fast_exp2((m - mn) * c);
+    const float ref = mn == -INFINITY ? 0.f : mn;  // no visible key so far: probabilities of zero, not NaN
     m = mn;
     float sum = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = fast_exp2((s[r] - mn) * c);  // (not s c - mn c: a row whose keys all have a mask of -1e9 or below)
+      s[r] = fast_exp2((s[r] - ref) * c);  // (not s c - mn c: a row whose keys all have a mask of -1e9 or below)
       sum += s[r];
     }
     l = l * alpha + sum;  // of this lane's keys; both halves are added at the end
@@ -379,7 +380,8 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_fwd_kernel(EvoParams p, in
     bf16* row = p.out + a.base + (int64_t)myq * a.ld;
 #pragma unroll
     for (int dt = 0; dt < T::DT; ++dt) store_row_block<D>(row, acc[dt], dt, hf, inv);
-    if (hf == 0) p.lse[((int64_t)a.bn * p.H + a.h) * L + myq] = (m * c + log2f(l)) / kLog2e;
+    // (no visible key: infinity, so that the backward's probabilities are zero)
+    if (hf == 0) p.lse[((int64_t)a.bn * p.H + a.h) * L + myq] = l == 0.f ? INFINITY : (m * c + log2f(l)) / kLog2e;
   }
 }
 
@@ -682,7 +684,8 @@ int waves_of(int L, int most) {
   }
 
 // q/k/v/o [B, N, L, H, D] bf16, 16-byte aligned; b1 [B, N, 1, 1, L] or null; b2 [B, 1, H, L, L] or null (bias dtype: 1 =
-// bf16, 0 = fp32); lse [B, N, H, L] fp32 (natural log of the softmax normaliser of the scaled + biased scores).
+// bf16, 0 = fp32); lse [B, N, H, L] fp32 (natural log of the softmax normaliser of the scaled + biased scores). A query whose keys
+// are all masked by minus infinity gives zeros (and no gradients); its lse is plus infinity.
 HDS_EXPORT int hds_evoformer_fwd(const void* q, const void* k, const void* v, const void* b1, const void* b2,
                                  int bias_dtype, void* o, float* lse, int B, int N, int L, int H, int D, float scale,
                                  hipStream_t st) {

@@ -105,3 +105,40 @@ def test_evoformer_edges_hip(cuda, B, N, L, H, D, which, bias_dtype):
     if b2 is not None:  # no atomics in these gradients
         again = torch.autograd.grad(DS4Sci_EvoformerAttention(q, k, v, [b1, b2]), leaves, do)
         assert all(torch.equal(x, y) for x, y in zip(got[1:], again))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bias_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("where", ["mask", "pair"])
+@pytest.mark.parametrize("low", ["inf", "lowest"])
+@pytest.mark.parametrize("L,D,first", [(70, 32, 32), (257, 64, 64), (96, 128, 32), (300, 32, 256)])
+def test_evoformer_leading_keys_masked(cuda, L, D, first, low, where, bias_dtype):
+    """Queries whose first one or several tiles of 32 keys (or of 256, a whole chunk) are masked by minus infinity or the
+    lowest value while later ones are visible, and queries without any visible key, whose result and gradients are zero.
+    Against float64, with the bound of the edge tests."""
+    B, N, H = 1, 3, 2
+    g = torch.Generator(device="cuda").manual_seed(L + D)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    q, k, v, do = (rnd(B, N, L, H, D).bfloat16() for _ in range(4))
+    low = -math.inf if low == "inf" else torch.finfo(bias_dtype).min
+    b1, b2 = torch.zeros(B, N, 1, 1, L, dtype=bias_dtype, device="cuda"), rnd(B, 1, H, L, L).to(bias_dtype)
+    if where == "mask":
+        b1[:, 1, ..., :first] = low
+        b1[:, 2] = -math.inf
+    else:
+        b2[:, :, 0, L // 2:, :first] = low
+        b2[:, :, 1, 3:40] = -math.inf
+    leaves = [t.requires_grad_() for t in (q, k, v, b2)]
+    out = DS4Sci_EvoformerAttention(q, k, v, [b1, b2])
+    got = [out] + list(torch.autograd.grad(out, leaves, do))
+    qh, kh, vh, pair = exact = [t.detach().double().requires_grad_() for t in leaves]
+    s = torch.matmul(qh.transpose(-2, -3), kh.transpose(-2, -3).transpose(-1, -2)) / math.sqrt(D) + b1.double() + pair
+    top = s.detach().amax(-1, keepdim=True)
+    p = torch.exp(s - torch.where(top.isinf(), 0., top))
+    ref = torch.matmul(p / p.sum(-1, keepdim=True).clamp_min(1e-300), vh.transpose(-2, -3)).transpose(-2, -3)
+    want = [ref] + list(torch.autograd.grad(ref, exact, do.double()))
+    if where == "mask":
+        assert not out[:, 2].any() and not got[1][:, 2].any()
+    for x, y in zip(got, want):
+        assert torch.isfinite(x).all()
+        assert (x.double() - y).norm() <= 4 * 2**-8 * y.norm() + 1e-6
