@@ -18,6 +18,8 @@
 // Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): forward 42 us, dQ 51, dK / dV 51, pair gradient 59 + 5
 // (before: one wave a workgroup with operands from global memory and 2-byte reads of V 169 us; the FlashAttention
 // backward kernels with 32-bit atomics into the pair gradient 271 + 1,585 us).
+#include <cmath>
+
 #include "attn_common.h"
 
 using namespace hds;
@@ -80,13 +82,16 @@ struct Tile {
 // ---------------------------------------------------------------------------------------------------------------
 // biases
 // ---------------------------------------------------------------------------------------------------------------
-// They are added to the raw scores, divided by the scale: x = scale * log2(e) * (q . k + bias / scale). bf16 biases go
-// through the matrix cores, which have room: a pair bias tile times the matrix (1 / scale) I, a mask as an outer product
-// with 1 / scale. 1 / scale is cut into bf16 pieces (one for D = 64, three otherwise, which make up all 24 bits), so
+// They are added to the raw scores. The scale is rest * 2^e with rest in [0.5, 1), and a score is rest * log2(e) * (2^e q . k
+// + bias / rest): the power of two goes into the operand that a wave keeps in registers and rounds nothing, and a finite
+// bias of up to 1.7e38 stays finite (divided by the whole scale it would not from 3e37 on: a query whose keys are all
+// masked by -1e38 has its softmax over them). bf16 biases go
+// through the matrix cores, which have room: a pair bias tile times the matrix (1 / rest) I, a mask as an outer product
+// with 1 / rest. 1 / rest is cut into bf16 pieces (one for D = 64, three otherwise, which make up all 24 bits), so
 // that the products are exact. That takes two 16-byte loads a lane and no vector instruction a score, where unpacking
 // and adding took four, and two-byte loads where keys are on the lanes (forward 53 -> 42 us, dQ 58 -> 51, dK / dV
 // 124 -> 51, pair gradient 78 -> 59). Zeros of I meet other keys of the same query only: minus
-// infinity is made the lowest finite value first, which 1 / scale > 1 takes back to minus infinity. fp32 biases are
+// infinity is made the lowest finite value first, which 1 / rest > 1 takes back to minus infinity. fp32 biases are
 // added by vector instructions.
 struct __attribute__((packed, aligned(2))) Eight {  // L may be odd: rows are aligned to their element only
   u32x4 v;
@@ -96,11 +101,11 @@ struct __attribute__((packed, aligned(4))) Four {
 };
 
 template <int D>
-struct Inverse {  // 1 / scale in bf16 pieces, rounded towards zero: all of one sign
+struct Inverse {  // 1 / rest in bf16 pieces, rounded towards zero: all of one sign
   static constexpr int N = D == 64 ? 1 : 3;
   bf16 v[N];
-  __device__ __forceinline__ explicit Inverse(float scale) {
-    float r = 1.f / scale;
+  __device__ __forceinline__ explicit Inverse(float rest) {
+    float r = 1.f / rest;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const float t = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r) & 0xffff0000u);
@@ -110,7 +115,7 @@ struct Inverse {  // 1 / scale in bf16 pieces, rounded towards zero: all of one 
   }
 };
 
-// Fragments of (1 / scale) I, either operand: row or column lane & 31, elements 16 ks + 8 hf ..
+// Fragments of (1 / rest) I, either operand: row or column lane & 31, elements 16 ks + 8 hf ..
 template <int D>
 struct Diagonal {
   bf16x8 f[Inverse<D>::N][2];
@@ -145,7 +150,7 @@ __device__ __forceinline__ u32x4 load_eight(const bf16* row, int k, int L) {
   return __builtin_bit_cast(u32x4, r);
 }
 
-// a mask value per lane (row or column lane & 31) against 1 / scale on the other side
+// a mask value per lane (row or column lane & 31) against 1 / rest on the other side
 template <int D>
 __device__ __forceinline__ bf16x8 spread(bf16 v) {
   bf16x8 f{};
@@ -175,8 +180,8 @@ struct QueryBias<D, bf16> {
   Diagonal<D> eye;
   bf16x8 inv;
   u32x4 seen;  // largest bit patterns met: above 0xff80 is a negative NaN, which finite() hides
-  __device__ __forceinline__ QueryBias(const bf16* m, const bf16* pair, float scale)
-      : b1(m), b2(pair), eye(Inverse<D>(scale)), inv(pieces<D>(Inverse<D>(scale))), seen{} {}
+  __device__ __forceinline__ QueryBias(const bf16* m, const bf16* pair, float rest)
+      : b1(m), b2(pair), eye(Inverse<D>(rest)), inv(pieces<D>(Inverse<D>(rest))), seen{} {}
   template <bool TAIL>
   __device__ __forceinline__ void load_pair(int k0, int L, u32x4 (&f)[2]) const {
 #pragma unroll
@@ -189,8 +194,10 @@ struct QueryBias<D, bf16> {
       for (int i = 0; i < Inverse<D>::N; ++i) s = mfma(eye.f[i][ks], __builtin_bit_cast(bf16x8, finite(f[ks])), s);
     return s;
   }
+  // what the scores start from: the mask, so that beside a huge one all keys' scores round alike
   template <bool TAIL>
-  __device__ __forceinline__ f32x16 add_mask(int k0, int L, f32x16 s) const {
+  __device__ __forceinline__ f32x16 start(int k0, int L) const {
+    f32x16 s{};
     if (TAIL || b1 != nullptr) {
       const int k = k0 + (threadIdx.x & 31);
       bf16 v = b1 != nullptr ? b1[TAIL ? min(k, L - 1) : k] : (bf16)0.f;
@@ -201,7 +208,6 @@ struct QueryBias<D, bf16> {
   }
   template <bool TAIL, bool WATCH = false>
   __device__ __forceinline__ f32x16 add(int k0, int hf, int L, f32x16 s) {
-    s = add_mask<TAIL>(k0, L, s);
     if (b2 != nullptr) {
       u32x4 f[2];
       load_pair<TAIL>(k0, L, f);
@@ -228,7 +234,7 @@ template <int D>
 struct QueryBias<D, float> {
   const float *b1, *b2;
   float r;
-  __device__ __forceinline__ QueryBias(const float* m, const float* pair, float scale) : b1(m), b2(pair), r(1.f / scale) {}
+  __device__ __forceinline__ QueryBias(const float* m, const float* pair, float rest) : b1(m), b2(pair), r(1.f / rest) {}
   template <bool TAIL>
   static __device__ __forceinline__ void row(const float* b, int k0, int hf, int L, float r, f32x16& s) {
 #pragma unroll
@@ -254,6 +260,10 @@ struct QueryBias<D, float> {
     }
     return s;
   }
+  template <bool TAIL>
+  __device__ __forceinline__ f32x16 start(int, int) const {
+    return f32x16{};
+  }
   template <bool TAIL, bool WATCH = false>
   __device__ __forceinline__ f32x16 add(int k0, int hf, int L, f32x16 s) {
     if (b1 != nullptr) row<TAIL>(b1, k0, hf, L, r, s);
@@ -271,7 +281,7 @@ struct EvoParams {
   float* db1;           // [B N, L] or null
   float* part;          // [chunks, B, H, L, L]
   int B, N, L, H;
-  float scale;
+  float scale, rest, power;  // scale = rest * power, see the biases
 };
 
 // Workgroups of one row n next to each other on one XCD: neighbouring heads share cache lines, q blocks share k and v
@@ -305,6 +315,13 @@ __device__ __forceinline__ void load_frags(const bf16* m, int64_t ld, int row, b
 #pragma unroll
   for (int ks = 0; ks < D / 16; ++ks) f[ks] = *reinterpret_cast<const bf16x8*>(r + 16 * ks);
 }
+template <int D>
+__device__ __forceinline__ void times(bf16x8 (&f)[D / 16], float power) {
+#pragma unroll
+  for (int ks = 0; ks < D / 16; ++ks)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[ks][e] = (bf16)((float)f[ks][e] * power);
+}
 
 // ---------------------------------------------------------------------------------------------------------------
 // forward
@@ -318,19 +335,20 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_fwd_kernel(EvoParams p, in
   const Place a = place<D>(p, blocks);
   const int q0 = 32 * (a.blk * nw + w), myq = q0 + j, qc = min(myq, L - 1);
   const bool live = q0 < L;
-  const float c = p.scale * kLog2e;
+  const float c = p.rest * kLog2e;
   bf16x8 qf[T::KS];
   load_frags<D>(p.q + a.base, a.ld, qc, qf);
+  times<D>(qf, p.power);
   f32x16 acc[T::DT];
 #pragma unroll
   for (int dt = 0; dt < T::DT; ++dt) acc[dt] = f32x16{};
   float m = -INFINITY, l = 0.f;  // largest raw score, sum of the exponentials
   QueryBias<D, TB> bias(p.b1 != nullptr ? (const TB*)p.b1 + (int64_t)a.bn * L : nullptr,
-                        p.b2 != nullptr ? (const TB*)p.b2 + ((int64_t)(a.b * p.H + a.h) * L + qc) * L : nullptr, p.scale);
+                        p.b2 != nullptr ? (const TB*)p.b2 + ((int64_t)(a.b * p.H + a.h) * L + qc) * L : nullptr, p.rest);
 
   auto tile = [&](const char* sk, const char* sv, int t0, int k0, auto tail) {
     constexpr bool TAIL = decltype(tail)::value;
-    f32x16 s = f32x16{};
+    f32x16 s = bias.template start<TAIL>(k0, L);
 #pragma unroll
     for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(sk, t0, ks), qf[ks], s);
     s = bias.template add<TAIL, true>(k0, hf, L, s);
@@ -397,9 +415,10 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_dq_kernel(EvoParams p, int
   const Place a = place<D>(p, blocks);
   const int q0 = 32 * (a.blk * nw + w), myq = q0 + j, qc = min(myq, L - 1);
   const bool live = q0 < L;
-  const float c = p.scale * kLog2e;
+  const float c = p.rest * kLog2e;
   bf16x8 qf[T::KS], df[T::KS];
   load_frags<D>(p.q + a.base, a.ld, qc, qf);
+  times<D>(qf, p.power);
   load_frags<D>(p.dout + a.base, a.ld, qc, df);
   const int64_t stat = ((int64_t)a.bn * p.H + a.h) * L;
   float delta = 0.f;
@@ -413,16 +432,16 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_dq_kernel(EvoParams p, int
     delta += __shfl_xor(delta, 32, 64);
     if (live && myq < L && hf == 0) p.delta[stat + myq] = delta;
   }
-  const float lse_raw = p.lse[stat + qc] / p.scale;
+  const float lse_raw = p.lse[stat + qc] / p.rest;
   f32x16 acc[T::DT];
 #pragma unroll
   for (int dt = 0; dt < T::DT; ++dt) acc[dt] = f32x16{};
   QueryBias<D, TB> bias(p.b1 != nullptr ? (const TB*)p.b1 + (int64_t)a.bn * L : nullptr,
-                        p.b2 != nullptr ? (const TB*)p.b2 + ((int64_t)(a.b * p.H + a.h) * L + qc) * L : nullptr, p.scale);
+                        p.b2 != nullptr ? (const TB*)p.b2 + ((int64_t)(a.b * p.H + a.h) * L + qc) * L : nullptr, p.rest);
 
   auto tile = [&](const char* sk, const char* sv, int t0, int k0, auto tail) {
     constexpr bool TAIL = decltype(tail)::value;
-    f32x16 s = f32x16{}, d = f32x16{};
+    f32x16 s = bias.template start<TAIL>(k0, L), d = f32x16{};
 #pragma unroll
     for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(sk, t0, ks), qf[ks], s);
     s = bias.template add<TAIL>(k0, hf, L, s);
@@ -473,14 +492,15 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_dkdv_kernel(EvoParams p, i
   const Place a = place<D>(p, blocks);
   const int k0 = 32 * (a.blk * nw + w), myk = k0 + j, kc = min(myk, L - 1);
   const bool live = k0 < L;
-  const float c = p.scale * kLog2e;
+  const float c = p.rest * kLog2e;
   bf16x8 kf[T::KS], vf[T::KS];
   load_frags<D>(p.k + a.base, a.ld, kc, kf);
+  times<D>(kf, p.power);
   load_frags<D>(p.v + a.base, a.ld, kc, vf);
   const int64_t stat = ((int64_t)a.bn * p.H + a.h) * L;
   const TB mask = p.b1 != nullptr ? ((const TB*)p.b1)[(int64_t)a.bn * L + kc] : (TB)0.f;
   const TB* b2 = p.b2 != nullptr ? (const TB*)p.b2 + (int64_t)(a.b * p.H + a.h) * L * L : nullptr;
-  const Inverse<D> inv(p.scale);
+  const Inverse<D> inv(p.rest);
   const Diagonal<D> eye(inv);
   const bf16x8 one = pieces<D>(inv), maskf = spread<D>((bf16)to_f(mask));
   const bool full = k0 + 32 <= L;
@@ -496,17 +516,17 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_dkdv_kernel(EvoParams p, i
     T::stage(smem + 16384, p.dout + a.base, a.ld, c0, nt, L, nw);
     for (int i = threadIdx.x; i < 32 * nt; i += blockDim.x) {
       const bool ok = c0 + i < L;  // queries past the end: a probability of zero
-      s_lse[i] = ok ? p.lse[stat + c0 + i] / p.scale : INFINITY;
+      s_lse[i] = ok ? p.lse[stat + c0 + i] / p.rest : INFINITY;
       s_delta[i] = ok ? p.delta[stat + c0 + i] : 0.f;
     }
     __syncthreads();
     if (!live) continue;
     for (int t = 0; t < nt; ++t) {
       f32x16 s = f32x16{}, d = f32x16{};
+      if (sizeof(TB) == 2 && p.b1 != nullptr) s = mfma(one, maskf, s);
 #pragma unroll
       for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(smem, 32 * t, ks), kf[ks], s);
       if constexpr (sizeof(TB) == 2) {  // queries down the rows: the pair bias is the left operand, its keys contract
-        if (p.b1 != nullptr) s = mfma(one, maskf, s);
         if (b2 != nullptr) {
           const bf16* row = (const bf16*)b2 + (int64_t)min(c0 + 32 * t + j, L - 1) * L;
           u32x4 f[2];
@@ -522,7 +542,7 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_dkdv_kernel(EvoParams p, i
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int qr = min(c0 + 32 * t + acc_row(r, hf), L - 1);
-          s[r] += (b2 != nullptr ? to_f(b2[(int64_t)qr * L + kc]) + to_f(mask) : to_f(mask)) / p.scale;
+          s[r] += (b2 != nullptr ? to_f(b2[(int64_t)qr * L + kc]) + to_f(mask) : to_f(mask)) / p.rest;
         }
       }
 #pragma unroll
@@ -584,9 +604,9 @@ __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblo
   const int q0 = 32 * (qb * nw + w), myq = q0 + j, qc = min(myq, L - 1);
   if (q0 >= L) return;
   const int n0 = chunk * rows_per, n1 = min(p.N, n0 + rows_per);
-  const float c = p.scale * kLog2e;
+  const float c = p.rest * kLog2e;
   const int64_t ld = (int64_t)p.H * D;
-  QueryBias<D, TB> bias(nullptr, (const TB*)p.b2 + ((int64_t)(b * p.H + h) * L + qc) * L, p.scale);
+  QueryBias<D, TB> bias(nullptr, (const TB*)p.b2 + ((int64_t)(b * p.H + h) * L + qc) * L, p.rest);
   const int kk0 = 32 * kb * kPairTiles;
   f32x16 sum[kPairTiles];
 #pragma unroll
@@ -605,7 +625,8 @@ __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblo
       bf16x8 qf[T::KS], df[T::KS];
       load_frags<D>(p.q + base, ld, qc, qf);
       load_frags<D>(p.dout + base, ld, qc, df);
-      const float lse_raw = p.lse[stat + qc] / p.scale, delta = p.delta[stat + qc];
+      times<D>(qf, p.power);
+      const float lse_raw = p.lse[stat + qc] / p.rest, delta = p.delta[stat + qc];
       if (p.b1 != nullptr) bias.b1 = (const TB*)p.b1 + bn * L;
 #pragma unroll
       for (int t = 0; t < kPairTiles; ++t) {
@@ -613,10 +634,10 @@ __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblo
         bf16x8 kf[T::KS], vf[T::KS];
         load_frags<D>(p.k + base, ld, kr, kf);
         load_frags<D>(p.v + base, ld, kr, vf);
-        f32x16 s = f32x16{}, d = f32x16{};
+        f32x16 s = bias.template start<TAIL>(k0, L), d = f32x16{};
 #pragma unroll
         for (int ks = 0; ks < T::KS; ++ks) s = mfma(kf[ks], qf[ks], s);
-        if constexpr (sizeof(TB) == 2) s = bias.add_pair(pair[t], bias.template add_mask<TAIL>(k0, L, s));
+        if constexpr (sizeof(TB) == 2) s = bias.add_pair(pair[t], s);
         else s = bias.template add<TAIL>(k0, hf, L, s);
 #pragma unroll
         for (int ks = 0; ks < T::KS; ++ks) d = mfma(vf[ks], df[ks], d);
@@ -668,6 +689,13 @@ bool bad_shape(int bias_dtype, int B, int N, int L, int H, int D) {
   return (D != 32 && D != 64 && D != 128) || (bias_dtype != kBF16 && bias_dtype != kF32) || blocks > 0x7fffffff;
 }
 
+void set_scale(EvoParams& p, float scale) {
+  int e;
+  p.scale = scale;
+  p.rest = std::frexp(scale, &e);
+  p.power = std::ldexp(1.f, e);
+}
+
 // Waves of a workgroup: 32 positions each, at most 256 of them (a row's operands are then staged once), evenly spread
 int waves_of(int L, int most) {
   const int tiles = (L + 31) / 32, blocks = (tiles + most - 1) / most;
@@ -693,7 +721,8 @@ HDS_EXPORT int hds_evoformer_fwd(const void* q, const void* k, const void* v, co
   if (bad_shape(bias_dtype, B, N, L, H, D)) return hipErrorInvalidValue;
   EvoParams p{};
   p.q = (const bf16*)q; p.k = (const bf16*)k; p.v = (const bf16*)v; p.b1 = b1; p.b2 = b2; p.out = (bf16*)o; p.lse = lse;
-  p.B = B; p.N = N; p.L = L; p.H = H; p.scale = scale;
+  p.B = B; p.N = N; p.L = L; p.H = H;
+  set_scale(p, scale);
   const int nw = waves_of(L, D == 128 ? kWaves<128> : kWaves<32>), blocks = (L + 32 * nw - 1) / (32 * nw);
 #define HDS_EVO(DD, TT)                                                                                             \
   hipLaunchKernelGGL((evo_fwd_kernel<DD, TT>), dim3(blocks * H * B * N), dim3(64 * nw), 0, st, p, blocks)
@@ -726,7 +755,8 @@ HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, co
   EvoParams p{};
   p.q = (const bf16*)q; p.k = (const bf16*)k; p.v = (const bf16*)v; p.o = (const bf16*)o; p.dout = (const bf16*)dout;
   p.b1 = b1; p.b2 = b2; p.dq = (bf16*)dq; p.dk = (bf16*)dk; p.dv = (bf16*)dv; p.lse = (float*)lse; p.delta = delta;
-  p.db1 = db1; p.part = part; p.B = B; p.N = N; p.L = L; p.H = H; p.scale = scale;
+  p.db1 = db1; p.part = part; p.B = B; p.N = N; p.L = L; p.H = H;
+  set_scale(p, scale);
   const int nw = waves_of(L, D == 128 ? kWaves<128> : kWaves<32>), blocks = (L + 32 * nw - 1) / (32 * nw);
   const dim3 grid(blocks * H * B * N), threads(64 * nw);
 #define HDS_EVO(DD, TT)                                                                                             \

@@ -142,3 +142,19 @@ def test_evoformer_leading_keys_masked(cuda, L, D, first, low, where, bias_dtype
     for x, y in zip(got, want):
         assert torch.isfinite(x).all()
         assert (x.double() - y).norm() <= 4 * 2**-8 * y.norm() + 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bias_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_evoformer_large_finite_mask(cuda, D, bias_dtype):
+    """A finite mask stays finite: a query whose keys are all masked by -1e38, beside which the scores do not count in 32
+    bits, has the mean of the values."""
+    torch.manual_seed(D)
+    q, k, v = (torch.randn(1, 2, 90, 2, D, device=cuda, dtype=torch.bfloat16) for _ in range(3))
+    b1 = torch.zeros(1, 2, 1, 1, 90, dtype=bias_dtype, device=cuda)
+    b1[:, 1] = -1e38
+    out = DS4Sci_EvoformerAttention(q, k, v, [b1, None])
+    torch.testing.assert_close(out[:, :1].float(), _ref(q, k, v, None, None)[:, :1], atol=2e-2, rtol=2e-2)
+    mean = v[:, 1:].double().mean(2, keepdim=True).expand(-1, -1, 90, -1, -1)
+    assert (out[:, 1:].double() - mean).norm() <= 2 * 2**-8 * mean.norm()
