@@ -154,6 +154,8 @@ __device__ __forceinline__ u32x4 load_eight(const bf16* row, int k, int L) {
 template <int D>
 __device__ __forceinline__ bf16x8 spread(bf16 v) {
   bf16x8 f{};
+  // minus infinity as in finite(): a piece of 1 / rest may be zero (NaN stays)
+  if (__builtin_bit_cast(uint16_t, v) == 0xff80u) v = __builtin_bit_cast(bf16, (uint16_t)kLowest);
   if ((threadIdx.x & 63) < 32) {
 #pragma unroll
     for (int i = 0; i < Inverse<D>::N; ++i) f[i] = v;
@@ -689,11 +691,21 @@ bool bad_shape(int bias_dtype, int B, int N, int L, int H, int D) {
   return (D != 32 && D != 64 && D != 128) || (bias_dtype != kBF16 && bias_dtype != kF32) || blocks > 0x7fffffff;
 }
 
-void set_scale(EvoParams& p, float scale) {
+// rest in [0.49, 0.99]: the lowest bf16 value over it is minus infinity. False for a scale that the kernels cannot take: one
+// that is not positive and normal, or with bf16 biases of D = 64 one whose 1 / rest is more than one bf16 piece.
+bool set_scale(EvoParams& p, float scale, int bias_dtype, int D) {
+  if (!std::isnormal(scale) || scale < 0.f) return false;
   int e;
   p.scale = scale;
   p.rest = std::frexp(scale, &e);
+  if (p.rest > 0.99f) {
+    p.rest *= 0.5f;
+    ++e;
+  }
   p.power = std::ldexp(1.f, e);
+  const float inv = 1.f / p.rest;
+  const bool one_piece = (__builtin_bit_cast(uint32_t, inv) & 0xffffu) == 0;
+  return D != 64 || bias_dtype != kBF16 || one_piece || (p.b1 == nullptr && p.b2 == nullptr);
 }
 
 // Waves of a workgroup: 32 positions each, at most 256 of them (a row's operands are then staged once), evenly spread
@@ -713,7 +725,8 @@ int waves_of(int L, int most) {
 
 // q/k/v/o [B, N, L, H, D] bf16, 16-byte aligned; b1 [B, N, 1, 1, L] or null; b2 [B, 1, H, L, L] or null (bias dtype: 1 =
 // bf16, 0 = fp32); lse [B, N, H, L] fp32 (natural log of the softmax normaliser of the scaled + biased scores). A query whose keys
-// are all masked by minus infinity gives zeros (and no gradients); its lse is plus infinity.
+// are all masked by minus infinity gives zeros (and no gradients); its lse is plus infinity. scale > 0; with D = 64 and
+// bf16 biases one over a power of two times at most eight bits (1 / 8 there: 64^-0.5), see set_scale.
 HDS_EXPORT int hds_evoformer_fwd(const void* q, const void* k, const void* v, const void* b1, const void* b2,
                                  int bias_dtype, void* o, float* lse, int B, int N, int L, int H, int D, float scale,
                                  hipStream_t st) {
@@ -722,7 +735,7 @@ HDS_EXPORT int hds_evoformer_fwd(const void* q, const void* k, const void* v, co
   EvoParams p{};
   p.q = (const bf16*)q; p.k = (const bf16*)k; p.v = (const bf16*)v; p.b1 = b1; p.b2 = b2; p.out = (bf16*)o; p.lse = lse;
   p.B = B; p.N = N; p.L = L; p.H = H;
-  set_scale(p, scale);
+  if (!set_scale(p, scale, bias_dtype, D)) return hipErrorInvalidValue;
   const int nw = waves_of(L, D == 128 ? kWaves<128> : kWaves<32>), blocks = (L + 32 * nw - 1) / (32 * nw);
 #define HDS_EVO(DD, TT)                                                                                             \
   hipLaunchKernelGGL((evo_fwd_kernel<DD, TT>), dim3(blocks * H * B * N), dim3(64 * nw), 0, st, p, blocks)
@@ -756,7 +769,7 @@ HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, co
   p.q = (const bf16*)q; p.k = (const bf16*)k; p.v = (const bf16*)v; p.o = (const bf16*)o; p.dout = (const bf16*)dout;
   p.b1 = b1; p.b2 = b2; p.dq = (bf16*)dq; p.dk = (bf16*)dk; p.dv = (bf16*)dv; p.lse = (float*)lse; p.delta = delta;
   p.db1 = db1; p.part = part; p.B = B; p.N = N; p.L = L; p.H = H;
-  set_scale(p, scale);
+  if (!set_scale(p, scale, bias_dtype, D)) return hipErrorInvalidValue;
   const int nw = waves_of(L, D == 128 ? kWaves<128> : kWaves<32>), blocks = (L + 32 * nw - 1) / (32 * nw);
   const dim3 grid(blocks * H * B * N), threads(64 * nw);
 #define HDS_EVO(DD, TT)                                                                                             \

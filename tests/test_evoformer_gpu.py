@@ -158,3 +158,32 @@ def test_evoformer_large_finite_mask(cuda, D, bias_dtype):
     torch.testing.assert_close(out[:, :1].float(), _ref(q, k, v, None, None)[:, :1], atol=2e-2, rtol=2e-2)
     mean = v[:, 1:].double().mean(2, keepdim=True).expand(-1, -1, 90, -1, -1)
     assert (out[:, 1:].double() - mean).norm() <= 2 * 2**-8 * mean.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bias_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,scale", [(32, 0.125), (32, 0.249), (128, 0.3), (64, 0.1), (64, 0.3), (64, 0.0), (32, -0.1)])
+def test_evoformer_kernel_takes_a_scale_or_refuses_it(cuda, D, scale, bias_dtype):
+    """The kernels' entry with other scales than D^-0.5: 1 / scale of one bf16 piece, of three, just above one; a mask of
+    minus infinity; scales that it cannot take are refused (64 columns with bf16 biases hold one piece)."""
+    from hcache_deepspeed_amd.ops import native
+    torch.manual_seed(D)
+    N, L, H = 3, 70, 2
+    q, k, v = (torch.randn(1, N, L, H, D, device=cuda, dtype=torch.bfloat16) for _ in range(3))
+    b1 = torch.zeros(1, N, 1, 1, L, device=cuda, dtype=bias_dtype)
+    b1[:, 1, ..., :40] = -math.inf
+    b2 = torch.randn(1, 1, H, L, L, device=cuda).mul_(100).to(bias_dtype)
+    o, lse = torch.empty_like(q), torch.empty(1, N, H, L, device=cuda)
+    rc = native.kernels().hds_evoformer_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), b1.data_ptr(), b2.data_ptr(),
+                                            native.dt(b1), o.data_ptr(), lse.data_ptr(), 1, N, L, H, D, scale,
+                                            native.stream())
+    if scale <= 0 or (scale == 0.3 and D == 64 and bias_dtype == torch.bfloat16):
+        assert rc != 0
+        return
+    assert rc == 0
+    scale = torch.tensor(scale, dtype=torch.float32).double().item()
+    s = (q.double().transpose(-2, -3) @ k.double().transpose(-2, -3).transpose(-1, -2)) * scale + b1.double() + b2.double()
+    ref = (torch.softmax(s, -1) @ v.double().transpose(-2, -3)).transpose(-2, -3)
+    assert (o.double() - ref).norm() <= 2 * 2**-8 * ref.norm()
+    # 32-bit scores of a few hundred, in units of 1 / scale
+    assert (lse.double() - torch.logsumexp(s, -1)).abs().max() <= 2e-6 * s.abs().nan_to_num(0, 0, 0).max() + 1e-4
