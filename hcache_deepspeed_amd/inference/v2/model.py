@@ -95,7 +95,7 @@ class RaggedTransformer:
         self.kv_cache = None
         self.copy_stream = torch.cuda.Stream(device) if device.type == "cuda" else None
         self._decode_graphs = {}
-        self._graph_pool = None
+        self._graph_pool = self._graph_stream = None
         # HCache latents inside the decode graph (device ring drained every `decode_latent_ring_steps` steps)
         self.decode_graph_latents = _os.environ.get("HDS_V2_DECODE_GRAPH_LATENTS", "1") == "1"
         self.decode_latent_ring_steps = int(_os.environ.get("HDS_V2_LATENT_RING_STEPS", "16"))
@@ -771,7 +771,11 @@ class _DecodeGraph:
 
     def capture(self, model):
         cur = torch.cuda.current_stream()
-        side = torch.cuda.Stream()
+        # one stream for all captures of a model: the graphs share a memory pool, and the caching allocator gives a block
+        # only to the stream that it was made for (so does the library its 76 MB of workspace a stream)
+        if model._graph_stream is None:
+            model._graph_stream = torch.cuda.Stream(model.device)
+        side = model._graph_stream
         side.wait_stream(cur)
         cap = self.ring is not None
         with torch.cuda.stream(side):

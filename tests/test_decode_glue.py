@@ -131,6 +131,33 @@ def test_graph_after_the_buffer_grew_gpu():
 
 
 @pytest.mark.gpu
+def test_graphs_of_several_sizes_share_memory_gpu():
+    """Smaller batch sizes' graphs use the memory that the largest one's capture took: beside their logits and what the
+    captures themselves round up to, nothing is reserved for them."""
+    from hcache_deepspeed_amd.inference.v2.arch import ArchSpec
+    from hcache_deepspeed_amd.inference.v2.engine import InferenceEngineV2, RaggedInferenceEngineConfig
+    H, I, V = 512, 32768, 211  # activations of 3 MB a step
+    g = torch.Generator().manual_seed(0)
+    dev = torch.device("cuda")
+    mat = lambda *s: (torch.randn(*s, generator=g) * s[-1]**-0.5).bfloat16().to(dev)  # noqa: E731
+    one = torch.ones(H, dtype=torch.bfloat16, device=dev)
+    layer = {"ln1.w": one, "ln2.w": one, "qkv.w": mat(4 * 128, H), "o.w": mat(H, 256), "up.w": mat(2 * I, H),
+             "down.w": mat(H, I)}
+    spec = ArchSpec("llama", V, H, 2, 2, 1, 128, I, max_position_embeddings=8192)
+    eng = InferenceEngineV2(spec, {"embed": mat(V, H), "final.w": one, "lm_head.w": mat(V, H), "layers": [layer, layer]},
+                            RaggedInferenceEngineConfig.from_dict(dict(dtype="bf16")), device=dev, num_kv_blocks=40)
+    toks = torch.randint(0, V, (24, 1), generator=g)
+    used = {}
+    for n in range(24, 16, -1):  # (library products, which take a workspace of their own for each stream)
+        for _ in range(3):
+            eng.put(list(range(n)), list(toks[:n]), capture_latents=False)
+        torch.cuda.synchronize()
+        used[n] = torch.cuda.memory_reserved()
+    assert all(eng._model._decode_graphs[n, False].graph is not None for n in used)
+    assert used[17] - used[24] <= 24 << 20, used
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("W", [512, 1024, 2048, 3072, 4096, 5120, 6144, 8192, 648])
 @pytest.mark.parametrize("rows", [1, 2, 3, 5, 130])
 @pytest.mark.parametrize("is_ln,res,dtype,wdtype", [(False, True, torch.bfloat16, torch.bfloat16),
