@@ -333,9 +333,11 @@ __device__ __forceinline__ void gg_flow_tile(char* smem, const bf16* const (&wp)
   issue(cur, 0);
   issue(next, 1);  // KT >= 2
   for (int kt = 0; kt < KT; ++kt) {
-    // this stage has arrived for every wave, and every wave is done with the one before
-    if (kt + 1 < KT) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(P) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    // this stage has arrived for every wave, and every wave is done with the one before: its reads have returned (lgkmcnt;
+    // the compiler may move the products that use them behind this statement), so that the stage after next may
+    // overwrite it
+    if (kt + 1 < KT) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(P) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (kt + 2 < KT) issue(last, kt + 2);
     const char* Xt = cur + 16384;
     if (mg < 2 * NX) {  // wave-uniform

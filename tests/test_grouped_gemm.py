@@ -3,6 +3,9 @@
 Reference test model: tests/unit/inference/v2/kernels/cutlass_ops/test_moe_gemm.py (grouped GEMM with ragged
 per-expert token counts, including empty experts, vs per-expert torch matmuls).
 """
+import pathlib
+import re
+
 import pytest
 import torch
 
@@ -139,3 +142,17 @@ def test_experts_gemm_hip(cuda, counts, N, K, gather, glu):
     else:
         ref, bound = z, 2**-8 * z.abs() + mag
     assert ((y[:, :N].double() - ref).abs() <= bound).all() and y[:, N:].isnan().all()
+
+
+def test_counted_waits_retire_lds_reads():
+    """A statement that waits for loads and joins a barrier, behind which others overwrite what the wave has read from LDS,
+    waits for those reads too: nothing else keeps their use in front of it."""
+    import hcache_deepspeed_amd
+    kernels = pathlib.Path(hcache_deepspeed_amd.__file__).parent / "csrc" / "kernels"
+    found = []
+    for f in sorted(kernels.glob("*.hip")):
+        found += [(f.name, a) for a in re.findall(r'asm volatile\("([^"]*)"', f.read_text())
+                  if "s_waitcnt" in a and "s_barrier" in a]
+    assert [f for f, _ in found].count("grouped_gemm.hip") == 2
+    for f, a in found:
+        assert "lgkmcnt(0)" in a.split("s_barrier")[0], (f, a)
