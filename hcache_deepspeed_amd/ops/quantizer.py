@@ -172,11 +172,12 @@ def wmix_gemm(x2, q_weight, scales, out_features, in_features, group_size, fmt, 
 
 def _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, fmt, ebits=3, bias=None, glu=0):
     """The packed-weight stream for few rows (csrc/kernels/wmix_gemm.hip ``wmix_skinny_kernel``), or None where it does not
-    apply. It wins up to 16 rows, with fp6 up to 32 ([28672, 4096], 24 rows: fp6 57 us against the tile kernel's 78, int8
+    apply (rows of whole groups of a multiple of 128; fp6 as e3m2 or e2m3). It wins up to 16 rows, with fp6 up to 32 ([28672, 4096], 24 rows: fp6 57 us against the tile kernel's 78, int8
     61 against 50), with int8 from the second row on (one row: 36.5 us against the GEMV's 34.7, two 36.5 against 39)."""
     M = x2.shape[0]
     if (_needs_grad(x2) or not native.use_native(x2) or x2.dtype != torch.bfloat16 or in_features % 128
-            or group_size % 128 or not (fmt == "int8") < M <= (32 if fmt == "fp6" and not glu else 16)):
+            or group_size % 128 or in_features % group_size or (fmt == "fp6" and ebits not in (2, 3))
+            or not (fmt == "int8") < M <= (32 if fmt == "fp6" and not glu else 16)):
         return None
     x2 = x2.contiguous()
     if x2.data_ptr() % 16:

@@ -112,3 +112,45 @@ def test_gated_projection_of_packed_weights(fmt, act, M, N, K, G):
     # each factor within half a unit of the last place and its sum's error; |act'| <= 1.13
     bound = 2**-8 * (1.13 * gate.abs() * up.abs() + 2 * ref.abs()) + 1.13 * (eg * up.abs() + eu * gate.abs()) + 1e-6
     assert ((y.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("fmt", ["int8", "int4", "fp6"])
+@pytest.mark.parametrize("M", [3, 9, 16, 32])
+def test_groups_that_do_not_divide_a_row(fmt, M):
+    """Groups that run on from one row to the next (384 columns in groups of 256) are no case for the packed-weight kernels:
+    the linears dequantize then. Few rows of fp6 are refused, as the GEMV of up to 8 rows does."""
+    torch.manual_seed(M)
+    N, K, G = 128, 384, 256
+    x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(N, K, device="cuda", dtype=torch.bfloat16) * K**-0.5
+    if fmt == "fp6":
+        q, s = Q.quantize_minifloat(w.reshape(-1), G, 6, 2)
+        wd = Q.dequantize_minifloat(q, s, G, 6, 2, torch.float32).view(N, K).double()
+        if M <= 8:
+            with pytest.raises(RuntimeError):
+                Q.fp6_linear(x, q, s, N, K, G)
+            return
+        y = Q.fp6_linear(x, q, s, N, K, G)
+    else:
+        bits = int(fmt[3:])
+        q, s, _ = Q.quantize(w.reshape(-1), G, bits, True)
+        wd = Q.dequantize(q, s, None, G, bits, True, torch.float32).view(N, K).double()
+        y = Q.int_linear(x, q, s, N, K, G, bits=bits)
+    assert Q.packed_glu(x, q, s, N // 2, K, G, fmt, "silu") is None
+    # the dequantized weight and the result, each rounded to bf16
+    bound = 2**-8 * ((x.double() @ wd.t()).abs() + x.double().abs() @ wd.abs().t())
+    assert ((y.double() - x.double() @ wd.t()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M", [1, 8])
+@pytest.mark.parametrize("mantissa", [1, 2, 3])
+def test_fp6_formats_that_only_the_gemv_takes(M, mantissa):
+    """e4m1 beside the formats of the packed-weight kernels: up to 8 rows the GEMV decodes them."""
+    torch.manual_seed(M)
+    N, K, G = 64, 256, 128
+    x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
+    q, s = Q.quantize_minifloat((torch.randn(N, K, device="cuda") * K**-0.5).bfloat16().reshape(-1), G, 6, mantissa)
+    wd = Q.dequantize_minifloat(q, s, G, 6, mantissa, torch.float32).view(N, K).double()
+    y = Q.fp6_linear(x, q, s, N, K, G, mantissa)
+    bound = 2**-8 * ((x.double() @ wd.t()).abs() + x.double().abs() @ wd.abs().t())
+    assert ((y.double() - x.double() @ wd.t()).abs() <= bound).all()
