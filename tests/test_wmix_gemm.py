@@ -154,3 +154,18 @@ def test_fp6_formats_that_only_the_gemv_takes(M, mantissa):
     y = Q.fp6_linear(x, q, s, N, K, G, mantissa)
     bound = 2**-8 * ((x.double() @ wd.t()).abs() + x.double().abs() @ wd.abs().t())
     assert ((y.double() - x.double() @ wd.t()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("bits,M", [(8, 1), (8, 2), (4, 2), (8, 3)])
+def test_int_linear_with_a_32_bit_bias(bits, M):
+    """One and two rows with a 32-bit bias give 32 bits (the products are bf16), more rows bf16."""
+    torch.manual_seed(M)
+    N, K, G = 128, 256, 128
+    x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(N, K, device="cuda", dtype=torch.bfloat16) * K**-0.5
+    q, s, _ = Q.quantize(w.reshape(-1), G, bits, True)
+    b = torch.randn(N, device="cuda")
+    y = Q.int_linear(x, q, s, N, K, G, bits=bits, bias=b)
+    assert y.dtype == (torch.float32 if M <= 2 else torch.bfloat16)
+    ref = x.double() @ Q.dequantize(q, s, None, G, bits, True, torch.float32).view(N, K).double().t()
+    assert ((y.double() - (ref + b.double())).abs() <= 2**-8 * (ref.abs() + b.abs() + x.double().abs() @ w.double().abs().t())).all()
