@@ -157,7 +157,7 @@ class InferenceEngineV2:
             sm.maybe_allocate_kv(seq, tokens.numel())
             seq.pre_forward(tokens.numel())
             batch.insert_sequence(seq, tokens, do_checks=do_checks, logits_at=want)
-        batch.finalize()
+        batch.finalize(self._model.id_limit())
         if self._model.decode_graph_eligible(batch, capture_latents):
             # HIP-graph decode step (latents, if captured, land in the graph's device ring)
             logits, latents = self._model.forward_decode_graph(batch, capture_latents=capture_latents)

@@ -209,6 +209,9 @@ class HybridTransformer(RaggedTransformer):
         if snapshot is not None:
             self.state_pool.data.index_copy_(0, batch.slots.long(), snapshot)
 
+    def id_limit(self):
+        return None  # ids outside the embedding give rows of NaN
+
     def decode_graph_eligible(self, batch, capture_latents):
         return self.dtype == torch.bfloat16 and super().decode_graph_eligible(batch, capture_latents)
 

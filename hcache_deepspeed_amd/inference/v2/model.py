@@ -300,6 +300,10 @@ class RaggedTransformer:
         batch.atoms = atoms.to(self.device, non_blocking=True)
         batch.n_atoms = n_atoms
 
+    def id_limit(self):
+        """Rows of the embedding: token ids outside them are refused."""
+        return self.embed.shape[0]
+
     def _embed(self, batch):
         return self.embed_mod(batch, self.embed, self.pos_embed)
 

@@ -303,11 +303,12 @@ class RaggedBatchWrapper:
             slots[i] = torch.empty(max(need, 4096), dtype=torch.int32, pin_memory=self.device.type == "cuda")
         return i, slots[i]
 
-    def finalize(self):
+    def finalize(self, id_limit=None):
         """Ship the batch description to the device: the native builder (csrc/host/ragged_meta.cpp) writes seq_meta,
         token -> sequence / position maps, last-token rows, the KV block table and the attention atoms into ONE
         pinned int32 buffer behind the 64-bit token ids, sent with one async H2D copy into a persistent device buffer;
-        the device tensors below are views of it."""
+        the device tensors below are views of it. ``id_limit``: token ids outside [0, id_limit) raise IndexError, before
+        anything is sent (a lookup on the device cannot refuse them)."""
         import ctypes
         import numpy as np
         from ...ops import native
@@ -339,7 +340,9 @@ class RaggedBatchWrapper:
         if A < 0:
             raise RuntimeError(f"ragged metadata builder failed ({A})")
         if T:
-            torch.cat(self._tokens, out=host[:head].view(torch.int64))
+            ids = torch.cat(self._tokens, out=host[:head].view(torch.int64)).numpy()
+            if id_limit is not None and (ids.min() < 0 or ids.max() >= id_limit):
+                raise IndexError(f"token ids from {ids.min()} to {ids.max()}: the embedding has {id_limit} rows")
         n = head + int(need.value)
         if extra:
             host.numpy()[n:n + len(extra)] = extra

@@ -41,7 +41,7 @@ def embedding_grad_add_(grad, ids, dy, padding_idx=None):
 
 def lookup_rows(table, ids):
     """``F.embedding(ids, table)``, on the GPU by a kernel of one launch for tables without a gradient whose rows are whole
-    16-byte pieces; ids outside the table give NaN rows there."""
+    16-byte pieces. Ids outside the table, which a caller with ids on the host refuses, give NaN rows there."""
     row = table.shape[-1] * table.element_size()
     if native.use_native(table) and table.dim() == 2 and ids.dim() == 1 and ids.dtype == torch.int64 and \
             ids.device == table.device and table.is_floating_point() and row % 16 == 0 and \

@@ -246,6 +246,25 @@ def test_allocator_and_scheduling():
     assert eng.can_schedule([1], [64 * 3 + 1]) != SchedulingResult.Success
 
 
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("bad", [[-1], [64], [3, 64, 1], [1 << 40]])
+def test_token_ids_outside_the_embedding_are_refused(dev, bad):
+    """Decode steps (eager, then from a graph) and prompts; other sequences of the refused step go on as if it had not been."""
+    gpu = dev == "cuda"
+    m = _model(dev, torch.bfloat16 if gpu else torch.float32, vocab_size=64)
+    conf = {"dtype": "bf16" if gpu else "fp32", "state_manager": {"max_context": 256}}
+    engs = [build_engine_from_model(m, conf, device=torch.device(dev), num_kv_blocks=16) for _ in range(2)]
+    for step in range(4):
+        if step:
+            for uids, batch in (([1, 2], [torch.tensor([5]), torch.tensor(bad)]), ([3], [torch.tensor(bad)])):
+                with pytest.raises(IndexError):
+                    engs[0].put(uids, batch, capture_latents=False)
+            engs[0].flush(3)
+        toks = [torch.arange(7), torch.arange(3)] if step == 0 else [torch.tensor([step]), torch.tensor([9])]
+        a, b = (e.put([1, 2], toks, capture_latents=False)[0] for e in engs)
+        assert torch.equal(a, b) and torch.isfinite(a.float()).all()
+
+
 def test_native_ragged_metadata_matches_python_reference():
     """csrc/host/ragged_meta.cpp packs seq_meta / token maps / last rows / block tables / atoms exactly as the
     Python reference (ops/paged.build_atoms and the per-sequence loops) would build them."""
