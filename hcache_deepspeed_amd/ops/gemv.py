@@ -71,10 +71,15 @@ def skinny(x2, w, b=None):
     return y
 
 
+def _needs_grad(*tensors):
+    """The kernels have no backward: with gradients wanted the products are torch's."""
+    return torch.is_grad_enabled() and any(torch.is_tensor(t) and t.requires_grad for t in tensors)
+
+
 def glu_linear(x, w, b, act):
     """act(x . gate^T) * (x . up^T) for ``w`` = [gate; up] (and ``b``) in one kernel, for 2..16 rows of the skinny GEMM; None
     for anything else. The projections are rounded to bf16 first, as the separate kernels store them."""
-    if act not in _GATHER_ACTS or not (x.dim() >= 1 and x.is_cuda and torch.is_tensor(w)):
+    if act not in _GATHER_ACTS or not (x.dim() >= 1 and x.is_cuda and torch.is_tensor(w)) or _needs_grad(x, w, b):
         return None
     x2 = x.reshape(-1, x.shape[-1])
     if not skinny_ok(x2, w, b) or w.shape[0] % 2:
@@ -89,8 +94,8 @@ def glu_linear(x, w, b, act):
 
 def linear(x, w, b=None):
     """``F.linear(x, w, b)``; decode-sized bf16 inputs run the HIP GEMV (one row) or the skinny matrix-core GEMM
-    (2..16 rows)."""
-    if x.dim() >= 1 and x.is_cuda:
+    (2..16 rows), unless a gradient is wanted."""
+    if x.dim() >= 1 and x.is_cuda and not _needs_grad(x, w, b):
         x2 = x.reshape(-1, x.shape[-1])
         if skinny_ok(x2, w, b):
             return skinny(x2, w, b).view(*x.shape[:-1], w.shape[0])

@@ -58,6 +58,30 @@ def test_linear_implementations(act, mode, tol):
     assert err < tol, (mode, act, float(err))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 8, 16])
+@pytest.mark.parametrize("leaf", ["rows", "weight"])
+def test_few_rows_keep_their_gradient_gpu(rows, leaf):
+    """Logits, a projection and a gated one of as few rows as run on kernels without a backward, with gradients wanted of
+    the rows or of the weight alone."""
+    from hcache_deepspeed_amd.inference.v2.modules import DSUnembedConfig, instantiate_unembed
+    torch.manual_seed(rows)
+    x, w = (torch.randn(n, 256, device="cuda", dtype=torch.bfloat16) * 256**-0.25 for n in (rows, 64))
+    t = (x if leaf == "rows" else w).requires_grad_()
+    unembed = instantiate_unembed(DSUnembedConfig(model_dim=256, vocab_size=64))
+    lin, glu = (instantiate_linear(DSLinearConfig(256, 64, activation=a)) for a in ("identity", "silu_glu"))
+    gate, up = torch.nn.functional.linear(x.float(), w.float()).chunk(2, -1)
+    full = torch.cat([gate, up], -1)
+    for got, ref in ((unembed.project(x, w), full), (lin(x, w), full),
+                     (glu(x, w), torch.nn.functional.silu(gate) * up)):
+        assert got.requires_grad
+        do = torch.randn_like(ref)
+        a, b = torch.autograd.grad(got, t, do.bfloat16())[0], torch.autograd.grad(ref, t, do, retain_graph=True)[0]
+        assert (a.float() - b).norm() <= 3 * 2**-8 * b.norm()
+        with torch.no_grad():
+            assert (got - (lin(x, w) if ref is full else glu(x, w))).norm() <= 2**-7 * ref.norm()
+
+
 def test_pre_norm_and_moe_modules():
     torch.manual_seed(0)
     n = instantiate_pre_norm(DSNormConfig(32, "rms", 1e-6))
