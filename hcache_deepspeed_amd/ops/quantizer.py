@@ -183,8 +183,8 @@ def _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, fm
     if x2.data_ptr() % 16:
         return None
     if bias is not None:
-        if bias.dtype != torch.bfloat16:
-            return None  # (up to _INT_GEMV_MAX_M rows a wider bias makes a wider result)
+        if bias.dtype != torch.bfloat16 or _needs_grad(bias):
+            return None  # (up to _INT_GEMV_MAX_M rows the bias is added by itself: a wider one makes a wider result)
         bias = bias.contiguous()
     y = torch.empty(M, out_features, dtype=torch.bfloat16, device=x2.device)
     native.check(native.kernels().hds_wmix_skinny(x2.data_ptr(), q_weight.data_ptr(), scales.data_ptr(),

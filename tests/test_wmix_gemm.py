@@ -167,5 +167,7 @@ def test_int_linear_with_a_32_bit_bias(bits, M):
     b = torch.randn(N, device="cuda")
     y = Q.int_linear(x, q, s, N, K, G, bits=bits, bias=b)
     assert y.dtype == (torch.float32 if M <= 2 else torch.bfloat16)
+    narrow = b.bfloat16().requires_grad_()
+    assert Q.int_linear(x, q, s, N, K, G, bits=bits, bias=narrow).requires_grad == (M <= 2)
     ref = x.double() @ Q.dequantize(q, s, None, G, bits, True, torch.float32).view(N, K).double().t()
     assert ((y.double() - (ref + b.double())).abs() <= 2**-8 * (ref.abs() + b.abs() + x.double().abs() @ w.double().abs().t())).all()
