@@ -321,12 +321,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   // moderate constant, not -inf or a multiple of 1e30: a row whose keys in the first tile are all masked takes its
   // running max from masked scores, and fma(s, c, -max) must not round above 0 by more than exp2 can take (a 1e30
   // scale rounds by ~1e22 there: exp2 -> inf, and inf x alpha = 0 -> NaN); 2^20 keeps the rounding < 0.01 and still
-  // sends every masked exp2 to 0 once a real key arrives (alpha = exp2(-2^20 c) = 0 rescales the masked start away)
+  // sends every masked exp2 to 0 once a real key arrives (alpha = exp2(-2^20 c) = 0 rescales the masked start away).
+  // PAGED: masked scores are replaced: whatever a later token's key is (infinite, NaN, a score 2^20 above the visible ones),
+  // earlier rows do not see it. The value (scale > 0) is the power of two that makes 2^28 to 2^29 in the exponent: a row
+  // that starts with masked tiles rounds by at most 2^4 there. It is made in the branch: as a value that lives through the
+  // kernel it cost 5 % (16,000 tokens, 16 / 4 heads: 929 -> 974 us, so 937; 512 behind 789, 32 / 8: 43.5 -> 42.6).
   auto mask_tile = [&](f32x16 (&sn)[2][2], int kt) {
     const int k0 = kt * BN;
     const bool need_mask = (k0 + BN > len) || (p.causal && k0 + BN - 1 > wq_lo) ||
                            (p.window > 0 && k0 <= wq_hi - p.window) || (wq_hi >= len);
     if (need_mask) {
+      const int masked = 0x80000000 | ((127 + 28 + 127 - (__float_as_int(c) >> 23)) << 23);
 #pragma unroll
       for (int qh = 0; qh < 2; ++qh)
 #pragma unroll
@@ -337,7 +342,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
           for (int r = 0; r < 16; ++r) {
             const int ar = (r & 3) + 8 * (r >> 2);
             const int pen = ((A + ar) | (B - ar)) >> 31;  // -1 outside [lo, hi], 0 inside
-            sn[t][qh][r] = __builtin_fmaf((float)pen, kMaskPen, sn[t][qh][r]);
+            if constexpr (PAGED)
+              sn[t][qh][r] = __int_as_float((pen & masked) | (~pen & __float_as_int(sn[t][qh][r])));
+            else
+              sn[t][qh][r] = __builtin_fmaf((float)pen, kMaskPen, sn[t][qh][r]);
           }
         }
     }

@@ -87,6 +87,49 @@ def test_portions_match_float64(lens, seen, hq, hkv, bs, window):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("window", [0, 100])
+@pytest.mark.parametrize("later", ["rising", math.inf, -math.inf, math.nan])
+def test_later_keys_do_not_reach_earlier_rows(later, window):
+    """Scores that rise by 131,072 a position, so that every masked one is far above the visible ones, and keys that are
+    infinite or NaN from the middle of a portion on: rows in front of them are what they are without them."""
+    lens, seen, hq, hkv = [300, 130], [37, 0], 8, 2
+    g = torch.Generator().manual_seed(1)
+    dev = torch.device("cuda")
+    cache, tab, metas, T, batch = _setup(lens, seen, hkv, 64, dev, g)
+    qkv = torch.randn(T, hq + 2 * hkv, D, generator=g).bfloat16().to(dev)
+    u = torch.where(torch.rand(D, generator=g) < 0.5, -1.0, 1.0).bfloat16().to(dev)
+    good = []
+    for i, (q0, n, s) in enumerate(metas):
+        at = torch.arange(s + n)
+        blk, slot = tab[i, at // 64].long().to(dev), (at % 64).to(dev)
+        if later == "rising":
+            qkv[q0:q0 + n, :hq] = 16 * u
+            cache[blk, slot, 0] = ((at // 4) * 256).bfloat16().to(dev)[:, None, None] * u
+        else:
+            cache[blk[s + n // 2:], slot[s + n // 2:], 0] = later
+        good.append(n if later == "rising" else n // 2)
+    q = qkv[:, :hq]
+    toks, blocks = make_portions(metas)
+    assert not toks
+    blocks = torch.tensor(blocks, dtype=torch.int32, device=dev).view(-1, 2)
+    o = paged_attention_portions(q, cache, None, blocks, batch, hq, hkv, 1 / math.sqrt(D), window)
+    for i, (q0, _, s) in enumerate(metas):
+        n = good[i]
+        at = torch.arange(s + n)
+        rows = cache[tab[i, at // 64].long().to(dev), (at % 64).to(dev)].double()
+        k, v = (rows[:, j].repeat_interleave(hq // hkv, 1).transpose(0, 1) for j in (0, 1))
+        sc = q[q0:q0 + n].double().transpose(0, 1) @ k.transpose(1, 2) / math.sqrt(D)
+        mine = (s + torch.arange(n))[:, None]
+        hide = at[None] > mine
+        if window:
+            hide |= at[None] <= mine - window
+        want = (torch.softmax(sc.masked_fill(hide.to(dev), float("-inf")), -1) @ v).transpose(0, 1)
+        got = o[q0:q0 + n].double()
+        worst = (got - want).norm(dim=-1) / want.norm(dim=-1)  # p and the result rounded to bf16, as above
+        assert torch.isfinite(got).all() and worst.max() < 0.03, (i, worst.max())
+
+
+@pytest.mark.gpu
 def test_engine_steps_in_pieces_match_whole_prompts():
     """A prompt taken in pieces beside decoding sequences gives the logits of the prompt taken whole."""
     from hcache_deepspeed_amd.inference.v2.engine import build_engine_from_model
