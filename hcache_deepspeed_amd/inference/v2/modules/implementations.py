@@ -83,8 +83,9 @@ class DSDenseBlockedAttention(DSSelfAttentionBase):
                         do_rope=rope, rotary_dim=c.rotary_dim)
         portions = getattr(batch, "portions", None)
         if portions is not None and portions_ok(qkv[:, :nq], cache, nq, nkv):
-            return paged_attention_portions(qkv[:, :nq], cache, *portions, batch, nq, nkv, c.scale_factor,
-                                            c.sliding_window).reshape(T, nq * D)
+            toks, blocks, rows = portions
+            return paged_attention_portions(qkv[:, :nq], cache, toks, blocks, batch, nq, nkv, c.scale_factor,
+                                            c.sliding_window, rows).reshape(T, nq * D)
         o = paged_attention(qkv[:, :nq], cache, batch.atoms, batch.n_atoms, batch.seq_meta, batch.block_tables, nq,
                             nkv, c.scale_factor, c.sliding_window, batch.seq_meta_host, batch.tables_host,
                             decode=T == batch.current_sequences)

@@ -312,7 +312,7 @@ class RaggedBatchWrapper:
         import ctypes
         import numpy as np
         from ...ops import native
-        from ...ops.paged_prefill import make_portions
+        from ...ops.paged_prefill import divide_step
         S, T = len(self._seqs), self.current_tokens
         mb = self.max_blocks
         n_new = np.fromiter((nn for (_, nn, _) in self.seq_meta_host), dtype=np.int32, count=S)
@@ -331,8 +331,8 @@ class RaggedBatchWrapper:
         # after the builder's part: the sequences' state slots, explicit logits rows, the division of a step that is not
         # single tokens only
         mixed = any(nn != 1 for (_, nn, _) in self.seq_meta_host)
-        toks, blocks = make_portions(self.seq_meta_host) if mixed else ([], [])
-        extra = [seq.tracking_id for seq in self._seqs] + (self._logit_rows or []) + blocks + toks
+        toks, blocks, rows = divide_step(self.seq_meta_host, n_q, n_kv) if mixed else ([], [], [])
+        extra = [seq.tracking_id for seq in self._seqs] + (self._logit_rows or []) + blocks + toks + rows
         head = 2 * T  # the ids, first: 8-byte aligned
         si, host = self._pinned_slot(head + int(need.value) + len(extra))
         A = lib.hds_ragged_meta_build(P(n_new), P(seen), S, P(flat), P(off), mb, n_q, n_kv, rpa,
@@ -383,7 +383,7 @@ class RaggedBatchWrapper:
         self.portions = None
         if mixed:
             blocks = take(len(blocks), (-1, 2)) if blocks else None
-            self.portions = (take(len(toks), (-1, )) if toks else None, blocks)
+            self.portions = (take(len(toks), (-1, )) if toks else None, blocks, take(len(rows), (-1, 3)) if rows else None)
         self.tables_host = host[head + 4 * S + 2 * T:head + 4 * S + 2 * T + S * mb].view(S, mb).clone() if S else \
             torch.zeros(1, mb, dtype=torch.int32)
         if S == 0:  # keep 1-row shapes for empty batches (kernels never run on them)

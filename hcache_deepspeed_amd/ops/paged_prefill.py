@@ -1,25 +1,81 @@
 """Serving steps with more than single tokens: portions of prompts on the one-wave-per-SIMD attention kernel over block tables
-(csrc/kernels/flash_attn_w64.hip), single tokens on the split-key kernel (csrc/kernels/paged_attn.hip)."""
+(csrc/kernels/flash_attn_w64.hip) or in row blocks, single tokens on the split-key kernel (both csrc/kernels/paged_attn.hip)."""
 import torch
 
 from . import native
-from .paged import DECODE_MAX
+from .paged import DECODE_MAX, ROWS_PER_ATOM
 
 # new tokens of a workgroup of the prefill kernel
 PREFILL_ROWS = 256
 
 
-def make_portions(seq_meta_host):
+def make_portions(seq_meta_host, portions=None):
     """How a step with more than single tokens is divided: (rows of the tokens that run one by one, flat list of (sequence,
-    first new token) of the prefill kernel's workgroups, those that see the most keys first)."""
+    first new token) of the prefill kernel's workgroups, those that see the most keys first). ``portions``: the sequences
+    that run on it (default: those of more than ``DECODE_MAX`` new tokens)."""
     toks, blocks = [], []
     for s, (q0, n, seen) in enumerate(seq_meta_host):
-        if n <= DECODE_MAX:
+        if n <= DECODE_MAX if portions is None else s not in portions:
             toks += range(q0, q0 + n)
         else:
             blocks += [(seen + min(r + PREFILL_ROWS, n), s, r) for r in range(0, n, PREFILL_ROWS)]
     blocks.sort(reverse=True)
     return toks, [v for b in blocks for v in b[1:]]
+
+
+# Microseconds of the kernels, fitted to 1 to 64 sequences of 2 to 256 new tokens behind 60 to 4,000 earlier ones, 8 / 1 to 64 / 8
+# and 32 / 32 heads (within a fifth, at least about the lines between them). Prefill kernel and row blocks: the longest
+# workgroup, or all of them over the CUs (256 at a time; of the row blocks about 270). One by one: the contexts are read from
+# memory once, from the caches once a token.
+def _prefill_us(seqs, heads):
+    longest = max(7 + 0.031 * (seen + n) for n, seen in seqs)
+    return max(longest, heads / 256 * sum(-(-n // PREFILL_ROWS) * (7 + 0.031 * (seen + n / 2)) for n, seen in seqs))
+
+
+def _rows_us(seqs, heads, kv_heads):
+    G, R = heads // kv_heads, ROWS_PER_ATOM
+    longest = max(4 + 0.05 * (seen + n) for n, seen in seqs)
+    return max(longest, kv_heads / 270 * sum(-(-n * G // R) * (2.5 + 4.5 * min(1, n * G / R) + 0.05 * (seen + n / 2))
+                                             for n, seen in seqs))
+
+
+def _tokens_us(seqs, kv_heads):
+    return 6 + kv_heads * sum((seen + n) * (6e-5 + 3.8e-5 * n) + 6e-3 * n for n, seen in seqs)
+
+
+def divide_step(seq_meta_host, heads, kv_heads):
+    """``make_portions`` for these head counts, and flat list of (sequence, kv head, first row) of the sequences that run in
+    row blocks: (tokens, blocks, atoms). Two cases leave ``make_portions``'s division:
+
+    * many portions of few tokens: the prefill kernel has a workgroup a query head for each of them, 256 at a time, row
+      blocks have one a key head (32 sequences of 16 tokens, up to 4,000 keys, 32 / 8 heads: 331 us against 226; 16
+      sequences 176 / 213, of 64 tokens 140 / 220);
+    * many sequences of 2 to ``DECODE_MAX`` tokens, whose contexts are read once a token: 32 of 8 tokens there 237 us
+      against 221 in row blocks, up to 1,000 keys 69 / 58, up to 300 34 / 20; of 4 tokens 155 / 224, 41 / 57, 20 / 20.
+
+    Beside row blocks single tokens join them where that takes less than a launch of their own (32 of them and 32 sequences
+    of 8 tokens, up to 2,000 keys: 161 us apart, 129 together)."""
+    new = {s: (n, seen) for s, (_, n, seen) in enumerate(seq_meta_host) if n}
+    ones = [s for s, (n, _) in new.items() if n == 1]
+    few = [s for s, (n, _) in new.items() if 1 < n <= DECODE_MAX]
+    many = [s for s, (n, _) in new.items() if n > DECODE_MAX]
+    of = lambda which: [new[s] for s in which]  # noqa: E731
+    best = lambda which: min(_prefill_us(of(which), heads), _rows_us(of(which), heads, kv_heads)) if which else 0  # noqa: E731
+    if kv_heads * sum(new[s][0] for s in few) > 512 and _tokens_us(of(few), kv_heads) > best(few + many) - best(many):
+        few, many = [], few + many
+    if heads * sum(-(-new[s][0] // PREFILL_ROWS) for s in many) <= 256 or \
+            _prefill_us(of(many), heads) <= _rows_us(of(many), heads, kv_heads):
+        return (*make_portions(seq_meta_host, set(many)), [])
+    if ones and _tokens_us(of(ones), kv_heads) > _rows_us(of(ones + many), heads, kv_heads) - _rows_us(of(many), heads, kv_heads):
+        many = many + ones
+    G, gone = heads // kv_heads, set(many)
+    toks = [t for s, (q0, n, _) in enumerate(seq_meta_host) if s not in gone for t in range(q0, q0 + n)]
+    atoms = []
+    for s in sorted(many, key=lambda s: -sum(new[s])):  # those that see the most keys first
+        for r in range(0, new[s][0] * G, ROWS_PER_ATOM)[::-1]:
+            for h in range(kv_heads):
+                atoms += (s, h, r)
+    return toks, [], atoms
 
 
 def portions_ok(q, cache, n_q, n_kv):
@@ -30,11 +86,11 @@ def portions_ok(q, cache, n_q, n_kv):
             and q.stride(0) % 8 == 0 and q.stride(1) == 128 and q.data_ptr() % 16 == 0)
 
 
-def paged_attention_portions(q, cache, toks, blocks, batch, n_q, n_kv, scale, window=0):
+def paged_attention_portions(q, cache, toks, blocks, batch, n_q, n_kv, scale, window=0, atoms=None):
     """``paged_attention`` of a step that mixes single tokens and portions of prompts: ``toks`` (int32 rows of q) on the
-    split-key kernel, which spreads a token's context over the chip, ``blocks`` ([n, 2] int32) on the prefill kernel. In
-    row blocks of the matrix-core kernel a single token walks its whole context in one workgroup (9 such tokens, up to 3,000
-    keys, 8 key heads, beside 512 new ones: 171 us; apart 29 + 38 us)."""
+    split-key kernel, which spreads a token's context over the chip, ``blocks`` ([n, 2] int32) on the prefill kernel,
+    ``atoms`` ([n, 3] int32) in row blocks. There a single token walks its whole context in one workgroup (9 such tokens,
+    up to 3,000 keys, 8 key heads, beside 512 new ones: 171 us; apart 29 + 38 us)."""
     T, _, D = q.shape
     o = torch.empty(T, n_q, D, device=q.device, dtype=q.dtype)
     lib, st, tab = native.kernels(), native.stream(), batch.block_tables
@@ -58,4 +114,9 @@ def paged_attention_portions(q, cache, toks, blocks, batch, n_q, n_kv, scale, wi
             lib.hds_paged_prefill(q.data_ptr(), q.stride(0), cache.data_ptr(), o.data_ptr(), n_q * D,
                                   blocks.data_ptr(), blocks.shape[0], batch.seq_meta.data_ptr(), tab.data_ptr(), mb, bs,
                                   n_q, n_kv, float(scale), int(window), st), "paged_prefill")
+    if atoms is not None and atoms.shape[0]:
+        native.check(
+            lib.hds_paged_attn(q.data_ptr(), q.stride(0), cache.data_ptr(), o.data_ptr(), n_q * D, atoms.data_ptr(),
+                               atoms.shape[0], batch.seq_meta.data_ptr(), tab.data_ptr(), mb, bs, n_q, n_kv, D, D,
+                               float(scale), int(window), 0, 0, 0.0, None, None, 0, 1, st), "paged_attn")
     return o

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from hcache_deepspeed_amd.ops.paged import DECODE_MAX
-from hcache_deepspeed_amd.ops.paged_prefill import make_portions, paged_attention_portions, portions_ok
+from hcache_deepspeed_amd.ops.paged_prefill import divide_step, make_portions, paged_attention_portions, portions_ok
 
 D = 128
 
@@ -27,6 +27,36 @@ def test_portions_cover_every_token_once():
     assert rows == set(range(q0)) and len(toks) == 1 + DECODE_MAX
     last = [metas[s][2] + min(r + 256, metas[s][1]) for s, r in blocks]
     assert last == sorted(last, reverse=True)
+
+
+@pytest.mark.parametrize("lens,seen,heads,one_by_one,kernel", [
+    ([512, 1, 1], [700, 3000, 9], (32, 8), [1, 1], "prefill"),        # a piece of a prompt beside single tokens
+    ([2048], [0], (32, 8), [], "prefill"), ([9], [0], (8, 1), [], "prefill"),
+    ([8] * 8 + [1], [3000] * 9, (32, 8), [8] * 8 + [1], None),        # few sequences of a few tokens each
+    ([8] * 32 + [1], [2400] * 33, (32, 8), [], "rows"),               # many of them
+    ([1] * 100 + [8] * 32, [4000] * 100 + [200, 1000] * 16, (32, 8), [1] * 100, "rows"),
+    ([4] * 32, [200, 1000] * 16, (32, 8), [4] * 32, None), ([8] * 32, [200, 1000] * 16, (16, 4), [8] * 32, None),
+    ([16] * 32 + [1, 0], [2400] * 34, (32, 8), [], "rows"),           # many short portions
+    ([60] * 30, [0] * 30, (32, 32), [], "rows"), ([20] * 32, [2400] * 32, (32, 32), [], "prefill"),
+    ([16] * 8, [2400] * 8, (32, 8), [], "prefill"), ([256] * 32, [2400] * 32, (32, 8), [], "prefill"),
+    ([8] * 32 + [512] * 4, [2400] * 36, (32, 32), [], "prefill")])
+def test_division_of_a_step(lens, seen, heads, one_by_one, kernel):
+    """Which kernel runs which sequences, and that every row of every head runs once."""
+    metas, q0 = [], 0
+    for n, s in zip(lens, seen):
+        metas.append((q0, n, s))
+        q0 += n
+    toks, blocks, atoms = divide_step(metas, *heads)
+    assert len(toks) == sum(one_by_one) and bool(blocks) == (kernel == "prefill") and bool(atoms) == (kernel == "rows")
+    G = heads[0] // heads[1]
+    seen_rows = [(t, h) for t in toks for h in range(heads[0])]
+    for s, r in zip(blocks[::2], blocks[1::2]):
+        q0, n, _ = metas[s]
+        seen_rows += [(q0 + i, h) for i in range(r, min(r + 256, n)) for h in range(heads[0])]
+    for s, hk, r in zip(atoms[::3], atoms[1::3], atoms[2::3]):
+        q0, n, _ = metas[s]
+        seen_rows += [(q0 + i // G, hk * G + i % G) for i in range(r, min(r + 128, n * G))]
+    assert len(seen_rows) == len(set(seen_rows)) == sum(lens) * heads[0]
 
 
 def _setup(lens, seen, hkv, bs, device, g):
@@ -83,6 +113,34 @@ def test_portions_match_float64(lens, seen, hq, hkv, bs, window):
         got = o[q0:q0 + n].double()
         assert (got - want).norm() <= 4 * 2**-8 * want.norm(), i
         worst = (got - want).norm(dim=-1) / want.norm(dim=-1)  # no single row off either
+        assert worst.max() < 0.03, (i, worst.max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lens,window", [([20] * 40 + [1, 1], 0), ([8] * 40 + [1] * 3, 0), ([33, 2] * 20, 90)])
+def test_many_short_portions_match_float64(lens, window):
+    """Steps that run in row blocks beside single tokens; the bounds of the test above."""
+    seen = [(37 * i) % 290 for i in range(len(lens))]
+    hq, hkv = 32, 8
+    g = torch.Generator().manual_seed(len(lens))
+    dev = torch.device("cuda")
+    cache, tab, metas, T, batch = _setup(lens, seen, hkv, 64, dev, g)
+    q = torch.randn(T, hq, D, generator=g).bfloat16().to(dev)
+    i32 = lambda v, shape: torch.tensor(v, dtype=torch.int32, device=dev).view(shape) if v else None  # noqa: E731
+    toks, blocks, atoms = divide_step(metas, hq, hkv)
+    assert atoms and not blocks
+    o = paged_attention_portions(q, cache, i32(toks, (-1, )), None, batch, hq, hkv, D**-0.5, window, i32(atoms, (-1, 3)))
+    for i, (q0, n, s) in enumerate(metas):
+        at = torch.arange(s + n)
+        rows = cache[tab[i, at // 64].long().to(dev), (at % 64).to(dev)].double()
+        k, v = (rows[:, j].repeat_interleave(hq // hkv, 1).transpose(0, 1) for j in (0, 1))
+        sc = q[q0:q0 + n].double().transpose(0, 1) @ k.transpose(1, 2) * D**-0.5
+        mine = (s + torch.arange(n))[:, None]
+        hide = at[None] > mine
+        if window:
+            hide |= at[None] <= mine - window
+        want = (torch.softmax(sc.masked_fill(hide.to(dev), float("-inf")), -1) @ v).transpose(0, 1)
+        worst = (o[q0:q0 + n].double() - want).norm(dim=-1) / want.norm(dim=-1)
         assert worst.max() < 0.03, (i, worst.max())
 
 
