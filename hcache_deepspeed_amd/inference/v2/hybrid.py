@@ -209,6 +209,9 @@ class HybridTransformer(RaggedTransformer):
         if snapshot is not None:
             self.state_pool.data.index_copy_(0, batch.slots.long(), snapshot)
 
+    def uses_portions(self):
+        return False  # the mixers plan their own steps
+
     def id_limit(self):
         return None  # ids outside the embedding give rows of NaN
 

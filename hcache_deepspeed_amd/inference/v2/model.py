@@ -300,6 +300,10 @@ class RaggedTransformer:
         batch.atoms = atoms.to(self.device, non_blocking=True)
         batch.n_atoms = n_atoms
 
+    def uses_portions(self):
+        """Is attention asked to divide steps with more than single tokens (ops/paged_prefill.py ``portions_ok``)?"""
+        return self.device.type == "cuda" and self.dtype == torch.bfloat16 and self.d == 128
+
     def id_limit(self):
         """Rows of the embedding: token ids outside them are refused."""
         return self.embed.shape[0]

@@ -287,9 +287,11 @@ class RaggedBatchWrapper:
         self._tokens.append(tokens.reshape(-1).to(torch.int64))
         self.current_tokens += n
 
-    def set_attention_geometry(self, n_q, n_kv, rows_per_atom):
-        """Lets ``finalize`` also build the paged-attention work atoms (the model's query/KV head counts)."""
+    def set_attention_geometry(self, n_q, n_kv, rows_per_atom, portions=True):
+        """Lets ``finalize`` also build the paged-attention work atoms (the model's query/KV head counts). ``portions``:
+        and the division of steps with more than single tokens (ops/paged_prefill.py), for models that use it."""
         self._geom = (int(n_q), int(n_kv), int(rows_per_atom))
+        self._portions = portions
 
     def _pinned_slot(self, need):
         """One of two rotating pinned int32 staging buffers; a slot is reused only after its H2D drained."""
@@ -330,7 +332,7 @@ class RaggedBatchWrapper:
                                   ctypes.byref(need))
         # after the builder's part: the sequences' state slots, explicit logits rows, the division of a step that is not
         # single tokens only
-        mixed = any(nn != 1 for (_, nn, _) in self.seq_meta_host)
+        mixed = getattr(self, "_portions", True) and any(nn != 1 for (_, nn, _) in self.seq_meta_host)
         toks, blocks, rows = divide_step(self.seq_meta_host, n_q, n_kv) if mixed else ([], [], [])
         extra = [seq.tracking_id for seq in self._seqs] + (self._logit_rows or []) + blocks + toks + rows
         head = 2 * T  # the ids, first: 8-byte aligned

@@ -187,6 +187,25 @@ def test_later_keys_do_not_reach_earlier_rows(later, window):
         assert torch.isfinite(got).all() and worst.max() < 0.03, (i, worst.max())
 
 
+def test_division_is_made_for_models_that_use_it(monkeypatch):
+    """Neither for the hybrid designs, whose mixers plan their own steps, nor where the kernels do not apply."""
+    from hcache_deepspeed_amd.inference.v2 import build_engine_from_model
+    from hcache_deepspeed_amd.models.llama import LlamaForCausalLM, tiny
+    from hcache_deepspeed_amd.ops import paged_prefill
+
+    from .test_gofasun import engine
+    made = []
+    monkeypatch.setattr(paged_prefill, "divide_step", lambda *a: made.append(a) or divide_step(*a))
+    cpu = torch.device("cpu")
+    dense = build_engine_from_model(LlamaForCausalLM(tiny()).eval(), {"dtype": "fp32"}, device=cpu, num_kv_blocks=8)
+    for eng in (engine("mixed", (cpu, torch.float32)), dense):
+        eng.put([1, 2], [torch.arange(20) % 7, torch.arange(3)], capture_latents=False)
+    assert not made
+    dense._batch.set_attention_geometry(4, 2, 128)
+    dense.put([1, 2], [torch.arange(20) % 7, torch.arange(3)], capture_latents=False)
+    assert len(made) == 1
+
+
 @pytest.mark.gpu
 def test_engine_steps_in_pieces_match_whole_prompts():
     """A prompt taken in pieces beside decoding sequences gives the logits of the prompt taken whole."""
