@@ -223,7 +223,7 @@ class GroupedGemmMoE(DSMoEBase):
         ws13, ws2, gate = shared if shared is not None else (None, None, None)
         mats = [t for t in (router_w, w13, w2, ws13, ws2, gate) if t is not None]
         if not (c.activation == "silu_glu" and E <= 1024 and H % PAD == 0 and I % PAD == 0 and w13.is_cuda
-                and all(t.dtype == torch.bfloat16 and t.is_contiguous() for t in mats)
+                and all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in mats)
                 and (ws2 is None or ws2.shape[1] % PAD == 0)):
             return None
         return {"router.w": router_w if gate is None else torch.cat([router_w, gate]), "router.c": None, "w13": w13,
@@ -238,6 +238,8 @@ class GroupedGemmMoE(DSMoEBase):
         if laid is None and x.dtype == torch.bfloat16 and not grad:
             laid = self.lay_out(router_w, w13, w2)
         if laid is not None and T:
+            if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:  # the kernels read 16-byte pieces of rows
+                x = x.clone(memory_format=torch.contiguous_format)
             shape = RouterShape(w2.shape[0], top=c.top_k, normalize=bool(c.normalize_scores) and c.top_k > 1)
             return sum_experts(x, routed_experts(x, laid, shape), x.dtype)
         logits = F.linear(x.float(), router_w.float())

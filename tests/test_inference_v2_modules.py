@@ -206,6 +206,29 @@ def test_routed_moe_module_gpu(T, E, top, normalize, has_shared):
     assert torch.equal(z.gather(1, expert.long()), z.topk(top, -1).values)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [5, 130])
+@pytest.mark.parametrize("how", ["columns first", "odd row stride", "shifted rows", "shifted weights"])
+def test_routed_moe_module_takes_any_layout_gpu(T, how):
+    """Rows that are no whole 16-byte pieces in order give what a copy in order gives; weights that are not aligned are not
+    laid out."""
+    H, I, E = 256, 128, 8
+    g = torch.Generator(device="cuda").manual_seed(T)
+    mat = lambda *s: (torch.randn(*s, generator=g, device="cuda") * s[-1]**-0.5).bfloat16()  # noqa: E731
+    x, rw, w13, w2 = mat(T, H) * 16, mat(E, H) * 4, mat(E, 2 * I, H), mat(E, H, I)
+    moe = instantiate_moe(DSMoEConfig(H, I, E, 2, "silu_glu", True))
+    want = moe(x, rw, w13, w2)
+    shifted = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)  # noqa: E731
+    if how == "shifted weights":
+        assert moe.lay_out(rw, shifted(w13), w2) is None and moe.lay_out(shifted(rw), w13, w2) is None
+        return
+    if how == "columns first":
+        v = x.t().contiguous().t()
+    else:
+        v = shifted(x) if how == "shifted rows" else torch.cat([x, x[:, :5]], 1)[:, :H]
+    assert torch.equal(v, x) and torch.equal(moe(v, rw, w13, w2), want)
+
+
 def test_route_normalizes():
     from hcache_deepspeed_amd.ops.experts import RouterShape, route
     z = torch.randn(5, 12, generator=torch.Generator().manual_seed(0))
