@@ -71,8 +71,9 @@ __device__ __forceinline__ void lpt_ids(int& blk, int& head, int& b) {
   b = rem / heads;
 }
 
-// The per-element mask as an interval test (two compares, no branches): the keys a query may see, or the queries
-// that may see a key, form [lo, hi] (empty when lo > hi). Same predicate as masked() below.
+// The per-element mask as an interval test (two compares, no branches). A query sees the keys of its sequence, causal up to
+// its own position and with a window the last `window` of those: the keys a query may see, or the queries that may see a
+// key, form [lo, hi] (empty when lo > hi).
 __device__ __forceinline__ void key_span(const AttnParams& p, int qi, int len, int& lo, int& hi) {
   lo = p.window > 0 ? max(0, qi - p.window + 1) : 0;
   hi = p.causal ? min(qi, len - 1) : len - 1;
@@ -84,13 +85,6 @@ __device__ __forceinline__ void query_span(const AttnParams& p, int kj, int len,
   if (kj >= len) lo = 1, hi = 0;
 }
 __device__ __forceinline__ bool outside(int i, int lo, int hi) { return i < lo || i > hi; }
-
-__device__ __forceinline__ bool masked(const AttnParams& p, int qi, int kj, int len) {
-  if (kj >= len || qi >= len) return true;
-  if (p.causal && kj > qi) return true;
-  if (p.window > 0 && kj <= qi - p.window) return true;
-  return false;
-}
 
 // =====================================================================================
 // forward
