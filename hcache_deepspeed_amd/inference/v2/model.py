@@ -363,7 +363,8 @@ class RaggedTransformer:
         """Replay the decode step for ``batch.current_sequences`` sequences: the graph reads the step's token ids and
         metadata from the batch's device buffer (``RaggedBatchWrapper.finalize``), replays every layer's kernels with
         one launch, and the logits are copied out. A graph of before that buffer grew keeps the old one, into which
-        they are copied. The first step of a batch size runs the forward eagerly over the same buffers, for a size may come once; the second captures it.
+        they are copied. The first step of a batch size runs the forward eagerly over the same buffers, for a size may
+        come once; the second captures it.
 
         ``capture_latents``: the graph also stores each layer's latent rows into a device ring slot (HCache during
         decode, reference llama_v2/model.py:211-218 captures in every forward); returns ``(logits, latents)`` with

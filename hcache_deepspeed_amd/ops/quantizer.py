@@ -211,8 +211,9 @@ def int_linear(x, q_weight, scales, out_features, in_features, group_size, bits=
     """y = x @ dequant(W)^T for a symmetric group-quantized int8/int4 weight [out, in] (groups along ``in``).
 
     Up to 16 rows stream the packed weight through the matrix cores (``_wmix_skinny``, groups of a multiple of 128; one row
-    of int8 and other groups up to 2 rows, ``HDS_INT_GEMV_MAX_M``: the HIP GEMV of csrc/kernels/quant.hip); batches of up to 64 rows run the
-    tile kernel on packed weights, larger ones dequantize once to bf16."""
+    of int8, other groups and a bias that is not bf16 up to 2 rows, ``HDS_INT_GEMV_MAX_M``: the HIP GEMV of
+    csrc/kernels/quant.hip); batches of up to 64 rows run the tile kernel on packed weights, larger ones and groups that do
+    not divide a row dequantize once to bf16."""
     lead = x.shape[:-1]
     x2 = x.reshape(-1, in_features)
     M = x2.shape[0]
