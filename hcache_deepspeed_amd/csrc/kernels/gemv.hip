@@ -378,7 +378,7 @@ int launch_row(const OneRow& p, const Gather& gather, hipStream_t st) {
 // The VALU GEMV above spends 4 dot2 instructions per 16-B weight chunk PER ROW, so from a few rows on it is VALU-bound
 // (o projection at M = 8: 1.7 TB/s) and hipBLASLt's small-M tiles stream at 3.5-3.7 TB/s. Here one
 // mfma_f32_16x16x32_bf16 contracts a 16-row x 32-k weight tile with all (up to 16) token rows at once, so the
-// kernels are pure weight streams: A = W rows (lane l: row l & 15, k = 8 (l >> 4) .. +8), B = x^T
+// kernel is a pure weight stream: A = W rows (lane l: row l & 15, k = 8 (l >> 4) .. +8), B = x^T
 // (lane l: token l & 15, same k), C: token = l & 15, weight row 4 (l >> 4) + reg. A workgroup owns 16
 // weight rows; its waves share K, and the partial tiles are summed through LDS.
 // GLU: W is [gate; up] of 2 N rows, a tile is 8 gate rows and the 8 up rows that belong to them, so that there are as many
@@ -433,51 +433,19 @@ __device__ __forceinline__ void skinny_store(const SkinnyOut& o, const Gather& g
   }
 }
 
-// Up to 4 tokens: weights straight into the operand's registers, 16-B pieces of 16 rows a load. Four waves take turns at
-// 32 U columns (at K below that times four, a quarter each): [4096, 14336] at 3 rows 25.0 us with a quarter of K a wave, 22.1
-// in turns.
-template <int U, bool GATHER, bool GLU>
-__global__ __launch_bounds__(256) void skinny_mfma_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w, int K,
-                                                          int64_t ldx, SkinnyOut o, Gather gather) {
-  __shared__ f32x4 red[3][64];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int part = min(32 * U, K >> 2);  // K % 128 == 0
-  const bf16* wp = w + skinny_row<GLU>(lane & 15, o.N) * K + 8 * (lane >> 4);
-  const bf16* xp = x + (int64_t)min(lane & 15, o.M - 1) * ldx + 8 * (lane >> 4);  // (columns past M are not stored)
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = wid * part; k0 < K; k0 += 4 * part) {
-    const int k1 = min(k0 + part, K);
-    if (k1 - k0 == 32 * U) {
-      bf16x8_t a[U], b[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) a[u] = *reinterpret_cast<const bf16x8_t*>(wp + k0 + 32 * u);
-#pragma unroll
-      for (int u = 0; u < U; ++u) b[u] = *reinterpret_cast<const bf16x8_t*>(xp + k0 + 32 * u);
-      __builtin_amdgcn_sched_barrier(0);  // all loads first: the compiler moves some behind the first products
-#pragma unroll
-      for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u], acc, 0, 0, 0);
-    } else {
-      for (int k = k0; k < k1; k += 32)
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(wp + k),
-                                                      *reinterpret_cast<const bf16x8_t*>(xp + k), acc, 0, 0, 0);
-    }
-  }
-  if (wid > 0) red[wid - 1][lane] = acc;
-  __syncthreads();
-  if (wid > 0) return;
-#pragma unroll
-  for (int v = 0; v < 3; ++v) acc += red[v][lane];
-  skinny_store<GATHER, GLU>(o, gather, acc, lane);
-}
-
-// 5 to 16 tokens. The tokens are then as many bytes of loads as the weights, served by the L2, and what bounds the kernel
-// above is how many cache lines a CU can have on the way: its loads ask for half a line of 16 weight rows each. Here a load
-// takes whole lines (8 rows of 64 columns), which pass through the wave's own piece of LDS into the operand's layout
-// (16-B pieces, placed by row ^ piece so that the reads spread over the banks); a wave has 128 columns in flight and there
-// are up to 32 waves a CU to overlap them. 16 rows, the kernel above -> this one: [28672, 4096] 60 -> 48.0 us (4.9 TB/s),
-// [4096, 14336] 29.8 -> 26.5, [6144, 4096] 17.6 -> 13.5, [32000, 4096] 66 -> 53 (library 57); 7 rows: 45.6 -> 40.1, 26.1 -> 23.8,
-// 14.1 -> 12.2, 50.6 -> 44.7; at 3 rows the kernel above is ahead at K = 2048 ([16384, 2048] 13.4 against 15.7) and level
-// elsewhere. Two tiles a workgroup halve the tokens' loads but were slower (54 to 59 us), the DMA into LDS is level.
+// The tokens are as many bytes of loads as the weights, served by the L2, and what bounds such a kernel is how many cache
+// lines a CU can have on the way; with 16-B pieces of 16 weight rows, straight into the operand's registers, a load asks
+// for half a line of each. Here a load takes whole lines (8 rows of 64 columns), which pass through the wave's own piece
+// of LDS into the operand's layout (16-B pieces, placed by row ^ piece so that the reads spread over the banks); a wave has
+// 128 columns in flight and there are up to 32 waves a CU to overlap them. Pieces (a quarter of K a wave) -> this, 2 / 4 / 8
+// / 16 rows: [28672, 4096] 40.1 / 42.0 / 48.1 / 60.6 -> 39.6 / 40.0 / 41.3 / 48.8 us (4.8 TB/s at 16), [4096, 14336] 26.8 / 25.8 /
+// 26.9 / 29.9 -> 22.8 / 22.1 / 22.4 / 25.5, [6144, 4096] 13.5 / 13.5 / 14.7 / 17.6 -> 12.8 / 12.2 / 12.7 / 13.8, [2048, 5632]
+// 13.0 / 13.0 / 13.6 / 15.1 -> 8.7 / 7.7 / 8.5 / 10.2, [32000, 2048] 25.2 / 25.7 / 29.7 / 36.4 -> 24.9 / 25.4 / 26.2 / 29.9. Two
+// tiles a workgroup halve the tokens' loads but were slower (54 to 59 us), the DMA into LDS is level.
+// Weight rows of a multiple of 4 KB lie alike in the memory's channels, and workgroups that walk them side by side meet in
+// the same ones. There each begins somewhere else, by the fractions of the golden ratio (any distance apart is far apart):
+// 8 rows, [4096, 16384] 35.8 -> 24.0 us, [4096, 32768] 60 -> 46, [4096, 4096] 8.5 -> 7.7, [32000, 2048] level. With other rows
+// it gains or loses up to 4 % ([5120, 13824]), with gate and up rows, which are a matrix apart, nothing.
 template <int NW, bool GATHER, bool GLU>
 __global__ __launch_bounds__(64 * NW) void skinny_lines_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                                                int K, int64_t ldx, SkinnyOut o, Gather gather) {
@@ -492,7 +460,10 @@ __global__ __launch_bounds__(64 * NW) void skinny_lines_kernel(const bf16* __res
   const char* get0 = mine + rr * 128 + (rp ^ (rr & 7)) * 16;
   const char* get1 = mine + rr * 128 + ((rp + 4) ^ (rr & 7)) * 16;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k = 128 * wid; k < K; k += 128 * NW) {  // K % 128 == 0
+  const int parts = K >> 7, turn = GLU || K % 2048 ? 0 : (int)__umulhi(blockIdx.x * 2654435769u, (unsigned)parts);
+  for (int c = wid; c < parts; c += NW) {  // K % 128 == 0
+    int k = c + turn;
+    k = (k < parts ? k : k - parts) << 7;
     bf16x8_t a[2][2], b[4];
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
@@ -523,8 +494,6 @@ __global__ __launch_bounds__(64 * NW) void skinny_lines_kernel(const bf16* __res
   skinny_store<GATHER, GLU>(o, gather, acc, lane);
 }
 
-int g_skinny_u = 16;
-
 // Waves a workgroup: four where there are at least two workgroups a CU of whole K walks ([6144, 4096] 13.7 us against 14.7
 // with eight, [28672, 4096] 48.6 / 50.4), eight where those are few ([4096, 14336] 26.6 against 27.9, [2048, 8192] 13.0 / 14.0)
 // or short ([16384, 2048] 17.9 / 19.0), and at up to 8 rows, whose tokens take fewer loads ([28672, 4096], 7 rows: 40.1 / 41.7).
@@ -534,18 +503,10 @@ int launch_skinny(const void* x, const void* w, int K, int64_t ldx, const Skinny
   const int per = GLU ? 8 : 16, tiles = (o.N + per - 1) / per;
 #define HDS_SK(T, ...) \
   hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(T), 0, st, (const bf16*)x, (const bf16*)w, K, ldx, o, gather)
-  if (o.M > 4 || K < 2048) {  // (a wave of the other kernel wants 16 loads a turn)
-    if (o.M > 8 && tiles > 256 && K >= 4096)
-      HDS_SK(256, skinny_lines_kernel<4, GATHER, GLU>);
-    else
-      HDS_SK(512, skinny_lines_kernel<8, GATHER, GLU>);
-  } else if (g_skinny_u == 32 && K % 1024 == 0) {
-    HDS_SK(256, skinny_mfma_kernel<32, GATHER, GLU>);
-  } else if (g_skinny_u >= 16) {
-    HDS_SK(256, skinny_mfma_kernel<16, GATHER, GLU>);
-  } else {
-    HDS_SK(256, skinny_mfma_kernel<8, GATHER, GLU>);
-  }
+  if (o.M > 8 && tiles > 256 && K >= 4096)
+    HDS_SK(256, skinny_lines_kernel<4, GATHER, GLU>);
+  else
+    HDS_SK(512, skinny_lines_kernel<8, GATHER, GLU>);
 #undef HDS_SK
   return hipGetLastError();
 }
@@ -655,13 +616,6 @@ HDS_EXPORT int hds_skinny_gemm_bf16(const void* x, const void* w, const void* bi
   const SkinnyOut o{(const bf16*)bias, (bf16*)y, M, N, ldy, glu - 1};
   return glu ? launch_skinny<false, true>(x, w, K, ldx, o, Gather{}, st)
              : launch_skinny<false, false>(x, w, K, ldx, o, Gather{}, st);
-}
-
-// weight loads per lane in flight in the skinny GEMM of up to 4 rows (8, 16 or 32); returns the previous value
-HDS_EXPORT int hds_skinny_set_unroll(int u) {
-  const int prev = g_skinny_u;
-  g_skinny_u = u >= 32 ? 32 : (u >= 16 ? 16 : 8);
-  return prev;
 }
 
 // Fused decode GEMV (see gemv_fused_kernel): y[M, N] = norm(h (+ res)) . W^T, or with glu = 1 + activation code

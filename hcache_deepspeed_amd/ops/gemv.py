@@ -44,7 +44,7 @@ def gemv(x2, w, b=None):
     return y
 
 
-# 2..16 token rows: the matrix-core skinny GEMM (csrc/kernels/gemv.hip skinny_mfma_kernel) instead of the VALU GEMV /
+# 2..16 token rows: the matrix-core skinny GEMM (csrc/kernels/gemv.hip skinny_lines_kernel) instead of the VALU GEMV /
 # hipBLASLt's small-M tiles (HDS_SKINNY_GEMM=0: those)
 SKINNY = _os.environ.get("HDS_SKINNY_GEMM", "1") == "1"
 SKINNY_MIN_M = int(_os.environ.get("HDS_SKINNY_MIN_M", "2"))  # 1: one-row linears too (instead of the VALU GEMV)

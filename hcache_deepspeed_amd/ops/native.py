@@ -118,7 +118,6 @@ _KERNEL_SIGS = {
     "hds_gemv_fused_bf16": "ppp" + "f" + "pppp" + "if" + "iii" + "ll" + "s",
     "hds_gather_gemv_bf16": "ppp" + "l" + "p" + "ii" + "p" + "iii" + "ll" + "s",
     "hds_skinny_gemm_bf16": "pppp" + "iii" + "ll" + "i" + "s",
-    "hds_skinny_set_unroll": "i",
     "hds_wmix_splits": "iii",
     "hds_wmix_supported": "iiii",
     "hds_paged_prefill": "pl" + "p" + "pl" + "pi" + "pp" + "iiii" + "f" + "i" + "s",
@@ -230,9 +229,6 @@ def _klib_init(lib):
         check(lib.hds_attn_fwd_variant(fwd_variant_default()), "hds_attn_fwd_variant")
         # FlashAttention backward dQ kernel (hds_attn_bwd_dq_variant; 1 = one wave per SIMD, 64 rows per wave)
         lib.hds_attn_bwd_dq_variant(int(os.environ.get("HDS_ATTN_DQ_VAR", "0")))
-    if hasattr(lib, "hds_skinny_set_unroll"):
-        # skinny GEMM weight loads in flight per lane (16: B = 4 decode 925 vs 881 tok/s with 8, profiles/r6/skinny_u)
-        lib.hds_skinny_set_unroll(int(os.environ.get("HDS_SKINNY_U", "16")))
 
 
 # FlashAttention forward variants of the shipped library (flash_attn.hip hds_attn_fwd_variant): 20 the default, 5 the

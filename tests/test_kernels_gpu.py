@@ -877,11 +877,28 @@ def test_one_row_edges(N, K, kind):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [2, 3, 8, 16])
+@pytest.mark.parametrize("N,K", [(4113, 2048), (33, 4096), (4113, 4096), (17, 6144), (300, 16384), (7, 32768)])
+def test_skinny_gemm_walks_every_column_once(M, N, K):
+    """Rows of a multiple of 4 KB, whose walks begin at different places: small integers, whose sums are exact in 32 bits
+    and the result in bf16."""
+    from hcache_deepspeed_amd.ops.gemv import gather_gemv, skinny
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    rnd = lambda *s: torch.randint(-1, 2, s, device="cuda", generator=g)  # noqa: E731
+    w, x = rnd(N, K).bfloat16(), (rnd(M, K) * (torch.rand(M, K, device="cuda", generator=g) < 0.1)).bfloat16()
+    ref = x.float() @ w.float().t()
+    assert ref.abs().max() <= 256
+    assert torch.equal(skinny(x, w).float(), ref)
+    table, ids = rnd(5, N).bfloat16(), torch.arange(M, device="cuda") % 5
+    assert torch.equal(gather_gemv(x, w, "relu", table, ids).float(), torch.relu(ref) * table[ids].float())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("act", [None, "silu", "gelu_tanh", "relu"])
 @pytest.mark.parametrize("M", [2, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("N,K", [(7, 128), (1000, 640), (16, 2048), (4104, 2176), (24, 4224), (4112, 4096)])
 def test_skinny_gemm_edges(act, M, N, K):
-    """Both skinny kernels and their gated form against 64 bits: tiles with a remainder, K shorter than a workgroup's waves
+    """The skinny kernel and its gated form against 64 bits: tiles with a remainder, K shorter than a workgroup's waves
     take and no multiple of it. 32-bit sums of K products, then one rounding; gated: the projections rounded first."""
     from hcache_deepspeed_amd.ops.gemv import glu_linear, skinny
     g = torch.Generator(device="cuda").manual_seed(M * 13 + N)
