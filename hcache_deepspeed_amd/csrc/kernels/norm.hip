@@ -28,15 +28,17 @@ constexpr int kFewRows = 64;
 // ---------------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------------
-// pick (may be null): output row i is made from rows pick[i] of x and res, of which there are n_in; negative ones count from
-// the end, and a row outside them gives NaN. A serving step normalises only the rows whose logits are wanted: gathering
+// PICK: output row i is made from rows pick[i] of x and res, of which there are n_in; negative ones count from
+// the end, and a row outside them gives NaN (a kernel of its own: asked for at run time it cost every norm 0.1 us, 3 to 5 %
+// of 256 rows of 512 to 2,048). A serving step normalises only the rows whose logits are wanted: gathering
 // them first took four launches (two index conversions, two gathers; 18 us of a 490 us decode step of 16 sequences).
 struct PickedRow {
   int row;
   bool ok;
 };
+template <bool PICK>
 __device__ __forceinline__ PickedRow picked_row(const int* pick, int row, int n_in) {
-  if (pick == nullptr) return {row, true};
+  if constexpr (!PICK) return {row, true};
   int r = pick[row];
   if (r < 0) r += n_in;
   const bool ok = r >= 0 && r < n_in;
@@ -59,7 +61,7 @@ __device__ __forceinline__ float row_sum(float v, float* red) {
 
 // WPR waves take a row. The few rows of a decode step would leave the latencies of a whole row's loads and stores to one wave
 // each: with a residual, 16 rows of 2048 / 4096 / 8192 2.6 / 3.4 / 5.1 us, with four waves a row 2.1 / 2.4 / 2.7.
-template <typename T, typename WT, int NV, bool LN, int WPR>
+template <typename T, typename WT, int NV, bool LN, int WPR, bool PICK>
 __global__ __launch_bounds__(256) void norm_fwd_kernel(const T* __restrict__ x, const T* __restrict__ res,
                                                        T* __restrict__ res_out, const WT* __restrict__ w,
                                                        const WT* __restrict__ b, T* __restrict__ y,
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const T* __restrict__ x, 
   const bool live = row_at < rows;  // (the waves of a workgroup stay together for the sums)
   const int row = live ? row_at : rows - 1;
   const int c0 = (wid % WPR * V * 64 + lane) * 8;
-  const PickedRow in = picked_row(pick, row, n_in);
+  const PickedRow in = picked_row<PICK>(pick, row, n_in);
   const T* xr = x + (int64_t)in.row * cols;
   float v[V][8], wv[V][8];
 #pragma unroll
@@ -144,7 +146,7 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const T* __restrict__ x, 
 }
 
 // Generic-width forward (cols % 8 == 0, any cols): two passes over the row (second hits L1/L2).
-template <typename T, typename WT, bool LN>
+template <typename T, typename WT, bool LN, bool PICK>
 __global__ __launch_bounds__(256) void norm_fwd_generic(const T* __restrict__ x, const T* __restrict__ res,
                                                         T* __restrict__ res_out, const WT* __restrict__ w,
                                                         const WT* __restrict__ b, T* __restrict__ y,
@@ -154,7 +156,7 @@ __global__ __launch_bounds__(256) void norm_fwd_generic(const T* __restrict__ x,
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
   if (row >= rows) return;
-  const PickedRow in = picked_row(pick, row, n_in);
+  const PickedRow in = picked_row<PICK>(pick, row, n_in);
   const T* xr = x + (int64_t)in.row * cols;
   const T* rr = res ? res + (int64_t)in.row * cols : nullptr;
   T* ro = res_out ? res_out + (int64_t)row * cols : nullptr;
@@ -387,10 +389,10 @@ __global__ __launch_bounds__(1024) void reduce_parts_kernel(const float* __restr
   out[c] = from_f<WT>(t);
 }
 
-template <typename T, typename WT, bool LN>
-hipError_t launch_fwd(const void* x, const void* res, void* res_out, const void* w, const void* b, void* y,
-                      float* mean, float* rstd, int rows, int cols, float eps, const int* pick, int n_in,
-                      hipStream_t st) {
+template <typename T, typename WT, bool LN, bool PICK>
+hipError_t launch_fwd_rows(const void* x, const void* res, void* res_out, const void* w, const void* b, void* y,
+                           float* mean, float* rstd, int rows, int cols, float eps, const int* pick, int n_in,
+                           hipStream_t st) {
   auto args = [&](auto kern, int wpr) {
     hipLaunchKernelGGL(kern, dim3((rows * wpr + kRowsPerBlock - 1) / kRowsPerBlock), dim3(256), 0, st, (const T*)x,
                        (const T*)res, (T*)res_out, (const WT*)w, (const WT*)b, (T*)y, mean, rstd, rows, cols, eps, pick, n_in);
@@ -399,11 +401,11 @@ hipError_t launch_fwd(const void* x, const void* res, void* res_out, const void*
   // 93): longer steps, the training ones among them, keep the sums of one wave in their order.
 #define HDS_NF(COLS, NV, WPR)                                              \
   case COLS:                                                               \
-    if (rows <= kFewRows) args(norm_fwd_kernel<T, WT, NV, LN, WPR>, WPR);  \
-    else args(norm_fwd_kernel<T, WT, NV, LN, 1>, 1);                       \
+    if (rows <= kFewRows) args(norm_fwd_kernel<T, WT, NV, LN, WPR, PICK>, WPR); \
+    else args(norm_fwd_kernel<T, WT, NV, LN, 1, PICK>, 1);                 \
     break
   switch (cols) {
-    case 512: args(norm_fwd_kernel<T, WT, 1, LN, 1>, 1); break;
+    case 512: args(norm_fwd_kernel<T, WT, 1, LN, 1, PICK>, 1); break;
     HDS_NF(1024, 2, 2);
     HDS_NF(2048, 4, 4);
     HDS_NF(3072, 6, 2);
@@ -411,10 +413,19 @@ hipError_t launch_fwd(const void* x, const void* res, void* res_out, const void*
     HDS_NF(5120, 10, 2);
     HDS_NF(6144, 12, 4);
     HDS_NF(8192, 16, 4);
-    default: args(norm_fwd_generic<T, WT, LN>, 1); break;
+    default: args(norm_fwd_generic<T, WT, LN, PICK>, 1); break;
   }
 #undef HDS_NF
   return hipGetLastError();
+}
+
+template <typename T, typename WT, bool LN>
+hipError_t launch_fwd(const void* x, const void* res, void* res_out, const void* w, const void* b, void* y,
+                      float* mean, float* rstd, int rows, int cols, float eps, const int* pick, int n_in,
+                      hipStream_t st) {
+  if (pick != nullptr)
+    return launch_fwd_rows<T, WT, LN, true>(x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, pick, n_in, st);
+  return launch_fwd_rows<T, WT, LN, false>(x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, pick, n_in, st);
 }
 
 template <typename T, typename WT, bool LN>
