@@ -499,6 +499,9 @@ struct PagedDecodeParams {
   // HIP-graph replay finds it zeroed again.
   int* counters;
   int tiles;  // the matrix-core kernel: splits are runs of whole tiles of 32 positions
+  // the others: keys that a workgroup takes at a time. One number for all (64) left heads of 256 with too few splits at work:
+  // 16 / 1 heads, 16 tokens, up to 300 keys 36.5 us, with the kernel's own turn of 16 25.8; 64 tokens 40.4 and 34.4
+  int turn;
 };
 
 struct DecodeToken {
@@ -515,8 +518,6 @@ __device__ __forceinline__ DecodeToken decode_token(const PagedDecodeParams<T>& 
 // this split's keys: an equal share of what the token sees, counted without the gap between the kept keys and the others,
 // but no less than one turn of a workgroup: of the launched splits only the first `used` have keys then, and only those
 // are merged
-constexpr int kDecKeys = 64;
-
 struct DecodeKeys {
   int j0, j1, keep, gap, used;
   __device__ __forceinline__ int pos(int j) const { return j < keep ? j : j + gap; }
@@ -524,7 +525,7 @@ struct DecodeKeys {
 template <typename T>
 __device__ __forceinline__ DecodeKeys decode_keys(const PagedDecodeParams<T>& p, int pos, int split) {
   const int gap = max(first_key(pos, p.window, p.chunk) - p.keep, 0), n = pos + 1 - gap;
-  const int per = max((n + p.splits - 1) / p.splits, min(n, kDecKeys));
+  const int per = max((n + p.splits - 1) / p.splits, min(n, p.turn));
   return {split * per, min(n, split * per + per), p.keep, gap, (n + per - 1) / per};
 }
 
@@ -584,10 +585,14 @@ __device__ __forceinline__ float dot8(const bf16x8& a, const bf16x8& b) {
   return c;
 }
 
+// keys of a lane group on their way (registers)
+template <int GM>
+constexpr int kDecUnroll = GM >= 8 ? 2 : 4;
+
 template <int LPK, int GM>
 __global__ __launch_bounds__(256) void paged_decode_kernel(PagedDecodeParams<bf16> p) {
   constexpr int KPW = 64 / LPK;
-  constexpr int U = GM >= 8 ? 2 : 4;  // (registers)
+  constexpr int U = kDecUnroll<GM>;
   __shared__ float red[4][GM][2 + 8 * LPK];
   const int G = p.hq / p.hkv, gb = (G + GM - 1) / GM;
   const int split = blockIdx.x, hk = blockIdx.y / gb, g0 = (blockIdx.y % gb) * GM, b = blockIdx.z;
@@ -1091,10 +1096,13 @@ void launch_combine(const PagedDecodeParams<T>& p, int n, hipStream_t st) {
 }
 
 template <int LPK>
-int launch_decode(const PagedDecodeParams<bf16>& p, int n, hipStream_t st) {
+int launch_decode(PagedDecodeParams<bf16> p, int n, hipStream_t st) {
   const int G = p.hq / p.hkv;
 #define HDS_DEC(GM)                                                                                                 \
-  hipLaunchKernelGGL((paged_decode_kernel<LPK, GM>), dim3(p.splits, p.hkv * ((G + GM - 1) / GM), n), dim3(256), 0, st, p)
+  do {                                                                                                              \
+    p.turn = 4 * (64 / LPK) * kDecUnroll<GM>;                                                                       \
+    hipLaunchKernelGGL((paged_decode_kernel<LPK, GM>), dim3(p.splits, p.hkv * ((G + GM - 1) / GM), n), dim3(256), 0, st, p); \
+  } while (0)
   if (G == 1) HDS_DEC(1); else if (G == 2) HDS_DEC(2); else if (G <= 4) HDS_DEC(4); else HDS_DEC(8);
 #undef HDS_DEC
   if (p.splits > 1 && p.counters == nullptr) launch_combine(p, n, st);
@@ -1116,7 +1124,8 @@ int launch_decode_mfma(PagedDecodeParams<bf16> p, const DecodeRope& rope, int n,
 }
 
 template <typename T>
-int launch_plain(const PagedDecodeParams<T>& p, int n, hipStream_t st) {
+int launch_plain(PagedDecodeParams<T> p, int n, hipStream_t st) {
+  p.turn = kPlainKeys;
   const size_t lds = (p.dk + p.dv + kPlainKeys) * sizeof(float);
   if (lds > 64 * 1024 || p.hq > 65535) return hipErrorInvalidValue;
   hipLaunchKernelGGL(paged_plain_kernel<T>, dim3(p.splits, p.hq, n), dim3(256), lds, st, p);
@@ -1256,12 +1265,12 @@ HDS_EXPORT int hds_paged_decode(int dtype, int plain, const void* q, int64_t sq,
     return launch_plain(PagedDecodeParams<float>{(const float*)q, sq, (const float*)cache, (float*)o, so, part_o,
                                                  part_ml, seq_meta, toks, tok_seq, tok_pos, block_tables, max_blocks,
                                                  block_size, hq, hkv, dk, dv, splits, scale, window, chunk, keep, softcap,
-                                                 sink, (const float*)gate, sg, gw, nullptr, 0}, n, st);
+                                                 sink, (const float*)gate, sg, gw, nullptr, 0, 0}, n, st);
   }
   if (dtype != kBF16) return hipErrorInvalidValue;
   PagedDecodeParams<bf16> p{(const bf16*)q, sq, (const bf16*)cache, (bf16*)o, so, part_o, part_ml, seq_meta, toks,
                             tok_seq, tok_pos, block_tables, max_blocks, block_size, hq, hkv, dk, dv, splits, scale,
-                            window, chunk, keep, softcap, sink, (const bf16*)gate, sg, gw, counters, 0};
+                            window, chunk, keep, softcap, sink, (const bf16*)gate, sg, gw, counters, 0, 0};
   if (plain) {
     p.counters = nullptr;
     return launch_plain(p, n, st);
@@ -1291,7 +1300,7 @@ HDS_EXPORT int hds_paged_decode_qkv(const void* qkv, int64_t sq, void* cache, vo
     return hipErrorInvalidValue;
   PagedDecodeParams<bf16> p{(const bf16*)qkv, sq, (const bf16*)cache, (bf16*)o, so, part_o, part_ml, seq_meta, nullptr,
                             nullptr, nullptr, block_tables, max_blocks, block_size, hq, hkv, 128, 128, splits, scale,
-                            window, 0, 0, 0.f, nullptr, nullptr, 0, 1, nullptr, 0};
+                            window, 0, 0, 0.f, nullptr, nullptr, 0, 1, nullptr, 0, 0};
   if (!decode_mfma_ok(p)) return hipErrorInvalidValue;
   return launch_decode_mfma<true>(p, DecodeRope{(bf16*)cache, cos_t, sin_t, rot}, n, st);
 }

@@ -74,6 +74,20 @@ def test_decode_splits_and_merge(D, nq, nkv, lens, mb):
     assert ((got.double() - ref).abs() <= 2**-8 * ref.abs() + 2e-4).all()
 
 
+@pytest.mark.parametrize("D,nq,nkv,turn", [(256, 16, 1, 16), (256, 8, 8, 32), (64, 34, 2, 64), (64, 2, 2, 128), (80, 2, 2, 64)])
+def test_decode_splits_of_one_turn(D, nq, nkv, turn):
+    """Lengths around one and two turns of a workgroup of the vector kernel, where the number of splits with keys changes."""
+    lens = [1, turn - 1, turn, turn + 1, 2 * turn - 1, 2 * turn, 2 * turn + 1, 9 * turn + 3]
+    scale = D**-0.5
+    cache, tables, meta, qkv = _setup(lens, nq, nkv, D, 64, 20, seed=4)
+    seq = torch.arange(len(lens), dtype=torch.int32, device="cuda")
+    kv_rope_scatter(qkv, cache, seq, meta[:, 2].contiguous(), tables, None, None, nq, nkv, do_rope=False)
+    got = paged_attention(qkv[:, :nq], cache, None, 0, meta, tables, nq, nkv, scale, decode=True)
+    ref = _exact(qkv[:, :nq], cache, tables, lens, nq, nkv, scale, 0)
+    # one rounding of the result; 32-bit sums and exponentials in front of it (|v| <= 6)
+    assert ((got.double() - ref).abs() <= 2**-8 * ref.abs() + 2e-4).all()
+
+
 @pytest.mark.parametrize("sink", [False, True])
 @pytest.mark.parametrize("gate_width", [0, 1, 128])
 @pytest.mark.parametrize("window", [0, 50])
