@@ -1109,6 +1109,17 @@ int launch_decode(PagedDecodeParams<bf16> p, int n, hipStream_t st) {
   return hipGetLastError();
 }
 
+// Where it is the faster one. The 16 columns of its tiles are the query heads of a key head: with one or two of those most are
+// empty, and the launch that it saves counts for less the more (token, key head) pairs there are. With G heads a key head the
+// measured line is at 256 G^2 pairs; us, this kernel against the rotation's launch and the vector kernel, windows of 256 keys:
+// 32 / 32 heads, 4 tokens 12.4 / 11.9 (50 keys 10.7 / 11.6), 8 tokens 16.1 / 14.7, 16 20.1 / 17.7, 64 67.3 / 47.7;
+// 32 / 16 heads, 16 tokens 16.4 / 16.2 (50 keys 11.4 / 13.1), 32 20.0 / 19.4 (50 keys 7.7 / 9.6), 64 34.2 / 30.3;
+// 24 / 8 heads, 64 tokens 20.3 / 20.6.
+bool decode_mfma_wins(int n, int hq, int hkv) {
+  const int64_t G = hq / hkv;
+  return (int64_t)n * hkv < 256 * G * G;
+}
+
 // tokens of plain heads of 128: the matrix-core kernel
 bool decode_mfma_ok(const PagedDecodeParams<bf16>& p) {
   return p.dk == 128 && p.dv == 128 && p.hq / p.hkv <= 16 && p.block_size % 32 == 0 && p.chunk == 0 && p.keep == 0 &&
@@ -1278,12 +1289,17 @@ HDS_EXPORT int hds_paged_decode(int dtype, int plain, const void* q, int64_t sq,
   if (!hds_paged_decode_supported(dk, dv) || sq % 8 || so % 8 || hkv > 65535 / kDecGMax ||
       (counters != nullptr && hq / hkv > kDecGMax))
     return hipErrorInvalidValue;
-  if (decode_mfma_ok(p)) return launch_decode_mfma<false>(p, DecodeRope{}, n, st);
+  if (decode_mfma_ok(p) && decode_mfma_wins(n, hq, hkv)) return launch_decode_mfma<false>(p, DecodeRope{}, n, st);
   const int d = dk > dv ? dk : dv;
   if (d <= 32) return launch_decode<4>(p, n, st);
   if (d <= 64) return launch_decode<8>(p, n, st);
   if (d <= 128) return launch_decode<16>(p, n, st);
   return launch_decode<32>(p, n, st);
+}
+
+// Is such a step faster by hds_paged_decode_qkv than by a launch for rotation and append and hds_paged_decode?
+HDS_EXPORT int hds_paged_decode_qkv_wins(int n, int hq, int hkv) {
+  return hkv > 0 && hq >= hkv && decode_mfma_wins(n, hq, hkv);
 }
 
 // A step of n single tokens, one of each sequence, from its projection: qkv [n, hq + 2 hkv, 128] with token stride sq is

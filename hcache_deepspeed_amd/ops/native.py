@@ -146,6 +146,7 @@ _KERNEL_SIGS = {
     "hds_nhwc_bias_add": "i" + "ppppp" + "l" + "ii" + "s",
     "hds_paged_decode_supported": "ii",
     "hds_paged_decode_splits": "iii",
+    "hds_paged_decode_qkv_wins": "iii",
     "hds_paged_decode_qkv": "pl" + "p" + "pl" + "ppppi" + "iiiii" + "f" + "i" + "ppi" + "s",
     "hds_paged_decode": "ii" + "pl" + "p" + "pl" + "pp" + "ppppp" + "i" * 8 + "f" + "iii" + "f" + "pp" + "li" + "p" + "s",
     "hds_copy_d2h": "pp" + "l" + "i" + "s",

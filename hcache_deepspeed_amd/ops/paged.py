@@ -160,7 +160,7 @@ def paged_attention(q, cache, atoms, n_atoms, seq_meta, block_tables, n_q, n_kv,
 
 
 def decode_qkv_ok(qkv, cache, n_q, n_kv, cos, sin, rotary_dim=0):
-    """Does ``paged_decode_qkv`` take this projection [T, n_q + 2 n_kv, D], cache and rotation?"""
+    """Does ``paged_decode_qkv`` take this projection [T, n_q + 2 n_kv, D], cache and rotation, and is it the faster way?"""
     if not (native.use_native(qkv) and qkv.dtype == torch.bfloat16 and cache.dtype == qkv.dtype and cache.dim() == 5):
         return False
     rot = rotary_dim or 128
@@ -170,7 +170,8 @@ def decode_qkv_ok(qkv, cache, n_q, n_kv, cos, sin, rotary_dim=0):
     return (rope_ok and not _MERGE_IN_KERNEL and qkv.shape[2] == 128 and n_q % n_kv == 0 and n_q // n_kv <= 16
             and qkv.shape[1] == n_q + 2 * n_kv and qkv.stride(2) == 1 and qkv.stride(1) == 128 and qkv.stride(0) % 8 == 0
             and qkv.data_ptr() % 16 == 0 and cache.is_contiguous() and cache.shape[1] % 32 == 0
-            and tuple(cache.shape[2:]) == (2, n_kv, 128) and cache.data_ptr() % 16 == 0)
+            and tuple(cache.shape[2:]) == (2, n_kv, 128) and cache.data_ptr() % 16 == 0
+            and bool(native.kernels().hds_paged_decode_qkv_wins(qkv.shape[0], n_q, n_kv)))
 
 
 def paged_decode_qkv(qkv, cache, seq_meta, block_tables, n_q, n_kv, scale, window, cos, sin, rotary_dim=0):

@@ -88,6 +88,26 @@ def test_decode_splits_of_one_turn(D, nq, nkv, turn):
     assert ((got.double() - ref).abs() <= 2**-8 * ref.abs() + 2e-4).all()
 
 
+@pytest.mark.parametrize("nq,nkv,line", [(8, 8, 32), (32, 16, 64)])
+@pytest.mark.parametrize("over", [0, 1])
+@pytest.mark.parametrize("window", [0, 33])
+def test_few_query_heads_a_key_head_on_both_kernels(nq, nkv, line, over, window):
+    """One token below the number from which the vector kernel is the faster one, and at it: the same step by both ways.
+    Without rotation: the two rotations may round an element differently, and both kernels are to see the same numbers."""
+    T, D, scale = line - 1 + over, 128, 0.11
+    lens = [1 + 7 * (i % 23) for i in range(T)]
+    cache, tables, meta, qkv = _setup(lens, nq, nkv, D, 32, 5, seed=5)
+    seq = torch.arange(T, dtype=torch.int32, device="cuda")
+    want_cache, want_qkv = cache.clone(), qkv.clone()
+    kv_rope_scatter(want_qkv, want_cache, seq, meta[:, 2].contiguous(), tables, None, None, nq, nkv, do_rope=False)
+    ref = _exact(want_qkv[:, :nq], want_cache, tables, lens, nq, nkv, scale, window)
+    plain = paged_attention(want_qkv[:, :nq], want_cache, None, 0, meta, tables, nq, nkv, scale, window, decode=True)
+    fused = paged_decode_qkv(qkv, cache, meta, tables, nq, nkv, scale, window, None, None)
+    assert decode_qkv_ok(qkv, cache, nq, nkv, None, None) == (over == 0)
+    for got in (plain, fused):  # one rounding of the result; 32-bit sums and exponentials in front of it (|v| <= 6)
+        assert ((got.double() - ref).abs() <= 2**-8 * ref.abs() + 2e-4).all()
+
+
 @pytest.mark.parametrize("sink", [False, True])
 @pytest.mark.parametrize("gate_width", [0, 1, 128])
 @pytest.mark.parametrize("window", [0, 50])
