@@ -361,12 +361,30 @@ __global__ __launch_bounds__(256) void gemv_row_kernel(OneRow p, Gather gather) 
   }
 }
 
-// Two pieces a wave on the way where K has them for all waves and N leaves several rounds of workgroups ([2 x 14336, 4096] 41.9
-// us with one piece, 38.6 with two; [6144, 4096] 12.0 / 12.3, [2 x 5632, 2048] 10.7 / 13.8).
+// One row: where the kernels above, a column (or a few) of a wave, are still the faster ones. A turn of gemv_row_kernel is 2048 of
+// K, and with a norm each pair of columns reads h and gamma again. us, this kernel / those:
+// K up to 1024 (half of its waves have nothing to read): [1024, 512] 2.31 / 2.07, [3072, 1024] 3.36 / 3.16, [16384, 256] 6.86 / 4.32;
+// with a norm [16384, 1024] 12.1 / 9.3. K = 768 is a piece and a half of those, which they make up for from 6144 columns on: [512,
+// 768] 2.31 / 2.38, [6144, 768] 4.19 / 3.90;
+// plain, K to 2048 and few columns: [2048, 2048] 3.61 / 3.44, [3072, 2048] 4.51 / 4.35, [4096, 2048] 5.16 / 5.46;
+// a norm before many columns: [27648, 5120] 57.9 / 53.7, [28672, 14336] 163 / 152, [16384, 2560] 19.7 / 18.5; of K = 2048, 4096, 6144 and
+// 8192, whole turns, this one: [16384, 2048] 14.8 / 17.9, [28672, 4096] 45.7 / 47.3, [12288, 6144] 31.4 / 34.0;
+// gated without a norm, K of no whole turns: [2 x 2048, 2560] 6.6 / 6.4, [2 x 2048, 5120] 10.2 / 9.8, [2 x 4096, 2560] 9.9 / 10.2.
+template <bool NORM, bool GLU>
+bool row_by_columns(int N, int K) {
+  if (K <= 1024) return (GLU && !NORM) || K % 512 == 0 || K < 512 || N >= 6144;
+  if (NORM) return !GLU && N >= 12288 && (K % 2048 != 0 || K > 8192);
+  if (GLU) return K % 2048 != 0 && K <= 5120 && N <= 2048;
+  return K <= 2048 && K % 512 == 0 && N >= 768 && N <= 3072;
+}
+
+// Two pieces a wave on the way instead of one from the second turn on: plain [6144, 2560] 7.6 for 8.2 us, [28672, 4096] 39.7 / 39.5,
+// [12288, 14336] 60.9 / 62.6, gated [2 x 14336, 3072] 31.3 / 32.0. With a norm, whose work a piece past the end repeats, only gated and
+// where K has whole pairs: [2 x 8192, 4096] 26.8 for 27.7, [2 x 14336, 6144] 70.0 for 62.5; not gated [27648, 5120] 64.5 for 57.9.
 template <bool NORM, bool GLU, bool GATHER>
 int launch_row(const OneRow& p, const Gather& gather, hipStream_t st) {
   const dim3 grid((p.N + 1) / 2);
-  if (p.K >= 4096 && p.N >= 12288)
+  if (NORM ? GLU && p.K % 4096 == 0 : p.K > 2048)
     hipLaunchKernelGGL((gemv_row_kernel<2, NORM, GLU, GATHER>), grid, dim3(256), 0, st, p, gather);
   else
     hipLaunchKernelGGL((gemv_row_kernel<1, NORM, GLU, GATHER>), grid, dim3(256), 0, st, p, gather);
@@ -628,7 +646,8 @@ HDS_EXPORT int hds_gemv_fused_bf16(const void* h, const void* res, const void* g
   if (M < 1 || M > 8 || N < 1 || K < 8 || K % 8 || ldh % 8 || glu < 0 || glu > 6 || glu == 4 || glu == 5) return hipErrorInvalidValue;
   const int act = glu - 1;
   if (gamma == nullptr && (r_out != nullptr || x_out != nullptr || res != nullptr)) return hipErrorInvalidValue;
-  if (M == 1) {
+  if (M == 1 && !(gamma != nullptr ? (glu ? row_by_columns<true, true>(N, K) : row_by_columns<true, false>(N, K))
+                                   : row_by_columns<false, true>(N, K))) {
     const OneRow p{(const bf16*)h, (const bf16*)res, (const bf16*)gamma, eps, (const bf16*)w, nullptr, (bf16*)y,
                    (bf16*)r_out, (bf16*)x_out, N, K, act, limit};
     if (gamma != nullptr) return glu ? launch_row<true, true, false>(p, Gather{}, st) : launch_row<true, false, false>(p, Gather{}, st);
@@ -640,7 +659,7 @@ HDS_EXPORT int hds_gemv_fused_bf16(const void* h, const void* res, const void* g
                      (const bf16*)h, (const bf16*)res, (const bf16*)gamma, eps, (const bf16*)w, (bf16*)y,      \
                      (bf16*)r_out, (bf16*)x_out, act, limit, M, N, K, ldh, ldy)
 #define HDS_GFM(RR, NN, GG)                                                                                    \
-  if (M <= 2) HDS_GF(2, RR, NN, GG);                                                                           \
+  if (M == 1) HDS_GF(1, RR, NN, GG); else if (M <= 2) HDS_GF(2, RR, NN, GG);                                   \
   else if (M <= 4) HDS_GF(4, RR, NN, GG); else HDS_GF(8, RR, NN, GG);
 #define HDS_GFR(NN, GG)                                                                                        \
   if (R == 4) { HDS_GFM(4, NN, GG) } else if (R == 2) { HDS_GFM(2, NN, GG) } else { HDS_GFM(1, NN, GG) }
@@ -661,7 +680,7 @@ HDS_EXPORT int hds_gemv_bf16_supported(int M, int N, int K) { return M >= 1 && M
 HDS_EXPORT int hds_gemv_bf16(const void* x, const void* w, const void* bias, void* y, int M, int N, int K, int64_t ldx,
                              int64_t ldy, hipStream_t st) {
   if (!hds_gemv_bf16_supported(M, N, K) || ldx % 8) return hipErrorInvalidValue;
-  if (M == 1)
+  if (M == 1 && !row_by_columns<false, false>(N, K))
     return launch_row<false, false, false>(OneRow{(const bf16*)x, nullptr, nullptr, 0.f, (const bf16*)w, (const bf16*)bias,
                                                   (bf16*)y, nullptr, nullptr, N, K, 0, 0.f}, Gather{}, st);
   // R = 4 rows per wave while that still leaves >= 2 waves per SIMD on 256 CUs, else 2 / 1 (parallelism)
@@ -669,7 +688,7 @@ HDS_EXPORT int hds_gemv_bf16(const void* x, const void* w, const void* bias, voi
   hipLaunchKernelGGL((gemv_bf16_kernel<MM, RR>), dim3((N + 4 * RR - 1) / (4 * RR)), dim3(256), 0, st, (const bf16*)x, \
                      (const bf16*)w, (const bf16*)bias, (bf16*)y, M, N, K, ldx, ldy)
 #define HDS_GVM(RR)                                                                                           \
-  if (M <= 2) HDS_GV(2, RR); else if (M <= 4) HDS_GV(4, RR); else HDS_GV(8, RR);
+  if (M == 1) HDS_GV(1, RR); else if (M <= 2) HDS_GV(2, RR); else if (M <= 4) HDS_GV(4, RR); else HDS_GV(8, RR);
   if (N >= 8192) {
     HDS_GVM(4)
   } else if (N >= 4096) {

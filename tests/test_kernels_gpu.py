@@ -922,6 +922,19 @@ def test_skinny_gemm_edges(act, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,N,K", [
+    (kind, N, K) for kind, sizes in (
+        ("plain", [(767, 2048), (768, 2048), (3072, 2048), (3073, 2048), (1001, 1536), (6143, 768), (6145, 768), (9, 248), (4099, 2560)]),
+        ("norm_res", [(300, 1024), (300, 1032), (12287, 2560), (12291, 2560), (12291, 8192), (12291, 8200), (12291, 6144)]),
+        ("norm_glu", [(300, 1024), (300, 1032), (6143, 768), (6145, 768), (300, 8192), (300, 6144)]),
+        ("glu", [(300, 1024), (300, 1032), (2048, 2560), (2049, 2560), (1001, 5120), (1001, 5128), (1001, 2048)]))
+    for N, K in sizes])
+def test_one_row_of_both_kernels(kind, N, K):
+    """Both sides of each size at which one row changes from a kernel of columns to one of pieces of K, or its pieces a turn."""
+    test_one_row_edges(N, K, kind)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,glu,res", [(1, 6144, 4096, False, True), (1, 14336, 4096, True, True),
                                            (3, 4100, 4096, False, False), (8, 1000, 1032, True, True),
                                            (5, 8192, 512, True, False)])
