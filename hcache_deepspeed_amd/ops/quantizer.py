@@ -170,15 +170,34 @@ def wmix_gemm(x2, q_weight, scales, out_features, in_features, group_size, fmt, 
     return y
 
 
+def _gemv_wins(M, out_features, in_features, fmt):
+    """Do the GEMVs of csrc/kernels/quant.hip and fpq.hip, which keep weights exact and sums in 32 bits too, beat the packed-weight
+    stream? us, GEMV / stream. int4, one row: up to 100M weights, 48M of long rows ([6144, 4096] 7.2 / 9.4, [8192, 8192] 14.7 / 16.8;
+    [4096, 14336] 17.3 / 15.6, [28672, 4096] 30.2 / 26.7). int8, two rows: where the last round of 256 tiles of 16 weight rows leaves
+    the chip idle ([1024, 1024] 3.3 / 3.9, [6144, 4096] 11.3 / 12.7, [4096, 4096] 8.2 / 7.9, [11264, 2048] 11.0 / 9.4). int4, two
+    rows, and fp6, one: small weights ([1024, 1024] 3.4 / 4.0 and 3.5 / 3.6, [3072, 2048] 5.3 / 4.8 and 6.4 / 4.7)."""
+    weights, tiles = out_features * in_features, (out_features + 15) // 16
+    if fmt == "fp6":
+        return M == 1 and weights < 4_000_000
+    if M > _INT_GEMV_MAX_M:
+        return False
+    if fmt == "int8":
+        return M == 1 or M == 2 and tiles / ((tiles + 255) // 256 * 256) < 0.8
+    return M == 1 and weights < (48_000_000 if in_features > 8192 else 100_000_000) or M == 2 and weights < 4_000_000
+
+
 def _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, fmt, ebits=3, bias=None, glu=0):
     """The packed-weight stream for few rows (csrc/kernels/wmix_gemm.hip ``wmix_skinny_kernel``), or None where it does not
-    apply (rows of whole groups of a multiple of 128; fp6 as e3m2 or e2m3). It wins up to 16 rows, with fp6 up to 32 ([28672, 4096], 24 rows: fp6 57 us against the tile kernel's 78, int8
-    61 against 50), with int8 from the second row on (one row: 36.5 us against the GEMV's 34.7, two 36.5 against 39)."""
+    apply (rows of whole groups of a multiple of 128; fp6 as e3m2 or e2m3). It wins up to 16 rows, with fp6 up to 32
+    ([28672, 4096], 24 rows: fp6 57 us against the tile kernel's 78, int8 61 against 50; fp6 at 32 rows 87 against 78, but the
+    tile kernel rounds the weights), with int8 from the second row on (one row: 36.5 us against the GEMV's 34.7)."""
     M = x2.shape[0]
     if (_needs_grad(x2) or not native.use_native(x2) or x2.dtype != torch.bfloat16 or in_features % 128
             or group_size % 128 or in_features % group_size or (fmt == "fp6" and ebits not in (2, 3))
             or not (fmt == "int8") < M <= (32 if fmt == "fp6" and not glu else 16)):
         return None
+    if bias is None and not glu and _gemv_wins(M, out_features, in_features, fmt):
+        return None  # (with a bias, which the GEMVs' results would get after their rounding, the stream)
     x2 = x2.contiguous()
     if x2.data_ptr() % 16:
         return None
@@ -211,7 +230,7 @@ def int_linear(x, q_weight, scales, out_features, in_features, group_size, bits=
     """y = x @ dequant(W)^T for a symmetric group-quantized int8/int4 weight [out, in] (groups along ``in``).
 
     Up to 16 rows stream the packed weight through the matrix cores (``_wmix_skinny``, groups of a multiple of 128; one row
-    of int8, other groups and a bias that is not bf16 up to 2 rows, ``HDS_INT_GEMV_MAX_M``: the HIP GEMV of
+    of int8, one and two rows where ``_gemv_wins``, other groups and a bias that is not bf16 up to 2 rows, ``HDS_INT_GEMV_MAX_M``: the HIP GEMV of
     csrc/kernels/quant.hip); batches of up to 64 rows run the tile kernel on packed weights, larger ones and groups that do
     not divide a row dequantize once to bf16."""
     lead = x.shape[:-1]
@@ -462,7 +481,7 @@ def fp6_linear(x, q_weight, scales, out_features, in_features, group_size, manti
     """y = x @ dequant(W)^T for an FP6-packed weight [out, in] (row-major, groups along ``in``).
 
     Up to 32 rows stream the packed weight through the matrix cores (``_wmix_skinny``, groups of a multiple of 128; other
-    groups: the HIP GEMV of csrc/kernels/fpq.hip up to 8 rows); batches of up to 64 rows run the tile kernel on packed
+    groups up to 8 rows and one row where ``_gemv_wins``: the HIP GEMV of csrc/kernels/fpq.hip); batches of up to 64 rows run the tile kernel on packed
     weights, larger ones dequantize once to bf16 and use hipBLASLt."""
     lead = x.shape[:-1]
     x2 = x.reshape(-1, in_features)

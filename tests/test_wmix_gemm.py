@@ -87,6 +87,31 @@ def test_few_rows_keep_the_weights_exact(fmt, M, N, K, G):
     assert ((y.double() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("fmt,M,N,K,gemv", [
+    ("int4", 1, 1024, 1024, True), ("int4", 1, 4096, 11648, True), ("int4", 1, 4096, 11776, False), ("int4", 1, 12200, 8192, True),
+    ("int4", 1, 12224, 8192, False), ("int4", 2, 3900, 1024, True), ("int4", 2, 3920, 1024, False), ("int8", 2, 1000, 640, True),
+    ("int8", 2, 6500, 640, True), ("int8", 2, 6560, 640, False), ("int8", 2, 4096, 640, False), ("fp6", 1, 3900, 1024, True),
+    ("fp6", 1, 3920, 1024, False)])
+def test_one_and_two_rows_keep_the_weights_exact_on_both_kernels(fmt, M, N, K, gemv):
+    """Both sides of the sizes at which the packed GEMVs give way to the stream, to the stream's bound: 32-bit sums of K exact
+    products and the result's rounding."""
+    assert Q._gemv_wins(M, N, K, fmt) == gemv
+    torch.manual_seed(K + M)
+    x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(N, K, device="cuda", dtype=torch.bfloat16) * 0.05
+    if fmt == "fp6":
+        q, s = Q.quantize_minifloat(w.reshape(-1), 128, 6, 2)
+        wd = Q.dequantize_minifloat(q, s, 128, 6, 2, torch.float32).view(N, K).double()
+        y = Q.fp6_linear(x, q, s, N, K, 128, 2)
+    else:
+        bits = int(fmt[3:])
+        q, s, _ = Q.quantize(w.reshape(-1), 128, bits, True)
+        wd = Q.dequantize(q, s, None, 128, bits, True, torch.float32).view(N, K).double()
+        y = Q.int_linear(x, q, s, N, K, 128, bits=bits)
+    ref = x.double() @ wd.t()
+    assert ((y.double() - ref).abs() <= 2**-8 * ref.abs() + 1e-5 * (x.double().abs() @ wd.abs().t())).all()
+
+
 @pytest.mark.parametrize("fmt", ["int8", "int4", "fp6"])
 @pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu"])
 @pytest.mark.parametrize("M,N,K,G", [(2, 7, 128, 128), (8, 1000, 640, 128), (16, 4104, 4224, 128), (9, 8200, 4096, 128),
