@@ -378,13 +378,14 @@ bool row_by_columns(int N, int K) {
   return K <= 2048 && K % 512 == 0 && N >= 768 && N <= 3072;
 }
 
-// Two pieces a wave on the way instead of one from the second turn on: plain [6144, 2560] 7.6 for 8.2 us, [28672, 4096] 39.7 / 39.5,
+// Two pieces a wave on the way instead of one from the second turn on: plain [6144, 2560] 7.6 for 8.2 us (fewer columns stay with one:
+// in a chain of launches [2048, 5632] takes 0.3 us more with two, where repeated by itself it is level), [28672, 4096] 39.7 / 39.5,
 // [12288, 14336] 60.9 / 62.6, gated [2 x 14336, 3072] 31.3 / 32.0. With a norm, whose work a piece past the end repeats, only gated and
 // where K has whole pairs: [2 x 8192, 4096] 26.8 for 27.7, [2 x 14336, 6144] 70.0 for 62.5; not gated [27648, 5120] 64.5 for 57.9.
 template <bool NORM, bool GLU, bool GATHER>
 int launch_row(const OneRow& p, const Gather& gather, hipStream_t st) {
   const dim3 grid((p.N + 1) / 2);
-  if (NORM ? GLU && p.K % 4096 == 0 : p.K > 2048)
+  if (NORM ? GLU && p.K % 4096 == 0 : p.K > 2048 && p.N >= 4096)
     hipLaunchKernelGGL((gemv_row_kernel<2, NORM, GLU, GATHER>), grid, dim3(256), 0, st, p, gather);
   else
     hipLaunchKernelGGL((gemv_row_kernel<1, NORM, GLU, GATHER>), grid, dim3(256), 0, st, p, gather);
