@@ -28,9 +28,9 @@ constexpr int kFewRows = 64;
 // ---------------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------------
-// PICK: output row i is made from rows pick[i] of x and res, of which there are n_in; negative ones count from
-// the end, and a row outside them gives NaN (a kernel of its own: asked for at run time it cost every norm 0.1 us, 3 to 5 %
-// of 256 rows of 512 to 2,048). A serving step normalises only the rows whose logits are wanted: gathering
+// PICK: with pick, output row i is made from rows pick[i] of x and res, of which there are n_in; negative ones count from
+// the end, and a row outside them gives NaN. (Without PICK nothing asks at run time, which cost norms of one wave a row 0.1 us, 3 to
+// 5 % of 256 rows of 512 to 2,048.) A serving step normalises only the rows whose logits are wanted: gathering
 // them first took four launches (two index conversions, two gathers; 18 us of a 490 us decode step of 16 sequences).
 struct PickedRow {
   int row;
@@ -38,7 +38,7 @@ struct PickedRow {
 };
 template <bool PICK>
 __device__ __forceinline__ PickedRow picked_row(const int* pick, int row, int n_in) {
-  if constexpr (!PICK) return {row, true};
+  if (!PICK || pick == nullptr) return {row, true};
   int r = pick[row];
   if (r < 0) r += n_in;
   const bool ok = r >= 0 && r < n_in;
@@ -401,7 +401,7 @@ hipError_t launch_fwd_rows(const void* x, const void* res, void* res_out, const 
   // 93): longer steps, the training ones among them, keep the sums of one wave in their order.
 #define HDS_NF(COLS, NV, WPR)                                              \
   case COLS:                                                               \
-    if (rows <= kFewRows) args(norm_fwd_kernel<T, WT, NV, LN, WPR, PICK>, WPR); \
+    if (rows <= kFewRows) args(norm_fwd_kernel<T, WT, NV, LN, WPR, true>, WPR); \
     else args(norm_fwd_kernel<T, WT, NV, LN, 1, PICK>, 1);                 \
     break
   switch (cols) {
