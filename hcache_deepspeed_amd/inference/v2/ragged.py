@@ -343,7 +343,7 @@ class RaggedBatchWrapper:
             raise RuntimeError(f"ragged metadata builder failed ({A})")
         if T:
             ids = torch.cat(self._tokens, out=host[:head].view(torch.int64)).numpy()
-            if id_limit is not None and (ids.min() < 0 or ids.max() >= id_limit):
+            if id_limit is not None and ids.view(np.uint64).max() >= id_limit:  # (negative ones are the largest)
                 raise IndexError(f"token ids from {ids.min()} to {ids.max()}: the embedding has {id_limit} rows")
         n = head + int(need.value)
         if extra:

@@ -55,6 +55,14 @@ def divide_step(seq_meta_host, heads, kv_heads):
 
     Beside row blocks single tokens join them where that takes less than a launch of their own (32 of them and 32 sequences
     of 8 tokens, up to 2,000 keys: 161 us apart, 129 together)."""
+    short = blocks = 0
+    for _, n, _ in seq_meta_host:
+        if n > DECODE_MAX:
+            blocks += -(-n // PREFILL_ROWS)
+        elif n > 1:
+            short += n
+    if kv_heads * short <= 512 and heads * blocks <= 256:  # neither case (8 us of host time a step otherwise, 4 so)
+        return (*make_portions(seq_meta_host), [])
     new = {s: (n, seen) for s, (_, n, seen) in enumerate(seq_meta_host) if n}
     ones = [s for s, (n, _) in new.items() if n == 1]
     few = [s for s, (n, _) in new.items() if 1 < n <= DECODE_MAX]
