@@ -82,7 +82,7 @@ class DSDenseBlockedAttention(DSSelfAttentionBase):
         kv_rope_scatter(qkv, cache, batch.tok_seq, batch.tok_pos, batch.block_tables, cos, sin, nq, nkv,
                         do_rope=rope, rotary_dim=c.rotary_dim)
         portions = getattr(batch, "portions", None)
-        if portions is not None and portions_ok(qkv[:, :nq], cache, nq, nkv):
+        if portions is not None and portions_ok(qkv[:, :nq], cache, nq, nkv, c.scale_factor):
             toks, blocks, rows = portions
             return paged_attention_portions(qkv[:, :nq], cache, toks, blocks, batch, nq, nkv, c.scale_factor,
                                             c.sliding_window, rows).reshape(T, nq * D)

@@ -86,9 +86,10 @@ def divide_step(seq_meta_host, heads, kv_heads):
     return toks, [], atoms
 
 
-def portions_ok(q, cache, n_q, n_kv):
-    """Does the prefill kernel take these heads and this cache?"""
-    return (native.use_native(q) and q.dtype == torch.bfloat16 and cache.dtype == q.dtype and cache.dim() == 5
+def portions_ok(q, cache, n_q, n_kv, scale=1.0):
+    """Does the prefill kernel take these heads, this cache and this scale (it keeps the maximum of the raw scores, so a positive
+    one; row blocks take any)?"""
+    return (2**-64 <= scale <= 2**64 and native.use_native(q) and q.dtype == torch.bfloat16 and cache.dtype == q.dtype and cache.dim() == 5
             and q.shape[2] == 128 and cache.is_contiguous() and cache.shape[1] % 64 == 0 and n_q % n_kv == 0
             and cache.shape[0] * cache.shape[1] < 2**31 and cache.stride(0) // cache.shape[1] <= 2**23
             and q.stride(0) % 8 == 0 and q.stride(1) == 128 and q.data_ptr() % 16 == 0)

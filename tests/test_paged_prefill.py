@@ -6,7 +6,9 @@ import types
 import pytest
 import torch
 
-from hcache_deepspeed_amd.ops.paged import DECODE_MAX
+from hcache_deepspeed_amd.inference.v2.modules.configs import DSSelfAttentionConfig
+from hcache_deepspeed_amd.inference.v2.modules.implementations import DSDenseBlockedAttention
+from hcache_deepspeed_amd.ops.paged import DECODE_MAX, build_atoms
 from hcache_deepspeed_amd.ops.paged_prefill import divide_step, make_portions, paged_attention_portions, portions_ok
 
 D = 128
@@ -139,6 +141,36 @@ def test_many_short_portions_match_float64(lens, window):
         hide = at[None] > mine
         if window:
             hide |= at[None] <= mine - window
+        want = (torch.softmax(sc.masked_fill(hide.to(dev), float("-inf")), -1) @ v).transpose(0, 1)
+        worst = (o[q0:q0 + n].double() - want).norm(dim=-1) / want.norm(dim=-1)
+        assert worst.max() < 0.03, (i, worst.max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [0.0, -0.09, 1e-30, -1e-30, 0.09, 2.0])
+def test_any_scale_in_a_portion(scale):
+    """The attention module takes any scale: zero and tiny ones give every visible key the same weight, negative ones turn the
+    order round. The prefill kernel takes positive ones, the others run in row blocks. Bounds as above."""
+    lens, seen, hq, hkv = [70, 1, 300], [100, 50, 7], 8, 2
+    g = torch.Generator().manual_seed(5)
+    dev = torch.device("cuda")
+    cache, tab, metas, T, batch = _setup(lens, seen, hkv, 64, dev, g)
+    qkv = torch.randn(T, hq + 2 * hkv, D, generator=g).bfloat16().to(dev)
+    i32 = lambda v, shape: torch.tensor(v, dtype=torch.int32, device=dev).view(shape) if v else None  # noqa: E731
+    toks, blocks, rows = divide_step(metas, hq, hkv)
+    assert blocks and portions_ok(qkv[:, :hq], cache, hq, hkv, scale) == (scale > 1e-20)
+    batch.portions = i32(toks, (-1, )), i32(blocks, (-1, 2)), i32(rows, (-1, 3))
+    atoms, batch.n_atoms = build_atoms(metas, hq, hkv)
+    batch.atoms = atoms.to(dev)
+    batch.current_sequences, batch.max_new, batch.seq_meta_host, batch.tables_host = len(lens), max(lens), metas, tab
+    o = DSDenseBlockedAttention(DSSelfAttentionConfig(hq, hkv, D, scale_factor=scale, positional_embedding_type="none"))(
+        qkv, cache, batch, None, None).view(T, hq, D)
+    for i, (q0, n, s) in enumerate(metas):
+        at = torch.arange(s + n)
+        kv = cache[tab[i, at // 64].long().to(dev), (at % 64).to(dev)].double()
+        k, v = (kv[:, j].repeat_interleave(hq // hkv, 1).transpose(0, 1) for j in (0, 1))
+        sc = qkv[q0:q0 + n, :hq].double().transpose(0, 1) @ k.transpose(1, 2) * scale
+        hide = at[None] > (s + torch.arange(n))[:, None]
         want = (torch.softmax(sc.masked_fill(hide.to(dev), float("-inf")), -1) @ v).transpose(0, 1)
         worst = (o[q0:q0 + n].double() - want).norm(dim=-1) / want.norm(dim=-1)
         assert worst.max() < 0.03, (i, worst.max())
