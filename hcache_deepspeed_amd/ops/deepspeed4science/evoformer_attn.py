@@ -65,7 +65,8 @@ def _hip_backward(ctx, do, qh, kh, vh, oh, lse, bias1, bias2, scale):
     """HIP backward (csrc/kernels/evoformer.hip)."""
     from .. import native
     B, N, H, L, D = qh.shape
-    q, k, v, o = (x.transpose(-2, -3) for x in (qh, kh, vh, oh))  # back to the contiguous [B, N, L, H, D]
+    # back to [B, N, L, H, D], contiguous already unless saved-tensor hooks (save_on_cpu with pinned memory) laid them out anew
+    q, k, v, o = (x.transpose(-2, -3).contiguous() for x in (qh, kh, vh, oh))
     do = do.contiguous()
     if do.data_ptr() % 16:
         do = do.clone()

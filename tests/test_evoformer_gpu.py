@@ -187,3 +187,16 @@ def test_evoformer_kernel_takes_a_scale_or_refuses_it(cuda, D, scale, bias_dtype
     assert (o.double() - ref).norm() <= 2 * 2**-8 * ref.norm()
     # 32-bit scores of a few hundred, in units of 1 / scale
     assert (lse.double() - torch.logsumexp(s, -1)).abs().max() <= 2e-6 * s.abs().nan_to_num(0, 0, 0).max() + 1e-4
+
+
+@pytest.mark.gpu
+def test_evoformer_saved_tensors_in_another_order(cuda):
+    """Saved tensors that come back from pinned host memory are contiguous as they were saved, [B, N, H, L, D]."""
+    g = torch.Generator(cuda).manual_seed(2)
+    q, k, v, do = (torch.randn(1, 3, 70, 4, 32, device=cuda, generator=g).bfloat16().requires_grad_(i < 3) for i in range(4))
+    want = torch.autograd.grad(DS4Sci_EvoformerAttention(q, k, v, []), (q, k, v), do)
+    with torch.autograd.graph.save_on_cpu(pin_memory=True):
+        out = DS4Sci_EvoformerAttention(q, k, v, [])
+    torch.cuda.synchronize()
+    for a, b in zip(torch.autograd.grad(out, (q, k, v), do), want):
+        assert torch.equal(a, b)
