@@ -634,8 +634,8 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(PagedDecodeParams<bf1
     for (int u = 0; u < U; ++u) r[u] = pages.slot(keys.pos(min(j + u * STEP, j1 - 1))) * kv_row;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      kn[u] = *reinterpret_cast<const bf16x8*>(kbase + r[u]);
-      vn[u] = *reinterpret_cast<const bf16x8*>(vbase + r[u]);
+      kn[u] = load_nt(reinterpret_cast<const bf16x8*>(kbase + r[u]));
+      vn[u] = load_nt(reinterpret_cast<const bf16x8*>(vbase + r[u]));
     }
   };
   int j = j0 + w * KPW + kl;
@@ -765,7 +765,8 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(PagedDecodeParams<bf1
 // Measured with the merge, the vector kernel and its merge -> this: 16 sequences of up to 4,000 keys, 32 / 8 heads, 54.0 ->
 // 47.4 us (168 MB; 4 TB/s without the merge), up to 2,000 33.5 -> 28.3; 32 of up to 500 22.6 -> 17.3; one of 1,000, 16 / 4
 // heads, 13.9 -> 8.5, and the rotation's own launch (4 us) saved. More or smaller splits are level or slower (1,024 and
-// 2,048 workgroups: 46.4 and 45.3 us there, but 8 sequences of 1,000 keys 12.3 -> 15.4 and 22.5).
+// 2,048 workgroups: 46.4 and 45.3 us there, but 8 sequences of 1,000 keys 12.3 -> 15.4 and 22.5). Keys and values, which a
+// step reads once, past the caches: 16 sequences of up to 4,000 keys 42.7 -> 40.8 us, 9 of up to 3,000 19.8 -> 18.3 (no merge).
 struct DecodeRope {
   bf16* cache;
   const float* cos;  // [pos][rot / 2], null: k is appended as it is
@@ -803,8 +804,8 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(PagedDecodePa
     const bf16* base = p.cache + ((int64_t)blk * p.block_size + pos % p.block_size) * kv_row + hk * D + 8 * hd;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      kr[i] = *reinterpret_cast<const bf16x8*>(base + (4 * i + g) * kv_row);
-      vr[i] = *reinterpret_cast<const bf16x8*>(base + (4 * i + g) * kv_row + p.hkv * D);
+      kr[i] = load_nt(reinterpret_cast<const bf16x8*>(base + (4 * i + g) * kv_row));
+      vr[i] = load_nt(reinterpret_cast<const bf16x8*>(base + (4 * i + g) * kv_row + p.hkv * D));
     }
   };
   int T = tiles.a + w;
