@@ -351,8 +351,13 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
 // ---------------------------------------------------------------------------------------------------------------
 // out[a] = act(x[a / kx] . Wg[e]^T) * (x[a / kx] . Wu[e]^T) (GLU) or x[a / kx] . W[e]^T, for every choice a of expert e;
 // W of expert e is [rows, K] with rows = 2N (GLU: gate rows, then up rows) or N. Behind the routed slots, n_sh tokens
-// through the shared expert. A workgroup: one expert and 16 output columns; its four waves split K and hold the
-// weights of one pass over up to 16 rows each (mfma_f32_16x16x32_bf16, A = weights, B = rows), as in gemv.hip.
+// through the shared expert. A workgroup: one expert and 16 of its weight rows (16 output columns, or the gate and up rows of
+// eight); its waves split K and hold the weights of one pass over up to 16 rows (mfma_f32_16x16x32_bf16, A = weights, B = rows).
+// A weight stream: loads of whole cache lines past the caches, through a wave's own LDS into the operand's layout, as
+// skinny_lines_kernel in gemv.hip. Half lines straight into the operand (and 16 gate and 16 up rows a workgroup) -> this:
+// [8, 2 x 14336, 4096] and 32 choices 336 -> 276 us (6.8 TB/s), its down product 164 -> 140; [64, 2 x 1024, 2048] with a shared expert,
+// 96 choices 93 -> 74, down 43.8 -> 39.5, 24 choices 35.3 -> 35.2, down 20.7 -> 19.4; 6 choices level. Half lines past the caches are
+// fetched twice (both products of the first 500 -> 560 us). The next piece already on its way while one is multiplied: level.
 struct SkinnyParams {
   const bf16* x;
   int64_t ldx;
@@ -380,14 +385,25 @@ __device__ __forceinline__ float gated_unit(float g, float u, int act, float lim
 
 constexpr int kSkinnyMax = 2048;  // choices
 
+// one of the 16 weight rows of tile id: with GLU eight gate rows and the up rows that belong to them (rows past the end
+// re-read the last one, not stored)
 template <bool GLU>
-__global__ __launch_bounds__(256) void experts_skinny_kernel(SkinnyParams p) {
-  constexpr int R = GLU ? 2 : 1;
-  __shared__ f32x4 red[3][R][64];
-  __shared__ int list[kSkinnyMax];
+__device__ __forceinline__ int64_t skinny_row(int id, int r, int N) {
+  if constexpr (GLU) {
+    const int n = min(id * 8 + (r & 7), N - 1);
+    return r < 8 ? n : (int64_t)N + n;
+  }
+  return min(id * 16 + r, N - 1);
+}
+
+template <bool GLU, int NW>
+__global__ __launch_bounds__(64 * NW) void experts_skinny_kernel(SkinnyParams p) {
+  __shared__ __attribute__((aligned(16))) char buf[NW][4096];
+  __shared__ uint16_t list[kSkinnyMax];
   __shared__ int s_n;
+  constexpr int PER = GLU ? 8 : 16;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int nt = (p.N + 15) / 16;
+  const int nt = (p.N + PER - 1) / PER;
   int id = blockIdx.x;
   const bf16 *x, *w;
   bf16* out;
@@ -402,82 +418,85 @@ __global__ __launch_bounds__(256) void experts_skinny_kernel(SkinnyParams p) {
     if (e < 0 || e >= p.E) return;
     if (threadIdx.x == 0) s_n = 0;
     __syncthreads();
-    for (int a0 = 0; a0 < p.n; a0 += 256) {
+    for (int a0 = 0; a0 < p.n; a0 += 64 * NW) {
       const int a = a0 + threadIdx.x;
-      if (a < p.n && p.expert[a] == e) list[atomicAdd(&s_n, 1)] = a;
+      if (a < p.n && p.expert[a] == e) list[atomicAdd(&s_n, 1)] = (uint16_t)a;
     }
     __syncthreads();
     rows = s_n;
     if (rows == 0) return;
     if (p.slots == p.n) {
       int first = list[0];
-      for (int i = 1; i < rows; ++i) first = min(first, list[i]);
+      for (int i = 1; i < rows; ++i) first = min(first, (int)list[i]);
       if (first != slot) return;
     }
     x = p.x; ldx = p.ldx; kx = p.kx; out = p.out; ldo = p.ldo; N = p.N; K = p.K;
-    w = p.w + (int64_t)e * (R * N) * K;
+    w = p.w + (int64_t)e * (GLU ? 2 * N : N) * K;
   } else {
     id -= p.slots * nt;
     rows = p.n_sh;
     x = p.xs; ldx = p.ldxs; kx = 1; out = p.outs; ldo = p.ldos; N = p.Ns; K = p.Ks;
     w = p.ws;
   }
-  const int n0 = id * 16;
-  const int kq = K >> 2, kb = wid * kq + 8 * (lane >> 4);
-  const bf16* wp[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) wp[r] = w + ((int64_t)r * N + min(n0 + (lane & 15), N - 1)) * K + kb;
+  const int wr = lane >> 3, wz = lane & 7, rr = lane & 15, rp = lane >> 4;
+  const bf16* w0 = w + skinny_row<GLU>(id, wr, N) * K + 8 * wz;
+  const bf16* w1 = w + skinny_row<GLU>(id, 8 + wr, N) * K + 8 * wz;
+  char* mine = buf[wid];
+  char* put = mine + wr * 128 + (wz ^ wr) * 16;
+  const char* get0 = mine + rr * 128 + (rp ^ (rr & 7)) * 16;
+  const char* get1 = mine + rr * 128 + ((rp + 4) ^ (rr & 7)) * 16;
+  const int parts = K >> 7, turn = GLU || K % 2048 ? 0 : (int)__umulhi(blockIdx.x * 2654435769u, (unsigned)parts);
   for (int g = 0; g < rows; g += 16) {
-    const int i = g + (lane & 15);
+    const int i = g + rr;
     const bool ok = i < rows;
     const int a = routed ? list[ok ? i : rows - 1] : (ok ? i : rows - 1);
-    const bf16* xp = x + (int64_t)(a / kx) * ldx + kb;
-    f32x4 acc[R];
+    const bf16* xp = x + (int64_t)(a / kx) * ldx + 8 * rp;
+    f32x4 acc{};
+    for (int c = wid; c < parts; c += NW) {
+      int k = c + turn;
+      k = (k < parts ? k : k - parts) << 7;
+      bf16x8 wv[2][2], xv[4];
 #pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] = f32x4{};
-    constexpr int U = GLU ? 8 : 8;
-    int k = 0;
-    for (; k + 32 * U <= kq; k += 32 * U) {
-      bf16x8 wv[U][R], xv[U];
+      for (int u = 0; u < 2; ++u) {
+        wv[u][0] = load_nt(reinterpret_cast<const bf16x8*>(w0 + k + 64 * u));
+        wv[u][1] = load_nt(reinterpret_cast<const bf16x8*>(w1 + k + 64 * u));
+      }
 #pragma unroll
-      for (int u = 0; u < U; ++u)
+      for (int u = 0; u < 4; ++u) xv[u] = *reinterpret_cast<const bf16x8*>(xp + k + 32 * u);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < R; ++r) wv[u][r] = *reinterpret_cast<const bf16x8*>(wp[r] + k + 32 * u);
+      for (int u = 0; u < 2; ++u) {
+        *reinterpret_cast<bf16x8*>(put + u * 2048) = wv[u][0];
+        *reinterpret_cast<bf16x8*>(put + u * 2048 + 1024) = wv[u][1];
+      }
 #pragma unroll
-      for (int u = 0; u < U; ++u) xv[u] = *reinterpret_cast<const bf16x8*>(xp + k + 32 * u);
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-          acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u][r], xv[u], acc[r], 0, 0, 0);
+      for (int u = 0; u < 2; ++u) {
+        const bf16x8 p0 = *reinterpret_cast<const bf16x8*>(get0 + u * 2048);
+        const bf16x8 p1 = *reinterpret_cast<const bf16x8*>(get1 + u * 2048);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p0, xv[2 * u], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(p1, xv[2 * u + 1], acc, 0, 0, 0);
+      }
     }
-    for (; k < kq; k += 32) {
-      const bf16x8 xv = *reinterpret_cast<const bf16x8*>(xp + k);
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(wp[r] + k), xv, acc[r], 0, 0,
-                                                         0);
-    }
-    if (g > 0) __syncthreads();  // the previous rows' partial sums have been read
-    if (wid > 0) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) red[wid - 1][r][lane] = acc[r];
-    }
+    reinterpret_cast<f32x4*>(mine)[lane] = acc;
     __syncthreads();
-    if (wid == 0 && ok) {
+    if (wid == 0) {
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int v = 0; v < 3; ++v) acc[r] += red[v][r][lane];
+      for (int v = 1; v < NW; ++v) acc += reinterpret_cast<const f32x4*>(buf[v])[lane];
       const float rw = GLU && routed && p.weight != nullptr ? p.weight[a] : 1.f;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int n = n0 + 4 * (lane >> 4) + q;
-        float v = acc[0][q];
-        if constexpr (GLU) v = gated_unit(v * rw, acc[R - 1][q] * rw, p.act, p.limit);
-        if (n < N) out[(int64_t)a * ldo + n] = (bf16)v;
+        const int n = GLU ? id * 8 + 4 * (rp & 1) + q : id * 16 + 4 * rp + q;
+        float v = acc[q];
+        bool mine_to_store = ok && n < N;
+        if constexpr (GLU) {  // lanes of the upper half hold the up rows of those 32 below
+          const float up = __shfl_down(v, 32, 64);
+          v = gated_unit(v * rw, up * rw, p.act, p.limit);
+          mine_to_store = mine_to_store && lane < 32;
+        }
+        if (mine_to_store) out[(int64_t)a * ldo + n] = (bf16)v;
       }
     }
+    if (g + 16 < rows) __syncthreads();  // the partial sums have been read
   }
 }
 
@@ -601,11 +620,16 @@ HDS_EXPORT int hds_experts_skinny(int glu, const void* x, int64_t ldx, const voi
   // n == E: a slot may be read as a choice or as an expert; both cover everything once
   SkinnyParams p{(const bf16*)x, ldx, (const bf16*)w, (bf16*)out, ldo, expert, n, kx, E, N, K, slots, (const bf16*)xs,
                  ldxs, (const bf16*)ws, (bf16*)outs, ldos, sh ? n_sh : 0, Ns, Ks, act, limit, weight};
-  const int64_t blocks = (int64_t)slots * ((N + 15) / 16) + (sh ? (Ns + 15) / 16 : 0);
+  const int per = glu ? 8 : 16;
+  const int64_t blocks = (int64_t)slots * ((N + per - 1) / per) + (sh ? (Ns + per - 1) / per : 0);
+  // Eight waves share a long sum (N = 4096, 32 choices: K = 14336 140 us against 150 with four, 5632 29 / 30), four a short one (K
+  // = 1024 39.5 / 46.7: a wave of eight has one turn) and the gated products (level)
   if (glu)
-    hipLaunchKernelGGL(experts_skinny_kernel<true>, dim3(blocks), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((experts_skinny_kernel<true, 4>), dim3(blocks), dim3(256), 0, st, p);
+  else if (K >= 2048)
+    hipLaunchKernelGGL((experts_skinny_kernel<false, 8>), dim3(blocks), dim3(512), 0, st, p);
   else
-    hipLaunchKernelGGL(experts_skinny_kernel<false>, dim3(blocks), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((experts_skinny_kernel<false, 4>), dim3(blocks), dim3(256), 0, st, p);
   return hipGetLastError();
 }
 

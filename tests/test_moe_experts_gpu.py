@@ -74,3 +74,39 @@ def test_mixtral_engine_direct_expert_wgrad_matches():
             losses.append(float(loss))
         res[direct] = losses
     assert res[True] == pytest.approx(res[False], rel=2e-2, abs=2e-2), res
+
+
+# tiles of 16 weight rows (8 + 8 with the gate) and of 128 columns; more waves from K = 2048 on; rotated walks at multiples of 2048
+@pytest.mark.parametrize("N,K", [(8, 128), (24, 384), (17, 1920), (40, 2048), (33, 2176), (16, 4096)])
+@pytest.mark.parametrize("T,E,k", [(1, 8, 2), (5, 3, 2), (40, 4, 2)])  # fewer choices than experts; more; over 16 rows an expert
+@pytest.mark.parametrize("glu", [0, 1])
+def test_experts_of_few_rows(N, K, T, E, k, glu):
+    from hcache_deepspeed_amd.ops import native
+    gen = torch.Generator(device="cuda").manual_seed(N * K + T)
+
+    def rand(*shape):
+        return torch.randn(*shape, device="cuda", generator=gen).mul_(K**-0.25).to(torch.bfloat16)
+
+    expert = torch.stack([torch.randperm(E, device="cuda", generator=gen)[:k] for _ in range(T)]).int()
+    n, Ns, Ks = T * k, N + 8, 256
+    x, w, xs, ws = rand(T, K), rand(E, (1 + glu) * N, K), rand(T, Ks), rand((1 + glu) * Ns, Ks)
+    out, outs = torch.full((n + 1, N), 7.0, device="cuda", dtype=torch.bfloat16), rand(T, Ns)
+    weight = torch.rand(n, device="cuda", generator=gen)
+    native.check(
+        native.kernels().hds_experts_skinny(glu, x.data_ptr(), K, w.data_ptr(), out.data_ptr(), N, expert.data_ptr(), n, k, E, N, K,
+                                            xs.data_ptr(), Ks, ws.data_ptr(), outs.data_ptr(), Ns, T, Ns, Ks, 0, 0.0,
+                                            weight.data_ptr(), native.stream()), "experts_skinny")
+
+    def product(rows, m, scale):
+        z = rows.double() @ m.double().T
+        if not glu:
+            return z
+        g, u = (z * scale).chunk(2, -1)
+        return torch.nn.functional.silu(g) * u
+
+    for a in range(n):
+        want = product(x[a // k], w[int(expert[a // k, a % k])], weight[a].double())
+        # a result of bf16, and sums of K products in 32 bits
+        torch.testing.assert_close(out[a].double(), want, rtol=2**-7, atol=1e-3)
+    torch.testing.assert_close(outs.double(), product(xs, ws, 1.0), rtol=2**-7, atol=1e-3)
+    assert (out[n:] == 7.0).all()
