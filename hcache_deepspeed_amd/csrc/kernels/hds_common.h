@@ -51,6 +51,32 @@ __device__ __forceinline__ void store_nt(V* p, const V& v) {
   __builtin_nontemporal_store(__builtin_bit_cast(u32x4, v), reinterpret_cast<u32x4*>(p));
 }
 
+// Four elements as one non-temporal access
+template <typename T>
+__device__ __forceinline__ void load4_nt(const T* p, float (&v)[4]) {
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  if constexpr (sizeof(T) == 4) {
+    const f32x4 r = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = r[i];
+  } else {
+    const t4 r = __builtin_bit_cast(t4, __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p)));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = to_f(r[i]);
+  }
+}
+template <typename T>
+__device__ __forceinline__ void store4_nt(T* p, const float (&v)[4]) {
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  t4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = from_f<T>(v[i]);
+  if constexpr (sizeof(T) == 4)
+    __builtin_nontemporal_store(__builtin_bit_cast(u32x4, r), reinterpret_cast<u32x4*>(p));
+  else
+    __builtin_nontemporal_store(__builtin_bit_cast(u32x2, r), reinterpret_cast<u32x2*>(p));
+}
+
 // 8-element vector load/store in f32 registers. For bf16/f16 this is ONE
 // 16-byte global access per lane; for f32 two 16-byte accesses.
 template <typename T> struct Vec8;

@@ -6,7 +6,7 @@
 //
 // MI355X-first design:
 //   * ZeRO keeps every optimizer partition as ONE flat fp32 buffer, so the hot path is the flat
-//     kernel: a grid-stride stream over [p32, m, v] (fp32) + g (bf16 or fp32), 16-byte accesses,
+//     kernel: one pass over [p32, m, v] (fp32) + g (bf16 or fp32), 16-byte accesses,
 //     that also writes the bf16 working copy of the parameter in the same pass (no separate
 //     fp32->bf16 cast kernel, no separate unscale/clip kernel: `gscale` and the optional
 //     device-side `dev_scale` are folded into the gradient read).
@@ -44,50 +44,44 @@ __device__ __forceinline__ void adam_elem(float& p, float g, float& m, float& v,
   p -= h.lr * upd;
 }
 
-// NT (variant 1): the fp32 state and the bf16 copy are written with non-temporal (streaming) stores -- every byte the
-// step writes is read again only in the next step, so allocating it in L2 only evicts the stream's read lines
-__device__ __forceinline__ void st8_nt(float* p, const float (&v)[8]) {
-  __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, reinterpret_cast<f32x4*>(p));
-  __builtin_nontemporal_store(f32x4{v[4], v[5], v[6], v[7]}, reinterpret_cast<f32x4*>(p + 4));
-}
-__device__ __forceinline__ void st8_nt(bf16* p, const float (&v)[8]) {
-  bf16x8 r;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = (bf16)v[i];
-  __builtin_nontemporal_store(*reinterpret_cast<u32x4*>(&r), reinterpret_cast<u32x4*>(p));
-}
+// p: master (PT = float or bf16), g: grad, m/v: fp32 state, lp: optional low-precision copy of p.
+// Bound by memory, 28 bytes an element with a 16-bit gradient and copy. A workgroup takes 2048 elements once, and a wave's
+// accesses are whole runs of 1 KB (32-bit) and 512 bytes: 213M elements 1,223 -> 1,040 us (5.7 TB/s), 37M 218 -> 176. By their
+// accesses alone: these 1,087, from 4,096 workgroups that walk through the buffers 1,160, eight neighbouring elements a
+// lane 1,169, both of these with temporal accesses 1,290.
+constexpr int kAdamPer = 2048;
 
-// p: master (PT = float or bf16), g: grad, m/v: fp32 state, lp: optional low-precision copy of p
-template <typename PT, typename GT, bool NT = false>
+template <typename PT, typename GT>
 __global__ __launch_bounds__(256) void adam_flat(PT* __restrict__ p, const GT* __restrict__ g, float* __restrict__ m,
                                                  float* __restrict__ v, bf16* __restrict__ lp, int64_t n, AdamHP h,
                                                  float gscale, const float* __restrict__ dev_scale,
                                                  const int* __restrict__ found_inf) {
   if (found_inf && *found_inf) return;
   const float sc = load_scale(gscale, dev_scale);
-  const int64_t nvec = n / 8;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nvec; i += (int64_t)gridDim.x * 256) {
-    float pv[8], gv[8], mv[8], vv[8];
-    Vec8<PT>::load(p + i * 8, pv);
-    Vec8<GT>::load(g + i * 8, gv);
-    Vec8<float>::load(m + i * 8, mv);
-    Vec8<float>::load(v + i * 8, vv);
+  const int64_t i0 = (int64_t)blockIdx.x * kAdamPer + 4 * threadIdx.x, i1 = i0 + kAdamPer / 2;
+  if ((int64_t)(blockIdx.x + 1) * kAdamPer <= n) {
+    float pv[2][4], gv[2][4], mv[2][4], vv[2][4];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) adam_elem<PT, GT>(pv[j], gv[j] * sc, mv[j], vv[j], h);
-    if constexpr (NT) {
-      st8_nt(p + i * 8, pv);
-      st8_nt(m + i * 8, mv);
-      st8_nt(v + i * 8, vv);
-      if (lp) st8_nt(lp + i * 8, pv);
-    } else {
-      Vec8<PT>::store(p + i * 8, pv);
-      Vec8<float>::store(m + i * 8, mv);
-      Vec8<float>::store(v + i * 8, vv);
-      if (lp) Vec8<bf16>::store(lp + i * 8, pv);
+    for (int u = 0; u < 2; ++u) {
+      const int64_t i = u ? i1 : i0;
+      load4_nt(p + i, pv[u]);
+      load4_nt(m + i, mv[u]);
+      load4_nt(v + i, vv[u]);
+      load4_nt(g + i, gv[u]);
     }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int64_t i = u ? i1 : i0;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) adam_elem<PT, GT>(pv[u][j], gv[u][j] * sc, mv[u][j], vv[u][j], h);
+      store4_nt(p + i, pv[u]);
+      store4_nt(m + i, mv[u]);
+      store4_nt(v + i, vv[u]);
+      if (lp) store4_nt(lp + i, pv[u]);
+    }
+    return;
   }
-  // tail
-  for (int64_t i = nvec * 8 + (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+  for (int64_t i = (int64_t)blockIdx.x * kAdamPer + threadIdx.x; i < n; i += 256) {  // the last workgroup
     float pv = to_f(p[i]), mv = m[i], vv = v[i];
     adam_elem<PT, GT>(pv, to_f(g[i]) * sc, mv, vv, h);
     p[i] = from_f<PT>(pv);
@@ -255,28 +249,76 @@ __global__ __launch_bounds__(256) void lamb_phase2(const int64_t* __restrict__ t
 
 // ---- grad norm / overflow ------------------------------------------------------------------
 // out[0] += sum(x^2) (fp32 atomics, one per block);  found_inf[0] |= any non-finite
+// Bound by memory, and by the workgroups' sums: the atomics meet at one address, about 15 ns each, so there are few
+// workgroups of 16 waves, with four 16-byte loads of a lane on the way: 213M elements of bf16 84 -> 69 us (6.2 TB/s; before:
+// 1,024 workgroups of four waves, one load each on the way), 37M 28 -> 19.
+constexpr int kSumsqBlocks = 256;
+
+// eight elements as floats, and the largest bit pattern of their magnitudes: not finite from the exponent's last value on
 template <typename T>
-__global__ __launch_bounds__(256) void sumsq_kernel(const T* __restrict__ x, int64_t n, float* __restrict__ out,
-                                                    int* __restrict__ found_inf) {
-  __shared__ float red[4];
-  float s = 0.f;
-  int bad = 0;
-  const int64_t nvec = n / 8;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nvec; i += (int64_t)gridDim.x * 256) {
-    float v[8];
-    Vec8<T>::load(x + i * 8, v);
+__device__ __forceinline__ void squares8(const u32x4 (&r)[sizeof(T) / 2], float& s, uint32_t& top) {
+  typedef T vec8 __attribute__((ext_vector_type(8)));
+  const vec8 v = __builtin_bit_cast(vec8, r);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      s += v[j] * v[j];
-      bad |= !isfinite(v[j]);
+  for (int j = 0; j < 8; ++j) {
+    const float f = to_f(v[j]);
+    s += f * f;
+  }
+  if constexpr (sizeof(T) == 2) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      top = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, top),
+                                                                   __builtin_bit_cast(u16x2, r[0][j] & 0x7fff7fffu)));
+  } else {
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) top = max(top, r[k][j] & 0x7fffffffu);
+  }
+}
+template <typename T>
+__device__ __forceinline__ bool not_finite(uint32_t top) {
+  if constexpr (sizeof(T) == 4) {
+    return top >= 0x7f800000u;
+  } else {
+    const uint32_t inf = __builtin_bit_cast(uint16_t, from_f<T>(INFINITY));
+    return (top & 0xffffu) >= inf || (top >> 16) >= inf;
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(1024) void sumsq_kernel(const T* __restrict__ x, int64_t n, float* __restrict__ out,
+                                                     int* __restrict__ found_inf) {
+  __shared__ float red[16];
+  constexpr int U = 4, P = sizeof(T) / 2;  // vectors of eight on the way, 16-byte pieces of one
+  float s = 0.f;
+  uint32_t top = 0;
+  const int64_t nvec = n / 8, step = (int64_t)gridDim.x * 1024 * U;
+  int64_t i = (int64_t)blockIdx.x * 1024 * U + threadIdx.x;
+  for (; i + (U - 1) * 1024 < nvec; i += step) {
+    u32x4 r[U][P];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int k = 0; k < P; ++k) r[u][k] = load_nt(reinterpret_cast<const u32x4*>(x + (i + u * 1024) * 8) + k);
+#pragma unroll
+    for (int u = 0; u < U; ++u) squares8<T>(r[u], s, top);
+  }
+  for (int u = 0; u < U && i < nvec; ++u, i += 1024) {  // the last, partial round
+    u32x4 r[P];
+#pragma unroll
+    for (int k = 0; k < P; ++k) r[k] = load_nt(reinterpret_cast<const u32x4*>(x + i * 8) + k);
+    squares8<T>(r, s, top);
+  }
+  bool bad = not_finite<T>(top);
+  if (blockIdx.x == 0)
+    for (int64_t k = nvec * 8 + threadIdx.x; k < n; k += 1024) {
+      const float v = to_f(x[k]);
+      s += v * v;
+      bad |= !isfinite(v);
     }
-  }
-  for (int64_t i = nvec * 8 + (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    const float v = to_f(x[i]);
-    s += v * v;
-    bad |= !isfinite(v);
-  }
-  s = block_sum<256>(s, red);
+  s = block_sum<1024>(s, red);
   const int anybad = __syncthreads_or(bad);
   if (threadIdx.x == 0) {
     atomicAdd(out, s);
@@ -328,20 +370,12 @@ HDS_EXPORT int hds_adam_flat(int pdtype, int gdtype, void* p, const void* g, flo
                              float lr, float b1, float b2, float eps, float wd, float bc1, float bc2, int adamw,
                              float gscale, const float* dev_scale, const int* found_inf, hipStream_t st) {
   AdamHP h{lr, b1, b2, eps, wd, bc1, bc2, adamw};
-  dim3 grid(stream_grid(n / 8 + 1, 256, 4096)), block(256);
-  static const int nt = [] {
-    const char* e = getenv("HDS_ADAM_NT");
-    return e ? atoi(e) : 0;
-  }();
-  if (nt && pdtype == kF32) {  // fp32 master: the training configuration
-    PG_SWITCH(pdtype, gdtype,
-              hipLaunchKernelGGL((adam_flat<PT, GT, true>), grid, block, 0, st, (PT*)p, (const GT*)g, m, v,
-                                 (bf16*)lp, n, h, gscale, dev_scale, found_inf));
-  } else {
-    PG_SWITCH(pdtype, gdtype,
-              hipLaunchKernelGGL((adam_flat<PT, GT>), grid, block, 0, st, (PT*)p, (const GT*)g, m, v, (bf16*)lp, n,
-                                 h, gscale, dev_scale, found_inf));
-  }
+  if (n <= 0) return 0;
+  if (n > (int64_t)kAdamPer * 0x7fffffff) return hipErrorInvalidValue;
+  dim3 grid((n + kAdamPer - 1) / kAdamPer), block(256);
+  PG_SWITCH(pdtype, gdtype,
+            hipLaunchKernelGGL((adam_flat<PT, GT>), grid, block, 0, st, (PT*)p, (const GT*)g, m, v, (bf16*)lp, n, h,
+                               gscale, dev_scale, found_inf));
   return hipGetLastError();
 }
 
@@ -394,7 +428,7 @@ HDS_EXPORT int hds_lamb_multi(int pdtype, int gdtype, const int64_t* tensors, co
 }
 
 HDS_EXPORT int hds_sumsq(int dtype, const void* x, int64_t n, float* out, int* found_inf, hipStream_t st) {
-  dim3 grid(stream_grid(n / 8 + 1, 256, 1024)), block(256);
+  dim3 grid(stream_grid(n / 8 + 1, 4096, kSumsqBlocks)), block(1024);
   if (dtype == kF32)
     hipLaunchKernelGGL(sumsq_kernel<float>, grid, block, 0, st, (const float*)x, n, out, found_inf);
   else if (dtype == kBF16)

@@ -1,5 +1,5 @@
 """Fused Adam (hds_adam_flat) at ZeRO-3 dp1 Llama-3-8B-like size: fp32 master/m/v, bf16 grad, bf16 copy.
-Prints ms and effective TB/s (28 B moved per element). Run once per HDS_ADAM_NT setting (read once per process)."""
+Prints ms and effective TB/s (28 B moved per element)."""
 import json
 import os
 import sys
@@ -33,7 +33,7 @@ def main():
     e1.record()
     e1.synchronize()
     ms = e0.elapsed_time(e1) / it
-    print(json.dumps({"n": n, "nt": os.environ.get("HDS_ADAM_NT", "0"), "ms": round(ms, 3),
+    print(json.dumps({"n": n, "ms": round(ms, 3),
                       "TBps": round(28 * n / ms / 1e9, 2), "ms_at_8.03B": round(ms * 8.03e9 / n, 2)}), flush=True)
 
 
