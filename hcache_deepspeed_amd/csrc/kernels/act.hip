@@ -13,7 +13,7 @@
 // backward consumes, so no cat/split copies exist anywhere in the MLP.
 #include <cstdlib>
 
-#include "hds_common.h"
+#include "transpose_tile.h"
 
 using namespace hds;
 
@@ -162,6 +162,8 @@ __global__ __launch_bounds__(256) void glu_bwd(const T* __restrict__ dy, const T
 // v2 of the gated kernels: two independent 16-B vectors per thread per grid-stride iteration, every load of both
 // issued before any math (twice the bytes in flight per wave: the v1 loop is one dependent load -> math -> store
 // chain per iteration and sat at ~5.1-5.4 TB/s). `total` vectors of 8; the tail iteration guards the second vector.
+// Every workgroup has one iteration, and the inputs, met once, are not kept in the caches: forward [2048, 14336] 36.1 -> 30.9
+// us (5.7 TB/s), [521, 14336] 11.1 -> 9.6, [16000, 5632] 105 -> 96, backward [8192, 14336] 226 -> 214 (2,048 workgroups before).
 template <typename T, int A>
 __global__ __launch_bounds__(256) void glu_fwd2(const T* __restrict__ gu, T* __restrict__ y, int64_t rows, int I) {
   const int vpr = I / 8;
@@ -176,10 +178,10 @@ __global__ __launch_bounds__(256) void glu_fwd2(const T* __restrict__ gu, T* __r
     split_idx(i0, vpr, small, r0, c0);
     split_idx(has1 ? i1 : i0, vpr, small, r1, c1);
     float g0[8], u0[8], g1[8], u1[8], o[8];
-    Vec8<T>::load(gu + r0 * 2 * I + c0, g0);
-    Vec8<T>::load(gu + r0 * 2 * I + I + c0, u0);
-    Vec8<T>::load(gu + r1 * 2 * I + c1, g1);
-    Vec8<T>::load(gu + r1 * 2 * I + I + c1, u1);
+    Vec8<T>::load_nt(gu + r0 * 2 * I + c0, g0);
+    Vec8<T>::load_nt(gu + r0 * 2 * I + I + c0, u0);
+    Vec8<T>::load_nt(gu + r1 * 2 * I + c1, g1);
+    Vec8<T>::load_nt(gu + r1 * 2 * I + I + c1, u1);
 #pragma unroll
     for (int j = 0; j < 8; ++j) o[j] = act_f<A>(g0[j]) * u0[j];
     Vec8<T>::store(y + r0 * I + c0, o);
@@ -208,9 +210,9 @@ __global__ __launch_bounds__(256) void glu_bwd2(const T* __restrict__ dy, const 
     float g[2][8], u[2][8], d[2][8];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-      Vec8<T>::load(gu + r[k] * 2 * I + c[k], g[k]);
-      Vec8<T>::load(gu + r[k] * 2 * I + I + c[k], u[k]);
-      Vec8<T>::load(dy + r[k] * I + c[k], d[k]);
+      Vec8<T>::load_nt(gu + r[k] * 2 * I + c[k], g[k]);
+      Vec8<T>::load_nt(gu + r[k] * 2 * I + I + c[k], u[k]);
+      Vec8<T>::load_nt(dy + r[k] * I + c[k], d[k]);
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -232,20 +234,19 @@ __global__ __launch_bounds__(256) void glu_bwd2(const T* __restrict__ dy, const 
 // SwiGLU-family backward that ALSO writes the transposed gradient dguT [2I, rows] (bf16): the gate|up weight
 // gradient runs hipBLASLt's NT form on dguT (ops/gemm.wgrad "nt"), which otherwise needs a separate HBM transpose of
 // the [rows, 2I] gradient (read + write of 2 x rows x I x 2 B). Block = 64 rows x 128 columns of I: the dg / du tiles
-// go to HBM row-major as in glu_bwd and through LDS (16-B writes, 8-B reads + v_perm, as transpose.hip v2) to their
-// transposed rows i and I + i. rows % 8 == 0, I % 8 == 0.
-constexpr int GT_R = 64, GT_C = 128;
-
-template <int A>
+// go to HBM row-major as in glu_bwd and through LDS (16-B writes, 8-B reads + v_perm, transpose_tile.h) to their
+// transposed rows i and I + i. rows % 8 == 0, I % 8 == 0. [8192, 14336] 370 -> 346 us with transpose_tile.h's order and stores
+// (the forward below 210 -> 188); inputs past the caches are slower (384, 213).
+template <int A, bool LINES>
 __global__ __launch_bounds__(256) void glu_bwd_t(const bf16* __restrict__ dy, const bf16* __restrict__ gu,
                                                  bf16* __restrict__ dgu, bf16* __restrict__ dgut, int rows, int I) {
-  __shared__ __attribute__((aligned(16))) bf16 tile[2][GT_R * GT_C];
-  const int r0 = blockIdx.y * GT_R, c0 = blockIdx.x * GT_C;
+  __shared__ __attribute__((aligned(16))) bf16 tile[2][kTrRows * kTrCols];
+  const TileAt at = tile_at<LINES>(rows, I);
   const int tid = threadIdx.x;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const int v = tid + 256 * k, rr = v >> 4, cc = (v & 15) * 8;
-    const int r = r0 + rr, c = c0 + cc;
+    const int v = tid + 256 * k, rr = v >> 4, ch = v & 15;
+    const int r = at.r0 + rr, c = at.c0 + 8 * ch;
     float dg[8], du[8];
     if (r < rows && c < I) {  // I % 8 == 0: a vector is all in or all out
       float g[8], u[8], d[8];
@@ -265,44 +266,27 @@ __global__ __launch_bounds__(256) void glu_bwd_t(const bf16* __restrict__ dy, co
 #pragma unroll
       for (int j = 0; j < 8; ++j) dg[j] = du[j] = 0.f;
     }
-    Vec8<bf16>::store(&tile[0][rr * GT_C + cc], dg);
-    Vec8<bf16>::store(&tile[1][rr * GT_C + cc], du);
+    Vec8<bf16>::store(&tile[0][tile_chunk(rr, ch)], dg);
+    Vec8<bf16>::store(&tile[1][tile_chunk(rr, ch)], du);
   }
   __syncthreads();
-  const int lr = tid >> 5, lc = tid & 31;
-  const int r = r0 + 8 * lr;
-  if (r >= rows) return;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    u32x2 v[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const u32x2*>(&tile[h][(8 * lr + j) * GT_C + 4 * lc]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = c0 + 4 * lc + i;
-      if (c >= I) break;
-      const uint32_t sel = (i & 1) ? 0x07060302u : 0x05040100u;
-      u32x4 y;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) y[k] = __builtin_amdgcn_perm(v[2 * k + 1][i >> 1], v[2 * k][i >> 1], sel);
-      *reinterpret_cast<u32x4*>(dgut + (int64_t)(h * I + c) * rows + r) = y;
-    }
-  }
+  store_transposed<LINES>(tile[0], dgut, at, rows, I);
+  store_transposed<LINES>(tile[1], dgut + (int64_t)I * rows, at, rows, I);
 }
 
 // Gated forward that ALSO writes the transposed output yT [I, rows] (bf16): the down projection saves yT instead of
 // y for its weight gradient (hipBLASLt NT form), so the backward's [rows, I] transpose disappears. Same tiling as
 // glu_bwd_t.
-template <int A>
+template <int A, bool LINES>
 __global__ __launch_bounds__(256) void glu_fwd_t(const bf16* __restrict__ gu, bf16* __restrict__ y,
                                                  bf16* __restrict__ yt, int rows, int I) {
-  __shared__ __attribute__((aligned(16))) bf16 tile[GT_R * GT_C];
-  const int r0 = blockIdx.y * GT_R, c0 = blockIdx.x * GT_C;
+  __shared__ __attribute__((aligned(16))) bf16 tile[kTrRows * kTrCols];
+  const TileAt at = tile_at<LINES>(rows, I);
   const int tid = threadIdx.x;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const int v = tid + 256 * k, rr = v >> 4, cc = (v & 15) * 8;
-    const int r = r0 + rr, c = c0 + cc;
+    const int v = tid + 256 * k, rr = v >> 4, ch = v & 15;
+    const int r = at.r0 + rr, c = at.c0 + 8 * ch;
     float o[8];
     if (r < rows && c < I) {
       float g[8], u[8];
@@ -315,25 +299,10 @@ __global__ __launch_bounds__(256) void glu_fwd_t(const bf16* __restrict__ gu, bf
 #pragma unroll
       for (int j = 0; j < 8; ++j) o[j] = 0.f;
     }
-    Vec8<bf16>::store(&tile[rr * GT_C + cc], o);
+    Vec8<bf16>::store(&tile[tile_chunk(rr, ch)], o);
   }
   __syncthreads();
-  const int lr = tid >> 5, lc = tid & 31;
-  const int r = r0 + 8 * lr;
-  if (r >= rows) return;
-  u32x2 v[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const u32x2*>(&tile[(8 * lr + j) * GT_C + 4 * lc]);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int c = c0 + 4 * lc + i;
-    if (c >= I) break;
-    const uint32_t sel = (i & 1) ? 0x07060302u : 0x05040100u;
-    u32x4 w;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) w[k] = __builtin_amdgcn_perm(v[2 * k + 1][i >> 1], v[2 * k][i >> 1], sel);
-    *reinterpret_cast<u32x4*>(yt + (int64_t)c * rows + r) = w;
-  }
+  store_transposed<LINES>(tile, yt, at, rows, I);
 }
 
 // y = act(x + bias)   (bias optional, [C])
@@ -434,7 +403,7 @@ static int glu_variant() {
 HDS_EXPORT int hds_glu_fwd(int dtype, int act, const void* gu, void* y, int64_t rows, int I, hipStream_t st) {
   if (I % 8) return hipErrorInvalidValue;
   if (glu_variant() == 2) {
-    dim3 grid(stream_grid(rows * (I / 8), 512)), block(256);
+    dim3 grid(stream_grid(rows * (I / 8), 512, 1 << 30)), block(256);
     DT_SWITCH(dtype, ACT_SWITCH(act, glu_fwd2, T, grid, block, 0, st, (const T*)gu, (T*)y, rows, I));
   } else {
     dim3 grid(stream_grid(rows * (I / 8), 256)), block(256);
@@ -510,7 +479,7 @@ HDS_EXPORT int hds_glu_bwd(int dtype, int act, const void* dy, const void* gu, v
                            hipStream_t st) {
   if (I % 8) return hipErrorInvalidValue;
   if (glu_variant() == 2) {
-    dim3 grid(stream_grid(rows * (I / 8), 512)), block(256);
+    dim3 grid(stream_grid(rows * (I / 8), 512, 1 << 30)), block(256);
     DT_SWITCH(dtype, ACT_SWITCH(act, glu_bwd2, T, grid, block, 0, st, (const T*)dy, (const T*)gu, (T*)dgu, rows, I));
   } else {
     dim3 grid(stream_grid(rows * (I / 8), 256)), block(256);
@@ -519,21 +488,25 @@ HDS_EXPORT int hds_glu_bwd(int dtype, int act, const void* dy, const void* gu, v
   return hipGetLastError();
 }
 
-#define GLU_T_SWITCH(act, KERN, ...)                                                 \
-  switch (act) {                                                                     \
-    case kSilu: hipLaunchKernelGGL((KERN<kSilu>), __VA_ARGS__); break;               \
-    case kGeluTanh: hipLaunchKernelGGL((KERN<kGeluTanh>), __VA_ARGS__); break;       \
-    case kRelu: hipLaunchKernelGGL((KERN<kRelu>), __VA_ARGS__); break;               \
-    case kGeluErf: hipLaunchKernelGGL((KERN<kGeluErf>), __VA_ARGS__); break;         \
-    default: hipLaunchKernelGGL((KERN<kIdentity>), __VA_ARGS__); break;              \
+#define GLU_T_CASE(AA, KERN, lines, ...)                            \
+  if (lines) hipLaunchKernelGGL((KERN<AA, true>), __VA_ARGS__);     \
+  else hipLaunchKernelGGL((KERN<AA, false>), __VA_ARGS__);          \
+  break;
+#define GLU_T_SWITCH(act, KERN, lines, ...)                         \
+  switch (act) {                                                    \
+    case kSilu: GLU_T_CASE(kSilu, KERN, lines, __VA_ARGS__)         \
+    case kGeluTanh: GLU_T_CASE(kGeluTanh, KERN, lines, __VA_ARGS__) \
+    case kRelu: GLU_T_CASE(kRelu, KERN, lines, __VA_ARGS__)         \
+    case kGeluErf: GLU_T_CASE(kGeluErf, KERN, lines, __VA_ARGS__)   \
+    default: GLU_T_CASE(kIdentity, KERN, lines, __VA_ARGS__)        \
   }
 
 // bf16 only: y [rows, I] and its transpose yt [I, rows] in one pass
 HDS_EXPORT int hds_glu_fwd_t(int act, const void* gu, void* y, void* yt, int rows, int I, hipStream_t st) {
   if (I % 8 || rows % 8 || rows <= 0 || I <= 0) return hipErrorInvalidValue;
   if (((uintptr_t)gu | (uintptr_t)y | (uintptr_t)yt) & 15) return hipErrorInvalidValue;
-  dim3 grid((I + GT_C - 1) / GT_C, (rows + GT_R - 1) / GT_R), block(256);
-  GLU_T_SWITCH(act, glu_fwd_t, grid, block, 0, st, (const bf16*)gu, (bf16*)y, (bf16*)yt, rows, I);
+  const dim3 grid(tile_count(rows, I)), block(256);
+  GLU_T_SWITCH(act, glu_fwd_t, tile_lines(rows, yt), grid, block, 0, st, (const bf16*)gu, (bf16*)y, (bf16*)yt, rows, I);
   return hipGetLastError();
 }
 
@@ -542,8 +515,8 @@ HDS_EXPORT int hds_glu_bwd_t(int act, const void* dy, const void* gu, void* dgu,
                              hipStream_t st) {
   if (I % 8 || rows % 8 || rows <= 0 || I <= 0) return hipErrorInvalidValue;
   if (((uintptr_t)dy | (uintptr_t)gu | (uintptr_t)dgu | (uintptr_t)dgut) & 15) return hipErrorInvalidValue;
-  dim3 grid((I + GT_C - 1) / GT_C, (rows + GT_R - 1) / GT_R), block(256);
-  GLU_T_SWITCH(act, glu_bwd_t, grid, block, 0, st, (const bf16*)dy, (const bf16*)gu, (bf16*)dgu, (bf16*)dgut, rows,
+  const dim3 grid(tile_count(rows, I)), block(256);
+  GLU_T_SWITCH(act, glu_bwd_t, tile_lines(rows, dgut), grid, block, 0, st, (const bf16*)dy, (const bf16*)gu, (bf16*)dgu, (bf16*)dgut, rows,
                I);
   return hipGetLastError();
 }

@@ -81,6 +81,11 @@ __device__ __forceinline__ void store4_nt(T* p, const float (&v)[4]) {
 // 16-byte global access per lane; for f32 two 16-byte accesses.
 template <typename T> struct Vec8;
 template <> struct Vec8<bf16> {
+  __device__ __forceinline__ static void load_nt(const bf16* p, float (&v)[8]) {
+    const bf16x8 r = hds::load_nt(reinterpret_cast<const bf16x8*>(p));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = (float)r[i];
+  }
   __device__ __forceinline__ static void load(const bf16* p, float (&v)[8]) {
     bf16x8 r = *reinterpret_cast<const bf16x8*>(p);
 #pragma unroll
@@ -95,6 +100,11 @@ template <> struct Vec8<bf16> {
 };
 template <> struct Vec8<_Float16> {
   typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+  __device__ __forceinline__ static void load_nt(const _Float16* p, float (&v)[8]) {
+    const h8 r = hds::load_nt(reinterpret_cast<const h8*>(p));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = (float)r[i];
+  }
   __device__ __forceinline__ static void load(const _Float16* p, float (&v)[8]) {
     h8 r = *reinterpret_cast<const h8*>(p);
 #pragma unroll
@@ -108,6 +118,12 @@ template <> struct Vec8<_Float16> {
   }
 };
 template <> struct Vec8<float> {
+  __device__ __forceinline__ static void load_nt(const float* p, float (&v)[8]) {
+    const f32x4 a = hds::load_nt(reinterpret_cast<const f32x4*>(p));
+    const f32x4 b = hds::load_nt(reinterpret_cast<const f32x4*>(p + 4));
+    v[0] = a[0]; v[1] = a[1]; v[2] = a[2]; v[3] = a[3];
+    v[4] = b[0]; v[5] = b[1]; v[6] = b[2]; v[7] = b[3];
+  }
   __device__ __forceinline__ static void load(const float* p, float (&v)[8]) {
     f32x4 a = *reinterpret_cast<const f32x4*>(p);
     f32x4 b = *reinterpret_cast<const f32x4*>(p + 4);

@@ -3,7 +3,7 @@
 // copies are written once at HBM rate instead of the TN GEMM running ~25 % below the NT one at the bench shapes.
 // Tile 64 x 64 through LDS: 16-B global loads along src rows, 16-B global stores along dst rows; the LDS tile is
 // padded to 66 elements per row so the column reads of the store phase spread over the banks.
-#include "hds_common.h"
+#include "transpose_tile.h"
 
 namespace {
 using namespace hds;
@@ -50,25 +50,19 @@ __global__ __launch_bounds__(256) void transpose_bf16_kernel(const bf16* __restr
   }
 }
 
-// v2 (default): tile 64 rows x 128 columns, 256 threads, every LDS access 8 or 16 B wide.
-//   load : 16-B global loads along src rows (16 lanes = one 256-B row), one ds_write_b128 each -- a 16-lane group
-//          writes a whole 256-B LDS row, conflict-free.
-//   store: thread (lr = t / 32, lc = t % 32) owns the 8 x 4 block rows 8lr..8lr+7, columns 4lc..4lc+3: eight
-//          ds_read_b64 (a half-wave reads the 32 8-B granules of one LDS row -> all 64 banks), 16 v_perm_b32 pack the
-//          four transposed 8-element vectors, four 16-B stores to dst rows c0 + 4lc + i.
-// v1's LDS traffic was one 2-B write and one 2-B read per element (32 LDS instructions per thread per 16 B moved).
-constexpr int TR = 64, TC = 128;
-
+// v2 (default): 64 x 128 tiles, every LDS access 8 or 16 B wide (transpose_tile.h). v1's LDS traffic was one 2-B write and
+// one 2-B read per element (32 LDS instructions per thread per 16 B moved).
+template <bool LINES>
 __global__ __launch_bounds__(256) void transpose_bf16_v2_kernel(const bf16* __restrict__ src, bf16* __restrict__ dst,
                                                                 int rows, int cols, int64_t lds) {
-  __shared__ __attribute__((aligned(16))) bf16 tile[TR * TC];
-  const int r0 = blockIdx.y * TR, c0 = blockIdx.x * TC;
+  __shared__ __attribute__((aligned(16))) bf16 tile[kTrRows * kTrCols];
+  const TileAt at = tile_at<LINES>(rows, cols);
   const int tid = threadIdx.x;
-  const bool full = (r0 + TR <= rows) && (c0 + TC <= cols);
+  const bool full = (at.r0 + kTrRows <= rows) && (at.c0 + kTrCols <= cols);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int v = tid + 256 * i, rr = v >> 4, cc = (v & 15) * 8;
-    const int r = r0 + rr, c = c0 + cc;
+    const int v = tid + 256 * i, rr = v >> 4, ch = v & 15;
+    const int r = at.r0 + rr, c = at.c0 + 8 * ch;
     bf16x8 x;
     if (full || (r < rows && c + 7 < cols)) {
       x = *reinterpret_cast<const bf16x8*>(src + (int64_t)r * lds + c);
@@ -76,26 +70,10 @@ __global__ __launch_bounds__(256) void transpose_bf16_v2_kernel(const bf16* __re
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = (r < rows && c + j < cols) ? src[(int64_t)r * lds + c + j] : (bf16)0.f;
     }
-    *reinterpret_cast<bf16x8*>(&tile[rr * TC + cc]) = x;
+    *reinterpret_cast<bf16x8*>(&tile[tile_chunk(rr, ch)]) = x;
   }
   __syncthreads();
-  const int lr = tid >> 5, lc = tid & 31;
-  u32x2 v[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const u32x2*>(&tile[(8 * lr + j) * TC + 4 * lc]);
-  const int r = r0 + 8 * lr;
-  if (r >= rows) return;  // rows % 8 == 0: a block row is all in or all out
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int c = c0 + 4 * lc + i;
-    if (!full && c >= cols) break;
-    // element i of row j sits in dword i/2 of v[j], low half for even i; pack rows (2k, 2k+1) into word k
-    const uint32_t sel = (i & 1) ? 0x07060302u : 0x05040100u;
-    u32x4 y;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) y[k] = __builtin_amdgcn_perm(v[2 * k + 1][i >> 1], v[2 * k][i >> 1], sel);
-    *reinterpret_cast<u32x4*>(dst + (int64_t)c * rows + r) = y;
-  }
+  store_transposed<LINES>(tile, dst, at, rows, cols);
 }
 
 }  // namespace
@@ -111,9 +89,13 @@ HDS_EXPORT int hds_transpose_bf16_var(const void* src, void* dst, int rows, int 
     hipLaunchKernelGGL(transpose_bf16_kernel, grid, dim3(256), 0, st, (const bf16*)src, (bf16*)dst, rows, cols,
                        (int64_t)lds);
   } else {
-    dim3 grid((cols + TC - 1) / TC, (rows + TR - 1) / TR);
-    hipLaunchKernelGGL(transpose_bf16_v2_kernel, grid, dim3(256), 0, st, (const bf16*)src, (bf16*)dst, rows, cols,
-                       (int64_t)lds);
+    const dim3 grid(tile_count(rows, cols));
+    if (tile_lines(rows, dst))
+      hipLaunchKernelGGL(transpose_bf16_v2_kernel<true>, grid, dim3(256), 0, st, (const bf16*)src, (bf16*)dst, rows,
+                         cols, (int64_t)lds);
+    else
+      hipLaunchKernelGGL(transpose_bf16_v2_kernel<false>, grid, dim3(256), 0, st, (const bf16*)src, (bf16*)dst, rows,
+                         cols, (int64_t)lds);
   }
   return hipGetLastError();
 }
