@@ -24,20 +24,32 @@ HDS_EXPORT int64_t hds_ragged_meta_size(int n_seqs, int64_t n_tokens, int max_bl
   return 4LL * n_seqs + 2LL * n_tokens + (int64_t)n_seqs * max_blocks + 3LL * n_atoms;
 }
 
-HDS_EXPORT int64_t hds_ragged_meta_build(const int32_t* n_new, const int32_t* seen, int n_seqs,
-                                         const int32_t* blocks, const int64_t* block_off, int max_blocks, int n_q,
-                                         int n_kv, int rows_per_atom, int32_t* out, int64_t cap, int64_t* need) {
-  if (n_seqs < 0 || n_kv <= 0 || n_q % n_kv != 0 || rows_per_atom <= 0 || max_blocks < 0) return -2;
-  const int G = n_q / n_kv;
-  int64_t T = 0, A = 0;
+namespace {
+
+struct Seq {
+  int32_t n_new, seen;
+  const int32_t* blocks;
+  int64_t n_blocks;
+};
+
+struct Counts {
+  int64_t tokens, atoms;
+};
+
+template <typename At>
+Counts count(const At& at, int n_seqs, int n_q, int n_kv, int rows_per_atom) {
+  Counts c{0, 0};
   for (int s = 0; s < n_seqs; ++s) {
-    T += n_new[s];
-    const int64_t rows = (int64_t)n_new[s] * G;
-    A += (int64_t)n_kv * ((rows + rows_per_atom - 1) / rows_per_atom);
+    const int64_t n = at(s).n_new;
+    c.tokens += n;
+    c.atoms += (int64_t)n_kv * ((n * (n_q / n_kv) + rows_per_atom - 1) / rows_per_atom);
   }
-  const int64_t size = hds_ragged_meta_size(n_seqs, T, max_blocks, A);
-  if (need) *need = size;
-  if (size > cap) return -1;
+  return c;
+}
+
+template <typename At>
+void build(const At& at, int n_seqs, int64_t T, int max_blocks, int n_q, int n_kv, int rows_per_atom, int32_t* out) {
+  const int G = n_q / n_kv;
   int32_t* meta = out;
   int32_t* tok_seq = meta + 3LL * n_seqs;
   int32_t* tok_pos = tok_seq + T;
@@ -46,7 +58,8 @@ HDS_EXPORT int64_t hds_ragged_meta_build(const int32_t* n_new, const int32_t* se
   int32_t* atoms = tables + (int64_t)n_seqs * max_blocks;
   int64_t q0 = 0, a = 0;
   for (int s = 0; s < n_seqs; ++s) {
-    const int32_t n = n_new[s], sn = seen[s];
+    const Seq q = at(s);
+    const int32_t n = q.n_new, sn = q.seen;
     meta[3 * s] = (int32_t)q0;
     meta[3 * s + 1] = n;
     meta[3 * s + 2] = sn;
@@ -55,10 +68,9 @@ HDS_EXPORT int64_t hds_ragged_meta_build(const int32_t* n_new, const int32_t* se
       tok_pos[q0 + i] = sn + i;
     }
     last[s] = (int32_t)(q0 + (n > 0 ? n - 1 : 0));
-    const int64_t b0 = block_off[s], nb = block_off[s + 1] - b0;
     int32_t* row = tables + (int64_t)s * max_blocks;
-    const int64_t ncopy = nb < max_blocks ? nb : max_blocks;
-    if (ncopy > 0) std::memcpy(row, blocks + b0, sizeof(int32_t) * ncopy);
+    const int64_t ncopy = q.n_blocks < max_blocks ? q.n_blocks : max_blocks;
+    if (ncopy > 0) std::memcpy(row, q.blocks, sizeof(int32_t) * ncopy);
     if (ncopy < max_blocks) std::memset(row + ncopy, 0, sizeof(int32_t) * (max_blocks - ncopy));
     const int64_t rows = (int64_t)n * G;
     for (int hk = 0; hk < n_kv; ++hk)
@@ -70,5 +82,55 @@ HDS_EXPORT int64_t hds_ragged_meta_build(const int32_t* n_new, const int32_t* se
       }
     q0 += n;
   }
-  return A;
+}
+
+}  // namespace
+
+HDS_EXPORT int64_t hds_ragged_meta_build(const int32_t* n_new, const int32_t* seen, int n_seqs,
+                                         const int32_t* blocks, const int64_t* block_off, int max_blocks, int n_q,
+                                         int n_kv, int rows_per_atom, int32_t* out, int64_t cap, int64_t* need) {
+  if (n_seqs < 0 || n_kv <= 0 || n_q % n_kv != 0 || rows_per_atom <= 0 || max_blocks < 0) return -2;
+  auto at = [&](int s) { return Seq{n_new[s], seen[s], blocks + block_off[s], block_off[s + 1] - block_off[s]}; };
+  const Counts c = count(at, n_seqs, n_q, n_kv, rows_per_atom);
+  const int64_t size = hds_ragged_meta_size(n_seqs, c.tokens, max_blocks, c.atoms);
+  if (need) *need = size;
+  if (size > cap) return -1;
+  build(at, n_seqs, c.tokens, max_blocks, n_q, n_kv, rows_per_atom, out);
+  return c.atoms;
+}
+
+// A whole step in one call, from the sequences' own buffers: the 64-bit token ids, the layout above and `n_extra` further values
+// go to `out` (8-byte aligned) one behind the other. seqs [n_seqs][5]: address of the tokens (int64), their number, tokens
+// seen, address of the KV blocks (int32), their number. id_limit: ids must lie in [0, id_limit) (0: any). info: ints needed,
+// smallest and largest id. Returns the number of atoms; -1 when `cap` is too small (nothing is written), -3 with an id outside.
+HDS_EXPORT int64_t hds_ragged_step_build(const int64_t* seqs, int n_seqs, int max_blocks, int n_q, int n_kv,
+                                         int rows_per_atom, int64_t id_limit, const int32_t* extra, int64_t n_extra,
+                                         int32_t* out, int64_t cap, int64_t* info) {
+  if (n_seqs < 0 || n_kv <= 0 || n_q % n_kv != 0 || rows_per_atom <= 0 || max_blocks < 0 || n_extra < 0) return -2;
+  auto at = [&](int s) {
+    const int64_t* q = seqs + 5 * (int64_t)s;
+    return Seq{(int32_t)q[1], (int32_t)q[2], reinterpret_cast<const int32_t*>(q[3]), q[4]};
+  };
+  const Counts c = count(at, n_seqs, n_q, n_kv, rows_per_atom);
+  const int64_t size = hds_ragged_meta_size(n_seqs, c.tokens, max_blocks, c.atoms);
+  info[0] = 2 * c.tokens + size + n_extra;
+  if (info[0] > cap) return -1;
+  int64_t* ids = reinterpret_cast<int64_t*>(out);
+  int64_t lo = INT64_MAX, hi = INT64_MIN;
+  for (int s = 0; s < n_seqs; ++s) {
+    const int64_t* t = reinterpret_cast<const int64_t*>(seqs[5 * (int64_t)s]);
+    const int64_t n = seqs[5 * (int64_t)s + 1];
+    for (int64_t i = 0; i < n; ++i) {
+      lo = t[i] < lo ? t[i] : lo;
+      hi = t[i] > hi ? t[i] : hi;
+      *ids++ = t[i];
+    }
+  }
+  info[1] = lo;
+  info[2] = hi;
+  if (c.tokens > 0 && id_limit > 0 && (lo < 0 || hi >= id_limit)) return -3;
+  int32_t* meta = out + 2 * c.tokens;
+  build(at, n_seqs, c.tokens, max_blocks, n_q, n_kv, rows_per_atom, meta);
+  if (n_extra > 0) std::memcpy(meta + size, extra, sizeof(int32_t) * (size_t)n_extra);
+  return c.atoms;
 }

@@ -152,11 +152,14 @@ class InferenceEngineV2:
         sm, batch = self._state_manager, self._batch
         batch.clear()
         places = [None] * len(batch_uids) if logits_at is None else [list(p) for p in logits_at]
+        seqs = []
         for uid, tokens, want in zip(batch_uids, batch_tokens, places):
             seq = sm.get_or_create_sequence(uid)
-            sm.maybe_allocate_kv(seq, tokens.numel())
-            seq.pre_forward(tokens.numel())
+            n = tokens.numel()
+            sm.maybe_allocate_kv(seq, n)
+            seq.pre_forward(n)
             batch.insert_sequence(seq, tokens, do_checks=do_checks, logits_at=want)
+            seqs.append(seq)
         batch.finalize(self._model.id_limit())
         if self._model.decode_graph_eligible(batch, capture_latents):
             # HIP-graph decode step (latents, if captured, land in the graph's device ring)
@@ -167,11 +170,9 @@ class InferenceEngineV2:
             logits, latents = self._model.forward(batch, capture_latents=capture_latents,
                                                   sync_latents=True if sync_latents is None else sync_latents)
             self._latent_event = getattr(self._model, "latent_event", None)
-        split = []
-        for (q0, n, _) in batch.seq_meta_host:
-            split.append(latents[:, q0:q0 + n] if latents is not None else None)
-        for uid in batch_uids:
-            sm.get_sequence(uid).post_forward()
+        split = [None if latents is None else latents[:, q0:q0 + n] for (q0, n, _) in batch.seq_meta_host]
+        for seq in seqs:
+            seq.post_forward()
         return logits, split
 
     def latents_ready(self) -> bool:
@@ -259,8 +260,8 @@ class InferenceEngineV2:
         sm = self._state_manager
         cfg = self._config.state_manager
         uids, lengths = list(uids), list(lengths)
-        new_seqs = sum(1 for u in uids if sm.get_sequence(u) is None)
-        if sm.n_tracked_sequences + new_seqs > cfg.max_tracked_sequences:
+        seqs = [sm.get_sequence(u) for u in uids]
+        if sm.n_tracked_sequences + sum(seq is None for seq in seqs) > cfg.max_tracked_sequences:
             return SchedulingResult.EngineSequenceLimitExceeded
         if len(uids) > cfg.max_ragged_sequence_count:
             return SchedulingResult.BatchSequenceLimitExceeded
@@ -268,10 +269,8 @@ class InferenceEngineV2:
             return SchedulingResult.BatchTokenLimitExceeded
         need = 0
         bs = self._kv.block_size
-        for u, n in zip(uids, lengths):
-            seq = sm.get_sequence(u)
-            seen = seq.seen_tokens if seq else 0
-            alloc = seq.cur_allocated_blocks if seq else 0
+        for seq, n in zip(seqs, lengths):
+            seen, alloc = (seq.seen_tokens, len(seq._blocks)) if seq else (0, 0)
             if seen + n > cfg.max_context:
                 return SchedulingResult.SequenceTokenLimitExceeded
             need += max(0, (seen + n + bs - 1) // bs - alloc)

@@ -37,6 +37,7 @@ import torch
 import torch.nn.functional as F
 
 from ... import comm as dist
+from ...ops import native
 from ...ops.activations import glu
 from ...ops.norm import layer_norm, rms_norm
 from ...ops.paged import build_atoms, kv_rope_scatter
@@ -540,18 +541,25 @@ class RaggedTransformer:
         return dequantize_fp8(q, sc, group_size=H, dtype=self.dtype).view(T, H)
 
     def _d2h(self, src, dst, events):
-        if self.copy_stream is None:
+        """``src`` to the pinned ``dst`` on the copy stream, behind what the current stream has been given; ``events`` gets the
+        event after the last copy (the earlier ones are in front of it)."""
+        cs = self.copy_stream
+        if cs is None:
             dst.copy_(src)
             return
-        ev = torch.cuda.Event()
-        ev.record()
-        with torch.cuda.stream(self.copy_stream):
-            self.copy_stream.wait_event(ev)
-            dst.copy_(src, non_blocking=True)
-            src.record_stream(self.copy_stream)
-            done = torch.cuda.Event()
-            done.record(self.copy_stream)
-        events.append(done)
+        now = torch.cuda.Event()
+        now.record(torch.cuda.current_stream(src.device))
+        cs.wait_event(now)
+        if src.is_contiguous() and dst.is_contiguous() and src.dtype == dst.dtype and src.shape == dst.shape:
+            native.check(native.host_lib().hds_memcpy_async(dst.data_ptr(), src.data_ptr(), src.numel() * src.element_size(),
+                                                            1, cs.cuda_stream), "memcpy_async")
+        else:
+            with torch.cuda.stream(cs):
+                dst.copy_(src, non_blocking=True)
+        src.record_stream(cs)
+        if not events:
+            events.append(torch.cuda.Event())
+        events[0].record(cs)
 
     # ------------------------------------------------------------------------------------------
     @torch.no_grad()

@@ -10,6 +10,7 @@ MI355X sizing: the KV pool is carved out of the 288 GB HBM after weights (``memo
 "reserve" keeps ``size`` bytes free, "allocate" takes exactly ``size`` bytes). Host metadata lives in
 pinned buffers so ``finalize`` is one async H2D copy.
 """
+from array import array
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional
 
@@ -96,7 +97,7 @@ class DSSequenceDescriptor:
         self.seen_tokens = 0
         self.in_flight_tokens = 0
         self.evicted_state = None  # (tokens seen, host copy of the state row) of an evicted sequence
-        self._blocks: List[int] = []
+        self._blocks = array("i")  # the step's builder reads it in place
         self.max_blocks = max_blocks
 
     @property
@@ -112,7 +113,7 @@ class DSSequenceDescriptor:
                                               new_blocks))
 
     def free_kv_cache(self):
-        b, self._blocks = self._blocks, []
+        b, self._blocks = list(self._blocks), array("i")
         return b
 
     def pre_forward(self, num_tokens):
@@ -250,13 +251,28 @@ class DSStateManager:
 # ragged batch
 # -----------------------------------------------------------------------------------------------
 class RaggedBatchWrapper:
-    """Host-built batch metadata; ``finalize`` ships it to the device in one async copy each."""
+    """Host-built batch metadata; ``finalize`` ships it to the device in one async copy. The device tensors
+    (``input_ids``, ``seq_meta``, ``tok_seq``, ``tok_pos``, ``last_token_idx``, ``block_tables``, ``atoms``, ``slots``) and the
+    host's ``tables_host`` are views of its buffer, made when they are asked for: a replayed decode step asks for none."""
 
     def __init__(self, config: DSStateManagerConfig, device, max_blocks_per_seq):
         self._config = config
         self.device = device
         self.max_blocks = max_blocks_per_seq
         self.clear()
+
+    def __getattr__(self, name):  # (only what the instance does not hold)
+        try:
+            o, k, shape = self.__dict__["_layout"][name]
+        except KeyError:
+            raise AttributeError(name) from None
+        if name == "tables_host":
+            v = self._host_now[o:o + k].view(shape).clone()
+        else:
+            v = self._dev_meta[o:o + k]
+            v = v.view(torch.int64) if name == "input_ids" else v.view(shape)
+        self.__dict__[name] = v
+        return v
 
     def clear(self):
         self._seqs: List[DSSequenceDescriptor] = []
@@ -284,7 +300,9 @@ class RaggedBatchWrapper:
             self._logit_rows = (self._logit_rows or []) + [self.current_tokens + int(i) for i in logits_at]
         self.seq_meta_host.append((self.current_tokens, n, seq.seen_tokens))
         self._seqs.append(seq)
-        self._tokens.append(tokens.reshape(-1).to(torch.int64))
+        if tokens.dim() != 1 or tokens.dtype != torch.int64 or not tokens.is_contiguous():
+            tokens = tokens.reshape(-1).to(torch.int64).contiguous()
+        self._tokens.append(tokens)
         self.current_tokens += n
 
     def set_attention_geometry(self, n_q, n_kv, rows_per_atom, portions=True):
@@ -293,7 +311,7 @@ class RaggedBatchWrapper:
         self._geom = (int(n_q), int(n_kv), int(rows_per_atom))
         self._portions = portions
 
-    def _pinned_slot(self, need):
+    def _pinned_slot(self):
         """One of two rotating pinned int32 staging buffers; a slot is reused only after its H2D drained."""
         slots = self.__dict__.setdefault("_slots", [None, None])
         evs = self.__dict__.setdefault("_slot_events", [None, None])
@@ -301,94 +319,102 @@ class RaggedBatchWrapper:
         self._slot_next = i ^ 1
         if evs[i] is not None:
             evs[i].synchronize()
-        if slots[i] is None or slots[i].numel() < need:
-            slots[i] = torch.empty(max(need, 4096), dtype=torch.int32, pin_memory=self.device.type == "cuda")
-        return i, slots[i]
+        if slots[i] is None:
+            slots[i] = self._pinned(4096)
+        return i
+
+    def _pinned(self, n):
+        return torch.empty(max(n, 4096), dtype=torch.int32, pin_memory=self.device.type == "cuda")
 
     def finalize(self, id_limit=None):
         """Ship the batch description to the device: the native builder (csrc/host/ragged_meta.cpp) writes seq_meta,
         token -> sequence / position maps, last-token rows, the KV block table and the attention atoms into ONE
         pinned int32 buffer behind the 64-bit token ids, sent with one async H2D copy into a persistent device buffer;
-        the device tensors below are views of it. ``id_limit``: token ids outside [0, id_limit) raise IndexError, before
+        the device tensors are views of it. ``id_limit``: token ids outside [0, id_limit) raise IndexError, before
         anything is sent (a lookup on the device cannot refuse them)."""
-        import ctypes
-        import numpy as np
         from ...ops import native
         from ...ops.paged_prefill import divide_step
-        S, T = len(self._seqs), self.current_tokens
-        mb = self.max_blocks
-        n_new = np.fromiter((nn for (_, nn, _) in self.seq_meta_host), dtype=np.int32, count=S)
-        seen = np.fromiter((sn for (_, _, sn) in self.seq_meta_host), dtype=np.int32, count=S)
-        blk_lists = [seq.kv_blocks for seq in self._seqs]
-        off = np.zeros(S + 1, dtype=np.int64)
-        if S:
-            off[1:] = np.cumsum([len(b) for b in blk_lists])
-        flat = np.fromiter((b for bl in blk_lists for b in bl), dtype=np.int32, count=int(off[-1]))
-        n_q, n_kv, rpa = getattr(self, "_geom", (1, 1, 1 << 30))
+        seqs, meta = self._seqs, self.seq_meta_host
+        S, T, mb = len(seqs), self.current_tokens, self.max_blocks
+        geom = self.__dict__.get("_geom")
+        n_q, n_kv, rpa = geom or (1, 1, 1 << 30)
         lib = native.host_lib()
-        P = lambda a: a.ctypes.data_as(ctypes.c_void_p)  # noqa: E731
-        need = ctypes.c_int64(0)
-        lib.hds_ragged_meta_build(P(n_new), P(seen), S, P(flat), P(off), mb, n_q, n_kv, rpa, None, 0,
-                                  ctypes.byref(need))
         # after the builder's part: the sequences' state slots, explicit logits rows, the division of a step that is not
         # single tokens only
-        mixed = getattr(self, "_portions", True) and any(nn != 1 for (_, nn, _) in self.seq_meta_host)
-        toks, blocks, rows = divide_step(self.seq_meta_host, n_q, n_kv) if mixed else ([], [], [])
-        extra = [seq.tracking_id for seq in self._seqs] + (self._logit_rows or []) + blocks + toks + rows
-        head = 2 * T  # the ids, first: 8-byte aligned
-        si, host = self._pinned_slot(head + int(need.value) + len(extra))
-        A = lib.hds_ragged_meta_build(P(n_new), P(seen), S, P(flat), P(off), mb, n_q, n_kv, rpa,
-                                      ctypes.c_void_p(host.data_ptr() + 4 * head), host.numel() - head, ctypes.byref(need))
+        max_new = max((m[1] for m in meta), default=0)
+        mixed = getattr(self, "_portions", True) and any(m[1] != 1 for m in meta)
+        toks, blocks, rows = divide_step(meta, n_q, n_kv) if mixed else ([], [], [])
+        self.slots_host = [seq.tracking_id for seq in seqs]
+        extra = array("i", self.slots_host + (self._logit_rows or []) + blocks + toks + rows)
+        desc = array("q")
+        for seq, t, m in zip(seqs, self._tokens, meta):
+            if not t.is_cpu:
+                raise RuntimeError(f"token ids come from the host, not from {t.device}")
+            at, n = seq._blocks.buffer_info()
+            desc.extend((t.data_ptr(), m[1], m[2], at, n))
+        info = array("q", (0, 0, 0))
+        si = self._pinned_slot()
+        while True:
+            host = self._slots[si]
+            A = lib.hds_ragged_step_build(desc.buffer_info()[0], S, mb, n_q, n_kv, rpa, id_limit or 0,
+                                          extra.buffer_info()[0], len(extra), host.data_ptr(), host.numel(),
+                                          info.buffer_info()[0])
+            if A != -1:
+                break
+            self._slots[si] = self._pinned(info[0])
+        if A == -3:
+            raise IndexError(f"token ids from {info[1]} to {info[2]}: the embedding has {id_limit} rows")
         if A < 0:
             raise RuntimeError(f"ragged metadata builder failed ({A})")
-        if T:
-            ids = torch.cat(self._tokens, out=host[:head].view(torch.int64)).numpy()
-            if id_limit is not None and ids.view(np.uint64).max() >= id_limit:  # (negative ones are the largest)
-                raise IndexError(f"token ids from {ids.min()} to {ids.max()}: the embedding has {id_limit} rows")
-        n = head + int(need.value)
-        if extra:
-            host.numpy()[n:n + len(extra)] = extra
-        n += len(extra)
-        dev_buf = self.__dict__.get("_dev_meta")
+        n, held = info[0], self.__dict__
+        dev_buf = held.get("_dev_meta")
         if dev_buf is None or dev_buf.numel() < n:
             dev_buf = self._dev_meta = torch.empty(max(n, 4096), dtype=torch.int32, device=self.device)
-        dev_buf[:n].copy_(host[:n], non_blocking=True)
         if self.device.type == "cuda":
-            ev = torch.cuda.Event()
-            ev.record()
-            self._slot_events[si] = ev
-        self.input_ids = dev_buf[:head].view(torch.int64)
-        o = head
-
-        def take(k, shape):
-            nonlocal o
-            v = dev_buf[o:o + k].view(*shape)
+            stream = torch.cuda.current_stream(self.device)
+            if n:
+                native.check(lib.hds_memcpy_async(dev_buf.data_ptr(), host.data_ptr(), 4 * n, 0, stream.cuda_stream),
+                             "memcpy_async")
+            ev = self._slot_events[si]
+            if ev is None:
+                ev = self._slot_events[si] = torch.cuda.Event()
+            ev.record(stream)
+        else:
+            dev_buf[:n].copy_(host[:n])
+        self._host_now = host
+        head = o = 2 * T  # the ids, first: 8-byte aligned
+        parts = [("seq_meta", (S, 3)), ("tok_seq", (T, )), ("tok_pos", (T, )), ("last_token_idx", (S, )),
+                 ("block_tables", (S, mb)), ("atoms", (A, 3)), ("slots", (S, ))]
+        layout = {"input_ids": (0, head, None)}
+        for name, shape in parts:
+            k = shape[0] * shape[1] if len(shape) == 2 else shape[0]
+            layout[name] = (o, k, shape)
             o += k
-            return v
-
-        self.seq_meta = take(3 * S, (S, 3))
-        self.tok_seq = take(T, (T, ))
-        self.tok_pos = take(T, (T, ))
-        self.last_token_idx = take(S, (S, ))
-        self.block_tables = take(S * mb, (S, mb))
-        self.atoms = take(3 * A, (A, 3)) if hasattr(self, "_geom") else None
-        self.n_atoms = int(A) if hasattr(self, "_geom") else None
-        if self.atoms is None:
-            take(3 * A, (3 * A, ))
-        self.slots = take(S, (S, ))
-        self.slots_host = [seq.tracking_id for seq in self._seqs]
-        self.max_new = int(n_new.max()) if S else 0
+        layout["tables_host"] = layout["block_tables"]
+        if self._logit_rows is not None:
+            layout["last_token_idx"] = (o, len(self._logit_rows), (-1, ))
+            o += len(self._logit_rows)
+        for name in layout:
+            held.pop(name, None)
+        self._layout = layout
+        self.n_atoms = int(A) if geom else None
+        if geom is None:
+            self.atoms = None
+        self.max_new = max_new
         self.plans = {}
         self.carry = {}
-        if self._logit_rows is not None:
-            self.last_token_idx = take(len(self._logit_rows), (-1, ))
         self.portions = None
         if mixed:
+            def take(k, shape):
+                nonlocal o
+                v = dev_buf[o:o + k].view(shape)
+                o += k
+                return v
+
             blocks = take(len(blocks), (-1, 2)) if blocks else None
             self.portions = (take(len(toks), (-1, )) if toks else None, blocks, take(len(rows), (-1, 3)) if rows else None)
-        self.tables_host = host[head + 4 * S + 2 * T:head + 4 * S + 2 * T + S * mb].view(S, mb).clone() if S else \
-            torch.zeros(1, mb, dtype=torch.int32)
         if S == 0:  # keep 1-row shapes for empty batches (kernels never run on them)
+            self.tables_host = torch.zeros(1, mb, dtype=torch.int32)
             self.seq_meta = torch.zeros(1, 3, dtype=torch.int32, device=self.device)
             self.block_tables = torch.zeros(1, mb, dtype=torch.int32, device=self.device)
             self.last_token_idx = torch.zeros(1, dtype=torch.int32, device=self.device)

@@ -124,6 +124,8 @@ def glu(gu, act="silu", transposed=False):
     and attaches it as ``out._hds_t``; a ZeRO linear consuming ``out`` saves that copy instead of ``out`` for its
     weight gradient (hipBLASLt's NT form needs the token dimension contiguous). The backward likewise hands the
     gate|up projection the transpose of d(gate|up). Both replace a separate HBM transpose pass in the backward."""
+    if gu.is_cuda and not transposed and native.plain(gu) and not _ap.tracking():
+        return _glu_out(gu, act_code(act))  # (a serving step's activations)
     return _GLUFn.apply(gu, act_code(act), bool(transposed))
 
 

@@ -47,6 +47,7 @@ def gemv(x2, w, b=None):
 # 2..16 token rows: the matrix-core skinny GEMM (csrc/kernels/gemv.hip skinny_lines_kernel) instead of the VALU GEMV /
 # hipBLASLt's small-M tiles (HDS_SKINNY_GEMM=0: those)
 SKINNY = _os.environ.get("HDS_SKINNY_GEMM", "1") == "1"
+MAX_ROWS = 16  # of either kernel
 SKINNY_MIN_M = int(_os.environ.get("HDS_SKINNY_MIN_M", "2"))  # 1: one-row linears too (instead of the VALU GEMV)
 
 
@@ -55,7 +56,7 @@ def skinny_ok(x2, w, b=None):
             and w.dim() == 2):
         return False
     M, K = x2.shape
-    if not SKINNY_MIN_M <= M <= 16 or w.shape[1] != K or K % 128 or not w.is_contiguous() or x2.stride(1) != 1 or x2.stride(0) % 8:
+    if not SKINNY_MIN_M <= M <= MAX_ROWS or w.shape[1] != K or K % 128 or not w.is_contiguous() or x2.stride(1) != 1 or x2.stride(0) % 8:
         return False
     if x2.data_ptr() % 16 or w.data_ptr() % 16:
         return False
@@ -79,7 +80,8 @@ def _needs_grad(*tensors):
 def glu_linear(x, w, b, act):
     """act(x . gate^T) * (x . up^T) for ``w`` = [gate; up] (and ``b``) in one kernel, for 2..16 rows of the skinny GEMM; None
     for anything else. The projections are rounded to bf16 first, as the separate kernels store them."""
-    if act not in _GATHER_ACTS or not (x.dim() >= 1 and x.is_cuda and torch.is_tensor(w)) or _needs_grad(x, w, b):
+    if act not in _GATHER_ACTS or not (x.dim() >= 1 and x.is_cuda and torch.is_tensor(w)) or \
+            x.numel() > MAX_ROWS * x.shape[-1] or _needs_grad(x, w, b):
         return None
     x2 = x.reshape(-1, x.shape[-1])
     if not skinny_ok(x2, w, b) or w.shape[0] % 2:
@@ -95,7 +97,7 @@ def glu_linear(x, w, b, act):
 def linear(x, w, b=None):
     """``F.linear(x, w, b)``; decode-sized bf16 inputs run the HIP GEMV (one row) or the skinny matrix-core GEMM
     (2..16 rows), unless a gradient is wanted."""
-    if x.dim() >= 1 and x.is_cuda and not _needs_grad(x, w, b):
+    if x.dim() >= 1 and x.is_cuda and x.numel() <= MAX_ROWS * x.shape[-1] and not _needs_grad(x, w, b):
         x2 = x.reshape(-1, x.shape[-1])
         if skinny_ok(x2, w, b):
             return skinny(x2, w, b).view(*x.shape[:-1], w.shape[0])

@@ -22,6 +22,7 @@ SIGS = {
     # ragged_meta.cpp
     "hds_ragged_meta_size": (L, [I, L, I, L]),
     "hds_ragged_meta_build": (L, [P, P, I, P, P, I, I, I, I, P, L, P]),
+    "hds_ragged_step_build": (L, [P, I, I, I, I, I, L, P, L, P, L, P]),
     # cpu_optim.cpp
     "hds_cpu_adam": (I, [P, P, I, P, P, P, L, F, F, F, F, F, F, F, I, F]),
     "hds_cpu_lion": (I, [P, P, I, P, P, L, F, F, F, F, F]),

@@ -320,6 +320,14 @@ def check(err, what):
             raise RuntimeError(f"hcache_deepspeed_amd: device fault after {what}: {e}") from e
 
 
+def plain(*tensors):
+    """No gradient, functorch transform or dual number can want a record of what is done with these tensors: an autograd
+    function around a kernel (about 10 us of host time) may be passed by."""
+    return (not torch.is_grad_enabled() and not torch._C._are_functorch_transforms_active()
+            and torch.autograd.forward_ad._current_level < 0
+            and all(t is None or type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors))
+
+
 def use_native(*tensors):
     """True when the tensors live on the GPU (native path mandatory there)."""
     for t in tensors:

@@ -130,15 +130,22 @@ class _NormFn(torch.autograd.Function):
         return dx, dres_out, dw, db, None, None
 
 
+def _norm(x, residual, weight, bias, eps, is_ln):
+    if x.is_cuda and x.dim() == 2 and x.is_contiguous() and native.plain(x, residual, weight, bias) and \
+            (residual is None or (residual.shape == x.shape and residual.is_contiguous())) and not _ap.tracking():
+        y, h = _native_fwd(x, residual, weight, bias, eps, is_ln)[:2]  # (a serving step's norms)
+    else:
+        y, h = _NormFn.apply(x, residual, weight, bias, eps, is_ln)
+    return (y, h) if residual is not None else y
+
+
 def rms_norm(x, weight, eps=1e-6, residual=None):
     """Returns y, or (y, new_residual) when ``residual`` is given (fused add + norm)."""
-    y, h = _NormFn.apply(x, residual, weight, None, eps, False)
-    return (y, h) if residual is not None else y
+    return _norm(x, residual, weight, None, eps, False)
 
 
 def layer_norm(x, weight, bias=None, eps=1e-5, residual=None):
-    y, h = _NormFn.apply(x, residual, weight, bias, eps, True)
-    return (y, h) if residual is not None else y
+    return _norm(x, residual, weight, bias, eps, True)
 
 
 def norm_picked_ok(x, residual, pick, *params):

@@ -99,6 +99,64 @@ def test_step_description_on_the_host():
         assert b.slots.tolist() == [sm.get_sequence(i).tracking_id for i in range(S)] and b.current_tokens == T
 
 
+def test_step_description_of_any_tokens():
+    """Ids of other types and strides, more of them than the first buffer holds, wanted places, an empty step, refused ids."""
+    from hcache_deepspeed_amd.inference.v2.ragged import (BlockedKVCache, DSStateManager, DSStateManagerConfig,
+                                                          RaggedBatchWrapper)
+    cfg = DSStateManagerConfig(max_context=8192, max_ragged_batch_size=8192)
+    kv = BlockedKVCache(1, 2, 16, 64, torch.float32, torch.device("cpu"), cfg.memory_config, num_blocks=200)
+    sm = DSStateManager(cfg, kv)
+    b = RaggedBatchWrapper(cfg, torch.device("cpu"), sm.max_blocks_per_seq)
+    assert not hasattr(b, "seq_meta")
+    b.set_attention_geometry(4, 2, 128)
+    steps = [[torch.arange(5, dtype=torch.int32), torch.arange(12)[::3]], [torch.arange(6000) % 100, torch.tensor(7)],
+             [torch.arange(8).view(2, 4), torch.tensor([99], dtype=torch.uint8)], []]
+    for toks in steps:
+        for where in (None, [[0, t.numel() - 1] for t in toks]):
+            b.clear()
+            for u in range(2):
+                sm.flush_sequence(u)
+            for i, t in enumerate(toks):
+                seq = sm.get_or_create_sequence(i)
+                sm.maybe_allocate_kv(seq, t.numel())
+                b.insert_sequence(seq, t, logits_at=None if where is None else where[i])
+            b.finalize(100)
+            flat = [t.reshape(-1).long() for t in toks]
+            ends = [sum(t.numel() for t in flat[:i + 1]) for i in range(len(flat))]
+            if toks:
+                assert torch.equal(b.input_ids, torch.cat(flat)) and b.seq_meta[:, 0].tolist() == [0] + ends[:-1]
+                last = [e - 1 for e in ends] if where is None else [e - t.numel() + i for e, t, w in zip(ends, flat, where) for i in w]
+                assert b.last_token_idx.tolist() == last and b.atoms.shape[0] == b.n_atoms
+                for i in range(len(toks)):
+                    blocks = sm.get_sequence(i).kv_blocks
+                    assert b.tables_host[i, :len(blocks)].tolist() == blocks and b.tables_host[i, len(blocks):].eq(0).all()
+            else:
+                assert b.seq_meta.shape == (1, 3) and b.input_ids.numel() == 0 and b.tables_host.shape[0] == 1
+    for bad in (-1, 100, 2**40):
+        b.clear()
+        b.insert_sequence(sm.get_or_create_sequence(0), torch.tensor([3, bad]))
+        with pytest.raises(IndexError, match=str(bad)):
+            b.finalize(100)
+
+
+def test_only_plain_tensors_pass_autograd_by():
+    from hcache_deepspeed_amd.ops import native
+    x = torch.ones(2)
+    assert not native.plain(x)
+    with torch.no_grad():
+        assert native.plain(x, None, torch.nn.Parameter(x))
+        seen = []
+        torch.func.vmap(lambda t: seen.append(native.plain(x)) or t)(x)
+        with torch.autograd.forward_ad.dual_level():
+            seen.append(native.plain(x))
+
+        class Sub(torch.Tensor):
+            pass
+
+        seen.append(native.plain(x.as_subclass(Sub)))
+        assert seen == [False, False, False]
+
+
 @pytest.mark.gpu
 def test_graph_after_the_buffer_grew_gpu():
     """A graph reads the batch's device buffer; when a larger step has replaced that, later steps reach the graph's own."""
