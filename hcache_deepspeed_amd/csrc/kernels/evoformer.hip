@@ -12,11 +12,13 @@
 //     statistics are lane-local and the S^T accumulator is the B operand of the next product (acc_to_b); V^T and K^T
 //     come out of the row-major tiles by transposing LDS reads. dQ also makes rowsum(dO * O), which the others read.
 //   * dK / dV: the same with 32 keys on the lanes and queries and output gradients in LDS.
+//   * dQ, dK and dV of rows of up to 256 positions, heads of 32 and bf16 biases: in one kernel, see evo_bwd_kernel.
 //   * pair-bias gradient: the sum of dS over the N rows stays in registers. A wave owns 32 queries x 64 keys of one
 //     (b, h) and walks over a chunk of the rows, recomputing the two products that dS needs; chunks are added by a second
 //     kernel that also rounds. No atomics, the same result every time.
-// Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): a forward and backward 198 us; in a kernel trace, where
-// launches do not overlap, forward 43 us, dQ 55, dK / dV 53, pair gradient 60 + 5
+// Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): a forward and backward 161 us (with dQ and dK / dV
+// apart 198); in a kernel trace, where launches do not overlap, forward 42 us, dQ + dK + dV 66 (apart 52 + 51), pair
+// gradient 56 + 4
 // (before: one wave a workgroup with operands from global memory and 2-byte reads of V 169 us; the FlashAttention
 // backward kernels with 32-bit atomics into the pair gradient 271 + 1,585 us).
 #include <cmath>
@@ -123,11 +125,17 @@ struct Diagonal {
   __device__ __forceinline__ explicit Diagonal(const Inverse<D>& inv) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int i = 0; i < Inverse<D>::N; ++i)
+    for (int ks = 0; ks < 2; ++ks) {
+      const int at = (lane & 31) - 16 * ks - 8 * (lane >> 5);  // the element that is not zero, if it is one of 0 .. 7
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
+      for (int i = 0; i < Inverse<D>::N; ++i) {
+        const uint32_t v = (uint32_t)__builtin_bit_cast(uint16_t, inv.v[i]) << (16 * (at & 1));
+        u32x4 r;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) f[i][ks][e] = 16 * ks + 8 * (lane >> 5) + e == (lane & 31) ? inv.v[i] : (bf16)0.f;
+        for (int e = 0; e < 4; ++e) r[e] = at >> 1 == e ? v : 0u;
+        f[i][ks] = __builtin_bit_cast(bf16x8, r);
+      }
+    }
   }
 };
 
@@ -190,11 +198,11 @@ struct QueryBias<D, bf16> {
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) f[ks] = load_eight<TAIL>(b2, k0 + 16 * ks + 8 * ((threadIdx.x & 63) >> 5), L);
   }
-  __device__ __forceinline__ f32x16 add_pair(const u32x4 (&f)[2], f32x16 s) const {
+  __device__ __forceinline__ f32x16 add_pair(const u32x4 (&f)[2], f32x16 s) const {  // made finite
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-      for (int i = 0; i < Inverse<D>::N; ++i) s = mfma(eye.f[i][ks], __builtin_bit_cast(bf16x8, finite(f[ks])), s);
+      for (int i = 0; i < Inverse<D>::N; ++i) s = mfma(eye.f[i][ks], __builtin_bit_cast(bf16x8, f[ks]), s);
     return s;
   }
   // what the scores start from: the mask, so that beside a huge one all keys' scores round alike
@@ -221,6 +229,8 @@ struct QueryBias<D, bf16> {
           seen = __builtin_bit_cast(u32x4, __builtin_elementwise_max(__builtin_bit_cast(u16x8, seen),
                                                                      __builtin_bit_cast(u16x8, f[ks])));
       }
+      f[0] = finite(f[0]);
+      f[1] = finite(f[1]);
       s = add_pair(f, s);
     }
     return s;
@@ -587,6 +597,237 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_dkdv_kernel(EvoParams p, i
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// dQ, dK, dV and the mask's gradient of short rows: all of a (b, n, h) in one workgroup
+// ---------------------------------------------------------------------------------------------------------------
+template <int D>
+struct Whole {  // a workgroup of one wave per 32 positions, a matrix of nt tiles in LDS
+  using T = Tile<D>;
+  static constexpr int CH = T::CH, PER = CH / 2;  // 16-byte chunks of a row; chunks of a matrix that a thread moves
+  static constexpr int SB = 128;                  // bytes of a row of dS^T: one key, 64 queries
+  static __host__ __device__ int bytes(int nt) { return 32 * nt * (3 * T::RB + SB + 8); }
+  // the thread's number, made anew where it is asked for: addresses that are needed once a row of the loop shall not
+  // stay in registers through it
+  static __device__ __forceinline__ int tid() {
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+  }
+  static __device__ __forceinline__ int row(int i, int t) { return (i * (int)blockDim.x + t) / CH; }
+  // (32-bit offsets from a base that all lanes share: a register each where addresses would take two per matrix)
+  static __device__ __forceinline__ void load(const bf16* m, uint32_t ld, int L, int t, u32x4 (&r)[PER]) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      r[i] = *reinterpret_cast<const u32x4*>((const char*)m + 2 * ((uint32_t)min(row(i, t), L - 1) * ld + 8 * (t % CH)));
+  }
+  static __device__ __forceinline__ void put(char* lds, int t, const u32x4 (&r)[PER]) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) *reinterpret_cast<u32x4*>(lds + T::off(row(i, t), t % CH)) = r[i];
+  }
+  // a transposed 4 x 16 piece and the one `step` bytes further
+  static __device__ __forceinline__ bf16x8 tr_pair(const char* a, int step) {
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(a));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(a + step));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+  // dS^T: 16 lanes that write 8 bytes of 16 keys, and 32 lanes that read 32 bytes of 8 keys, meet every bank once
+  static __device__ __forceinline__ int ds_off(int key, int ch) {
+    return key * SB + 16 * (ch ^ ((key & 2) | ((key >> 1) & 4) | ((key >> 2) & 1)));
+  }
+};
+
+// Wave w holds keys 32 w .. on its lanes, as the dK / dV kernel does, and walks over the queries. Every 64 queries the
+// waves leave their dS in LDS and each makes 16 x 16 pieces of dQ from all keys. The workgroup walks over rows n of one
+// head: the pair bias stays in registers, and the operands of the next row are on the way while this one is computed.
+// Against a dQ and a dK / dV kernel: scores, exponentials and differences once, the inputs read once (66 us against 103,
+// see the head of the file). Two waves a SIMD is what 230 to 256 registers leave, so that latencies bound it: products and
+// vector instructions take 87,000 of its 135,000 cycles. Pair tiles loaded when they are needed (205 registers, but every
+// wait for them waits for the next row's operands too) 86 us. Wider heads do not fit: dK and dV alone take twice as many.
+template <int D, int NT, bool MASK>
+__global__ __launch_bounds__(64 * NT, 2) void evo_bwd_kernel(EvoParams p, int rows_per) {
+  using T = Tile<D>;
+  using W = Whole<D>;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nt = blockDim.x >> 6;
+  constexpr int Lp = 32 * NT;  // (places in LDS are offsets of the instructions)
+  const int hf = lane >> 5, j = lane & 31, L = p.L;
+  char *sq = smem, *sd = sq + Lp * T::RB, *sk = sd + Lp * T::RB, *ss = sk + Lp * T::RB;
+  float *s_lse = (float*)(ss + Lp * W::SB), *s_delta = s_lse + Lp;
+  int id = xcd_id();
+  const int h = id % p.H;
+  id /= p.H;
+  const int chunks = (p.N + rows_per - 1) / rows_per, b = id / chunks;
+  const int n0 = (id % chunks) * rows_per, n1 = min(p.N, n0 + rows_per);
+  const int k0 = 32 * w, myk = k0 + j, kc = min(myk, L - 1);
+  const bool full = k0 + 32 <= L;
+  const float c = p.rest * kLog2e;
+  const uint32_t ld = p.H * D;
+  const Inverse<D> inv(p.rest);
+  const Diagonal<D> eye(inv);
+  const bf16x8 one = pieces<D>(inv);
+  u32x4 pair[NT][2] = {};
+  if (p.b2 != nullptr) {
+    const bf16* b2 = (const bf16*)p.b2 + (int64_t)(b * p.H + h) * L * L;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      if (t < nt) {
+        const bf16* row = b2 + (int64_t)min(32 * t + j, L - 1) * L;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          const int k = k0 + 16 * ks + 8 * hf;
+          pair[t][ks] = finite(full ? load_eight<false>(row, k, L) : load_eight<true>(row, k, L));
+        }
+      }
+  }
+
+  u32x4 rq[W::PER], rd[W::PER], ro[W::PER], rk[W::PER];
+  bf16x8 rv[T::KS];
+  float rl = INFINITY;  // queries past the end: a probability of zero
+  bf16 rm = (bf16)0.f;
+  auto load = [&](int n) {
+    const int64_t bn = (int64_t)b * p.N + n, base = bn * L * ld + (int64_t)h * D;
+    const int tid = W::tid(), kc = min(k0 + (tid & 31), L - 1);
+    W::load(p.q + base, ld, L, tid, rq);
+    W::load(p.dout + base, ld, L, tid, rd);
+    W::load(p.o + base, ld, L, tid, ro);
+    W::load(p.k + base, ld, L, tid, rk);
+#pragma unroll
+    for (int ks = 0; ks < T::KS; ++ks)
+      rv[ks] = *reinterpret_cast<const bf16x8*>((const char*)(p.v + base) + 2 * (kc * ld + 16 * ks + 8 * ((tid & 63) >> 5)));
+    if (tid < L) rl = (p.lse + (bn * p.H + h) * L)[(uint32_t)tid];
+    if (p.b1 != nullptr) rm = ((const bf16*)p.b1 + bn * L)[(uint32_t)kc];
+  };
+  load(n0);
+
+#pragma unroll 1
+  for (int n = n0; n < n1; ++n) {
+    const int64_t bn = (int64_t)b * p.N + n, base = bn * L * ld + (int64_t)h * D, stat = (bn * p.H + h) * L;
+    if (n > n0) __syncthreads();
+    const int tid = W::tid();
+    W::put(sq, tid, rq);
+    W::put(sd, tid, rd);
+    W::put(sk, tid, rk);
+#pragma unroll
+    for (int i = 0; i < W::PER; ++i) {  // rowsum(dO * O)
+      const bf16x8 a = __builtin_bit_cast(bf16x8, rd[i]), o = __builtin_bit_cast(bf16x8, ro[i]);
+      float delta = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) delta += (float)a[e] * (float)o[e];
+#pragma unroll
+      for (int x = 1; x < W::CH; x *= 2) delta += __shfl_xor(delta, x, 64);
+      if (tid % W::CH == 0) {
+        const int q = W::row(i, tid);
+        s_delta[q] = -delta;
+        if (q < L) (p.delta + stat)[(uint32_t)q] = delta;
+      }
+    }
+    if (tid < Lp) s_lse[tid] = rl / p.rest;
+    bf16x8 vf[T::KS], kf[T::KS];
+#pragma unroll
+    for (int ks = 0; ks < T::KS; ++ks) vf[ks] = rv[ks];
+    const bf16x8 maskf = spread<D>(rm);
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < T::KS; ++ks) kf[ks] = T::rows(sk, k0, ks);
+    times<D>(kf, p.power);
+    if (n + 1 < n1) load(n + 1);
+    f32x16 dk[T::DT], dv[T::DT];
+#pragma unroll
+    for (int dt = 0; dt < T::DT; ++dt) dk[dt] = dv[dt] = f32x16{};
+    float db1 = 0.f;
+
+#pragma unroll
+    for (int u = 0; u < (NT + 1) / 2; ++u) {
+      if (2 * u >= nt) break;
+      if (u > 0) __syncthreads();  // the waves have read dS of the queries before
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        const int t = 2 * u + tt;
+        if (t >= NT || t >= nt) break;
+        __builtin_amdgcn_sched_barrier(0);  // (tile by tile: the scheduler would spill)
+        f32x16 s = mfma(one, maskf, f32x16{}), d;
+#pragma unroll
+        for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(sq, 32 * t, ks), kf[ks], s);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int i = 0; i < Inverse<D>::N; ++i)
+            s = mfma(__builtin_bit_cast(bf16x8, pair[t < NT ? t : 0][ks]), eye.f[i][ks], s);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 de = *reinterpret_cast<const f32x4*>(&s_delta[32 * t + 8 * g + 4 * hf]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) d[4 * g + i] = de[i];
+        }
+#pragma unroll
+        for (int ks = 0; ks < T::KS; ++ks) d = mfma(T::rows(sd, 32 * t, ks), vf[ks], d);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 ls = *reinterpret_cast<const f32x4*>(&s_lse[32 * t + 8 * g + 4 * hf]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int r = 4 * g + i;
+            const float pr = fast_exp2((s[r] - ls[i]) * c);
+            s[r] = pr;
+            d[r] *= pr;
+            if (MASK) db1 += d[r];
+          }
+        }
+        const bf16x8 pb[2] = {acc_to_b<0>(s), acc_to_b<1>(s)};
+        const bf16x8 sb[2] = {acc_to_b<0>(d), acc_to_b<1>(d)};
+#pragma unroll
+        for (int dt = 0; dt < T::DT; ++dt)
+#pragma unroll
+          for (int st = 0; st < 2; ++st) {
+            dv[dt] = mfma(T::cols(sd, 32 * t, st, dt), pb[st], dv[dt]);
+            dk[dt] = mfma(T::cols(sq, 32 * t, st, dt), sb[st], dk[dt]);
+          }
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+          u32x4 x = __builtin_bit_cast(u32x4, sb[st]);
+          if (!full && myk >= L) x = u32x4{0, 0, 0, 0};
+          *reinterpret_cast<u32x2*>(ss + W::ds_off(myk, 4 * tt + 2 * st) + 8 * hf) = u32x2{x[0], x[1]};
+          *reinterpret_cast<u32x2*>(ss + W::ds_off(myk, 4 * tt + 2 * st + 1) + 8 * hf) = u32x2{x[2], x[3]};
+        }
+      }
+      __syncthreads();
+      // lane group g reads keys 4 perm(g) .. + 3 of 16, so that two groups read at once from all banks
+      const int ln = W::tid() & 63, g = ln >> 4, i16 = ln & 15, kq = 4 * (((g & 1) << 1) | (g >> 1)) + (i16 >> 2), pp = i16 & 3;
+      const int pieces16 = min(2, nt - 2 * u) * 2 * (D / 16);
+      for (int x = w; x < pieces16; x += nt) {
+        const int d16 = x % (D / 16), q16 = x / (D / 16);
+        const char* ka = sk + T::off(kq, 2 * d16 + (pp >> 1)) + 8 * (pp & 1);
+        const char* ea = ss + W::ds_off(kq, 2 * q16 + (pp >> 1)) + 8 * (pp & 1);
+        f32x4 acc[2] = {};
+#pragma unroll
+        for (int kb = 0; kb < NT; ++kb) {
+          if (kb >= nt) break;
+          acc[kb & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W::tr_pair(ka + 32 * kb * T::RB, 16 * T::RB),
+                                                                W::tr_pair(ea + 32 * kb * W::SB, 16 * W::SB), acc[kb & 1], 0, 0, 0);
+        }
+        const int q = 64 * u + 16 * q16 + i16;
+        if (q < L) {
+          bf16x4 v;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = (bf16)((acc[0][i] + acc[1][i]) * p.scale);
+          *reinterpret_cast<bf16x4*>((char*)(p.dq + base) + 2 * (q * ld + 16 * d16 + 4 * g)) = v;
+        }
+      }
+    }
+    if (MASK) db1 += __shfl_xor(db1, 32, 64);
+    const int ek = k0 + (W::tid() & 31);
+    if (ek < L) {
+      const uint32_t row = 2 * ek * ld;
+#pragma unroll
+      for (int dt = 0; dt < T::DT; ++dt) {
+        store_row_block<D>((bf16*)((char*)(p.dk + base) + row), dk[dt], dt, hf, p.scale);
+        store_row_block<D>((bf16*)((char*)(p.dv + base) + row), dv[dt], dt, hf, 1.f);
+      }
+      if (MASK && hf == 0) unsafeAtomicAdd(p.db1 + bn * L + myk, db1);
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
 // gradient of the pair bias: sum of dS over the rows
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int kPairTiles = 2;  // of 32 keys: a wave's 32 sums and 32 biases a lane leave room for four waves a SIMD
@@ -596,7 +837,7 @@ __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblo
   using T = Tile<D>;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const int hf = lane >> 5, j = lane & 31, L = p.L;
-  int id = blockIdx.x;
+  int id = xcd_id();
   const int qb = id % qblocks;
   id /= qblocks;
   const int kb = id % kblocks;
@@ -620,7 +861,11 @@ __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblo
     u32x4 pair[kPairTiles][2];
     if constexpr (sizeof(TB) == 2) {
 #pragma unroll
-      for (int t = 0; t < kPairTiles; ++t) bias.template load_pair<TAIL>(kk0 + 32 * t, L, pair[t]);
+      for (int t = 0; t < kPairTiles; ++t) {
+        bias.template load_pair<TAIL>(kk0 + 32 * t, L, pair[t]);
+        pair[t][0] = finite(pair[t][0]);
+        pair[t][1] = finite(pair[t][1]);
+      }
     }
 #pragma unroll 1
     for (int n = n0; n < n1; ++n) {
@@ -771,8 +1016,30 @@ HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, co
   p.b1 = b1; p.b2 = b2; p.dq = (bf16*)dq; p.dk = (bf16*)dk; p.dv = (bf16*)dv; p.lse = (float*)lse; p.delta = delta;
   p.db1 = db1; p.part = part; p.B = B; p.N = N; p.L = L; p.H = H;
   if (!set_scale(p, scale, bias_dtype, D)) return hipErrorInvalidValue;
-  const int nw = waves_of(L, D == 128 ? kWaves<128> : kWaves<32>), blocks = (L + 32 * nw - 1) / (32 * nw);
-  const dim3 grid(blocks * H * B * N), threads(64 * nw);
+  const int nt = (L + 31) / 32;
+  if (bias_dtype == kBF16 && D == 32 && nt <= 8 && (int64_t)L * H * D < (1 << 30)) {  // (offsets in 32 bits)
+    // as many workgroups as the chip holds at once, two waves a SIMD, if there are rows for them
+    const int64_t rows = (int64_t)B * N * H, slots = 256 * (8 / nt);
+    const int per = (int)((rows + slots - 1) / slots);
+    const dim3 grid(B * H * ((N + per - 1) / per)), threads(64 * nt);
+    auto launch = [&](auto tiles, auto mask) {
+      constexpr int NT = decltype(tiles)::value;
+      auto* kernel = evo_bwd_kernel<32, NT, decltype(mask)::value>;
+      static const hipError_t attr = hipFuncSetAttribute(
+          (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, Whole<32>::bytes(NT));
+      if (attr == hipSuccess) hipLaunchKernelGGL(kernel, grid, threads, Whole<32>::bytes(NT), st, p, per);
+      return attr;
+    };
+    auto choose = [&](auto mask) {
+      if (nt <= 2) return launch(std::integral_constant<int, 2>{}, mask);
+      if (nt <= 4) return launch(std::integral_constant<int, 4>{}, mask);
+      return launch(std::integral_constant<int, 8>{}, mask);
+    };
+    const hipError_t e = db1 != nullptr ? choose(std::true_type{}) : choose(std::false_type{});
+    if (e != hipSuccess) return e;
+  } else {
+    const int nw = waves_of(L, D == 128 ? kWaves<128> : kWaves<32>), blocks = (L + 32 * nw - 1) / (32 * nw);
+    const dim3 grid(blocks * H * B * N), threads(64 * nw);
 #define HDS_EVO(DD, TT)                                                                                             \
   do {                                                                                                              \
     hipLaunchKernelGGL((evo_dq_kernel<DD, TT>), grid, threads, 0, st, p, blocks);                                   \
@@ -781,8 +1048,9 @@ HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, co
     else                                                                                                            \
       hipLaunchKernelGGL((evo_dkdv_kernel<DD, TT, false>), grid, threads, 0, st, p, blocks);                        \
   } while (0)
-  HDS_EVO_ALL(HDS_EVO)
+    HDS_EVO_ALL(HDS_EVO)
 #undef HDS_EVO
+  }
   if (db2 != nullptr) {
     const int chunks = hds_evoformer_pair_chunks(B, N, L, H), per = (N + chunks - 1) / chunks;
     const int w4 = waves_of(L, 4), qblocks = (L + 32 * w4 - 1) / (32 * w4);
