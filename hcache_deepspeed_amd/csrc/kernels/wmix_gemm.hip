@@ -230,11 +230,15 @@ __global__ __launch_bounds__(256) void wmix_reduce_kernel(const float* __restric
 // together), and mfma_f32_16x16x32_bf16 contracts elements 8 j .. 8 j + 7 of the four lane groups with the same k of up
 // to 16 MT rows of A. The operand is the weight's CODE, which bf16 holds exactly; the group's scale multiplies the 32-bit
 // sum of each group (every chunk lies in one group), so no weight is rounded. fp6 codes become bf16 in one instruction
-// for 32 of them. Measured at 8 rows, [28672, 4096] / [4096, 14336]: fp6 38 / 22 us (92 / 46 MB; the GEMV that decodes and
-// multiplies on the VALU 112 / 77; 27 us with A resident, below), int8 39 / 20 us (121 / 61 MB; the tile kernel above 45 / 28), int4 29 / 16 us (41 /
-// 29). A third of the time at 8 rows goes to reading A again from L2 in every workgroup.
+// for 32 of them, int8 and int4 in one and a half and two a code (int4, [11264, 2048] gated, 2 rows: 8.0 us with the offset
+// of unsigned nibbles subtracted, 7.1 without). Measured at 8 rows, [28672, 4096] / [4096, 14336]: fp6 38 / 22 us (92 / 46 MB;
+// the GEMV that decodes and multiplies on the VALU 112 / 77), int8 39 / 20 (121 / 61 MB; the tile kernel above 45 / 28), int4
+// 29 / 16 (41 / 29). What is left to it are the sizes that the two kernels below do not gain on.
 typedef uint32_t u32x6 __attribute__((ext_vector_type(6)));
 typedef __bf16 bf16x32 __attribute__((ext_vector_type(32)));
+
+template <int FMT>
+constexpr float kUnit = FMT == kInt4 ? 0.0625f : 1.f;
 
 template <int FMT, int E>
 __device__ __forceinline__ void codes(const WRaw<FMT>& r, bf16x8 (&f)[4]) {
@@ -250,20 +254,18 @@ __device__ __forceinline__ void codes(const WRaw<FMT>& r, bf16x8 (&f)[4]) {
   } else if constexpr (FMT == kInt8) {
     const uint32_t dw[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint32_t u = dw[i] ^ 0x80808080u;  // unsigned bytes, 128 too large
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) f[i >> 1][4 * (i & 1) + t] = (bf16)((float)((u >> (8 * t)) & 0xff) - 128.f);
-    }
+      for (int t = 0; t < 4; ++t) f[i >> 1][4 * (i & 1) + t] = (bf16)(float)(int8_t)(dw[i] >> (8 * t));
   } else {
     const uint32_t dw[4] = {r.a.x, r.a.y, r.a.z, r.a.w};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t lo = (dw[i] & 0x0f0f0f0fu) ^ 0x08080808u, hi = ((dw[i] >> 4) & 0x0f0f0f0fu) ^ 0x08080808u;
+    for (int i = 0; i < 4; ++i) {  // in the upper halves of bytes, with their sign: 16 times the code (kUnit)
+      const uint32_t lo = (dw[i] << 4) & 0xf0f0f0f0u, hi = dw[i] & 0xf0f0f0f0u;
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        f[i][2 * t] = (bf16)((float)((lo >> (8 * t)) & 0xff) - 8.f);
-        f[i][2 * t + 1] = (bf16)((float)((hi >> (8 * t)) & 0xff) - 8.f);
+        f[i][2 * t] = (bf16)(float)(int8_t)(lo >> (8 * t));
+        f[i][2 * t + 1] = (bf16)(float)(int8_t)(hi >> (8 * t));
       }
     }
   }
@@ -365,7 +367,7 @@ __global__ __launch_bounds__(64 * NW, MW) void wmix_skinny_kernel(const bf16* __
 #pragma unroll
           for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[j], x[m][j], s, 0, 0, 0);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[t][m][i] += s[i] * sc[t][i][c];
+          for (int i = 0; i < 4; ++i) acc[t][m][i] += s[i] * (kUnit<FMT> * sc[t][i][c]);
         }
       }
     }
@@ -388,103 +390,199 @@ __global__ __launch_bounds__(64 * NW, MW) void wmix_skinny_kernel(const bf16* __
     }
 }
 
-// The same for fp6 and many weight rows, with A resident. At 8 rows A is more bytes of loads than the packed weights (2
-// against 0.75 a code), and every workgroup above loads all of it: [28672, 4096] 37.4 us, 2.5 TB/s. Here a workgroup of 16
-// waves stays on its CU: A lies in LDS in the order of the products (MP = its rows rounded up to 4, 8 or 16), RW waves
-// share a tile's K in runs of 512, and while a tile's sums are reduced the other waves' next runs are on their way. 2 / 8 /
-// 16 rows: 30.3 / 37.6 / 40.3 -> 25.2 / 26.6 / 28.9 us (3.5 TB/s). int8 and int4 are bound by turning codes into bf16 and
-// gain nothing (8 rows: 38.8 -> 37.8, 27.9 -> 30.2).
-constexpr int kResWaves = 16;
-constexpr int kResTiles = 1024;
+// With whole cache lines: a load above asks for 8 to 16 bytes a lane of 16 weight rows, and for 16-byte pieces of A. Here
+// a wave loads its run of 512 k of 16 rows in 16-byte pieces side by side, which pass through its piece of LDS into the
+// operand's layout (rows 16 bytes apart beyond their length: pieces of 16 rows lie in different banks).
+template <int FMT>
+struct Lines {
+  static constexpr int RB = FMT == kFp6 ? 384 : FMT == kInt8 ? 512 : 256;  // bytes of a run of a row
+  static constexpr int PR = RB / 16, NL = PR / 4;                          // its pieces; loads of a lane
+  static constexpr int ST = RB + 16, WB = 16 * ST;
+  static __device__ __forceinline__ u32x4 piece(const uint8_t* p) {
+    typedef u32x4 __attribute__((aligned(8))) v4;
+    return __builtin_nontemporal_load(reinterpret_cast<const v4*>(p));
+  }
+  static __device__ __forceinline__ int place(int x) { return x / PR * ST + 16 * (x % PR); }
+  // k = 128 c + 32 g .. + 31 of row r
+  static __device__ __forceinline__ WRaw<FMT> raw(const char* wl, int r, int g, int c) {
+    const char* q = wl + r * ST + (RB / 4) * c + (RB / 16) * g;
+    WRaw<FMT> v;
+    if constexpr (FMT == kInt8) {
+      v.a = *reinterpret_cast<const uint4*>(q);
+      v.b = *reinterpret_cast<const uint4*>(q + 16);
+    } else if constexpr (FMT == kInt4) {
+      v.a = *reinterpret_cast<const uint4*>(q);
+    } else {
+      v.a = *reinterpret_cast<const uint2*>(q);
+      v.b = *reinterpret_cast<const uint2*>(q + 8);
+      v.c = *reinterpret_cast<const uint2*>(q + 16);
+    }
+    return v;
+  }
+};
+
+// a row's scales of the four chunks of a run
+__device__ __forceinline__ f32x4 run_scales(const float* s, int run, int K, int G, int groups) {
+  if (G == 128 && groups % 4 == 0) return *reinterpret_cast<const f32x4*>(s + 4 * run);
+  f32x4 v;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) v[c] = s[min(512 * run + 128 * c, K - 128) / G];
+  return v;
+}
+
+// Up to MR (8 or 16) rows: A in the same way, 1 KB of each row a run; the next run's loads are on their way meanwhile.
+template <int FMT, int E, int MR, int NW, bool GLU>
+__global__ __launch_bounds__(64 * NW) void wmix_lines_kernel(const bf16* __restrict__ A, const uint8_t* __restrict__ W,
+                                                             const float* __restrict__ scales,
+                                                             const bf16* __restrict__ bias, bf16* __restrict__ C, int M,
+                                                             int N, int K, int G, int act) {
+  using L = Lines<FMT>;
+  __shared__ __attribute__((aligned(16))) char buf[NW][L::WB + 1024 * MR];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, g = lane >> 4, groups = K / G;
+  const int row_bytes = K / 512 * L::RB + K % 512 * L::RB / 512, runs = (K + 511) / 512;
+  char *wl = buf[wid], *al = wl + L::WB;
+  const uint8_t* wp[L::NL];
+#pragma unroll
+  for (int i = 0; i < L::NL; ++i) wp[i] = W + (int64_t)wmix_row<GLU>(blockIdx.x, (64 * i + lane) / L::PR, N) * row_bytes;
+  const float* sp[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) sp[i] = scales + (int64_t)wmix_row<GLU>(blockIdx.x, 4 * g + i, N) * groups;
+  u32x4 wr[L::NL], ar[MR];
+  f32x4 sn[4];
+  auto load = [&](int run) {
+#pragma unroll
+    for (int i = 0; i < L::NL; ++i)  // (past the row's end: its last piece, unused)
+      wr[i] = L::piece(wp[i] + min(run * L::RB + 16 * ((64 * i + lane) % L::PR), row_bytes - 16));
+    const int k = min(512 * run + 8 * lane, K - 8);
+#pragma unroll
+    for (int m = 0; m < MR; ++m)
+      if (m < M) ar[m] = *reinterpret_cast<const u32x4*>(A + (int64_t)m * K + k);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sn[i] = run_scales(sp[i], run, K, G, groups);
+  };
+  f32x4 acc{};
+  if (wid < runs) load(wid);
+  for (int run = wid; run < runs; run += NW) {
+#pragma unroll
+    for (int i = 0; i < L::NL; ++i) *reinterpret_cast<u32x4*>(wl + L::place(64 * i + lane)) = wr[i];
+#pragma unroll
+    for (int m = 0; m < MR; ++m)
+      if (m < M) *reinterpret_cast<u32x4*>(al + 1024 * m + 16 * (lane ^ m)) = ar[m];
+    f32x4 sc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sc[i] = sn[i];
+    if (run + NW < runs) load(run + NW);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      if (512 * run + 128 * c >= K) break;  // wave-uniform
+      bf16x8 x[4], f[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        x[j] = *reinterpret_cast<const bf16x8*>(al + 1024 * (r & (MR - 1)) + 16 * ((16 * c + 4 * g + j) ^ (r & (MR - 1))));
+      codes<FMT, E>(L::raw(wl, r, g, c), f);
+      f32x4 s{};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[j], x[j], s, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] += s[i] * (kUnit<FMT> * sc[i][c]);
+    }
+  }
+  reinterpret_cast<f32x4*>(wl)[lane] = acc;
+  __syncthreads();
+  if (wid > 0) return;
+#pragma unroll
+  for (int v = 1; v < NW; ++v) acc += reinterpret_cast<const f32x4*>(buf[v])[lane];
+  wmix_store<GLU>(acc, blockIdx.x, r, g, lane, bias, C, M, N, act);
+}
+
+// Many weight rows of up to 4,096 k: workgroups that stay on their CU. Wave w of RW holds run w of A in registers, in the
+// operands' layout, and walks over the workgroup's tiles; it loads whole lines as above, two tiles ahead.
+constexpr int kResWaves = 8;
 
 template <int FMT, int E, int RW, bool GLU>
-__global__ __launch_bounds__(64 * kResWaves) void wmix_resident_kernel(const bf16* __restrict__ A,
-                                                                       const uint8_t* __restrict__ W,
-                                                                       const float* __restrict__ scales,
-                                                                       const bf16* __restrict__ bias,
-                                                                       bf16* __restrict__ C, int M, int N, int K, int G,
-                                                                       int act, int tiles, int MP) {
-  extern __shared__ __attribute__((aligned(16))) char sm[];  // A: K * MP * 2, sums: [2][waves][64] of 16 bytes
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+__global__ __launch_bounds__(64 * kResWaves, 2) void wmix_resident_kernel(const bf16* __restrict__ A,
+                                                                          const uint8_t* __restrict__ W,
+                                                                          const float* __restrict__ scales,
+                                                                          const bf16* __restrict__ bias,
+                                                                          bf16* __restrict__ C, int M, int N, int K, int G,
+                                                                          int act, int tiles) {
   constexpr int TG = kResWaves / RW;
-  const int tg = wid / RW, w = wid % RW;
-  const int runs = (K + 511) / 512, groups = K / G;
-  f32x4* red = reinterpret_cast<f32x4*>(sm + (int64_t)K * MP * 2);
-  const int t0 = blockIdx.x * TG, dt = gridDim.x * TG;
-  const int rounds = (tiles - t0 + dt - 1) / dt;  // the same for all waves: every round has one barrier
-  WRaw<FMT> raw[4];
-  f32x4 sc[4];
-  int lt = t0 + tg, lrun = w;  // the wave's next run to load
-  auto load = [&]() {
-    if (lt >= tiles || lrun >= runs) return;
+  using L = Lines<FMT>;
+  __shared__ __attribute__((aligned(16))) char buf[kResWaves][L::WB];
+  __shared__ f32x4 red[2][4][kResWaves][64];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, g = lane >> 4, groups = K / G;
+  const int row_bytes = K / 512 * L::RB + K % 512 * L::RB / 512;
+  const int tg = wid / RW, w = wid % RW, t0 = blockIdx.x * TG + tg, dt = gridDim.x * TG;
+  const int rounds = (tiles - (int)blockIdx.x * TG + dt - 1) / dt;  // the same for all waves: every round has one barrier
+  const bool on = 512 * w < K;
+  const int wr = on ? w : 0;
+  char* wl = buf[wid];
+  struct Run {
+    u32x4 wr[L::NL];
+    f32x4 sc[4];
+  } ahead;
+  // Unconditional: past the end a tile that has just been read. Behind a branch the compiler, which counts loads that are
+  // on their way, would have every run wait for the one after it
+  auto load = [&](int t, Run& n) {
+    t = min(t, tiles - 1);
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      raw[c] = load_w<FMT>(W, wmix_row<GLU>(lt, r, N), K, min(512 * lrun + 128 * c, K - 128) + 32 * g);
+    for (int i = 0; i < L::NL; ++i) {
+      const int x = 64 * i + lane;  // (past the row's end: its last piece, unused)
+      n.wr[i] = L::piece(W + (int64_t)wmix_row<GLU>(t, x / L::PR, N) * row_bytes +
+                         min(wr * L::RB + 16 * (x % L::PR), row_bytes - 16));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      n.sc[i] = run_scales(scales + (int64_t)wmix_row<GLU>(t, 4 * g + i, N) * groups, wr, K, G, groups);
+  };
+  load(t0, ahead);
+  bf16x8 x[4][4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      x[c][j] = *reinterpret_cast<const bf16x8*>(A + (int64_t)min(r, M - 1) * K + min(512 * w + 128 * c, K - 128) + 32 * g + 8 * j);
+  auto step = [&](int round, f32x4 (*rb)[64], Run& cur) {
+    const int t = t0 + round * dt;
+    f32x4 acc{};
+#pragma unroll
+    for (int i = 0; i < L::NL; ++i) *reinterpret_cast<u32x4*>(wl + L::place(64 * i + lane)) = cur.wr[i];
+    f32x4 sc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sc[i] = cur.sc[i];
+    load(t + dt, cur);
+    __builtin_amdgcn_sched_barrier(0);
+    if (t < tiles && on) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if (512 * w + 128 * c >= K) break;  // wave-uniform
+        bf16x8 f[4];
+        codes<FMT, E>(L::raw(wl, r, g, c), f);
+        f32x4 s{};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[j], x[c][j], s, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] += s[i] * (kUnit<FMT> * sc[i][c]);
+      }
+    }
+    rb[wid][lane] = acc;
+  };
+  for (int round = 0; round < rounds; round += 4) {
+    auto* rb = red[round >> 2 & 1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) step(round + i, rb[i], ahead);
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float* s = scales + (int64_t)wmix_row<GLU>(lt, 4 * g + i, N) * groups;
-      if (G == 128 && groups % 4 == 0) {
-        sc[i] = *reinterpret_cast<const f32x4*>(s + 4 * lrun);
-      } else {
+      const int t = t0 + (round + i) * dt;
+      if (t >= tiles || w != i) continue;
+      f32x4 s = rb[i][tg * RW][lane];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) sc[i][c] = s[min(512 * lrun + 128 * c, K - 128) / G];
-      }
-    }
-    lrun += RW;
-    if (lrun >= runs) {
-      lrun = w;
-      lt += dt;
-    }
-  };
-  load();
-  // piece p of A: row p % MP, 8 columns of lane group (p / MP) % 4 for product (p / 4 MP) % 4 of 128-chunk p / 16 MP
-  for (int i = wid; i < K * MP / 512; i += kResWaves) {
-    const int p = 64 * i + lane, k = 128 * (p / (16 * MP)) + 32 * ((p / MP) & 3) + 8 * ((p / (4 * MP)) & 3);
-    __builtin_amdgcn_global_load_lds(
-        (const __attribute__((address_space(1))) void*)(A + (int64_t)min(p % MP, M - 1) * K + k),
-        (__attribute__((address_space(3))) void*)(sm + i * 1024), 16, 0, 0);
-  }
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-  __syncthreads();
-  const char* xs = sm + (g * MP + (r & (MP - 1))) * 16;
-  for (int round = 0, t = t0 + tg; round < rounds; ++round, t += dt) {
-    f32x4 acc{};
-    if (t < tiles) {
-      for (int run = w; run < runs; run += RW) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          if (512 * run + 128 * c >= K) break;  // wave-uniform
-          bf16x8 f[4];
-          codes<FMT, E>(raw[c], f);
-          f32x4 s{};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const bf16x8 x = *reinterpret_cast<const bf16x8*>(xs + (16 * (4 * run + c) + 4 * j) * MP * 16);
-            s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[j], x, s, 0, 0, 0);
-          }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc[i] += s[i] * sc[i][c];
-        }
-        load();
-      }
-    }
-    f32x4* rb = red + (round & 1) * kResWaves * 64;
-    rb[wid * 64 + lane] = acc;
-    __syncthreads();
-    if (t < tiles && w == round % RW) {
-      f32x4 s = rb[tg * RW * 64 + lane];
-#pragma unroll
-      for (int v = 1; v < RW; ++v) s += rb[(tg * RW + v) * 64 + lane];
+      for (int v = 1; v < RW; ++v) s += rb[i][tg * RW + v][lane];
       wmix_store<GLU>(s, t, r, g, lane, bias, C, M, N, act);
     }
   }
-}
-
-// rows of A the resident kernel makes room for, and its LDS (0: it does not take the size)
-int resident_rows(int M) { return M <= 4 ? 4 : (M <= 8 ? 8 : 16); }
-size_t resident_bytes(int M, int K) {
-  const size_t b = (size_t)K * resident_rows(M) * 2 + 2 * kResWaves * 1024;
-  return M <= 16 && b <= 160 * 1024 ? b : 0;
 }
 
 int pick_mb(int M) { return M <= 32 ? 1 : 2; }
@@ -547,8 +645,16 @@ HDS_EXPORT int hds_wmix_gemm(const void* A, const void* W, const float* scales, 
   return hipGetLastError();
 }
 
-// The same product for few rows as a stream of packed weights (wmix_skinny_kernel, wmix_resident_kernel): 1 <= M <= 16, fp6
-// up to 32. K and G multiples of 128, A 16-byte aligned. glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu) for
+// Does wmix_resident_kernel take M rows by [N, K] (N: weight rows, gate and up rows together)? From four tiles a CU on: the
+// barriers and a last round that is not full cost more than what is saved below (8 rows, fp6 [11264, 2048] gated 10.8 us
+// against 10.1, [12288, 4096] 16.3 with A resident in LDS against 15.5 of whole lines). With up to 2,048 k two tiles are at
+// work at a time.
+HDS_EXPORT int hds_wmix_resident(int M, int N, int K) {
+  return M <= 16 && K <= 4096 && (N + 15) / 16 >= (K > 2048 ? 1024 : 2048);
+}
+
+// The same product for few rows as a stream of packed weights (wmix_skinny_kernel, wmix_lines_kernel,
+// wmix_resident_kernel): 1 <= M <= 16, fp6 up to 32. K and G multiples of 128, A 16-byte aligned. glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu) for
 // W = [gate; up] of 2 N rows (M <= 16, no bias).
 HDS_EXPORT int hds_wmix_skinny(const void* A, const void* W, const float* scales, const void* bias, void* C, int M, int N,
                                int K, int G, int fmt, int ebits, int glu, hipStream_t st) {
@@ -563,26 +669,27 @@ HDS_EXPORT int hds_wmix_skinny(const void* A, const void* W, const float* scales
   };
   auto resident = [&](auto kern, int rw) {
     const int wg = (tiles + kResWaves / rw - 1) / (kResWaves / rw);
-    const size_t lds = resident_bytes(M, K);
-    const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(wg < 256 ? wg : 256), dim3(64 * kResWaves), lds, st, (const bf16*)A, (const uint8_t*)W,
-                       scales, (const bf16*)bias, (bf16*)C, M, N, K, G, glu - 1, tiles, resident_rows(M));
+    hipLaunchKernelGGL(kern, dim3(wg < 256 ? wg : 256), dim3(64 * kResWaves), 0, st, (const bf16*)A, (const uint8_t*)W,
+                       scales, (const bf16*)bias, (bf16*)C, M, N, K, G, glu - 1, tiles);
     return hipGetLastError();
   };
-  // A resident from four tiles a CU on, where it fits: [16384, 4096], 8 rows 20.8 -> 16.8 us, [32768, 2048] 21.2 -> 15.8,
-  // [27648, 5120] 53 -> 33, [16384, 7168] 37.5 -> 25.6; at [12288, 4096] 2 / 8 / 16 rows 13.8 / 16.2 / 21.0 -> 15.0 / 16.3
-  // / 18.5, at [8192, 4096] level: the last round of tiles and the way of A into LDS.
-  const bool res = fmt == 2 && resident_bytes(M, K) != 0 && tiles >= kResTiles;
+  const bool res = hds_wmix_resident(M, glu ? 2 * N : N, K);
+  // Whole lines pay where a wave walks far: 8 rows, fp6 [2048, 2048] 4.8 us against 4.9, [11264, 2048] gated 10.3 / 10.1; int8
+  // [4096, 4096] 8.7 / 8.6, [6144, 4096] 12.1 / 12.5, [2048, 5632] 8.2 / 8.7; int4 [4096, 4096] 6.5 / 6.2, [2048, 5632] 7.3 / 7.1,
+  // [4096, 14336] 14.3 / 15.7. From nine rows on the wider codes lose (int8 [4096, 14336], 16 rows, 24.7 / 23.8) and fp6 gains
+  // where a CU's one workgroup is not followed by another or is long ([6144, 4096] 14.8 / 14.6, [5120, 13824] 37.9 / 47.2).
+  const bool lines = K > (fmt == 2 ? 2048 : fmt == 0 ? 4096 : 8192);
   // From nine rows on two tiles of weight rows share what is read of A ([28672, 4096], 16 rows: fp6 48 -> 41 us), where
   // enough workgroups remain. Short sums on many rows: four waves a workgroup, otherwise eight ([4096, 14336] fp6, 8 rows 27
   // -> 22 us).
 #define HDS_WS(F, E, GL)                                                                                            \
   do {                                                                                                              \
-    if constexpr (F == kFp6) {                                                                                      \
-      if (res && (K + 511) / 512 % 8 == 0) return resident(wmix_resident_kernel<F, E, 8, GL>, 8);                   \
-      if (res) return resident(wmix_resident_kernel<F, E, 4, GL>, 4);                                               \
-    }                                                                                                               \
+    if (res && K > 2048) return resident(wmix_resident_kernel<F, E, 8, GL>, 8);                                     \
+    if (res) return resident(wmix_resident_kernel<F, E, 4, GL>, 4);                                                 \
+    if (lines && M <= 8 && tiles > 256) return launch(wmix_lines_kernel<F, E, 8, 4, GL>, 1, 4);                     \
+    if (lines && M <= 8) return launch(wmix_lines_kernel<F, E, 8, 8, GL>, 1, 8);                                    \
+    if constexpr (F == kFp6)                                                                                        \
+      if (lines && M <= 16 && (K > 4096 || tiles <= 256)) return launch(wmix_lines_kernel<F, E, 16, 6, GL>, 1, 6);  \
     if (M > 8 && M <= 16 && tiles >= 2 * 512) return launch(wmix_skinny_kernel<F, E, 2, 1, 4, 3, GL>, 2, 4);        \
     if (M <= 16 && K <= 4096 && tiles >= 384) return launch(wmix_skinny_kernel<F, E, 1, 1, 4, 1, GL>, 1, 4);        \
     if (M <= 16) return launch(wmix_skinny_kernel<F, E, 1, 1, 8, 1, GL>, 1, 8);                                     \

@@ -175,11 +175,12 @@ def _gemv_wins(M, out_features, in_features, fmt):
     stream? us, GEMV / stream. int4, one row: up to 100M weights, 48M of long rows ([6144, 4096] 7.2 / 9.4, [8192, 8192] 14.7 / 16.8;
     [4096, 14336] 17.3 / 15.6, [28672, 4096] 30.2 / 26.7). int8, two rows: where the last round of 256 tiles of 16 weight rows leaves
     the chip idle ([1024, 1024] 3.3 / 3.9, [6144, 4096] 11.3 / 12.7, [4096, 4096] 8.2 / 7.9, [11264, 2048] 11.0 / 9.4). int4, two
-    rows, and fp6, one: small weights ([1024, 1024] 3.4 / 4.0 and 3.5 / 3.6, [3072, 2048] 5.3 / 4.8 and 6.4 / 4.7)."""
+    rows, and fp6, one: small weights ([1024, 1024] 3.4 / 4.0 and 3.5 / 3.6, [3072, 2048] 5.3 / 4.8 and 6.4 / 4.7). Not where the
+    stream's rows stay resident (one row, int8 [28672, 4096] 34.1 / 27.4, [32768, 2048] 19.5 / 17.0, int4 [16384, 4096] 17.8 / 12.9)."""
     weights, tiles = out_features * in_features, (out_features + 15) // 16
     if fmt == "fp6":
         return M == 1 and weights < 4_000_000
-    if M > _INT_GEMV_MAX_M:
+    if M > _INT_GEMV_MAX_M or native.kernels().hds_wmix_resident(M, out_features, in_features):
         return False
     if fmt == "int8":
         return M == 1 or M == 2 and tiles / ((tiles + 255) // 256 * 256) < 0.8
@@ -190,11 +191,14 @@ def _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, fm
     """The packed-weight stream for few rows (csrc/kernels/wmix_gemm.hip ``wmix_skinny_kernel``), or None where it does not
     apply (rows of whole groups of a multiple of 128; fp6 as e3m2 or e2m3). It wins up to 16 rows, with fp6 up to 32
     ([28672, 4096], 24 rows: fp6 57 us against the tile kernel's 78, int8 61 against 50; fp6 at 32 rows 87 against 78, but the
-    tile kernel rounds the weights), with int8 from the second row on (one row: 36.5 us against the GEMV's 34.7)."""
+    tile kernel rounds the weights), one row of int8 only where the stream's rows stay resident (see ``_gemv_wins``)."""
     M = x2.shape[0]
     if (_needs_grad(x2) or not native.use_native(x2) or x2.dtype != torch.bfloat16 or in_features % 128
             or group_size % 128 or in_features % group_size or (fmt == "fp6" and ebits not in (2, 3))
-            or not (fmt == "int8") < M <= (32 if fmt == "fp6" and not glu else 16)):
+            or not 0 < M <= (32 if fmt == "fp6" and not glu else 16)):
+        return None
+    if fmt == "int8" and M == 1 and (bias is not None or not native.kernels().hds_wmix_resident(
+            M, out_features * (2 if glu else 1), in_features)):
         return None
     if bias is None and not glu and _gemv_wins(M, out_features, in_features, fmt):
         return None  # (with a bias, which the GEMVs' results would get after their rounding, the stream)

@@ -87,6 +87,31 @@ def test_few_rows_keep_the_weights_exact(fmt, M, N, K, G):
     assert ((y.double() - ref).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("fmt,M,N,K", [
+    ("fp6_e3m2", 1, 4090, 2176), ("fp6_e2m3", 8, 4200, 4224), ("fp6_e3m2", 9, 4000, 2176), ("fp6_e3m2", 16, 5000, 4352),
+    ("int8", 3, 4096, 4224), ("int8", 8, 4112, 4608), ("int4", 1, 4096, 14336), ("int4", 7, 5000, 8320), ("int8", 1, 16400, 2176),
+    ("int8", 16, 20500, 4096), ("int4", 16, 32790, 1920), ("fp6_e3m2", 5, 16390, 2176), ("int4", 2, 16384, 3200)])
+def test_whole_lines_of_packed_weights(fmt, M, N, K):
+    """The kernels that load whole lines, to the stream's bound: walks that end inside a run of 512 or leave waves without one,
+    four, six and eight waves, partial tiles, one to three rounds of resident rows; packed weights 8 bytes off a line."""
+    torch.manual_seed(K + M)
+    x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
+    w = torch.randn(N, K, device="cuda", dtype=torch.bfloat16) * 0.05
+    off = lambda q: torch.cat([q.new_zeros(8), q.reshape(-1)])[8:]  # noqa: E731
+    if fmt.startswith("int"):
+        bits = int(fmt[3:])
+        q, s, _ = Q.quantize(w.reshape(-1), 128, bits, True)
+        wd = Q.dequantize(q, s, None, 128, bits, True, torch.float32).view(N, K).double()
+        y = Q.int_linear(x, off(q), s, N, K, 128, bits=bits)
+    else:
+        mb = 2 if fmt.endswith("e3m2") else 3
+        q, s = Q.quantize_minifloat(w.reshape(-1), 128, 6, mb)
+        wd = Q.dequantize_minifloat(q, s, 128, 6, mb, torch.float32).view(N, K).double()
+        y = Q.fp6_linear(x, off(q), s, N, K, 128, mb)
+    ref = x.double() @ wd.t()
+    assert ((y.double() - ref).abs() <= 2**-8 * ref.abs() + 1e-5 * (x.double().abs() @ wd.abs().t())).all()
+
+
 @pytest.mark.parametrize("fmt,M,N,K,gemv", [
     ("int4", 1, 1024, 1024, True), ("int4", 1, 4096, 11648, True), ("int4", 1, 4096, 11776, False), ("int4", 1, 12200, 8192, True),
     ("int4", 1, 12224, 8192, False), ("int4", 2, 3900, 1024, True), ("int4", 2, 3920, 1024, False), ("int8", 2, 1000, 640, True),
@@ -196,3 +221,9 @@ def test_int_linear_with_a_32_bit_bias(bits, M):
     assert Q.int_linear(x, q, s, N, K, G, bits=bits, bias=narrow).requires_grad == (M <= 2)
     ref = x.double() @ Q.dequantize(q, s, None, G, bits, True, torch.float32).view(N, K).double().t()
     assert ((y.double() - (ref + b.double())).abs() <= 2**-8 * (ref.abs() + b.abs() + x.double().abs() @ w.double().abs().t())).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8200, 4096), (4, 8190, 2304), (16, 16400, 1920)])
+def test_gated_projection_of_resident_rows(M, N, K):
+    """One row of int8 in the gated kernel, waves without a run, two tiles at work at a time."""
+    test_gated_projection_of_packed_weights("int8", "silu", M, N, K, 128)
