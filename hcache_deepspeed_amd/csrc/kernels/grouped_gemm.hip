@@ -21,6 +21,8 @@
 //     wave then holds the accumulators of the same features of both halves; a tile list made elsewhere (experts.hip);
 //   * blockIdx.x walks N tiles fastest so the (consecutively dispatched, XCD-round-robin) blocks of one
 //     token tile share the X tile in L2 while W[e] streams.
+#include <algorithm>
+
 #include "attn_common.h"
 
 using namespace hds;
@@ -302,100 +304,117 @@ __global__ __launch_bounds__(512) void gg_big_kernel(const bf16* __restrict__ x,
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Many experts with few rows each (serving): bound by the stream of weights, of which an expert's share should be read
-// once and be on its way all the time. Tile: all rows of an expert up to 256 (64 NX of them are loaded and multiplied) x 128
-// weight rows, BK = 64, 8 waves. Three LDS buffers of 48 KB: a stage is waited for with a count while the next one is in
-// flight and the one after is issued, one barrier a stage. Waves: 2 along the weight rows x 4 along the tokens, a wave's
-// token blocks are mg and mg + 4 of 32. Each XCD takes a contiguous range of the real tiles (expert after expert), so
-// that the workgroups of one expert share its rows in one L2.
-// A layer of 64 experts, 6 a token, 1024 x 2048, 250 / 1,000 / 1,500 tokens: 206 / 245 / 374 us with the 128 x 128 tiles
-// above -> 196 / 235 / 264 (805 MB of weights); 64 experts, 4 a token, 2048 x 4096, 65 / 1,500 tokens: 706 / 829 -> 574 /
-// 700; 8 experts, 2 a token, 14336 x 4096, 65 / 500: 597 / 871 -> 509 / 659. The products
-// alone at 1,600 tokens of the first: gate and up 229 -> 158 us (537 MB), down 129 -> 85 (268 MB).
+// Many experts with few rows each (serving). Neither the weights from memory, nor the rows from L2, nor the products alone
+// take the time (146 us; 131, 144 and 133 without one of them): what bounds it is how many cache lines a CU can have on the
+// way, at about 20 bytes a cycle. So the tile is as large as the rounds over the CUs allow: all rows of an expert up to 256
+// (64 NX of them are loaded and multiplied) x WR = 256, 128 or 64 weight rows. LDS is a ring of 20 chunks of 64 rows x 64 k: a
+// step multiplies the chunks of 64 k, whose places are refilled one step later, so that R - 2 C to R - C chunks are on their
+// way at any time, waited for with a count, one barrier a step. (Twelve or sixteen chunks are level, and so are fragments read
+// a step ahead.) Waves: WR / 64 along the weight rows, the others along the tokens. Each XCD takes a contiguous range of the
+// real tiles (expert after expert), so that the workgroups of one expert share its rows in one L2.
+// 128 weight rows and three stages of 48 KB -> this, gate and up / down, us: 64 experts, 6 a token, 1024 x 2048, 66 / 700 / 1,600
+// / 3,000 tokens 121 + 44 / 126 + 71 / 153 + 95 / 265 + 147 -> 96 + 44 / 104 + 63 / 132 + 89 / 254 + 142; 64 experts, 4 a token, 2048
+// x 4096, 66 / 1,500 tokens 361 + 174 / 480 + 244 -> 349 + 176 / 430 + 220; 8 experts, 2 a token, 14336 x 4096, 66 / 500 / 1,700
+// tokens 322 + 163 / 463 + 222 / 1,125 + 538 -> 321 + 159 / 463 + 230 / 1,035 + 502; 5632 x 2048, 66 / 500 / 1,400 tokens 87 + 37 /
+// 108 + 76 / 243 + 102 -> 73 + 42 / 110 + 61 / 204 + 101.
 // ---------------------------------------------------------------------------------------------------------------
-constexpr int kFlowStage = 128 * 128 + 256 * 128;
+constexpr int kChunk = 64 * 128, kRing = 20;
+// operand of s_waitcnt: no LDS access and at most n loads on their way
+constexpr int flow_wait(int n) { return 0x70 | (n & 15) | n >> 4 << 14; }
 
-template <int NX, bool GLU>
-__device__ __forceinline__ void gg_flow_tile(char* smem, const bf16* const (&wp)[2], const bf16* const (&xp)[4], int KT,
-                                             f32x16 (&acc)[2][2]) {
-  constexpr int P = 2 + NX, NJ = NX > 2 ? 2 : 1;  // a wave's loads a stage; its token blocks
-  const int w = threadIdx.x >> 6, p = w & 1, mg = w >> 1;
-  auto issue = [&](char* s, int kt) {
-    const int64_t k0 = (int64_t)kt * BK2;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      __builtin_amdgcn_global_load_lds((gbl_void*)(wp[i] + k0), (lds_void*)(s + (2 * w + i) * 1024), 16, 0, 0);
-#pragma unroll
-    for (int i = 0; i < NX; ++i)
-      __builtin_amdgcn_global_load_lds((gbl_void*)(xp[i] + k0), (lds_void*)(s + 16384 + (8 * i + w) * 1024), 16, 0, 0);
+template <int NX, int WR, bool GLU>
+__device__ __forceinline__ void gg_flow_tile(char* smem, const bf16* const (&wp)[WR / 64], const bf16* const (&xp)[4], int KT,
+                                             int turn, f32x16 (&acc)[2][WR / 64]) {
+  constexpr int CW = WR / 64, C = CW + NX, TG = 8 / CW, NB = (2 * NX + TG - 1) / TG;
+  constexpr int R = kRing;
+  const int w = threadIdx.x >> 6, wq = w % CW, tg = w / CW;  // wave-uniform
+  auto issue = [&](int s, int i, int place) {  // chunk i of step s
+    s += turn;
+    const int64_t k0 = (int64_t)(s < KT ? s : s - KT) * BK2;
+    const bf16* src = i < CW ? wp[i < CW ? i : 0] : xp[i < CW ? 0 : i - CW];
+    __builtin_amdgcn_global_load_lds((gbl_void*)(src + k0), (lds_void*)(smem + place * kChunk + w * 1024), 16, 0, 0);
   };
-  char *cur = smem, *next = smem + kFlowStage, *last = smem + 2 * kFlowStage;
-  issue(cur, 0);
-  issue(next, 1);  // KT >= 2
+  auto wrap = [](int p) { return p < R ? p : p - R; };
+#pragma unroll
+  for (int c = 0; c < R - C; ++c)
+    if (c < C * KT) issue(c / C, c % C, c);
+  int base = 0;  // place of the step's first chunk
   for (int kt = 0; kt < KT; ++kt) {
-    // this stage has arrived for every wave, and every wave is done with the one before: its reads have returned (lgkmcnt;
-    // the compiler may move the products that use them behind this statement), so that the stage after next may
-    // overwrite it
-    if (kt + 1 < KT) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(P) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (kt + 2 < KT) issue(last, kt + 2);
-    const char* Xt = cur + 16384;
-    if (mg < 2 * NX) {  // wave-uniform
-      bf16x8 a0[4], a1[4], b[4];  // all of a stage's reads on their way
+    // this step's chunks have arrived for every wave, and every wave is done with the last step's (its reads have returned)
+    if (C * (kt - 1) + R <= C * KT) __builtin_amdgcn_s_waitcnt(flow_wait(R - 2 * C));
+    else __builtin_amdgcn_s_waitcnt(flow_wait(0));
+    asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+      constexpr int first = R - C;
+      const int s = kt + (first + u) / C;
+      if (s < KT) issue(s, (first + u) % C, wrap(base + first + u));
+    }
+    const char *a0p, *a1p;
+    if constexpr (GLU) {
+      a0p = smem + wrap(base + (wq >> 1)) * kChunk + (wq & 1) * 4096;
+      a1p = CW == 1 ? a0p + 4096 : smem + wrap(base + CW / 2 + (wq >> 1)) * kChunk + (wq & 1) * 4096;
+    } else {
+      a0p = smem + wrap(base + wq) * kChunk;
+      a1p = a0p + 4096;
+    }
+    // all reads of the step on their way ahead of its products (waited for k by k: 516 us instead of 463 at 8 experts of
+    // 14336 x 4096 and 500 tokens)
+    constexpr bool some = 2 * NX % TG != 0;  // the last block is not every wave's
+    const bool last = !some || tg + TG * (NB - 1) < 2 * NX;  // wave-uniform
+    bf16x8 a0[4], a1[4], b[NB][4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      a0[ks] = frag128(a0p, 0, ks);
+      a1[ks] = frag128(a1p, 0, ks);
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int blk = min(tg + TG * j, 2 * NX - 1);
+      const char* bp = smem + wrap(base + CW + (blk >> 1)) * kChunk + (blk & 1) * 4096;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) b[j][ks] = frag128(bp, 0, ks);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      if (some && j == NB - 1 && !last) break;
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
-        a0[ks] = frag128(cur, GLU ? 32 * p : 64 * p, ks);
-        a1[ks] = frag128(cur, GLU ? 64 + 32 * p : 64 * p + 32, ks);
-        b[ks] = frag128(Xt, 32 * mg, ks);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        acc[0][0] = mfma(a0[ks], b[ks], acc[0][0]);
-        acc[1][0] = mfma(a1[ks], b[ks], acc[1][0]);
-      }
-      if (NJ > 1 && mg + 4 < 2 * NX) {
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) b[ks] = frag128(Xt, 32 * (mg + 4), ks);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          acc[0][1] = mfma(a0[ks], b[ks], acc[0][1]);
-          acc[1][1] = mfma(a1[ks], b[ks], acc[1][1]);
-        }
+        acc[0][j] = mfma(a0[ks], b[j][ks], acc[0][j]);
+        acc[1][j] = mfma(a1[ks], b[j][ks], acc[1][j]);
       }
     }
-    char* t = cur;
-    cur = next;
-    next = last;
-    last = t;
+    base = wrap(base + C);
   }
 }
 
-template <bool GATHER, bool GLU>
+template <bool GATHER, bool GLU, int WR>
 __global__ __launch_bounds__(512) void gg_flow_kernel(const bf16* __restrict__ x, int64_t ldx,
                                                       const int* __restrict__ src, int n_src,
                                                       const bf16* __restrict__ w, bf16* __restrict__ y,
                                                       const int* __restrict__ offs, const int* __restrict__ tile_e,
                                                       const int* __restrict__ tile_m, const int* __restrict__ n_tiles,
-                                                      int T, int N, int K, int ldy, int ntn, GatedUnit unit) {
-  __shared__ __attribute__((aligned(1024))) char smem[3 * kFlowStage];
+                                                      int T, int N, int K, int ldy, int ntn, GatedUnit unit, int apart) {
+  constexpr int CW = WR / 64, TG = 8 / CW;
+  __shared__ __attribute__((aligned(1024))) char smem[kRing * kChunk];
   const int nwg = *n_tiles * ntn, orig = blockIdx.x;
   if (orig >= nwg) return;  // block-uniform exit before any barrier
   const int q = nwg / 8, r = nwg % 8, xcd = orig % 8;
   const int id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + orig / 8;
-  const int t = id / ntn, n0 = (id % ntn) * (GLU ? 64 : 128);
+  const int t = id / ntn, n0 = (id % ntn) * (GLU ? WR / 2 : WR);
   const int e = tile_e[t], m0 = tile_m[t];
   const int row0 = min(max(offs[e], 0), T);
   const int rows = min(max(offs[e + 1], row0), T) - row0;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   // LDS-DMA sources: lane l fills 16 bytes of row l >> 3 of a group of 8, the piece that off128 keeps there
-  const bf16* wp[2];
+  const bf16* wp[CW];
   const bf16* xp[4];
   const bf16* wb = w + (int64_t)e * (GLU ? 2 : 1) * N * K + (int64_t)n0 * K;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int row = 8 * (2 * wv + i) + (lane >> 3);
-    wp[i] = wb + ((int64_t)row + (GLU && row >= 64 ? N - 64 : 0)) * K + 8 * ((lane & 7) ^ ((row >> 1) & 7));
+  for (int i = 0; i < CW; ++i) {
+    const int row = 64 * i + 8 * wv + (lane >> 3);
+    wp[i] = wb + ((int64_t)row + (GLU && row >= WR / 2 ? N - WR / 2 : 0)) * K + 8 * ((lane & 7) ^ ((row >> 1) & 7));
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -404,22 +423,23 @@ __global__ __launch_bounds__(512) void gg_flow_kernel(const bf16* __restrict__ x
     if constexpr (GATHER) at = min(max(src[row0 + m], 0), n_src - 1);
     xp[i] = x + at * ldx + 8 * ((lane & 7) ^ ((row >> 1) & 7));
   }
-  f32x16 acc[2][2];
+  f32x16 acc[2][CW];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x16{};
+    for (int j = 0; j < CW; ++j) acc[i][j] = f32x16{};
   const int nx = (min(rows - m0, BM2) + 63) / 64, KT = K / BK2;
-  if (nx <= 1) gg_flow_tile<1, GLU>(smem, wp, xp, KT, acc);
-  else if (nx == 2) gg_flow_tile<2, GLU>(smem, wp, xp, KT, acc);
-  else if (nx == 3) gg_flow_tile<3, GLU>(smem, wp, xp, KT, acc);
-  else gg_flow_tile<4, GLU>(smem, wp, xp, KT, acc);
+  const int turn = apart ? (int)__umulhi(blockIdx.x * 2654435769u, (unsigned)KT) : 0;
+  if (nx <= 1) gg_flow_tile<1, WR, GLU>(smem, wp, xp, KT, turn, acc);
+  else if (nx == 2) gg_flow_tile<2, WR, GLU>(smem, wp, xp, KT, turn, acc);
+  else if (nx == 3) gg_flow_tile<3, WR, GLU>(smem, wp, xp, KT, turn, acc);
+  else gg_flow_tile<4, WR, GLU>(smem, wp, xp, KT, turn, acc);
 
   // lane = token, registers 4g .. 4g + 3 = 4 consecutive output features
-  const int h = lane >> 5, p = wv & 1, mg = wv >> 1;
+  const int h = lane >> 5, p = wv % CW, tg = wv / CW;
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int m = m0 + 32 * (mg + 4 * j) + (lane & 31);
+  for (int j = 0; j < CW; ++j) {
+    const int m = m0 + 32 * (tg + TG * j) + (lane & 31);
     if (m >= rows) continue;
     bf16* yr = y + (int64_t)(row0 + m) * ldy + n0 + (GLU ? 32 : 64) * p;
     const float rw = GLU ? unit.factor(row0 + m) : 1.f;
@@ -488,21 +508,46 @@ HDS_EXPORT int hds_experts_gemm(const void* x, int64_t ldx, const int* src, int 
   // experts, 2 a token, 14336 x 4096: 1,500 tokens 1,774 us against 1,534 here, 2,000 2,063 / 2,054, 2,700 2,390 / 2,488; 64
   // experts, 6 a token, 1024 x 2048: 3,000 540 / 427, 6,000 786 / 733, 12,000 1,262 / 1,315.
   const bool big = N % big_cols == 0 && T >= 2 * BM2 * E;
-  const int cols = big ? big_cols : big_cols / 2;
+  // Otherwise the tile of weight rows with which the rounds over the CUs take least; a round of 64, 128 and 256 weight rows
+  // takes about 3, 4 and 6 parts (one round of [2048, 5632]: 41.5 / 44.7 / 57 us at 66 tokens, 60 / 77 / 118 at 500). Experts
+  // are taken to be alike.
+  const int cols_of = glu ? 2 : 1, avg = T / E + 1;
+  const int64_t tiles = (int64_t)std::min(E, T) * ((avg + avg / 8 + BM2 - 1) / BM2);
+  int wr = 64;
+  int64_t least = 0;
+  for (int r = 64; r <= 256; r *= 2) {
+    const int64_t cost = (tiles * (N / (r / cols_of)) + 255) / 256 * (r / 64 + 2);
+    if (N % (r / cols_of) == 0 && (r == 64 || cost < least)) {
+      wr = r;
+      least = cost;
+    }
+  }
+  // Weight rows an odd multiple of 4 KB apart lie alike in the memory's channels, and workgroups that walk them side by side
+  // meet in the same ones: there each begins its walk along K somewhere else. It helps gate and up rows, which are two such
+  // walks a workgroup (1024 x 2048, 66 tokens 123 -> 96 us, 1,600 147 -> 135; 3,000, with two tiles an expert, 244 -> 275),
+  // and single rounds, whose workgroups stay in step ([4096, 14336], 66 tokens 175 -> 160); over several rounds ([4096, 2048],
+  // 200 tokens 180 -> 192) and with rows of 8 KB ([28672, 4096] 351 -> 386) it costs what is shared in L2.
+  const int apart = K % 2048 == 0 && K / 2048 % 2 && avg <= 192 && (glu || tiles * (N / wr) <= 256);
+  const int cols = big ? big_cols : wr / cols_of;
   if (N % cols || K % BK || ldx < K || ldx % 8 || ldy < N || ldy % 8 || max_tiles < 1 || max_tiles > 65535 ||
       (src != nullptr && n_src < 1) || (act != 0 && act != 5) || (int64_t)(N / cols) * max_tiles > INT32_MAX)
     return hipErrorInvalidValue;
-#define HDS_EGK(KERNEL, GA, GL)                                                                                     \
-  hipLaunchKernelGGL((KERNEL<GA, GL>), dim3(N / cols * max_tiles), dim3(512), 0, st, (const bf16*)x, ldx, src, n_src, \
-                     (const bf16*)w, (bf16*)y, offs, tile_e, tile_m, n_tiles, T, N, K, ldy, N / cols, unit)
-#define HDS_EG(GA, GL)                                                                    \
-  if (big) { HDS_EGK(gg_big_kernel, GA, GL); } else { HDS_EGK(gg_flow_kernel, GA, GL); }
+  auto run = [&](auto kernel, auto... more) {
+    hipLaunchKernelGGL(kernel, dim3(N / cols * max_tiles), dim3(512), 0, st, (const bf16*)x, ldx, src, n_src, (const bf16*)w,
+                       (bf16*)y, offs, tile_e, tile_m, n_tiles, T, N, K, ldy, N / cols, unit, more...);
+  };
+#define HDS_EG(GA, GL)                                                     \
+  do {                                                                     \
+    if (big) run(gg_big_kernel<GA, GL>);                                   \
+    else if (wr == 256) run(gg_flow_kernel<GA, GL, 256>, apart);           \
+    else if (wr == 128) run(gg_flow_kernel<GA, GL, 128>, apart);           \
+    else run(gg_flow_kernel<GA, GL, 64>, apart);                           \
+  } while (0)
   if (src != nullptr) {
-    if (glu) { HDS_EG(true, true); } else { HDS_EG(true, false); }
+    if (glu) HDS_EG(true, true); else HDS_EG(true, false);
   } else {
-    if (glu) { HDS_EG(false, true); } else { HDS_EG(false, false); }
+    if (glu) HDS_EG(false, true); else HDS_EG(false, false);
   }
 #undef HDS_EG
-#undef HDS_EGK
   return hipGetLastError();
 }

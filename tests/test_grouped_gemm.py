@@ -144,6 +144,16 @@ def test_experts_gemm_hip(cuda, counts, N, K, gather, glu):
     assert ((y[:, :N].double() - ref).abs() <= bound).all() and y[:, N:].isnan().all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts", [[129, 192, 193, 3], [64, 1, 256, 65]])
+@pytest.mark.parametrize("N,K,gather,glu", [(4096, 128, True, True), (8192, 384, False, True), (16384, 128, True, False),
+                                            (8192, 256, False, False), (4096, 2048, True, True), (8192, 2048, False, False)])
+def test_experts_gemm_tiles_of_weight_rows(cuda, counts, N, K, gather, glu):
+    """128 and 256 weight rows a tile, which many rounds choose, with one to four blocks of 64 rows; fewer steps than the ring
+    holds; walks along K that begin apart."""
+    test_experts_gemm_hip(cuda, counts, N, K, gather, glu)
+
+
 def test_counted_waits_retire_lds_reads():
     """A statement that waits for loads and joins a barrier, behind which others overwrite what the wave has read from LDS,
     waits for those reads too: nothing else keeps their use in front of it."""
