@@ -51,12 +51,12 @@ __global__ __launch_bounds__(256) void transpose_bf16_kernel(const bf16* __restr
 }
 
 // v2 (default): 64 x 128 tiles, every LDS access 8 or 16 B wide (transpose_tile.h). v1's LDS traffic was one 2-B write and
-// one 2-B read per element (32 LDS instructions per thread per 16 B moved).
+// one 2-B read per element (32 LDS instructions per thread per 16 B moved). dst rows may be longer than src has rows: zeros.
 template <bool LINES>
 __global__ __launch_bounds__(256) void transpose_bf16_v2_kernel(const bf16* __restrict__ src, bf16* __restrict__ dst,
-                                                                int rows, int cols, int64_t lds) {
+                                                                int rows, int cols, int64_t lds, int ldd) {
   __shared__ __attribute__((aligned(16))) bf16 tile[kTrRows * kTrCols];
-  const TileAt at = tile_at<LINES>(rows, cols);
+  const TileAt at = tile_at<LINES>(ldd, cols);
   const int tid = threadIdx.x;
   const bool full = (at.r0 + kTrRows <= rows) && (at.c0 + kTrCols <= cols);
 #pragma unroll
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256) void transpose_bf16_v2_kernel(const bf16* __re
     *reinterpret_cast<bf16x8*>(&tile[tile_chunk(rr, ch)]) = x;
   }
   __syncthreads();
-  store_transposed<LINES>(tile, dst, at, rows, cols);
+  store_transposed<LINES>(tile, dst, at, ldd, cols);
 }
 
 }  // namespace
@@ -92,14 +92,25 @@ HDS_EXPORT int hds_transpose_bf16_var(const void* src, void* dst, int rows, int 
     const dim3 grid(tile_count(rows, cols));
     if (tile_lines(rows, dst))
       hipLaunchKernelGGL(transpose_bf16_v2_kernel<true>, grid, dim3(256), 0, st, (const bf16*)src, (bf16*)dst, rows,
-                         cols, (int64_t)lds);
+                         cols, (int64_t)lds, rows);
     else
       hipLaunchKernelGGL(transpose_bf16_v2_kernel<false>, grid, dim3(256), 0, st, (const bf16*)src, (bf16*)dst, rows,
-                         cols, (int64_t)lds);
+                         cols, (int64_t)lds, rows);
   }
   return hipGetLastError();
 }
 
 HDS_EXPORT int hds_transpose_bf16(const void* src, void* dst, int rows, int cols, long lds, hipStream_t st) {
   return hds_transpose_bf16_var(src, dst, rows, cols, lds, 2, st);
+}
+
+// The same for any number of rows, to rows of ldd (a multiple of 64, at least `rows`) whose ends are zeros: as operands of a
+// product over the rows they are aligned and add nothing. dst 128-byte aligned. [1018, 11264] 9 us; by strided copies 28 us
+// for half as many columns.
+HDS_EXPORT int hds_transpose_bf16_pad(const void* src, void* dst, int rows, int cols, long lds, int ldd, hipStream_t st) {
+  if (rows <= 0 || cols <= 0) return hipSuccess;
+  if (lds % 8 || ldd % 64 || ldd < rows || ((uintptr_t)src & 15) || ((uintptr_t)dst & 127)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(transpose_bf16_v2_kernel<true>, dim3(tile_count(ldd, cols)), dim3(256), 0, st, (const bf16*)src,
+                     (bf16*)dst, rows, cols, (int64_t)lds, ldd);
+  return hipGetLastError();
 }

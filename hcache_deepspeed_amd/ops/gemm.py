@@ -76,6 +76,21 @@ def transpose2d(x, variant=None):
     return out
 
 
+def transpose2d_padded(x):
+    """[R, C] (unit last stride) -> [C, R rounded up to a multiple of 64], zeros behind the R columns, by the HIP kernel; None
+    where it does not apply. Rows of a transpose that are no multiple of 16 bytes cost the GEMM its fast loads."""
+    R, C = x.shape
+    if not (native.use_native(x) and x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and R and C):
+        return None
+    out = torch.empty(C, -(-R // 64) * 64, dtype=x.dtype, device=x.device)
+    if out.data_ptr() % 128:
+        return None
+    native.check(native.kernels().hds_transpose_bf16_pad(x.data_ptr(), out.data_ptr(), R, C, x.stride(0), out.shape[1],
+                                                         native.stream()), "transpose_bf16_pad")
+    return out
+
+
 _WGRAD_LAYOUT = os.environ.get("HDS_WGRAD_LAYOUT", "auto")  # auto | direct | nt | direct_sk2 | nt_sk2
 _WGRAD_CHOICE = {}
 _SPLITK = os.environ.get("HDS_WGRAD_SPLITK", "0") == "1"  # two-stream split-K candidates in the timed choice
@@ -131,8 +146,14 @@ def _wgrad_run(layout, dy2, x2, out, accumulate, dyt=None, xt=None):
     None)."""
     base, sk2, b2 = layout.split("_")[0], layout.endswith("_sk2"), layout.endswith("_b2")
     if base == "nt":  # hipBLASLt's NT form on transposed copies (the forward GEMM's fast layout)
-        a = dyt if dyt is not None else transpose2d(dy2)
-        bt = (xt if xt is not None else transpose2d(x2)).t()
+        a = b = None
+        if dyt is None and xt is None and dy2.shape[0] % 8:  # odd token counts: both operands padded alike
+            a = transpose2d_padded(dy2)
+            b = transpose2d_padded(x2) if a is not None else None
+        if b is None:
+            a = dyt if dyt is not None else transpose2d(dy2)
+            b = xt if xt is not None else transpose2d(x2)
+        bt = b.t()
     else:
         a, bt = dy2.t(), x2
     split_a, split_b = (lambda t, lo, hi: t[:, lo:hi]), (lambda t, lo, hi: t[lo:hi])

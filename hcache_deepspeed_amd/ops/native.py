@@ -113,6 +113,7 @@ _KERNEL_SIGS = {
     "hds_fp6_gemv": "pppp" + "iiiiii" + "s",
     "hds_transpose_bf16": "pp" + "ii" + "l" + "s",
     "hds_transpose_bf16_var": "pp" + "ii" + "l" + "i" + "s",
+    "hds_transpose_bf16_pad": "pp" + "ii" + "l" + "i" + "s",
     "hds_gemv_bf16_supported": "iii",
     "hds_gemv_bf16": "pppp" + "iii" + "ll" + "s",
     "hds_gemv_fused_bf16": "ppp" + "f" + "pppp" + "if" + "iii" + "ll" + "s",

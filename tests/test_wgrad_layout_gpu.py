@@ -99,6 +99,21 @@ def test_wgrad_pretransposed_operands(pre, monkeypatch):
     assert (out.float() - 2 * ref).abs().max().item() <= 4e-2 * ref.abs().max().item()
 
 
+@pytest.mark.parametrize("R,C,ld", [(1, 8, 8), (63, 130, 136), (65, 128, 128), (509, 2048, 2048), (1018, 264, 512)])
+def test_padded_transpose(R, C, ld):
+    """Any number of rows: the transpose exactly, zeros behind it; weight gradients of odd token counts on it, a sum of R
+    products rounded once to bf16."""
+    from hcache_deepspeed_amd.ops import gemm
+    x = torch.randn(R, ld, device="cuda").bfloat16()[:, :C]
+    y = gemm.transpose2d_padded(x)
+    assert y.shape == (C, (R + 63) // 64 * 64) and torch.equal(y[:, :R], x.t()) and not y[:, R:].any()
+    dy = torch.randn(R, 72, device="cuda").bfloat16()
+    out = torch.empty(72, C, device="cuda", dtype=torch.bfloat16)
+    gemm._wgrad_run("nt", dy, x, out, False)
+    ref, mag = dy.double().t() @ x.double(), dy.double().abs().t() @ x.double().abs()
+    assert ((out.double() - ref).abs() <= 2**-8 * ref.abs() + 2**-20 * mag).all()
+
+
 def test_zero_linear_saves_transposed_input():
     """runtime/zero/linear: an input carrying _hds_t is saved as its transpose; gradients match F.linear's."""
     from hcache_deepspeed_amd.runtime.zero.linear import zero3_linear
