@@ -207,15 +207,22 @@ struct QueryBias<D, bf16> {
   }
   // what the scores start from: the mask, so that beside a huge one all keys' scores round alike
   template <bool TAIL>
-  __device__ __forceinline__ f32x16 start(int k0, int L) const {
+  __device__ __forceinline__ bf16 mask(int k0, int L) const {
+    const int k = k0 + (threadIdx.x & 31);
+    return b1 != nullptr ? b1[TAIL ? min(k, L - 1) : k] : (bf16)0.f;
+  }
+  template <bool TAIL>
+  __device__ __forceinline__ f32x16 start(bf16 v, int k0, int L) const {
     f32x16 s{};
     if (TAIL || b1 != nullptr) {
-      const int k = k0 + (threadIdx.x & 31);
-      bf16 v = b1 != nullptr ? b1[TAIL ? min(k, L - 1) : k] : (bf16)0.f;
-      if (TAIL && k >= L) v = __builtin_bit_cast(bf16, (uint16_t)kLowest);
+      if (TAIL && k0 + (int)(threadIdx.x & 31) >= L) v = __builtin_bit_cast(bf16, (uint16_t)kLowest);
       s = mfma(spread<D>(v), inv, s);
     }
     return s;
+  }
+  template <bool TAIL>
+  __device__ __forceinline__ f32x16 start(int k0, int L) const {
+    return start<TAIL>(mask<TAIL>(k0, L), k0, L);
   }
   template <bool TAIL, bool WATCH = false>
   __device__ __forceinline__ f32x16 add(int k0, int hf, int L, f32x16 s) {
@@ -272,6 +279,14 @@ struct QueryBias<D, float> {
         if (k0 + acc_row(i, hf) >= L) s[i] = -INFINITY;
     }
     return s;
+  }
+  template <bool TAIL>
+  __device__ __forceinline__ float mask(int, int) const {
+    return 0.f;
+  }
+  template <bool TAIL>
+  __device__ __forceinline__ f32x16 start(float, int, int) const {
+    return f32x16{};
   }
   template <bool TAIL>
   __device__ __forceinline__ f32x16 start(int, int) const {
@@ -832,6 +847,22 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_bwd_kernel(EvoParams p, int ro
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int kPairTiles = 2;  // of 32 keys: a wave's 32 sums and 32 biases a lane leave room for four waves a SIMD
 
+__device__ __forceinline__ void store_pair_sums(float* out, const f32x16 (&sum)[kPairTiles], int k0, int hf, int L) {
+#pragma unroll
+  for (int t = 0; t < kPairTiles; ++t)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int k = k0 + 32 * t + 8 * g + 4 * hf;
+      if (L % 4 == 0 && k < L) {
+        *reinterpret_cast<f32x4*>(out + k) = f32x4{sum[t][4 * g], sum[t][4 * g + 1], sum[t][4 * g + 2], sum[t][4 * g + 3]};
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (k + i < L) out[k + i] = sum[t][4 * g + i];
+      }
+    }
+}
+
 template <int D, typename TB>
 __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblocks, int kblocks, int rows_per) {
   using T = Tile<D>;
@@ -896,20 +927,109 @@ __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblo
   };
   if (kk0 + 32 * kPairTiles <= L) walk(std::false_type{}); else walk(std::true_type{});
   if (myq >= L) return;
-  float* out = p.part + (((int64_t)chunk * p.B + b) * p.H + h) * L * L + (int64_t)myq * L;
+  store_pair_sums(p.part + (((int64_t)chunk * p.B + b) * p.H + h) * L * L + (int64_t)myq * L, sum, kk0, hf, L);
+}
+
+// The same for narrower heads, whose operands of two rows fit in LDS (64 or 128 KB; D = 128 would want 256): a workgroup of
+// up to 4 x 2 waves stages the queries and the keys that its waves share, a row ahead. In the kernel above each wave
+// loads its own, between them almost three times the bytes, in pieces of 16 bytes a row, and waits for them. 128 rows of
+// 256, 8 heads, D = 32: 58 -> 42 us; a training pass with D = 64 296 -> 251 us. The exponents and what is around them,
+// some 8 vector instructions a score, bound it now.
+template <int D, typename TB>
+__global__ __launch_bounds__(512, 2) void evo_dpair_rows_kernel(EvoParams p, int qblocks, int kblocks, int rows_per,
+                                                                int nwq) {
+  using T = Tile<D>;
+  constexpr int M = 128 * T::RB;  // of a matrix: 128 rows
+  extern __shared__ __attribute__((aligned(1024))) char smem[];  // two rows n: Q, dO, K, V
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6, nwk = nw / nwq;
+  const int hf = lane >> 5, j = lane & 31, L = p.L, wq = w % nwq, wk = w / nwq;
+  int id = xcd_id();
+  const int qb = id % qblocks;
+  id /= qblocks;
+  const int kb = id % kblocks;
+  id /= kblocks;
+  const int h = id % p.H;
+  id /= p.H;
+  const int b = id % p.B, chunk = id / p.B;
+  const int qs = 32 * qb * nwq, ks0 = 32 * kPairTiles * kb * nwk;  // of the workgroup
+  const int myq = qs + 32 * wq + j, qc = min(myq, L - 1), kk0 = ks0 + 32 * kPairTiles * wk;
+  const bool live = qs + 32 * wq < L && kk0 < L;
+  const int n0 = chunk * rows_per, n1 = min(p.N, n0 + rows_per);
+  const float c = p.rest * kLog2e;
+  const int64_t ld = (int64_t)p.H * D;
+  QueryBias<D, TB> bias(nullptr, (const TB*)p.b2 + ((int64_t)(b * p.H + h) * L + qc) * L, p.rest);
+  f32x16 sum[kPairTiles];
 #pragma unroll
-  for (int t = 0; t < kPairTiles; ++t)
+  for (int t = 0; t < kPairTiles; ++t) sum[t] = f32x16{};
+
+  auto walk = [&](auto tail) {
+    constexpr bool TAIL = decltype(tail)::value;
+    u32x4 pair[kPairTiles][2];
+    if constexpr (sizeof(TB) == 2) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int k = 32 * (kb * kPairTiles + t) + 8 * g + 4 * hf;
-      if (L % 4 == 0 && k < L) {
-        *reinterpret_cast<f32x4*>(out + k) = f32x4{sum[t][4 * g], sum[t][4 * g + 1], sum[t][4 * g + 2], sum[t][4 * g + 3]};
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (k + i < L) out[k + i] = sum[t][4 * g + i];
+      for (int t = 0; t < kPairTiles; ++t) {
+        bias.template load_pair<TAIL>(kk0 + 32 * t, L, pair[t]);
+        pair[t][0] = finite(pair[t][0]);
+        pair[t][1] = finite(pair[t][1]);
       }
     }
+    float lse_n, delta_n;
+    TB mask_n[kPairTiles];
+    auto mask_row = [&](int n) {
+      if (p.b1 != nullptr) bias.b1 = (const TB*)p.b1 + ((int64_t)b * p.N + n) * L;
+    };
+    auto load = [&](int n) {
+      const int64_t bn = (int64_t)b * p.N + n, base = bn * L * ld + (int64_t)h * D, stat = (bn * p.H + h) * L;
+      char* s = smem + (n - n0) % 2 * 4 * M;
+      lse_n = p.lse[stat + qc];
+      delta_n = p.delta[stat + qc];
+      mask_row(n);
+#pragma unroll
+      for (int t = 0; t < kPairTiles; ++t) mask_n[t] = bias.template mask<TAIL>(kk0 + 32 * t, L);
+      T::stage(s, p.q + base, ld, qs, nwq, L, nw);
+      T::stage(s + M, p.dout + base, ld, qs, nwq, L, nw);
+      T::stage(s + 2 * M, p.k + base, ld, ks0, kPairTiles * nwk, L, nw);
+      T::stage(s + 3 * M, p.v + base, ld, ks0, kPairTiles * nwk, L, nw);
+    };
+    load(n0);
+#pragma unroll 1
+    for (int n = n0; n < n1; ++n) {
+      const char* s = smem + (n - n0) % 2 * 4 * M;
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this row has arrived, and every wave is done with the one before
+      __syncthreads();
+      const float lse_raw = lse_n / p.rest, delta = delta_n;
+      TB mask[kPairTiles];
+#pragma unroll
+      for (int t = 0; t < kPairTiles; ++t) mask[t] = mask_n[t];
+      if (n + 1 < n1) load(n + 1);
+      if (!live) continue;
+      mask_row(n);
+      bf16x8 qf[T::KS], df[T::KS];
+#pragma unroll
+      for (int ks = 0; ks < T::KS; ++ks) {
+        qf[ks] = T::rows(s, 32 * wq, ks);
+        df[ks] = T::rows(s + M, 32 * wq, ks);
+      }
+      times<D>(qf, p.power);
+#pragma unroll
+      for (int t = 0; t < kPairTiles; ++t) {
+        const int k0 = kk0 + 32 * t, kr = 32 * (kPairTiles * wk + t);
+        f32x16 x = bias.template start<TAIL>(mask[t], k0, L), d = f32x16{};
+#pragma unroll
+        for (int ks = 0; ks < T::KS; ++ks) x = mfma(T::rows(s + 2 * M, kr, ks), qf[ks], x);
+        if constexpr (sizeof(TB) == 2) x = bias.add_pair(pair[t], x);
+        else x = bias.template add<TAIL>(k0, hf, L, x);
+#pragma unroll
+        for (int ks = 0; ks < T::KS; ++ks) d = mfma(T::rows(s + 3 * M, kr, ks), df[ks], d);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[t][r] += fast_exp2((x[r] - lse_raw) * c) * (d[r] - delta);
+      }
+    }
+  };
+  // the workgroup's tail is every wave's: they meet at barriers
+  if (ks0 + 32 * kPairTiles * nwk <= L) walk(std::false_type{}); else walk(std::true_type{});
+  if (!live || myq >= L) return;
+  store_pair_sums(p.part + (((int64_t)chunk * p.B + b) * p.H + h) * L * L + (int64_t)myq * L, sum, kk0, hf, L);
 }
 
 template <typename TB>
@@ -991,7 +1111,7 @@ HDS_EXPORT int hds_evoformer_fwd(const void* q, const void* k, const void* v, co
 }
 
 // Chunks of rows that the pair bias' gradient is summed in, and so the floats of scratch it wants: chunks * B * H * L * L.
-// A wave walks over its chunk alone, so there are as many as fill the chip twice over, of at least four rows.
+// A workgroup walks over its chunk alone, so there are as many as fill the chip twice over, of at least four rows.
 HDS_EXPORT int hds_evoformer_pair_chunks(int B, int N, int L, int H) {
   if (B <= 0 || N <= 0 || L <= 0 || H <= 0) return 0;
   const int64_t waves = (int64_t)B * H * ((L + 31) / 32) * ((L + 32 * kPairTiles - 1) / (32 * kPairTiles));
@@ -1053,14 +1173,32 @@ HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, co
   }
   if (db2 != nullptr) {
     const int chunks = hds_evoformer_pair_chunks(B, N, L, H), per = (N + chunks - 1) / chunks;
+    const int64_t n = (int64_t)B * H * L * L;
     const int w4 = waves_of(L, 4), qblocks = (L + 32 * w4 - 1) / (32 * w4);
-    const int kblocks = (L + 32 * kPairTiles - 1) / (32 * kPairTiles);
-    const int64_t n = (int64_t)B * H * L * L, grid2 = (int64_t)chunks * B * H * kblocks * qblocks;
+    const int kt = (L + 32 * kPairTiles - 1) / (32 * kPairTiles);
+    const int kblocks = D == 128 ? kt : (kt + 1) / 2, wk = (kt + kblocks - 1) / kblocks;
+    const int64_t grid2 = (int64_t)chunks * B * H * kblocks * qblocks;
     if (grid2 > 0x7fffffff || (n + 1023) / 1024 > 0x7fffffff) return hipErrorInvalidValue;
-#define HDS_EVO(DD, TT)                                                                                             \
-  hipLaunchKernelGGL((evo_dpair_kernel<DD, TT>), dim3(grid2), dim3(64 * w4), 0, st, p, qblocks, kblocks, per)
-    HDS_EVO_ALL(HDS_EVO)
-#undef HDS_EVO
+    auto rows = [&](auto kernel, int lds) {
+      const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      if (e == hipSuccess)
+        hipLaunchKernelGGL(kernel, dim3(grid2), dim3(64 * w4 * wk), lds, st, p, qblocks, kblocks, per, w4);
+      return e;
+    };
+    hipError_t e = hipSuccess;
+    if (D == 128) {
+      if (bias_dtype == kBF16)
+        hipLaunchKernelGGL((evo_dpair_kernel<128, bf16>), dim3(grid2), dim3(64 * w4), 0, st, p, qblocks, kblocks, per);
+      else
+        hipLaunchKernelGGL((evo_dpair_kernel<128, float>), dim3(grid2), dim3(64 * w4), 0, st, p, qblocks, kblocks, per);
+    } else if (D == 32) {
+      constexpr int lds = 8 * 128 * Tile<32>::RB;
+      e = bias_dtype == kBF16 ? rows(evo_dpair_rows_kernel<32, bf16>, lds) : rows(evo_dpair_rows_kernel<32, float>, lds);
+    } else {
+      constexpr int lds = 8 * 128 * Tile<64>::RB;
+      e = bias_dtype == kBF16 ? rows(evo_dpair_rows_kernel<64, bf16>, lds) : rows(evo_dpair_rows_kernel<64, float>, lds);
+    }
+    if (e != hipSuccess) return e;
     if (bias_dtype == kBF16)
       hipLaunchKernelGGL(evo_pair_sum_kernel<bf16>, dim3((n + 1023) / 1024), dim3(256), 0, st, part, (bf16*)db2, n,
                          chunks);

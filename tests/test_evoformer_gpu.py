@@ -118,6 +118,18 @@ def test_evoformer_rows_of_one_head(cuda, B, N, L, H, which):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("bias_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,N,L,D,which", [(1, 9, 2, 32, "both"), (1, 33, 65, 32, "both"), (2, 21, 129, 64, "both"),
+                                           (1, 17, 161, 32, "pair"), (1, 13, 256, 64, "both"), (1, 7, 290, 64, "pair")])
+def test_evoformer_pair_gradient_of_shared_rows(cuda, B, N, L, D, which, bias_dtype):
+    """The pair bias' gradient summed over rows staged by a workgroup: one or two waves of keys, the second past the end,
+    queries past the end, several workgroups of either, one and several chunks of rows of which the last is shorter. (Two keys at least: with one, dS is exactly zero and
+    a relative bound has nothing to hold against the 2^-24 sum |dO V| that dP and delta may differ by, 1.06e-6 in dQ's
+    norm here.)"""
+    test_evoformer_edges_hip(cuda, B, N, L, 3, D, which, bias_dtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bias_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("where", ["mask", "pair"])
 @pytest.mark.parametrize("low", ["inf", "lowest"])
 @pytest.mark.parametrize("L,D,first", [(70, 32, 32), (257, 64, 64), (96, 128, 32), (300, 32, 256)])
