@@ -21,7 +21,7 @@ using namespace hds;
 // ---------------------------------------------------------------------------------------------------------------
 // logits[T, R] = x[T, K] . w[R, K]^T in 32-bit. A workgroup: 16 RT router rows x 16 tokens, its NW waves take every
 // NW-th 32 of K (K % 32 == 0). mfma_f32_16x16x32_bf16 with A = router rows, B = tokens (accumulator column = token).
-// Long steps use a large RT (the tokens are read once for most routers), short ones spread over workgroups.
+// What a CU can fetch bounds it, 16 bytes a clock of 16 (RT + 1) rows of K: see the launch for the choice of RT.
 template <int RT, int NW>
 __global__ __launch_bounds__(64 * NW) void router_logits_kernel(const bf16* __restrict__ x, int64_t ldx,
                                                             const bf16* __restrict__ w, float* __restrict__ z,
@@ -569,7 +569,21 @@ HDS_EXPORT int hds_router_logits(const void* x, int64_t ldx, const void* w, floa
 #define HDS_RL(RT, NW)                                                                                               \
   hipLaunchKernelGGL((router_logits_kernel<RT, NW>), dim3((R + 16 * RT - 1) / (16 * RT), (T + 15) / 16),            \
                      dim3(64 * NW), 0, st, (const bf16*)x, ldx, (const bf16*)w, z, ldz, T, R, K)
-  if (T >= 512) HDS_RL(5, 8); else if (T > 64) HDS_RL(1, 4); else HDS_RL(1, 16);
+  // Rounds of workgroups over the chip times the rows that one of them fetches; among equals the larger RT, which reads the
+  // tokens less often. 65 routers, K = 2048: 700 tokens RT = 5 12.2, RT = 1 5.7 us; 1,100 12.2, RT = 2 7.6; 1,623 12.3,
+  // RT = 3 9.6; 2,500 and more RT = 5 12.3, RT = 2 13.1. 257 routers, K = 5120, 1,100 tokens: 56.6, RT = 3 39.4. 8 routers,
+  // K = 4096, 4,096 tokens: 13.3, RT = 1 8.2. Four to sixteen waves: level.
+  int best = 5;
+  int64_t least = 0;
+  for (const int rt : {5, 3, 2, 1}) {
+    const int64_t groups = (int64_t)((R + 16 * rt - 1) / (16 * rt)) * ((T + 15) / 16);
+    const int64_t cost = (groups + 255) / 256 * (rt + 1);
+    if (least == 0 || cost < least) {
+      least = cost;
+      best = rt;
+    }
+  }
+  if (best == 5) HDS_RL(5, 8); else if (best == 3) HDS_RL(3, 8); else if (best == 2) HDS_RL(2, 8); else HDS_RL(1, 8);
 #undef HDS_RL
   return hipGetLastError();
 }

@@ -110,3 +110,20 @@ def test_experts_of_few_rows(N, K, T, E, k, glu):
         torch.testing.assert_close(out[a].double(), want, rtol=2**-7, atol=1e-3)
     torch.testing.assert_close(outs.double(), product(xs, ws, 1.0), rtol=2**-7, atol=1e-3)
     assert (out[n:] == 7.0).all()
+
+
+@pytest.mark.parametrize("T,R,K", [(1, 8, 128), (700, 65, 384), (1100, 65, 2048), (1623, 65, 2048), (1623, 33, 256),
+                                   (2500, 65, 1024), (513, 257, 128)])
+def test_router_logits_tiles(T, R, K):
+    """16, 32, 48 and 80 routers a workgroup, by how many workgroups there are, with both sides' last tiles part-filled.
+    The products are exact and summed in 32 bits: within K 2^-24 of their magnitudes' sum."""
+    from hcache_deepspeed_amd.ops import native
+    g = torch.Generator(device="cuda").manual_seed(T + R)
+    x = torch.randn(T, K + 8, device="cuda", generator=g).bfloat16()[:, :K]
+    w = torch.randn(R, K, device="cuda", generator=g).bfloat16()
+    z = torch.full((T, R + 3), 7.0, device="cuda")
+    native.check(native.kernels().hds_router_logits(x.data_ptr(), x.stride(0), w.data_ptr(), z.data_ptr(), R + 3, T, R, K,
+                                                    native.stream()), "router_logits")
+    bound = K * 2.0**-24 * (x.double().abs() @ w.double().abs().t())
+    assert ((z[:, :R].double() - x.double() @ w.double().t()).abs() <= bound).all()
+    assert (z[:, R:] == 7.0).all()
