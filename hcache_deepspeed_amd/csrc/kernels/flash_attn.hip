@@ -886,7 +886,9 @@ __device__ __forceinline__ void stage_full8(char* tile, const bf16* tile_base, c
 // PIPE: LDS operand reads issued two MFMAs ahead of their use as inline asm with counted lgkmcnt waits (a ring of
 // three fragments), instead of the compiler's load -> lgkmcnt(0) -> MFMA per product, which exposes the LDS latency
 // of every read (the MFMA pipe sat idle ~2/3 of the time: PMC 37 % MFMA busy).
-template <int D, int PRIO, int PIPE = 0>
+// SLICED: where the key blocks and heads are too few for the chip (a workgroup walks the queries of all heads that share
+// its keys), grid.y holds p.slices slices of each walk, which leave 32-bit sums for attn_bwd_slices_kernel.
+template <int D, int PRIO, int PIPE = 0, bool SLICED = false>
 __global__ __launch_bounds__(512) void attn_bwd_dkdv_split_kernel(AttnParams p) {
   constexpr int BK = 128;
   constexpr int KS = Dim<D>::KS, DT = Dim<D>::DT;
@@ -900,6 +902,11 @@ __global__ __launch_bounds__(512) void attn_bwd_dkdv_split_kernel(AttnParams p) 
   float* const LDbase = reinterpret_cast<float*>(smem + 8 * 16384);
   int kb, hk, b;
   lpt_ids(kb, hk, b);
+  int slice = 0;
+  if constexpr (SLICED) {
+    slice = hk / p.hkv;
+    hk -= slice * p.hkv;
+  }
   int start, len;
   seq_bounds(p, b, start, len);
   const int nkb = (len + BK - 1) / BK;
@@ -949,6 +956,7 @@ __global__ __launch_bounds__(512) void attn_bwd_dkdv_split_kernel(AttnParams p) 
   }
   const int nqt = qt_end - qt_begin;
   const int total = nqt * G;
+  const int it0 = SLICED ? total * slice / p.slices : 0, it1 = SLICED ? total * (slice + 1) / p.slices : total;
 
   int32_t oq[2] = {0, 0}, odo[2] = {0, 0};
   if constexpr (PIPE >= 2 && D == 128) {
@@ -988,14 +996,14 @@ __global__ __launch_bounds__(512) void attn_bwd_dkdv_split_kernel(AttnParams p) 
     }
   };
 
-  if (total > 0) stage(0, 0);
+  if (it0 < it1) stage(it0, it0 & 1);
   __syncthreads();
   if constexpr (PRIO != 0) {
     if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256) __builtin_amdgcn_s_setprio(1);
   }
-  for (int it = 0; it < total; ++it) {
+  for (int it = it0; it < it1; ++it) {
     const int buf = it & 1;
-    if (it + 1 < total) stage(it + 1, buf ^ 1);
+    if (it + 1 < it1) stage(it + 1, buf ^ 1);
     const int qt = qt_begin + it % nqt;
     const char* Qt = Qbase + buf * 16384;
     const char* Ot = Obase + buf * 16384;
@@ -1124,6 +1132,25 @@ __global__ __launch_bounds__(512) void attn_bwd_dkdv_split_kernel(AttnParams p) 
       }
   }
   __syncthreads();
+  if constexpr (SLICED) {  // a lane's sums as they are, whole lines; of every block and slice, past the last key too
+    if (qh != 0) return;
+    const int64_t unit = (((int64_t)slice * gridDim.z + b) * p.hkv + hk) * gridDim.x + kb;
+    f32x4* out = reinterpret_cast<f32x4*>(p.part) + (unit * 4 + kg) * (16 * D) + lane;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 a, b;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          a[j] = dk[dt][4 * g + j] + red[(dt * 16 + 4 * g + j) * 64 + lane];
+          b[j] = dv[dt][4 * g + j] + red[(64 + dt * 16 + 4 * g + j) * 64 + lane];
+        }
+        out[(4 * dt + g) * 64] = a;
+        out[(4 * (DT + dt) + g) * 64] = b;
+      }
+    return;
+  }
   if (qh == 0 && myk < len) {
     bf16* kp = p.dk + (int64_t)(start + myk) * p.sdk + (int64_t)hk * D;
     bf16* vp = p.dv + (int64_t)(start + myk) * p.sdv + (int64_t)hk * D;
@@ -1139,6 +1166,35 @@ __global__ __launch_bounds__(512) void attn_bwd_dkdv_split_kernel(AttnParams p) 
       store_row_block<D>(vp, b, dt, h, 1.f);
     }
   }
+}
+
+// The slices' sums of a wave's 32 keys: a wave takes 32 columns of dK, then of dV (grid: as above without the slices, times
+// four key groups).
+template <int D>
+__global__ __launch_bounds__(2 * D) void attn_bwd_slices_kernel(AttnParams p, int blocks) {
+  constexpr int DT = Dim<D>::DT;
+  const int lane = threadIdx.x & 63, dt = threadIdx.x >> 6, h = lane >> 5;
+  const int kg = blockIdx.x & 3, kb = blockIdx.x >> 2, hk = blockIdx.y, b = blockIdx.z;
+  int start, len;
+  seq_bounds(p, b, start, len);
+  const int k = kb * 128 + 32 * kg + (lane & 31);
+  if (kb * 128 >= len) return;  // (its sums are not written)
+  const int64_t units = (int64_t)gridDim.z * p.hkv * blocks, unit = ((int64_t)b * p.hkv + hk) * blocks + kb;
+  const f32x4* in = reinterpret_cast<const f32x4*>(p.part) + (unit * 4 + kg) * (16 * D) + lane;
+  f32x16 sum[2] = {};
+  for (int s = 0; s < p.slices; ++s, in += units * 4 * (16 * D)) {
+#pragma unroll
+    for (int w = 0; w < 2; ++w)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 v = in[(4 * (w * DT + dt) + g) * 64];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum[w][4 * g + j] += v[j];
+      }
+  }
+  if (k >= len) return;
+  store_row_block<D>(p.dk + (int64_t)(start + k) * p.sdk + (int64_t)hk * D, sum[0], dt, h, p.scale);
+  store_row_block<D>(p.dv + (int64_t)(start + k) * p.sdv + (int64_t)hk * D, sum[1], dt, h, 1.f);
 }
 
 // =====================================================================================
@@ -1487,7 +1543,16 @@ int launch_bwd(const AttnParams& p, int batch, int max_len, int total_tokens, in
   if constexpr (D <= 128) {
     if (g_dkdv_nw == 8) {
       const dim3 grid((max_len + 127) / 128, hkv, batch);
-      if (g_bwd_pipe == 2 && D == 128 && p.lse2)
+      if constexpr (D == 128) {
+        if (g_bwd_pipe == 2 && p.lse2 && p.slices > 1) {
+          hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, 1, 2, true>), dim3(grid.x, hkv * p.slices, batch), dim3(512), 0,
+                             st, p);
+          hipLaunchKernelGGL(attn_bwd_slices_kernel<D>, dim3(4 * grid.x, hkv, batch), dim3(2 * D), 0, st, p, (int)grid.x);
+          done = true;
+        }
+      }
+      if (done) {
+      } else if (g_bwd_pipe == 2 && D == 128 && p.lse2)
         hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, 1, 2>), grid, dim3(512), 0, st, p);
       else if (g_bwd_pipe && D == 128)
         hipLaunchKernelGGL((attn_bwd_dkdv_split_kernel<D, 1, 1>), grid, dim3(512), 0, st, p);
@@ -1571,14 +1636,35 @@ HDS_EXPORT int hds_attn_fwd(const void* q, const void* k, const void* v, void* o
   return hipErrorInvalidValue;
 }
 
+// Slices of the queries that dK and dV of few keys are summed in (1: none), and the floats of scratch they want (at most
+// 2^24). One workgroup a CU with walks of at least four steps (64 queries of a head), two with walks of sixteen, which
+// even out the causal blocks. A whole backward, 1 slice -> this: 2 x 509 tokens, 16 / 4 heads 88.6 -> 55.5 us (4: 58.0,
+// 16: 68.0); 1 x 2,048, 32 / 8 283 -> 172 (2: 200, 8: 191); 1 x 4,000, 8 / 1 890 -> 214 (8: 243); 4 x 512, 32 / 8
+// 95.6 -> 81.5 (4: 84.9). Short walks lose what the sums cost: 1 x 100, 16 / 16 21.5, with 2 slices 24.4.
+HDS_EXPORT int hds_attn_bwd_slices(int batch, int max_len, int hq, int hkv, int head_dim) {
+  if (head_dim != 128 || batch < 1 || max_len < 1 || hkv < 1 || hq < hkv) return 1;
+  const int64_t groups = (int64_t)((max_len + 127) / 128) * hkv * batch;
+  const int64_t steps = (int64_t)((max_len + 63) / 64) * (hq / hkv);  // of the longest walk
+  auto fit = [&](int64_t most, int64_t least) { return most / groups < steps / least ? most / groups : steps / least; };
+  int64_t s = fit(256, 4) > fit(512, 16) ? fit(256, 4) : fit(512, 16);
+  if (s > 16) s = 16;
+  return s < 2 ? 1 : (int)s;
+}
+HDS_EXPORT int hds_attn_bwd_part(int slices, int batch, int max_len, int hkv, int head_dim) {
+  return slices < 2 ? 0 : slices * batch * hkv * ((max_len + 127) / 128) * 256 * head_dim;
+}
+
+// part: hds_attn_bwd_part floats, or null with slices 1
 HDS_EXPORT int hds_attn_bwd(const void* q, const void* k, const void* v, const void* o, const float* lse,
                             const void* dout, void* dq, void* dk, void* dv, float* delta, const int64_t* strides,
                             const int* cu_seqlens, const int* seq_lens, int batch, int seq_len, int max_len,
                             int total_tokens, int hq, int hkv, int head_dim, float scale, int causal, int window,
-                            hipStream_t st) {
-  if (hq % hkv) return hipErrorInvalidValue;
+                            float* part, int slices, hipStream_t st) {
+  if (hq % hkv || slices < 1 || slices > 65535 / hkv || (slices > 1 && part == nullptr)) return hipErrorInvalidValue;
   AttnParams p = make_params(q, k, v, (void*)o, (float*)lse, dout, dq, dk, dv, delta, strides, cu_seqlens, seq_lens,
                              batch, seq_len, total_tokens, hq, hkv, scale, causal, window);
+  p.part = part;
+  p.slices = slices;
   p.lse2 = delta + (int64_t)hq * total_tokens;  // delta scratch is [2][Hq][T]: rowsum(dO * O), then lse * log2(e)
 #define HDS_CASE(d) \
   if (head_dim == d) return launch_bwd<d>(p, batch, max_len, total_tokens, hq, hkv, st);

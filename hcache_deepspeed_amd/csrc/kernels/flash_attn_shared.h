@@ -42,6 +42,8 @@ struct AttnParams {
   float scale;
   int causal;
   int window;  // >0: sliding window (keys in (q - window, q])
+  float* part;  // dK / dV of slices of the queries: [slices][batch, hkv, blocks of 128 keys, 4][dK, dV][32 x head size]
+  int slices;
   // paged forward: [n][2] sequence, first new token; [sequences][3] first row, new tokens, earlier tokens; block tables
   const int* blocks;
   const int* meta;

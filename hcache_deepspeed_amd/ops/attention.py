@@ -104,11 +104,16 @@ def _native_bwd(q, k, v, o, lse, do, dq, dk, dv, causal, scale, cu, B, seq_len, 
     T, Hq, D = q.shape
     delta = torch.empty(2, Hq, T, device=q.device, dtype=torch.float32)  # rowsum(dO * O), lse * log2(e)
     strides = _strides8(q, k, v, o, do, dq, dk, dv)
+    lib, part = native.kernels(), None
+    slices = lib.hds_attn_bwd_slices(B, max_len, Hq, k.shape[1], D)
+    if slices > 1:  # 32-bit sums of dK and dV
+        part = torch.empty(lib.hds_attn_bwd_part(slices, B, max_len, k.shape[1], D), device=q.device, dtype=torch.float32)
     native.check(
-        native.kernels().hds_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
-                                      do.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr(),
-                                      strides.data_ptr(), native.ptr(cu), native.ptr(seq_lens), B, seq_len, max_len,
-                                      T, Hq, k.shape[1], D, float(scale), int(causal), int(window), native.stream()),
+        lib.hds_attn_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
+                         do.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), delta.data_ptr(),
+                         strides.data_ptr(), native.ptr(cu), native.ptr(seq_lens), B, seq_len, max_len,
+                         T, Hq, k.shape[1], D, float(scale), int(causal), int(window), native.ptr(part),
+                         slices, native.stream()),
         "attn_bwd")
 
 

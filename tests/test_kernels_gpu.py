@@ -273,6 +273,27 @@ def test_flash_attn_head_dims(D, causal, window, no_attn_fallback):
     assert _rel(v.grad.reshape(B * S, Hkv, D), vr.grad) < 2e-2
 
 
+@pytest.mark.parametrize("lens,Hq,Hkv,causal,window", [
+    ([509, 509], 16, 4, True, 0), ([300, 1, 130, 64], 8, 1, True, 0), ([1025], 4, 4, True, 0), ([700], 8, 2, False, 0),
+    ([900, 200], 8, 1, True, 97), ([2048], 32, 8, True, 0)])
+def test_flash_attn_bwd_slices(lens, Hq, Hkv, causal, window, no_attn_fallback):
+    """dK and dV of few keys, summed in slices of the queries: blocks with fewer steps than slices, sequences shorter than
+    the grid's blocks, windows that leave few steps. Against the 32-bit reference: the products' operands P and dS and the
+    results are rounded to 8 bits, each by at most 2^-9 of itself, and dS is made of outputs that were."""
+    from hcache_deepspeed_amd.ops import native
+    from hcache_deepspeed_amd.ops.attention import flash_attn
+    assert native.kernels().hds_attn_bwd_slices(len(lens), max(lens), Hq, Hkv, 128) > 1
+    g = torch.Generator(device="cuda").manual_seed(Hq + len(lens))
+    T, cu = sum(lens), torch.tensor([0] + lens).cumsum(0).int()
+    rnd = lambda h: torch.randn(T, h, 128, device="cuda", generator=g).bfloat16()  # noqa: E731
+    q, k, v, do = rnd(Hq).requires_grad_(), rnd(Hkv).requires_grad_(), rnd(Hkv).requires_grad_(), rnd(Hq)
+    flash_attn(q, k, v, causal=causal, cu_seqlens=cu.cuda(), window=window).backward(do)
+    qr, kr, vr = (t.detach().float().requires_grad_() for t in (q, k, v))
+    _attn_ref(qr, kr, vr, causal, window, cu, None).backward(do.float())
+    for x, y in ((q, qr), (k, kr), (v, vr)):
+        assert _rel(x.grad, y.grad) < 4 * 2**-8
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_flash_attn_padding_seq_lens(D, no_attn_fallback):
     """Right-padded batch + key-padding lengths (the BERT mask case) on the HIP kernels: valid rows match the
