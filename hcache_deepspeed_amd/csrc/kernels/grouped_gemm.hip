@@ -340,10 +340,16 @@ __device__ __forceinline__ void gg_flow_tile(char* smem, const bf16* const (&wp)
     if (c < C * KT) issue(c / C, c % C, c);
   int base = 0;  // place of the step's first chunk
   for (int kt = 0; kt < KT; ++kt) {
-    // this step's chunks have arrived for every wave, and every wave is done with the last step's (its reads have returned)
-    if (C * (kt - 1) + R <= C * KT) __builtin_amdgcn_s_waitcnt(flow_wait(R - 2 * C));
-    else __builtin_amdgcn_s_waitcnt(flow_wait(0));
-    asm volatile("s_barrier" ::: "memory");
+    // This step's chunks have arrived for every wave, and every wave is done with the last step's: its reads have returned
+    // (lgkmcnt), in one statement with the barrier, so that none can be moved between the two. The builtins in front tell
+    // the compiler of the wait, which otherwise adds its own for all loads.
+    if (C * (kt - 1) + R <= C * KT) {
+      __builtin_amdgcn_s_waitcnt(flow_wait(R - 2 * C));
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(R - 2 * C) : "memory");
+    } else {
+      __builtin_amdgcn_s_waitcnt(flow_wait(0));
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
 #pragma unroll
     for (int u = 0; u < C; ++u) {
       constexpr int first = R - C;
