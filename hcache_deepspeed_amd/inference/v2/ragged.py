@@ -10,7 +10,9 @@ MI355X sizing: the KV pool is carved out of the 288 GB HBM after weights (``memo
 "reserve" keeps ``size`` bytes free, "allocate" takes exactly ``size`` bytes). Host metadata lives in
 pinned buffers so ``finalize`` is one async H2D copy.
 """
+import weakref
 from array import array
+from collections import deque
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional
 
@@ -250,6 +252,26 @@ class DSStateManager:
 # -----------------------------------------------------------------------------------------------
 # ragged batch
 # -----------------------------------------------------------------------------------------------
+# Staging buffers of wrappers that are gone, each with the event behind its last copy to the device. The copy is a raw one, of
+# which torch's pinned allocator knows nothing: given back before the event has passed, a buffer could be another's, and
+# written, while a queued step has still to read it.
+_IN_FLIGHT = deque()
+
+
+def _retire(slots, events):  # (no call to the GPU: it may run anywhere, also while a stream captures)
+    _IN_FLIGHT.extend((ev, buf) for ev, buf in zip(events, slots) if ev is not None)
+
+
+def _give_back():
+    for _ in range(len(_IN_FLIGHT)):
+        try:
+            held = _IN_FLIGHT.popleft()
+        except IndexError:  # another thread was here
+            return
+        if not held[0].query():
+            _IN_FLIGHT.append(held)
+
+
 class RaggedBatchWrapper:
     """Host-built batch metadata; ``finalize`` ships it to the device in one async copy. The device tensors
     (``input_ids``, ``seq_meta``, ``tok_seq``, ``tok_pos``, ``last_token_idx``, ``block_tables``, ``atoms``, ``slots``) and the
@@ -313,8 +335,12 @@ class RaggedBatchWrapper:
 
     def _pinned_slot(self):
         """One of two rotating pinned int32 staging buffers; a slot is reused only after its H2D drained."""
-        slots = self.__dict__.setdefault("_slots", [None, None])
-        evs = self.__dict__.setdefault("_slot_events", [None, None])
+        if "_slots" not in self.__dict__:
+            self._slots, self._slot_events = [None, None], [None, None]
+            weakref.finalize(self, _retire, self._slots, self._slot_events).atexit = False
+        slots, evs = self._slots, self._slot_events
+        if _IN_FLIGHT:
+            _give_back()
         i = self.__dict__.get("_slot_next", 0)
         self._slot_next = i ^ 1
         if evs[i] is not None:

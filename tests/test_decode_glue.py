@@ -139,6 +139,43 @@ def test_step_description_of_any_tokens():
             b.finalize(100)
 
 
+def test_staging_buffers_outlive_their_copies():
+    """A wrapper that is dropped while its step's copy is queued: the pinned buffers stay until their events have passed."""
+    import gc
+    import weakref
+    from hcache_deepspeed_amd.inference.v2 import ragged
+
+    class Event:
+        passed = False
+
+        def query(self):
+            return self.passed
+
+        synchronize = record = None  # not to be called here
+
+    def step(events=None):
+        b = ragged.RaggedBatchWrapper(ragged.DSStateManagerConfig(), torch.device("cpu"), 4)
+        b.finalize()
+        if events:
+            b.finalize()
+            b._slot_events[:] = events
+        return [weakref.ref(t) for t in b._slots if t is not None]
+
+    events = [Event(), Event()]
+    held = step(events)
+    gc.collect()
+    assert all(r() is not None for r in held)
+    step()
+    assert all(r() is not None for r in held)
+    events[1].passed = True
+    step()
+    assert held[0]() is not None and held[1]() is None
+    events[0].passed = True
+    step()
+    gc.collect()
+    assert held[0]() is None and not ragged._IN_FLIGHT
+
+
 def test_only_plain_tensors_pass_autograd_by():
     from hcache_deepspeed_amd.ops import native
     x = torch.ones(2)
