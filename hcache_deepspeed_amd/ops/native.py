@@ -325,10 +325,11 @@ def check(err, what):
 
 
 def plain(*tensors):
-    """No gradient, functorch transform or dual number can want a record of what is done with these tensors: an autograd
-    function around a kernel (about 10 us of host time) may be passed by."""
+    """No gradient, functorch transform, dual number or trace can want a record of what is done with these tensors: an autograd
+    function around a kernel (about 10 us of host time) may be passed by. (A trace holds the function as one node that runs it
+    again; of a bare kernel it would see the allocation of the result only.)"""
     return (not torch.is_grad_enabled() and not torch._C._are_functorch_transforms_active()
-            and torch.autograd.forward_ad._current_level < 0
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._get_tracing_state() is None
             and all(t is None or type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors))
 
 

@@ -191,7 +191,20 @@ def test_only_plain_tensors_pass_autograd_by():
             pass
 
         seen.append(native.plain(x.as_subclass(Sub)))
-        assert seen == [False, False, False]
+        torch.jit.trace(lambda t: seen.append(native.plain(x)) or t, (x, ), check_trace=False)
+        assert seen == [False, False, False, False]
+
+
+@pytest.mark.gpu
+def test_traced_norms_and_gated_units_run_again():
+    """A graph recorded without gradients computes them for its own inputs."""
+    from hcache_deepspeed_amd.ops.activations import glu
+    from hcache_deepspeed_amd.ops.norm import layer_norm, rms_norm
+    w = torch.rand(256, device="cuda").bfloat16()
+    with torch.no_grad():
+        x, y = (torch.randn(64, 256, device="cuda").bfloat16() for _ in range(2))
+        for f in (lambda t: rms_norm(t, w), lambda t: rms_norm(t, w, residual=t)[0], lambda t: layer_norm(t, w, w), glu):
+            assert torch.equal(torch.jit.trace(f, (x, ), check_trace=False)(y), f(y))
 
 
 @pytest.mark.gpu
