@@ -1145,10 +1145,10 @@ HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, co
     auto launch = [&](auto tiles, auto mask) {
       constexpr int NT = decltype(tiles)::value;
       auto* kernel = evo_bwd_kernel<32, NT, decltype(mask)::value>;
-      static const hipError_t attr = hipFuncSetAttribute(
-          (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, Whole<32>::bytes(NT));
-      if (attr == hipSuccess) hipLaunchKernelGGL(kernel, grid, threads, Whole<32>::bytes(NT), st, p, per);
-      return attr;
+      const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               Whole<32>::bytes(NT));  // (of the current device)
+      if (e == hipSuccess) hipLaunchKernelGGL(kernel, grid, threads, Whole<32>::bytes(NT), st, p, per);
+      return e;
     };
     auto choose = [&](auto mask) {
       if (nt <= 2) return launch(std::integral_constant<int, 2>{}, mask);

@@ -221,3 +221,12 @@ def test_evoformer_saved_tensors_in_another_order(cuda):
     torch.cuda.synchronize()
     for a, b in zip(torch.autograd.grad(out, (q, k, v), do), want):
         assert torch.equal(a, b)
+
+
+def test_launch_attributes_are_set_for_the_current_device():
+    """A kernel's largest LDS size belongs to a device: set once a process, the others would refuse the launch."""
+    import pathlib
+    import re
+    import hcache_deepspeed_amd
+    src = (pathlib.Path(hcache_deepspeed_amd.__file__).parent / "csrc" / "kernels" / "evoformer.hip").read_text()
+    assert "hipFuncSetAttribute" in src and re.search(r"\bstatic\b[^;{]*hipFuncSetAttribute", src) is None
