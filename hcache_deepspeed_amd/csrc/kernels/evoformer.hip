@@ -619,7 +619,7 @@ struct Whole {  // a workgroup of one wave per 32 positions, a matrix of nt tile
   using T = Tile<D>;
   static constexpr int CH = T::CH, PER = CH / 2;  // 16-byte chunks of a row; chunks of a matrix that a thread moves
   static constexpr int SB = 128;                  // bytes of a row of dS^T: one key, 64 queries
-  static __host__ __device__ int bytes(int nt) { return 32 * nt * (3 * T::RB + SB + 8); }
+  static constexpr __host__ __device__ int bytes(int nt) { return 32 * nt * (3 * T::RB + SB + 8); }
   // the thread's number, made anew where it is asked for: addresses that are needed once a row of the loop shall not
   // stay in registers through it
   static __device__ __forceinline__ int tid() {
@@ -1138,12 +1138,15 @@ HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, co
   if (!set_scale(p, scale, bias_dtype, D)) return hipErrorInvalidValue;
   const int nt = (L + 31) / 32;
   if (bias_dtype == kBF16 && D == 32 && nt <= 8 && (int64_t)L * H * D < (1 << 30)) {  // (offsets in 32 bits)
-    // as many workgroups as the chip holds at once, two waves a SIMD, if there are rows for them
+    // as many workgroups as the chip holds at once, two waves a SIMD, if there are rows for them. Each size has its LDS: with
+    // the 21 KB of two tiles for one, seven workgroups fit where eight are counted on (512 rows of 16 / 32, 8 heads: 17.7 /
+    // 20.4 us, with its own 10 KB 12.0 / 18.0; 256 of 32 11.6 and 9.1)
     const int64_t rows = (int64_t)B * N * H, slots = 256 * (8 / nt);
     const int per = (int)((rows + slots - 1) / slots);
     const dim3 grid(B * H * ((N + per - 1) / per)), threads(64 * nt);
     auto launch = [&](auto tiles, auto mask) {
-      constexpr int NT = decltype(tiles)::value;
+      constexpr int NT = decltype(tiles)::value, least = NT <= 2 ? NT : NT / 2 + 1;
+      static_assert(Whole<32>::bytes(NT) * (8 / least) <= 160 * 1024, "fewer workgroups on a CU than are counted on");
       auto* kernel = evo_bwd_kernel<32, NT, decltype(mask)::value>;
       const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                Whole<32>::bytes(NT));  // (of the current device)
@@ -1151,7 +1154,8 @@ HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, co
       return e;
     };
     auto choose = [&](auto mask) {
-      if (nt <= 2) return launch(std::integral_constant<int, 2>{}, mask);
+      if (nt == 1) return launch(std::integral_constant<int, 1>{}, mask);
+      if (nt == 2) return launch(std::integral_constant<int, 2>{}, mask);
       if (nt <= 4) return launch(std::integral_constant<int, 4>{}, mask);
       return launch(std::integral_constant<int, 8>{}, mask);
     };

@@ -109,10 +109,11 @@ def test_evoformer_edges_hip(cuda, B, N, L, H, D, which, bias_dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,N,L,H,which", [(1, 70, 250, 8, "both"), (2, 75, 100, 4, "both"), (1, 1100, 40, 2, "mask"),
-                                           (1, 3, 256, 2, "pair"), (1, 5, 160, 1, "both"), (1, 2100, 32, 1, "both")])
+                                           (1, 3, 256, 2, "pair"), (1, 5, 160, 1, "both"), (1, 2100, 32, 1, "both"),
+                                           (1, 515, 20, 8, "both"), (1, 520, 64, 8, "mask")])
 def test_evoformer_rows_of_one_head(cuda, B, N, L, H, which):
     """The gradient kernel that takes a whole row in a workgroup: one and several rows after each other, the last chunk of
-    them shorter, full and partial tiles of 32, odd counts of tiles, each of its three sizes."""
+    them shorter, full and partial tiles of 32, odd counts of tiles, each of its four sizes."""
     test_evoformer_edges_hip(cuda, B, N, L, H, 32, which, torch.bfloat16)
 
 
