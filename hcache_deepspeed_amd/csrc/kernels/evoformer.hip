@@ -930,7 +930,8 @@ __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblo
   store_pair_sums(p.part + (((int64_t)chunk * p.B + b) * p.H + h) * L * L + (int64_t)myq * L, sum, kk0, hf, L);
 }
 
-// The same for narrower heads, whose operands of two rows fit in LDS (64 or 128 KB; D = 128 would want 256): a workgroup of
+// The same for narrower heads, whose operands of two rows fit in LDS (64 or 128 KB; D = 128 would want 256), where
+// hds_evoformer_pair_staged says so: a workgroup of
 // up to 4 x 2 waves stages the queries and the keys that its waves share, a row ahead. In the kernel above each wave
 // loads its own, between them almost three times the bytes, in pieces of 16 bytes a row, and waits for them. 128 rows of
 // 256, 8 heads, D = 32: 58 -> 42 us; a training pass with D = 64 296 -> 251 us. The exponents and what is around them,
@@ -1026,8 +1027,8 @@ __global__ __launch_bounds__(512, 2) void evo_dpair_rows_kernel(EvoParams p, int
       }
     }
   };
-  // the workgroup's tail is every wave's: they meet at barriers
-  if (ks0 + 32 * kPairTiles * nwk <= L) walk(std::false_type{}); else walk(std::true_type{});
+  // the workgroup's tail is every wave's: they meet at barriers (with 32-bit biases there is none)
+  if (sizeof(TB) == 4 || ks0 + 32 * kPairTiles * nwk <= L) walk(std::false_type{}); else walk(std::true_type{});
   if (!live || myq >= L) return;
   store_pair_sums(p.part + (((int64_t)chunk * p.B + b) * p.H + h) * L * L + (int64_t)myq * L, sum, kk0, hf, L);
 }
@@ -1122,6 +1123,24 @@ HDS_EXPORT int hds_evoformer_pair_chunks(int B, int N, int L, int H) {
   return (N + per - 1) / per;
 }
 
+// Are the rows of the pair bias' gradient staged by workgroups (evo_dpair_rows_kernel), rather than loaded by each wave for
+// itself? Where waves share something (more than one tile of keys) and there are enough of them that the rate counts and not
+// the way of a row through LDS. D = 32 wants most of its workgroups' tiles to be real, and 32-bit biases, whose tail is
+// vector instructions of every wave in the workgroup, none of them beyond the end. us, waves / staged: D = 32, 512 x 32
+// positions, 8 heads 25.9 / 30.1, 64 x 128, 4 heads 14.5 / 16.4, 128 x 96, 8 heads 21.5 / 20.4, 512 x 160 132 / 170, 512 x 192
+// 158 / 133, 4 x 512 19.1 / 20.8, 20 x 512, 4 heads 25.5 / 20.3; D = 64, 512 x 32 30.2 / 60.8, 512 x 64 44.5 / 55.8, 64 x 96, 4
+// heads 16.6 / 20.0, 64 x 128 19.4 / 18.3, 512 x 80, 8 heads 102 / 71, 512 x 160 232 / 213; 32-bit biases, D = 32, 512 x 192 264 /
+// 349, 512 x 256 333 / 294, D = 64, 418 / 440 and 524 / 330.
+HDS_EXPORT int hds_evoformer_pair_staged(int B, int N, int L, int H, int D, int bias_dtype) {
+  if (D == 128 || L <= 32 * kPairTiles) return 0;
+  const int64_t q32 = (L + 31) / 32, k64 = (L + 32 * kPairTiles - 1) / (32 * kPairTiles);
+  const int64_t waves = (int64_t)hds_evoformer_pair_chunks(B, N, L, H) * B * H * q32 * k64;
+  if (bias_dtype != kBF16) return waves > 1024 && L % (64 * kPairTiles) == 0;
+  if (D == 64) return waves >= 512;
+  const int64_t w4 = waves_of(L, 4), q = (q32 + w4 - 1) / w4 * w4 * 32, k = (k64 + 1) / 2 * 64 * kPairTiles;
+  return waves > 1024 && 4 * (int64_t)L * L >= 3 * q * k;
+}
+
 // Gradients of the forward above from its result and lse. delta [B, N, H, L] fp32 scratch. db1 [B, N, L] fp32, zeroed, or
 // null; db2 [B, H, L, L] of the biases' dtype, or null; part: see hds_evoformer_pair_chunks (with db2).
 HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, const void* o, const float* lse,
@@ -1178,30 +1197,32 @@ HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, co
   if (db2 != nullptr) {
     const int chunks = hds_evoformer_pair_chunks(B, N, L, H), per = (N + chunks - 1) / chunks;
     const int64_t n = (int64_t)B * H * L * L;
+    const bool staged = hds_evoformer_pair_staged(B, N, L, H, D, bias_dtype);
     const int w4 = waves_of(L, 4), qblocks = (L + 32 * w4 - 1) / (32 * w4);
     const int kt = (L + 32 * kPairTiles - 1) / (32 * kPairTiles);
-    const int kblocks = D == 128 ? kt : (kt + 1) / 2, wk = (kt + kblocks - 1) / kblocks;
+    const int kblocks = staged ? (kt + 1) / 2 : kt, wk = (kt + kblocks - 1) / kblocks;
     const int64_t grid2 = (int64_t)chunks * B * H * kblocks * qblocks;
     if (grid2 > 0x7fffffff || (n + 1023) / 1024 > 0x7fffffff) return hipErrorInvalidValue;
-    auto rows = [&](auto kernel, int lds) {
-      const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-      if (e == hipSuccess)
-        hipLaunchKernelGGL(kernel, dim3(grid2), dim3(64 * w4 * wk), lds, st, p, qblocks, kblocks, per, w4);
-      return e;
+    auto pair = [&](auto dim, auto type) -> hipError_t {
+      constexpr int DD = decltype(dim)::value;
+      using TB = decltype(type);
+      if constexpr (DD < 128) {
+        if (staged) {
+          auto* kernel = evo_dpair_rows_kernel<DD, TB>;
+          constexpr int lds = 8 * 128 * Tile<DD>::RB;
+          const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+          if (e == hipSuccess)
+            hipLaunchKernelGGL(kernel, dim3(grid2), dim3(64 * w4 * wk), lds, st, p, qblocks, kblocks, per, w4);
+          return e;
+        }
+      }
+      hipLaunchKernelGGL((evo_dpair_kernel<DD, TB>), dim3(grid2), dim3(64 * w4), 0, st, p, qblocks, kblocks, per);
+      return hipSuccess;
     };
-    hipError_t e = hipSuccess;
-    if (D == 128) {
-      if (bias_dtype == kBF16)
-        hipLaunchKernelGGL((evo_dpair_kernel<128, bf16>), dim3(grid2), dim3(64 * w4), 0, st, p, qblocks, kblocks, per);
-      else
-        hipLaunchKernelGGL((evo_dpair_kernel<128, float>), dim3(grid2), dim3(64 * w4), 0, st, p, qblocks, kblocks, per);
-    } else if (D == 32) {
-      constexpr int lds = 8 * 128 * Tile<32>::RB;
-      e = bias_dtype == kBF16 ? rows(evo_dpair_rows_kernel<32, bf16>, lds) : rows(evo_dpair_rows_kernel<32, float>, lds);
-    } else {
-      constexpr int lds = 8 * 128 * Tile<64>::RB;
-      e = bias_dtype == kBF16 ? rows(evo_dpair_rows_kernel<64, bf16>, lds) : rows(evo_dpair_rows_kernel<64, float>, lds);
-    }
+    auto of_type = [&](auto dim) { return bias_dtype == kBF16 ? pair(dim, bf16{}) : pair(dim, 0.f); };
+    const hipError_t e = D == 32 ? of_type(std::integral_constant<int, 32>{})
+                         : D == 64 ? of_type(std::integral_constant<int, 64>{})
+                                   : of_type(std::integral_constant<int, 128>{});
     if (e != hipSuccess) return e;
     if (bias_dtype == kBF16)
       hipLaunchKernelGGL(evo_pair_sum_kernel<bf16>, dim3((n + 1023) / 1024), dim3(256), 0, st, part, (bf16*)db2, n,

@@ -122,8 +122,8 @@ def test_evoformer_rows_of_one_head(cuda, B, N, L, H, which):
 @pytest.mark.parametrize("B,N,L,D,which", [(1, 9, 2, 32, "both"), (1, 33, 65, 32, "both"), (2, 21, 129, 64, "both"),
                                            (1, 17, 161, 32, "pair"), (1, 13, 256, 64, "both"), (1, 7, 290, 64, "pair")])
 def test_evoformer_pair_gradient_of_shared_rows(cuda, B, N, L, D, which, bias_dtype):
-    """The pair bias' gradient summed over rows staged by a workgroup: one or two waves of keys, the second past the end,
-    queries past the end, several workgroups of either, one and several chunks of rows of which the last is shorter. (Two keys at least: with one, dS is exactly zero and
+    """The pair bias' gradient, of few rows: one or two blocks of keys, the second past the end, queries past the end, several
+    workgroups of either, one and several chunks of rows of which the last is shorter. (Two keys at least: with one, dS is exactly zero and
     a relative bound has nothing to hold against the 2^-24 sum |dO V| that dP and delta may differ by, 1.06e-6 in dQ's
     norm here.)"""
     test_evoformer_edges_hip(cuda, B, N, L, 3, D, which, bias_dtype)
@@ -222,6 +222,24 @@ def test_evoformer_saved_tensors_in_another_order(cuda):
     torch.cuda.synchronize()
     for a, b in zip(torch.autograd.grad(out, (q, k, v), do), want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bias_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,L,H,D,bf16,fp32", [
+    (512, 32, 8, 64, 0, 0), (512, 64, 8, 64, 0, 0), (20, 100, 4, 64, 0, 0), (128, 32, 8, 32, 0, 0), (64, 128, 4, 32, 0, 0),
+    (512, 160, 8, 32, 0, 0), (4, 512, 8, 32, 0, 0), (128, 192, 8, 32, 1, 0), (128, 256, 8, 32, 1, 1), (128, 256, 8, 128, 0, 0),
+    (114, 65, 3, 64, 1, 0), (38, 161, 3, 64, 1, 0), (14, 290, 3, 64, 1, 0), (43, 256, 3, 64, 1, 1), (170, 120, 3, 32, 1, 0),
+    (43, 250, 3, 32, 1, 0), (18, 384, 3, 32, 1, 1), (170, 128, 3, 32, 1, 1)])
+def test_evoformer_pair_gradient_kernels(cuda, N, L, H, D, bf16, fp32, bias_dtype):
+    """Which kernel sums the pair bias' gradient: staged rows want a filled chip and full workgroups. The smaller sizes run: one
+    and two waves of keys, the second past the end, queries past the end, a last chunk of one row."""
+    from hcache_deepspeed_amd.ops import native
+    want = bf16 if bias_dtype == torch.bfloat16 else fp32
+    dt = native.dt(torch.empty(0, dtype=bias_dtype))
+    assert native.kernels().hds_evoformer_pair_staged(1, N, L, H, D, dt) == want
+    if H == 3:
+        test_evoformer_edges_hip(cuda, 1, N, L, H, D, "both", bias_dtype)
 
 
 def test_launch_attributes_are_set_for_the_current_device():
