@@ -1640,14 +1640,21 @@ HDS_EXPORT int hds_attn_fwd(const void* q, const void* k, const void* v, void* o
 // 2^24). One workgroup a CU with walks of at least four steps (64 queries of a head), two with walks of sixteen, which
 // even out the causal blocks. A whole backward, 1 slice -> this: 2 x 509 tokens, 16 / 4 heads 88.6 -> 55.5 us (4: 58.0,
 // 16: 68.0); 1 x 2,048, 32 / 8 283 -> 172 (2: 200, 8: 191); 1 x 4,000, 8 / 1 890 -> 214 (8: 243); 4 x 512, 32 / 8
-// 95.6 -> 81.5 (4: 84.9). Short walks lose what the sums cost: 1 x 100, 16 / 16 21.5, with 2 slices 24.4.
-HDS_EXPORT int hds_attn_bwd_slices(int batch, int max_len, int hq, int hkv, int head_dim) {
+// 95.6 -> 81.5 (4: 84.9). Behind a window a walk ends with it, and the blocks' walks are alike: one workgroup a CU (4,096
+// tokens, 32 / 8 heads, window 128 107 us, with 2 slices 128; 1,024 tokens 63.3 -> 53.4 with 4; 8,192, 8 / 1, window 1,024
+// 331 -> 158 with 4, 172 with 8). A slice has to save what its sums cost, about nine steps where the sums are of a whole chip
+// (1 x 512, 16 / 16 46.4, with 2 slices 52.4; 4 x 1,000, 16 / 4, window 64 60.5 / 63.2; 1,024, 32 / 8, window 64 53.4 / 48.7 with 3).
+HDS_EXPORT int hds_attn_bwd_slices(int batch, int max_len, int hq, int hkv, int head_dim, int causal, int window) {
   if (head_dim != 128 || batch < 1 || max_len < 1 || hkv < 1 || hq < hkv) return 1;
   const int64_t groups = (int64_t)((max_len + 127) / 128) * hkv * batch;
-  const int64_t steps = (int64_t)((max_len + 63) / 64) * (hq / hkv);  // of the longest walk
+  const int64_t tiles = ((int64_t)max_len + 63) / 64, seen = (126 + (int64_t)window) / 64 + 1;
+  const bool ends = causal && window > 0 && seen < tiles;
+  const int64_t steps = (ends ? seen : tiles) * (hq / hkv);  // of the longest walk
   auto fit = [&](int64_t most, int64_t least) { return most / groups < steps / least ? most / groups : steps / least; };
-  int64_t s = fit(256, 4) > fit(512, 16) ? fit(256, 4) : fit(512, 16);
+  int64_t s = fit(256, 4);
+  if (!ends && fit(512, 16) > s) s = fit(512, 16);
   if (s > 16) s = 16;
+  while (s > 1 && 256 * (steps - steps / s) < 9 * groups * s) --s;
   return s < 2 ? 1 : (int)s;
 }
 HDS_EXPORT int hds_attn_bwd_part(int slices, int batch, int max_len, int hkv, int head_dim) {

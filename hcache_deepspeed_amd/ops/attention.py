@@ -105,7 +105,7 @@ def _native_bwd(q, k, v, o, lse, do, dq, dk, dv, causal, scale, cu, B, seq_len, 
     delta = torch.empty(2, Hq, T, device=q.device, dtype=torch.float32)  # rowsum(dO * O), lse * log2(e)
     strides = _strides8(q, k, v, o, do, dq, dk, dv)
     lib, part = native.kernels(), None
-    slices = lib.hds_attn_bwd_slices(B, max_len, Hq, k.shape[1], D)
+    slices = lib.hds_attn_bwd_slices(B, max_len, Hq, k.shape[1], D, int(causal), int(window))
     if slices > 1:  # 32-bit sums of dK and dV
         part = torch.empty(lib.hds_attn_bwd_part(slices, B, max_len, k.shape[1], D), device=q.device, dtype=torch.float32)
     native.check(

@@ -82,7 +82,7 @@ _KERNEL_SIGS = {
     "hds_xent": "i" + "pppp" + "l" + "i" + "l" + "i" + "f" + "i" + "f" + "s",
     "hds_attn_fwd": "p" * 8 + "i" * 7 + "f" + "ii" + "s",
     "hds_attn_bwd": "p" * 13 + "i" * 7 + "f" + "ii" + "pi" + "s",
-    "hds_attn_bwd_slices": "iiiii",
+    "hds_attn_bwd_slices": "iiiiiii",
     "hds_attn_bwd_part": "iiiii",
     "hds_attn_head_dim_supported": "i",
     "hds_attn_config": "iii",

@@ -282,7 +282,7 @@ def test_flash_attn_bwd_slices(lens, Hq, Hkv, causal, window, no_attn_fallback):
     results are rounded to 8 bits, each by at most 2^-9 of itself, and dS is made of outputs that were."""
     from hcache_deepspeed_amd.ops import native
     from hcache_deepspeed_amd.ops.attention import flash_attn
-    assert native.kernels().hds_attn_bwd_slices(len(lens), max(lens), Hq, Hkv, 128) > 1
+    assert native.kernels().hds_attn_bwd_slices(len(lens), max(lens), Hq, Hkv, 128, int(causal), window) > 1
     g = torch.Generator(device="cuda").manual_seed(Hq + len(lens))
     T, cu = sum(lens), torch.tensor([0] + lens).cumsum(0).int()
     rnd = lambda h: torch.randn(T, h, 128, device="cuda", generator=g).bfloat16()  # noqa: E731
@@ -292,6 +292,16 @@ def test_flash_attn_bwd_slices(lens, Hq, Hkv, causal, window, no_attn_fallback):
     _attn_ref(qr, kr, vr, causal, window, cu, None).backward(do.float())
     for x, y in ((q, qr), (k, kr), (v, vr)):
         assert _rel(x.grad, y.grad) < 4 * 2**-8
+
+
+@pytest.mark.parametrize("B,T,Hq,Hkv,window,want", [
+    (1, 4096, 32, 8, 128, 1), (1, 4096, 32, 8, 2048, 1), (1, 8192, 16, 4, 128, 1), (4, 1000, 16, 4, 64, 1), (1, 2048, 8, 8, 256, 1),
+    (1, 512, 16, 16, 0, 1), (2, 600, 8, 8, 0, 1), (1, 100, 16, 16, 0, 1), (1, 4096, 32, 8, 0, 2), (1, 2048, 32, 8, 256, 2),
+    (1, 1024, 32, 8, 64, 3), (1, 8192, 8, 1, 1024, 4), (2, 509, 16, 4, 0, 8), (1, 2048, 16, 4, 2000, 8)])
+def test_attn_bwd_slices_are_worth_their_sums(B, T, Hq, Hkv, window, want):
+    """Steps behind a window are no work to share: walks of few steps, and many of them, stay whole."""
+    from hcache_deepspeed_amd.ops import native
+    assert native.kernels().hds_attn_bwd_slices(B, T, Hq, Hkv, 128, 1, window) == want
 
 
 @pytest.mark.parametrize("D", [64, 128])
