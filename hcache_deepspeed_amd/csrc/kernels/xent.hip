@@ -98,16 +98,18 @@ template <typename T>
 __global__ __launch_bounds__(256) void scaled_grad_kernel(const float* __restrict__ x, const float* __restrict__ scale,
                                                           T* __restrict__ out, int64_t n, int accumulate) {
   const float s = *scale;
-  const int64_t i = (int64_t)blockIdx.x * 1024 + 4 * threadIdx.x;
-  if (i + 4 <= n) {
-    float v[4], o[4];
-    load4_nt(x + i, v);
-    if (accumulate) load4_nt(out + i, o);
+  for (int64_t b = blockIdx.x; b * 1024 < n; b += gridDim.x) {
+    const int64_t i = b * 1024 + 4 * threadIdx.x;
+    if (i + 4 <= n) {
+      float v[4], o[4];
+      load4_nt(x + i, v);
+      if (accumulate) load4_nt(out + i, o);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = accumulate ? o[j] + v[j] * s : v[j] * s;
-    store4_nt(out + i, v);
-  } else {
-    for (int64_t k = i; k < n; ++k) out[k] = from_f<T>(accumulate ? to_f(out[k]) + x[k] * s : x[k] * s);
+      for (int j = 0; j < 4; ++j) v[j] = accumulate ? o[j] + v[j] * s : v[j] * s;
+      store4_nt(out + i, v);
+    } else {
+      for (int64_t k = i; k < n; ++k) out[k] = from_f<T>(accumulate ? to_f(out[k]) + x[k] * s : x[k] * s);
+    }
   }
 }
 
@@ -117,8 +119,7 @@ __global__ __launch_bounds__(256) void scaled_grad_kernel(const float* __restric
 HDS_EXPORT int hds_scaled_grad(int dtype, const float* x, const float* scale, void* out, int64_t n, int accumulate,
                                hipStream_t st) {
   if (n <= 0) return 0;
-  if (n > (int64_t)1024 * 0x7fffffff) return hipErrorInvalidValue;
-  dim3 grid((n + 1023) / 1024), block(256);
+  dim3 grid(stream_grid(n, 1024, 1 << 23)), block(256);  // (a launch has fewer than 2^32 threads)
   if (dtype == kBF16)
     hipLaunchKernelGGL(scaled_grad_kernel<bf16>, grid, block, 0, st, x, scale, (bf16*)out, n, accumulate);
   else if (dtype == kF32)

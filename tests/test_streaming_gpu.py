@@ -66,3 +66,20 @@ def test_scaled_grad(n, dtype, accumulate):
     _scaled_grad_(out, x, scale, accumulate)
     eps = {BF16: 2**-8, torch.float16: 2**-11, torch.float32: 2**-22}[dtype]
     torch.testing.assert_close(out.double(), want, rtol=eps, atol=1e-6)
+
+
+def test_scaled_grad_of_more_threads_than_a_launch_has():
+    """A launch has fewer than 2^32 threads: with four elements a thread, gradients of 2^34 and more go round again."""
+    from hcache_deepspeed_amd.ops.cross_entropy import _scaled_grad_
+    n = 2**34 + 1027
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 7 * n:
+        pytest.skip("needs 120 GB")
+    x, out = torch.ones(n, device="cuda"), torch.zeros(n, device="cuda", dtype=BF16)
+    x[-1], x[0], x[2**33] = 5.0, 3.0, 2.0
+    _scaled_grad_(out, x, torch.tensor([0.5], device="cuda"), False)
+    assert [out[i].item() for i in (0, 1, 2**33, 2**33 + 1, n - 2, n - 1)] == [1.5, 0.5, 1.0, 0.5, 0.5, 2.5]
+    whole = all((c == 0.5).sum().item() >= c.numel() - 2 for c in out.split(2**31))
+    del x, out
+    torch.cuda.empty_cache()
+    assert whole
