@@ -312,11 +312,11 @@ __global__ __launch_bounds__(512) void gg_big_kernel(const bf16* __restrict__ x,
 // way at any time, waited for with a count, one barrier a step. (Twelve or sixteen chunks are level, and so are fragments read
 // a step ahead.) Waves: WR / 64 along the weight rows, the others along the tokens. Each XCD takes a contiguous range of the
 // real tiles (expert after expert), so that the workgroups of one expert share its rows in one L2.
-// 128 weight rows and three stages of 48 KB -> this, gate and up / down, us: 64 experts, 6 a token, 1024 x 2048, 66 / 700 / 1,600
-// / 3,000 tokens 121 + 44 / 126 + 71 / 153 + 95 / 265 + 147 -> 96 + 44 / 104 + 63 / 132 + 89 / 254 + 142; 64 experts, 4 a token, 2048
-// x 4096, 66 / 1,500 tokens 361 + 174 / 480 + 244 -> 349 + 176 / 430 + 220; 8 experts, 2 a token, 14336 x 4096, 66 / 500 / 1,700
-// tokens 322 + 163 / 463 + 222 / 1,125 + 538 -> 321 + 159 / 463 + 230 / 1,035 + 502; 5632 x 2048, 66 / 500 / 1,400 tokens 87 + 37 /
-// 108 + 76 / 243 + 102 -> 73 + 42 / 110 + 61 / 204 + 101.
+// 128 weight rows and three stages of 48 KB -> this, gate and up + down, us, weights not in the caches: 64 experts, 6 a token,
+// 1024 x 2048, 66 / 700 / 1,600 / 3,000 tokens 125 + 54 / 125 + 63 / 153 + 85 / 247 + 141 -> 98 + 54 / 104 + 62 / 132 + 80 / 234 +
+// 141; 64 experts, 4 a token, 2048 x 4096, 66 / 1,500 tokens 366 + 184 / 435 + 231 -> 351 + 183 / 394 + 216; 8 experts, 2 a token,
+// 14336 x 4096, 66 / 500 / 1,000 tokens 332 + 165 / 450 + 214 / 760 + 473 -> 326 + 159 / 424 + 221 / 690 + 415; 5632 x 2048, 66 / 500 /
+// 1,400 tokens 84 + 55 / 105 + 75 / 217 + 100 -> 78 + 43 / 109 + 60 / 195 + 104.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int kChunk = 64 * 128, kRing = 20;
 // operand of s_waitcnt: no LDS access and at most n loads on their way
@@ -498,6 +498,52 @@ HDS_EXPORT int hds_grouped_gemm(const void* x, const void* w, void* y, const int
 // Rows of a tile of hds_experts_gemm's tile list
 HDS_EXPORT int hds_experts_gemm_tile() { return BM2; }
 
+// gg_flow_kernel's weight rows a tile, and whether its workgroups' walks along K begin apart
+struct FlowTile {
+  int rows, apart;
+};
+static FlowTile flow_tile(int T, int N, int K, int E, int glu) {
+  // The tile of weight rows with which the rounds over the CUs take least; a round of 64, 128 and 256 weight rows
+  // takes about 3, 4 and 6 parts (one round of [2048, 5632]: 41.5 / 44.7 / 57 us at 66 tokens, 60 / 77 / 118 at 500), the last 7
+  // where an expert has few or very many rows (16 experts, 4 a token, 6400 x 4096, 66 tokens: 322 us with 256, 308 with 128; one
+  // round of [3072, 8192], 1,000 tokens 238 / 147). Experts are taken to be alike within 20 rows: near 256 only some have a
+  // second tile (6400 x 4096, 1,000 tokens, down: 386 / 353). One that has it costs 64 weight rows, which fill the chip
+  // without room, a whole round (8 experts, 2 a token, 5632 x 2048, 900 tokens, down: 73 us without one, 128 with; 128 weight rows
+  // 91 and 92).
+  const int cols_of = glu ? 2 : 1, avg = (int)(((int64_t)T + E - 1) / E);
+  int part = 40;  // tiles of an expert, in 40ths
+  for (int m = BM2; m < avg + 20; m += BM2) part += std::min(40, avg + 20 - m);
+  const int64_t tiles = (int64_t)std::min(E, T) * part / 40;
+  int wr = 64;
+  int64_t least = 0;
+  for (int r = 64; r <= 256; r *= 2) {
+    const int64_t groups = (tiles + (r == 64 && avg > 216)) * (N / (r / cols_of));
+    const int64_t cost = (groups + 255) / 256 * (r == 256 && (avg <= 64 || avg > 192) ? 7 : r / 64 + 2);
+    if (N % (r / cols_of) == 0 && (r == 64 || cost < least)) {
+      wr = r;
+      least = cost;
+    }
+  }
+  // Weight rows a multiple of 4 KB apart lie alike in the memory's channels, and workgroups that walk them side by side
+  // meet in the same ones: there each begins its walk along K somewhere else. It helps single rounds, whose workgroups stay in
+  // step ([4096, 14336], 66 tokens 184 -> 161 us, [4096, 4096] of 16 experts 121 -> 91, 1,000 tokens 136 -> 120, gate and up
+  // of 4 experts, 8192 x 4096 130 -> 103), and gate and up rows of an odd number of 4 KB, which are two such walks a workgroup (1024
+  // x 2048, 66 tokens 123 -> 96, 1,600 147 -> 135). Several rounds or many rows share in L2 what it takes apart: there only
+  // down rows of few tokens ([4096, 2048] of 64 experts, 200 tokens 193 -> 186; of 32, K = 4096, 300 tokens 196 -> 186) and gate
+  // and up in 128 weight rows (14336 x 4096, 66 tokens 328 -> 323) gain, others lose ([28672, 4096] 351 -> 386, 1024 x 2048, 3,000 tokens 244
+  // -> 275, [4096, 8192], 1,000 tokens 219 -> 236).
+  const int64_t rounds = (tiles * (N / (wr / cols_of)) + 255) / 256;
+  const bool one = rounds == 1 && avg <= (K % 8192 ? 192 : 96);
+  const bool more = glu ? (K / 2048 % 2 && avg <= 192) || (wr == 128 && avg <= 64) : avg <= 64;
+  return {wr, K % 2048 == 0 && (one || more)};
+}
+// the same as one number, rows + apart
+HDS_EXPORT int hds_experts_gemm_rows(int T, int N, int K, int E, int glu) {
+  if (T <= 0 || E <= 0) return 0;
+  const FlowTile t = flow_tile(T, N, K, E, glu);
+  return t.rows + t.apart;
+}
+
 // Grouped product of sorted rows with a ready tile list (hds_experts_gemm_tile rows a tile; at most
 // max_tiles entries, the number on the device). src: row of x [n_src, ldx] for every sorted row, or null: x is sorted.
 // glu: w [E, 2N, K] is gate rows then up rows and y = silu(gate) * up, or the clamped unit with its limit (act 5); weight [T]
@@ -514,27 +560,10 @@ HDS_EXPORT int hds_experts_gemm(const void* x, int64_t ldx, const int* src, int 
   // experts, 2 a token, 14336 x 4096: 1,500 tokens 1,774 us against 1,534 here, 2,000 2,063 / 2,054, 2,700 2,390 / 2,488; 64
   // experts, 6 a token, 1024 x 2048: 3,000 540 / 427, 6,000 786 / 733, 12,000 1,262 / 1,315.
   const bool big = N % big_cols == 0 && T >= 2 * BM2 * E;
-  // Otherwise the tile of weight rows with which the rounds over the CUs take least; a round of 64, 128 and 256 weight rows
-  // takes about 3, 4 and 6 parts (one round of [2048, 5632]: 41.5 / 44.7 / 57 us at 66 tokens, 60 / 77 / 118 at 500). Experts
-  // are taken to be alike.
-  const int cols_of = glu ? 2 : 1, avg = T / E + 1;
-  const int64_t tiles = (int64_t)std::min(E, T) * ((avg + avg / 8 + BM2 - 1) / BM2);
-  int wr = 64;
-  int64_t least = 0;
-  for (int r = 64; r <= 256; r *= 2) {
-    const int64_t cost = (tiles * (N / (r / cols_of)) + 255) / 256 * (r / 64 + 2);
-    if (N % (r / cols_of) == 0 && (r == 64 || cost < least)) {
-      wr = r;
-      least = cost;
-    }
-  }
-  // Weight rows an odd multiple of 4 KB apart lie alike in the memory's channels, and workgroups that walk them side by side
-  // meet in the same ones: there each begins its walk along K somewhere else. It helps gate and up rows, which are two such
-  // walks a workgroup (1024 x 2048, 66 tokens 123 -> 96 us, 1,600 147 -> 135; 3,000, with two tiles an expert, 244 -> 275),
-  // and single rounds, whose workgroups stay in step ([4096, 14336], 66 tokens 175 -> 160); over several rounds ([4096, 2048],
-  // 200 tokens 180 -> 192) and with rows of 8 KB ([28672, 4096] 351 -> 386) it costs what is shared in L2.
-  const int apart = K % 2048 == 0 && K / 2048 % 2 && avg <= 192 && (glu || tiles * (N / wr) <= 256);
-  const int cols = big ? big_cols : wr / cols_of;
+  // otherwise gg_flow_kernel's tiles
+  const FlowTile flow = flow_tile(T, N, K, E, glu);
+  const int wr = flow.rows, apart = flow.apart;
+  const int cols = big ? big_cols : wr / (glu ? 2 : 1);
   if (N % cols || K % BK || ldx < K || ldx % 8 || ldy < N || ldy % 8 || max_tiles < 1 || max_tiles > 65535 ||
       (src != nullptr && n_src < 1) || (act != 0 && act != 5) || (int64_t)(N / cols) * max_tiles > INT32_MAX)
     return hipErrorInvalidValue;

@@ -50,6 +50,7 @@ _KERNEL_SIGS = {
     "hds_experts_skinny": "i" + "pl" + "p" + "pl" + "p" + "iiiii" + "pl" + "p" + "pl" + "iii" + "i" + "f" + "p" + "s",
     "hds_experts_gemm_f32": "pl" + "p" + "pl" + "ppppp" + "i" + "p" + "iii" + "s",
     "hds_experts_gemm_tile": "",
+    "hds_experts_gemm_rows": "iiiii",
     "hds_experts_gemm": "pl" + "pi" + "pp" + "i" + "pppp" + "iiiiii" + "i" + "f" + "p" + "s",
     "hds_norm_rows": "i" + "pppp" + "i" + "p" + "ii" + "f" + "s",
     "hds_gated_scan": "i" + "pl" + "pp" + "pl" + "pl" + "pp" + "iii" + "s",

@@ -147,11 +147,25 @@ def test_experts_gemm_hip(cuda, counts, N, K, gather, glu):
 @pytest.mark.gpu
 @pytest.mark.parametrize("counts", [[129, 192, 193, 3], [64, 1, 256, 65]])
 @pytest.mark.parametrize("N,K,gather,glu", [(4096, 128, True, True), (8192, 384, False, True), (16384, 128, True, False),
-                                            (8192, 256, False, False), (4096, 2048, True, True), (8192, 2048, False, False)])
+                                            (8192, 256, False, False), (4096, 2048, True, True), (8192, 2048, False, False),
+                                            (1024, 4096, False, False), (512, 4096, True, True)])
 def test_experts_gemm_tiles_of_weight_rows(cuda, counts, N, K, gather, glu):
     """128 and 256 weight rows a tile, which many rounds choose, with one to four blocks of 64 rows; fewer steps than the ring
     holds; walks along K that begin apart."""
     test_experts_gemm_hip(cuda, counts, N, K, gather, glu)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,k,T,N,K,glu,rows,apart", [
+    (8, 2, 66, 14336, 4096, 1, 128, 1), (8, 2, 300, 14336, 4096, 1, 256, 0), (16, 4, 66, 6400, 4096, 1, 128, 1),
+    (4, 1, 66, 8192, 4096, 1, 256, 1), (64, 6, 66, 1024, 2048, 1, 256, 1), (64, 6, 3000, 1024, 2048, 1, 256, 0),
+    (8, 2, 66, 2048, 5632, 0, 64, 0), (8, 2, 900, 2048, 5632, 0, 128, 0), (8, 2, 1000, 3072, 8192, 0, 128, 0),
+    (16, 4, 1000, 4096, 6400, 0, 128, 0), (16, 2, 66, 4096, 4096, 0, 256, 1), (16, 2, 1000, 4096, 8192, 0, 256, 0),
+    (64, 4, 200, 4096, 2048, 0, 256, 1), (64, 4, 1500, 4096, 2048, 0, 256, 0), (2, 1, 10, 96, 128, 0, 64, 0)])
+def test_experts_gemm_choice_of_tiles(E, k, T, N, K, glu, rows, apart):
+    """Tiles by rounds over the chip, with room for an expert that has a second one; walks apart in single rounds."""
+    from hcache_deepspeed_amd.ops import native
+    assert native.kernels().hds_experts_gemm_rows(T * k, N, K, E, glu) == rows + apart
 
 
 def test_counted_waits_retire_lds_reads():
