@@ -497,7 +497,7 @@ __global__ __launch_bounds__(64 * NW) void wmix_lines_kernel(const bf16* __restr
 }
 
 // Many weight rows of up to 4,096 k: workgroups that stay on their CU. Wave w of RW holds run w of A in registers, in the
-// operands' layout, and walks over the workgroup's tiles; it loads whole lines as above, two tiles ahead.
+// operands' layout, and walks over the workgroup's tiles; it loads whole lines as above, a tile ahead.
 constexpr int kResWaves = 8;
 
 template <int FMT, int E, int RW, bool GLU>
@@ -674,14 +674,21 @@ HDS_EXPORT int hds_wmix_skinny(const void* A, const void* W, const float* scales
     return hipGetLastError();
   };
   const bool res = hds_wmix_resident(M, glu ? 2 * N : N, K);
-  // Whole lines pay where a wave walks far: 8 rows, fp6 [2048, 2048] 4.8 us against 4.9, [11264, 2048] gated 10.3 / 10.1; int8
-  // [4096, 4096] 8.7 / 8.6, [6144, 4096] 12.1 / 12.5, [2048, 5632] 8.2 / 8.7; int4 [4096, 4096] 6.5 / 6.2, [2048, 5632] 7.3 / 7.1,
-  // [4096, 14336] 14.3 / 15.7. From nine rows on the wider codes lose (int8 [4096, 14336], 16 rows, 24.7 / 23.8) and fp6 gains
-  // where a CU's one workgroup is not followed by another or is long ([6144, 4096] 14.8 / 14.6, [5120, 13824] 37.9 / 47.2).
-  const bool lines = K > (fmt == 2 ? 2048 : fmt == 0 ? 4096 : 8192);
+  // Whole lines pay where a wave walks far: 8 rows, fp6 [2048, 2048] 4.8 us against 4.9, [11264, 2048] gated 10.3 / 10.1,
+  // [16384, 7168] 26.3 (with A resident in LDS 27.5), [27648, 5120] gated 35.1 (34.6); int8 [4096, 4096] 8.7 / 8.6, [6144, 4096]
+  // 12.1 / 12.5, [2048, 5632] 8.2 / 8.7; int4 [4096, 4096] 6.5 / 6.2, [2048, 5632] 7.3 / 7.1, [4096, 14336] 14.3 / 15.7, and with
+  // many weight rows from 4,096 k on ([20480, 5120], 4 / 8 rows 25.0 / 27.1, without 26.5 / 29.6; 2 rows [18432, 7168] 28.9 / 26.9).
+  const bool lines = K > (fmt == 2 ? 2048 : fmt == 0 ? 4096 : 8192) || (fmt == 1 && K > 4096 && tiles >= 1024 && M > 2);
+  // From nine rows on the wider codes lose (int8 [4096, 14336], 16 rows, 24.7 / 23.8) and fp6 gains where a CU's one workgroup
+  // is not followed by another or is long ([6144, 4096] 14.8 / 14.6, [5120, 13824] 37.9 / 47.2), but up to 6,144 k of many
+  // weight rows the last round has to be full ([22016, 6144] gated 51.1 / 47.3, [20480, 5120] 37.4 / 40.7).
+  const int rounds = (tiles + 255) / 256;
+  const bool lines16 = lines && (tiles <= 256 || K > 6144 || (K > 4096 && (tiles < 1024 || tiles >= 240 * rounds)));
   // From nine rows on two tiles of weight rows share what is read of A ([28672, 4096], 16 rows: fp6 48 -> 41 us), where
-  // enough workgroups remain. Short sums on many rows: four waves a workgroup, otherwise eight ([4096, 14336] fp6, 8 rows 27
-  // -> 22 us).
+  // enough workgroups remain. int4 with the registers of two waves a SIMD where a third would save no round ([27648, 5120]
+  // gated, 12 / 16 rows 41.6 / 44.4 -> 37.2 / 39.5; [22016, 6144] gated 30.9 / 34.6). Short sums on many rows: four waves a
+  // workgroup, otherwise eight ([4096, 14336] fp6, 8 rows 27 -> 22 us).
+  const bool two = ((tiles + 1) / 2 + 511) / 512 == ((tiles + 1) / 2 + 767) / 768;
 #define HDS_WS(F, E, GL)                                                                                            \
   do {                                                                                                              \
     if (res && K > 2048) return resident(wmix_resident_kernel<F, E, 8, GL>, 8);                                     \
@@ -689,7 +696,9 @@ HDS_EXPORT int hds_wmix_skinny(const void* A, const void* W, const float* scales
     if (lines && M <= 8 && tiles > 256) return launch(wmix_lines_kernel<F, E, 8, 4, GL>, 1, 4);                     \
     if (lines && M <= 8) return launch(wmix_lines_kernel<F, E, 8, 8, GL>, 1, 8);                                    \
     if constexpr (F == kFp6)                                                                                        \
-      if (lines && M <= 16 && (K > 4096 || tiles <= 256)) return launch(wmix_lines_kernel<F, E, 16, 6, GL>, 1, 6);  \
+      if (lines16 && M <= 16) return launch(wmix_lines_kernel<F, E, 16, 6, GL>, 1, 6);                              \
+    if constexpr (F == kInt4)                                                                                       \
+      if (M > 8 && tiles >= 2 * 512 && two) return launch(wmix_skinny_kernel<F, E, 2, 1, 4, 2, GL>, 2, 4);          \
     if (M > 8 && M <= 16 && tiles >= 2 * 512) return launch(wmix_skinny_kernel<F, E, 2, 1, 4, 3, GL>, 2, 4);        \
     if (M <= 16 && K <= 4096 && tiles >= 384) return launch(wmix_skinny_kernel<F, E, 1, 1, 4, 1, GL>, 1, 4);        \
     if (M <= 16) return launch(wmix_skinny_kernel<F, E, 1, 1, 8, 1, GL>, 1, 8);                                     \

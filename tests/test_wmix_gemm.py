@@ -90,10 +90,11 @@ def test_few_rows_keep_the_weights_exact(fmt, M, N, K, G):
 @pytest.mark.parametrize("fmt,M,N,K", [
     ("fp6_e3m2", 1, 4090, 2176), ("fp6_e2m3", 8, 4200, 4224), ("fp6_e3m2", 9, 4000, 2176), ("fp6_e3m2", 16, 5000, 4352),
     ("int8", 3, 4096, 4224), ("int8", 8, 4112, 4608), ("int4", 1, 4096, 14336), ("int4", 7, 5000, 8320), ("int8", 1, 16400, 2176),
-    ("int8", 16, 20500, 4096), ("int4", 16, 32790, 1920), ("fp6_e3m2", 5, 16390, 2176), ("int4", 2, 16384, 3200)])
+    ("int8", 16, 20500, 4096), ("int4", 16, 32790, 1920), ("fp6_e3m2", 5, 16390, 2176), ("int4", 2, 16384, 3200), ("int4", 5, 16390, 4224),
+    ("int4", 16, 16380, 4224), ("int4", 9, 16400, 4224), ("fp6_e3m2", 12, 16400, 4224), ("fp6_e2m3", 9, 19300, 4224)])
 def test_whole_lines_of_packed_weights(fmt, M, N, K):
     """The kernels that load whole lines, to the stream's bound: walks that end inside a run of 512 or leave waves without one,
-    four, six and eight waves, partial tiles, one to three rounds of resident rows; packed weights 8 bytes off a line."""
+    four, six and eight waves, partial tiles, one to three rounds of resident rows, many weight rows beside them; packed weights 8 bytes off a line."""
     torch.manual_seed(K + M)
     x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
     w = torch.randn(N, K, device="cuda", dtype=torch.bfloat16) * 0.05
