@@ -76,12 +76,17 @@ def transpose2d(x, variant=None):
     return out
 
 
+def _pads(x):
+    """Does ``transpose2d_padded`` take x?"""
+    return (native.use_native(x) and x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and x.shape[0] > 0 and x.shape[1] > 0)
+
+
 def transpose2d_padded(x):
     """[R, C] (unit last stride) -> [C, R rounded up to a multiple of 64], zeros behind the R columns, by the HIP kernel; None
     where it does not apply. Rows of a transpose that are no multiple of 16 bytes cost the GEMM its fast loads."""
     R, C = x.shape
-    if not (native.use_native(x) and x.dtype == torch.bfloat16 and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and x.data_ptr() % 16 == 0 and R and C):
+    if not _pads(x):
         return None
     out = torch.empty(C, -(-R // 64) * 64, dtype=x.dtype, device=x.device)
     if out.data_ptr() % 128:
@@ -147,7 +152,7 @@ def _wgrad_run(layout, dy2, x2, out, accumulate, dyt=None, xt=None):
     base, sk2, b2 = layout.split("_")[0], layout.endswith("_sk2"), layout.endswith("_b2")
     if base == "nt":  # hipBLASLt's NT form on transposed copies (the forward GEMM's fast layout)
         a = b = None
-        if dyt is None and xt is None and dy2.shape[0] % 8:  # odd token counts: both operands padded alike
+        if dyt is None and xt is None and dy2.shape[0] % 8 and _pads(dy2) and _pads(x2):  # odd token counts: both padded alike
             a = transpose2d_padded(dy2)
             b = transpose2d_padded(x2) if a is not None else None
         if b is None:
@@ -225,7 +230,7 @@ def wgrad(dy2, x2, out, accumulate=False, dyt=None, xt=None):
     """out[N, K] (+)= dy2[T, N]^T @ x2[T, K] with the fastest layout for this shape: the TN GEMM autograd issues
     (``direct``), two HBM-rate HIP transposes + the NT GEMM (``nt``), or either as one batched GEMM over the two
     token halves (``_b2``, shapes whose tile grid ends in a half-empty wave). ``HDS_WGRAD_LAYOUT=auto`` times the
-    candidates once per (shape, dtype, accumulate, pre-transposed operands) on the first call
+    candidates once per (shape, dtype, accumulate, pre-transposed operands, odd token count) on the first call
     (profiles/wgrad_layout_r2.log: NT runs 1.44-1.47 PF/s where TN runs 0.94-1.10 at the o / gate_up shapes).
     ``dyt`` [N, T] / ``xt`` [K, T]: transposes the producers already wrote (glu, runtime/zero/linear.py); with
     ``x2`` None only the NT forms are possible."""
@@ -237,7 +242,8 @@ def wgrad(dy2, x2, out, accumulate=False, dyt=None, xt=None):
                 and dy2.stride(1) == 1 and (x2 is None or x2.stride(1) == 1)):
             layout = "direct" if x2 is not None else "nt"
         else:
-            key = (_rows_bucket(T), N, K, out.dtype, bool(accumulate), x2 is None, dyt is not None)
+            # (odd token counts run other transposes, see _wgrad_run)
+            key = (_rows_bucket(T), N, K, out.dtype, bool(accumulate), x2 is None, dyt is not None, T % 8 != 0)
             layout = _WGRAD_CHOICE.get(key)
             if layout is None:
                 b2 = ("_b2", ) if _b2_useful(N, K) else ()

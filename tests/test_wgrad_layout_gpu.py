@@ -129,3 +129,33 @@ def test_zero_linear_saves_transposed_input():
     torch.nn.functional.linear(x2, w2).backward(dy.float())
     for a, b in ((w.grad, w2.grad), (x.grad, x2.grad)):
         assert (a.float() - b).abs().max().item() <= 2e-2 * b.abs().max().item()
+
+
+def test_odd_token_counts_choose_their_own_layout(monkeypatch):
+    """Odd token counts run other transposes than multiples of 8 of the same bucket: each is timed once."""
+    from hcache_deepspeed_amd.ops import gemm
+    monkeypatch.setattr(gemm, "_WGRAD_LAYOUT", "auto")
+    monkeypatch.setattr(gemm, "_WGRAD_CHOICE", {})
+    monkeypatch.setattr(gemm, "_NT_BY_N", {})
+    timed = []
+    monkeypatch.setattr(gemm, "_time_layout", lambda layout, dy2, *a: timed.append((layout, dy2.shape[0])) or
+                        (1.0 if (layout == "nt") == (dy2.shape[0] % 8 == 0) else 2.0))
+    ran = []
+    run = gemm._wgrad_run
+    monkeypatch.setattr(gemm, "_wgrad_run", lambda layout, *a: ran.append(layout) or run(layout, *a))
+    out = torch.empty(72, 64, device="cuda", dtype=torch.bfloat16)
+    for T in (1018, 1024, 1017, 1000):
+        gemm.wgrad(torch.randn(T, 72, device="cuda").bfloat16(), torch.randn(T, 64, device="cuda").bfloat16(), out)
+    assert ran == ["direct", "nt", "direct", "nt"] and {t for _, t in timed} == {1018, 1024}
+
+
+def test_one_operand_that_does_not_pad(monkeypatch):
+    """Neither operand is padded where one cannot be: no transpose is made and thrown away."""
+    from hcache_deepspeed_amd.ops import gemm
+    made = []
+    monkeypatch.setattr(gemm, "transpose2d_padded", lambda x: made.append(x))
+    dy, x = torch.randn(57, 64, device="cuda").bfloat16(), torch.randn(57, 68, device="cuda").bfloat16()[:, 2:66]
+    out = torch.empty(64, 64, device="cuda", dtype=torch.bfloat16)
+    gemm._wgrad_run("nt", dy, x, out, False)
+    ref, mag = dy.double().t() @ x.double(), dy.double().abs().t() @ x.double().abs()
+    assert not made and ((out.double() - ref).abs() <= 2**-8 * ref.abs() + 2**-20 * mag).all()
