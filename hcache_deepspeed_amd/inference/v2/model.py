@@ -357,7 +357,7 @@ class RaggedTransformer:
             return False
         S = batch.current_sequences
         return (batch.logits_of_last_tokens and 0 < S <= self.decode_graph_max_batch and batch.current_tokens == S
-                and getattr(batch, "atoms", None) is not None and getattr(batch, "_dev_meta", None) is not None)
+                and getattr(batch, "n_atoms", None) is not None and getattr(batch, "_dev_meta", None) is not None)
 
     @torch.no_grad()
     def forward_decode_graph(self, batch, capture_latents=False):

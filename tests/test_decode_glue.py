@@ -139,6 +139,30 @@ def test_step_description_of_any_tokens():
             b.finalize(100)
 
 
+def test_a_step_that_may_replay_makes_no_views():
+    """Whether a decode step can replay its graph is known without a view of the step's buffer."""
+    import types
+    from hcache_deepspeed_amd.inference.v2.model import RaggedTransformer
+    from hcache_deepspeed_amd.inference.v2.ragged import (BlockedKVCache, DSStateManager, DSStateManagerConfig,
+                                                          RaggedBatchWrapper)
+    cfg = DSStateManagerConfig(max_context=256)
+    sm = DSStateManager(cfg, BlockedKVCache(1, 2, 16, 64, torch.float32, torch.device("cpu"), cfg.memory_config, num_blocks=8))
+    b = RaggedBatchWrapper(cfg, torch.device("cpu"), sm.max_blocks_per_seq)
+    model = types.SimpleNamespace(device=torch.device("cuda"), tp=1, decode_graph_max_batch=4, decode_graph_latents=True,
+                                  spec=types.SimpleNamespace(moe=None), layers=[])
+    assert not RaggedTransformer.decode_graph_eligible(model, b, False)
+    for geometry in (False, True):
+        b.clear()
+        seq = sm.get_or_create_sequence(0)
+        sm.maybe_allocate_kv(seq, 1)
+        b.insert_sequence(seq, torch.tensor([3]))
+        if geometry:
+            b.set_attention_geometry(4, 2, 128)
+        b.finalize(100)
+        assert RaggedTransformer.decode_graph_eligible(model, b, False) == geometry
+    assert not set(b.__dict__) & set(b._layout)
+
+
 def test_staging_buffers_outlive_their_copies():
     """A wrapper that is dropped while its step's copy is queued: the pinned buffers stay until their events have passed."""
     import gc
