@@ -14,15 +14,10 @@
 //   [3S+2T, 4S+2T)          last      index of each sequence's last token (logits rows)
 //   [4S+2T, 4S+2T+S*MB)     tables    KV block ids per sequence, MB = max_blocks columns, zero padded
 //   [..., + 3A)             atoms     (seq, kv_head, row_start) with rows = n_new * (n_q / n_kv) per (seq, kv head)
-// Returns A, or -1 when `cap` is too small (the required size is then written to *need).
 #include <cstdint>
 #include <cstring>
 
 #define HDS_EXPORT extern "C" __attribute__((visibility("default")))
-
-HDS_EXPORT int64_t hds_ragged_meta_size(int n_seqs, int64_t n_tokens, int max_blocks, int64_t n_atoms) {
-  return 4LL * n_seqs + 2LL * n_tokens + (int64_t)n_seqs * max_blocks + 3LL * n_atoms;
-}
 
 namespace {
 
@@ -32,23 +27,26 @@ struct Seq {
   int64_t n_blocks;
 };
 
+Seq seq_of(const int64_t* seqs, int s) {
+  const int64_t* q = seqs + 5 * (int64_t)s;
+  return Seq{(int32_t)q[1], (int32_t)q[2], reinterpret_cast<const int32_t*>(q[3]), q[4]};
+}
+
 struct Counts {
   int64_t tokens, atoms;
 };
 
-template <typename At>
-Counts count(const At& at, int n_seqs, int n_q, int n_kv, int rows_per_atom) {
+Counts count(const int64_t* seqs, int n_seqs, int n_q, int n_kv, int rows_per_atom) {
   Counts c{0, 0};
   for (int s = 0; s < n_seqs; ++s) {
-    const int64_t n = at(s).n_new;
+    const int64_t n = seq_of(seqs, s).n_new;
     c.tokens += n;
     c.atoms += (int64_t)n_kv * ((n * (n_q / n_kv) + rows_per_atom - 1) / rows_per_atom);
   }
   return c;
 }
 
-template <typename At>
-void build(const At& at, int n_seqs, int64_t T, int max_blocks, int n_q, int n_kv, int rows_per_atom, int32_t* out) {
+void build(const int64_t* seqs, int n_seqs, int64_t T, int max_blocks, int n_q, int n_kv, int rows_per_atom, int32_t* out) {
   const int G = n_q / n_kv;
   int32_t* meta = out;
   int32_t* tok_seq = meta + 3LL * n_seqs;
@@ -58,7 +56,7 @@ void build(const At& at, int n_seqs, int64_t T, int max_blocks, int n_q, int n_k
   int32_t* atoms = tables + (int64_t)n_seqs * max_blocks;
   int64_t q0 = 0, a = 0;
   for (int s = 0; s < n_seqs; ++s) {
-    const Seq q = at(s);
+    const Seq q = seq_of(seqs, s);
     const int32_t n = q.n_new, sn = q.seen;
     meta[3 * s] = (int32_t)q0;
     meta[3 * s + 1] = n;
@@ -86,19 +84,6 @@ void build(const At& at, int n_seqs, int64_t T, int max_blocks, int n_q, int n_k
 
 }  // namespace
 
-HDS_EXPORT int64_t hds_ragged_meta_build(const int32_t* n_new, const int32_t* seen, int n_seqs,
-                                         const int32_t* blocks, const int64_t* block_off, int max_blocks, int n_q,
-                                         int n_kv, int rows_per_atom, int32_t* out, int64_t cap, int64_t* need) {
-  if (n_seqs < 0 || n_kv <= 0 || n_q % n_kv != 0 || rows_per_atom <= 0 || max_blocks < 0) return -2;
-  auto at = [&](int s) { return Seq{n_new[s], seen[s], blocks + block_off[s], block_off[s + 1] - block_off[s]}; };
-  const Counts c = count(at, n_seqs, n_q, n_kv, rows_per_atom);
-  const int64_t size = hds_ragged_meta_size(n_seqs, c.tokens, max_blocks, c.atoms);
-  if (need) *need = size;
-  if (size > cap) return -1;
-  build(at, n_seqs, c.tokens, max_blocks, n_q, n_kv, rows_per_atom, out);
-  return c.atoms;
-}
-
 // A whole step in one call, from the sequences' own buffers: the 64-bit token ids, the layout above and `n_extra` further values
 // go to `out` (8-byte aligned) one behind the other. seqs [n_seqs][5]: address of the tokens (int64), their number, tokens
 // seen, address of the KV blocks (int32), their number. id_limit: ids must lie in [0, id_limit) (0: any). info: ints needed,
@@ -107,12 +92,8 @@ HDS_EXPORT int64_t hds_ragged_step_build(const int64_t* seqs, int n_seqs, int ma
                                          int rows_per_atom, int64_t id_limit, const int32_t* extra, int64_t n_extra,
                                          int32_t* out, int64_t cap, int64_t* info) {
   if (n_seqs < 0 || n_kv <= 0 || n_q % n_kv != 0 || rows_per_atom <= 0 || max_blocks < 0 || n_extra < 0) return -2;
-  auto at = [&](int s) {
-    const int64_t* q = seqs + 5 * (int64_t)s;
-    return Seq{(int32_t)q[1], (int32_t)q[2], reinterpret_cast<const int32_t*>(q[3]), q[4]};
-  };
-  const Counts c = count(at, n_seqs, n_q, n_kv, rows_per_atom);
-  const int64_t size = hds_ragged_meta_size(n_seqs, c.tokens, max_blocks, c.atoms);
+  const Counts c = count(seqs, n_seqs, n_q, n_kv, rows_per_atom);
+  const int64_t size = 4LL * n_seqs + 2 * c.tokens + (int64_t)n_seqs * max_blocks + 3 * c.atoms;
   info[0] = 2 * c.tokens + size + n_extra;
   if (info[0] > cap) return -1;
   int64_t* ids = reinterpret_cast<int64_t*>(out);
@@ -130,7 +111,7 @@ HDS_EXPORT int64_t hds_ragged_step_build(const int64_t* seqs, int n_seqs, int ma
   info[2] = hi;
   if (c.tokens > 0 && id_limit > 0 && (lo < 0 || hi >= id_limit)) return -3;
   int32_t* meta = out + 2 * c.tokens;
-  build(at, n_seqs, c.tokens, max_blocks, n_q, n_kv, rows_per_atom, meta);
+  build(seqs, n_seqs, c.tokens, max_blocks, n_q, n_kv, rows_per_atom, meta);
   if (n_extra > 0) std::memcpy(meta + size, extra, sizeof(int32_t) * (size_t)n_extra);
   return c.atoms;
 }

@@ -20,8 +20,6 @@ SIGS = {
     "hds_ring_query": (I, [P, I]),
     "hds_memcpy_async": (I, [P, P, Z, I, P]),
     # ragged_meta.cpp
-    "hds_ragged_meta_size": (L, [I, L, I, L]),
-    "hds_ragged_meta_build": (L, [P, P, I, P, P, I, I, I, I, P, L, P]),
     "hds_ragged_step_build": (L, [P, I, I, I, I, I, L, P, L, P, L, P]),
     # cpu_optim.cpp
     "hds_cpu_adam": (I, [P, P, I, P, P, P, L, F, F, F, F, F, F, F, I, F]),

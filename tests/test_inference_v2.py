@@ -266,9 +266,8 @@ def test_token_ids_outside_the_embedding_are_refused(dev, bad):
 
 
 def test_native_ragged_metadata_matches_python_reference():
-    """csrc/host/ragged_meta.cpp packs seq_meta / token maps / last rows / block tables / atoms exactly as the
-    Python reference (ops/paged.build_atoms and the per-sequence loops) would build them."""
-    import ctypes
+    """csrc/host/ragged_meta.cpp packs ids / seq_meta / token maps / last rows / block tables / atoms / further values exactly
+    as the Python reference (ops/paged.build_atoms and the per-sequence loops) would build them."""
     import numpy as np
     from hcache_deepspeed_amd.ops import native
     from hcache_deepspeed_amd.ops.paged import build_atoms
@@ -279,15 +278,19 @@ def test_native_ragged_metadata_matches_python_reference():
         n_new = rng.integers(1, 70, S).astype(np.int32)
         seen = rng.integers(0, 200, S).astype(np.int32)
         blocks = [list(rng.integers(0, 1000, rng.integers(1, mb + 1))) for _ in range(S)]
-        off = np.zeros(S + 1, dtype=np.int64)
-        if S:
-            off[1:] = np.cumsum([len(b) for b in blocks])
-        flat = np.array([b for bl in blocks for b in bl], dtype=np.int32)
-        P = lambda a: a.ctypes.data_as(ctypes.c_void_p)  # noqa: E731
-        need = ctypes.c_int64(0)
+        ids = [rng.integers(0, 500, n).astype(np.int64) for n in n_new]
+        tabs = [np.array(b, dtype=np.int32) for b in blocks]
+        desc = np.array([(i.ctypes.data, n, s, t.ctypes.data, t.size) for i, n, s, t in zip(ids, n_new, seen, tabs)],
+                        dtype=np.int64).reshape(S, 5)
+        extra, info = np.array([7, 8, 9], dtype=np.int32), np.zeros(3, dtype=np.int64)
         out = np.zeros(1 << 16, dtype=np.int32)
-        A = lib.hds_ragged_meta_build(P(n_new), P(seen), S, P(flat), P(off), mb, n_q, n_kv, rpa, P(out),
-                                      out.size, ctypes.byref(need))
+
+        def step(cap, limit=500):
+            return lib.hds_ragged_step_build(desc.ctypes.data, S, mb, n_q, n_kv, rpa, limit, extra.ctypes.data, extra.size,
+                                             out.ctypes.data, cap, info.ctypes.data)
+
+        assert step(3) == (-1 if S else 0)  # (nothing but the further values without a sequence)
+        A = step(out.size)
         meta_host = []
         q0 = 0
         for i in range(S):
@@ -295,14 +298,16 @@ def test_native_ragged_metadata_matches_python_reference():
             q0 += int(n_new[i])
         T = q0
         ref_atoms, nref = build_atoms(meta_host, n_q, n_kv)
-        assert A == nref and need.value == 4 * S + 2 * T + S * mb + 3 * A
-        o = 0
+        assert A == nref and info[0] == 4 * S + 4 * T + S * mb + 3 * A + 3
+        assert out[:2 * T].view(np.int64).tolist() == [int(v) for i in ids for v in i]
+        o = 2 * T
         meta = out[o:o + 3 * S].reshape(S, 3); o += 3 * S
         tok_seq = out[o:o + T]; o += T
         tok_pos = out[o:o + T]; o += T
         last = out[o:o + S]; o += S
         tables = out[o:o + S * mb].reshape(S, mb); o += S * mb
-        atoms = out[o:o + 3 * A].reshape(A, 3)
+        atoms = out[o:o + 3 * A].reshape(A, 3); o += 3 * A
+        assert out[o:o + 3].tolist() == [7, 8, 9] and not out[o + 3:].any()
         assert meta.tolist() == [list(m) for m in meta_host]
         for i, (q, n, sn) in enumerate(meta_host):
             assert (tok_seq[q:q + n] == i).all() and tok_pos[q:q + n].tolist() == list(range(sn, sn + n))
@@ -310,6 +315,9 @@ def test_native_ragged_metadata_matches_python_reference():
             assert tables[i, :len(blocks[i])].tolist() == blocks[i] and (tables[i, len(blocks[i]):] == 0).all()
         if A:
             assert atoms.tolist() == ref_atoms.tolist()
+        if T:
+            top = max(int(i.max()) for i in ids)
+            assert info[2] == top and step(out.size, top) == -3 and step(out.size, 0) == A
 
 
 @pytest.mark.parametrize("latent_mode", ["hidden", "kv"])
