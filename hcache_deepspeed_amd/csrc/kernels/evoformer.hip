@@ -16,9 +16,9 @@
 //   * pair-bias gradient: the sum of dS over the N rows stays in registers. A wave owns 32 queries x 64 keys of one
 //     (b, h) and walks over a chunk of the rows, recomputing the two products that dS needs; chunks are added by a second
 //     kernel that also rounds. No atomics, the same result every time.
-// Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): a forward and backward 161 us (with dQ and dK / dV
-// apart 198); in a kernel trace, where launches do not overlap, forward 42 us, dQ + dK + dV 66 (apart 52 + 51), pair
-// gradient 56 + 4
+// Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): a forward and backward 146 us (with dQ and dK / dV
+// apart and the pair gradient's rows loaded by wave 199); in a kernel trace, where launches do not overlap, forward 43 us, dQ +
+// dK + dV 67 (apart 52 + 51), pair gradient 43 + 4 (rows by wave 56 + 4)
 // (before: one wave a workgroup with operands from global memory and 2-byte reads of V 169 us; the FlashAttention
 // backward kernels with 32-bit atomics into the pair gradient 271 + 1,585 us).
 #include <cmath>

@@ -12,6 +12,8 @@
 // sums are reduced across the wave once at the end. Here and below the weights are loaded past the caches (load_nt), whole
 // lines by one instruction: temporal -> not, 1 row [32000, 2048] 23.5 -> 21.7 us, [28672, 4096] 40.4 -> 37.2 (6.3 TB/s), with norm and
 // GLU 43.6 -> 39.9; 8 rows [28672, 4096] 45.3 -> 40.5, [4096, 14336] 24.5 -> 22.5; 16 rows 51.8 -> 47.9, 28.1 -> 27.0.
+// Weights that the memory-side cache would hold from one step to the next lose by it (all of them under 256 MB: [2048, 5632], 1
+// / 4 rows 6.3 / 6.9 -> 6.6 / 9.4 us).
 #include "hds_common.h"
 
 namespace {

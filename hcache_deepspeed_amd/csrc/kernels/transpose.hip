@@ -50,8 +50,10 @@ __global__ __launch_bounds__(256) void transpose_bf16_kernel(const bf16* __restr
   }
 }
 
-// v2 (default): 64 x 128 tiles, every LDS access 8 or 16 B wide (transpose_tile.h). v1's LDS traffic was one 2-B write and
-// one 2-B read per element (32 LDS instructions per thread per 16 B moved). dst rows may be longer than src has rows: zeros.
+// v2: 64 x 128 tiles, every LDS access 8 or 16 B wide (transpose_tile.h). v1's LDS traffic is one 2-B write and one 2-B read
+// per element (32 LDS instructions per thread per 16 B moved). v1 / v2: [8192, 28672] 216 / 176 us, [8192, 4096] 32 / 22, [1024,
+// 5632] 6.9 / 4.9, [1016, 11264] 13.1 / 12.3, [72, 4096] 2.8 / 3.2. v2 makes the padded transposes and runs where variant 2 is
+// asked for, v1 is ops/gemm.py's default. dst rows may be longer than src has rows: zeros.
 template <bool LINES>
 __global__ __launch_bounds__(256) void transpose_bf16_v2_kernel(const bf16* __restrict__ src, bf16* __restrict__ dst,
                                                                 int rows, int cols, int64_t lds, int ldd) {
@@ -79,7 +81,7 @@ __global__ __launch_bounds__(256) void transpose_bf16_v2_kernel(const bf16* __re
 }  // namespace
 
 // rows % 8 == 0 and lds % 8 == 0 keep the vector accesses aligned (checked by the caller)
-// variant 1: 64 x 64 tile, 2-B LDS accesses; variant 2 (default): 64 x 128 tile, 16-B writes / 8-B reads + v_perm
+// variant 1: 64 x 64 tile, 2-B LDS accesses; 2: 64 x 128 tile, 16-B writes / 8-B reads + v_perm
 HDS_EXPORT int hds_transpose_bf16_var(const void* src, void* dst, int rows, int cols, long lds, int variant,
                                       hipStream_t st) {
   if (rows <= 0 || cols <= 0) return hipSuccess;
@@ -98,10 +100,6 @@ HDS_EXPORT int hds_transpose_bf16_var(const void* src, void* dst, int rows, int 
                          cols, (int64_t)lds, rows);
   }
   return hipGetLastError();
-}
-
-HDS_EXPORT int hds_transpose_bf16(const void* src, void* dst, int rows, int cols, long lds, hipStream_t st) {
-  return hds_transpose_bf16_var(src, dst, rows, cols, lds, 2, st);
 }
 
 // The same for any number of rows, to rows of ldd (a multiple of 64, at least `rows`) whose ends are zeros: as operands of a

@@ -58,8 +58,8 @@ def gemm_nt(a, b, out=None, alpha=1.0, accumulate=False, variant=None):
 # ----------------------------------------------------------------------------------------------------------------
 # weight-gradient GEMM layout: dW[N, K] (+)= dY[T, N]^T X[T, K]
 # ----------------------------------------------------------------------------------------------------------------
-# 1: 64x64 tile, 2-B LDS ops; 2: 64x128, 8/16-B LDS ops -- the same ~4.5-5 TB/s at the step's shapes
-# (profiles/r3/transpose_bench_r3.log): HBM read/write mix, not LDS, bounds both
+# 1: 64x64 tile, 2-B LDS ops, the default; 2: 64x128, 8/16-B LDS ops and whole lines, faster from about 2048 x 2048 on and
+# slower by half a us below (csrc/kernels/transpose.hip has the figures)
 _TRANSPOSE_VAR = int(os.environ.get("HDS_TRANSPOSE_VAR", "1"))
 
 

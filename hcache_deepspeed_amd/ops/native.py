@@ -114,7 +114,6 @@ _KERNEL_SIGS = {
     "hds_quant_minifloat": "i" + "ppp" + "l" + "iiiii" + "s",
     "hds_dequant_minifloat": "i" + "ppp" + "l" + "iii" + "s",
     "hds_fp6_gemv": "pppp" + "iiiiii" + "s",
-    "hds_transpose_bf16": "pp" + "ii" + "l" + "s",
     "hds_transpose_bf16_var": "pp" + "ii" + "l" + "i" + "s",
     "hds_transpose_bf16_pad": "pp" + "ii" + "l" + "i" + "s",
     "hds_gemv_bf16_supported": "iii",
