@@ -73,8 +73,10 @@ def skinny(x2, w, b=None):
 
 
 def _needs_grad(*tensors):
-    """The kernels have no backward: with gradients wanted the products are torch's."""
-    return torch.is_grad_enabled() and any(torch.is_tensor(t) and t.requires_grad for t in tensors)
+    """The kernels have no backward, and a trace would hold the allocation of their result only: with gradients wanted, or a
+    trace in progress, the products are torch's."""
+    return (torch.is_grad_enabled() and any(torch.is_tensor(t) and t.requires_grad for t in tensors)) or \
+        torch._C._get_tracing_state() is not None
 
 
 def glu_linear(x, w, b, act):

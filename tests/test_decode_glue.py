@@ -232,6 +232,19 @@ def test_traced_norms_and_gated_units_run_again():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 5])
+def test_traced_few_row_products_run_again(rows):
+    """A graph recorded without gradients computes few-row products for its own inputs: they are torch's in it."""
+    from hcache_deepspeed_amd.ops.gemv import glu_linear, linear
+    w = torch.randn(512, 256, device="cuda").bfloat16()
+    with torch.no_grad():
+        x, y = (torch.randn(rows, 256, device="cuda").bfloat16() for _ in range(2))
+        for f in (lambda t: linear(t, w), lambda t: (lambda z: linear(t, w) if z is None else z)(glu_linear(t, w, None, "silu"))):
+            g = torch.jit.trace(f, (x, ), check_trace=False)
+            assert torch.equal(g(y), torch.nn.functional.linear(y, w))
+
+
+@pytest.mark.gpu
 def test_graph_after_the_buffer_grew_gpu():
     """A graph reads the batch's device buffer; when a larger step has replaced that, later steps reach the graph's own."""
     from hcache_deepspeed_amd.inference.v2.arch import ArchSpec
