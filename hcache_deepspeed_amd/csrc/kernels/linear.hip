@@ -1,0 +1,304 @@
+// y[M, N] = x[M, K] . w[N, K]^T (+ bias) in bf16, sums in 32 bits: projections of more rows than the decode kernels take
+// (gemv.hip) and fewer than a library product fills the chip with. What bounds these shapes is idle CUs: [4096, 14336] at 521
+// rows has 48 tiles of 192 x 256, and the library's smaller tiles leave L2 as the limit (111 us, 0.56 PFLOP/s). So the
+// reduction is split: every (tile, slice of K) is a workgroup, partial sums go to memory in 32 bits and a second kernel adds
+// them in their order, so that results repeat bit for bit.
+//
+// A workgroup keeps a ring of D stages of 64 k in LDS, filled by LDS-DMA through a buffer descriptor (what lies behind the
+// matrices is read as zeros, and unlike global_load_lds it leaves the compiler its counted LDS waits). Rows of 128 bytes keep their
+// 16-byte pieces at c ^ ((row >> 1) & 7), which spreads a fragment read over all banks. Half a stage (32 k) is read into
+// registers while the half before it is multiplied, with one barrier a stage; waiting for all reads of a stage first, as two
+// groups of waves in turn, took 0.62 instead of 0.50 us a stage at 128 x 128.
+//
+// Tiles and their time a stage of a full chip, us (PFLOP/s): 32 x 64 0.16, 64 x 64 0.20, 64 x 128 0.32 (0.85), 128 x 128 0.43 - 0.50
+// (1.08), 192 x 128 0.65 - 0.76 (1.1), 256 x 128 0.73 - 0.90 (1.2), 256 x 256 1.36 - 1.59 (1.35). The small ones are bound by the lines
+// that a CU has on the way (64 bytes a ns), the large ones by LDS reads beside the products; 8 waves need fewer stages in
+// flight than 4, which read less (192 x 256 by 4 waves 1.41, by 8 1.19).
+//
+// Weights not in the caches, us, library -> here: [4096, 14336] 64 / 128 / 192 / 286 / 521 / 1,018 rows 40 / 75 / 103 / 77 / 111 / 129 -> 30 / 35
+// / 40 / 55 / 83 / 105; [4096, 4096] 96 / 128 / 192 / 256 22 / 24 / 33 / 23 -> 15 / 16 / 19 / 19; [6144, 4096] 128 / 192 / 256 26 / 34 / 40 -> 24 / 27 / 32.
+#include <algorithm>
+#include <cmath>
+
+#include "attn_common.h"
+
+using namespace hds;
+using namespace hds::attn;
+
+namespace {
+
+constexpr int BK = 64;  // reduction depth of a stage: rows of 128 bytes
+
+struct LinearArgs {
+  const bf16* x;  // [M, ldx]
+  const bf16* w;  // [N, K]
+  const bf16* bias;  // [N] or null
+  bf16* y;  // [M, ldy]
+  float* part;  // [S, M, N] where S > 1 (gated: [S, M, 2N])
+  int64_t ldx, ldy;
+  int M, N, K, S, tm, tn, act;
+};
+
+// gated unit, by the codes of act.hip: 0 silu, 1 gelu_tanh, 2 relu; the projections rounded as a kernel of its own reads them
+__device__ __forceinline__ bf16 gated(float g, float u, int act) {
+  const float v = (float)(bf16)g;
+  float a;
+  if (act == 2) a = fmaxf(v, 0.f);
+  else if (act == 1) a = 0.5f * v * (1.f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
+  else a = v * __builtin_amdgcn_rcpf(1.f + __expf(-v));
+  return (bf16)(a * (float)(bf16)u);
+}
+
+__device__ __forceinline__ f32x4 mfma16(const bf16x8& a, const bf16x8& b, const f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// 16 bytes a lane from `base` + voff + soff into LDS, lane after lane; zeros from `bytes` on
+__device__ __forceinline__ void load_lds(const void* base, uint32_t bytes, char* lds, uint32_t voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, bytes, 0x00020000),
+                                           (lds_void*)lds, 16, voff, soff, 0, 0);
+}
+
+// RB, CB: 16-row blocks of x and of w a wave; WM x WN waves, a workgroup a CU. GLU: w is [gate; up] of N rows each; half of a
+// tile's and of a wave's columns are gates, the others the same features of up.
+template <int RB, int CB, int WM, int WN, bool GLU>
+__global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void linear_kernel(LinearArgs p) {
+  constexpr int R = 16 * RB * WM, W = 16 * CB * WN, NW = WM * WN, PER = (R + W) / (8 * NW);
+  constexpr int kStage = (R + W) * 128, D = std::min(12, 160 * 1024 / kStage);
+  static_assert((R + W) % (8 * NW) == 0 && R % 8 == 0 && D >= 2, "tile");
+  __shared__ __attribute__((aligned(1024))) char smem[D * kStage];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = wv / WN, wc = wv % WN;
+
+  // an XCD takes neighbouring tiles, those of the same weight rows first: they meet in its L2
+  const int nwg = gridDim.x, orig = blockIdx.x;
+  const int q = nwg / 8, r = nwg % 8, xcd = orig % 8;
+  int id = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + orig / 8;
+  const int s = id / (p.tm * p.tn);
+  id -= s * p.tm * p.tn;
+  const int m0 = id % p.tm * R, n0 = id / p.tm * (GLU ? W / 2 : W);
+  const int KT = p.K / BK, k0 = (int)((int64_t)KT * s / p.S), n = (int)((int64_t)KT * (s + 1) / p.S) - k0;
+
+  // a wave fills 8 rows of a stage with a load: x rows, then w rows. What lies behind the matrices is read as zeros.
+  auto rest = [&](int64_t rows, int64_t ld) { return (uint32_t)std::min<int64_t>(((rows - 1) * ld + p.K) * 2, 0xfffffff0); };
+  const bf16 *xb = p.x + m0 * p.ldx, *wb = p.w + (int64_t)n0 * p.K;
+  const uint32_t xs = rest(p.M - m0, p.ldx), ws = rest((GLU ? 2 : 1) * p.N - n0, p.K);
+  uint32_t src[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int row = 8 * (NW * i + wv) + (lane >> 3);
+    const int ch = (lane & 7) ^ ((row >> 1) & 7);
+    const int of_w = row - R + (GLU && row - R >= W / 2 ? p.N - W / 2 : 0);
+    src[i] = 16 * ch + 2 * (row < R ? (uint32_t)row * (uint32_t)p.ldx : (uint32_t)of_w * (uint32_t)p.K);
+  }
+  auto issue = [&](int t) {
+    char* d = smem + (t % D) * kStage + wv * 1024;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const bool of_x = 8 * (NW * i + wv) < R;  // wave-uniform
+      load_lds(of_x ? xb : wb, of_x ? xs : ws, d + i * NW * 1024, src[i], (k0 + t) * 128);
+    }
+  };
+
+  // a fragment: row lane % 16, 16-byte piece 4 ks + lane / 16
+  const int sw = (lane >> 1) & 7;
+  int foff[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) foff[ks] = (lane & 15) * 128 + 16 * ((4 * ks + (lane >> 4)) ^ sw);
+  const int xo = wr * 16 * RB * 128, wo = (R + wc * (GLU ? 8 : 16) * CB) * 128;
+
+  f32x4 acc[RB][CB];
+#pragma unroll
+  for (int i = 0; i < RB; ++i)
+#pragma unroll
+    for (int j = 0; j < CB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 a[2][RB], b[2][CB];
+  auto read = [&](int t, int ks) {
+    const char* st = smem + (t % D) * kStage + foff[ks];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) a[ks][i] = *reinterpret_cast<const bf16x8*>(st + xo + i * 2048);
+#pragma unroll
+    for (int j = 0; j < CB; ++j) b[ks][j] = *reinterpret_cast<const bf16x8*>(st + wo + j * 2048 + (GLU && j >= CB / 2 ? (W / 2 - 8 * CB) * 128 : 0));
+  };
+  auto multiply = [&](int ks) {
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int j = 0; j < CB; ++j) acc[i][j] = mfma16(b[ks][j], a[ks][i], acc[i][j]);
+  };
+
+#pragma unroll
+  for (int t = 0; t < D; ++t)
+    if (t < n) issue(t);
+  if (D <= n) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((D - 1) * PER) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  read(0, 0);
+  // this stage's second half is on its way while the first is multiplied, and the next stage's first while the second is
+  int t = 0;
+  for (; t + D < n; ++t) {
+    read(t, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(0);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((D - 2) * PER) : "memory");
+    read(t + 1, 0);
+    issue(t + D);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  for (; t < n; ++t) {
+    read(t, 1);
+    multiply(0);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (t + 1 < n) read(t + 1, 0);
+    multiply(1);
+  }
+
+  // lane: row lane % 16 of x, 4 neighbouring columns
+  constexpr int CJ = GLU ? CB / 2 : CB;
+#pragma unroll
+  for (int i = 0; i < RB; ++i) {
+    const int m = m0 + (wr * RB + i) * 16 + (lane & 15);
+    if (m >= p.M) continue;
+#pragma unroll
+    for (int j = 0; j < CJ; ++j) {
+      const int c = n0 + (wc * CJ + j) * 16 + 4 * (lane >> 4);
+      if (c >= p.N) continue;
+      if (p.S > 1) {
+        float* d = p.part + ((int64_t)s * p.M + m) * (GLU ? 2 * p.N : p.N) + c;
+        *reinterpret_cast<f32x4*>(d) = acc[i][j];
+        if constexpr (GLU) *reinterpret_cast<f32x4*>(d + p.N) = acc[i][j + CJ];
+        continue;
+      }
+      bf16x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float v = acc[i][j][e] + (p.bias != nullptr ? (float)p.bias[c + e] : 0.f);
+        if constexpr (GLU) o[e] = gated(v, acc[i][j + CJ][e] + (p.bias != nullptr ? (float)p.bias[p.N + c + e] : 0.f), p.act);
+        else o[e] = (bf16)v;
+      }
+      *reinterpret_cast<bf16x4*>(p.y + m * p.ldy + c) = o;
+    }
+  }
+}
+
+// y = sum over the S parts, in their order
+template <bool GLU>
+__global__ __launch_bounds__(256) void linear_sum_kernel(LinearArgs p) {
+  const int i = blockIdx.x * 256 + threadIdx.x, quads = p.N / 4;
+  if (i >= p.M * quads) return;
+  const int m = i / quads, c = 4 * (i - m * quads), width = GLU ? 2 * p.N : p.N;
+  const float* src = p.part + (int64_t)m * width + c;
+  f32x4 v[GLU ? 2 : 1];
+#pragma unroll
+  for (int h = 0; h < (GLU ? 2 : 1); ++h) {
+    v[h] = *reinterpret_cast<const f32x4*>(src + h * p.N);
+    for (int s = 1; s < p.S; ++s) v[h] += *reinterpret_cast<const f32x4*>(src + h * p.N + (int64_t)s * p.M * width);
+    if (p.bias != nullptr)
+      for (int e = 0; e < 4; ++e) v[h][e] += (float)p.bias[h * p.N + c + e];
+  }
+  bf16x4 o;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = GLU ? gated(v[0][e], v[GLU ? 1 : 0][e], p.act) : (bf16)v[0][e];
+  *reinterpret_cast<bf16x4*>(p.y + m * p.ldy + c) = o;
+}
+
+// time of a tile's workgroup in us: fixed + a stage
+struct Tile {
+  int rows, cols;
+  float fixed, stage;
+};
+constexpr Tile kTiles[] = {{32, 64, 5.3f, 0.16f},   {64, 64, 5.5f, 0.20f},   {64, 128, 5.3f, 0.32f}, {128, 128, 6.6f, 0.43f},
+                           {192, 128, 7.5f, 0.65f}, {256, 128, 7.6f, 0.73f}, {256, 256, 7.9f, 1.36f}};
+constexpr int kMaxSlices = 12;
+
+// The tile and the slices of K that take least by this estimate: rounds over the CUs of the tile's stages, the weights at 7.2
+// TB/s (a last round that is part full has few CUs to read them) and all stages at 21 TB/s from L2, cubes added, since they
+// overlap in part; a further round costs 2.8 us and a sum of slices 1.9 + 1.2 a million floats, and 2 of the host's. Fitted to 9,000 times of 14
+// shapes, 17 to 1,018 rows (7 % rms); the choice is 3 % slower than the best one measured.
+static int linear_choice(int M, int N, int K) {
+  float least = 0.f;
+  int best = 0;
+  for (int t = 0; t < (int)(sizeof(kTiles) / sizeof(Tile)); ++t)
+    for (int S = 1; S <= kMaxSlices && (S == 1 || K / BK / S >= 4); ++S) {
+      const Tile& c = kTiles[t];
+      const float groups = (float)((M + c.rows - 1) / c.rows) * ((N + c.cols - 1) / c.cols) * S;
+      const float rounds = std::ceil(groups / 256.f);
+      const int stages = (K / BK + S - 1) / S;
+      const float a = rounds * c.stage * stages, b = 2e-6f / 7.2f * N * K * rounds * 256.f / std::max(128.f, groups);
+      const float d = groups * (c.rows + c.cols) * 128.f * stages / 21e6f;
+      float us = c.fixed + std::cbrt(a * a * a + b * b * b + d * d * d) + 2.8f * (rounds - 1);
+      if (S > 1) us += 4.f + 1.2e-6f * S * M * N;
+      if (best == 0 || us < least) {
+        least = us;
+        best = t + 16 * S;
+      }
+    }
+  return best;
+}
+
+}  // namespace
+
+// Slices of K with which hds_linear_bf16 takes these rows, or 0 where a library product is the faster one. N: columns of y; glu:
+// of 2N rows of w.
+HDS_EXPORT int hds_linear_slices(int M, int N, int K, int glu) {
+  if (M < 17 || M > 1100 || N < 8 || K < 4 * BK || K % BK || N % 8 || K > 1 << 22 || N > 1 << 22) return 0;
+  const int rows = glu ? 2 * N : N;
+  const int64_t size = (int64_t)rows * K;
+  if (size >= (int64_t)1 << 31) return 0;
+  // Weights not in the caches, times as fast as the library:
+  // - long reductions into few columns, whatever the rows: [4096, 14336] 1.0 - 2.5, [5120, 13824] 1.05 - 2.4, [3072, 8192] 0.9 - 2.1;
+  //   smaller matrices leave nothing to split ([2048, 5632] 0.8 - 1.1)
+  const bool deep = K >= 8192 && 2 * rows <= K && size >= 1 << 24;
+  // - not much wider than deep, rows enough to be bound by products: [6144, 4096] 1.1 - 1.3, [4096, 4096] 1.1 - 1.7, [8192, 8192]
+  //   0.9 - 1.4; at 384 rows 0.9, 1.0, 0.9
+  const bool square = K >= 4096 && 2 * rows <= 3 * K && M >= 80 && M <= 256;
+  // - where a step is bound by its launches: level as kernels ([2048, 2048] 0.8 - 1.0, [3072, 2048] 0.8 - 1.35, [11264, 2048] 1.0 - 1.2), but
+  //   10 us of host time instead of the library's 19. Gated products save a kernel and its pass too ([28672, 4096] 52 + 5 us -> 53 at
+  //   96 rows). Two layers of width 2048, 200 tokens 463 -> 330 us, 310 452 -> 345; of width 4096, 40 tokens 470 -> 344, 190 501 -> 468.
+  //   Beyond, the library's products are the faster ones (521 rows: [28672, 4096] 0.8, [11264, 2048] 0.8, [6144, 4096] 1.05).
+  const bool few = glu ? M <= 256 : M <= 320 && size <= 1 << 25;
+  return deep || square || few ? linear_choice(M, rows, K) / 16 : 0;
+}
+
+// x [M, ldx], w [N, K], bias [N] or null, y [M, ldy], part: S x M x N floats where the slices S (hds_linear_slices) are more
+// than one. glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu): w [2N, K] is gate rows, then up rows, y = act(gate) up,
+// and bias and part are of 2N columns. Rows of x and w begin at 16 bytes, of y at 8.
+HDS_EXPORT int hds_linear_bf16(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy, float* part,
+                               int M, int N, int K, int glu, hipStream_t st) {
+  const int S = hds_linear_slices(M, N, K, glu);
+  if (S < 1 || ldx < K || ldx % 8 || ldx > 1 << 22 || ldy < N || ldy % 4 || (S > 1 && part == nullptr) || glu < 0 || glu > 3 ||
+      ((uintptr_t)x | (uintptr_t)w) & 15 || (uintptr_t)y & 7)
+    return hipErrorInvalidValue;
+  const int rows = glu ? 2 * N : N, tile = linear_choice(M, rows, K) % 16, R = kTiles[tile].rows, W = kTiles[tile].cols;
+  LinearArgs p{(const bf16*)x, (const bf16*)w, (const bf16*)bias, (bf16*)y, part, ldx, ldy, M, N, K, S, (M + R - 1) / R,
+               (rows + W - 1) / W, glu - 1};
+  if (glu) p.tn = (N + W / 2 - 1) / (W / 2);
+  auto run = [&](auto kernel, int waves) {
+    hipLaunchKernelGGL(kernel, dim3(p.tm * p.tn * S), dim3(64 * waves), 0, st, p);
+  };
+#define HDS_LINEAR(id, RB, CB, WM, WN)                                          \
+  case id:                                                                      \
+    if (glu) run(linear_kernel<RB, CB, WM, WN, true>, WM * WN);                 \
+    else run(linear_kernel<RB, CB, WM, WN, false>, WM * WN);                    \
+    break
+  switch (tile) {
+    HDS_LINEAR(0, 1, 2, 2, 2);
+    HDS_LINEAR(1, 2, 2, 2, 2);
+    HDS_LINEAR(2, 2, 2, 2, 4);
+    HDS_LINEAR(3, 4, 2, 2, 4);
+    HDS_LINEAR(4, 6, 4, 2, 2);
+    HDS_LINEAR(5, 4, 4, 4, 2);
+    default: break;
+    HDS_LINEAR(6, 8, 4, 2, 4);
+  }
+#undef HDS_LINEAR
+  if (S > 1) {
+    const dim3 grid((M * (N / 4) + 255) / 256);
+    if (glu) hipLaunchKernelGGL(linear_sum_kernel<true>, grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL(linear_sum_kernel<false>, grid, dim3(256), 0, st, p);
+  }
+  return hipGetLastError();
+}

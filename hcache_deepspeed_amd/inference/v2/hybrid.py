@@ -52,8 +52,8 @@ _MATRICES = ("in.w", "up.w", "out.w", "down.w", "uq.w", "ukv.w", "router.w", "w1
 
 class HybridTransformer(RaggedTransformer):
     # kernel sources this class runs on, for builds of just those (ops/build.py)
-    KERNEL_SOURCES = ("act.hip", "gated_scan.hip", "gemv.hip", "input_norm.hip", "latent_attn.hip", "output_norm.hip",
-                      "paged_rows.hip")
+    KERNEL_SOURCES = ("act.hip", "gated_scan.hip", "gemv.hip", "input_norm.hip", "latent_attn.hip", "linear.hip",
+                      "output_norm.hip", "paged_rows.hip")
 
     def __init__(self, spec, weights, device, dtype=torch.bfloat16, tp_group=None, latent_mode="hidden",
                  engine_config=None):
@@ -305,8 +305,8 @@ class HybridTransformer(RaggedTransformer):
 
 class PostNormTransformer(HybridTransformer):
     """Layers with the norm on their sublayers' outputs and routed experts: x += n1(mixer(x)), x += n2(experts(x))."""
-    KERNEL_SOURCES = ("act.hip", "experts.hip", "gemv.hip", "grouped_gemm.hip", "output_norm.hip", "paged_attn.hip",
-                      "paged_rows.hip")
+    KERNEL_SOURCES = ("act.hip", "experts.hip", "gemv.hip", "grouped_gemm.hip", "linear.hip", "output_norm.hip",
+                      "paged_attn.hip", "paged_rows.hip")
 
     def _build_layers(self, ec):
         spec, H = self.spec, self.spec.hidden_size
@@ -354,8 +354,8 @@ class SandwichTransformer(HybridTransformer):
     """Layers with a norm on both sides of every sublayer: x += n1b(mixer(n1(x))), x += n2b(ff(n2(x))); a factor of the
     residual sum is part of the gains of n1b and n2b. With ``token_side``, behind it x += n(proj(gelu(gate x) * e)), e the
     token's row of this layer."""
-    KERNEL_SOURCES = ("act.hip", "delta_rule.hip", "gemv.hip", "latent_attn.hip", "output_norm.hip", "paged_attn.hip",
-                      "paged_rows.hip")
+    KERNEL_SOURCES = ("act.hip", "delta_rule.hip", "gemv.hip", "latent_attn.hip", "linear.hip", "output_norm.hip",
+                      "paged_attn.hip", "paged_rows.hip")
 
     def _build_layers(self, ec):
         spec, H = self.spec, self.spec.hidden_size
@@ -452,5 +452,5 @@ class SandwichTransformer(HybridTransformer):
 
 class MemorySandwichTransformer(SandwichTransformer):
     """The same layers on layer norms, with matrix memories and parallel mixers (the kernels it runs on are others)."""
-    KERNEL_SOURCES = ("act.hip", "experts.hip", "gemv.hip", "grouped_gemm.hip", "head_prep.hip", "matrix_memory.hip",
-                      "output_norm.hip", "paged_attn.hip", "paged_rows.hip")
+    KERNEL_SOURCES = ("act.hip", "experts.hip", "gemv.hip", "grouped_gemm.hip", "head_prep.hip", "linear.hip",
+                      "matrix_memory.hip", "output_norm.hip", "paged_attn.hip", "paged_rows.hip")

@@ -13,6 +13,7 @@ import torch.nn.functional as F
 
 from . import native
 from .activations import glu_rows
+from .gemv import rows_linear
 
 PAD = 128  # bf16 expert weights: every dimension is zero-padded to a multiple of the grouped product's tile
 
@@ -99,9 +100,12 @@ def route(z, correction, shape):
 
 def _shared_product(x, w):
     """Gate / up product, activation and down product of the shared expert for a long step."""
-    gu = F.linear(x, w["ws13"])
-    h = torch.empty(x.shape[0], w["ws2"].shape[1], dtype=x.dtype, device=x.device)
-    return F.linear(glu_rows(gu, "silu", h), w["ws2"])
+    h = rows_linear(x, w["ws13"], glu=1)
+    if h is None:
+        gu = F.linear(x, w["ws13"])
+        h = glu_rows(gu, "silu", torch.empty(x.shape[0], w["ws2"].shape[1], dtype=x.dtype, device=x.device))
+    y = rows_linear(h, w["ws2"])
+    return F.linear(h, w["ws2"]) if y is None else y
 
 
 def routed_experts(x, w, shape, identity=True, act="silu", limit=0.0):

@@ -120,6 +120,8 @@ _KERNEL_SIGS = {
     "hds_gemv_bf16": "pppp" + "iii" + "ll" + "s",
     "hds_gemv_fused_bf16": "ppp" + "f" + "pppp" + "if" + "iii" + "ll" + "s",
     "hds_gather_gemv_bf16": "ppp" + "l" + "p" + "ii" + "p" + "iii" + "ll" + "s",
+    "hds_linear_slices": "iiii",
+    "hds_linear_bf16": "plppplp" + "iiii" + "s",
     "hds_skinny_gemm_bf16": "pppp" + "iii" + "ll" + "i" + "s",
     "hds_wmix_splits": "iii",
     "hds_wmix_supported": "iiii",

@@ -1,0 +1,82 @@
+"""Products of 17 to 1,100 rows that split their reduction (csrc/kernels/linear.hip)."""
+import pytest
+import torch
+
+from hcache_deepspeed_amd.ops import gemv
+
+# smallest and largest rows of either rule, one and several row tiles, rows and columns behind the last tile, slices that
+# differ by a stage, slices of fewer stages than the ring holds
+SHAPES = [(17, 4096, 8192), (31, 4104, 8256), (33, 2056, 14336), (65, 2048, 8192), (80, 4096, 4096), (129, 4096, 4160), (193, 6144, 4096),
+          (256, 8192, 8192), (256, 4120, 4096), (20, 72, 256), (40, 2048, 320), (256, 8, 2048), (257, 4096, 8192), (521, 4096, 14336), (700, 3080, 8192), (1100, 4096, 8192)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_linear_rows_match_64_bits(M, N, K):
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    w = (torch.randn(N, K, device="cuda", generator=g) * K**-0.5).to(torch.bfloat16)
+    x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
+    x[-1, -64:] = 100  # what the last row's last stage holds counts
+    b = torch.randn(N, device="cuda", generator=g).to(torch.bfloat16) if M % 2 else None
+    assert gemv._slices(M, N, K)
+    with torch.no_grad():
+        y, again = gemv.linear(x, w, b), gemv.linear(x, w, b)
+    ref = x.double() @ w.double().t() + (0 if b is None else b.double())
+    # 32-bit sums of K products, then one rounding
+    bound = 2**-8 * ref.abs() + 2**-24 * K**0.5 * 8 * (x.double().abs() @ w.double().abs().t()) + 1e-6
+    assert y.shape == ref.shape and ((y.double() - ref).abs() <= bound).all()
+    assert torch.equal(y, again)
+
+
+@pytest.mark.gpu
+def test_linear_rows_all_tiles_exact():
+    """Every tile and number of slices that the choice takes over its range: small integers, whose sums are exact in 32 bits
+    and the result in bf16."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    K, N = 8192, 4096
+    w = torch.randint(-1, 2, (N, K), device="cuda", generator=g).bfloat16()
+    x = (torch.randint(-1, 2, (1100, K), device="cuda", generator=g) * (torch.rand(1100, K, device="cuda", generator=g) < 0.05)).bfloat16()
+    ref = x.float() @ w.float().t()
+    assert ref.abs().max() <= 256
+    for M in list(range(17, 300, 16)) + list(range(300, 1100, 97)):
+        with torch.no_grad():
+            assert torch.equal(gemv.linear(x[:M], w).float(), ref[:M]), M
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", ["silu", "gelu_tanh", "relu"])
+@pytest.mark.parametrize("M,N,K", [(17, 8, 256), (33, 1000, 2048), (64, 5632, 2048), (129, 72, 8192), (200, 4096, 4160), (256, 14336, 4096)])
+def test_linear_rows_gated(act, M, N, K):
+    """One and several slices, features behind the last tile, against 64 bits with the projections rounded first."""
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    w = (torch.randn(2 * N, K, device="cuda", generator=g) * K**-0.5).to(torch.bfloat16)
+    x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
+    b = torch.randn(2 * N, device="cuda", generator=g).to(torch.bfloat16) if M % 2 else None
+    with torch.no_grad():
+        y = gemv.glu_linear(x, w, b, act)
+    ref = x.double() @ w.double().t() + (0 if b is None else b.double())
+    sums = 2**-24 * K**0.5 * 8 * (x.double().abs() @ w.double().abs().t())
+    gate, up = ref[:, :N], ref[:, N:]
+    f = {"silu": torch.nn.functional.silu, "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh"), "relu": torch.relu}[act]
+    # each factor within half a unit of the last place and its sum's error; |act'| <= 1.13
+    bound = 2**-8 * (1.13 * gate.abs() * up.abs() + 2 * (f(gate) * up).abs()) + 1.13 * (sums[:, :N] * up.abs() + sums[:, N:] * gate.abs())
+    assert y.shape == (M, N) and ((y.double() - f(gate) * up).abs() <= bound + 1e-6).all()
+
+
+@pytest.mark.gpu
+def test_linear_rows_refuse():
+    """What the kernel does not take goes where it went: rows, K, widths, types, alignment, gradients and transforms."""
+    assert not any(gemv._slices(*s) for s in [(16, 4096, 8192), (1101, 4096, 8192), (128, 4096, 4000), (128, 4095, 8192), (128, 32768, 4096),
+                                              (321, 4096, 4096), (257, 4096, 8192, 1)])
+    x = torch.zeros(128, 8200, dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros(4096, 8192, dtype=torch.bfloat16, device="cuda")
+    with torch.no_grad():
+        assert gemv.rows_linear(x[:, :8192], w) is not None and gemv.rows_linear(x[:, :8192].view(2, 64, -1), w).shape == (2, 64, 4096)
+        for a, b in ((x[:, 4:8196], w), (x[:, :8192].half(), w), (x, w), (x[:, :8192], w.t().contiguous().t())):
+            assert gemv.rows_linear(a, b) is None
+        with pytest.raises(RuntimeError):
+            gemv.linear(x, w)
+        rows = x[:, :8192].contiguous().view(2, 64, 8192)
+        assert torch.func.vmap(gemv.linear, in_dims=(0, None))(rows, w).shape == (2, 64, 4096)
+    w.requires_grad_()
+    assert gemv.linear(x[:, :8192], w).grad_fn is not None
