@@ -41,6 +41,7 @@ HIPCC_FLAGS = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}", "-ffp-con
 FILE_FLAGS = {"flash_attn.hip": ["-fno-slp-vectorize"],
               # the one-wave-per-SIMD forward keeps S in VGPRs (builtin MFMAs, schedulable) and O in AGPRs (asm)
               "flash_attn_w64.hip": ["-fno-slp-vectorize", "-mllvm", "-amdgpu-mfma-vgpr-form"],
+              "flash_attn_pair.hip": ["-fno-slp-vectorize", "-mllvm", "-amdgpu-mfma-vgpr-form"],
               "flash_attn_bwd_w64.hip": ["-fno-slp-vectorize", "-mllvm", "-amdgpu-mfma-vgpr-form"],
               # whole tiles of accumulators beside the fragments of two halves: moves from and to AGPRs cost as much as the products
               "linear.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],

@@ -1,11 +1,11 @@
-"""Serving steps with more than single tokens: portions of prompts on the one-wave-per-SIMD attention kernel over block tables
-(csrc/kernels/flash_attn_w64.hip) or in row blocks, single tokens on the split-key kernel (both csrc/kernels/paged_attn.hip)."""
+"""Serving steps with more than single tokens: portions of prompts on the FlashAttention kernels over block tables
+(csrc/kernels/flash_attn_pair.hip, flash_attn_w64.hip) or in row blocks, single tokens on the split-key kernel (both csrc/kernels/paged_attn.hip)."""
 import torch
 
 from . import native
 from .paged import DECODE_MAX, ROWS_PER_ATOM
 
-# new tokens of a workgroup of the prefill kernel
+# new tokens of an entry of the prefill kernel's list: one workgroup a head, or two of half the rows where there are few
 PREFILL_ROWS = 256
 
 
