@@ -1,7 +1,9 @@
 // y[M, N] = x[M, K] . w[N, K]^T (+ bias) in bf16, sums in 32 bits: projections of more rows than the decode kernels take
-// (gemv.hip) and fewer than a library product fills the chip with. What bounds these shapes is idle CUs: [4096, 14336] at 521
-// rows has 48 tiles of 192 x 256, and the library's smaller tiles leave L2 as the limit (111 us, 0.56 PFLOP/s). So the
-// reduction is split: every (tile, slice of K) is a workgroup, partial sums go to memory in 32 bits and a second kernel adds
+// (gemv.hip) and fewer than a library product fills the chip with, with the gated unit of w = [gate; up] in the epilogue.
+//
+// What bounds these shapes is idle CUs, or a weight stream that library tiles do not keep up: [4096, 14336] at 521 rows has 48
+// tiles of 192 x 256, and the library's smaller ones leave L2 as the limit (111 us, 0.56 PFLOP/s). So the reduction is split
+// where that pays: every (tile, slice of K) is a workgroup, partial sums go to memory in 32 bits and a second kernel adds
 // them in their order, so that results repeat bit for bit.
 //
 // A workgroup keeps a ring of D stages of 64 k in LDS, filled by LDS-DMA through a buffer descriptor (what lies behind the
@@ -10,13 +12,15 @@
 // registers while the half before it is multiplied, with one barrier a stage; waiting for all reads of a stage first, as two
 // groups of waves in turn, took 0.62 instead of 0.50 us a stage at 128 x 128.
 //
-// Tiles and their time a stage of a full chip, us (PFLOP/s): 32 x 64 0.16, 64 x 64 0.20, 64 x 128 0.32 (0.85), 128 x 128 0.43 - 0.50
-// (1.08), 192 x 128 0.65 - 0.76 (1.1), 256 x 128 0.73 - 0.90 (1.2), 256 x 256 1.36 - 1.59 (1.35). The small ones are bound by the lines
-// that a CU has on the way (64 bytes a ns), the large ones by LDS reads beside the products; 8 waves need fewer stages in
-// flight than 4, which read less (192 x 256 by 4 waves 1.41, by 8 1.19).
+// Time a stage with a full chip, us (PFLOP/s): 64 x 128 0.32 (0.85), 128 x 128 0.43 - 0.50 (1.1), 192 x 128 0.76 (1.1), 256 x 128
+// 0.73 - 0.90 (1.2), 256 x 256 1.36 - 1.59 (1.35). The small ones are bound by the lines that a CU has on the way (64 bytes a
+// ns), the large ones by LDS reads beside the products. Tiles of 32 rows share a CU, so that one's prologue and epilogue lie
+// beside another's stream. Weight rows a multiple of 4 KB apart lie alike in the memory's channels: there each column of
+// tiles begins its walk along K somewhere else ([28672, 4096], 24 rows 42.5 -> 38.2 us).
 //
 // Weights not in the caches, us, library -> here: [4096, 14336] 64 / 128 / 192 / 286 / 521 / 1,018 rows 40 / 75 / 103 / 77 / 111 / 129 -> 30 / 35
-// / 40 / 55 / 83 / 105; [4096, 4096] 96 / 128 / 192 / 256 22 / 24 / 33 / 23 -> 15 / 16 / 19 / 19; [6144, 4096] 128 / 192 / 256 26 / 34 / 40 -> 24 / 27 / 32.
+// / 40 / 55 / 83 / 105; [4096, 4096] 96 / 128 / 192 / 256 22 / 24 / 33 / 23 -> 15 / 16 / 19 / 20; [28672, 4096] gated 24 / 64 / 128 53 / 54 /
+// 58 -> 38 / 40 / 49; [11264, 2048] gated 24 / 128 / 256 20 / 22 / 31 -> 14 / 20 / 25.
 #include <algorithm>
 #include <cmath>
 
@@ -36,7 +40,7 @@ struct LinearArgs {
   bf16* y;  // [M, ldy]
   float* part;  // [S, M, N] where S > 1 (gated: [S, M, 2N])
   int64_t ldx, ldy;
-  int M, N, K, S, tm, tn, act;
+  int M, N, K, S, tm, tn, act, nt, apart;
 };
 
 // gated unit, by the codes of act.hip: 0 silu, 1 gelu_tanh, 2 relu; the projections rounded as a kernel of its own reads them
@@ -53,18 +57,19 @@ __device__ __forceinline__ f32x4 mfma16(const bf16x8& a, const bf16x8& b, const 
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// 16 bytes a lane from `base` + voff + soff into LDS, lane after lane; zeros from `bytes` on
+// 16 bytes a lane from `base` + voff + soff into LDS, lane after lane; zeros from `bytes` on. NT: past the caches
+template <bool NT>
 __device__ __forceinline__ void load_lds(const void* base, uint32_t bytes, char* lds, uint32_t voff, int soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, bytes, 0x00020000),
-                                           (lds_void*)lds, 16, voff, soff, 0, 0);
+                                           (lds_void*)lds, 16, voff, soff, 0, NT ? 2 : 0);
 }
 
-// RB, CB: 16-row blocks of x and of w a wave; WM x WN waves, a workgroup a CU. GLU: w is [gate; up] of N rows each; half of a
+// RB, CB: 16-row blocks of x and of w a wave; WM x WN waves, OCC workgroups a CU. GLU: w is [gate; up] of N rows each; half of a
 // tile's and of a wave's columns are gates, the others the same features of up.
-template <int RB, int CB, int WM, int WN, bool GLU>
-__global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void linear_kernel(LinearArgs p) {
+template <int RB, int CB, int WM, int WN, int OCC, bool GLU>
+__global__ __launch_bounds__(64 * WM * WN, WM * WN * OCC / 4) void linear_kernel(LinearArgs p) {
   constexpr int R = 16 * RB * WM, W = 16 * CB * WN, NW = WM * WN, PER = (R + W) / (8 * NW);
-  constexpr int kStage = (R + W) * 128, D = std::min(12, 160 * 1024 / kStage);
+  constexpr int kStage = (R + W) * 128, D = std::min(12, 160 * 1024 / OCC / kStage);
   static_assert((R + W) % (8 * NW) == 0 && R % 8 == 0 && D >= 2, "tile");
   __shared__ __attribute__((aligned(1024))) char smem[D * kStage];
   const int lane = threadIdx.x & 63;
@@ -92,12 +97,15 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN / 4) void linear_kernel(Linea
     const int of_w = row - R + (GLU && row - R >= W / 2 ? p.N - W / 2 : 0);
     src[i] = 16 * ch + 2 * (row < R ? (uint32_t)row * (uint32_t)p.ldx : (uint32_t)of_w * (uint32_t)p.K);
   }
+  const int turn = p.apart ? (int)__umulhi((unsigned)(id / p.tm) * 2654435769u, (unsigned)n) : 0;
   auto issue = [&](int t) {
     char* d = smem + (t % D) * kStage + wv * 1024;
+    const int k = (k0 + (t + turn < n ? t + turn : t + turn - n)) * 128;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const bool of_x = 8 * (NW * i + wv) < R;  // wave-uniform
-      load_lds(of_x ? xb : wb, of_x ? xs : ws, d + i * NW * 1024, src[i], (k0 + t) * 128);
+      if (p.nt && !of_x) load_lds<true>(wb, ws, d + i * NW * 1024, src[i], k);
+      else load_lds<false>(of_x ? xb : wb, of_x ? xs : ws, d + i * NW * 1024, src[i], k);
     }
   };
 
@@ -205,19 +213,19 @@ __global__ __launch_bounds__(256) void linear_sum_kernel(LinearArgs p) {
   *reinterpret_cast<bf16x4*>(p.y + m * p.ldy + c) = o;
 }
 
-// time of a tile's workgroup in us: fixed + a stage
+// tiles: workgroups a CU, time of a workgroup in us: once + a stage
 struct Tile {
-  int rows, cols;
-  float fixed, stage;
+  int rows, cols, each;
+  float once, stage;
 };
-constexpr Tile kTiles[] = {{32, 64, 5.3f, 0.16f},   {64, 64, 5.5f, 0.20f},   {64, 128, 5.3f, 0.32f}, {128, 128, 6.6f, 0.43f},
-                           {192, 128, 7.5f, 0.65f}, {256, 128, 7.6f, 0.73f}, {256, 256, 7.9f, 1.36f}};
+constexpr Tile kTiles[] = {{32, 64, 2, 5.5f, 0.13f},   {32, 128, 2, 5.8f, 0.23f},  {64, 64, 1, 5.8f, 0.26f},   {64, 128, 1, 6.4f, 0.33f},
+                           {128, 128, 1, 8.3f, 0.43f}, {192, 128, 1, 9.2f, 0.78f}, {256, 128, 1, 10.f, 0.72f}, {256, 256, 1, 10.7f, 1.41f}};
 constexpr int kMaxSlices = 12;
 
-// The tile and the slices of K that take least by this estimate: rounds over the CUs of the tile's stages, the weights at 7.2
-// TB/s (a last round that is part full has few CUs to read them) and all stages at 21 TB/s from L2, cubes added, since they
-// overlap in part; a further round costs 2.8 us and a sum of slices 1.9 + 1.2 a million floats, and 2 of the host's. Fitted to 9,000 times of 14
-// shapes, 17 to 1,018 rows (7 % rms); the choice is 3 % slower than the best one measured.
+// The tile and the slices of K that take least by this estimate: the stages of the fullest CU, the weights at 8.4 TB/s (fewer
+// bytes a second where CUs have fewer workgroups than the fullest) and all stages at 19 TB/s from L2, cubes added, since
+// they overlap in part; a further round costs 2.6 us and a sum of slices 1.8 + 1.1 a million floats, and 2 of the host's. Fitted to
+// 11,000 times of 20 shapes, 5 to 1,018 rows (8 % rms); the choice is 2 % slower than the best one measured.
 static int linear_choice(int M, int N, int K) {
   float least = 0.f;
   int best = 0;
@@ -225,12 +233,12 @@ static int linear_choice(int M, int N, int K) {
     for (int S = 1; S <= kMaxSlices && (S == 1 || K / BK / S >= 4); ++S) {
       const Tile& c = kTiles[t];
       const float groups = (float)((M + c.rows - 1) / c.rows) * ((N + c.cols - 1) / c.cols) * S;
-      const float rounds = std::ceil(groups / 256.f);
+      const float fullest = std::ceil(groups / 256.f);
       const int stages = (K / BK + S - 1) / S;
-      const float a = rounds * c.stage * stages, b = 2e-6f / 7.2f * N * K * rounds * 256.f / std::max(128.f, groups);
-      const float d = groups * (c.rows + c.cols) * 128.f * stages / 21e6f;
-      float us = c.fixed + std::cbrt(a * a * a + b * b * b + d * d * d) + 2.8f * (rounds - 1);
-      if (S > 1) us += 4.f + 1.2e-6f * S * M * N;
+      const float a = fullest * c.stage * stages, b = 2e-6f / 8.4f * N * K * fullest * 256.f / std::max(128.f, groups);
+      const float d = groups * (c.rows + c.cols) * 128.f * stages / 19e6f;
+      float us = c.once + std::cbrt(a * a * a + b * b * b + d * d * d) + 2.6f * (std::ceil(groups / (256.f * c.each)) - 1);
+      if (S > 1) us += 3.8f + 1.1e-6f * S * M * N;
       if (best == 0 || us < least) {
         least = us;
         best = t + 16 * S;
@@ -244,23 +252,31 @@ static int linear_choice(int M, int N, int K) {
 // Slices of K with which hds_linear_bf16 takes these rows, or 0 where a library product is the faster one. N: columns of y; glu:
 // of 2N rows of w.
 HDS_EXPORT int hds_linear_slices(int M, int N, int K, int glu) {
-  if (M < 17 || M > 1100 || N < 8 || K < 4 * BK || K % BK || N % 8 || K > 1 << 22 || N > 1 << 22) return 0;
+  if (M < 9 || M > 1100 || N < 8 || K < 4 * BK || K % BK || N % 8 || K > 1 << 22 || N > 1 << 22) return 0;
   const int rows = glu ? 2 * N : N;
   const int64_t size = (int64_t)rows * K;
   if (size >= (int64_t)1 << 31) return 0;
-  // Weights not in the caches, times as fast as the library:
-  // - long reductions into few columns, whatever the rows: [4096, 14336] 1.0 - 2.5, [5120, 13824] 1.05 - 2.4, [3072, 8192] 0.9 - 2.1;
-  //   smaller matrices leave nothing to split ([2048, 5632] 0.8 - 1.1)
-  const bool deep = K >= 8192 && 2 * rows <= K && size >= 1 << 24;
-  // - not much wider than deep, rows enough to be bound by products: [6144, 4096] 1.1 - 1.3, [4096, 4096] 1.1 - 1.7, [8192, 8192]
-  //   0.9 - 1.4; at 384 rows 0.9, 1.0, 0.9
-  const bool square = K >= 4096 && 2 * rows <= 3 * K && M >= 80 && M <= 256;
-  // - where a step is bound by its launches: level as kernels ([2048, 2048] 0.8 - 1.0, [3072, 2048] 0.8 - 1.35, [11264, 2048] 1.0 - 1.2), but
-  //   10 us of host time instead of the library's 19. Gated products save a kernel and its pass too ([28672, 4096] 52 + 5 us -> 53 at
-  //   96 rows). Two layers of width 2048, 200 tokens 463 -> 330 us, 310 452 -> 345; of width 4096, 40 tokens 470 -> 344, 190 501 -> 468.
-  //   Beyond, the library's products are the faster ones (521 rows: [28672, 4096] 0.8, [11264, 2048] 0.8, [6144, 4096] 1.05).
-  const bool few = glu ? M <= 256 : M <= 320 && size <= 1 << 25;
-  return deep || square || few ? linear_choice(M, rows, K) / 16 : 0;
+  // Weights not in the caches, times as fast as the library (up to 16 rows as skinny_lines_kernel):
+  // - up to 128 rows, which read the weights once at 6 TB/s and more: [28672, 4096] gated 24 / 64 / 128 rows 53 / 54 / 58 us ->
+  //   38 / 40 / 49, [32000, 4096] 59 / 56 / 59 -> 41 / 42 / 51, [10240, 8192] 1.0 - 1.8, [15360, 5120] 0.9 - 1.1; small matrices level as
+  //   kernels ([2048, 2048], [3072, 2048] 0.8 - 1.05), but 10 us of host time instead of the library's 19, which is what bounds
+  //   steps of short prompts. Up to 16 rows where the matrix is large and not sliced: [28672, 4096] 8 / 12 / 16 rows 38.8 / 42.6 /
+  //   45.1 -> 37.3 / 37.3 / 37.5, [32000, 4096] 41.5 / 44.9 / 49.2 -> 40.0 / 40.4 / 40.4; smaller ones 0.6 - 1.03.
+  const int choice = linear_choice(M, rows, K), S = choice / 16;
+  if (M <= 16) return S == 1 && size >= 1 << 25 ? S : 0;
+  // 17 to 32 are decode steps, whose launches are recorded once: smaller matrices are the library's ([2048, 2048], 24 rows 8.2 us in
+  // a step / 10.4).
+  if (M <= 32 && !glu && size < 3 << 23) return 0;
+  bool take = M <= 128;
+  // - up to 256 with a gated unit, whose kernel and pass it saves ([28672, 4096] 0.93 - 1.04, [11264, 2048] 1.2), or not
+  //   much wider than deep ([6144, 4096] 1.04 - 1.35, [4096, 4096] 1.1 - 1.7, [8192, 8192] 1.2 - 1.6), as [32000, 4096] (0.95 - 1.02) is;
+  take = take || (M <= 256 && (glu || (K >= 4096 && 2 * rows <= 3 * K)));
+  // - to 320 where the library's call is the longer half (0.8 - 1.1; two layers of width 2048, 310 tokens 452 -> 345 us);
+  take = take || (M <= 320 && !glu && size <= 1 << 25);
+  // - long reductions into few columns, whatever the rows: [4096, 14336] 1.0 - 2.3, [5120, 13824] 0.94 - 2.4. Beyond, the library's
+  //   products are the faster ones (521 rows: [28672, 4096] 0.8, [11264, 2048] 0.85, [6144, 4096] 1.0).
+  take = take || (K >= 8192 && 2 * rows <= K && size >= 1 << 24);
+  return take ? S : 0;
 }
 
 // x [M, ldx], w [N, K], bias [N] or null, y [M, ldy], part: S x M x N floats where the slices S (hds_linear_slices) are more
@@ -274,25 +290,28 @@ HDS_EXPORT int hds_linear_bf16(const void* x, int64_t ldx, const void* w, const 
     return hipErrorInvalidValue;
   const int rows = glu ? 2 * N : N, tile = linear_choice(M, rows, K) % 16, R = kTiles[tile].rows, W = kTiles[tile].cols;
   LinearArgs p{(const bf16*)x, (const bf16*)w, (const bf16*)bias, (bf16*)y, part, ldx, ldy, M, N, K, S, (M + R - 1) / R,
-               (rows + W - 1) / W, glu - 1};
+               (rows + W - 1) / W, glu - 1, 0, K % 2048 == 0};
   if (glu) p.tn = (N + W / 2 - 1) / (W / 2);
+  // Weights that one row of tiles reads go past the caches: [28672, 4096] 24 / 64 rows 43.5 / 44.7 -> 38.2 / 40.0 us. Not with
+  // slices, whose walks are short ([4096, 14336], 128 rows 33.8 / 38.1), but in the smallest tile (24 rows 25.4 -> 24.0).
+  p.nt = p.tm == 1 && (S == 1 || (R == 32 && p.apart));
   auto run = [&](auto kernel, int waves) {
     hipLaunchKernelGGL(kernel, dim3(p.tm * p.tn * S), dim3(64 * waves), 0, st, p);
   };
-#define HDS_LINEAR(id, RB, CB, WM, WN)                                          \
+#define HDS_LINEAR(id, RB, CB, WM, WN, OCC)                                     \
   case id:                                                                      \
-    if (glu) run(linear_kernel<RB, CB, WM, WN, true>, WM * WN);                 \
-    else run(linear_kernel<RB, CB, WM, WN, false>, WM * WN);                    \
+    if (glu) run(linear_kernel<RB, CB, WM, WN, OCC, true>, WM * WN);            \
+    else run(linear_kernel<RB, CB, WM, WN, OCC, false>, WM * WN);               \
     break
   switch (tile) {
-    HDS_LINEAR(0, 1, 2, 2, 2);
-    HDS_LINEAR(1, 2, 2, 2, 2);
-    HDS_LINEAR(2, 2, 2, 2, 4);
-    HDS_LINEAR(3, 4, 2, 2, 4);
-    HDS_LINEAR(4, 6, 4, 2, 2);
-    HDS_LINEAR(5, 4, 4, 4, 2);
-    default: break;
-    HDS_LINEAR(6, 8, 4, 2, 4);
+    HDS_LINEAR(0, 1, 2, 2, 2, 2);
+    HDS_LINEAR(1, 2, 2, 1, 4, 2);
+    HDS_LINEAR(2, 2, 2, 2, 2, 1);
+    HDS_LINEAR(3, 2, 2, 2, 4, 1);
+    HDS_LINEAR(4, 4, 2, 2, 4, 1);
+    HDS_LINEAR(5, 6, 4, 2, 2, 1);
+    HDS_LINEAR(6, 4, 4, 4, 2, 1);
+    HDS_LINEAR(7, 8, 4, 2, 4, 1);
   }
 #undef HDS_LINEAR
   if (S > 1) {

@@ -74,7 +74,7 @@ def skinny(x2, w, b=None):
     return y
 
 
-# 17 to 1,100 rows: csrc/kernels/linear.hip where hds_linear_slices takes them (HDS_LINEAR=0: never)
+# 9 to 1,100 rows: csrc/kernels/linear.hip where hds_linear_slices takes them (HDS_LINEAR=0: never)
 LINEAR = _os.environ.get("HDS_LINEAR", "1") == "1"
 
 
@@ -85,7 +85,7 @@ def _slices(M, N, K, glu=0):
 
 
 def rows_linear(x, w, b=None, glu=0):
-    """``F.linear(x, w, b)`` of 17 rows and more, or with ``glu`` = 1 + activation code the gated unit of w = [gate; up]; None
+    """``F.linear(x, w, b)`` of 9 rows and more, or with ``glu`` = 1 + activation code the gated unit of w = [gate; up]; None
     where the kernel does not take the call, as where anything could want a record of it (``native.plain``)."""
     if not x.is_cuda or not native.plain(x, w, b) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() < 1 or \
             w.dim() != 2 or not w.is_contiguous():
@@ -120,12 +120,14 @@ def _needs_grad(*tensors):
 
 
 def glu_linear(x, w, b, act):
-    """act(x . gate^T) * (x . up^T) for ``w`` = [gate; up] (and ``b``) in one call, for 2..16 rows of the skinny GEMM and 17..256 of
+    """act(x . gate^T) * (x . up^T) for ``w`` = [gate; up] (and ``b``) in one call, for 2..16 rows of the skinny GEMM and 9..256 of
     ``rows_linear``; None for anything else. The projections are rounded to bf16 first, as the separate kernels store them."""
     if act not in _GATHER_ACTS or not (x.dim() >= 1 and x.is_cuda and torch.is_tensor(w)) or _needs_grad(x, w, b):
         return None
-    if x.numel() > MAX_ROWS * x.shape[-1]:
-        return rows_linear(x, w, b, 1 + _GATHER_ACTS[act])
+    if x.numel() > 8 * x.shape[-1]:
+        y = rows_linear(x, w, b, 1 + _GATHER_ACTS[act])
+        if y is not None or x.numel() > MAX_ROWS * x.shape[-1]:
+            return y
     x2 = x.reshape(-1, x.shape[-1])
     if not skinny_ok(x2, w, b) or w.shape[0] % 2:
         return None
@@ -139,9 +141,13 @@ def glu_linear(x, w, b, act):
 
 def linear(x, w, b=None):
     """``F.linear(x, w, b)``; decode-sized bf16 inputs run the HIP GEMV (one row) or the skinny matrix-core GEMM
-    (2..16 rows), 17 to 1,100 the sliced matrix-core
-    GEMM where it is the faster one, unless a gradient is wanted."""
+    (2..16 rows), 9 to 1,100 the tiled and
+    sliced one where it is the faster, unless a gradient is wanted."""
     if x.dim() >= 1 and x.is_cuda and x.numel() <= MAX_ROWS * x.shape[-1] and not _needs_grad(x, w, b):
+        if x.numel() > 8 * x.shape[-1]:
+            y = rows_linear(x, w, b)
+            if y is not None:
+                return y
         x2 = x.reshape(-1, x.shape[-1])
         if skinny_ok(x2, w, b):
             return skinny(x2, w, b).view(*x.shape[:-1], w.shape[0])
