@@ -322,7 +322,7 @@ constexpr int kChunk = 64 * 128, kRing = 20;
 // operand of s_waitcnt: no LDS access and at most n loads on their way
 constexpr int flow_wait(int n) { return 0x70 | (n & 15) | n >> 4 << 14; }
 
-template <int NX, int WR, bool GLU>
+template <int NX, int WR, bool GLU, bool NT>
 __device__ __forceinline__ void gg_flow_tile(char* smem, const bf16* const (&wp)[WR / 64], const bf16* const (&xp)[4], int KT,
                                              int turn, f32x16 (&acc)[2][WR / 64]) {
   constexpr int CW = WR / 64, C = CW + NX, TG = 8 / CW, NB = (2 * NX + TG - 1) / TG;
@@ -332,7 +332,9 @@ __device__ __forceinline__ void gg_flow_tile(char* smem, const bf16* const (&wp)
     s += turn;
     const int64_t k0 = (int64_t)(s < KT ? s : s - KT) * BK2;
     const bf16* src = i < CW ? wp[i < CW ? i : 0] : xp[i < CW ? 0 : i - CW];
-    __builtin_amdgcn_global_load_lds((gbl_void*)(src + k0), (lds_void*)(smem + place * kChunk + w * 1024), 16, 0, 0);
+    char* to = smem + place * kChunk + w * 1024;
+    if (NT && i < CW) __builtin_amdgcn_global_load_lds((gbl_void*)(src + k0), (lds_void*)to, 16, 0, 2);
+    else __builtin_amdgcn_global_load_lds((gbl_void*)(src + k0), (lds_void*)to, 16, 0, 0);
   };
   auto wrap = [](int p) { return p < R ? p : p - R; };
 #pragma unroll
@@ -395,7 +397,7 @@ __device__ __forceinline__ void gg_flow_tile(char* smem, const bf16* const (&wp)
   }
 }
 
-template <bool GATHER, bool GLU, int WR>
+template <bool GATHER, bool GLU, int WR, bool NT>
 __global__ __launch_bounds__(512) void gg_flow_kernel(const bf16* __restrict__ x, int64_t ldx,
                                                       const int* __restrict__ src, int n_src,
                                                       const bf16* __restrict__ w, bf16* __restrict__ y,
@@ -436,10 +438,10 @@ __global__ __launch_bounds__(512) void gg_flow_kernel(const bf16* __restrict__ x
     for (int j = 0; j < CW; ++j) acc[i][j] = f32x16{};
   const int nx = (min(rows - m0, BM2) + 63) / 64, KT = K / BK2;
   const int turn = apart ? (int)__umulhi(blockIdx.x * 2654435769u, (unsigned)KT) : 0;
-  if (nx <= 1) gg_flow_tile<1, WR, GLU>(smem, wp, xp, KT, turn, acc);
-  else if (nx == 2) gg_flow_tile<2, WR, GLU>(smem, wp, xp, KT, turn, acc);
-  else if (nx == 3) gg_flow_tile<3, WR, GLU>(smem, wp, xp, KT, turn, acc);
-  else gg_flow_tile<4, WR, GLU>(smem, wp, xp, KT, turn, acc);
+  if (nx <= 1) gg_flow_tile<1, WR, GLU, NT>(smem, wp, xp, KT, turn, acc);
+  else if (nx == 2) gg_flow_tile<2, WR, GLU, NT>(smem, wp, xp, KT, turn, acc);
+  else if (nx == 3) gg_flow_tile<3, WR, GLU, NT>(smem, wp, xp, KT, turn, acc);
+  else gg_flow_tile<4, WR, GLU, NT>(smem, wp, xp, KT, turn, acc);
 
   // lane = token, registers 4g .. 4g + 3 = 4 consecutive output features
   const int h = lane >> 5, p = wv % CW, tg = wv / CW;
@@ -559,6 +561,7 @@ HDS_EXPORT int hds_experts_gemm(const void* x, int64_t ldx, const int* src, int 
   // 256 x 256 tiles, which read the rows half as often and the weights once per 256 of them, from 512 rows an expert on: 8
   // experts, 2 a token, 14336 x 4096: 1,500 tokens 1,774 us against 1,534 here, 2,000 2,063 / 2,054, 2,700 2,390 / 2,488; 64
   // experts, 6 a token, 1024 x 2048: 3,000 540 / 427, 6,000 786 / 733, 12,000 1,262 / 1,315.
+  const int cols_of = glu ? 2 : 1;
   const bool big = N % big_cols == 0 && T >= 2 * BM2 * E;
   // otherwise gg_flow_kernel's tiles
   const FlowTile flow = flow_tile(T, N, K, E, glu);
@@ -571,12 +574,22 @@ HDS_EXPORT int hds_experts_gemm(const void* x, int64_t ldx, const int* src, int 
     hipLaunchKernelGGL(kernel, dim3(N / cols * max_tiles), dim3(512), 0, st, (const bf16*)x, ldx, src, n_src, (const bf16*)w,
                        (bf16*)y, offs, tile_e, tile_m, n_tiles, T, N, K, ldy, N / cols, unit, more...);
   };
+  // Weights that one tile of rows reads go past the caches: 66 tokens, gate and up + down, 64 experts of 1024 x 2048 98.5 + 53.8 -> 87 + 46
+  // us, 8 of 14336 x 4096 325 + 160 -> 297 + 140, 16 of 4096 x 4096 199 + 92 -> 180 + 80; 1,600 131 + 80 -> 128 + 74. Tiles of one expert
+  // find them in L2 or the memory-side cache (past it 3,000 tokens of the first, gate and up 235 / 252, 1,400 of 8 of 5632 x 2048
+  // 191 / 202), unless an expert's are too many (2,090 choices of 8 of 14336 x 4096, 117 and 235 MB, a layer 1,470 -> 1,333).
+  const bool once = T <= BM2 * E || (int64_t)cols_of * N * K >= 1 << 25;
+#define HDS_FLOW(GA, GL, NT)                                               \
+  do {                                                                     \
+    if (wr == 256) run(gg_flow_kernel<GA, GL, 256, NT>, apart);            \
+    else if (wr == 128) run(gg_flow_kernel<GA, GL, 128, NT>, apart);       \
+    else run(gg_flow_kernel<GA, GL, 64, NT>, apart);                       \
+  } while (0)
 #define HDS_EG(GA, GL)                                                     \
   do {                                                                     \
     if (big) run(gg_big_kernel<GA, GL>);                                   \
-    else if (wr == 256) run(gg_flow_kernel<GA, GL, 256>, apart);           \
-    else if (wr == 128) run(gg_flow_kernel<GA, GL, 128>, apart);           \
-    else run(gg_flow_kernel<GA, GL, 64>, apart);                           \
+    else if (once) HDS_FLOW(GA, GL, true);                                 \
+    else HDS_FLOW(GA, GL, false);                                          \
   } while (0)
   if (src != nullptr) {
     if (glu) HDS_EG(true, true); else HDS_EG(true, false);
@@ -584,5 +597,6 @@ HDS_EXPORT int hds_experts_gemm(const void* x, int64_t ldx, const int* src, int 
     if (glu) HDS_EG(false, true); else HDS_EG(false, false);
   }
 #undef HDS_EG
+#undef HDS_FLOW
   return hipGetLastError();
 }

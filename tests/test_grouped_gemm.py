@@ -156,6 +156,14 @@ def test_experts_gemm_tiles_of_weight_rows(cuda, counts, N, K, gather, glu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,K,gather,glu", [(8192, 384, False, True), (16384, 128, True, False), (4096, 2048, True, True),
+                                            (8192, 2048, False, False), (1024, 4096, False, False)])
+def test_experts_gemm_weights_of_several_row_tiles(cuda, N, K, gather, glu):
+    """More rows an expert than a tile holds: weights through the caches, whatever the tile of weight rows."""
+    test_experts_gemm_hip(cuda, [300, 420], N, K, gather, glu)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("E,k,T,N,K,glu,rows,apart", [
     (8, 2, 66, 14336, 4096, 1, 128, 1), (8, 2, 300, 14336, 4096, 1, 256, 0), (16, 4, 66, 6400, 4096, 1, 128, 1),
     (4, 1, 66, 8192, 4096, 1, 256, 1), (64, 6, 66, 1024, 2048, 1, 256, 1), (64, 6, 3000, 1024, 2048, 1, 256, 0),
