@@ -6,8 +6,9 @@
 // in the mainloop so the weight stream stays at 8 / 6 / 4 bits; this kernel does the same on MFMA.
 //
 // Regime: 8 < M <= a few hundred rows (batched decode, chunked prefill) where a bf16 GEMM is bound by the 16-bit
-// weight stream. Decode-sized M (<= 8) runs the GEMVs (quant.hip / fpq.hip); prefill-sized M dequantizes once and
-// runs hipBLASLt (compute-bound there, so the weight bytes no longer matter).
+// weight stream, and groups or rows that linear_packed.hip does not take (it is 1.2 to 3 times as fast). Decode-sized M (<= 8)
+// runs the GEMVs (quant.hip / fpq.hip); prefill-sized M dequantizes once and runs hipBLASLt (compute-bound there, so the weight
+// bytes no longer matter).
 //
 // Structure: workgroup = 4 waves = 512 weight rows (wave = 4 fragments of 32 rows, the weight row on the MFMA lane)
 // x 32*MB activation rows, over one K split. Per 64-k chunk a lane reads 32 consecutive k of each of its 4 weight
@@ -18,7 +19,7 @@
 // version that read A per 32-row wave from L2 moved 2x (M = 16) to 30x (M = 256) more A bytes than weight bytes
 // and ran at 0.2-0.8x the bf16 GEMM. The next chunk's weights and A are loaded before the current chunk's MFMAs.
 // K splits (grid.z) write fp32 partials reduced by wmix_reduce_kernel.
-#include "hds_common.h"
+#include "packed_codes.h"
 
 namespace {
 using namespace hds;
@@ -28,13 +29,6 @@ __device__ __forceinline__ f32x16 mma(const bf16x8& a, const bf16x8& b, const f3
 }
 
 __device__ __forceinline__ int acc_row(int r, int h) { return (r & 3) + 8 * (r >> 2) + 4 * h; }
-
-enum WFmt : int { kInt8 = 0, kInt4 = 1, kFp6 = 2 };
-
-template <int FMT> struct WRaw;
-template <> struct WRaw<kInt8> { uint4 a, b; };
-template <> struct WRaw<kInt4> { uint4 a; };
-template <> struct WRaw<kFp6> { uint2 a, b, c; };
 
 // raw bytes of the 32 weights k = ks .. ks + 31 of row n
 template <int FMT>
@@ -234,43 +228,6 @@ __global__ __launch_bounds__(256) void wmix_reduce_kernel(const float* __restric
 // of unsigned nibbles subtracted, 7.1 without). Measured at 8 rows, [28672, 4096] / [4096, 14336]: fp6 38 / 22 us (92 / 46 MB;
 // the GEMV that decodes and multiplies on the VALU 112 / 77), int8 39 / 20 (121 / 61 MB; the tile kernel above 45 / 28), int4
 // 29 / 16 (41 / 29). What is left to it are the sizes that the two kernels below do not gain on.
-typedef uint32_t u32x6 __attribute__((ext_vector_type(6)));
-typedef __bf16 bf16x32 __attribute__((ext_vector_type(32)));
-
-template <int FMT>
-constexpr float kUnit = FMT == kInt4 ? 0.0625f : 1.f;
-
-template <int FMT, int E>
-__device__ __forceinline__ void codes(const WRaw<FMT>& r, bf16x8 (&f)[4]) {
-  if constexpr (FMT == kFp6) {
-    const u32x6 q = {r.a.x, r.a.y, r.b.x, r.b.y, r.c.x, r.c.y};
-    bf16x32 v;
-    if constexpr (E == 3) v = __builtin_amdgcn_cvt_scalef32_pk32_bf16_bf6(q, 1.f);  // "bf6" is e3m2
-    else v = __builtin_amdgcn_cvt_scalef32_pk32_bf16_fp6(q, 1.f);
-    f[0] = __builtin_shufflevector(v, v, 0, 1, 2, 3, 4, 5, 6, 7);
-    f[1] = __builtin_shufflevector(v, v, 8, 9, 10, 11, 12, 13, 14, 15);
-    f[2] = __builtin_shufflevector(v, v, 16, 17, 18, 19, 20, 21, 22, 23);
-    f[3] = __builtin_shufflevector(v, v, 24, 25, 26, 27, 28, 29, 30, 31);
-  } else if constexpr (FMT == kInt8) {
-    const uint32_t dw[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) f[i >> 1][4 * (i & 1) + t] = (bf16)(float)(int8_t)(dw[i] >> (8 * t));
-  } else {
-    const uint32_t dw[4] = {r.a.x, r.a.y, r.a.z, r.a.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {  // in the upper halves of bytes, with their sign: 16 times the code (kUnit)
-      const uint32_t lo = (dw[i] << 4) & 0xf0f0f0f0u, hi = dw[i] & 0xf0f0f0f0u;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        f[i][2 * t] = (bf16)(float)(int8_t)(lo >> (8 * t));
-        f[i][2 * t + 1] = (bf16)(float)(int8_t)(hi >> (8 * t));
-      }
-    }
-  }
-}
-
 // GLU: W is [gate; up] of 2 N rows, a tile of 16 weight rows holds 8 gate rows and their 8 up rows (as many workgroups as
 // without), and the result is bf16(act(bf16(gate)) * bf16(up)) [M, N].
 template <bool GLU>

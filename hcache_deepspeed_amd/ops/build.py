@@ -45,6 +45,7 @@ FILE_FLAGS = {"flash_attn.hip": ["-fno-slp-vectorize"],
               "flash_attn_bwd_w64.hip": ["-fno-slp-vectorize", "-mllvm", "-amdgpu-mfma-vgpr-form"],
               # whole tiles of accumulators beside the fragments of two halves: moves from and to AGPRs cost as much as the products
               "linear.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+              "linear_packed.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               # the chunk scan works on its accumulators with vector instructions too: no moves from and to AGPRs
               "delta_rule.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
               "matrix_memory.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}

@@ -120,6 +120,8 @@ _KERNEL_SIGS = {
     "hds_gemv_bf16": "pppp" + "iii" + "ll" + "s",
     "hds_gemv_fused_bf16": "ppp" + "f" + "pppp" + "if" + "iii" + "ll" + "s",
     "hds_gather_gemv_bf16": "ppp" + "l" + "p" + "ii" + "p" + "iii" + "ll" + "s",
+    "hds_packed_slices": "iiiiii",
+    "hds_packed_rows": "pppppp" + "iiiiiii" + "s",
     "hds_linear_slices": "iiii",
     "hds_linear_bf16": "plppplp" + "iiii" + "s",
     "hds_skinny_gemm_bf16": "pppp" + "iii" + "ll" + "i" + "s",
@@ -329,9 +331,14 @@ def check(err, what):
 
 def plain(*tensors):
     """No gradient, functorch transform, dual number or trace can want a record of what is done with these tensors: an autograd
-    function around a kernel (about 10 us of host time) may be passed by. (A trace holds the function as one node that runs it
-    again; of a bare kernel it would see the allocation of the result only.)"""
-    return (not torch.is_grad_enabled() and not torch._C._are_functorch_transforms_active()
+    function around a kernel (about 10 us of host time) may be passed by."""
+    return not torch.is_grad_enabled() and bare(*tensors)
+
+
+def bare(*tensors):
+    """``plain`` beside gradients, which the caller has looked for itself. (A trace holds an autograd function as one node that
+    runs it again; of a bare kernel it would see the allocation of the result only.)"""
+    return (not torch._C._are_functorch_transforms_active()
             and torch.autograd.forward_ad._current_level < 0 and torch._C._get_tracing_state() is None
             and all(t is None or type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors))
 

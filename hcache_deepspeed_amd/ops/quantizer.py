@@ -5,6 +5,7 @@ Reference parity: ops/quantizer (``ds_quantizer``, csrc/quantization pt_binding:
 (``FP_Quantize.quantize/dequantize/selective_dequantize`` :43). GPU path: csrc/kernels/quant.hip; CPU
 path: the same math in torch (used by the CPU tests and as the numerics reference).
 """
+import functools
 import os
 
 import torch
@@ -166,7 +167,7 @@ def wmix_gemm(x2, q_weight, scales, out_features, in_features, group_size, fmt, 
         bias = bias.to(torch.bfloat16).contiguous()
     native.check(lib.hds_wmix_gemm(x2.data_ptr(), q_weight.data_ptr(), scales.data_ptr(), native.ptr(bias),
                                    y.data_ptr(), native.ptr(ws), M, out_features, in_features, group_size,
-                                   {"int8": 0, "int4": 1, "fp6": 2}[fmt], int(ebits), native.stream()), "wmix_gemm")
+                                   _FMTS[fmt], int(ebits), native.stream()), "wmix_gemm")
     return y
 
 
@@ -187,15 +188,48 @@ def _gemv_wins(M, out_features, in_features, fmt):
     return M == 1 and weights < (48_000_000 if in_features > 8192 else 100_000_000) or M == 2 and weights < 4_000_000
 
 
+_FMTS = {"int8": 0, "int4": 1, "fp6": 2}
+
+
+@functools.lru_cache(maxsize=4096)
+def _packed_slices(M, N, K, group_size, fmt, glu):
+    """Slices of K on csrc/kernels/linear_packed.hip, 0 for products that stay with the other kernels."""
+    return int(native.kernels().hds_packed_slices(M, N, K, group_size, _FMTS[fmt], glu)) if max(M, N, K) < 1 << 30 else 0
+
+
+def _packed_rows(x2, q_weight, scales, out_features, in_features, group_size, fmt, ebits, bias, glu):
+    """The packed-weight product of more rows (csrc/kernels/linear_packed.hip): mostly 17 to 256; None where it does not apply or
+    anything could want a record of it."""
+    M, N, K = x2.shape[0], out_features, in_features
+    S = _packed_slices(M, N, K, group_size, fmt, 1 if glu else 0)
+    if S == 0 or not native.bare(x2, q_weight, bias) or (bias is not None and _needs_grad(bias)):
+        return None
+    x2 = x2.contiguous()
+    if (x2.data_ptr() | q_weight.data_ptr()) % 16 or (bias is not None and bias.dtype != torch.bfloat16):
+        return None
+    if bias is not None:
+        bias = bias.contiguous()
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=x2.device)
+    part = torch.empty(S, M, 2 * N if glu else N, dtype=torch.float32, device=x2.device) if S > 1 else None
+    native.check(native.kernels().hds_packed_rows(x2.data_ptr(), q_weight.data_ptr(), scales.data_ptr(), native.ptr(bias),
+                                                  y.data_ptr(), native.ptr(part), M, N, K, group_size, _FMTS[fmt], int(ebits),
+                                                  int(glu), native.stream()), "packed_rows")
+    return y
+
+
 def _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, fmt, ebits=3, bias=None, glu=0):
     """The packed-weight stream for few rows (csrc/kernels/wmix_gemm.hip ``wmix_skinny_kernel``), or None where it does not
-    apply (rows of whole groups of a multiple of 128; fp6 as e3m2 or e2m3). It wins up to 16 rows, with fp6 up to 32
-    ([28672, 4096], 24 rows: fp6 57 us against the tile kernel's 78, int8 61 against 50; fp6 at 32 rows 87 against 78, but the
-    tile kernel rounds the weights), one row of int8 only where the stream's rows stay resident (see ``_gemv_wins``)."""
+    apply (rows of whole groups of a multiple of 128; fp6 as e3m2 or e2m3). More rows, and some of 4 to 16, go
+    to ``_packed_rows``; the stream takes up to 16, of small fp6 weights up to 32 ([2048, 2048], 24 rows: 0.97 of the time of the
+    tiles), and one row of int8 only where its rows stay resident (see ``_gemv_wins``)."""
     M = x2.shape[0]
     if (_needs_grad(x2) or not native.use_native(x2) or x2.dtype != torch.bfloat16 or in_features % 128
-            or group_size % 128 or in_features % group_size or (fmt == "fp6" and ebits not in (2, 3))
-            or not 0 < M <= (32 if fmt == "fp6" and not glu else 16)):
+            or group_size % 128 or in_features % group_size or (fmt == "fp6" and ebits not in (2, 3))):
+        return None
+    y = _packed_rows(x2, q_weight, scales, out_features, in_features, group_size, fmt, ebits, bias, glu)
+    if y is not None:
+        return y
+    if not 0 < M <= (32 if fmt == "fp6" and not glu else 16):
         return None
     if fmt == "int8" and M == 1 and (bias is not None or not native.kernels().hds_wmix_resident(
             M, out_features * (2 if glu else 1), in_features)):
@@ -212,7 +246,7 @@ def _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, fm
     y = torch.empty(M, out_features, dtype=torch.bfloat16, device=x2.device)
     native.check(native.kernels().hds_wmix_skinny(x2.data_ptr(), q_weight.data_ptr(), scales.data_ptr(),
                                                   native.ptr(bias), y.data_ptr(), M, out_features, in_features,
-                                                  group_size, {"int8": 0, "int4": 1, "fp6": 2}[fmt], int(ebits), int(glu),
+                                                  group_size, _FMTS[fmt], int(ebits), int(glu),
                                                   native.stream()), "wmix_skinny")
     return y
 
@@ -235,8 +269,9 @@ def int_linear(x, q_weight, scales, out_features, in_features, group_size, bits=
 
     Up to 16 rows stream the packed weight through the matrix cores (``_wmix_skinny``, groups of a multiple of 128; one row
     of int8, one and two rows where ``_gemv_wins``, other groups and a bias that is not bf16 up to 2 rows, ``HDS_INT_GEMV_MAX_M``: the HIP GEMV of
-    csrc/kernels/quant.hip); batches of up to 64 rows run the tile kernel on packed weights, larger ones and groups that do
-    not divide a row dequantize once to bf16."""
+    csrc/kernels/quant.hip); batches of up to 256 rows, of small weights 512, run tiles on packed weights (``_packed_rows``; groups
+    of a multiple of 32 only, up to 64 rows, ``wmix_gemm``), larger ones and groups that do not divide a row dequantize once to
+    bf16."""
     lead = x.shape[:-1]
     x2 = x.reshape(-1, in_features)
     M = x2.shape[0]
@@ -485,8 +520,9 @@ def fp6_linear(x, q_weight, scales, out_features, in_features, group_size, manti
     """y = x @ dequant(W)^T for an FP6-packed weight [out, in] (row-major, groups along ``in``).
 
     Up to 32 rows stream the packed weight through the matrix cores (``_wmix_skinny``, groups of a multiple of 128; other
-    groups up to 8 rows and one row where ``_gemv_wins``: the HIP GEMV of csrc/kernels/fpq.hip); batches of up to 64 rows run the tile kernel on packed
-    weights, larger ones dequantize once to bf16 and use hipBLASLt."""
+    groups up to 8 rows and one row where ``_gemv_wins``: the HIP GEMV of csrc/kernels/fpq.hip); batches of up to 256 rows, of small
+    weights 512, run tiles on packed weights (``_packed_rows``; groups of a multiple of 32 only, up to 64 rows, ``wmix_gemm``), larger
+    ones dequantize once to bf16 and use hipBLASLt."""
     lead = x.shape[:-1]
     x2 = x.reshape(-1, in_features)
     M = x2.shape[0]

@@ -1,0 +1,61 @@
+"""Products of more rows on packed weights (csrc/kernels/linear_packed.hip)."""
+import pytest
+import torch
+
+from hcache_deepspeed_amd.ops import quantizer as Q
+
+pytestmark = pytest.mark.gpu
+
+
+def _packed(fmt, N, K, G):
+    w = torch.randn(N, K, device="cuda", dtype=torch.bfloat16) * K**-0.5
+    if fmt.startswith("int"):
+        q, s, _ = Q.quantize(w.reshape(-1), G, int(fmt[3:]), True)
+        return q, s, Q.dequantize(q, s, None, G, int(fmt[3:]), True, torch.float32).view(N, K).double()
+    mb = 2 if fmt.endswith("e3m2") else 3
+    q, s = Q.quantize_minifloat(w.reshape(-1), G, 6, mb)
+    return q, s, Q.dequantize_minifloat(q, s, G, 6, mb, torch.float32).view(N, K).double()
+
+
+@pytest.mark.parametrize("fmt", ["int8", "int4", "fp6_e3m2", "fp6_e2m3"])
+@pytest.mark.parametrize("M,N,K,G", [(17, 68, 256, 128), (24, 4100, 2048, 128), (32, 12296, 1152, 384), (33, 1000, 640, 128),
+                                     (64, 4104, 4224, 128), (65, 520, 5632, 256), (100, 16392, 1024, 1024), (128, 2052, 896, 128),
+                                     (256, 3080, 1152, 128), (512, 260, 4096, 4096), (16, 8204, 8320, 128)])
+def test_rows_on_packed_weights(fmt, M, N, K, G):
+    """All tiles, with remainders of rows and of weight rows; one slice and several, whose groups begin inside a slice; a bias.
+    The codes are exact in bf16: 32-bit sums of K exact products, each rounded once more with its scale, and the result's rounding."""
+    torch.manual_seed(K + M)
+    x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
+    q, s, wd = _packed(fmt, N, K, G)
+    assert N * K < 1 << 23 and M <= 32 and fmt[0] == "f" or Q._packed_slices(M, N, K, G, fmt[:4] if fmt[0] == "i" else "fp6", 0)
+    if fmt[0] == "i":
+        bias = torch.randn(N, device="cuda").bfloat16()
+        y = Q.int_linear(x, q, s, N, K, G, bits=int(fmt[3:]), bias=bias)
+    else:
+        bias = torch.zeros(N, device="cuda").bfloat16()
+        y = Q.fp6_linear(x, q, s, N, K, G, 2 if fmt.endswith("e3m2") else 3)
+    ref = x.double() @ wd.t() + bias.double()
+    bound = 2**-8 * ref.abs() + 1e-5 * (x.double().abs() @ wd.abs().t() + bias.double().abs())
+    assert ((y.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("fmt", ["int8", "int4", "fp6"])
+@pytest.mark.parametrize("M,N,K,act", [(17, 36, 256, "silu"), (32, 4100, 4224, "gelu_tanh"), (64, 2052, 1024, "relu"),
+                                       (100, 1028, 8320, "silu"), (256, 516, 640, "silu")])
+def test_gated_rows_on_packed_weights(fmt, M, N, K, act):
+    """The gated unit in the epilogue and in the sum of slices, tiles of 32 and 64 columns with remainders."""
+    torch.manual_seed(K + M)
+    x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
+    q, s, wd = _packed(fmt if fmt[0] == "i" else "fp6_e3m2", 2 * N, K, 128)
+    y = Q.packed_glu(x, q, s, N, K, 128, fmt, act)
+    if fmt == "fp6" and M <= 32 and 2 * N * K < 1 << 23:
+        assert y is None
+        return
+    gate, up = (x.double() @ wd.t()).split(N, 1)
+    f = {"silu": torch.nn.functional.silu, "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh"),
+         "relu": torch.relu}[act]
+    ref = f(gate) * up
+    eg, eu = (1e-5 * (x.double().abs() @ wd.abs().t())).split(N, 1)
+    # each factor within half a unit of the last place and its sum's error; |act'| <= 1.13
+    bound = 2**-8 * (1.13 * gate.abs() * up.abs() + 2 * ref.abs()) + 1.13 * (eg * up.abs() + eu * gate.abs()) + 1e-6
+    assert ((y.double() - ref).abs() <= bound).all()
