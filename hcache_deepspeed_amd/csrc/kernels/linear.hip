@@ -204,9 +204,9 @@ static int linear_choice(int M, int N, int K) {
 
 }  // namespace
 
-// Slices of K with which hds_linear_bf16 takes these rows, or 0 where a library product is the faster one. N: columns of y; glu:
-// of 2N rows of w.
-HDS_EXPORT int hds_linear_slices(int M, int N, int K, int glu) {
+// How hds_linear_bf16 takes these rows, as tile + 16 x slices of K, or 0 where a library product is the faster one. N: columns of
+// y; glu: of 2N rows of w. For callers to keep by size: the estimates take 3 us of the host.
+HDS_EXPORT int hds_linear_plan(int M, int N, int K, int glu) {
   if (M < 9 || M > 1100 || N < 8 || K < 4 * BK || K % BK || N % 8 || K > 1 << 22 || N > 1 << 22) return 0;
   const int rows = glu ? 2 * N : N;
   const int64_t size = (int64_t)rows * K;
@@ -218,7 +218,7 @@ HDS_EXPORT int hds_linear_slices(int M, int N, int K, int glu) {
   //   steps of short prompts. Up to 16 rows where the matrix is large and not sliced: [28672, 4096] 8 / 12 / 16 rows 38.8 / 42.6 /
   //   45.1 -> 37.3 / 37.3 / 37.5, [32000, 4096] 41.5 / 44.9 / 49.2 -> 40.0 / 40.4 / 40.4; smaller ones 0.6 - 1.03.
   const int choice = linear_choice(M, rows, K), S = choice / 16;
-  if (M <= 16) return S == 1 && size >= 1 << 25 ? S : 0;
+  if (M <= 16) return S == 1 && size >= 1 << 25 ? choice : 0;
   // 17 to 32 are decode steps, whose launches are recorded once: smaller matrices are the library's ([2048, 2048], 24 rows 8.2 us in
   // a step / 10.4).
   if (M <= 32 && !glu && size < 3 << 23) return 0;
@@ -231,19 +231,21 @@ HDS_EXPORT int hds_linear_slices(int M, int N, int K, int glu) {
   // - long reductions into few columns, whatever the rows: [4096, 14336] 1.0 - 2.3, [5120, 13824] 0.94 - 2.4. Beyond, the library's
   //   products are the faster ones (521 rows: [28672, 4096] 0.8, [11264, 2048] 0.85, [6144, 4096] 1.0).
   take = take || (K >= 8192 && 2 * rows <= K && size >= 1 << 24);
-  return take ? S : 0;
+  return take ? choice : 0;
 }
 
-// x [M, ldx], w [N, K], bias [N] or null, y [M, ldy], part: S x M x N floats where the slices S (hds_linear_slices) are more
+// x [M, ldx], w [N, K], bias [N] or null, y [M, ldy], plan: hds_linear_plan's, part: S x M x N floats where its slices S are more
 // than one. glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu): w [2N, K] is gate rows, then up rows, y = act(gate) up,
 // and bias and part are of 2N columns. Rows of x and w begin at 16 bytes, of y at 8.
 HDS_EXPORT int hds_linear_bf16(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy, float* part,
-                               int M, int N, int K, int glu, hipStream_t st) {
-  const int S = hds_linear_slices(M, N, K, glu);
-  if (S < 1 || ldx < K || ldx % 8 || ldx > 1 << 22 || ldy < N || ldy % 4 || (S > 1 && part == nullptr) || glu < 0 || glu > 3 ||
-      ((uintptr_t)x | (uintptr_t)w) & 15 || (uintptr_t)y & 7)
+                               int M, int N, int K, int glu, int plan, hipStream_t st) {
+  const int S = plan / 16, tile = plan % 16;
+  if (M < 1 || M > 1100 || N < 8 || K < 4 * BK || K % BK || N % 8 || K > 1 << 22 || N > 1 << 22 || glu < 0 || glu > 3 ||
+      (int64_t)(glu ? 2 * N : N) * K >= (int64_t)1 << 31 || S < 1 || S > kMaxSlices || S > K / BK || tile < 0 ||
+      tile >= (int)(sizeof(kTiles) / sizeof(Tile)) || (S > 1 && part == nullptr) || ldx < K || ldx % 8 || ldx > 1 << 22 || ldy < N ||
+      ldy % 4 || ((uintptr_t)x | (uintptr_t)w) & 15 || (uintptr_t)y & 7)
     return hipErrorInvalidValue;
-  const int rows = glu ? 2 * N : N, tile = linear_choice(M, rows, K) % 16, R = kTiles[tile].rows, W = kTiles[tile].cols;
+  const int rows = glu ? 2 * N : N, R = kTiles[tile].rows, W = kTiles[tile].cols;
   LinearArgs p{(const bf16*)x, (const bf16*)w, (const bf16*)bias, (bf16*)y, part, ldx, ldy, M, N, K, S, (M + R - 1) / R,
                (rows + W - 1) / W, glu - 1, 0, K % 2048 == 0};
   if (glu) p.tn = (N + W / 2 - 1) / (W / 2);

@@ -235,9 +235,9 @@ static int packed_choice(int M, int N, int K, int G, int fmt) {
 
 }  // namespace
 
-// Slices of K with which hds_packed_rows takes these rows, or 0 where other kernels are faster or it does not apply. N: columns
-// of y; glu: of 2N rows of w; fmt: 0 int8, 1 int4, 2 fp6.
-HDS_EXPORT int hds_packed_slices(int M, int N, int K, int G, int fmt, int glu) {
+// How hds_packed_rows takes these rows, as tile + 16 x slices of K, or 0 where other kernels are faster or it does not apply. N:
+// columns of y; glu: of 2N rows of w; fmt: 0 int8, 1 int4, 2 fp6. For callers to keep by size, as hds_linear_plan.
+HDS_EXPORT int hds_packed_plan(int M, int N, int K, int G, int fmt, int glu) {
   if (M < 4 || M > 512 || N < 4 || N % 4 || K < 2 * BK || K % BK || G < BK || G % BK || K % G || fmt < 0 || fmt > 2 ||
       N > 1 << 22 || K > 1 << 20)
     return 0;
@@ -258,19 +258,21 @@ HDS_EXPORT int hds_packed_slices(int M, int N, int K, int G, int fmt, int glu) {
   // - beyond, the weights are decoded for more rows than it saves passes: [28672, 4096] 384 / 512 rows 0.91 / 0.76; small matrices
   //   gain by their launches ([2048, 2048] 1.1 / 1.2 - 1.4, [4096, 4096] 1.05 - 1.1 / 1.05 - 1.14, [6144, 4096] 0.9).
   if (M > 256 && (size > 1 << 24 || K > 4096)) return 0;
-  return packed_choice(M, rows, K, G, fmt) / 16;
+  return packed_choice(M, rows, K, G, fmt);
 }
 
-// x [M, K], w packed, scales [N, K / G], bias [N] or null, y [M, N], part: S x M x N floats where the slices S (hds_packed_slices)
-// are more than one. ebits: fp6 3 (e3m2) or 2 (e2m3). glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu): w is 2N rows,
+// x [M, K], w packed, scales [N, K / G], bias [N] or null, y [M, N], plan: hds_packed_plan's, part: S x M x N floats where its
+// slices S are more than one. ebits: fp6 3 (e3m2) or 2 (e2m3). glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu): w is 2N rows,
 // gate, then up, without a bias, and part of 2N columns. x and w begin at 16 bytes, y at 8.
 HDS_EXPORT int hds_packed_rows(const void* x, const void* w, const float* scales, const void* bias, void* y, float* part, int M,
-                               int N, int K, int G, int fmt, int ebits, int glu, hipStream_t st) {
-  const int S = hds_packed_slices(M, N, K, G, fmt, glu);
-  if (S < 1 || (S > 1 && part == nullptr) || glu < 0 || glu > 3 || (glu && bias) || ((uintptr_t)x | (uintptr_t)w) & 15 ||
-      (uintptr_t)y & 7)
+                               int N, int K, int G, int fmt, int ebits, int glu, int plan, hipStream_t st) {
+  const int S = plan / 16, tile = plan % 16, stages = S < 1 ? 0 : (K / BK + S - 1) / S;
+  if (M < 1 || M > 512 || N < 4 || N % 4 || K < BK || K % BK || G < BK || G % BK || K % G || glu < 0 || glu > 3 || (glu && bias) ||
+      N > 1 << 22 || K > 1 << 20 || (int64_t)(glu ? 2 * N : N) * K >= (int64_t)1 << 31 || S < 1 || S > kMaxSlices || S > K / BK ||
+      std::min(stages, stages * BK / G + 2) > kGroups || tile < 0 || tile >= (int)(sizeof(kTiles) / sizeof(Tile)) ||
+      (S > 1 && part == nullptr) || ((uintptr_t)x | (uintptr_t)w) & 15 || (uintptr_t)y & 7)
     return hipErrorInvalidValue;
-  const int rows = glu ? 2 * N : N, tile = packed_choice(M, rows, K, G, fmt) % 16, R = kTiles[tile].rows, W = kTiles[tile].cols;
+  const int rows = glu ? 2 * N : N, R = kTiles[tile].rows, W = kTiles[tile].cols;
   // Weights that one row of tiles reads go past the caches where a stage's share of a row is a whole line: int8 [28672, 4096] 16 /
   // 64 rows 27.8 / 37.2 -> 25.8 / 36.8 us; fp6's three quarters of one 28.3 -> 33 us at 24 rows.
   PackedArgs p{(const bf16*)x, (const uint8_t*)w, scales, (const bf16*)bias, (bf16*)y, part, M, N, K, G, S, (M + R - 1) / R,

@@ -74,41 +74,44 @@ def skinny(x2, w, b=None):
     return y
 
 
-# 9 to 1,100 rows: csrc/kernels/linear.hip where hds_linear_slices takes them (HDS_LINEAR=0: never)
-LINEAR = _os.environ.get("HDS_LINEAR", "1") == "1"
+# 9 to 1,100 rows: csrc/kernels/linear.hip where hds_linear_plan takes them
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
 @functools.lru_cache(maxsize=4096)
-def _slices(M, N, K, glu=0):
-    """Slices of K on csrc/kernels/linear.hip, 0 for products that stay the library's."""
-    return int(native.kernels().hds_linear_slices(M, N, K, glu)) if LINEAR and max(M, N, K) < 1 << 31 else 0
+def _plan(M, N, K, glu=0):
+    """Tile + 16 x slices of K on csrc/kernels/linear.hip, 0 for products that stay the library's."""
+    return int(native.kernels().hds_linear_plan(M, N, K, glu)) if max(M, N, K) < 1 << 31 else 0
 
 
 def rows_linear(x, w, b=None, glu=0):
     """``F.linear(x, w, b)`` of 9 rows and more, or with ``glu`` = 1 + activation code the gated unit of w = [gate; up]; None
     where the kernel does not take the call, as where anything could want a record of it (``native.plain``)."""
-    if not x.is_cuda or not native.plain(x, w, b) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() < 1 or \
-            w.dim() != 2 or not w.is_contiguous():
+    # (sizes first: a call of a prompt that stays the library's pays 2 us less for having asked)
+    if type(x) not in _TENSORS or not x.is_cuda or torch._C._get_tracing_state() is not None:
         return None
-    K = x.shape[-1]
-    if not 0 < K == w.shape[1] or w.get_device() != x.get_device():
+    shape = x.shape
+    K = shape[-1] if len(shape) else 0
+    if K == 0:
         return None
-    M, N = x.numel() // K, w.shape[0] // 2 if glu else w.shape[0]
-    S = _slices(M, N, K, 1 if glu else 0)
-    if S == 0:
+    rows = w.shape[0]
+    M, N = x.numel() // K, rows // 2 if glu else rows
+    plan = _plan(M, N, K, 1 if glu else 0)
+    if plan == 0 or not native.plain(x, w, b) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.dim() != 2 or \
+            not w.is_contiguous() or K != w.shape[1] or w.get_device() != x.get_device():
         return None
     x2 = x if x.dim() == 2 else x.reshape(M, K)
     ld, one = x2.stride()
     px, pw = x2.data_ptr(), w.data_ptr()
-    if one != 1 or ld % 8 or not K <= ld <= 1 << 22 or (px | pw) % 16 or (glu and w.shape[0] % 2):
+    if one != 1 or ld % 8 or not K <= ld <= 1 << 22 or (px | pw) % 16 or (glu and rows % 2):
         return None
     if b is not None and (b.dtype != torch.bfloat16 or not b.is_contiguous() or b.shape != w.shape[:1] or
                           b.get_device() != x.get_device()):
         return None
     y = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
-    part = torch.empty(S, M, w.shape[0], dtype=torch.float32, device=x.device) if S > 1 else None
+    part = torch.empty(plan // 16, M, rows, dtype=torch.float32, device=x.device) if plan >= 32 else None
     native.check(native.kernels().hds_linear_bf16(px, ld, pw, native.ptr(b), y.data_ptr(), N, native.ptr(part), M, N, K, glu,
-                                                  native.stream()), "linear_bf16")
+                                                  plan, native.stream()), "linear_bf16")
     return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 
 
@@ -122,7 +125,9 @@ def _needs_grad(*tensors):
 def glu_linear(x, w, b, act):
     """act(x . gate^T) * (x . up^T) for ``w`` = [gate; up] (and ``b``) in one call, for 2..16 rows of the skinny GEMM and 9..256 of
     ``rows_linear``; None for anything else. The projections are rounded to bf16 first, as the separate kernels store them."""
-    if act not in _GATHER_ACTS or not (x.dim() >= 1 and x.is_cuda and torch.is_tensor(w)) or _needs_grad(x, w, b):
+    if act not in _GATHER_ACTS or not (x.dim() >= 1 and x.is_cuda and torch.is_tensor(w)):
+        return None
+    if x.numel() > 256 * x.shape[-1] or _needs_grad(x, w, b):
         return None
     if x.numel() > 8 * x.shape[-1]:
         y = rows_linear(x, w, b, 1 + _GATHER_ACTS[act])
@@ -143,20 +148,23 @@ def linear(x, w, b=None):
     """``F.linear(x, w, b)``; decode-sized bf16 inputs run the HIP GEMV (one row) or the skinny matrix-core GEMM
     (2..16 rows), 9 to 1,100 the tiled and
     sliced one where it is the faster, unless a gradient is wanted."""
-    if x.dim() >= 1 and x.is_cuda and x.numel() <= MAX_ROWS * x.shape[-1] and not _needs_grad(x, w, b):
-        if x.numel() > 8 * x.shape[-1]:
-            y = rows_linear(x, w, b)
+    if x.dim() >= 1 and x.is_cuda:
+        n, K = x.numel(), x.shape[-1]
+        if n > MAX_ROWS * K:
+            # (hds_linear_plan takes none beyond; what asking costs, 1 us, is 3 % of the host's time for a prompt of that length)
+            y = rows_linear(x, w, b) if n <= 320 * K or K >= 8192 else None
             if y is not None:
                 return y
-        x2 = x.reshape(-1, x.shape[-1])
-        if skinny_ok(x2, w, b):
-            return skinny(x2, w, b).view(*x.shape[:-1], w.shape[0])
-        if gemv_ok(x2, w, b):
-            return gemv(x2, w, b).view(*x.shape[:-1], w.shape[0])
-    else:
-        y = rows_linear(x, w, b)
-        if y is not None:
-            return y
+        elif not _needs_grad(x, w, b):
+            if n > 8 * K:
+                y = rows_linear(x, w, b)
+                if y is not None:
+                    return y
+            x2 = x.reshape(-1, K)
+            if skinny_ok(x2, w, b):
+                return skinny(x2, w, b).view(*x.shape[:-1], w.shape[0])
+            if gemv_ok(x2, w, b):
+                return gemv(x2, w, b).view(*x.shape[:-1], w.shape[0])
     return F.linear(x, w, b)
 
 

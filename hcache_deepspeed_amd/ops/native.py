@@ -120,10 +120,10 @@ _KERNEL_SIGS = {
     "hds_gemv_bf16": "pppp" + "iii" + "ll" + "s",
     "hds_gemv_fused_bf16": "ppp" + "f" + "pppp" + "if" + "iii" + "ll" + "s",
     "hds_gather_gemv_bf16": "ppp" + "l" + "p" + "ii" + "p" + "iii" + "ll" + "s",
-    "hds_packed_slices": "iiiiii",
-    "hds_packed_rows": "pppppp" + "iiiiiii" + "s",
-    "hds_linear_slices": "iiii",
-    "hds_linear_bf16": "plppplp" + "iiii" + "s",
+    "hds_packed_plan": "iiiiii",
+    "hds_packed_rows": "pppppp" + "iiiiiiii" + "s",
+    "hds_linear_plan": "iiii",
+    "hds_linear_bf16": "plppplp" + "iiiii" + "s",
     "hds_skinny_gemm_bf16": "pppp" + "iii" + "ll" + "i" + "s",
     "hds_wmix_splits": "iii",
     "hds_wmix_supported": "iiii",

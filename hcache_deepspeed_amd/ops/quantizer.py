@@ -192,17 +192,17 @@ _FMTS = {"int8": 0, "int4": 1, "fp6": 2}
 
 
 @functools.lru_cache(maxsize=4096)
-def _packed_slices(M, N, K, group_size, fmt, glu):
-    """Slices of K on csrc/kernels/linear_packed.hip, 0 for products that stay with the other kernels."""
-    return int(native.kernels().hds_packed_slices(M, N, K, group_size, _FMTS[fmt], glu)) if max(M, N, K) < 1 << 30 else 0
+def _packed_plan(M, N, K, group_size, fmt, glu):
+    """Tile + 16 x slices of K on csrc/kernels/linear_packed.hip, 0 for products that stay with the other kernels."""
+    return int(native.kernels().hds_packed_plan(M, N, K, group_size, _FMTS[fmt], glu)) if max(M, N, K) < 1 << 30 else 0
 
 
 def _packed_rows(x2, q_weight, scales, out_features, in_features, group_size, fmt, ebits, bias, glu):
     """The packed-weight product of more rows (csrc/kernels/linear_packed.hip): mostly 17 to 256; None where it does not apply or
     anything could want a record of it."""
     M, N, K = x2.shape[0], out_features, in_features
-    S = _packed_slices(M, N, K, group_size, fmt, 1 if glu else 0)
-    if S == 0 or not native.bare(x2, q_weight, bias) or (bias is not None and _needs_grad(bias)):
+    plan = _packed_plan(M, N, K, group_size, fmt, 1 if glu else 0)
+    if plan == 0 or not native.bare(x2, q_weight, bias) or (bias is not None and _needs_grad(bias)):
         return None
     x2 = x2.contiguous()
     if (x2.data_ptr() | q_weight.data_ptr()) % 16 or (bias is not None and bias.dtype != torch.bfloat16):
@@ -210,10 +210,10 @@ def _packed_rows(x2, q_weight, scales, out_features, in_features, group_size, fm
     if bias is not None:
         bias = bias.contiguous()
     y = torch.empty(M, N, dtype=torch.bfloat16, device=x2.device)
-    part = torch.empty(S, M, 2 * N if glu else N, dtype=torch.float32, device=x2.device) if S > 1 else None
+    part = torch.empty(plan // 16, M, 2 * N if glu else N, dtype=torch.float32, device=x2.device) if plan >= 32 else None
     native.check(native.kernels().hds_packed_rows(x2.data_ptr(), q_weight.data_ptr(), scales.data_ptr(), native.ptr(bias),
                                                   y.data_ptr(), native.ptr(part), M, N, K, group_size, _FMTS[fmt], int(ebits),
-                                                  int(glu), native.stream()), "packed_rows")
+                                                  int(glu), plan, native.stream()), "packed_rows")
     return y
 
 

@@ -18,7 +18,7 @@ def test_linear_rows_match_64_bits(M, N, K):
     x = torch.randn(M, K + 8, device="cuda", generator=g).to(torch.bfloat16)[:, :K]
     x[-1, -64:] = 100  # what the last row's last stage holds counts
     b = torch.randn(N, device="cuda", generator=g).to(torch.bfloat16) if M % 2 else None
-    assert gemv._slices(M, N, K)
+    assert gemv._plan(M, N, K)
     with torch.no_grad():
         y, again = gemv.linear(x, w, b), gemv.linear(x, w, b)
     ref = x.double() @ w.double().t() + (0 if b is None else b.double())
@@ -66,7 +66,7 @@ def test_linear_rows_gated(act, M, N, K):
 @pytest.mark.gpu
 def test_linear_rows_refuse():
     """What the kernel does not take goes where it went: rows, K, widths, types, alignment, gradients and transforms."""
-    assert not any(gemv._slices(*s) for s in [(8, 32768, 4096), (32, 4096, 4096), (16, 4096, 8192), (1101, 4096, 8192), (128, 4096, 4000), (128, 4095, 8192), (129, 32768, 4096),
+    assert not any(gemv._plan(*s) for s in [(8, 32768, 4096), (32, 4096, 4096), (16, 4096, 8192), (1101, 4096, 8192), (128, 4096, 4000), (128, 4095, 8192), (129, 32768, 4096),
                                               (321, 4096, 4096), (257, 4096, 8192, 1)])
     x = torch.zeros(128, 8200, dtype=torch.bfloat16, device="cuda")
     w = torch.zeros(4096, 8192, dtype=torch.bfloat16, device="cuda")

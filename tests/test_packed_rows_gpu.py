@@ -27,7 +27,7 @@ def test_rows_on_packed_weights(fmt, M, N, K, G):
     torch.manual_seed(K + M)
     x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
     q, s, wd = _packed(fmt, N, K, G)
-    assert N * K < 1 << 23 and M <= 32 and fmt[0] == "f" or Q._packed_slices(M, N, K, G, fmt[:4] if fmt[0] == "i" else "fp6", 0)
+    assert N * K < 1 << 23 and M <= 32 and fmt[0] == "f" or Q._packed_plan(M, N, K, G, fmt[:4] if fmt[0] == "i" else "fp6", 0)
     if fmt[0] == "i":
         bias = torch.randn(N, device="cuda").bfloat16()
         y = Q.int_linear(x, q, s, N, K, G, bits=int(fmt[3:]), bias=bias)
