@@ -767,6 +767,9 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(PagedDecodeParams<bf1
 // heads, 13.9 -> 8.5, and the rotation's own launch (4 us) saved. More or smaller splits are level or slower (1,024 and
 // 2,048 workgroups: 46.4 and 45.3 us there, but 8 sequences of 1,000 keys 12.3 -> 15.4 and 22.5). Keys and values, which a
 // step reads once, past the caches: 16 sequences of up to 4,000 keys 42.7 -> 40.8 us, 9 of up to 3,000 19.8 -> 18.3 (no merge).
+// A tile's place in the cache is known before its turn: looked up then, the block table's answer came behind keys and values
+// of all other waves (with the merge, 16 sequences of up to 4,000 keys 45.2 -> 41.6 us, of up to 2,000 29.2 -> 27.0; equal
+// lengths of 2,400 37.3 -> 36.4).
 struct DecodeRope {
   bf16* cache;
   const float* cos;  // [pos][rot / 2], null: k is appended as it is
@@ -789,7 +792,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(PagedDecodePa
   __shared__ __attribute__((aligned(1024))) char smem[4][2 * kTile];
   __shared__ float s_m[4][16], s_l[4][16];
   const int split = blockIdx.x, hk = blockIdx.y, b = blockIdx.z, G = p.hq / p.hkv;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, hd = lane & 15, g = lane >> 4;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), hd = lane & 15, g = lane >> 4;
   const DecodeToken tk = decode_token(p, b);
   const DecodeTiles tiles = decode_tiles(p, tk.pos, split);
   if (split >= tiles.used) return;
@@ -798,10 +801,17 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(PagedDecodePa
   char* kt = smem[w];
   char* vt = kt + kTile;
 
+  // cache rows of the wave's next 64 tiles, a lane each
+  int rows = 0, nth = 0;
+  auto look_up = [&](int T) {
+    const int pos = 32 * min(T + 4 * lane, tiles.b - 1), at = pos / p.block_size;
+    rows = table[at] * p.block_size + (pos - at * p.block_size);
+  };
   bf16x8 kr[8], vr[8];
   auto fetch = [&](int T) {
-    const int pos = 32 * T, blk = __builtin_amdgcn_readfirstlane(table[pos / p.block_size]);
-    const bf16* base = p.cache + ((int64_t)blk * p.block_size + pos % p.block_size) * kv_row + hk * D + 8 * hd;
+    if ((nth & 63) == 0) look_up(T);
+    const bf16* base = p.cache + (int64_t)__builtin_amdgcn_readlane(rows, nth & 63) * kv_row + hk * D + 8 * hd;
+    ++nth;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       kr[i] = load_nt(reinterpret_cast<const bf16x8*>(base + (4 * i + g) * kv_row));

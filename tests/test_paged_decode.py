@@ -143,3 +143,21 @@ def test_matrix_core_kernel_against_the_plain_one(sink, gate_width, window, rows
     a, b = out
     # both sum in 32 bits and round once
     assert ((a - b).abs() <= 2**-7 * b.abs() + 2e-4).all() and a.abs().sum() > 0
+
+
+@pytest.mark.parametrize("bs,mb", [(32, 520), (96, 174)])
+@pytest.mark.parametrize("window", [0, 8200])
+def test_splits_of_more_tiles_than_a_wave_looks_up_at_once(bs, mb, window):
+    """One split for the whole sequence: around 64 and 128 tiles a wave, whose places it looks up 64 at a time."""
+    from hcache_deepspeed_amd.ops import native
+    lens, nq, nkv, D = [8161, 8192, 8193, 8320, 16400, 16600], 4, 1, 128
+    cache, tables, meta, qkv = _setup(lens, nq, nkv, D, bs, mb, seed=4)
+    seq = torch.arange(len(lens), dtype=torch.int32, device="cuda")
+    kv_rope_scatter(qkv, cache, seq, meta[:, 2].contiguous(), tables, None, None, nq, nkv, do_rope=False)
+    o = torch.zeros(len(lens), nq * D, device="cuda", dtype=torch.bfloat16)
+    native.check(
+        native.kernels().hds_paged_decode(native.dt(qkv), 0, qkv.data_ptr(), qkv.stride(0), cache.data_ptr(), o.data_ptr(), o.stride(0),
+                                          None, None, meta.data_ptr(), None, None, None, tables.data_ptr(), mb, bs, len(lens), nq,
+                                          nkv, D, D, 1, 0.09, window, 0, 0, 0.0, None, None, 0, 1, None, native.stream()), "decode")
+    ref = _exact(qkv[:, :nq], cache, tables, lens, nq, nkv, 0.09, window)
+    assert ((o.view(-1, nq, D).double() - ref).abs() <= 2**-8 * ref.abs() + 2e-4).all()
