@@ -20,6 +20,8 @@ import math
 
 import torch
 
+from .. import native
+
 _CHUNK_BYTES = 256 << 20
 
 
@@ -38,18 +40,19 @@ def _scores(q, k, b1, b2, i0, i1, scale):
 
 
 def _hip_eligible(q, k, v, b1, b2):
-    from .. import native
-    if not native.use_native(q):
+    if not native.use_native(q) or not q.dtype == k.dtype == v.dtype == torch.bfloat16 or q.shape[-1] not in (32, 64, 128):
         return False
-    ok_b = all(b is None or (b.dtype in (torch.bfloat16, torch.float32) and b.is_contiguous()) for b in (b1, b2))
-    same_b = b1 is None or b2 is None or b1.dtype == b2.dtype
-    return (q.dtype == k.dtype == v.dtype == torch.bfloat16 and q.shape[-1] in (32, 64, 128) and ok_b and same_b
-            and all(x.is_contiguous() and x.data_ptr() % 16 == 0 for x in (q, k, v)))
+    for b in (b1, b2):
+        if b is not None and not (b.dtype in (torch.bfloat16, torch.float32) and b.is_contiguous()):
+            return False
+    if b1 is not None and b2 is not None and b1.dtype != b2.dtype:
+        return False
+    return q.is_contiguous() and k.is_contiguous() and v.is_contiguous() and \
+        (q.data_ptr() | k.data_ptr() | v.data_ptr()) % 16 == 0
 
 
 def _hip_forward(q, k, v, b1, b2, scale):
     """HIP forward (csrc/kernels/evoformer.hip): O [B, N, L, H, D] and the natural-log LSE [B, N, H, L]."""
-    from .. import native
     B, N, L, H, D = q.shape
     o = torch.empty_like(q)
     lse = torch.empty(B, N, H, L, dtype=torch.float32, device=q.device)
@@ -61,13 +64,13 @@ def _hip_forward(q, k, v, b1, b2, scale):
     return o, lse
 
 
-def _hip_backward(ctx, do, qh, kh, vh, oh, lse, bias1, bias2, scale):
+def _hip_backward(ctx, do):
     """HIP backward (csrc/kernels/evoformer.hip)."""
-    from .. import native
-    B, N, H, L, D = qh.shape
-    # back to [B, N, L, H, D], contiguous already unless saved-tensor hooks (save_on_cpu with pinned memory) laid them out anew
-    q, k, v, o = (x.transpose(-2, -3).contiguous() for x in (qh, kh, vh, oh))
-    do = do.contiguous()
+    q, k, v, o, lse, bias1, bias2 = ctx.saved_tensors
+    scale = ctx.scale
+    B, N, L, H, D = q.shape
+    # contiguous already unless saved-tensor hooks laid them out anew
+    q, k, v, o, do = (x.contiguous() for x in (q, k, v, o, do))
     if do.data_ptr() % 16:
         do = do.clone()
     delta = torch.empty(B, N, H, L, dtype=torch.float32, device=q.device)
@@ -95,16 +98,17 @@ class EvoformerFusedAttention(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, bias1=None, bias2=None):
+        # saved as they came: views of them to [B, N, H, L, D] and back were 10 of the 80 us that a training step of few rows
+        # costs the host, which bounds it
+        ctx.scale = scale = 1.0 / math.sqrt(q.shape[-1])
+        ctx.hip = _hip_eligible(q, k, v, bias1, bias2)
+        if ctx.hip:
+            o, lse = _hip_forward(q, k, v, bias1, bias2, scale)
+            ctx.save_for_backward(q, k, v, o, lse, bias1, bias2)
+            return o
         # [B, N, L, H, D] -> [B, N, H, L, D]
         qh, kh, vh = (x.transpose(-2, -3) for x in (q, k, v))
         B, N, H, L, D = qh.shape
-        scale = 1.0 / math.sqrt(D)
-        if _hip_eligible(q, k, v, bias1, bias2):
-            o, lse = _hip_forward(q, k, v, bias1, bias2, scale)
-            ctx.save_for_backward(qh, kh, vh, o.transpose(-2, -3), lse, bias1, bias2)
-            ctx.scale = scale
-            ctx.hip = True
-            return o
         o = torch.empty(qh.shape, dtype=q.dtype, device=q.device)
         lse = torch.empty(B, N, H, L, dtype=torch.float32, device=q.device)
         c = _chunk_rows(B, N, H, L)
@@ -116,16 +120,15 @@ class EvoformerFusedAttention(torch.autograd.Function):
             p = torch.exp(s - m[..., None])
             o[..., i0:i1, :] = torch.matmul(p.to(v.dtype), vh)
         ctx.save_for_backward(qh, kh, vh, o, lse, bias1, bias2)
-        ctx.scale = scale
         return o.transpose(-2, -3)
 
     @staticmethod
     def backward(ctx, do):
+        if ctx.hip:
+            return _hip_backward(ctx, do)
         qh, kh, vh, o, lse, bias1, bias2 = ctx.saved_tensors
         scale = ctx.scale
         B, N, H, L, D = qh.shape
-        if getattr(ctx, "hip", False):
-            return _hip_backward(ctx, do, qh, kh, vh, o, lse, bias1, bias2, scale)
         doh = do.transpose(-2, -3)
         delta = (doh.float() * o.float()).sum(-1)  # [B, N, H, L]
         dq = torch.empty(qh.shape, dtype=torch.float32, device=qh.device)
@@ -165,4 +168,6 @@ def DS4Sci_EvoformerAttention(Q, K, V, biases):
         assert biases[0].shape == (Q.shape[0], Q.shape[1], 1, 1, Q.shape[2]), "bias1 shape is incorrect"
     if biases[1] is not None:
         assert biases[1].shape == (Q.shape[0], 1, Q.shape[3], Q.shape[2], Q.shape[2]), "bias2 shape is incorrect"
+    if native.plain(Q, K, V, *biases) and _hip_eligible(Q, K, V, *biases):  # (what nobody records needs no node: 16 -> 14 us of few rows)
+        return _hip_forward(Q, K, V, *biases, 1.0 / math.sqrt(Q.shape[-1]))[0]
     return EvoformerFusedAttention.apply(Q, K, V, biases[0], biases[1])
