@@ -39,13 +39,15 @@ import torch.nn.functional as F
 from ... import comm as dist
 from ...ops import native
 from ...ops.activations import glu
+from ...ops.experts import ExpertSum
 from ...ops.norm import layer_norm, rms_norm
+from ...ops.output_norm import experts_pre_norm
 from ...ops.paged import build_atoms, kv_rope_scatter
 from ...ops.rope import rope_tables
 from .modules import (DSEmbeddingsConfig, DSLinearConfig, DSMoEConfig, DSNormConfig, DSSelfAttentionConfig,
                       DSUnembedConfig, instantiate_attention, instantiate_embed, instantiate_linear, instantiate_moe,
                       instantiate_pre_norm, instantiate_unembed)
-from .modules.implementations import _PackedWeight
+from .modules.implementations import DSPreRMSNorm, RaggedUnembed, _PackedWeight
 
 
 class _Layer:
@@ -284,6 +286,15 @@ class RaggedTransformer:
             return self._moe(L, x)
         return self.down_lin(self.up_lin(x, L["up.w"], L["up.b"]), L["down.w"], L["down.b"])
 
+    def _expert_parts(self, L, x):
+        """A routed layer's output before it is summed (ops/experts.py ``ExpertSum``) where the norm behind it, the next layer's
+        or the logits', can sum it; else None."""
+        behind = self.unembed_mod if L is self.layers[-1] else self.norm_mod
+        if (self.tp != 1 or L["w13"] is None or L.routed is None or not x.shape[0] or not hasattr(self.moe_mod, "parts")
+                or type(behind) not in (DSPreRMSNorm, RaggedUnembed)):
+            return None
+        return self.moe_mod.parts(x, L["w2"], L.routed)
+
     def _moe(self, L, x):
         out = self.moe_mod(x, L["router.w"], L["w13"], L["w2"], L.routed)
         if L.routed is not None:
@@ -451,6 +462,8 @@ class RaggedTransformer:
             if residual is None:
                 x = self._norm(h, L["ln1.w"], L["ln1.b"])
                 residual = h
+            elif isinstance(h, ExpertSum):
+                x, residual = experts_pre_norm(h, residual, L["ln1.w"], spec.norm_eps)
             else:
                 x, residual = self._norm(h, L["ln1.w"], L["ln1.b"], residual)
             if capture_latents and self.latent_mode == "hidden":
@@ -467,7 +480,9 @@ class RaggedTransformer:
                 h = self._allreduce(a + self._mlp(L, xm))
             else:
                 x2, residual = self._norm(self._allreduce(a), L["ln2.w"], L["ln2.b"], residual)
-                h = self._allreduce(self._mlp(L, x2))
+                h = self._expert_parts(L, x2)
+                if h is None:
+                    h = self._allreduce(self._mlp(L, x2))
         logits = self.unembed_mod(h, residual, batch, self.lm_head, self.lm_head_b, self.final_w, self.final_b,
                                   spec.norm_eps, self.tp_group, self.vocab)
         self.latent_event = events[-1] if events else None

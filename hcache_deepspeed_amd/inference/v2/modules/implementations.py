@@ -16,7 +16,7 @@ from .... import comm as dist
 from ....ops.activations import bias_act, glu, glu_rows
 from ....ops.delta_rule import DeltaShape, delta_rule, make_delta_plan, step_ok
 from ....ops.embedding import lookup_rows
-from ....ops.experts import PAD, RouterShape, routed_experts
+from ....ops.experts import PAD, ExpertSum, RouterShape, routed_experts
 from ....ops.gated_scan import gated_scan, recur_step, recur_step_ok
 from ....ops.gemv import glu_gemv, glu_linear, linear  # decode-sized steps on the HIP kernels
 from ....ops.grouped_gemm import moe_ffn_dropless
@@ -27,8 +27,8 @@ from ....ops.matrix_memory import MemoryShape, make_memory_plan, matrix_memory
 from ....ops.matrix_memory import step_ok as memory_step_ok
 from ....ops.moe import moe_combine, moe_dispatch, topk_assign, topk_route
 from ....ops.norm import layer_norm, norm_picked, norm_picked_ok, rms_norm
-from ....ops.output_norm import (PairSum, embed_rows, padded, residual_norm, rms_rows, sandwich_norm, softcap_,
-                                 stream_norm, sum_experts)
+from ....ops.output_norm import (PairSum, embed_rows, experts_pre_norm, padded, residual_norm, rms_rows, sandwich_norm,
+                                 softcap_, stream_norm, sum_experts)
 from ....ops.paged import (HeadShape, decode_qkv_ok, head_attention, head_blocks_ok, kv_rope_scatter, make_head_plan,
                            paged_attention, paged_decode_qkv)
 from ....ops.paged_prefill import paged_attention_portions, portions_ok
@@ -229,6 +229,14 @@ class GroupedGemmMoE(DSMoEBase):
         return {"router.w": router_w if gate is None else torch.cat([router_w, gate]), "router.c": None, "w13": w13,
                 "w2": w2, "ws13": ws13, "ws2": ws2}
 
+    def parts(self, x, w2, laid):
+        """The output of ``forward`` with ``laid`` before it is summed, for a norm that sums it on the way in."""
+        c = self._config
+        if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:  # the kernels read 16-byte pieces of rows
+            x = x.clone(memory_format=torch.contiguous_format)
+        return routed_experts(x, laid, RouterShape(w2.shape[0], top=c.top_k,
+                                                   normalize=bool(c.normalize_scores) and c.top_k > 1))
+
     def forward(self, x, router_w, w13, w2, laid=None):
         """``laid``: the weights from ``lay_out``, the shared expert among them; its part is then in the result."""
         c = self._config
@@ -238,10 +246,7 @@ class GroupedGemmMoE(DSMoEBase):
         if laid is None and x.dtype == torch.bfloat16 and not grad:
             laid = self.lay_out(router_w, w13, w2)
         if laid is not None and T:
-            if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:  # the kernels read 16-byte pieces of rows
-                x = x.clone(memory_format=torch.contiguous_format)
-            shape = RouterShape(w2.shape[0], top=c.top_k, normalize=bool(c.normalize_scores) and c.top_k > 1)
-            return sum_experts(x, routed_experts(x, laid, shape), x.dtype)
+            return sum_experts(x, self.parts(x, w2, laid), x.dtype)
         logits = F.linear(x.float(), router_w.float())
         if x.is_cuda and x.dtype == torch.bfloat16 and H % 128 == 0 and w2.shape[2] % 128 == 0:
             expert, pos, w, counts = topk_assign(logits, c.top_k, normalize=c.normalize_scores)
@@ -341,6 +346,11 @@ class RaggedUnembed(DSUnembedBase):
                 vocab=None):
         idx = batch.last_token_idx
         is_ln = self._config.norm_type != "rms"
+        if isinstance(hidden, ExpertSum):
+            if final_w is not None and not is_ln and self._every_row(batch, residual):
+                hl, _ = experts_pre_norm(hidden, residual, final_w, norm_eps)
+                return self.project(hl, lm_head, lm_head_b, tp_group, vocab)
+            hidden = sum_experts(residual, hidden, residual.dtype)
         if self._every_row(batch, hidden):  # nothing to gather
             if final_w is None:
                 hl = hidden + residual

@@ -41,6 +41,7 @@ _KERNEL_SIGS = {
     "hds_head_prep": "i" + "pl" + "i" * 7 + "ppppp" + "pl" + "pp" + "ii" + "ppp" + "pl" + "ppp" + "ii" + "f" + "iii" + "s",
     "hds_row_norm": "i" + "pl" + "ppl" + "ii" + "f" + "s",
     "hds_softcap": "i" + "p" + "l" + "f" + "s",
+    "hds_experts_pre_norm": "pppp" + "pl" + "ppp" + "pl" + "pl" + "iiii" + "f" + "s",
     "hds_experts_norm": "i" + "ppp" + "l" + "pp" + "pl" + "ppp" + "pl" + "pl" + "iiiii" + "f" + "s",
     "hds_embed_rows": "i" + "pp" + "f" + "pp" + "l" + "iii" + "s",
     "hds_router_logits": "pl" + "p" + "pl" + "iii" + "s",

@@ -13,6 +13,7 @@ from dataclasses import dataclass
 import torch
 
 from . import native
+from .norm import rms_norm
 
 
 def padded(n, pad):
@@ -82,6 +83,25 @@ def sum_experts(x, parts, dtype):
         _experts_norm(x, None, 0, None, out, parts, 0.0)
         return out
     return out.copy_(parts.total(x))
+
+
+def experts_pre_norm(parts, residual, gain, eps):
+    """The next layer's RMS pre-norm of an ExpertSum without identity choices: (norm(r), r = residual + sum), as ``rms_norm`` of
+    its rows gives them; on the GPU in one kernel for bf16 rows of a multiple of 8 up to 8,192."""
+    T, W = residual.shape
+    sh, ts = parts.shared, (residual, gain, parts.y) + (() if parts.shared is None else (parts.shared, ))
+    if not (native.use_native(residual) and W % 8 == 0 and W <= 8192 and residual.is_contiguous() and gain.is_contiguous()
+            and all(t.dtype == torch.bfloat16 and t.data_ptr() % 16 == 0 and t.stride(0) % (8 if t.dim() > 1 else 1) == 0 for t in ts)):
+        return rms_norm(sum_experts(residual, parts, residual.dtype), gain, eps, residual)
+    y, r = torch.empty_like(residual), torch.empty_like(residual)
+    native.check(
+        native.kernels().hds_experts_pre_norm(
+            residual.data_ptr(), r.data_ptr(), gain.data_ptr(), y.data_ptr(), parts.y.data_ptr(), parts.y.stride(0),
+            parts.expert.data_ptr(), native.ptr(parts.weight), native.ptr(parts.row), native.ptr(sh),
+            0 if sh is None else sh.stride(0), None if sh is None else parts.gate.data_ptr(),
+            0 if sh is None else parts.gate.stride(0), parts.n_experts, parts.expert.shape[1], T, W, float(eps),
+            native.stream()), "experts_pre_norm")
+    return y, r
 
 
 def _experts_norm(x, xb, ld, gain, out, p, eps):
