@@ -502,7 +502,25 @@ struct PagedDecodeParams {
   // the others: keys that a workgroup takes at a time. One number for all (64) left heads of 256 with too few splits at work:
   // 16 / 1 heads, 16 tokens, up to 300 keys 36.5 us, with the kernel's own turn of 16 25.8; 64 tokens 40.4 and 34.4
   int turn;
+  int rounds = 1;  // see decode_grid
 };
+
+// Workgroups of `splits` splits by `y` by n tokens. Launches are sized by what a block table can hold, so that most of 64 or 32
+// splits of a short sequence have no keys; in rounds of 8 splits those come behind all that have some, instead of between them
+// (with the merge, 1,000 keys: 4 sequences of 4 key heads 12.2 -> 10.5 us, 4 of 8 12.1 -> 10.4, one of 8 11.8 -> 10.5; 8,000
+// keys level). A round that is not full would set workgroups of the same splits side by side on a CU (10 splits of 7
+// sequences, 4,000 keys 23 -> 32 us): only multiples of 8.
+inline dim3 decode_grid(int splits, int y, int n, int& rounds) {
+  rounds = splits > 8 && splits % 8 == 0 && (int64_t)n * (splits / 8) <= 65535 ? splits / 8 : 1;
+  return rounds > 1 ? dim3(8, y, n * rounds) : dim3(splits, y, n);
+}
+
+template <typename P>
+__device__ __forceinline__ void decode_place(const P& p, int& split, int& b) {
+  const int n = gridDim.z / p.rounds, round = p.rounds > 1 ? blockIdx.z / n : 0;
+  split = blockIdx.x + 8 * round;
+  b = blockIdx.z - round * n;
+}
 
 struct DecodeToken {
   int row, seq, pos;
@@ -595,7 +613,9 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(PagedDecodeParams<bf1
   constexpr int U = kDecUnroll<GM>;
   __shared__ float red[4][GM][2 + 8 * LPK];
   const int G = p.hq / p.hkv, gb = (G + GM - 1) / GM;
-  const int split = blockIdx.x, hk = blockIdx.y / gb, g0 = (blockIdx.y % gb) * GM, b = blockIdx.z;
+  const int hk = blockIdx.y / gb, g0 = (blockIdx.y % gb) * GM;
+  int split, b;
+  decode_place(p, split, b);
   const int gn = min(GM, G - g0), h0 = hk * G + g0;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int kl = lane / LPK, c = lane % LPK;
@@ -791,7 +811,9 @@ __global__ __launch_bounds__(256, 2) void paged_decode_mfma_kernel(PagedDecodePa
   constexpr int D = 128, kTile = 32 * 256;
   __shared__ __attribute__((aligned(1024))) char smem[4][2 * kTile];
   __shared__ float s_m[4][16], s_l[4][16];
-  const int split = blockIdx.x, hk = blockIdx.y, b = blockIdx.z, G = p.hq / p.hkv;
+  const int hk = blockIdx.y, G = p.hq / p.hkv;
+  int split, b;
+  decode_place(p, split, b);
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), hd = lane & 15, g = lane >> 4;
   const DecodeToken tk = decode_token(p, b);
   const DecodeTiles tiles = decode_tiles(p, tk.pos, split);
@@ -1112,7 +1134,8 @@ int launch_decode(PagedDecodeParams<bf16> p, int n, hipStream_t st) {
 #define HDS_DEC(GM)                                                                                                 \
   do {                                                                                                              \
     p.turn = 4 * (64 / LPK) * kDecUnroll<GM>;                                                                       \
-    hipLaunchKernelGGL((paged_decode_kernel<LPK, GM>), dim3(p.splits, p.hkv * ((G + GM - 1) / GM), n), dim3(256), 0, st, p); \
+    const dim3 grid = decode_grid(p.splits, p.hkv * ((G + GM - 1) / GM), n, p.rounds);                              \
+    hipLaunchKernelGGL((paged_decode_kernel<LPK, GM>), grid, dim3(256), 0, st, p);                                  \
   } while (0)
   if (G == 1) HDS_DEC(1); else if (G == 2) HDS_DEC(2); else if (G <= 4) HDS_DEC(4); else HDS_DEC(8);
 #undef HDS_DEC
@@ -1140,7 +1163,8 @@ bool decode_mfma_ok(const PagedDecodeParams<bf16>& p) {
 template <bool ROPE>
 int launch_decode_mfma(PagedDecodeParams<bf16> p, const DecodeRope& rope, int n, hipStream_t st) {
   p.tiles = 1;
-  hipLaunchKernelGGL((paged_decode_mfma_kernel<ROPE>), dim3(p.splits, p.hkv, n), dim3(256), 0, st, p, rope);
+  const dim3 grid = decode_grid(p.splits, p.hkv, n, p.rounds);
+  hipLaunchKernelGGL((paged_decode_mfma_kernel<ROPE>), grid, dim3(256), 0, st, p, rope);
   if (p.splits > 1) launch_combine(p, n, st);
   return hipGetLastError();
 }
@@ -1264,7 +1288,8 @@ HDS_EXPORT int hds_paged_decode_splits(int n_seqs, int hkv, int max_ctx) {
   int splits = (512 + groups - 1) / groups;
   const int by_len = (max_ctx + 31) / 32;
   splits = splits < by_len ? splits : by_len;
-  return splits < 1 ? 1 : (splits > 64 ? 64 : splits);
+  splits = splits < 1 ? 1 : (splits > 64 ? 64 : splits);
+  return splits > 8 && splits % 8 * 10 <= splits ? splits / 8 * 8 : splits;  // whole rounds (decode_grid) where they are near
 }
 
 // Single tokens. seq_meta: one sequence with one new token each (n of them); null: the n tokens toks (null: 0 .. n - 1)

@@ -161,3 +161,23 @@ def test_splits_of_more_tiles_than_a_wave_looks_up_at_once(bs, mb, window):
                                           nkv, D, D, 1, 0.09, window, 0, 0, 0.0, None, None, 0, 1, None, native.stream()), "decode")
     ref = _exact(qkv[:, :nq], cache, tables, lens, nq, nkv, 0.09, window)
     assert ((o.view(-1, nq, D).double() - ref).abs() <= 2**-8 * ref.abs() + 2e-4).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("splits", [8, 16, 24, 63, 64])
+def test_rounds_of_splits(D, splits):
+    """Splits in whole rounds of 8 and others, most of them without keys, on both kernels against 64 bits."""
+    from hcache_deepspeed_amd.ops import native
+    lens, nq, nkv, bs, mb = [1, 130, 3000, 257, 2049], 12, 3, 64, 48
+    cache, tables, meta, qkv = _setup(lens, nq, nkv, D, bs, mb, seed=5)
+    seq = torch.arange(len(lens), dtype=torch.int32, device="cuda")
+    kv_rope_scatter(qkv, cache, seq, meta[:, 2].contiguous(), tables, None, None, nq, nkv, do_rope=False)
+    o = torch.zeros(len(lens), nq * D, device="cuda", dtype=torch.bfloat16)
+    po, pm = (torch.empty(len(lens) * nq * splits * w, device="cuda") for w in (D, 2))
+    native.check(
+        native.kernels().hds_paged_decode(native.dt(qkv), 0, qkv.data_ptr(), qkv.stride(0), cache.data_ptr(), o.data_ptr(), o.stride(0),
+                                          po.data_ptr(), pm.data_ptr(), meta.data_ptr(), None, None, None, tables.data_ptr(), mb, bs,
+                                          len(lens), nq, nkv, D, D, splits, 0.09, 0, 0, 0, 0.0, None, None, 0, 1, None, native.stream()),
+        "decode")
+    ref = _exact(qkv[:, :nq], cache, tables, lens, nq, nkv, 0.09, 0)
+    assert ((o.view(-1, nq, D).double() - ref).abs() <= 2**-8 * ref.abs() + 2e-4).all()
