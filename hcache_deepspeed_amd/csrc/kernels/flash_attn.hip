@@ -24,7 +24,6 @@
 //   dq    : workgroup = 128 query rows of one (batch, q-head); sweeps key tiles; dQ in
 //           accumulators. Deterministic (no float atomics anywhere).
 // P is recomputed from the forward LSE; delta = rowsum(dO * O) comes from a tiny pre-kernel.
-#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -36,7 +35,6 @@ using namespace hds::attn;
 
 // variant 9 lives in its own translation unit (flash_attn_w64.hip: built with the VGPR-form MFMA selection)
 int hds_attn_fwd_w64_paged_launch(const void* params, size_t params_bytes, int n, int hq, hipStream_t st);
-int hds_attn_fwd_pair_launch(const void* params, size_t params_bytes, int batch, int max_len, int hq, hipStream_t st);
 int hds_attn_fwd_pair_paged_launch(const void* params, size_t params_bytes, int n, int hq, hipStream_t st);
 int hds_attn_fwd_w64_launch(const void* params, size_t params_bytes, int batch, int max_len, int hq, int mode,
                             hipStream_t st);
@@ -1492,24 +1490,6 @@ HDS_EXPORT int hds_attn_config(int fwd_nw, int dkdv_nw, int dq_nw) {
 
 namespace {
 
-// Time of a forward by workgroups of `rows` queries that step over `keys` keys: the longest of them, or all over the CUs and a
-// quarter of the longest for their uneven end. Fixed and step us of the 128-row kernel (flash_attn_pair.hip) 8 and 1.85 a
-// step of 128 keys, of the 256-row one (flash_attn_w64.hip) 10.2 and 1.9 a step of 64: steps cost a row and key alike, what
-// a workgroup costs once falls on half as many rows. 256 rows -> 128, us: 32 / 8 heads 1 x 512 23.5 -> 14.3, 1 x 1,024 38 ->
-// 22, 1 x 2,048 68 -> 46, 1 x 4,096 149 / 145, 1 x 8,192 520 / 526, 7 x 4,096 1,035 / 1,102, 16 x 1,024 233 / 266; 16 / 4 heads 2 x 509
-// 25.4 -> 16.0, 1 x 2,048 63 -> 33, 6 x 1,500 96 / 90; 64 x 128 of 16 / 16 heads, not causal, 54 -> 39, 8 x 1,024 80 / 89.
-float forward_us(const AttnParams& p, int len, int64_t heads, int rows, int keys, float fixed, float step) {
-  float longest = 0.f, all = 0.f;
-  for (int64_t q0 = 0; q0 < len; q0 += rows) {
-    const int64_t end = p.causal ? std::min<int64_t>(q0 + rows, len) : len;
-    const int64_t begin = p.window > 0 ? std::max<int64_t>(0, q0 - p.window + 1) / 64 * 64 : 0;
-    const float us = fixed + step * (float)((end - begin + keys - 1) / keys);
-    longest = std::max(longest, us);
-    all += us;
-  }
-  return std::max(longest, heads * all / 256 + longest / 4);
-}
-
 template <int D>
 int launch_fwd(const AttnParams& p, int batch, int max_len, int hq, hipStream_t st) {
   if constexpr (D <= 128) {
@@ -1518,12 +1498,7 @@ int launch_fwd(const AttnParams& p, int batch, int max_len, int hq, hipStream_t 
       if constexpr (D == 128) {  // the A/B variants exist for the training head dim only
         switch (g_fwd_var) {
           case 5: hipLaunchKernelGGL((attn_fwd_sp_kernel<D>), grid, dim3(512), 0, st, p); break;
-          case 20:
-            if (p.scale >= 0x1p-64f && p.scale <= 0x1p64f &&
-                forward_us(p, max_len, (int64_t)hq * batch, 128, 128, 8.f, 1.85f) <
-                    forward_us(p, max_len, (int64_t)hq * batch, 256, 64, 10.2f, 1.9f))
-              return hds_attn_fwd_pair_launch(&p, sizeof(p), batch, max_len, hq, st);
-            return hds_attn_fwd_w64_launch(&p, sizeof(p), batch, max_len, hq, 11, st);
+          case 20: return hds_attn_fwd_w64_launch(&p, sizeof(p), batch, max_len, hq, 11, st);
 #if HDS_FA_DIAG
           case 4: hipLaunchKernelGGL((attn_fwd_stg_kernel<D>), grid, dim3(512), 0, st, p); break;
           case 6: hipLaunchKernelGGL((attn_fwd_sp_kernel<D, false>), grid, dim3(512), 0, st, p); break;
@@ -1726,9 +1701,9 @@ HDS_EXPORT int hds_paged_prefill(const void* q, int64_t sq, const void* cache, v
   p.tables = block_tables;
   p.max_blocks = max_blocks;
   p.block_size = block_size;
-  // 128 rows a workgroup where those of 256 are at most two a CU (see forward_us; here the lengths lie on the device). New
-  // tokens, 256 rows -> 128, us: 512 behind 789, 32 / 8 heads 37 -> 21; 701, 527 and 279 of three prompts, 16 / 4 32 -> 18; 2,048,
-  // 32 / 8 79 -> 57; 16,000, 16 / 4, 1,008 workgroups of 256 rows level.
+  // 128 rows a workgroup (flash_attn_pair.hip) where those of 256 are at most two a CU. New tokens, 256 rows
+  // -> 128, us: 512 behind 789, 32 / 8 heads 37 -> 21; 701, 527 and 279 of three prompts, 16 / 4 32 -> 18; 2,048, 32 / 8 79 -> 57;
+  // 16,000, 16 / 4, 1,008 workgroups of 256 rows, level.
   if ((int64_t)n_blocks * hq <= 512) return hds_attn_fwd_pair_paged_launch(&p, sizeof(p), n_blocks, hq, st);
   return hds_attn_fwd_w64_paged_launch(&p, sizeof(p), n_blocks, hq, st);
 }

@@ -1,4 +1,4 @@
-// FlashAttention forward, head size 128, by workgroups of 128 query rows: for passes whose 256-row workgroups
+// FlashAttention forward over a paged cache, head size 128, by workgroups of 128 query rows: for steps whose 256-row workgroups
 // (flash_attn_w64.hip) leave CUs idle or are of few lengths, as prompts of up to some thousand tokens.
 //
 // What bounds the 256-row kernel there is its chain: each of its waves has a SIMD to itself and walks all keys, 1.9 us a tile
@@ -23,34 +23,20 @@ __device__ __forceinline__ float xor32_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// PAGED: queries are the new tokens of a sequence behind earlier ones, keys and values lie in the paged cache (as in
-// attn_fwd_w64_kernel; an entry of the list is 256 new tokens, which two workgroups share here).
-template <bool PAGED>
+// Queries are the new tokens of a sequence behind earlier ones, keys and values lie in the paged cache, causal (as in
+// attn_fwd_w64_kernel; an entry of the list is 256 new tokens, which two workgroups share here). A kernel of contiguous rows
+// made a forward of 2 x 509 tokens 25 -> 16 us, but the training step it is part of 1 % faster only.
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_pair_kernel(AttnParams p) {
   constexpr int D = 128, BM = 128, KS = 8, DT = 4, TL = 16384, PW = 4;
   __shared__ __attribute__((aligned(1024))) char smem[8 * TL];  // a group: K[2], V[2]
-  int hq, start, len, q0;
-  const int* table = nullptr;
-  if constexpr (PAGED) {
-    // the second 128 rows of an entry, which see more keys, before its first; the heads of a key head on one XCD
-    const int at = blockIdx.x / (2 * p.hq), r = blockIdx.x % (2 * p.hq), half = r < p.hq, rr = half ? r : r - p.hq;
-    hq = p.hq % 8 == 0 ? (rr % 8) * (p.hq / 8) + rr / 8 : rr;
-    const int seq = p.blocks[2 * at], row0 = p.blocks[2 * at + 1] + (half ? BM : 0);
-    const int n_new = p.meta[3 * seq + 1], seen = p.meta[3 * seq + 2];
-    start = p.meta[3 * seq] - seen;
-    len = seen + n_new;
-    q0 = seen + row0;
-    table = p.tables + (int64_t)seq * p.max_blocks;
-    if (row0 >= n_new) return;
-  } else {
-    int blk, b;
-    lpt_ids(blk, hq, b);
-    seq_bounds(p, b, start, len);
-    const int nqb = (len + BM - 1) / BM;
-    const int qb = p.causal ? (gridDim.x - 1 - blk) : blk;
-    if (qb >= nqb || len == 0) return;
-    q0 = qb * BM;
-  }
+  // the second 128 rows of an entry, which see more keys, before its first; the heads of a key head on one XCD
+  const int at = blockIdx.x / (2 * p.hq), r = blockIdx.x % (2 * p.hq), half = r < p.hq, rr = half ? r : r - p.hq;
+  const int hq = p.hq % 8 == 0 ? (rr % 8) * (p.hq / 8) + rr / 8 : rr;
+  const int seq = p.blocks[2 * at], row0 = p.blocks[2 * at + 1] + (half ? BM : 0);
+  const int n_new = p.meta[3 * seq + 1], seen = p.meta[3 * seq + 2];
+  const int start = p.meta[3 * seq] - seen, len = seen + n_new, q0 = seen + row0;
+  const int* table = p.tables + (int64_t)seq * p.max_blocks;
+  if (row0 >= n_new) return;
   const int hk = hq / (p.hq / p.hkv);
   const int lane = threadIdx.x & 63, h = lane >> 5;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = wv & 3, grp = wv >> 2;
@@ -64,30 +50,26 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(qp + 16 * ks);
   }
-  const int kt_end = ((p.causal ? min(q0 + BM, len) : len) + BN - 1) / BN;
+  const int kt_end = (min(q0 + BM, len) + BN - 1) / BN;
   const int kt_begin = p.window > 0 ? max(0, q0 - p.window + 1) / BN : 0;
   // tiles past kt_end_w follow all rows of the wave
-  const int kt_end_w = wq_lo >= len ? kt_begin : p.causal ? min(kt_end, wq_hi / BN + 1) : kt_end;
+  const int kt_end_w = wq_lo >= len ? kt_begin : min(kt_end, wq_hi / BN + 1);
   const int turns = (kt_end - kt_begin + 1) / 2;  // of the group with the first tile
 
   // a wave's four pieces of a tile: rows 4 (4 w + j) + lane / 16, whose 16-byte pieces lie at c ^ swz(row)
   const int drow = lane >> 4, dcol = 16 * ((lane & 15) ^ (drow << 2));
-  // paged: lane i holds the cache slot of tile win + i
+  // lane i holds the cache slot of tile win + i
   int win = kt_begin, slots = 0;
   auto load_slots = [&](int first) __attribute__((always_inline)) {
     win = first;
     const int per = p.block_size / BN, t = min(first + lane, kt_end - 1), b = t / per;
     slots = table[b] * p.block_size + (t - b * per) * BN;
   };
-  if constexpr (PAGED) load_slots(kt_begin);
+  load_slots(kt_begin);
   auto source = [&](const bf16* base, int64_t stride, int kt) {
-    if constexpr (PAGED) {
-      const int rows = min(BN, len - kt * BN), slot = __builtin_amdgcn_readlane(slots, kt - win);
-      return TileSrc{(const char*)(base + (int64_t)slot * stride + (int64_t)hk * D),
-                     (int)(((int64_t)(rows - 1) * stride + D) * 2)};
-    } else {
-      return tile_src<D>(base, stride, start, kt, hk, len);
-    }
+    const int rows = min(BN, len - kt * BN), slot = __builtin_amdgcn_readlane(slots, kt - win);
+    return TileSrc{(const char*)(base + (int64_t)slot * stride + (int64_t)hk * D),
+                   (int)(((int64_t)(rows - 1) * stride + D) * 2)};
   };
   // tile of turn i of this group; past the end the last tile, which nobody reads
   auto tile_of = [&](int i) { return min(kt_begin + 2 * i + grp, kt_end - 1); };
@@ -148,7 +130,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // 2^29 in the exponent (see attn_fwd_w64_kernel): whatever a key that a row does not see holds, it does not count.
   auto softmax = [&](int kt) __attribute__((always_inline)) {
     const int k0 = kt * BN;
-    if (k0 + BN > len || (p.causal && k0 + BN - 1 > wq_lo) || (p.window > 0 && k0 <= wq_hi - p.window) || wq_hi >= len) {
+    if (k0 + BN > len || k0 + BN - 1 > wq_lo || (p.window > 0 && k0 <= wq_hi - p.window) || wq_hi >= len) {
       const int masked = 0x80000000 | ((127 + 28 + 127 - (__float_as_int(c) >> 23)) << 23);
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
@@ -213,9 +195,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (mine > 0) products(no, yes, 0, 0);
   meet();
   auto stage_next = [&](int i) __attribute__((always_inline)) {
-    if constexpr (PAGED) {
-      if (tile_of(i + 2) >= win + 64) load_slots(tile_of(i + 1));
-    }
+    if (tile_of(i + 2) >= win + 64) load_slots(tile_of(i + 1));
     if (i + 2 < turns) stage(false, i + 2);
     if (i + 1 < turns) stage(true, i + 1);
   };
@@ -227,9 +207,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   };
   auto turn = [&](int i, auto S, auto STEADY) __attribute__((always_inline)) {  // STEADY: with all of a turn's loads
     if constexpr (STEADY) {
-      if constexpr (PAGED) {
-        if (tile_of(i + 2) >= win + 64) load_slots(tile_of(i + 1));
-      }
+      if (tile_of(i + 2) >= win + 64) load_slots(tile_of(i + 1));
       stage(false, i + 2);
       stage(true, i + 1);
       softmax(tile_of(i));
@@ -286,20 +264,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   bf16* op = p.o + (int64_t)(start + myq) * p.so + (int64_t)hq * D;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) store_row_block<D>(op, o[dt], dt, h, inv);
-  if (h == 0 && p.lse) p.lse[(int64_t)hq * p.total_tokens + start + myq] = l > 0.f ? (top + __log2f(l)) / kLog2e : -INFINITY;
 }
 
 }  // namespace
 
-int hds_attn_fwd_pair_launch(const void* params, size_t params_bytes, int batch, int max_len, int hq, hipStream_t st) {
-  if (params_bytes != sizeof(AttnParams)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(attn_fwd_pair_kernel<false>, dim3((max_len + 127) / 128, hq, batch), dim3(512), 0, st,
-                     *static_cast<const AttnParams*>(params));
-  return hipGetLastError();
-}
 // n: entries of 256 new tokens
 int hds_attn_fwd_pair_paged_launch(const void* params, size_t params_bytes, int n, int hq, hipStream_t st) {
   if (params_bytes != sizeof(AttnParams)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(attn_fwd_pair_kernel<true>, dim3(2 * n * hq), dim3(512), 0, st, *static_cast<const AttnParams*>(params));
+  hipLaunchKernelGGL(attn_fwd_pair_kernel, dim3(2 * n * hq), dim3(512), 0, st, *static_cast<const AttnParams*>(params));
   return hipGetLastError();
 }

@@ -1,10 +1,9 @@
-"""FlashAttention forward by 128 rows a workgroup (csrc/kernels/flash_attn_pair.hip) and where the 256-row kernel takes over."""
+"""Prefill attention by 128 rows a workgroup (csrc/kernels/flash_attn_pair.hip) and where the 256-row kernel takes over."""
 import math
 
 import pytest
 import torch
 
-from hcache_deepspeed_amd.ops.attention import flash_attn
 from hcache_deepspeed_amd.ops.paged_prefill import make_portions, paged_attention_portions
 from .test_paged_prefill import _setup
 
@@ -30,45 +29,29 @@ def _close(got, want):
     assert ((got.double() - want).norm(dim=-1) / want.norm(dim=-1)).max() < 0.03  # no single row off either
 
 
-@pytest.mark.parametrize("causal,window", [(True, 0), (False, 0), (True, 1), (True, 70), (True, 200)])
-@pytest.mark.parametrize("lens,hq,hkv", [([1], 2, 2), ([31, 33, 64], 4, 2), ([63, 65, 1, 96], 4, 1), ([127, 128, 129], 8, 2),
-                                         ([191, 193, 255, 257], 2, 1), ([640, 1100], 16, 4), ([2050], 8, 8)])
-def test_forward_of_few_rows(lens, hq, hkv, causal, window):
+@pytest.mark.parametrize("window", [0, 1, 70, 200])
+@pytest.mark.parametrize("lens,seen,hq,hkv", [([1], [0], 2, 2), ([31, 33, 64], [0, 1, 63], 4, 2), ([63, 65, 1, 96], [65, 0, 300, 33], 4, 1),
+                                              ([127, 128, 129], [0, 64, 127], 8, 2), ([191, 193, 255, 257], [1, 0, 130, 5000], 2, 1),
+                                              ([640, 1100], [0, 333], 16, 4), ([2050], [0], 8, 8)])
+def test_portions_of_few_rows(lens, seen, hq, hkv, window):
     """Edges of the 32 rows of a wave, of the 128 of a workgroup and of the tiles of 64 keys, one group without a tile, waves
-    that end before others, windows that hide whole tiles of either group."""
+    that end before others, windows that hide whole tiles of either group, more than 64 tiles."""
     g = torch.Generator(device="cuda").manual_seed(sum(lens) + window)
-    rnd = lambda h: torch.randn(sum(lens), h, D, device="cuda", generator=g).bfloat16()  # noqa: E731
-    q, k, v = rnd(hq), rnd(hkv), rnd(hkv)
-    cu = torch.tensor([0] + lens).cumsum(0).int()
-    with torch.no_grad():
-        o, lse = flash_attn(q, k, v, causal=causal, cu_seqlens=cu.cuda(), window=window, return_lse=True)
-    for a, b in zip(cu[:-1].tolist(), cu[1:].tolist()):
-        want, sums = _attend(q[a:b], k[a:b], v[a:b], 0, causal, window)
-        _close(o[a:b], want)
-        # a score of 128 products of bf16 values in 32 bits, and exp2 and log2 of a few units of the last place
-        assert (lse.view(hq, -1)[:, a:b] - sums).abs().max() < 1e-4
-
-
-def test_padded_batch_of_few_rows():
-    g = torch.Generator(device="cuda").manual_seed(3)
-    rnd = lambda h: torch.randn(3, 200, h, D, device="cuda", generator=g).bfloat16()  # noqa: E731
-    q, k, v, lens = rnd(4), rnd(2), rnd(2), [200, 37, 129]
-    k[1, 37:], v[1, 37:] = 300.0, 300.0
-    with torch.no_grad():
-        o = flash_attn(q, k, v, causal=False, seq_lens=torch.tensor(lens, dtype=torch.int32, device="cuda"))
-    for i, n in enumerate(lens):
-        _close(o[i, :n], _attend(q[i, :n], k[i, :n], v[i, :n], 0, False, 0)[0])
+    cache, tab, metas, T, batch = _setup(lens, seen, hkv, 64, "cuda", torch.Generator().manual_seed(6))
+    q = torch.randn(T, hq, D, device="cuda", generator=g).bfloat16()
+    blocks = [(i, r) for i, n in enumerate(lens) for r in range(0, n, 256)]
+    assert len(blocks) * hq <= 512
+    o = paged_attention_portions(q, cache, None, torch.tensor(blocks, dtype=torch.int32, device="cuda"), batch, hq, hkv, D**-0.5,
+                                 window)
+    for i, (q0, n, s) in enumerate(metas):
+        at = torch.arange(s + n)
+        kv = cache[tab[i, at // 64].long().cuda(), (at % 64).cuda()]
+        _close(o[q0:q0 + n], _attend(q[q0:q0 + n], kv[:, 0], kv[:, 1], s, True, window)[0])
 
 
 def test_many_blocks_take_the_larger_workgroups():
-    """More 256-row workgroups than two a CU: sequences, and portions behind earlier tokens."""
+    """More 256-row workgroups than two a CU."""
     g = torch.Generator(device="cuda").manual_seed(4)
-    rnd = lambda h: torch.randn(16, 1000, h, D, device="cuda", generator=g).bfloat16()  # noqa: E731
-    q, k, v = rnd(16), rnd(4), rnd(4)
-    with torch.no_grad():
-        o = flash_attn(q, k, v, causal=True)
-    for i in (0, 7, 15):
-        _close(o[i], _attend(q[i], k[i], v[i], 0, True, 0)[0])
     lens, seen, hq, hkv = [257, 300, 10] * 5, [0, 130, 900] * 5, 32, 8
     cache, tab, metas, T, batch = _setup(lens, seen, hkv, 64, "cuda", torch.Generator().manual_seed(5))
     q = torch.randn(T, hq, D, device="cuda", generator=g).bfloat16()
