@@ -47,7 +47,7 @@ from ...ops.rope import rope_tables
 from .modules import (DSEmbeddingsConfig, DSLinearConfig, DSMoEConfig, DSNormConfig, DSSelfAttentionConfig,
                       DSUnembedConfig, instantiate_attention, instantiate_embed, instantiate_linear, instantiate_moe,
                       instantiate_pre_norm, instantiate_unembed)
-from .modules.implementations import DSPreRMSNorm, RaggedUnembed, _PackedWeight
+from .modules.implementations import DSPreRMSNorm, GroupedGemmMoE, RaggedUnembed, _PackedWeight
 
 
 class _Layer:
@@ -288,9 +288,9 @@ class RaggedTransformer:
 
     def _expert_parts(self, L, x):
         """A routed layer's output before it is summed (ops/experts.py ``ExpertSum``) where the norm behind it, the next layer's
-        or the logits', can sum it; else None."""
+        or the logits', can sum it; else None. A registered module that derives from the stock one may compute something else."""
         behind = self.unembed_mod if L is self.layers[-1] else self.norm_mod
-        if (self.tp != 1 or L["w13"] is None or L.routed is None or not x.shape[0] or not hasattr(self.moe_mod, "parts")
+        if (self.tp != 1 or L["w13"] is None or L.routed is None or not x.shape[0] or type(self.moe_mod) is not GroupedGemmMoE
                 or type(behind) not in (DSPreRMSNorm, RaggedUnembed)):
             return None
         return self.moe_mod.parts(x, L["w2"], L.routed)

@@ -36,3 +36,30 @@ def test_norm_of_an_expert_sum(W, T, k, shared, sorted_rows):
 
 def test_norm_of_an_expert_sum_elsewhere():
     _check(*_parts(3, 24, 2, True, True, "cpu"))
+
+
+def test_parts_of_stock_modules_only():
+    """A module that derives from the stock one and computes something else is called, not passed by."""
+    from types import SimpleNamespace
+
+    from hcache_deepspeed_amd.inference.v2.model import RaggedTransformer, _Layer
+    from hcache_deepspeed_amd.inference.v2.modules import DSMoEConfig
+    from hcache_deepspeed_amd.inference.v2.modules.implementations import DSPreRMSNorm, GroupedGemmMoE, RaggedUnembed
+
+    class Own(GroupedGemmMoE):
+
+        def forward(self, x, *a):
+            return 2 * x
+
+        def parts(self, *a):
+            raise AssertionError("passed by")
+
+    L = _Layer()
+    L.w.update({"w13": torch.zeros(2, 8, 8), "w2": torch.zeros(2, 8, 4), "router.w": None})
+    L.routed = {}
+    m = SimpleNamespace(tp=1, layers=[L], moe_mod=Own(DSMoEConfig(8, 4, 2, 1, "silu_glu", True)),
+                        norm_mod=DSPreRMSNorm(None), unembed_mod=RaggedUnembed(None))
+    x = torch.ones(3, 8)
+    assert RaggedTransformer._expert_parts(m, L, x) is None
+    m._moe = lambda L, x: RaggedTransformer._moe(m, L, x)
+    assert torch.equal(RaggedTransformer._mlp(m, L, x), 2 * x)
