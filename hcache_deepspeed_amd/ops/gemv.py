@@ -97,7 +97,11 @@ def rows_linear(x, w, b=None, glu=0):
     rows = w.shape[0]
     M, N = x.numel() // K, rows // 2 if glu else rows
     plan = _plan(M, N, K, 1 if glu else 0)
-    if plan == 0 or not native.plain(x, w, b) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.dim() != 2 or \
+    # (autocast to another type is the library call's to see, and so is a tensor on another device than the current one, whose
+    # stream the launch would take)
+    if plan == 0 or torch.is_autocast_enabled() or x.get_device() != torch.cuda.current_device():
+        return None
+    if not native.plain(x, w, b) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.dim() != 2 or \
             not w.is_contiguous() or K != w.shape[1] or w.get_device() != x.get_device():
         return None
     x2 = x if x.dim() == 2 else x.reshape(M, K)

@@ -80,3 +80,16 @@ def test_linear_rows_refuse():
         assert torch.func.vmap(gemv.linear, in_dims=(0, None))(rows, w).shape == (2, 64, 4096)
     w.requires_grad_()
     assert gemv.linear(x[:, :8192], w).grad_fn is not None
+
+
+@pytest.mark.gpu
+def test_linear_rows_leave_autocast_and_other_devices(monkeypatch):
+    """Autocast to another type decides the result's type; a tensor of another device than the current one is the library's."""
+    x = torch.ones(64, 4096, dtype=torch.bfloat16, device="cuda")
+    w = torch.ones(4096, 4096, dtype=torch.bfloat16, device="cuda")
+    with torch.no_grad():
+        assert gemv.rows_linear(x, w) is not None
+        with torch.autocast("cuda", torch.float16):
+            assert gemv.linear(x, w).dtype == torch.float16
+        monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+        assert gemv.rows_linear(x, w) is None
