@@ -202,7 +202,8 @@ def _packed_rows(x2, q_weight, scales, out_features, in_features, group_size, fm
     anything could want a record of it."""
     M, N, K = x2.shape[0], out_features, in_features
     plan = _packed_plan(M, N, K, group_size, fmt, 1 if glu else 0)
-    if plan == 0 or not native.bare(x2, q_weight, bias) or (bias is not None and _needs_grad(bias)):
+    # (under autocast what runs otherwise decides the type of the result)
+    if plan == 0 or torch.is_autocast_enabled() or not native.bare(x2, q_weight, bias) or (bias is not None and _needs_grad(bias)):
         return None
     x2 = x2.contiguous()
     if (x2.data_ptr() | q_weight.data_ptr()) % 16 or (bias is not None and bias.dtype != torch.bfloat16):

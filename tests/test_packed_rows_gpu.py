@@ -59,3 +59,12 @@ def test_gated_rows_on_packed_weights(fmt, M, N, K, act):
     # each factor within half a unit of the last place and its sum's error; |act'| <= 1.13
     bound = 2**-8 * (1.13 * gate.abs() * up.abs() + 2 * ref.abs()) + 1.13 * (eg * up.abs() + eu * gate.abs()) + 1e-6
     assert ((y.double() - ref).abs() <= bound).all()
+
+
+def test_packed_rows_leave_autocast():
+    """Of 65 rows and more the weights are dequantized for a library product, whose type autocast decides."""
+    q, s, _ = _packed("int8", 4096, 4096, 128)
+    x = torch.ones(128, 4096, dtype=torch.bfloat16, device="cuda")
+    with torch.no_grad(), torch.autocast("cuda", torch.float16):
+        assert Q._packed_rows(x, q, s, 4096, 4096, 128, "int8", 3, None, 0) is None
+        assert Q.int_linear(x, q, s, 4096, 4096, 128).dtype == torch.float16
