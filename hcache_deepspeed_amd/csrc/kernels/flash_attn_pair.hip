@@ -91,7 +91,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt] = f32x16{};
   bf16x8 pb[4];
-  float m = -INFINITY, l = 0.f;
+  float m = -INFINITY, muse = 0.f, l = 0.f;  // muse: m, or 0 where all scores so far are minus infinity
 
   // P.V of one tile and S of the next: eight groups of four fragments, each read while the one before it is multiplied
   auto products = [&](auto PV, auto S, int vbuf, int kbuf) __attribute__((always_inline)) {
@@ -128,10 +128,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
   // S of tile kt -> P in bf16, the running maximum and sums. Masked scores are replaced by the power of two that makes 2^28 to
   // 2^29 in the exponent (see attn_fwd_w64_kernel): whatever a key that a row does not see holds, it does not count.
+  auto masked_score = [&] { return 0x80000000 | ((127 + 28 + 127 - (__float_as_int(c) >> 23)) << 23); };
   auto softmax = [&](int kt) __attribute__((always_inline)) {
     const int k0 = kt * BN;
     if (k0 + BN > len || k0 + BN - 1 > wq_lo || (p.window > 0 && k0 <= wq_hi - p.window) || wq_hi >= len) {
-      const int masked = 0x80000000 | ((127 + 28 + 127 - (__float_as_int(c) >> 23)) << 23);
+      const int masked = masked_score();
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
         const int base = k0 + 32 * t + 4 * h, A = base - klo, B = khi - base;
@@ -151,7 +152,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     t0 = max3_raw(t0, s[0][15], s[1][15]);
     const float top = xor32_max(max3_raw(t0, t1, t1)) * c;
     if (!__all(top <= m + kDeferThr)) {
-      const float next = fmaxf(m, top), alpha = fast_exp2(m - next);  // the scores are finite: so is the new maximum
+      const float next = fmaxf(m, top);
+      muse = next == -INFINITY ? 0.f : next;
+      const float alpha = fast_exp2(m - muse);
       m = next;
       l *= alpha;
 #pragma unroll
@@ -162,8 +165,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
-        s[t][r] = fast_exp2(__builtin_fmaf(s[t][r], c, -m));
-        s[t][r + 1] = fast_exp2(__builtin_fmaf(s[t][r + 1], c, -m));
+        s[t][r] = fast_exp2(__builtin_fmaf(s[t][r], c, -muse));
+        s[t][r + 1] = fast_exp2(__builtin_fmaf(s[t][r + 1], c, -muse));
         l0 += s[t][r];
         l1 += s[t][r + 1];
       }
@@ -252,7 +255,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const float m1 = sums[lane], l1 = sums[64 + lane], top = fmaxf(m, m1);
   const float a0 = m == -INFINITY ? 0.f : fast_exp2(m - top), a1 = m1 == -INFINITY ? 0.f : fast_exp2(m1 - top);
   l = l * a0 + l1 * a1;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  // A part that does not count may hold anything (values of masked keys). A sum that is not a number, of a NaN or of plus
+  // infinity, and a row that sees minus infinity alone, whose sum is 0 or of masked keys, come out NaN, as softmax gives them.
+  const float inv = top <= __int_as_float(masked_score()) * c ? NAN : 1.f / l;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll

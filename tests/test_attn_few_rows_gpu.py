@@ -63,3 +63,42 @@ def test_many_blocks_take_the_larger_workgroups():
         at = torch.arange(s + n)
         kv = cache[tab[i, at // 64].long().cuda(), (at % 64).cuda()]
         _close(o[q0:q0 + n], _attend(q[q0:q0 + n], kv[:, 0], kv[:, 1], s, True, 0)[0])
+
+
+@pytest.mark.parametrize("few", [True, False])
+@pytest.mark.parametrize("what,window", [("query", 0), ("query", 100), ("inf", 0), ("inf", 100), ("nan", 0), ("nan", 100), ("tile", 0),
+                                         ("all", 0)])
+def test_values_that_are_not_finite(what, window, few):
+    """On either side of the 512 workgroups: rows of a NaN query (with and without masked keys in their last tile), rows that
+    see a score of plus infinity, a NaN key, or minus infinity alone come out NaN, as softmax gives them; scores of minus
+    infinity, a whole tile of them too, count nothing. Finite rows as above."""
+    g = torch.Generator(device="cuda").manual_seed(7)
+    lens, seen, hq, hkv = ([130, 300, 40], [64, 200, 0], 8, 2) if few else ([130, 300] * 6, [64, 200] * 6, 32, 8)
+    cache, tab, metas, T, batch = _setup(lens, seen, hkv, 64, "cuda", torch.Generator().manual_seed(8))
+    q = torch.randn(T, hq, D, device="cuda", generator=g).bfloat16()
+    blocks = [(i, r) for i, n in enumerate(lens) for r in range(0, n, 256)]
+    assert (len(blocks) * hq <= 512) == few
+    for i, (q0, n, s) in enumerate(metas):
+        at = torch.arange(s + n)
+        blk, slot = tab[i, at // 64].long().cuda(), (at % 64).cuda()
+        if what == "query":
+            for row in {63 - s % 64, 0, 17, n // 2, n - 1} & set(range(n)):
+                q[q0 + row] = math.nan
+        elif what in ("inf", "nan"):  # half of the queries see plus, half minus infinity
+            first = s + n // 3
+            cache[blk[first], slot[first], 0, :, 0] = math.inf if what == "inf" else math.nan
+        else:
+            gone = slice(64, 128) if what == "tile" else slice(None)
+            q[q0:q0 + n, :, 0] = 1
+            cache[blk[gone], slot[gone], 0, :, 0] = -math.inf
+    o = paged_attention_portions(q, cache, None, torch.tensor(blocks, dtype=torch.int32, device="cuda"), batch, hq, hkv, D**-0.5,
+                                 window)
+    for i, (q0, n, s) in enumerate(metas):
+        at = torch.arange(s + n)
+        kv = cache[tab[i, at // 64].long().cuda(), (at % 64).cuda()]
+        want, got = _attend(q[q0:q0 + n], kv[:, 0], kv[:, 1], s, True, window)[0].transpose(0, 1), o[q0:q0 + n].transpose(0, 1)
+        gone = want.isnan().any(-1)
+        assert what == "tile" or gone.any()
+        assert got[gone].isnan().all() and not got[~gone].isnan().any(), i
+        if not gone.all():
+            _close(got[~gone], want[~gone])
