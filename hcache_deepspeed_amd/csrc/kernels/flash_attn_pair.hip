@@ -10,6 +10,8 @@
 // kernel takes 759 of 943 us at 16,000 tokens (without the softmax 836, without the loads too 768): the products at the
 // clock that they leave, 1.38 PFLOP/s, are what it runs at. The groups joined once a turn instead of twice: 998 us; one group
 // of MFMAs ahead 977.
+#include <algorithm>
+
 #include "flash_attn_shared.h"
 
 namespace {
@@ -26,17 +28,27 @@ __device__ __forceinline__ float xor32_sum(float x) {
 // Queries are the new tokens of a sequence behind earlier ones, keys and values lie in the paged cache, causal (as in
 // attn_fwd_w64_kernel; an entry of the list is 256 new tokens, which two workgroups share here). A kernel of contiguous rows
 // made a forward of 2 x 509 tokens 25 -> 16 us, but the training step it is part of 1 % faster only.
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_pair_kernel(AttnParams p) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_pair_kernel(AttnParams p, int n) {
   constexpr int D = 128, BM = 128, KS = 8, DT = 4, TL = 16384, PW = 4;
   __shared__ __attribute__((aligned(1024))) char smem[8 * TL];  // a group: K[2], V[2]
-  // the second 128 rows of an entry, which see more keys, before its first; the heads of a key head on one XCD
-  const int at = blockIdx.x / (2 * p.hq), r = blockIdx.x % (2 * p.hq), half = r < p.hq, rr = half ? r : r - p.hq;
+  // By groups of entries: a workgroup a head of each, for its second 128 rows, which see more keys, where it has them, then those
+  // for the first rows of such. A group is of a multiple of 32 heads: workgroups go round the XCDs and their 4 shader engines, and
+  // empty ones of short entries that come in shorter runs meet the same engines, which then idle (entry by entry, 16
+  // sequences of 16 tokens behind 60, 16 heads, 14.9 us, so 9.4; 64 of 64 tokens, 4 heads 19.7 and 10.5). Larger groups part the
+  // halves, of whose keys one finds the other's in L2 (all entries in one, 8 of 256 tokens behind 1,500, 32 / 32 heads 71 -> 88).
+  // The heads of a key head are on one XCD.
+  const int g = 32 >> min(5, __builtin_ctz(p.hq)), e0 = blockIdx.y * g, run = min(g, n - e0) * p.hq;
+  const int later = (int)blockIdx.x >= run, place = blockIdx.x - later * run;
+  if (place >= run) return;
+  const int at = e0 + place / p.hq, rr = place % p.hq;
   const int hq = p.hq % 8 == 0 ? (rr % 8) * (p.hq / 8) + rr / 8 : rr;
-  const int seq = p.blocks[2 * at], row0 = p.blocks[2 * at + 1] + (half ? BM : 0);
+  const int seq = p.blocks[2 * at], first = p.blocks[2 * at + 1];
   const int n_new = p.meta[3 * seq + 1], seen = p.meta[3 * seq + 2];
+  const bool two = first + BM < n_new;
+  if (first >= n_new || (later && !two)) return;
+  const int row0 = first + (two && !later ? BM : 0);
   const int start = p.meta[3 * seq] - seen, len = seen + n_new, q0 = seen + row0;
   const int* table = p.tables + (int64_t)seq * p.max_blocks;
-  if (row0 >= n_new) return;
   const int hk = hq / (p.hq / p.hkv);
   const int lane = threadIdx.x & 63, h = lane >> 5;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w = wv & 3, grp = wv >> 2;
@@ -276,6 +288,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // n: entries of 256 new tokens
 int hds_attn_fwd_pair_paged_launch(const void* params, size_t params_bytes, int n, int hq, hipStream_t st) {
   if (params_bytes != sizeof(AttnParams)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(attn_fwd_pair_kernel, dim3(2 * n * hq), dim3(512), 0, st, *static_cast<const AttnParams*>(params));
+  const int g = 32 >> std::min(5, __builtin_ctz(hq));
+  hipLaunchKernelGGL(attn_fwd_pair_kernel, dim3(2 * g * hq, (n + g - 1) / g), dim3(512), 0, st,
+                     *static_cast<const AttnParams*>(params), n);
   return hipGetLastError();
 }

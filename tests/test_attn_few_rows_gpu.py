@@ -102,3 +102,19 @@ def test_values_that_are_not_finite(what, window, few):
         assert got[gone].isnan().all() and not got[~gone].isnan().any(), i
         if not gone.all():
             _close(got[~gone], want[~gone])
+
+
+@pytest.mark.parametrize("hq,hkv", [(1, 1), (3, 1), (6, 2), (12, 4), (24, 8), (40, 8), (64, 8)])
+def test_every_row_of_every_head(hq, hkv):
+    """Short entries between long ones, heads and entries that do not fill a group of the launch's order."""
+    g = torch.Generator(device="cuda").manual_seed(hq)
+    lens, seen = [256, 9, 129, 1, 128, 300, 20], [0, 70, 3, 64, 0, 5, 130]
+    cache, tab, metas, T, batch = _setup(lens, seen, hkv, 64, "cuda", torch.Generator().manual_seed(9))
+    q = torch.randn(T, hq, D, device="cuda", generator=g).bfloat16()
+    blocks = [(i, r) for i, n in enumerate(lens) for r in range(0, n, 256)]
+    assert len(blocks) * hq <= 512
+    o = paged_attention_portions(q, cache, None, torch.tensor(blocks, dtype=torch.int32, device="cuda"), batch, hq, hkv, D**-0.5)
+    for i, (q0, n, s) in enumerate(metas):
+        at = torch.arange(s + n)
+        kv = cache[tab[i, at // 64].long().cuda(), (at % 64).cuda()]
+        _close(o[q0:q0 + n], _attend(q[q0:q0 + n], kv[:, 0], kv[:, 1], s, True, 0)[0])
