@@ -1684,12 +1684,13 @@ HDS_EXPORT int hds_attn_bwd(const void* q, const void* k, const void* v, const v
 // Causal attention of new tokens over the paged cache [blocks, block_size, 2, hkv, 128], head size 128, bf16. blocks: device
 // int32 [n_blocks][2], sequence and first of 256 new tokens; seq_meta: device int32 [sequences][3], first row of q, new
 // tokens, earlier tokens. q and o: [tokens, hq, 128] with token strides sq, so. block_size % 64 == 0, less than 2^31 slots.
-// scale from 2^-64 to 2^64: the maximum is one of raw scores, and masked ones are made from its exponent.
+// scale from 2^-64 to 2^64: the maximum is one of raw scores, and masked ones are made from its exponent. rows: 128 or 256 a
+// workgroup, 0: by the length of the list.
 HDS_EXPORT int hds_paged_prefill(const void* q, int64_t sq, const void* cache, void* o, int64_t so, const int* blocks,
                                  int n_blocks, const int* seq_meta, const int* block_tables, int max_blocks,
-                                 int block_size, int hq, int hkv, float scale, int window, hipStream_t st) {
+                                 int block_size, int hq, int hkv, float scale, int window, int rows, hipStream_t st) {
   if (n_blocks <= 0) return 0;
-  if (hq < 1 || hkv < 1 || hq % hkv || sq % 8 || so % 8 || block_size < 64 || block_size % 64 || max_blocks < 1 ||
+  if (hq < 1 || hkv < 1 || hq % hkv || (rows != 0 && rows != 128 && rows != 256) || sq % 8 || so % 8 || block_size < 64 || block_size % 64 || max_blocks < 1 ||
       window < 0 || !(scale >= 0x1p-64f && scale <= 0x1p64f) || (int64_t)n_blocks * hq > 0x7fffffff || (int64_t)64 * 2 * hkv * 128 * 2 > 0x7fffffff)
     return hipErrorInvalidValue;
   const int64_t slot = (int64_t)2 * hkv * 128;
@@ -1701,9 +1702,10 @@ HDS_EXPORT int hds_paged_prefill(const void* q, int64_t sq, const void* cache, v
   p.tables = block_tables;
   p.max_blocks = max_blocks;
   p.block_size = block_size;
-  // 128 rows a workgroup (flash_attn_pair.hip) where those of 256 are at most two a CU. New tokens, 256 rows
-  // -> 128, us: 512 behind 789, 32 / 8 heads 37 -> 21; 701, 527 and 279 of three prompts, 16 / 4 32 -> 18; 2,048, 32 / 8 79 -> 57;
-  // 16,000, 16 / 4, 1,008 workgroups of 256 rows, level.
-  if ((int64_t)n_blocks * hq <= 512) return hds_attn_fwd_pair_paged_launch(&p, sizeof(p), n_blocks, hq, st);
+  // By 128 rows (flash_attn_pair.hip) where workgroups of 256 are at most two a CU, if the caller, who knows the lengths, does not
+  // say. New tokens, 256 rows -> 128, us: 512 behind 789, 32 / 8 heads 37 -> 21; 701, 527 and 279 of three prompts, 16 / 4
+  // 32 -> 18; 2,048, 32 / 8 79 -> 57; 16,000, 16 / 4, 1,008 workgroups of 256 rows, level.
+  if (rows == 128 || (rows == 0 && (int64_t)n_blocks * hq <= 512))
+    return hds_attn_fwd_pair_paged_launch(&p, sizeof(p), n_blocks, hq, st);
   return hds_attn_fwd_w64_paged_launch(&p, sizeof(p), n_blocks, hq, st);
 }

@@ -85,7 +85,7 @@ class DSDenseBlockedAttention(DSSelfAttentionBase):
         if portions is not None and portions_ok(qkv[:, :nq], cache, nq, nkv, c.scale_factor):
             toks, blocks, rows = portions
             return paged_attention_portions(qkv[:, :nq], cache, toks, blocks, batch, nq, nkv, c.scale_factor,
-                                            c.sliding_window, rows).reshape(T, nq * D)
+                                            c.sliding_window, rows, getattr(batch, "prefill_rows", 0)).reshape(T, nq * D)
         o = paged_attention(qkv[:, :nq], cache, batch.atoms, batch.n_atoms, batch.seq_meta, batch.block_tables, nq,
                             nkv, c.scale_factor, c.sliding_window, batch.seq_meta_host, batch.tables_host,
                             decode=T == batch.current_sequences)

@@ -129,7 +129,7 @@ _KERNEL_SIGS = {
     "hds_wmix_splits": "iii",
     "hds_wmix_supported": "iiii",
     "hds_wmix_resident": "iii",
-    "hds_paged_prefill": "pl" + "p" + "pl" + "pi" + "pp" + "iiii" + "f" + "i" + "s",
+    "hds_paged_prefill": "pl" + "p" + "pl" + "pi" + "pp" + "iiii" + "f" + "ii" + "s",
     "hds_wmix_skinny": "ppppp" + "iiiiiii" + "s",
     "hds_wmix_gemm": "pppppp" + "iiiiii" + "s",
     "hds_token_gather": "i" + "ppp" + "iiii" + "s",

@@ -5,7 +5,7 @@ import torch
 from . import native
 from .paged import DECODE_MAX, ROWS_PER_ATOM
 
-# new tokens of an entry of the prefill kernel's list: one workgroup a head, or two of half the rows where there are few
+# new tokens of an entry of the prefill kernels' list: one workgroup a head, or two of half the rows (``prefill_rows``)
 PREFILL_ROWS = 256
 
 
@@ -25,11 +25,40 @@ def make_portions(seq_meta_host, portions=None):
 
 # Microseconds of the kernels, fitted to 1 to 64 sequences of 2 to 256 new tokens behind 60 to 4,000 earlier ones, 8 / 1 to 64 / 8
 # and 32 / 32 heads (within a fifth, at least about the lines between them). Prefill kernel and row blocks: the longest
-# workgroup, or all of them over the CUs (256 at a time; of the row blocks about 270). One by one: the contexts are read from
-# memory once, from the caches once a token.
+# workgroup, or all of them over the CUs (256 at a time, by 256 rows; of the row blocks about 270). One by one: the contexts
+# are read from memory once, from the caches once a token.
 def _prefill_us(seqs, heads):
     longest = max(7 + 0.031 * (seen + n) for n, seen in seqs)
     return max(longest, heads / 256 * sum(-(-n // PREFILL_ROWS) * (7 + 0.031 * (seen + n / 2)) for n, seen in seqs))
+
+
+# The prefill kernels on lists of up to so many workgroups of 256 rows, by the rows of a workgroup: us of one, and a key (of 1,736
+# lists of 9 to 2,048 new tokens, 4 / 4 to 32 / 32 heads, 130 to 512 workgroups: 13 % rms)
+SHORT_LIST = 512
+_WALK_US = {128: (7.5, 0.0145), 256: (8.5, 0.033)}
+
+
+def _launch_us(seqs, heads, rows):
+    """The longest workgroup, all of them over the CUs, or the rounds of 256 that workgroups of much the same length take."""
+    us, per_key = _WALK_US[rows]
+    last = sorted((seen + min(r + rows, n) for n, seen in seqs for r in range(0, n, rows)), reverse=True)
+    rounds = max((k + 1) * (us + per_key * last[256 * k // heads]) for k in range((heads * len(last) - 1) // 256 + 1))
+    return max(rounds, heads / 256 * (us * len(last) + per_key * sum(last)))
+
+
+def prefill_rows(seqs, heads):
+    """Rows of a workgroup of the prefill kernel for these (new, earlier) tokens, 128 (csrc/kernels/flash_attn_pair.hip) or 256
+    (flash_attn_w64.hip). Half of the rows take half of the time in twice the workgroups: where those of 256 fill the chip
+    in whole rounds, twice as many rounds of 128 take as long and longer (8 sequences of 200 tokens behind 60, 32 / 8 heads
+    23.0 us by 128 rows, 20.8 by 256; 16 43.2 and 38.8), unless lengths differ (8 behind up to 1,500 44 and 61) or the second
+    halves are empty (16 of 64 behind 500 30 and 44). Over 1,736 lists of 130 to 512 workgroups 0.77 of the time of 256 rows, at
+    most 1.07; with 128 rows for all of them 0.78 and 1.27."""
+    blocks = heads * sum(-(-n // PREFILL_ROWS) for n, _ in seqs)
+    if blocks > SHORT_LIST:
+        return 256
+    if 2 * blocks <= 256 or max(n for n, _ in seqs) <= 128:  # (no question: 128 rows are the faster ones)
+        return 128
+    return 128 if _launch_us(seqs, heads, 128) <= _launch_us(seqs, heads, 256) else 256
 
 
 def _rows_us(seqs, heads, kv_heads):
@@ -43,13 +72,21 @@ def _tokens_us(seqs, kv_heads):
     return 6 + kv_heads * sum((seen + n) * (6e-5 + 3.8e-5 * n) + 6e-3 * n for n, seen in seqs)
 
 
+def _many_us(seqs, heads):
+    """``_prefill_us``, of short lists by the rows that they run with: of 257 to 512 workgroups the division by it is 0.4 % slower
+    than the better of both (at most 1.16 of its time), by the estimate of 256 rows 5.6 % (2.25)."""
+    rows = prefill_rows(seqs, heads)
+    short = heads * sum(-(-n // PREFILL_ROWS) for n, _ in seqs) <= SHORT_LIST
+    return _launch_us(seqs, heads, rows) if short else _prefill_us(seqs, heads)
+
+
 def divide_step(seq_meta_host, heads, kv_heads):
     """``make_portions`` for these head counts, and flat list of (sequence, kv head, first row) of the sequences that run in
     row blocks: (tokens, blocks, atoms). Two cases leave ``make_portions``'s division:
 
     * many portions of few tokens: the prefill kernel has a workgroup a query head for each of them, 256 at a time, row
       blocks have one a key head (32 sequences of 16 tokens, up to 4,000 keys, 32 / 8 heads: 331 us against 226; 16
-      sequences 176 / 213, of 64 tokens 140 / 220);
+      sequences 76 / 206, up to 60 keys 16 / 10);
     * many sequences of 2 to ``DECODE_MAX`` tokens, whose contexts are read once a token: 32 of 8 tokens there 237 us
       against 221 in row blocks, up to 1,000 keys 69 / 58, up to 300 34 / 20; of 4 tokens 155 / 224, 41 / 57, 20 / 20.
 
@@ -72,7 +109,7 @@ def divide_step(seq_meta_host, heads, kv_heads):
     if kv_heads * sum(new[s][0] for s in few) > 512 and _tokens_us(of(few), kv_heads) > best(few + many) - best(many):
         few, many = [], few + many
     if heads * sum(-(-new[s][0] // PREFILL_ROWS) for s in many) <= 256 or \
-            _prefill_us(of(many), heads) <= _rows_us(of(many), heads, kv_heads):
+            _many_us(of(many), heads) <= _rows_us(of(many), heads, kv_heads):
         return (*make_portions(seq_meta_host, set(many)), [])
     if ones and _tokens_us(of(ones), kv_heads) > _rows_us(of(ones + many), heads, kv_heads) - _rows_us(of(many), heads, kv_heads):
         many = many + ones
@@ -95,10 +132,10 @@ def portions_ok(q, cache, n_q, n_kv, scale=1.0):
             and q.stride(0) % 8 == 0 and q.stride(1) == 128 and q.data_ptr() % 16 == 0)
 
 
-def paged_attention_portions(q, cache, toks, blocks, batch, n_q, n_kv, scale, window=0, atoms=None):
+def paged_attention_portions(q, cache, toks, blocks, batch, n_q, n_kv, scale, window=0, atoms=None, rows=0):
     """``paged_attention`` of a step that mixes single tokens and portions of prompts: ``toks`` (int32 rows of q) on the
-    split-key kernel, which spreads a token's context over the chip, ``blocks`` ([n, 2] int32) on the prefill kernel,
-    ``atoms`` ([n, 3] int32) in row blocks. There a single token walks its whole context in one workgroup (9 such tokens,
+    split-key kernel, which spreads a token's context over the chip, ``blocks`` ([n, 2] int32) on the prefill kernel by ``rows``
+    (``prefill_rows``; 0: by the length of the list), ``atoms`` ([n, 3] int32) in row blocks. There a single token walks its whole context in one workgroup (9 such tokens,
     up to 3,000 keys, 8 key heads, beside 512 new ones: 171 us; apart 29 + 38 us)."""
     T, _, D = q.shape
     o = torch.empty(T, n_q, D, device=q.device, dtype=q.dtype)
@@ -122,7 +159,7 @@ def paged_attention_portions(q, cache, toks, blocks, batch, n_q, n_kv, scale, wi
         native.check(
             lib.hds_paged_prefill(q.data_ptr(), q.stride(0), cache.data_ptr(), o.data_ptr(), n_q * D,
                                   blocks.data_ptr(), blocks.shape[0], batch.seq_meta.data_ptr(), tab.data_ptr(), mb, bs,
-                                  n_q, n_kv, float(scale), int(window), st), "paged_prefill")
+                                  n_q, n_kv, float(scale), int(window), int(rows), st), "paged_prefill")
     if atoms is not None and atoms.shape[0]:
         native.check(
             lib.hds_paged_attn(q.data_ptr(), q.stride(0), cache.data_ptr(), o.data_ptr(), n_q * D, atoms.data_ptr(),

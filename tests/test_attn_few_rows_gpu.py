@@ -118,3 +118,20 @@ def test_every_row_of_every_head(hq, hkv):
         at = torch.arange(s + n)
         kv = cache[tab[i, at // 64].long().cuda(), (at % 64).cuda()]
         _close(o[q0:q0 + n], _attend(q[q0:q0 + n], kv[:, 0], kv[:, 1], s, True, 0)[0])
+
+
+@pytest.mark.parametrize("rows", [128, 256])
+def test_either_kernel_on_request(rows):
+    """The caller's choice, on both sides of where the length of the list would make it."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    for lens, seen, hq, hkv in (([200, 300], [60, 5], 8, 2), ([200, 70, 140] * 6, [60, 0, 500] * 6, 32, 8)):
+        cache, tab, metas, T, batch = _setup(lens, seen, hkv, 64, "cuda", torch.Generator().manual_seed(2))
+        q = torch.randn(T, hq, D, device="cuda", generator=g).bfloat16()
+        blocks = torch.tensor([(i, r) for i, n in enumerate(lens) for r in range(0, n, 256)], dtype=torch.int32, device="cuda")
+        o = paged_attention_portions(q, cache, None, blocks, batch, hq, hkv, D**-0.5, rows=rows)
+        for i, (q0, n, s) in enumerate(metas):
+            at = torch.arange(s + n)
+            kv = cache[tab[i, at // 64].long().cuda(), (at % 64).cuda()]
+            _close(o[q0:q0 + n], _attend(q[q0:q0 + n], kv[:, 0], kv[:, 1], s, True, 0)[0])
+        with pytest.raises(RuntimeError):
+            paged_attention_portions(q, cache, None, blocks, batch, hq, hkv, D**-0.5, rows=64)
