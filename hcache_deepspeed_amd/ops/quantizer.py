@@ -205,13 +205,18 @@ def _packed_rows(x2, q_weight, scales, out_features, in_features, group_size, fm
     # (under autocast what runs otherwise decides the type of the result)
     if plan == 0 or torch.is_autocast_enabled() or not native.bare(x2, q_weight, bias) or (bias is not None and _needs_grad(bias)):
         return None
+    # (what the dequantized weight's view and the library's product refuse is theirs to refuse)
+    rows = 2 * N if glu else N
+    if scales.numel() * group_size != rows * K or q_weight.device != x2.device or scales.device != x2.device or (bias is not None and (
+            bias.dtype != torch.bfloat16 or bias.shape != (rows, ) or bias.device != x2.device)):
+        return None
     x2 = x2.contiguous()
-    if (x2.data_ptr() | q_weight.data_ptr()) % 16 or (bias is not None and bias.dtype != torch.bfloat16):
+    if (x2.data_ptr() | q_weight.data_ptr()) % 16:
         return None
     if bias is not None:
         bias = bias.contiguous()
     y = torch.empty(M, N, dtype=torch.bfloat16, device=x2.device)
-    part = torch.empty(plan // 16, M, 2 * N if glu else N, dtype=torch.float32, device=x2.device) if plan >= 32 else None
+    part = torch.empty(plan // 16, M, rows, dtype=torch.float32, device=x2.device) if plan >= 32 else None
     native.check(native.kernels().hds_packed_rows(x2.data_ptr(), q_weight.data_ptr(), scales.data_ptr(), native.ptr(bias),
                                                   y.data_ptr(), native.ptr(part), M, N, K, group_size, _FMTS[fmt], int(ebits),
                                                   int(glu), plan, native.stream()), "packed_rows")
