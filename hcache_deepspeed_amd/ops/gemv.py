@@ -53,6 +53,11 @@ MAX_ROWS = 16  # of either kernel
 SKINNY_MIN_M = int(_os.environ.get("HDS_SKINNY_MIN_M", "2"))  # 1: one-row linears too (instead of the VALU GEMV)
 
 
+def _skinny_wanted(n, K):
+    """Do the switches leave up to MAX_ROWS rows (n values of K) to the matrix-core kernels, the tiled one of 9 rows and more too?"""
+    return SKINNY and n >= SKINNY_MIN_M * K
+
+
 def skinny_ok(x2, w, b=None):
     if not (SKINNY and native.use_native(x2) and x2.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
             and w.dim() == 2):
@@ -133,9 +138,10 @@ def glu_linear(x, w, b, act):
         return None
     if x.numel() > 256 * x.shape[-1] or _needs_grad(x, w, b):
         return None
-    if x.numel() > 8 * x.shape[-1]:
+    n, K = x.numel(), x.shape[-1]
+    if n > MAX_ROWS * K or (n > 8 * K and _skinny_wanted(n, K)):
         y = rows_linear(x, w, b, 1 + _GATHER_ACTS[act])
-        if y is not None or x.numel() > MAX_ROWS * x.shape[-1]:
+        if y is not None or n > MAX_ROWS * K:
             return y
     x2 = x.reshape(-1, x.shape[-1])
     if not skinny_ok(x2, w, b) or w.shape[0] % 2:
@@ -160,7 +166,7 @@ def linear(x, w, b=None):
             if y is not None:
                 return y
         elif not _needs_grad(x, w, b):
-            if n > 8 * K:
+            if n > 8 * K and _skinny_wanted(n, K):
                 y = rows_linear(x, w, b)
                 if y is not None:
                     return y

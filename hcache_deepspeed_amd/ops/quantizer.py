@@ -140,6 +140,8 @@ _INT_GEMV_MAX_M = min(8, int(os.environ.get("HDS_INT_GEMV_MAX_M", "2")))
 
 # above 64 rows dequantize-once + hipBLASLt wins on most shapes (profiles/wmix_bench_r2.log)
 _WMIX_MAX_M = int(os.environ.get("HDS_WMIX_MAX_M", "64"))
+# set, it holds for the tiles of csrc/kernels/linear_packed.hip too (rows behind the streams', see ``_packed_rows``)
+_PACKED_MAX_M = int(os.environ.get("HDS_WMIX_MAX_M", "512"))
 
 
 def _needs_grad(x):
@@ -201,6 +203,8 @@ def _packed_rows(x2, q_weight, scales, out_features, in_features, group_size, fm
     """The packed-weight product of more rows (csrc/kernels/linear_packed.hip): mostly 17 to 256; None where it does not apply or
     anything could want a record of it."""
     M, N, K = x2.shape[0], out_features, in_features
+    if M > max(16, _PACKED_MAX_M):
+        return None
     plan = _packed_plan(M, N, K, group_size, fmt, 1 if glu else 0)
     # (under autocast what runs otherwise decides the type of the result)
     if plan == 0 or torch.is_autocast_enabled() or not native.bare(x2, q_weight, bias) or (bias is not None and _needs_grad(bias)):

@@ -93,3 +93,21 @@ def test_linear_rows_leave_autocast_and_other_devices(monkeypatch):
             assert gemv.linear(x, w).dtype == torch.float16
         monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
         assert gemv.rows_linear(x, w) is None
+
+
+@pytest.mark.gpu
+def test_linear_rows_heed_the_switches(monkeypatch):
+    """HDS_SKINNY_GEMM=0 and HDS_SKINNY_MIN_M leave 9 to 16 rows to the library, as those of the skinny kernel; 17 are not theirs."""
+    w = torch.ones(28672, 4096, dtype=torch.bfloat16, device="cuda")
+    asked = []
+    monkeypatch.setattr(gemv, "rows_linear", lambda x, *a: asked.append(x.shape[0]))
+    with torch.no_grad():
+        def call(M):
+            x = torch.ones(M, 4096, dtype=torch.bfloat16, device="cuda")
+            gemv.linear(x, w), gemv.glu_linear(x, w, None, "silu")
+        call(12)
+        monkeypatch.setattr(gemv, "SKINNY_MIN_M", 13)
+        call(12), call(13)
+        monkeypatch.setattr(gemv, "SKINNY", False)
+        call(13), call(17)
+    assert asked == [12, 12, 13, 13, 17, 17]

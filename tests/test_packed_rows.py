@@ -39,3 +39,14 @@ def test_bias_is_a_row_of_the_result(launched):
                  torch.zeros(N, dtype=torch.bfloat16, device="meta")):
         assert _rows(bias=bias) is None
     assert not launched and _rows(bias=torch.zeros(N).bfloat16()).shape == (M, N)
+
+
+def test_row_limit_of_the_environment(launched, monkeypatch):
+    """HDS_WMIX_MAX_M bounds these tiles too, but not the few rows that would run as a stream otherwise."""
+    monkeypatch.setattr(Q, "_PACKED_MAX_M", M - 1)
+    assert _rows() is None and not launched
+    monkeypatch.setattr(Q, "_PACKED_MAX_M", M)
+    assert _rows() is not None
+    monkeypatch.setattr(Q, "_PACKED_MAX_M", 0)
+    monkeypatch.setitem(globals(), "M", 16)
+    assert _rows() is not None
