@@ -111,3 +111,38 @@ def test_linear_rows_heed_the_switches(monkeypatch):
         monkeypatch.setattr(gemv, "SKINNY", False)
         call(13), call(17)
     assert asked == [12, 12, 13, 13, 17, 17]
+
+
+@pytest.mark.gpu
+def test_linear_rows_leave_watched_calls():
+    """Of 17 rows and more the product is the library's wherever something records or replaces operations: a dispatch mode (a
+    trace by make_fx, a counter), a function mode other than a default device, torch.compile."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+    M, N, K = 64, 4096, 4096
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x, other = (torch.randn(M, K, device="cuda", generator=g).bfloat16() for _ in range(2))
+    w = (torch.randn(N, K, device="cuda", generator=g) * K**-0.5).bfloat16()
+    with torch.no_grad():
+        traced = make_fx(lambda t: gemv.linear(t, w))(x)
+        assert torch.equal(traced(other), torch.nn.functional.linear(other, w))
+        with FlopCounterMode(display=False) as count:
+            gemv.linear(x, w)
+        assert count.get_total_flops() == 2 * M * N * K
+        seen = []
+
+        class Names(TorchFunctionMode):
+
+            def __torch_function__(self, f, types, args=(), kwargs=None):
+                seen.append(f)
+                return f(*args, **(kwargs or {}))
+
+        with Names():
+            gemv.linear(x, w)
+        assert torch.nn.functional.linear in seen
+        graphs = []
+        whole = torch.compile(gemv.linear, backend=lambda m, a: graphs.append(m) or m.forward, fullgraph=True)
+        assert torch.equal(whole(x, w), torch.nn.functional.linear(x, w)) and len(graphs) == 1
+        with torch.device("cuda"):
+            assert gemv.rows_linear(x, w) is not None
