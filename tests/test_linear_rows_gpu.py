@@ -30,8 +30,8 @@ def test_linear_rows_match_64_bits(M, N, K):
 
 @pytest.mark.gpu
 def test_linear_rows_all_tiles_exact():
-    """Every tile and number of slices that the choice takes over its range: small integers, whose sums are exact in 32 bits
-    and the result in bf16."""
+    """The tiles and numbers of slices that the choice takes for one matrix over its range of rows: small integers, whose sums are
+    exact in 32 bits and the result in bf16."""
     g = torch.Generator(device="cuda").manual_seed(1)
     K, N = 8192, 4096
     w = torch.randint(-1, 2, (N, K), device="cuda", generator=g).bfloat16()
@@ -41,6 +41,36 @@ def test_linear_rows_all_tiles_exact():
     for M in list(range(17, 300, 16)) + list(range(300, 1100, 97)):
         with torch.no_grad():
             assert torch.equal(gemv.linear(x[:M], w).float(), ref[:M]), M
+
+
+TILES = [(32, 64), (32, 128), (64, 64), (64, 128), (128, 128), (192, 128), (256, 128), (256, 256)]  # kTiles: rows, columns
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("glu", [0, 3])  # 3: relu, exact on integers
+@pytest.mark.parametrize("S", [1, 3])
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_linear_rows_each_tile(tile, S, glu):
+    """Every kernel by name, whatever the choice: one tile of rows and two, remainders of rows and columns, reductions that the ring holds
+    and longer ones, walks apart; nothing is written beside the result."""
+    from hcache_deepspeed_amd.ops import native
+    R, W = TILES[tile]
+    g = torch.Generator(device="cuda").manual_seed(tile)
+    for M, K in ((R - 3, 448), (R + 5, 2048), (9, 1088)):
+        N = (W // 2 if glu else W) + 24
+        rows = 2 * N if glu else N
+        w = torch.randint(-1, 2, (rows, K), device="cuda", generator=g).bfloat16()
+        x = (torch.randint(-1, 2, (M, K), device="cuda", generator=g) * (torch.rand(M, K, device="cuda", generator=g) < 8 / K)).bfloat16()
+        b = torch.randint(-2, 3, (rows, ), device="cuda", generator=g).bfloat16()
+        y = torch.full((M + 1, N + 8), 7.0, device="cuda", dtype=torch.bfloat16)
+        part = torch.empty(S, M, rows, device="cuda")
+        native.check(native.kernels().hds_linear_bf16(x.data_ptr(), K, w.data_ptr(), b.data_ptr(), y.data_ptr(), N + 8, part.data_ptr(), M,
+                                                      N, K, glu, tile + 16 * S, native.stream()), "linear_bf16")
+        ref = x.float() @ w.float().t() + b.float()
+        if glu:
+            ref = ref[:, :N].relu() * ref[:, N:]
+        assert 0 < ref.abs().max() <= 256
+        assert torch.equal(y[:M, :N].float(), ref) and (y[M:] == 7).all() and (y[:, N:] == 7).all(), (M, K)
 
 
 @pytest.mark.gpu

@@ -68,3 +68,38 @@ def test_packed_rows_leave_autocast():
     with torch.no_grad(), torch.autocast("cuda", torch.float16):
         assert Q._packed_rows(x, q, s, 4096, 4096, 128, "int8", 3, None, 0) is None
         assert Q.int_linear(x, q, s, 4096, 4096, 128).dtype == torch.float16
+
+
+TILES = [(16, 64), (32, 64), (64, 64), (128, 128)]  # kTiles: rows, weight rows
+
+
+@pytest.mark.parametrize("fmt", ["int8", "int4", "fp6_e3m2", "fp6_e2m3"])
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("S", [1, 3])
+@pytest.mark.parametrize("tile", range(len(TILES)))
+def test_each_tile_on_packed_weights(tile, S, glu, fmt):
+    """Every kernel by name, whatever the choice: one tile of rows and two, remainders, reductions that the ring holds and longer ones,
+    groups of a stage and of several; the bounds of the tests above."""
+    from hcache_deepspeed_amd.ops import native
+    R, W = TILES[tile]
+    torch.manual_seed(tile)
+    for M, K, G in ((R - 3, 512, 128), (R + 5, 2304, 1152), (4, 1536, 768)):
+        N = (W // 2 if glu else W) + 12
+        rows = 2 * N if glu else N
+        q, s, wd = _packed(fmt, rows, K, G)
+        x = torch.randn(M, K, device="cuda", dtype=torch.bfloat16)
+        bias = None if glu else torch.randn(N, device="cuda").bfloat16()
+        y = torch.full((M + 1, N), 7.0, device="cuda", dtype=torch.bfloat16)
+        part = torch.empty(S, M, rows, device="cuda")
+        native.check(native.kernels().hds_packed_rows(
+            x.data_ptr(), q.data_ptr(), s.data_ptr(), native.ptr(bias), y.data_ptr(), part.data_ptr(), M, N, K, G,
+            {"int8": 0, "int4": 1}.get(fmt, 2), 2 if fmt == "fp6_e2m3" else 3, 1 if glu else 0, tile + 16 * S, native.stream()), "packed_rows")
+        ref, err = x.double() @ wd.t(), 1e-5 * (x.double().abs() @ wd.abs().t())
+        if glu:
+            (gate, up), (eg, eu) = ref.split(N, 1), err.split(N, 1)
+            ref = torch.nn.functional.silu(gate) * up
+            bound = 2**-8 * (1.13 * gate.abs() * up.abs() + 2 * ref.abs()) + 1.13 * (eg * up.abs() + eu * gate.abs()) + 1e-6
+        else:
+            ref = ref + bias.double()
+            bound = 2**-8 * ref.abs() + err + 1e-5 * bias.double().abs()
+        assert ((y[:M].double() - ref).abs() <= bound).all() and (y[M:] == 7).all(), (M, K)
