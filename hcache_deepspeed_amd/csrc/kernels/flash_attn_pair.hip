@@ -1,15 +1,16 @@
-// FlashAttention forward over a paged cache, head size 128, by workgroups of 128 query rows: for steps whose 256-row workgroups
-// (flash_attn_w64.hip) leave CUs idle or are of few lengths, as prompts of up to some thousand tokens.
+// FlashAttention forward over a paged cache, head size 128, by workgroups of 128 query rows: for steps whose 256-row
+// workgroups (flash_attn_w64.hip) leave CUs idle or differ in their lengths, as prompts of up to some thousand tokens
+// (ops/paged_prefill.py ``prefill_rows`` chooses).
 //
 // What bounds the 256-row kernel there is its chain: each of its waves has a SIMD to itself and walks all keys, 1.9 us a tile
-// of 64, whether a quarter of the CUs work or all. Here two groups of four waves take the tiles of 64 keys in turn, for
-// the same 128 rows (32 a wave), and their parts are added through LDS at the end: half the rows and half the tiles a wave. The
+// of 64, whether a quarter of the CUs work or all. Here two groups of four waves take the tiles of 64 keys in turn, for the
+// same 128 rows (32 a wave), and their parts are added through LDS at the end: half the rows and half the tiles a wave. The
 // groups share the SIMDs and go round a turn half a turn apart, joined by barriers: while one group multiplies (P.V of its
-// tile and S of its next one, 32 MFMAs a wave), the other does its softmax. Fragments are read from LDS two groups of four MFMAs ahead.
-// At 32 rows a wave LDS reads are as long as the products; without them, without the softmax and without the loads the
-// kernel takes 759 of 943 us at 16,000 tokens (without the softmax 836, without the loads too 768): the products at the
-// clock that they leave, 1.38 PFLOP/s, are what it runs at. The groups joined once a turn instead of twice: 998 us; one group
-// of MFMAs ahead 977.
+// tile and S of its next one, 32 MFMAs a wave), the other does its softmax. Fragments are read from LDS two groups of four
+// MFMAs ahead. At 32 rows a wave LDS reads are as long as the products; without them, without the softmax and without the
+// loads the kernel takes 759 of 943 us at 16,000 tokens (without the softmax 836, without the loads too 768): the products at
+// the clock that they leave, 1.38 PFLOP/s, are what it runs at. The groups joined once a turn instead of twice: 998 us; one
+// group of MFMAs ahead 977.
 #include <algorithm>
 
 #include "flash_attn_shared.h"
@@ -31,12 +32,12 @@ __device__ __forceinline__ float xor32_sum(float x) {
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_pair_kernel(AttnParams p, int n) {
   constexpr int D = 128, BM = 128, KS = 8, DT = 4, TL = 16384, PW = 4;
   __shared__ __attribute__((aligned(1024))) char smem[8 * TL];  // a group: K[2], V[2]
-  // By groups of entries: a workgroup a head of each, for its second 128 rows, which see more keys, where it has them, then those
-  // for the first rows of such. A group is of a multiple of 32 heads: workgroups go round the XCDs and their 4 shader engines, and
-  // empty ones of short entries that come in shorter runs meet the same engines, which then idle (entry by entry, 16
-  // sequences of 16 tokens behind 60, 16 heads, 14.9 us, so 9.4; 64 of 64 tokens, 4 heads 19.7 and 10.5). Larger groups part the
-  // halves, of whose keys one finds the other's in L2 (all entries in one, 8 of 256 tokens behind 1,500, 32 / 32 heads 71 -> 88).
-  // The heads of a key head are on one XCD.
+  // By groups of entries: a workgroup a head of each, for its second 128 rows, which see more keys, where it has them, then
+  // those for the first rows of such. A group is of a multiple of 32 heads: workgroups go round the XCDs and their 4 shader
+  // engines, and empty ones of short entries that come in shorter runs meet the same engines, which then idle (entry by
+  // entry, 16 sequences of 16 tokens behind 60, 16 heads, 14.9 us, so 9.4; 64 of 64 tokens, 4 heads 19.7 and 10.5). Larger
+  // groups part the halves, of whose keys one finds the other's in L2 (all entries in one, 8 of 256 tokens behind 1,500, 32 /
+  // 32 heads 71 -> 88). The heads of a key head are on one XCD.
   const int g = 32 >> min(5, __builtin_ctz(p.hq)), e0 = blockIdx.y * g, run = min(g, n - e0) * p.hq;
   const int later = (int)blockIdx.x >= run, place = blockIdx.x - later * run;
   if (place >= run) return;
@@ -194,9 +195,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // The groups take turns at the matrix cores: while one multiplies, the other, on the same SIMDs, does its softmax.
-  // Turn i of a wave: the softmax of its tile i, then that tile's P.V beside S of the next.
-  // Loads of a turn: V of the next tile and K of the one behind it, into the buffers of the last one's. They have a turn to arrive.
+  // The groups take turns at the matrix cores: while one multiplies, the other, on the same SIMDs, does its softmax. Turn i
+  // of a wave: the softmax of its tile i, then that tile's P.V beside S of the next. Loads of a turn: V of the next tile and
+  // K of the one behind it, into the buffers of the last one's. They have a turn to arrive.
   stage(false, 0);
   stage(true, 0);
   if (turns > 1) {

@@ -837,8 +837,8 @@ int hds_attn_fwd_w64_launch(const void* params, size_t params_bytes, int batch, 
 // The forward over a paged cache (D = 128, causal): params as above with blocks, meta, tables, max_blocks, block_size set;
 // n: entries of blocks. Measured at 16,000 new tokens, 16 query and 4 key heads: the 128-row kernel of paged_attn.hip 2,625
 // us (0.40 PF/s), this one 937 us (1.12 PF/s; 1,080 in a model's step); 2,048 tokens, 32 and 8 heads: 143 and 62 us (77);
-// 512 new behind 789 earlier ones: about 80 and 43 us. Fewer workgroups than two a CU run in flash_attn_pair.hip, many short
-// portions in row blocks (ops/paged_prefill.py).
+// 512 new behind 789 earlier ones: about 80 and 43 us. Of up to two workgroups a CU most lists run in flash_attn_pair.hip, many
+// short portions in row blocks (ops/paged_prefill.py).
 int hds_attn_fwd_w64_paged_launch(const void* params, size_t params_bytes, int n, int hq, hipStream_t st) {
   if (params_bytes != sizeof(AttnParams)) return hipErrorInvalidValue;
   const AttnParams& p = *static_cast<const AttnParams*>(params);

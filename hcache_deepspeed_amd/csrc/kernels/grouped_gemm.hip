@@ -561,7 +561,6 @@ HDS_EXPORT int hds_experts_gemm(const void* x, int64_t ldx, const int* src, int 
   // 256 x 256 tiles, which read the rows half as often and the weights once per 256 of them, from 512 rows an expert on: 8
   // experts, 2 a token, 14336 x 4096: 1,500 tokens 1,774 us against 1,534 here, 2,000 2,063 / 2,054, 2,700 2,390 / 2,488; 64
   // experts, 6 a token, 1024 x 2048: 3,000 540 / 427, 6,000 786 / 733, 12,000 1,262 / 1,315.
-  const int cols_of = glu ? 2 : 1;
   const bool big = N % big_cols == 0 && T >= 2 * BM2 * E;
   // otherwise gg_flow_kernel's tiles
   const FlowTile flow = flow_tile(T, N, K, E, glu);
@@ -574,11 +573,12 @@ HDS_EXPORT int hds_experts_gemm(const void* x, int64_t ldx, const int* src, int 
     hipLaunchKernelGGL(kernel, dim3(N / cols * max_tiles), dim3(512), 0, st, (const bf16*)x, ldx, src, n_src, (const bf16*)w,
                        (bf16*)y, offs, tile_e, tile_m, n_tiles, T, N, K, ldy, N / cols, unit, more...);
   };
-  // Weights that one tile of rows reads go past the caches: 66 tokens, gate and up + down, 64 experts of 1024 x 2048 98.5 + 53.8 -> 87 + 46
-  // us, 8 of 14336 x 4096 325 + 160 -> 297 + 140, 16 of 4096 x 4096 199 + 92 -> 180 + 80; 1,600 131 + 80 -> 128 + 74. Tiles of one expert
-  // find them in L2 or the memory-side cache (past it 3,000 tokens of the first, gate and up 235 / 252, 1,400 of 8 of 5632 x 2048
-  // 191 / 202), unless an expert's are too many (2,090 choices of 8 of 14336 x 4096, 117 and 235 MB, a layer 1,470 -> 1,333).
-  const bool once = T <= BM2 * E || (int64_t)cols_of * N * K >= 1 << 25;
+  // Weights that one tile of rows reads go past the caches: 66 tokens, gate and up + down, 64 experts of 1024 x 2048
+  // 98.5 + 53.8 -> 87 + 46 us, 8 of 14336 x 4096 325 + 160 -> 297 + 140, 16 of 4096 x 4096 199 + 92 -> 180 + 80; 1,600 tokens of
+  // the first 131 + 80 -> 128 + 74. Tiles of one expert find them in L2 or the memory-side cache (past it 3,000 tokens of the first,
+  // gate and up 235 / 252, 1,400 of 8 of 5632 x 2048 191 / 202), unless an expert's are too many (2,090 choices of 8 of
+  // 14336 x 4096, 117 and 235 MB, a layer 1,470 -> 1,333).
+  const bool once = T <= BM2 * E || (int64_t)(glu ? 2 : 1) * N * K >= 1 << 25;
 #define HDS_FLOW(GA, GL, NT)                                               \
   do {                                                                     \
     if (wr == 256) run(gg_flow_kernel<GA, GL, 256, NT>, apart);            \

@@ -1,26 +1,27 @@
 // y[M, N] = x[M, K] . w[N, K]^T (+ bias) in bf16, sums in 32 bits: projections of more rows than the decode kernels take
 // (gemv.hip) and fewer than a library product fills the chip with, with the gated unit of w = [gate; up] in the epilogue.
 //
-// What bounds these shapes is idle CUs, or a weight stream that library tiles do not keep up: [4096, 14336] at 521 rows has 48
-// tiles of 192 x 256, and the library's smaller ones leave L2 as the limit (111 us, 0.56 PFLOP/s). So the reduction is split
-// where that pays: every (tile, slice of K) is a workgroup, partial sums go to memory in 32 bits and a second kernel adds
-// them in their order, so that results repeat bit for bit.
+// What bounds these shapes is idle CUs, or a weight stream that library tiles do not keep up: [4096, 14336] at 521 rows has
+// 48 tiles of 192 x 256, and the library's smaller ones leave L2 as the limit (111 us, 0.56 PFLOP/s). So the reduction is
+// split where that pays: every (tile, slice of K) is a workgroup, partial sums go to memory in 32 bits and a second kernel
+// adds them in their order, so that results repeat bit for bit.
 //
 // A workgroup keeps a ring of D stages of 64 k in LDS, filled by LDS-DMA through a buffer descriptor (what lies behind the
-// matrices is read as zeros, and unlike global_load_lds it leaves the compiler its counted LDS waits). Rows of 128 bytes keep their
-// 16-byte pieces at c ^ ((row >> 1) & 7), which spreads a fragment read over all banks. Half a stage (32 k) is read into
-// registers while the half before it is multiplied, with one barrier a stage; waiting for all reads of a stage first, as two
-// groups of waves in turn, took 0.62 instead of 0.50 us a stage at 128 x 128.
+// matrices is read as zeros, and unlike global_load_lds it leaves the compiler its counted LDS waits). Rows of 128 bytes keep
+// their 16-byte pieces at c ^ ((row >> 1) & 7), which spreads a fragment read over all banks. Half a stage (32 k) is read
+// into registers while the half before it is multiplied, with one barrier a stage; waiting for all reads of a stage first, as
+// two groups of waves in turn, took 0.62 instead of 0.50 us a stage at 128 x 128.
 //
-// Time a stage with a full chip, us (PFLOP/s): 64 x 128 0.32 (0.85), 128 x 128 0.43 - 0.50 (1.1), 192 x 128 0.76 (1.1), 256 x 128
-// 0.73 - 0.90 (1.2), 256 x 256 1.36 - 1.59 (1.35). The small ones are bound by the lines that a CU has on the way (64 bytes a
-// ns), the large ones by LDS reads beside the products. Tiles of 32 rows share a CU, so that one's prologue and epilogue lie
-// beside another's stream. Weight rows a multiple of 4 KB apart lie alike in the memory's channels: there each column of
-// tiles begins its walk along K somewhere else ([28672, 4096], 24 rows 42.5 -> 38.2 us).
+// Time a stage with a full chip, us (PFLOP/s): 64 x 128 0.32 (0.85), 128 x 128 0.43 - 0.50 (1.1), 192 x 128 0.76 (1.1), 256 x
+// 128 0.73 - 0.90 (1.2), 256 x 256 1.36 - 1.59 (1.35). The small ones are bound by the lines that a CU has on the way (64
+// bytes a ns), the large ones by LDS reads beside the products. Tiles of 32 rows share a CU, so that one's prologue and
+// epilogue lie beside another's stream. Weight rows a multiple of 4 KB apart lie alike in the memory's channels: there each
+// column of tiles begins its walk along K somewhere else ([28672, 4096], 24 rows 42.5 -> 38.2 us).
 //
-// Weights not in the caches, us, library -> here: [4096, 14336] 64 / 128 / 192 / 286 / 521 / 1,018 rows 40 / 75 / 103 / 77 / 111 / 129 -> 30 / 35
-// / 40 / 55 / 83 / 105; [4096, 4096] 96 / 128 / 192 / 256 22 / 24 / 33 / 23 -> 15 / 16 / 19 / 20; [28672, 4096] gated 24 / 64 / 128 53 / 54 /
-// 58 -> 38 / 40 / 49; [11264, 2048] gated 24 / 128 / 256 20 / 22 / 31 -> 14 / 20 / 25.
+// Weights not in the caches, us, library -> here: [4096, 14336] 64 / 128 / 192 / 286 / 521 / 1,018 rows 40 / 75 / 103 / 77 /
+// 111 / 129 -> 30 / 35 / 40 / 55 / 83 / 105; [4096, 4096] 96 / 128 / 192 / 256 22 / 24 / 33 / 23 -> 15 / 16 / 19 / 20;
+// [28672, 4096] gated 24 / 64 / 128 53 / 54 / 58 -> 38 / 40 / 49; [11264, 2048] gated 24 / 128 / 256 20 / 22 / 31 -> 14 / 20
+// / 25.
 #include <algorithm>
 #include <cmath>
 
@@ -40,8 +41,8 @@ struct LinearArgs {
   int M, N, K, S, tm, tn, act, nt, apart;
 };
 
-// RB, CB: 16-row blocks of x and of w a wave; WM x WN waves, OCC workgroups a CU. GLU: w is [gate; up] of N rows each; half of a
-// tile's and of a wave's columns are gates, the others the same features of up.
+// RB, CB: 16-row blocks of x and of w a wave; WM x WN waves, OCC workgroups a CU. GLU: w is [gate; up] of N rows each; half
+// of a tile's and of a wave's columns are gates, the others the same features of up.
 template <int RB, int CB, int WM, int WN, int OCC, bool GLU>
 __global__ __launch_bounds__(64 * WM * WN, WM * WN * OCC / 4) void linear_kernel(LinearArgs p) {
   constexpr int R = 16 * RB * WM, W = 16 * CB * WN, NW = WM * WN, PER = (R + W) / (8 * NW);
@@ -178,9 +179,9 @@ constexpr Tile kTiles[] = {{32, 64, 2, 5.5f, 0.13f},   {32, 128, 2, 5.8f, 0.23f}
 constexpr int kMaxSlices = 12;
 
 // The tile and the slices of K that take least by this estimate: the stages of the fullest CU, the weights at 8.4 TB/s (fewer
-// bytes a second where CUs have fewer workgroups than the fullest) and all stages at 19 TB/s from L2, cubes added, since
-// they overlap in part; a further round costs 2.6 us and a sum of slices 1.8 + 1.1 a million floats, and 2 of the host's. Fitted to
-// 11,000 times of 20 shapes, 5 to 1,018 rows (8 % rms); the choice is 2 % slower than the best one measured.
+// bytes a second where CUs have fewer workgroups than the fullest) and all stages at 19 TB/s from L2, cubes added, since they
+// overlap in part; a further round costs 2.6 us and a sum of slices 1.8 + 1.1 a million floats, and 2 of the host's. Fitted
+// to 11,000 times of 20 shapes, 5 to 1,018 rows (8 % rms); the choice is 2 % slower than the best one measured.
 static int linear_choice(int M, int N, int K) {
   float least = 0.f;
   int best = 0;
@@ -204,39 +205,45 @@ static int linear_choice(int M, int N, int K) {
 
 }  // namespace
 
-// How hds_linear_bf16 takes these rows, as tile + 16 x slices of K, or 0 where a library product is the faster one. N: columns of
-// y; glu: of 2N rows of w. For callers to keep by size: the estimates take 3 us of the host.
+// How hds_linear_bf16 takes these rows, as tile + 16 x slices of K, or 0 where a library product is the faster one. N:
+// columns of y; glu: of 2N rows of w. For callers to keep by size: the estimates take 3 us of the host.
 HDS_EXPORT int hds_linear_plan(int M, int N, int K, int glu) {
   if (M < 9 || M > 1100 || N < 8 || K < 4 * BK || K % BK || N % 8 || K > 1 << 22 || N > 1 << 22) return 0;
   const int rows = glu ? 2 * N : N;
   const int64_t size = (int64_t)rows * K;
   if (size >= (int64_t)1 << 31) return 0;
   // Weights not in the caches, times as fast as the library (up to 16 rows as skinny_lines_kernel):
-  // - up to 128 rows, which read the weights once at 6 TB/s and more: [28672, 4096] gated 24 / 64 / 128 rows 53 / 54 / 58 us ->
-  //   38 / 40 / 49, [32000, 4096] 59 / 56 / 59 -> 41 / 42 / 51, [10240, 8192] 1.0 - 1.8, [15360, 5120] 0.9 - 1.1; small matrices level as
-  //   kernels ([2048, 2048], [3072, 2048] 0.8 - 1.05), but 10 us of host time instead of the library's 19, which is what bounds
-  //   steps of short prompts. Up to 16 rows where the matrix is large and not sliced: [28672, 4096] 8 / 12 / 16 rows 38.8 / 42.6 /
-  //   45.1 -> 37.3 / 37.3 / 37.5, [32000, 4096] 41.5 / 44.9 / 49.2 -> 40.0 / 40.4 / 40.4; smaller ones 0.6 - 1.03.
+  // - up to 128 rows, which read the weights once at 6 TB/s and more: [28672, 4096] gated 24 / 64 / 128 rows 53 / 54 / 58 us
+  //   -> 38 / 40 / 49, [32000, 4096] 59 / 56 / 59 -> 41 / 42 / 51, [10240, 8192] 1.0 - 1.8, [15360, 5120] 0.9 - 1.1; small
+  //   matrices level as kernels ([2048, 2048], [3072, 2048] 0.8 - 1.05), but 10 us of host time instead of the library's 19,
+  //   which is what bounds steps of short prompts (40 tokens, four layers of width 2048 663 -> 519 us, of 4096 656 -> 540).
+  //   Up to 16 rows where the matrix is large and not sliced: [28672, 4096] 8 / 12 / 16 rows 38.8 / 42.6 / 45.1 -> 37.3 /
+  //   37.3 / 37.5, [32000, 4096] 41.5 / 44.9 / 49.2 -> 40.0 / 40.4 / 40.4; smaller ones 0.6 - 1.03.
   const int choice = linear_choice(M, rows, K), S = choice / 16;
   if (M <= 16) return S == 1 && size >= 1 << 25 ? choice : 0;
-  // 17 to 32 are decode steps, whose launches are recorded once: smaller matrices are the library's ([2048, 2048], 24 rows 8.2 us in
-  // a step / 10.4).
+  // 17 to 32 rows are decode steps, whose launches are recorded once, more often than prompts: smaller matrices are the
+  // library's (18 / 24 / 32 sequences, four layers of width 2048, with all of them here 296 / 283 / 315 -> 321 / 309 / 337
+  // us, two of 4096 299 / 300 / 358 -> 302 / 304 / 366; a prompt of 24 tokens 658 -> 513). From 33 on recorded steps are
+  // level or faster here too (33 / 48 / 64 sequences, four layers of width 2048 382 / 418 / 433 -> 366 / 393 / 396, two of
+  // 4096 352 / 376 / 381 -> 350 / 373 / 389, within the noise), although [2048, 2048] alone takes 8.6 / 10.4 us.
   if (M <= 32 && !glu && size < 3 << 23) return 0;
   bool take = M <= 128;
-  // - up to 256 with a gated unit, whose kernel and pass it saves ([28672, 4096] 0.93 - 1.04, [11264, 2048] 1.2), or not
-  //   much wider than deep ([6144, 4096] 1.04 - 1.35, [4096, 4096] 1.1 - 1.7, [8192, 8192] 1.2 - 1.6), as [32000, 4096] (0.95 - 1.02) is;
+  // - up to 256 with a gated unit, whose kernel and pass it saves ([28672, 4096] 0.93 - 1.04, [11264, 2048] 1.2), or not much
+  //   wider than deep ([6144, 4096] 0.87 - 1.35, [4096, 4096] 0.86 - 1.7, [8192, 8192] 1.2 - 1.6), as [32000, 4096] (0.95 -
+  //   1.02) is (prompts of 137 / 170 / 200 / 256 tokens, four layers of width 4096, qkv and o 818 / 782 / 779 / 885 -> 777 /
+  //   804 / 774 / 852);
   take = take || (M <= 256 && (glu || (K >= 4096 && 2 * rows <= 3 * K)));
   // - to 320 where the library's call is the longer half (0.8 - 1.1; two layers of width 2048, 310 tokens 452 -> 345 us);
   take = take || (M <= 320 && !glu && size <= 1 << 25);
-  // - long reductions into few columns, whatever the rows: [4096, 14336] 1.0 - 2.3, [5120, 13824] 0.94 - 2.4. Beyond, the library's
-  //   products are the faster ones (521 rows: [28672, 4096] 0.8, [11264, 2048] 0.85, [6144, 4096] 1.0).
+  // - long reductions into few columns, whatever the rows: [4096, 14336] 1.0 - 2.3, [5120, 13824] 0.94 - 2.4. Beyond, the
+  //   library's products are the faster ones (521 rows: [28672, 4096] 0.8, [11264, 2048] 0.85, [6144, 4096] 1.0).
   take = take || (K >= 8192 && 2 * rows <= K && size >= 1 << 24);
   return take ? choice : 0;
 }
 
-// x [M, ldx], w [N, K], bias [N] or null, y [M, ldy], plan: hds_linear_plan's, part: S x M x N floats where its slices S are more
-// than one. glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu): w [2N, K] is gate rows, then up rows, y = act(gate) up,
-// and bias and part are of 2N columns. Rows of x and w begin at 16 bytes, of y at 8.
+// x [M, ldx], w [N, K], bias [N] or null, y [M, ldy], plan: hds_linear_plan's, part: S x M x N floats where its slices S are
+// more than one. glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu): w [2N, K] is gate rows, then up rows, y =
+// act(gate) up, and bias and part are of 2N columns. Rows of x and w begin at 16 bytes, of y at 8.
 HDS_EXPORT int hds_linear_bf16(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy, float* part,
                                int M, int N, int K, int glu, int plan, hipStream_t st) {
   const int S = plan / 16, tile = plan % 16;

@@ -1,18 +1,20 @@
-// y[M, N] = x[M, K] . dequant(w)[N, K]^T (+ bias) for weight-only quantized w (int8, int4, FP6 e3m2 / e2m3, fp32 scales of groups
-// along k), x and y bf16, with the gated unit of w = [gate; up] in the epilogue: more rows than the streams of wmix_gemm.hip take.
+// y[M, N] = x[M, K] . dequant(w)[N, K]^T (+ bias) for weight-only quantized w (int8, int4, FP6 e3m2 / e2m3, fp32 scales of
+// groups along k), x and y bf16, with the gated unit of w = [gate; up] in the epilogue: more rows than the streams of
+// wmix_gemm.hip take.
 //
-// What bounds these shapes is the weight stream, as in linear.hip, whose ring of LDS-DMA stages, tiles, slices of K and walks it
-// shares; a stage is 128 k here, for one scale a weight row. Weights stay packed until a wave has its 32 rows' k in registers:
-// codes become bf16, which holds them exactly (packed_codes.h), and a group's 32-bit sum is scaled, so no weight is rounded. The
-// tile kernel of wmix_gemm.hip loads 32 bytes a lane from rows that lie apart and scales before it rounds.
+// What bounds these shapes is the weight stream, as in linear.hip, whose ring of LDS-DMA stages, tiles, slices of K and walks
+// it shares; a stage is 128 k here, for one scale a weight row. Weights stay packed until a wave has its 32 rows' k in
+// registers: codes become bf16, which holds them exactly (packed_codes.h), and a group's 32-bit sum is scaled, so no weight
+// is rounded. The tile kernel of wmix_gemm.hip loads 32 bytes a lane from rows that lie apart and scales before it rounds.
 //
-// Loads from the ring have to be of native vector types: where they were of uint2 and uint4 the compiler, which then sees that
-// they may alias the LDS-DMA, waited for every stage on its way (int8 [28672, 4096] gated, 24 rows 41.3 instead of 28.9 us).
+// Loads from the ring have to be of native vector types: where they were of uint2 and uint4 the compiler, which then sees
+// that they may alias the LDS-DMA, waited for every stage on its way (int8 [28672, 4096] gated, 24 rows 41.3 instead of 28.9
+// us).
 //
-// Weights not in the caches, us, tile kernel (to 64 rows) or dequantized for the library -> here, [28672, 4096] gated 24 / 64 / 128 / 256
-// rows: int8 50 / 59 / 119 / 142 -> 29 / 37 / 60 / 116, fp6 76 / 89 / 128 / 153 -> 29 / 38 / 60 / 116 (int8 at 16 rows reads 117 MB in 26 us);
-// [4096, 14336]: int8 29 / 33 / 91 / 92 -> 21 / 26 / 38 / 66, fp6 36 / 53 / 105 / 105 -> 20 / 26 / 40 / 66. Rows of 96 bytes a stage hold fp6 at
-// 3.8 TB/s.
+// Weights not in the caches, us, tile kernel (to 64 rows) or dequantized for the library -> here, [28672, 4096] gated 24 / 64
+// / 128 / 256 rows: int8 50 / 59 / 119 / 142 -> 29 / 37 / 60 / 116, fp6 76 / 89 / 128 / 153 -> 29 / 38 / 60 / 116 (int8 at 16
+// rows reads 117 MB in 26 us); [4096, 14336]: int8 29 / 33 / 91 / 92 -> 21 / 26 / 38 / 66, fp6 36 / 53 / 105 / 105 -> 20 / 26
+// / 40 / 66. Rows of 96 bytes a stage hold fp6 at 3.8 TB/s.
 #include <algorithm>
 #include <cmath>
 
@@ -207,9 +209,10 @@ struct Tile {
 constexpr Tile kTiles[] = {{16, 64, 2, 8.f, 0.25f}, {32, 64, 2, 8.1f, 0.28f}, {64, 64, 2, 8.7f, 0.39f}, {128, 128, 1, 10.3f, 1.29f}};
 constexpr int kMaxSlices = 14;
 
-// The tile and the slices of K that take least by this estimate: the stages of the fullest CU, the weights at 8.8 TB/s and all
-// stages at 16.5 TB/s from L2, cubes added, since they overlap in part; a further round costs 2.9 us and a sum of slices 0.2 + 1.1
-// a million floats. Fitted to 7,700 times of 17 shapes, 4 to 512 rows (7 % rms); the choice is 3 % slower than the best one measured.
+// The tile and the slices of K that take least by this estimate: the stages of the fullest CU, the weights at 8.8 TB/s and
+// all stages at 16.5 TB/s from L2, cubes added, since they overlap in part; a further round costs 2.9 us and a sum of slices
+// 0.2 + 1.1 a million floats. Fitted to 7,700 times of 17 shapes, 4 to 512 rows (7 % rms); the choice is 3 % slower than the
+// best one measured.
 static int packed_choice(int M, int N, int K, int G, int fmt) {
   const float bytes = fmt == kInt8 ? 1.f : fmt == kInt4 ? 0.5f : 0.75f;
   float least = 0.f;
@@ -235,8 +238,8 @@ static int packed_choice(int M, int N, int K, int G, int fmt) {
 
 }  // namespace
 
-// How hds_packed_rows takes these rows, as tile + 16 x slices of K, or 0 where other kernels are faster or it does not apply. N:
-// columns of y; glu: of 2N rows of w; fmt: 0 int8, 1 int4, 2 fp6. For callers to keep by size, as hds_linear_plan.
+// How hds_packed_rows takes these rows, as tile + 16 x slices of K, or 0 where other kernels are faster or it does not apply.
+// N: columns of y; glu: of 2N rows of w; fmt: 0 int8, 1 int4, 2 fp6. For callers to keep by size, as hds_linear_plan.
 HDS_EXPORT int hds_packed_plan(int M, int N, int K, int G, int fmt, int glu) {
   if (M < 4 || M > 512 || N < 4 || N % 4 || K < 2 * BK || K % BK || G < BK || G % BK || K % G || fmt < 0 || fmt > 2 ||
       N > 1 << 22 || K > 1 << 20)
@@ -245,25 +248,27 @@ HDS_EXPORT int hds_packed_plan(int M, int N, int K, int G, int fmt, int glu) {
   const int64_t size = (int64_t)rows * K;
   if (size >= (int64_t)1 << 31) return 0;
   // Weights not in the caches, times as fast as what runs otherwise:
-  // - up to 16 rows the streams of wmix_gemm.hip. Large int8 matrices 4 / 8 rows [10240, 8192] 1.22 / 1.34, [22016, 6144] gated 1.08 /
-  //   1.16, [28672, 4096] gated 8 rows 1.11; 9 / 16 rows [4096, 14336] 1.09 / 1.23, [20480, 5120] 1.22 / 1.28, [6144, 4096] 0.96 / 1.13,
-  //   [2048, 2048] 0.67 / 0.75. int4 and fp6 where the streams keep no rows resident: fp6 9 / 16 rows [15360, 5120] 1.28 / 1.37,
-  //   [8192, 8192] 1.02 / 1.13, [28672, 4096] gated 0.71 / 0.80; int4 12 rows [10240, 8192] 1.42, [22016, 6144] gated 0.96.
+  // - up to 16 rows the streams of wmix_gemm.hip. Large int8 matrices 4 / 8 rows [10240, 8192] 1.22 / 1.34, [22016, 6144]
+  //   gated 1.08 / 1.16, [28672, 4096] gated 8 rows 1.11; 9 / 16 rows [4096, 14336] 1.09 / 1.23, [20480, 5120] 1.22 / 1.28,
+  //   [6144, 4096] 0.96 / 1.13, [2048, 2048] 0.67 / 0.75. int4 and fp6 where the streams keep no rows resident: fp6 9 / 16
+  //   rows [15360, 5120] 1.28 / 1.37, [8192, 8192] 1.02 / 1.13, [28672, 4096] gated 0.71 / 0.80; int4 12 rows [10240, 8192]
+  //   1.42, [22016, 6144] gated 0.96.
   if (M <= 16 && size < (int64_t)1 << (fmt == kInt8 && M > 8 ? 25 : 26)) return 0;
   if (M <= 16 && fmt != kInt8 && (K <= 4096 || M < (fmt == kInt4 ? 12 : 9))) return 0;
-  // - to 64 rows the tiles of wmix_gemm.hip (and the fp6 stream of up to 32), to 256 the weights dequantized for a library product:
-  //   17 to 64 rows int8 1.16 - 1.77, int4 1.22 - 1.76, fp6 1.3 - 3.1 (small matrices to 32 rows 0.95 - 1.0); 96 and 128 rows 1.45 -
-  //   2.4 - 2.6; 192 and 256 rows 1.01 - 2.2.
+  // - to 64 rows the tiles of wmix_gemm.hip (and the fp6 stream of up to 32), to 256 the weights dequantized for a library
+  //   product: 17 to 64 rows int8 1.16 - 1.77, int4 1.22 - 1.76, fp6 1.3 - 3.1 (small matrices to 32 rows 0.95 - 1.0); 96 and
+  //   128 rows 1.45 - 2.6; 192 and 256 rows 1.01 - 2.2.
   if (M <= 32 && fmt == kFp6 && size < 1 << 23) return 0;
-  // - beyond, the weights are decoded for more rows than it saves passes: [28672, 4096] 384 / 512 rows 0.91 / 0.76; small matrices
-  //   gain by their launches ([2048, 2048] 1.1 / 1.2 - 1.4, [4096, 4096] 1.05 - 1.1 / 1.05 - 1.14, [6144, 4096] 0.9).
+  // - beyond, the weights are decoded for more rows than it saves passes: [28672, 4096] 384 / 512 rows 0.91 / 0.76; small
+  //   matrices gain by their launches ([2048, 2048] 1.1 / 1.2 - 1.4, [4096, 4096] 1.05 - 1.1 / 1.05 - 1.14, [6144, 4096]
+  //   0.9).
   if (M > 256 && (size > 1 << 24 || K > 4096)) return 0;
   return packed_choice(M, rows, K, G, fmt);
 }
 
-// x [M, K], w packed, scales [N, K / G], bias [N] or null, y [M, N], plan: hds_packed_plan's, part: S x M x N floats where its
-// slices S are more than one. ebits: fp6 3 (e3m2) or 2 (e2m3). glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu): w is 2N rows,
-// gate, then up, without a bias, and part of 2N columns. x and w begin at 16 bytes, y at 8.
+// x [M, K], w packed, scales [N, K / G], bias [N] or null, y [M, N], plan: hds_packed_plan's, part: S x M x N floats where
+// its slices S are more than one. ebits: fp6 3 (e3m2) or 2 (e2m3). glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2
+// relu): w is 2N rows, gate, then up, without a bias, and part of 2N columns. x and w begin at 16 bytes, y at 8.
 HDS_EXPORT int hds_packed_rows(const void* x, const void* w, const float* scales, const void* bias, void* y, float* part, int M,
                                int N, int K, int G, int fmt, int ebits, int glu, int plan, hipStream_t st) {
   const int S = plan / 16, tile = plan % 16, stages = S < 1 ? 0 : (K / BK + S - 1) / S;
@@ -273,8 +278,8 @@ HDS_EXPORT int hds_packed_rows(const void* x, const void* w, const float* scales
       (S > 1 && part == nullptr) || ((uintptr_t)x | (uintptr_t)w) & 15 || (uintptr_t)y & 7)
     return hipErrorInvalidValue;
   const int rows = glu ? 2 * N : N, R = kTiles[tile].rows, W = kTiles[tile].cols;
-  // Weights that one row of tiles reads go past the caches where a stage's share of a row is a whole line: int8 [28672, 4096] 16 /
-  // 64 rows 27.8 / 37.2 -> 25.8 / 36.8 us; fp6's three quarters of one 28.3 -> 33 us at 24 rows.
+  // Weights that one row of tiles reads go past the caches where a stage's share of a row is a whole line: int8 [28672, 4096]
+  // 16 / 64 rows 27.8 / 37.2 -> 25.8 / 36.8 us; fp6's three quarters of one 28.3 -> 33 us at 24 rows.
   PackedArgs p{(const bf16*)x, (const uint8_t*)w, scales, (const bf16*)bias, (bf16*)y, part, M, N, K, G, S, (M + R - 1) / R,
                glu ? (N + W / 2 - 1) / (W / 2) : (N + W - 1) / W, glu - 1, M <= R && fmt == kInt8};
   auto run = [&](auto kernel, int waves) {

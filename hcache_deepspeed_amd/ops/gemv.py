@@ -1,6 +1,7 @@
-"""Decode-sized bf16 linear on the HIP GEMV (csrc/kernels/gemv.hip): ``linear(x, w, b)`` equals ``F.linear`` and
-takes the GEMV path when x has at most 8 rows and the shape is one where the weight stream is faster than
-hipBLASLt's small-M GEMM (``profiles/gemv_bench_r2.jsonl``); everything else goes to ``F.linear``."""
+"""bf16 linears of up to 1,100 rows: ``linear(x, w, b)`` equals ``F.linear``. One row and the shapes where its weight stream is
+faster than hipBLASLt's small-M GEMM (``profiles/gemv_bench_r2.jsonl``) run the HIP GEMV, 2 to 16 rows the matrix-core skinny GEMM
+(both csrc/kernels/gemv.hip), 9 and more the tiled one (csrc/kernels/linear.hip) where ``hds_linear_plan`` takes them; everything
+else goes to ``F.linear``."""
 import functools
 
 import torch
@@ -55,7 +56,7 @@ SKINNY_MIN_M = int(_os.environ.get("HDS_SKINNY_MIN_M", "2"))  # 1: one-row linea
 
 
 def _skinny_wanted(n, K):
-    """Do the switches leave up to MAX_ROWS rows (n values of K) to the matrix-core kernels, the tiled one of 9 rows and more too?"""
+    """Do the switches leave up to MAX_ROWS rows (n values of K) to the matrix-core kernels, skinny or tiled?"""
     return SKINNY and n >= SKINNY_MIN_M * K
 
 
@@ -91,8 +92,8 @@ def _plan(M, N, K, glu=0):
 
 
 def _watched():
-    """Does a mode see or replace operations (a trace by make_fx, a counter, fake tensors; a default device does neither)? Behind
-    a bare kernel it would find the allocation of the result only."""
+    """Does a mode see or replace operations (a trace by make_fx, a counter, fake tensors; a default device does neither)?
+    Behind a bare kernel it would find the allocation of the result only."""
     n = torch._C._len_torch_function_stack()
     return torch._C._len_torch_dispatch_stack() > 0 or \
         (n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n)))
@@ -144,8 +145,8 @@ def _needs_grad(*tensors):
 
 
 def glu_linear(x, w, b, act):
-    """act(x . gate^T) * (x . up^T) for ``w`` = [gate; up] (and ``b``) in one call, for 2..16 rows of the skinny GEMM and 9..256 of
-    ``rows_linear``; None for anything else. The projections are rounded to bf16 first, as the separate kernels store them."""
+    """act(x . gate^T) * (x . up^T) for ``w`` = [gate; up] (and ``b``) in one call, for 2..16 rows of the skinny GEMM and 9..256
+    of ``rows_linear``; None for anything else. The projections are rounded to bf16 first, as the separate kernels store them."""
     if act not in _GATHER_ACTS or not (x.dim() >= 1 and x.is_cuda and torch.is_tensor(w)):
         return None
     if x.numel() > 256 * x.shape[-1] or _needs_grad(x, w, b):
@@ -167,13 +168,12 @@ def glu_linear(x, w, b, act):
 
 
 def linear(x, w, b=None):
-    """``F.linear(x, w, b)``; decode-sized bf16 inputs run the HIP GEMV (one row) or the skinny matrix-core GEMM
-    (2..16 rows), 9 to 1,100 the tiled and
-    sliced one where it is the faster, unless a gradient is wanted."""
+    """``F.linear(x, w, b)``; unless a gradient is wanted, bf16 inputs run the HIP GEMV (one row), the skinny matrix-core GEMM
+    (2..16 rows) or, of 9 to 1,100 rows, the tiled and sliced one where it is the faster."""
     if x.dim() >= 1 and x.is_cuda:
         n, K = x.numel(), x.shape[-1]
         if n > MAX_ROWS * K:
-            # (hds_linear_plan takes none beyond; what asking costs, 1 us, is 3 % of the host's time for a prompt of that length)
+            # (hds_linear_plan takes none beyond; asking costs 1 us, 3 % of the host's time for a prompt of that length)
             y = rows_linear(x, w, b) if n <= 320 * K or K >= 8192 else None
             if y is not None:
                 return y

@@ -1,5 +1,6 @@
 """Serving steps with more than single tokens: portions of prompts on the FlashAttention kernels over block tables
-(csrc/kernels/flash_attn_pair.hip, flash_attn_w64.hip) or in row blocks, single tokens on the split-key kernel (both csrc/kernels/paged_attn.hip)."""
+(csrc/kernels/flash_attn_pair.hip, flash_attn_w64.hip) or in row blocks, single tokens on the split-key kernel (both
+csrc/kernels/paged_attn.hip)."""
 import torch
 
 from . import native
@@ -135,8 +136,9 @@ def portions_ok(q, cache, n_q, n_kv, scale=1.0):
 def paged_attention_portions(q, cache, toks, blocks, batch, n_q, n_kv, scale, window=0, atoms=None, rows=0):
     """``paged_attention`` of a step that mixes single tokens and portions of prompts: ``toks`` (int32 rows of q) on the
     split-key kernel, which spreads a token's context over the chip, ``blocks`` ([n, 2] int32) on the prefill kernel by ``rows``
-    (``prefill_rows``; 0: by the length of the list), ``atoms`` ([n, 3] int32) in row blocks. There a single token walks its whole context in one workgroup (9 such tokens,
-    up to 3,000 keys, 8 key heads, beside 512 new ones: 171 us; apart 29 + 38 us)."""
+    (``prefill_rows``; 0: by the length of the list), ``atoms`` ([n, 3] int32) in row blocks. There a single token walks its
+    whole context in one workgroup (9 such tokens, up to 3,000 keys, 8 key heads, beside 512 new ones: 171 us; apart 29 + 38
+    us)."""
     T, _, D = q.shape
     o = torch.empty(T, n_q, D, device=q.device, dtype=q.dtype)
     lib, st, tab = native.kernels(), native.stream(), batch.block_tables

@@ -211,8 +211,9 @@ def _packed_rows(x2, q_weight, scales, out_features, in_features, group_size, fm
         return None
     # (what the dequantized weight's view and the library's product refuse is theirs to refuse)
     rows = 2 * N if glu else N
-    if scales.numel() * group_size != rows * K or q_weight.device != x2.device or scales.device != x2.device or (bias is not None and (
-            bias.dtype != torch.bfloat16 or bias.shape != (rows, ) or bias.device != x2.device)):
+    if scales.numel() * group_size != rows * K or q_weight.device != x2.device or scales.device != x2.device:
+        return None
+    if bias is not None and (bias.dtype != torch.bfloat16 or bias.shape != (rows, ) or bias.device != x2.device):
         return None
     x2 = x2.contiguous()
     if (x2.data_ptr() | q_weight.data_ptr()) % 16:
@@ -278,10 +279,10 @@ def int_linear(x, q_weight, scales, out_features, in_features, group_size, bits=
     """y = x @ dequant(W)^T for a symmetric group-quantized int8/int4 weight [out, in] (groups along ``in``).
 
     Up to 16 rows stream the packed weight through the matrix cores (``_wmix_skinny``, groups of a multiple of 128; one row
-    of int8, one and two rows where ``_gemv_wins``, other groups and a bias that is not bf16 up to 2 rows, ``HDS_INT_GEMV_MAX_M``: the HIP GEMV of
-    csrc/kernels/quant.hip); batches of up to 256 rows, of small weights 512, run tiles on packed weights (``_packed_rows``; groups
-    of a multiple of 32 only, up to 64 rows, ``wmix_gemm``), larger ones and groups that do not divide a row dequantize once to
-    bf16."""
+    of int8, one and two rows where ``_gemv_wins``, other groups and a bias that is not bf16 up to 2 rows, ``HDS_INT_GEMV_MAX_M``:
+    the HIP GEMV of csrc/kernels/quant.hip); batches of up to 256 rows, of small weights 512, and some of 4 to 16 run tiles on packed
+    weights (``_packed_rows``; groups of a multiple of 32 only, up to 64 rows, ``wmix_gemm``), larger ones and groups that do not
+    divide a row dequantize once to bf16."""
     lead = x.shape[:-1]
     x2 = x.reshape(-1, in_features)
     M = x2.shape[0]
@@ -529,10 +530,10 @@ def dequantize_minifloat(q, scales, group_size=512, q_bits=6, mantissa_bits=2, d
 def fp6_linear(x, q_weight, scales, out_features, in_features, group_size, mantissa_bits=2):
     """y = x @ dequant(W)^T for an FP6-packed weight [out, in] (row-major, groups along ``in``).
 
-    Up to 32 rows stream the packed weight through the matrix cores (``_wmix_skinny``, groups of a multiple of 128; other
-    groups up to 8 rows and one row where ``_gemv_wins``: the HIP GEMV of csrc/kernels/fpq.hip); batches of up to 256 rows, of small
-    weights 512, run tiles on packed weights (``_packed_rows``; groups of a multiple of 32 only, up to 64 rows, ``wmix_gemm``), larger
-    ones dequantize once to bf16 and use hipBLASLt."""
+    Up to 16 rows, of weights under 2^23 values 32, stream the packed weight through the matrix cores (``_wmix_skinny``, groups
+    of a multiple of 128; other groups up to 8 rows and one row where ``_gemv_wins``: the HIP GEMV of csrc/kernels/fpq.hip); batches
+    of up to 256 rows, of small weights 512, and some of 9 to 16 run tiles on packed weights (``_packed_rows``; groups of a multiple
+    of 32 only, up to 64 rows, ``wmix_gemm``), larger ones dequantize once to bf16 and use hipBLASLt."""
     lead = x.shape[:-1]
     x2 = x.reshape(-1, in_features)
     M = x2.shape[0]
