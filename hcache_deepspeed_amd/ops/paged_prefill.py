@@ -53,7 +53,7 @@ def prefill_rows(seqs, heads):
     in whole rounds, twice as many rounds of 128 take as long and longer (8 sequences of 200 tokens behind 60, 32 / 8 heads
     23.0 us by 128 rows, 20.8 by 256; 16 43.2 and 38.8), unless lengths differ (8 behind up to 1,500 44 and 61) or the second
     halves are empty (16 of 64 behind 500 30 and 44). Over 1,736 lists of 130 to 512 workgroups 0.77 of the time of 256 rows, at
-    most 1.07; with 128 rows for all of them 0.78 and 1.27."""
+    most 1.07; with 128 rows for all of them 0.78 and 1.27 (profiles/main_paths/prefill_rows.txt)."""
     blocks = heads * sum(-(-n // PREFILL_ROWS) for n, _ in seqs)
     if blocks > SHORT_LIST:
         return 256
