@@ -42,7 +42,11 @@ _WALK_US = {128: (7.5, 0.0145), 256: (8.5, 0.033)}
 def _launch_us(seqs, heads, rows):
     """The longest workgroup, all of them over the CUs, or the rounds of 256 that workgroups of much the same length take."""
     us, per_key = _WALK_US[rows]
-    last = sorted((seen + min(r + rows, n) for n, seen in seqs for r in range(0, n, rows)), reverse=True)
+    last = []  # the workgroups' last keys
+    for n, seen in seqs:
+        last.append(seen + n)
+        last += range(seen + (n - 1) // rows * rows, seen, -rows)
+    last.sort(reverse=True)
     rounds = max((k + 1) * (us + per_key * last[256 * k // heads]) for k in range((heads * len(last) - 1) // 256 + 1))
     return max(rounds, heads / 256 * (us * len(last) + per_key * sum(last)))
 
