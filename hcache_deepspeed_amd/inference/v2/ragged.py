@@ -359,7 +359,7 @@ class RaggedBatchWrapper:
         the device tensors are views of it. ``id_limit``: token ids outside [0, id_limit) raise IndexError, before
         anything is sent (a lookup on the device cannot refuse them)."""
         from ...ops import native
-        from ...ops.paged_prefill import divide_step, prefill_rows
+        from ...ops.paged_prefill import SHORT_LIST, divide_step, prefill_rows
         seqs, meta = self._seqs, self.seq_meta_host
         S, T, mb = len(seqs), self.current_tokens, self.max_blocks
         geom = self.__dict__.get("_geom")
@@ -370,7 +370,9 @@ class RaggedBatchWrapper:
         max_new = max((m[1] for m in meta), default=0)
         mixed = getattr(self, "_portions", True) and any(m[1] != 1 for m in meta)
         toks, blocks, rows = divide_step(meta, n_q, n_kv) if mixed else ([], [], [])
-        self.prefill_rows = prefill_rows([meta[s][1:] for s in dict.fromkeys(blocks[::2])], n_q) if blocks and geom else 0
+        # (0: the length of the list says it; 2 us less of the host)
+        ask = 256 < n_q * len(blocks) <= 2 * SHORT_LIST and geom
+        self.prefill_rows = prefill_rows([meta[s][1:] for s in dict.fromkeys(blocks[::2])], n_q) if ask else 0
         self.slots_host = [seq.tracking_id for seq in seqs]
         extra = array("i", self.slots_host + (self._logit_rows or []) + blocks + toks + rows)
         desc = array("q")

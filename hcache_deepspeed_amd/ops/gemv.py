@@ -91,18 +91,18 @@ def _plan(M, N, K, glu=0):
     return int(native.kernels().hds_linear_plan(M, N, K, glu)) if max(M, N, K) < 1 << 31 else 0
 
 
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+
+
 def _watched():
-    """Does a mode see or replace operations (a trace by make_fx, a counter, fake tensors; a default device does neither)?
-    Behind a bare kernel it would find the allocation of the result only."""
-    n = torch._C._len_torch_function_stack()
-    return torch._C._len_torch_dispatch_stack() > 0 or \
-        (n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n)))
+    """Does a function mode see or replace operations (a default device does neither)?"""
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(_function_modes()))
 
 
 def rows_linear(x, w, b=None, glu=0):
     """``F.linear(x, w, b)`` of 9 rows and more, or with ``glu`` = 1 + activation code the gated unit of w = [gate; up]; None
-    where the kernel does not take the call, as where anything could want a record of it (``native.plain``, ``_watched``,
-    torch.compile)."""
+    where the kernel does not take the call, as where anything could want a record of it (``native.plain``, torch.compile, a
+    dispatch or function mode: a trace by make_fx, a counter, fake tensors would find the allocation of the result only)."""
     if torch.compiler.is_compiling():
         return None
     # (sizes first: a call of a prompt that stays the library's pays 2 us less for having asked)
@@ -119,8 +119,10 @@ def rows_linear(x, w, b=None, glu=0):
     # stream the launch would take)
     if plan == 0 or torch.is_autocast_enabled() or x.get_device() != torch.cuda.current_device():
         return None
-    if not native.plain(x, w, b) or _watched() or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.dim() != 2 or \
-            not w.is_contiguous() or K != w.shape[1] or w.get_device() != x.get_device():
+    if not native.plain(x, w, b) or _dispatch_modes() or (_function_modes() and _watched()):
+        return None
+    if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or w.dim() != 2 or not w.is_contiguous() or K != w.shape[1] or \
+            w.get_device() != x.get_device():
         return None
     x2 = x if x.dim() == 2 else x.reshape(M, K)
     ld, one = x2.stride()

@@ -28,17 +28,21 @@ def test_estimates_are_of_the_kernel_that_runs():
 
 
 def test_a_step_carries_its_rows(monkeypatch):
-    """The batch hands the choice of its portions on to the kernel; steps of single tokens make none."""
+    """The batch hands the choice of its portions on to the kernel where there is one: not of single tokens, nor of lists whose
+    length says it."""
     from hcache_deepspeed_amd.inference.v2 import build_engine_from_model
     from hcache_deepspeed_amd.models.llama import LlamaForCausalLM, tiny
     eng = build_engine_from_model(LlamaForCausalLM(tiny()).eval(), {"dtype": "fp32"}, device=torch.device("cpu"), num_kv_blocks=8)
     asked = []
     monkeypatch.setattr(P, "prefill_rows", lambda seqs, heads: asked.append(([tuple(s) for s in seqs], heads)) or 256)
-    eng._batch.set_attention_geometry(4, 2, 128)
-    eng.put([1, 2], [torch.arange(20) % 7, torch.arange(3)], capture_latents=False)
-    assert asked == [([(20, 0)], 4)] and eng._batch.prefill_rows == 256
+    for heads, rows in ((128, 0), (130, 256), (256, 256)):
+        eng._batch.set_attention_geometry(heads, 2, 128)
+        eng.put([1, 2], [torch.arange(20) % 7, torch.arange(3)], capture_latents=False)
+        assert eng._batch.prefill_rows == rows
+        eng.flush(1), eng.flush(2)
+    assert asked == [([(20, 0)], 130), ([(20, 0)], 256)]
     eng.put([1], [torch.arange(1)], capture_latents=False)
-    assert len(asked) == 1 and eng._batch.prefill_rows == 0
+    assert eng._batch.prefill_rows == 0
 
 
 def test_rows_reach_the_kernel(monkeypatch):
