@@ -16,11 +16,13 @@
 //   * pair-bias gradient: the sum of dS over the N rows stays in registers. A wave owns 32 queries x 64 keys of one
 //     (b, h) and walks over a chunk of the rows, recomputing the two products that dS needs; chunks are added by a second
 //     kernel that also rounds. No atomics, the same result every time.
-// Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): a forward and backward 146 us (with dQ and dK / dV
-// apart and the pair gradient's rows loaded by wave 199); in a kernel trace, where launches do not overlap, forward 43 us, dQ +
-// dK + dV 67 (apart 52 + 51), pair gradient 43 + 4 (rows by wave 56 + 4)
+// Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): a forward and backward 136 us (with a forward workgroup a
+// row and the pair bias through the matrix cores in every row 147; with dQ and dK / dV apart and the pair gradient's rows
+// loaded by wave 199); in a kernel trace, where launches do not overlap, forward 34 us (a workgroup a row 42), dQ + dK + dV 67
+// (apart 52 + 51), pair gradient 32 + 4 (bias through the matrix cores 43 + 4, rows by wave 56 + 4)
 // (before: one wave a workgroup with operands from global memory and 2-byte reads of V 169 us; the FlashAttention
 // backward kernels with 32-bit atomics into the pair gradient 271 + 1,585 us).
+#include <algorithm>
 #include <cmath>
 
 #include "attn_common.h"
@@ -79,6 +81,61 @@ struct Tile {
     const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(a0));
     const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(a1));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+  // the same for both steps of a tile of 32 columns at `lds`, here when it returns
+  static __device__ __forceinline__ void cols_now(const char* lds, bf16x8 (&f)[2]) {
+    static_assert(D == 32, "rows of 64 bytes: 16 further ones have the same swizzle");
+    const int lane = threadIdx.x & 63;
+    const int g = lane >> 4, i = lane & 15, q = i >> 2, p = i & 3;
+    const int row = 4 * (g >> 1) + q, ch = 2 * (g & 1) + (p >> 1);
+    const uint32_t a0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)(lds + off(row, ch) + 8 * (p & 1));
+    const uint32_t a1 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)(lds + off(row + 8, ch) + 8 * (p & 1));
+    u32x2 r[4];
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %4\n\tds_read_b64_tr_b16 %1, %5\n\tds_read_b64_tr_b16 %2, %4 offset:1024\n\t"
+        "ds_read_b64_tr_b16 %3, %5 offset:1024\n\ts_waitcnt lgkmcnt(0)"
+        : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
+        : "v"(a0), "v"(a1)
+        : "memory");
+#pragma unroll
+    for (int st = 0; st < 2; ++st)
+      f[st] = __builtin_bit_cast(bf16x8, u32x4{r[2 * st][0], r[2 * st][1], r[2 * st + 1][0], r[2 * st + 1][1]});
+  }
+};
+
+// Tile::stage for a kernel that walks over rows n: nt tiles from position row0 on, at distances from the start of a row n that
+// are made once. Positions past the end are read as zeros.
+template <int D>
+struct Stager {
+  using T = Tile<D>;
+  static constexpr int PER = 1024 / T::RB;
+  uint32_t first, even, odd;  // of a lane: of the wave's first instruction; without its number, by the parity of the wave instruction's number: a tile's swizzle looks as far
+  int w, count, step;
+  uint32_t bytes, stride;
+  __device__ __forceinline__ Stager(int row0, int nt, int nw, int64_t ld, int L) {
+    const int lane = threadIdx.x & 63, row = lane / T::CH;
+    w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    count = nt * 32 / PER;
+    step = nw;
+    stride = PER * 2 * (uint32_t)ld;
+    bytes = (uint32_t)(L - 1) * 2 * (uint32_t)ld + 2 * D;
+    even = 2 * (uint32_t)ld * (row0 + row) + 16 * ((lane % T::CH) ^ T::mix(row));
+    odd = 2 * (uint32_t)ld * (row0 + row) + 16 * ((lane % T::CH) ^ T::mix(PER + row));
+    first = (w & 1 ? odd : even) + w * stride;
+  }
+  // (one: of whole workgroups that move 1 KB a wave)
+  __device__ __forceinline__ void stage(char* lds, const bf16* m, bool one) const {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)m, (short)0, bytes, 0x00020000);
+    const uint32_t at[2] = {even, odd};
+    if (one) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(lds + w * 1024), 16, first, 0, 0, 0);
+      return;
+    }
+    for (int i = w; i < count; i += step) {
+      uint32_t voff = at[0];
+      if (i & 1) voff = at[1];
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(lds + i * 1024), 16, voff, i * stride, 0, 0);
+    }
   }
 };
 
@@ -224,18 +281,19 @@ struct QueryBias<D, bf16> {
   __device__ __forceinline__ f32x16 start(int k0, int L) const {
     return start<TAIL>(mask<TAIL>(k0, L), k0, L);
   }
+  __device__ __forceinline__ void watch(const u32x4 (&f)[2]) {
+    typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      seen = __builtin_bit_cast(u32x4, __builtin_elementwise_max(__builtin_bit_cast(u16x8, seen),
+                                                                 __builtin_bit_cast(u16x8, f[ks])));
+  }
   template <bool TAIL, bool WATCH = false>
   __device__ __forceinline__ f32x16 add(int k0, int hf, int L, f32x16 s) {
     if (b2 != nullptr) {
       u32x4 f[2];
       load_pair<TAIL>(k0, L, f);
-      if constexpr (WATCH) {
-        typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-          seen = __builtin_bit_cast(u32x4, __builtin_elementwise_max(__builtin_bit_cast(u16x8, seen),
-                                                                     __builtin_bit_cast(u16x8, f[ks])));
-      }
+      if constexpr (WATCH) watch(f);
       f[0] = finite(f[0]);
       f[1] = finite(f[1]);
       s = add_pair(f, s);
@@ -301,6 +359,11 @@ struct QueryBias<D, float> {
   __device__ __forceinline__ bool nan() const { return false; }
 };
 
+// Exponents of base 2 are s c - ref with one rounding, where ref, the row's maximum or normaliser times c, is not far from
+// zero: its own rounding is a factor that the whole row shares. Far off (rows whose keys all have a mask of -1e9 or below)
+// that factor could be anything, and the difference is taken first.
+__device__ __forceinline__ bool far_off(float ref) { return fabsf(ref) > 256.f && fabsf(ref) < INFINITY; }
+
 struct EvoParams {
   const bf16 *q, *k, *v, *o, *dout;
   const void *b1, *b2;  // [B N, L], [B, H, L, L], or null
@@ -344,6 +407,11 @@ __device__ __forceinline__ void load_frags(const bf16* m, int64_t ld, int row, b
   for (int ks = 0; ks < D / 16; ++ks) f[ks] = *reinterpret_cast<const bf16x8*>(r + 16 * ks);
 }
 template <int D>
+__device__ __forceinline__ void times(bf16x8& f, float power) {
+#pragma unroll
+  for (int e = 0; e < 8; ++e) f[e] = (bf16)((float)f[e] * power);
+}
+template <int D>
 __device__ __forceinline__ void times(bf16x8 (&f)[D / 16], float power) {
 #pragma unroll
   for (int ks = 0; ks < D / 16; ++ks)
@@ -354,6 +422,40 @@ __device__ __forceinline__ void times(bf16x8 (&f)[D / 16], float power) {
 // ---------------------------------------------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------------------------------------------
+// one tile of 32 keys of a wave's 32 queries: m is the largest raw score, l this lane's sum of exponentials
+template <int D, bool TAIL, typename Bias>
+__device__ __forceinline__ void evo_tile(Bias& bias, const char* sk, const char* sv, int t0, int k0, int hf, int L, float c,
+                                       const bf16x8 (&qf)[D / 16], f32x16 (&acc)[D / 32], float& m, float& l) {
+  using T = Tile<D>;
+  f32x16 s = bias.template start<TAIL>(k0, L);
+#pragma unroll
+  for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(sk, t0, ks), qf[ks], s);
+  s = bias.template add<TAIL, true>(k0, hf, L, s);
+  float top = s[0];
+#pragma unroll
+  for (int r = 1; r < 15; r += 2) top = fmaxf(fmaxf(top, s[r]), s[r + 1]);
+  top = fmaxf(top, s[15]);
+  top = fmaxf(top, __shfl_xor(top, 32, 64));
+  const float mn = fmaxf(m, top);
+  const float alpha = m == -INFINITY ? 0.f : fast_exp2((m - mn) * c);
+  const float ref = mn == -INFINITY ? 0.f : mn;  // no visible key so far: probabilities of zero, not NaN
+  m = mn;
+  float sum = 0.f;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    s[r] = fast_exp2((s[r] - ref) * c);  // (not s c - mn c: a row whose keys all have a mask of -1e9 or below)
+    sum += s[r];
+  }
+  l = l * alpha + sum;  // of this lane's keys; both halves are added at the end
+  const bf16x8 pb[2] = {acc_to_b<0>(s), acc_to_b<1>(s)};
+#pragma unroll
+  for (int dt = 0; dt < T::DT; ++dt) {
+    acc[dt] *= alpha;
+#pragma unroll
+    for (int st = 0; st < 2; ++st) acc[dt] = mfma(T::cols(sv, t0, st, dt), pb[st], acc[dt]);
+  }
+}
+
 template <int D, typename TB>
 __global__ __launch_bounds__(64 * kWaves<D>) void evo_fwd_kernel(EvoParams p, int blocks) {
   using T = Tile<D>;
@@ -375,34 +477,7 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_fwd_kernel(EvoParams p, in
                         p.b2 != nullptr ? (const TB*)p.b2 + ((int64_t)(a.b * p.H + a.h) * L + qc) * L : nullptr, p.rest);
 
   auto tile = [&](const char* sk, const char* sv, int t0, int k0, auto tail) {
-    constexpr bool TAIL = decltype(tail)::value;
-    f32x16 s = bias.template start<TAIL>(k0, L);
-#pragma unroll
-    for (int ks = 0; ks < T::KS; ++ks) s = mfma(T::rows(sk, t0, ks), qf[ks], s);
-    s = bias.template add<TAIL, true>(k0, hf, L, s);
-    float top = s[0];
-#pragma unroll
-    for (int r = 1; r < 15; r += 2) top = fmaxf(fmaxf(top, s[r]), s[r + 1]);
-    top = fmaxf(top, s[15]);
-    top = fmaxf(top, __shfl_xor(top, 32, 64));
-    const float mn = fmaxf(m, top);
-    const float alpha = m == -INFINITY ? 0.f : fast_exp2((m - mn) * c);
-    const float ref = mn == -INFINITY ? 0.f : mn;  // no visible key so far: probabilities of zero, not NaN
-    m = mn;
-    float sum = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] = fast_exp2((s[r] - ref) * c);  // (not s c - mn c: a row whose keys all have a mask of -1e9 or below)
-      sum += s[r];
-    }
-    l = l * alpha + sum;  // of this lane's keys; both halves are added at the end
-    const bf16x8 pb[2] = {acc_to_b<0>(s), acc_to_b<1>(s)};
-#pragma unroll
-    for (int dt = 0; dt < T::DT; ++dt) {
-      acc[dt] *= alpha;
-#pragma unroll
-      for (int st = 0; st < 2; ++st) acc[dt] = mfma(T::cols(sv, t0, st, dt), pb[st], acc[dt]);
-    }
+    evo_tile<D, decltype(tail)::value>(bias, sk, sv, t0, k0, hf, L, c, qf, acc, m, l);
   };
 
   for (int c0 = 0; c0 < L; c0 += T::ROWS) {
@@ -428,6 +503,199 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_fwd_kernel(EvoParams p, in
     for (int dt = 0; dt < T::DT; ++dt) store_row_block<D>(row, acc[dt], dt, hf, inv);
     // (no visible key: infinity, so that the backward's probabilities are zero)
     if (hf == 0) p.lse[((int64_t)a.bn * p.H + a.h) * L + myq] = l == 0.f ? INFINITY : (m * c + log2f(l)) / kLog2e;
+  }
+}
+
+// The same for heads of 32, rows of up to 256 positions and bf16 biases. In the kernel above all workgroups of a launch are on
+// the chip at once and wait for their operands together, then compute together; here a workgroup walks over rows n of one head,
+// and a row's operands are on their way while the one before is computed. The pair bias is the same for all of them: each wave
+// keeps its 32 queries' as what the scores start from, in 32 bits (128 registers), instead of multiplying it in again. Scores
+// are q . k + bias / scale, a running maximum is raised only where a score exceeds it by 2^8, and exponents take one fused
+// operation (see far_off): 90 instructions a tile of 32 x 32, which is what bounds two waves a SIMD (about five cycles each,
+// whatever they are). Rows that this does not hold for are computed again as above.
+template <int NT>
+struct RowRing {
+  static constexpr int M = 32 * NT * 64, kMask = 256 * ((NT + 1) / 2);  // bytes of K or V, of the mask (4 a key)
+  static constexpr int kRow = 2 * M + kMask;
+};
+
+template <int NT>
+__global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, int rows_per) {
+  constexpr int D = 32;
+  using T = Tile<D>;
+  using W = RowRing<NT>;
+  __shared__ __attribute__((aligned(1024))) char smem[2 * W::kRow];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nt = blockDim.x >> 6;
+  const int hf = lane >> 5, j = lane & 31, L = p.L;
+  int id = xcd_id();
+  const int h = id % p.H;
+  id /= p.H;
+  const int chunks = (p.N + rows_per - 1) / rows_per, b = id / chunks;
+  const int n0 = (id % chunks) * rows_per, n1 = min(p.N, n0 + rows_per);
+  const int myq = 32 * w + j, qc = min(myq, L - 1);
+  const uint32_t ld = p.H * D;
+  const float c = p.rest * kLog2e, mul = p.scale * kLog2e, step = 8.f / mul;
+  // (made anew where it is asked for: its 30 registers shall not stay through the loop)
+  auto biases = [&](int n) {
+    int q = qc;
+    float rest = p.rest;
+    asm volatile("" : "+v"(q), "+v"(rest));
+    return QueryBias<D, bf16>(p.b1 != nullptr ? (const bf16*)p.b1 + ((int64_t)b * p.N + n) * L : nullptr,
+                              p.b2 != nullptr ? (const bf16*)p.b2 + ((int64_t)(b * p.H + h) * L + q) * L : nullptr, rest);
+  };
+
+  Stager<D> of_k(0, nt, nt, ld, L);
+  const uint32_t mask_at = 2 * threadIdx.x, q_at = 2 * (qc * ld + 8 * hf);
+  bf16x8 qn[2];
+  auto load = [&](int n) {
+    const int64_t bn = (int64_t)b * p.N + n, base = bn * L * ld + (int64_t)h * D;
+    char* s = smem + (n & 1) * W::kRow;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) qn[ks] = *reinterpret_cast<const bf16x8*>((const char*)(p.q + base) + (q_at + 32 * ks));
+    of_k.stage(s, p.k + base, false);
+    of_k.stage(s + W::M, p.v + base, false);
+    if (p.b1 != nullptr && w < (nt + 1) / 2)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          __builtin_amdgcn_make_buffer_rsrc((void*)((const bf16*)p.b1 + bn * L), (short)0, 2 * L, 0x00020000),
+          (lds_void*)(s + 2 * W::M + 256 * w), 2, mask_at, 0, 0, 0);
+  };
+  load(n0);
+
+  f32x16 start[NT];
+  bf16x8 inv = pieces<D>(Inverse<D>(p.rest));
+  times<16>(inv, 1.f / p.power);
+  QueryBias<D, bf16> bias = biases(n0);
+  u32x4 pair[NT][2] = {};  // (all on their way at once)
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+    if (t < nt && p.b2 != nullptr) {
+      if (32 * t + 32 <= L) bias.template load_pair<false>(32 * t, L, pair[t]);
+      else bias.template load_pair<true>(32 * t, L, pair[t]);
+    }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    start[t] = f32x16{};
+    if (t < nt) {
+      if (p.b2 != nullptr) {
+        bias.watch(pair[t]);
+        pair[t][0] = finite(pair[t][0]);
+        pair[t][1] = finite(pair[t][1]);
+        start[t] = bias.add_pair(pair[t], start[t]) * (1.f / p.power);
+      }
+      if (32 * t + 32 > L) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (32 * t + acc_row(r, hf) >= L) start[t][r] = -INFINITY;
+      }
+    }
+  }
+  const bool nan = bias.nan();
+
+  auto store = [&](int n, const f32x16& acc, float top, float l) {
+    if (nan) l = __builtin_nanf("");
+    l += __shfl_xor(l, 32, 64);  // both halves' keys
+    const int64_t bn = (int64_t)b * p.N + n;
+    if (myq < L) {
+      store_row_block<D>(p.out + bn * L * ld + (int64_t)h * D + myq * ld, acc, 0, hf, l == 0.f ? 0.f : 1.f / l);
+      if (hf == 0) p.lse[(bn * p.H + h) * L + myq] = l == 0.f ? INFINITY : (top + log2f(l)) / kLog2e;
+    }
+  };
+
+  auto arrived = [&] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : "+v"(qn[0]), "+v"(qn[1])::"memory"); };
+  arrived();
+  uint64_t again = 0;  // rows to be computed again
+#pragma unroll 1
+  for (int n = n0; n < n1; ++n) {
+    const char* sk = smem + (n & 1) * W::kRow;
+    const char* sv = sk + W::M;
+    __builtin_amdgcn_s_barrier();
+    bf16x8 qf[2] = {qn[0], qn[1]};
+    if (n + 1 < n1) load(n + 1);
+
+    float m = -INFINITY, l = 0.f, ref = 0.f;
+    f32x16 acc[1] = {};
+    // C tiles at a time: their products, and what follows of each, lie in the other's shadow
+    auto tiles = [&](auto count, int t0) {
+      constexpr int C = decltype(count)::value;
+      f32x16 x[C];
+      bf16x8 vt[C][2];
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        const bf16 v = p.b1 != nullptr ? *reinterpret_cast<const bf16*>(sv + W::M + 4 * (32 * (t0 + i) + j)) : (bf16)0.f;
+        x[i] = mfma(spread<D>(v), inv, start[t0 + i]);
+      }
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int i = 0; i < C; ++i) x[i] = mfma(T::rows(sk, 32 * (t0 + i), ks), qf[ks], x[i]);
+      // V^T beside the products. (The compiler lets such a read of its own wait for the next row's operands too.)
+#pragma unroll
+      for (int i = 0; i < C; ++i) T::cols_now(sv + 32 * (t0 + i) * T::RB, vt[i]);
+      float top = x[0][0];
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+#pragma unroll
+        for (int r = 1 - (i > 0); r < 15 - (i > 0); r += 2) top = fmaxf(fmaxf(top, x[i][r]), x[i][r + 1]);
+        if (i == 0) top = fmaxf(top, x[0][15]);
+        else top = fmaxf(fmaxf(top, x[i][14]), x[i][15]);
+      }
+      if (__any(top > m + step)) {
+        const auto o = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, top), __builtin_bit_cast(uint32_t, top), false, false);
+        top = fmaxf(__builtin_bit_cast(float, (uint32_t)o[0]), __builtin_bit_cast(float, (uint32_t)o[1]));
+        if (top > m + step) {
+          const float alpha = fast_exp2((m - top) * mul);
+          m = top;
+          ref = m * mul;
+          l *= alpha;
+          acc[0] *= alpha;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < C; ++i) {
+        float sum[2] = {};
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          x[i][r] = fast_exp2(__builtin_fmaf(x[i][r], mul, -ref));
+          sum[r & 1] += x[i][r];
+        }
+        l += sum[0] + sum[1];
+        const bf16x8 pb[2] = {acc_to_b<0>(x[i]), acc_to_b<1>(x[i])};
+#pragma unroll
+        for (int st = 0; st < 2; ++st) acc[0] = mfma(vt[i][st], pb[st], acc[0]);
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < NT; t += 2) {
+      if (t >= nt) break;
+      if (t + 1 < NT && t + 1 < nt) tiles(std::integral_constant<int, (NT > 1 ? 2 : 1)>{}, t);
+      else tiles(std::integral_constant<int, 1>{}, t);
+    }
+    if (!__all(fabsf(ref) <= 256.f && m > -INFINITY)) again |= 1ull << (n - n0);
+    arrived();  // the next row's; what is stored here is on its way while that one is computed
+    store(n, acc[0], ref, l);
+  }
+
+  // rows that want the finite biases as they are
+  __shared__ uint64_t s_again[NT];
+  if (lane == 0) s_again[w] = again;
+  __syncthreads();
+  uint64_t all = 0;
+  for (int i = 0; i < nt; ++i) all |= s_again[i];
+  for (int n = n0; n < n1; ++n) {
+    if (!(all >> (n - n0) & 1)) continue;  // (the same for all waves)
+    __syncthreads();
+    load(n);
+    arrived();
+    __builtin_amdgcn_s_barrier();
+    if (!(again >> (n - n0) & 1)) continue;
+    const char* sk = smem + (n & 1) * W::kRow;
+    bf16x8 qf[2] = {qn[0], qn[1]};
+    times<D>(qf, p.power);
+    float m = -INFINITY, l = 0.f;
+    f32x16 acc[1] = {};
+    QueryBias<D, bf16> rows = biases(n);
+    for (int t = 0; t < nt; ++t) evo_tile<D, true>(rows, sk, sk + W::M, 32 * t, 32 * t, hf, L, c, qf, acc, m, l);
+    store(n, acc[0], m * c, l);
   }
 }
 
@@ -689,9 +957,13 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_bwd_kernel(EvoParams p, int ro
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
           const int k = k0 + 16 * ks + 8 * hf;
-          pair[t][ks] = finite(full ? load_eight<false>(row, k, L) : load_eight<true>(row, k, L));
+          pair[t][ks] = full ? load_eight<false>(row, k, L) : load_eight<true>(row, k, L);
         }
       }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)  // (behind all loads)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) pair[t][ks] = finite(pair[t][ks]);
   }
 
   u32x4 rq[W::PER], rd[W::PER], ro[W::PER], rk[W::PER];
@@ -847,7 +1119,8 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_bwd_kernel(EvoParams p, int ro
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int kPairTiles = 2;  // of 32 keys: a wave's 32 sums and 32 biases a lane leave room for four waves a SIMD
 
-__device__ __forceinline__ void store_pair_sums(float* out, const f32x16 (&sum)[kPairTiles], int k0, int hf, int L) {
+template <typename Sums>
+__device__ __forceinline__ void store_pair_sums(float* out, const Sums& sum, int k0, int hf, int L) {
 #pragma unroll
   for (int t = 0; t < kPairTiles; ++t)
 #pragma unroll
@@ -930,18 +1203,27 @@ __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblo
   store_pair_sums(p.part + (((int64_t)chunk * p.B + b) * p.H + h) * L * L + (int64_t)myq * L, sum, kk0, hf, L);
 }
 
-// The same for narrower heads, whose operands of two rows fit in LDS (64 or 128 KB; D = 128 would want 256), where
-// hds_evoformer_pair_staged says so: a workgroup of
-// up to 4 x 2 waves stages the queries and the keys that its waves share, a row ahead. In the kernel above each wave
-// loads its own, between them almost three times the bytes, in pieces of 16 bytes a row, and waits for them. 128 rows of
-// 256, 8 heads, D = 32: 58 -> 42 us; a training pass with D = 64 296 -> 251 us. The exponents and what is around them,
-// some 8 vector instructions a score, bound it now.
+// The same for narrower heads, whose operands of two rows fit in LDS (32 or 64 KB a row; D = 128 would want 128), where
+// hds_evoformer_pair_staged says so: a workgroup of up to 4 x 2 waves stages the queries and the keys that its waves share, a
+// row ahead (three rows ahead is level). In the kernel above each wave loads its own, between them almost three times the bytes, in pieces of 16
+// bytes a row, and waits for them: 128 rows of 256, 8 heads, D = 32 58 -> 42 us; a training pass with D = 64 296 -> 251 us.
+// What bounds it is how many instructions a wave has, about five cycles each with two waves a SIMD: with the pair bias as what
+// the scores start from (of near rows, see far_off) instead of six products a tile, one operation for the exponent's argument
+// and the distances of a row's loads made once, 170 instead of 380 a row and 42 -> 32 us.
+template <int D>
+struct PairRows {
+  static constexpr int M = 128 * Tile<D>::RB;    // bytes of a matrix: 128 rows
+  static constexpr int kAux = 768;               // of a wave: its queries' lse and delta, its keys' mask, 4 bytes a lane
+  static constexpr int kRow = 4 * M + 8 * kAux;  // Q, dO, K, V of a row n, and the waves' own
+};
+
 template <int D, typename TB>
 __global__ __launch_bounds__(512, 2) void evo_dpair_rows_kernel(EvoParams p, int qblocks, int kblocks, int rows_per,
                                                                 int nwq) {
   using T = Tile<D>;
-  constexpr int M = 128 * T::RB;  // of a matrix: 128 rows
-  extern __shared__ __attribute__((aligned(1024))) char smem[];  // two rows n: Q, dO, K, V
+  using W = PairRows<D>;
+  constexpr int M = W::M;
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6, nwk = nw / nwq;
   const int hf = lane >> 5, j = lane & 31, L = p.L, wq = w % nwq, wk = w / nwq;
   int id = xcd_id();
@@ -959,76 +1241,147 @@ __global__ __launch_bounds__(512, 2) void evo_dpair_rows_kernel(EvoParams p, int
   const float c = p.rest * kLog2e;
   const int64_t ld = (int64_t)p.H * D;
   QueryBias<D, TB> bias(nullptr, (const TB*)p.b2 + ((int64_t)(b * p.H + h) * L + qc) * L, p.rest);
-  f32x16 sum[kPairTiles];
+  float sum[kPairTiles][16];  // (single values: as vectors they are copied where the paths below meet)
 #pragma unroll
-  for (int t = 0; t < kPairTiles; ++t) sum[t] = f32x16{};
+  for (int t = 0; t < kPairTiles; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sum[t][r] = 0.f;
 
-  auto walk = [&](auto tail) {
-    constexpr bool TAIL = decltype(tail)::value;
-    u32x4 pair[kPairTiles][2];
-    if constexpr (sizeof(TB) == 2) {
+  // the pair bias and the rows' normalisers, on their way together
+  u32x4 pair[kPairTiles][2] = {};
+  if constexpr (sizeof(TB) == 2) {
 #pragma unroll
-      for (int t = 0; t < kPairTiles; ++t) {
-        bias.template load_pair<TAIL>(kk0 + 32 * t, L, pair[t]);
-        pair[t][0] = finite(pair[t][0]);
-        pair[t][1] = finite(pair[t][1]);
+    for (int t = 0; t < kPairTiles; ++t) {
+      if (kk0 + 32 * t + 32 <= L) bias.template load_pair<false>(kk0 + 32 * t, L, pair[t]);
+      else bias.template load_pair<true>(kk0 + 32 * t, L, pair[t]);
+    }
+  }
+  bool far = false;
+  for (int n = n0; n < n1; n += 8) {
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = (p.lse + (((int64_t)b * p.N + min(n + i, n1 - 1)) * p.H + h) * L)[(uint32_t)qc];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) far |= far_off(v[i] * kLog2e);
+  }
+  far = __any(far);
+  if constexpr (sizeof(TB) == 2) {
+#pragma unroll
+    for (int t = 0; t < kPairTiles; ++t) {
+      pair[t][0] = finite(pair[t][0]);
+      pair[t][1] = finite(pair[t][1]);
+    }
+  }
+  auto walk = [&](auto tail, auto is_far) {
+    constexpr bool TAIL = decltype(tail)::value, FAR = decltype(is_far)::value;
+    // Near rows: scores are q . k + bias / scale, and a bias that overflows is one whose weight is zero. Far ones as elsewhere
+    constexpr bool kPlain = sizeof(TB) == 2 && !FAR;
+    const float mul = kPlain ? p.scale * kLog2e : c;
+    // (in the forward's order: beside 1e9 each sum rounds by more than what an exponent can take).
+    f32x16 start[kPairTiles];  // the pair bias, which the scores of near rows start from
+    if constexpr (sizeof(TB) == 2) {
+      if constexpr (!FAR) {
+#pragma unroll
+        for (int t = 0; t < kPairTiles; ++t) start[t] = bias.add_pair(pair[t], f32x16{}) * (1.f / p.power);
+        times<16>(bias.inv, 1.f / p.power);
       }
     }
-    float lse_n, delta_n;
-    TB mask_n[kPairTiles];
-    auto mask_row = [&](int n) {
-      if (p.b1 != nullptr) bias.b1 = (const TB*)p.b1 + ((int64_t)b * p.N + n) * L;
-    };
+    // What a lane takes from a row n lies at the same distance from the row's start for every n: the distances are made once
+    Stager<D> of_q(qs, nwq, nw, ld, L), of_k(ks0, kPairTiles * nwk, nw, ld, L);
+    const uint32_t stat_at = 4 * qc, mask_at = 2 * min(kk0 + lane, L - 1);
+    auto rsrc = [&](const void* m, int size) { return __builtin_amdgcn_make_buffer_rsrc((void*)m, (short)0, size * L, 0x00020000); };
+    const bool one = D == 32 && nw == 8 && nwq == 4;
     auto load = [&](int n) {
-      const int64_t bn = (int64_t)b * p.N + n, base = bn * L * ld + (int64_t)h * D, stat = (bn * p.H + h) * L;
-      char* s = smem + (n - n0) % 2 * 4 * M;
-      lse_n = p.lse[stat + qc];
-      delta_n = p.delta[stat + qc];
-      mask_row(n);
-#pragma unroll
-      for (int t = 0; t < kPairTiles; ++t) mask_n[t] = bias.template mask<TAIL>(kk0 + 32 * t, L);
-      T::stage(s, p.q + base, ld, qs, nwq, L, nw);
-      T::stage(s + M, p.dout + base, ld, qs, nwq, L, nw);
-      T::stage(s + 2 * M, p.k + base, ld, ks0, kPairTiles * nwk, L, nw);
-      T::stage(s + 3 * M, p.v + base, ld, ks0, kPairTiles * nwk, L, nw);
+      const int64_t bn = (int64_t)b * p.N + n, base = bn * L * ld + (int64_t)h * D;
+      char* s = smem + (n - n0) % 2 * W::kRow;
+      char* mine = s + 4 * M + w * W::kAux;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(p.lse + (bn * p.H + h) * L, 4), (lds_void*)mine, 4, stat_at, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc(p.delta + (bn * p.H + h) * L, 4), (lds_void*)(mine + 256), 4, stat_at, 0, 0, 0);
+      if (sizeof(TB) == 2 && p.b1 != nullptr)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc((const bf16*)p.b1 + bn * L, 2), (lds_void*)(mine + 512), 2, mask_at, 0, 0, 0);
+      of_q.stage(s, p.q + base, one);
+      of_q.stage(s + M, p.dout + base, one);
+      of_k.stage(s + 2 * M, p.k + base, one);
+      of_k.stage(s + 3 * M, p.v + base, one);
     };
     load(n0);
 #pragma unroll 1
     for (int n = n0; n < n1; ++n) {
-      const char* s = smem + (n - n0) % 2 * 4 * M;
-      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this row has arrived, and every wave is done with the one before
-      __syncthreads();
-      const float lse_raw = lse_n / p.rest, delta = delta_n;
-      TB mask[kPairTiles];
-#pragma unroll
-      for (int t = 0; t < kPairTiles; ++t) mask[t] = mask_n[t];
+      const char* s = smem + (n - n0) % 2 * W::kRow;
+      // this row has arrived, and every wave is done with the one whose place the next one takes
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
       if (n + 1 < n1) load(n + 1);
       if (!live) continue;
-      mask_row(n);
+      const char* mine = s + 4 * M + w * W::kAux;
+      const float lse = *reinterpret_cast<const float*>(mine + 4 * j), delta = *reinterpret_cast<const float*>(mine + 256 + 4 * j);
+      TB mask[kPairTiles];
+#pragma unroll
+      for (int t = 0; t < kPairTiles; ++t) {
+        if constexpr (sizeof(TB) == 2)
+          mask[t] = p.b1 != nullptr ? *reinterpret_cast<const bf16*>(mine + 512 + 128 * t + 4 * j) : (bf16)0.f;
+        else mask[t] = 0.f;
+      }
+      if (p.b1 != nullptr) bias.b1 = (const TB*)p.b1 + ((int64_t)b * p.N + n) * L;
       bf16x8 qf[T::KS], df[T::KS];
 #pragma unroll
       for (int ks = 0; ks < T::KS; ++ks) {
         qf[ks] = T::rows(s, 32 * wq, ks);
         df[ks] = T::rows(s + M, 32 * wq, ks);
       }
-      times<D>(qf, p.power);
+      if constexpr (!kPlain) times<D>(qf, p.power);
+      const float ref = lse * kLog2e, lse_raw = FAR ? lse / p.rest : 0.f;
+      f32x16 less;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) less[r] = -delta;
+      f32x16 x[kPairTiles], d[kPairTiles];
+      auto products = [&](int t) {
+        const int k0 = kk0 + 32 * t, kr = 32 * (kPairTiles * wk + t);
+        d[t] = less;
+        if constexpr (sizeof(TB) == 2) {
+          TB v = mask[t];
+          if (TAIL && k0 + j >= L) v = __builtin_bit_cast(bf16, (uint16_t)kLowest);
+          if constexpr (FAR) x[t] = mfma(spread<D>(v), bias.inv, f32x16{});
+          else x[t] = mfma(spread<D>(v), bias.inv, start[t]);
+        } else {
+          x[t] = f32x16{};
+        }
+#pragma unroll
+        for (int ks = 0; ks < T::KS; ++ks) {
+          x[t] = mfma(T::rows(s + 2 * M, kr, ks), qf[ks], x[t]);
+          d[t] = mfma(T::rows(s + 3 * M, kr, ks), df[ks], d[t]);
+        }
+        if constexpr (sizeof(TB) == 4) x[t] = bias.template add<TAIL>(k0, hf, L, x[t]);
+        else if constexpr (FAR) x[t] = bias.add_pair(pair[t], x[t]);
+      };
+      products(0);
 #pragma unroll
       for (int t = 0; t < kPairTiles; ++t) {
-        const int k0 = kk0 + 32 * t, kr = 32 * (kPairTiles * wk + t);
-        f32x16 x = bias.template start<TAIL>(mask[t], k0, L), d = f32x16{};
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + 1 < kPairTiles) products(t + 1);
 #pragma unroll
-        for (int ks = 0; ks < T::KS; ++ks) x = mfma(T::rows(s + 2 * M, kr, ks), qf[ks], x);
-        if constexpr (sizeof(TB) == 2) x = bias.add_pair(pair[t], x);
-        else x = bias.template add<TAIL>(k0, hf, L, x);
+        for (int r = 0; r < 16; ++r) {
+          const float v = FAR ? (x[t][r] - lse_raw) * c : __builtin_fmaf(x[t][r], mul, -ref);
+          sum[t][r] += fast_exp2(v) * d[t][r];
+        }
+        if (t + 1 < kPairTiles) {  // the products of one tile beside the exponents of the other
 #pragma unroll
-        for (int ks = 0; ks < T::KS; ++ks) d = mfma(T::rows(s + 3 * M, kr, ks), df[ks], d);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sum[t][r] += fast_exp2((x[r] - lse_raw) * c) * (d[r] - delta);
+          for (int i = 0; i < 8; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x400, 2, 0);
+          }
+        }
       }
     }
   };
   // the workgroup's tail is every wave's: they meet at barriers (with 32-bit biases there is none)
-  if (sizeof(TB) == 4 || ks0 + 32 * kPairTiles * nwk <= L) walk(std::false_type{}); else walk(std::true_type{});
+  const bool whole = sizeof(TB) == 4 || ks0 + 32 * kPairTiles * nwk <= L;
+  if (whole && !far) walk(std::false_type{}, std::false_type{});
+  else if (whole) walk(std::false_type{}, std::true_type{});
+  else if (!far) walk(std::true_type{}, std::false_type{});
+  else walk(std::true_type{}, std::true_type{});
   if (!live || myq >= L) return;
   store_pair_sums(p.part + (((int64_t)chunk * p.B + b) * p.H + h) * L * L + (int64_t)myq * L, sum, kk0, hf, L);
 }
@@ -1103,6 +1456,21 @@ HDS_EXPORT int hds_evoformer_fwd(const void* q, const void* k, const void* v, co
   p.q = (const bf16*)q; p.k = (const bf16*)k; p.v = (const bf16*)v; p.b1 = b1; p.b2 = b2; p.out = (bf16*)o; p.lse = lse;
   p.B = B; p.N = N; p.L = L; p.H = H;
   if (!set_scale(p, scale, bias_dtype, D)) return hipErrorInvalidValue;
+  // Workgroups that walk over three rows and more: us, a workgroup a row / walking, 8 heads: 256 positions, 48 / 65 / 112 / 128
+  // rows n 22.0 / 30.0 / 37.2 / 40.0 -> 22.9 / 28.3 / 35.0 / 36.3, 512 of 250 147 -> 111; of 128 positions, 130 / 256 16.7 / 25.5
+  // -> 16.5 / 21.8; 512 of 64 25.2 -> 17.8. (A row's bit in one word: no more than 64.)
+  const int nt = (L + 31) / 32;
+  const int64_t rows = (int64_t)B * N * H, slots = 256 * (8 / std::max(1, std::min(nt, 8)));
+  if (bias_dtype == kBF16 && D == 32 && nt <= 8 && rows > 2 * slots && rows <= 64 * slots &&
+      (int64_t)L * H * D < (1 << 30)) {  // (offsets in 32 bits)
+    const int per = (int)((rows + slots - 1) / slots);  // workgroups that fill the chip once
+    const dim3 grid(B * H * ((N + per - 1) / per)), threads(64 * nt);
+    if (nt == 1) hipLaunchKernelGGL(evo_fwd_rows_kernel<1>, grid, threads, 0, st, p, per);
+    else if (nt == 2) hipLaunchKernelGGL(evo_fwd_rows_kernel<2>, grid, threads, 0, st, p, per);
+    else if (nt <= 4) hipLaunchKernelGGL(evo_fwd_rows_kernel<4>, grid, threads, 0, st, p, per);
+    else hipLaunchKernelGGL(evo_fwd_rows_kernel<8>, grid, threads, 0, st, p, per);
+    return hipGetLastError();
+  }
   const int nw = waves_of(L, D == 128 ? kWaves<128> : kWaves<32>), blocks = (L + 32 * nw - 1) / (32 * nw);
 #define HDS_EVO(DD, TT)                                                                                             \
   hipLaunchKernelGGL((evo_fwd_kernel<DD, TT>), dim3(blocks * H * B * N), dim3(64 * nw), 0, st, p, blocks)
@@ -1209,7 +1577,7 @@ HDS_EXPORT int hds_evoformer_bwd(const void* q, const void* k, const void* v, co
       if constexpr (DD < 128) {
         if (staged) {
           auto* kernel = evo_dpair_rows_kernel<DD, TB>;
-          constexpr int lds = 8 * 128 * Tile<DD>::RB;
+          constexpr int lds = 2 * PairRows<DD>::kRow;
           const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
           if (e == hipSuccess)
             hipLaunchKernelGGL(kernel, dim3(grid2), dim3(64 * w4 * wk), lds, st, p, qblocks, kblocks, per, w4);

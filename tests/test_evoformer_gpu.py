@@ -249,3 +249,40 @@ def test_launch_attributes_are_set_for_the_current_device():
     import hcache_deepspeed_amd
     src = (pathlib.Path(hcache_deepspeed_amd.__file__).parent / "csrc" / "kernels" / "evoformer.hip").read_text()
     assert "hipFuncSetAttribute" in src and re.search(r"\bstatic\b[^;{]*hipFuncSetAttribute", src) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,N,L,H", [(1, 520, 17, 8), (1, 4100, 31, 1), (1, 260, 64, 8), (2, 140, 57, 8), (1, 140, 97, 8),
+                                     (1, 66, 200, 8), (2, 70, 256, 4)])
+def test_evoformer_walked_rows(cuda, B, N, L, H):
+    """Forward workgroups that walk over rows (three and more of a head), and both gradients from their normalisers, against
+    the general kernels, which 32-bit biases of the same values take. Among the rows: all keys masked by -1e9, by -1e38 and by
+    minus infinity, half of them by -1e38, and queries whose scores are large, far from zero or minus infinity. Both sides
+    round p and ds to bf16 (2^-9 each), the results too."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    q, k, v, do = (rnd(B, N, L, H, 32).bfloat16() for _ in range(4))
+    b1 = torch.where(rnd(B, N, 1, 1, L) < -1, -1e9, 0.).bfloat16()
+    b1[..., 0] = 0
+    b1[:, 1], b1[:, 2], b1[:, 3], b1[:, 5, ..., ::2] = -1e9, -1e38, -math.inf, -1e38
+    b2 = rnd(B, 1, H, L, L).bfloat16()
+    b2[:, :, 0, 5] += 300
+    b2[:, :, 0, 6] -= 300
+    b2[:, :, 0, 7, 3:9] = -math.inf
+    b2[:, :, H - 1, 8] = -1e9
+    do[:, 1:3] = 0  # (keys that are all masked: their weights add up to one only to the rounding of 1e9)
+    sides = []
+    for dtype in (torch.bfloat16, torch.float32):
+        leaves = [t.detach().clone().requires_grad_() for t in (q, k, v, b2.to(dtype))]
+        out = DS4Sci_EvoformerAttention(*leaves[:3], [b1.to(dtype), leaves[3]])
+        with torch.no_grad():
+            assert torch.equal(out, DS4Sci_EvoformerAttention(*leaves[:3], [b1.to(dtype), leaves[3]]))
+        sides.append([out] + list(torch.autograd.grad(out, leaves, do)))
+    for x, y in zip(*sides):
+        assert torch.isfinite(x).all() and torch.isfinite(y).all()
+        assert (x.double() - y.double()).norm() <= 4 * 2**-8 * y.double().norm()
+    x, y = (side[0].double() for side in sides)  # the rows out of the ordinary by themselves
+    for part in [(slice(None), n) for n in (1, 2, 5)] + [
+            (slice(None), slice(None), i, h) for i, h in ((5, 0), (6, 0), (7, 0), (8, H - 1))]:
+        assert (x[part] - y[part]).norm() <= 4 * 2**-8 * y[part].norm()
+    assert not x[:, 3].any() and not y[:, 3].any()
