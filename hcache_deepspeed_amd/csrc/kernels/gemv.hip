@@ -15,6 +15,7 @@
 // Weights that the memory-side cache would hold from one step to the next lose by it (all of them under 256 MB: [2048, 5632], 1
 // / 4 rows 6.3 / 6.9 -> 6.6 / 9.4 us).
 #include "hds_common.h"
+#include "row_norm.h"
 
 namespace {
 using namespace hds;
@@ -416,6 +417,8 @@ struct SkinnyOut {
   int M, N;
   int64_t ldy;
   int act;  // GLU
+  RowScale scale;  // SCALE
+  RowNorm norm;    // NORM: y, r and res [M, N]
 };
 
 // W's row r (of 16) of the workgroup's tile; rows past the end re-read the last one (not stored)
@@ -469,7 +472,8 @@ __device__ __forceinline__ void skinny_store(const SkinnyOut& o, const Gather& g
 // the same ones. There each begins somewhere else, by the fractions of the golden ratio (any distance apart is far apart):
 // 8 rows, [4096, 16384] 35.8 -> 24.0 us, [4096, 32768] 60 -> 46, [4096, 4096] 8.5 -> 7.7, [32000, 2048] level. With other rows
 // it gains or loses up to 4 % ([5120, 13824]), with gate and up rows, which are a matrix apart, nothing.
-template <int NW, bool GATHER, bool GLU>
+// SCALE: rows of a residual stream that is still to be scaled; NORM: what becomes of the sums is such a stream (row_norm.h)
+template <int NW, bool GATHER, bool GLU, bool SCALE = false, bool NORM = false>
 __global__ __launch_bounds__(64 * NW) void skinny_lines_kernel(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                                                int K, int64_t ldx, SkinnyOut o, Gather gather) {
   __shared__ __attribute__((aligned(16))) char buf[NW][4096];
@@ -482,6 +486,17 @@ __global__ __launch_bounds__(64 * NW) void skinny_lines_kernel(const bf16* __res
   char* put = mine + wr * 128 + (wz ^ wr) * 16;
   const char* get0 = mine + rr * 128 + (rp ^ (rr & 7)) * 16;
   const char* get1 = mine + rr * 128 + ((rp + 4) ^ (rr & 7)) * 16;
+  __shared__ __attribute__((aligned(16))) float red[SCALE ? NW * 16 : 4];
+  RowSums<64 * NW> sums;
+  if constexpr (SCALE) sums.load(o.scale);
+  bf16x4 res{}, gamma{};
+  const int64_t at = (int64_t)rr * o.N + blockIdx.x * 16 + 4 * rp;
+  if constexpr (NORM) {
+    if (wid == 0) {
+      if (rr < o.M) res = *reinterpret_cast<const bf16x4*>(o.norm.res + at);
+      gamma = *reinterpret_cast<const bf16x4*>(o.norm.gamma + blockIdx.x * 16 + 4 * rp);
+    }
+  }
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   const int parts = K >> 7, turn = GLU || K % 2048 ? 0 : (int)__umulhi(blockIdx.x * 2654435769u, (unsigned)parts);
   for (int c = wid; c < parts; c += NW) {  // K % 128 == 0
@@ -510,26 +525,29 @@ __global__ __launch_bounds__(64 * NW) void skinny_lines_kernel(const bf16* __res
     }
   }
   reinterpret_cast<f32x4*>(mine)[lane] = acc;
+  if constexpr (SCALE) sums.add(o.scale, red);
   __syncthreads();
   if (wid > 0) return;
 #pragma unroll
   for (int v = 1; v < NW; ++v) acc += reinterpret_cast<const f32x4*>(buf[v])[lane];
-  skinny_store<GATHER, GLU>(o, gather, acc, lane);
+  if constexpr (SCALE) acc *= RowSums<64 * NW>::rstd(o.scale, red, rr);
+  if constexpr (NORM) store_normed(o.norm, o.y, at, acc, res, gamma, blockIdx.x, lane, rr < o.M);
+  else skinny_store<GATHER, GLU>(o, gather, acc, lane);
 }
 
 // Waves a workgroup: four where there are at least two workgroups a CU of whole K walks ([6144, 4096] 13.7 us against 14.7
 // with eight, [28672, 4096] 48.6 / 50.4), eight where those are few ([4096, 14336] 26.6 against 27.9, [2048, 8192] 13.0 / 14.0)
 // or short ([16384, 2048] 17.9 / 19.0), and at up to 8 rows, whose tokens take fewer loads ([28672, 4096], 7 rows: 40.1 / 41.7).
-template <bool GATHER, bool GLU>
+template <bool GATHER, bool GLU, bool SCALE = false, bool NORM = false>
 int launch_skinny(const void* x, const void* w, int K, int64_t ldx, const SkinnyOut& o, const Gather& gather,
                   hipStream_t st) {
   const int per = GLU ? 8 : 16, tiles = (o.N + per - 1) / per;
 #define HDS_SK(T, ...) \
   hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(T), 0, st, (const bf16*)x, (const bf16*)w, K, ldx, o, gather)
   if (o.M > 8 && tiles > 256 && K >= 4096)
-    HDS_SK(256, skinny_lines_kernel<4, GATHER, GLU>);
+    HDS_SK(256, skinny_lines_kernel<4, GATHER, GLU, SCALE, NORM>);
   else
-    HDS_SK(512, skinny_lines_kernel<8, GATHER, GLU>);
+    HDS_SK(512, skinny_lines_kernel<8, GATHER, GLU, SCALE, NORM>);
 #undef HDS_SK
   return hipGetLastError();
 }
@@ -636,9 +654,23 @@ HDS_EXPORT int hds_gemv_recur_bf16(const void* x, const void* w, const float* ba
 HDS_EXPORT int hds_skinny_gemm_bf16(const void* x, const void* w, const void* bias, void* y, int M, int N, int K,
                                     int64_t ldx, int64_t ldy, int glu, hipStream_t st) {
   if (M < 1 || M > 16 || N < 1 || K < 128 || K % 128 || ldx % 8 || glu < 0 || glu > 3) return hipErrorInvalidValue;
-  const SkinnyOut o{(const bf16*)bias, (bf16*)y, M, N, ldy, glu - 1};
+  const SkinnyOut o{(const bf16*)bias, (bf16*)y, M, N, ldy, glu - 1, {}, {}};
   return glu ? launch_skinny<false, true>(x, w, K, ldx, o, Gather{}, st)
              : launch_skinny<false, false>(x, w, K, ldx, o, Gather{}, st);
+}
+
+// The same with a norm on either side (row_norm.h), M of 1 to 16 rows. ssq [parts][16] or null: x is a stream still to be scaled,
+// of K = 16 parts columns. res [M, N] or null: y = x . W^T is added to it, r and bf16(r gamma) in y's place are stored, and
+// the tiles' sums in ssq_out [N / 16][16]; N % 16 == 0, no gated unit.
+HDS_EXPORT int hds_skinny_norm_bf16(const void* x, const void* w, void* y, const float* ssq, float eps, const void* res,
+                                    const void* gamma, void* r, float* ssq_out, int M, int N, int K, int glu, hipStream_t st) {
+  if (M < 1 || M > 16 || N < 1 || K < 128 || K % 128 || glu < 0 || glu > 3 || (ssq == nullptr && res == nullptr) ||
+      (ssq != nullptr && res != nullptr) || (res != nullptr && (glu || N % 16 || !gamma || !r || !ssq_out)))
+    return hipErrorInvalidValue;
+  const SkinnyOut o{nullptr, (bf16*)y, M, N, N, glu - 1, {ssq, K / 16, eps}, {(const bf16*)res, (const bf16*)gamma, (bf16*)r, ssq_out}};
+  if (res != nullptr) return launch_skinny<false, false, false, true>(x, w, K, K, o, Gather{}, st);
+  return glu ? launch_skinny<false, true, true, false>(x, w, K, K, o, Gather{}, st)
+             : launch_skinny<false, false, true, false>(x, w, K, K, o, Gather{}, st);
 }
 
 // Fused decode GEMV (see gemv_fused_kernel): y[M, N] = norm(h (+ res)) . W^T, or with glu = 1 + activation code
@@ -719,6 +751,6 @@ HDS_EXPORT int hds_gather_gemv_bf16(const void* x, const void* w, const void* ta
     return launch_row<false, false, true>(OneRow{(const bf16*)x, nullptr, nullptr, 0.f, (const bf16*)w, nullptr, (bf16*)y,
                                                  nullptr, nullptr, N, K, 0, 0.f}, gather, st);
   else
-    return launch_skinny<true, false>(x, w, K, ldx, SkinnyOut{nullptr, (bf16*)y, M, N, ldy, 0}, gather, st);
+    return launch_skinny<true, false>(x, w, K, ldx, SkinnyOut{nullptr, (bf16*)y, M, N, ldy, 0, {}, {}}, gather, st);
   return hipGetLastError();
 }

@@ -26,6 +26,7 @@
 #include <cmath>
 
 #include "linear_common.h"
+#include "row_norm.h"
 
 namespace {
 
@@ -39,11 +40,12 @@ struct LinearArgs {
   float* part;  // [S, M, N] where S > 1 (gated: [S, M, 2N])
   int64_t ldx, ldy;
   int M, N, K, S, tm, tn, act, nt, apart;
+  RowScale scale;  // SCALE
 };
 
-// RB, CB: 16-row blocks of x and of w a wave; WM x WN waves, OCC workgroups a CU. GLU: w is [gate; up] of N rows each; half
+// SCALE: up to 16 rows of a residual stream that is still to be scaled (row_norm.h). RB, CB: 16-row blocks of x and of w a wave; WM x WN waves, OCC workgroups a CU. GLU: w is [gate; up] of N rows each; half
 // of a tile's and of a wave's columns are gates, the others the same features of up.
-template <int RB, int CB, int WM, int WN, int OCC, bool GLU>
+template <int RB, int CB, int WM, int WN, int OCC, bool GLU, bool SCALE = false>
 __global__ __launch_bounds__(64 * WM * WN, WM * WN * OCC / 4) void linear_kernel(LinearArgs p) {
   constexpr int R = 16 * RB * WM, W = 16 * CB * WN, NW = WM * WN, PER = (R + W) / (8 * NW);
   constexpr int kStage = (R + W) * 128, D = std::min(12, 160 * 1024 / OCC / kStage);
@@ -113,6 +115,8 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN * OCC / 4) void linear_kernel
       for (int j = 0; j < CB; ++j) acc[i][j] = mfma16(b[ks][j], a[ks][i], acc[i][j]);
   };
 
+  RowSums<64 * NW> sums;  // (ahead of the stages: a wait for them is none for those)
+  if constexpr (SCALE) sums.load(p.scale);
 #pragma unroll
   for (int t = 0; t < D; ++t)
     if (t < n) issue(t);
@@ -141,6 +145,17 @@ __global__ __launch_bounds__(64 * WM * WN, WM * WN * OCC / 4) void linear_kernel
     multiply(1);
   }
 
+  if constexpr (SCALE) {
+    float* red = reinterpret_cast<float*>(smem);
+    __syncthreads();  // (the last stage has been read)
+    sums.add(p.scale, red);
+    __syncthreads();
+    const float rstd = RowSums<64 * NW>::rstd(p.scale, red, lane & 15);
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int j = 0; j < CB; ++j) acc[i][j] *= rstd;
+  }
   // lane: row lane % 16 of x, 4 neighbouring columns
   constexpr int CJ = GLU ? CB / 2 : CB;
 #pragma unroll
@@ -244,8 +259,8 @@ HDS_EXPORT int hds_linear_plan(int M, int N, int K, int glu) {
 // x [M, ldx], w [N, K], bias [N] or null, y [M, ldy], plan: hds_linear_plan's, part: S x M x N floats where its slices S are
 // more than one. glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu): w [2N, K] is gate rows, then up rows, y =
 // act(gate) up, and bias and part are of 2N columns. Rows of x and w begin at 16 bytes, of y at 8.
-HDS_EXPORT int hds_linear_bf16(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy, float* part,
-                               int M, int N, int K, int glu, int plan, hipStream_t st) {
+static int linear(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy, float* part, int M, int N,
+                  int K, int glu, int plan, const RowScale& scale, hipStream_t st) {
   const int S = plan / 16, tile = plan % 16;
   if (M < 1 || M > 1100 || N < 8 || K < 4 * BK || K % BK || N % 8 || K > 1 << 22 || N > 1 << 22 || glu < 0 || glu > 3 ||
       (int64_t)(glu ? 2 * N : N) * K >= (int64_t)1 << 31 || S < 1 || S > kMaxSlices || S > K / BK || tile < 0 ||
@@ -254,7 +269,7 @@ HDS_EXPORT int hds_linear_bf16(const void* x, int64_t ldx, const void* w, const 
     return hipErrorInvalidValue;
   const int rows = glu ? 2 * N : N, R = kTiles[tile].rows, W = kTiles[tile].cols;
   LinearArgs p{(const bf16*)x, (const bf16*)w, (const bf16*)bias, (bf16*)y, part, ldx, ldy, M, N, K, S, (M + R - 1) / R,
-               (rows + W - 1) / W, glu - 1, 0, K % 2048 == 0};
+               (rows + W - 1) / W, glu - 1, 0, K % 2048 == 0, scale};
   if (glu) p.tn = (N + W / 2 - 1) / (W / 2);
   // Weights that one row of tiles reads go past the caches: [28672, 4096] 24 / 64 rows 43.5 / 44.7 -> 38.2 / 40.0 us. Not with
   // slices, whose walks are short ([4096, 14336], 128 rows 33.8 / 38.1), but in the smallest tile (24 rows 25.4 -> 24.0).
@@ -262,6 +277,12 @@ HDS_EXPORT int hds_linear_bf16(const void* x, int64_t ldx, const void* w, const 
   auto run = [&](auto kernel, int waves) {
     hipLaunchKernelGGL(kernel, dim3(p.tm * p.tn * S), dim3(64 * waves), 0, st, p);
   };
+  if (scale.ssq != nullptr) {
+    if (M > 16 || S > 1 || tile > 1) return hipErrorInvalidValue;
+    if (tile == 0) glu ? run(linear_kernel<1, 2, 2, 2, 2, true, true>, 4) : run(linear_kernel<1, 2, 2, 2, 2, false, true>, 4);
+    else glu ? run(linear_kernel<2, 2, 1, 4, 2, true, true>, 4) : run(linear_kernel<2, 2, 1, 4, 2, false, true>, 4);
+    return hipGetLastError();
+  }
 #define HDS_LINEAR(id, RB, CB, WM, WN, OCC)                                     \
   case id:                                                                      \
     if (glu) run(linear_kernel<RB, CB, WM, WN, OCC, true>, WM * WN);            \
@@ -285,4 +306,17 @@ HDS_EXPORT int hds_linear_bf16(const void* x, int64_t ldx, const void* w, const 
     else hipLaunchKernelGGL(linear_sum_kernel<false>, grid, dim3(256), 0, st, sum);
   }
   return hipGetLastError();
+}
+
+HDS_EXPORT int hds_linear_bf16(const void* x, int64_t ldx, const void* w, const void* bias, void* y, int64_t ldy, float* part,
+                               int M, int N, int K, int glu, int plan, hipStream_t st) {
+  return linear(x, ldx, w, bias, y, ldy, part, M, N, K, glu, plan, RowScale{}, st);
+}
+
+// The same of up to 16 rows of K = 16 parts columns that are still to be scaled, from the sums of their squares ssq [parts][16]:
+// plans of one slice and of the tiles of 32 rows
+HDS_EXPORT int hds_linear_scaled_bf16(const void* x, const void* w, void* y, const float* ssq, float eps, int M, int N, int K,
+                                      int glu, int plan, hipStream_t st) {
+  if (ssq == nullptr) return hipErrorInvalidValue;
+  return linear(x, K, w, nullptr, y, N, nullptr, M, N, K, glu, plan, RowScale{ssq, K / 16, eps}, st);
 }

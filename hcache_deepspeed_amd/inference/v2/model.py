@@ -40,6 +40,7 @@ from ... import comm as dist
 from ...ops import native
 from ...ops.activations import glu
 from ...ops.experts import ExpertSum
+from ...ops.gemv import ScaledRows, norm_linear, scaled_linear, scaled_rows_ok, scaled_weight_ok
 from ...ops.norm import layer_norm, rms_norm
 from ...ops.output_norm import experts_pre_norm
 from ...ops.paged import build_atoms, kv_rope_scatter
@@ -324,6 +325,9 @@ class RaggedTransformer:
         return self.embed_mod(batch, self.embed, self.pos_embed)
 
     def _attn(self, i, L, x, batch, T, capture, lat, events, sink=None, qkv=None):
+        return self.o_lin(self._attend(i, L, x, batch, T, capture, lat, events, sink, qkv), L["o.w"], L["o.b"])
+
+    def _attend(self, i, L, x, batch, T, capture, lat, events, sink=None, qkv=None):
         nq, nkv, D = self.n_q, self.n_kv, self.d
         qkv = (self.qkv_lin(x, L["qkv.w"], L["qkv.b"]) if qkv is None else qkv).view(T, nq + 2 * nkv, D)
         if capture and self.latent_mode == "kv":
@@ -331,8 +335,7 @@ class RaggedTransformer:
                 sink(i, qkv[:, nq:].reshape(T, -1))
             else:
                 self._d2h(qkv[:, nq:].reshape(T, -1).clone(), lat[i], events)  # pre-RoPE K|V
-        o = self.attn_mod(qkv, self.kv_cache.get_cache(i), batch, self.cos, self.sin)
-        return self.o_lin(o, L["o.w"], L["o.b"])
+        return self.attn_mod(qkv, self.kv_cache.get_cache(i), batch, self.cos, self.sin)
 
     def _fused_decode_ok(self, T):
         """Single-token decode steps of a plain pre-RMSNorm, SwiGLU-style dense model on the bf16 BLAS linears: the pre-norms
@@ -354,6 +357,31 @@ class RaggedTransformer:
         # one token row only: at B = 4 the per-row normalisation inside the (already VALU-bound) GEMV made the step
         # slower than the separate RMSNorm kernel (732 vs 773 tok/s); at B = 1: 247 vs 234 (profiles/r6/fused_decode/)
         return ok and T == 1
+
+    def _scaled_rows_ok(self, batch, T, capture):
+        """Decode steps of 2 to 16 sequences of a plain pre-RMSNorm, gated dense model on the bf16 BLAS linears, whose normed
+        rows nobody else reads: the products add the residual and make the norms' sums (ops/gemv.py ``norm_linear``,
+        ``scaled_linear``), so that a layer launches no norm. Registered modules that derive from the stock ones may compute
+        something else."""
+        if not scaled_rows_ok(T) or (capture and self.latent_mode != "kv"):
+            return False
+        ok = getattr(self, "_scaled_static", None)
+        if ok is None:
+            from .modules.implementations import BlasFPLinear, DSPreRMSNorm, RaggedUnembed
+            lins = (self.qkv_lin, self.o_lin, self.up_lin, self.down_lin) if self.layers and self.spec.moe is None else (None, )
+            ok = (self.device.type == "cuda" and self.dtype == torch.bfloat16 and self.tp == 1 and self.spec.gated
+                  and self.spec.parallel not in ("shared_ln", "two_ln") and self._act_name() in ("silu", "gelu_tanh", "relu")
+                  and type(self.norm_mod) is DSPreRMSNorm and type(self.unembed_mod) is RaggedUnembed
+                  and all(type(m) is BlasFPLinear for m in lins)
+                  and all(L[k] is None for L in self.layers for k in ("ln1.b", "ln2.b", "qkv.b", "o.b", "up.b", "down.b"))
+                  and all(scaled_weight_ok(L[k], k in ("o.w", "down.w"))
+                          for L in self.layers for k in ("qkv.w", "o.w", "up.w", "down.w"))
+                  and scaled_weight_ok(self.lm_head) and self.lm_head_b is None and self.final_b is None
+                  and all(torch.is_tensor(g) and g.dtype == torch.bfloat16 and g.is_contiguous()
+                          for g in [self.final_w] + [L[k] for L in self.layers for k in ("ln1.w", "ln2.w")]))
+            self._scaled_static = ok
+        return (ok and getattr(batch, "logits_of_last_tokens", False) and getattr(batch, "max_new", 0) == 1
+                and T == batch.current_sequences == batch.last_token_idx.shape[0] and torch.cuda.current_device() == self.lm_head.get_device())
 
     # ------------------------------------------------------------------------------------------
     def decode_graph_eligible(self, batch, capture_latents):
@@ -458,10 +486,13 @@ class RaggedTransformer:
                 h = self.down_lin(g, L["down.w"], L["down.b"])
             if stage is not None:
                 ring.flush_stage()  # every layer's latent rows into the ring slot, one store
+        scaled = self._scaled_rows_ok(batch, T, capture_latents)
         for i, L in (enumerate(self.layers) if not self._fused_decode_ok(T) else ()):
             if residual is None:
                 x = self._norm(h, L["ln1.w"], L["ln1.b"])
                 residual = h
+            elif scaled:
+                x = h
             elif isinstance(h, ExpertSum):
                 x, residual = experts_pre_norm(h, residual, L["ln1.w"], spec.norm_eps)
             else:
@@ -472,6 +503,14 @@ class RaggedTransformer:
                 emit(i, self._pack_fp8(x))
             elif capture_latents and self.latent_mode == "hidden_int8":
                 emit(i, self._pack_int8(x))
+            if scaled:
+                qkv = scaled_linear(x, L["qkv.w"]) if isinstance(x, ScaledRows) else None
+                a = self._attend(i, L, x, batch, T, capture_latents, lat, events, sink, qkv).view(T, -1)
+                x, residual = norm_linear(a, L["o.w"], residual, L["ln2.w"], spec.norm_eps)
+                behind = self.layers[i + 1]["ln1.w"] if i + 1 < len(self.layers) else self.final_w
+                h, residual = norm_linear(scaled_linear(x, L["up.w"], self._act_name()), L["down.w"], residual, behind,
+                                          spec.norm_eps)
+                continue
             a = self._attn(i, L, x, batch, T, capture_latents, lat, events, sink)
             if spec.parallel == "shared_ln":
                 h = self._allreduce(a + self._mlp(L, x))
@@ -483,8 +522,11 @@ class RaggedTransformer:
                 h = self._expert_parts(L, x2)
                 if h is None:
                     h = self._allreduce(self._mlp(L, x2))
-        logits = self.unembed_mod(h, residual, batch, self.lm_head, self.lm_head_b, self.final_w, self.final_b,
-                                  spec.norm_eps, self.tp_group, self.vocab)
+        if scaled:
+            logits = self.unembed_mod.project(h, self.lm_head, None, self.tp_group, self.vocab)
+        else:
+            logits = self.unembed_mod(h, residual, batch, self.lm_head, self.lm_head_b, self.final_w, self.final_b,
+                                      spec.norm_eps, self.tp_group, self.vocab)
         self.latent_event = events[-1] if events else None
         if events and sync_latents:
             events[-1].synchronize()

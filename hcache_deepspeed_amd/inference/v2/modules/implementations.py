@@ -18,7 +18,7 @@ from ....ops.delta_rule import DeltaShape, delta_rule, make_delta_plan, step_ok
 from ....ops.embedding import lookup_rows
 from ....ops.experts import PAD, ExpertSum, RouterShape, routed_experts
 from ....ops.gated_scan import gated_scan, recur_step, recur_step_ok
-from ....ops.gemv import glu_gemv, glu_linear, linear  # decode-sized steps on the HIP kernels
+from ....ops.gemv import ScaledRows, glu_gemv, glu_linear, linear, scaled_linear  # decode-sized steps on the HIP kernels
 from ....ops.grouped_gemm import moe_ffn_dropless
 from ....ops.head_prep import HeadPrep
 from ....ops.input_norm import input_norm
@@ -375,8 +375,8 @@ class RaggedUnembed(DSUnembedBase):
                 and hidden.shape[0] == batch.current_sequences == batch.last_token_idx.shape[0])
 
     def project(self, hl, lm_head, lm_head_b=None, tp_group=None, vocab=None):
-        """Logits of already normed rows."""
-        logits = linear(hl, lm_head, lm_head_b)
+        """Logits of already normed rows (``ScaledRows``: without a bias)."""
+        logits = scaled_linear(hl, lm_head) if isinstance(hl, ScaledRows) else linear(hl, lm_head, lm_head_b)
         tp = dist.get_world_size(tp_group) if tp_group is not None else 1
         if tp > 1:
             parts = [torch.empty_like(logits) for _ in range(tp)]

@@ -139,6 +139,64 @@ def rows_linear(x, w, b=None, glu=0):
     return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 
 
+# Norms between the products of 2 to 16 rows, without a launch of their own (csrc/kernels/row_norm.h)
+class ScaledRows:
+    """RMS-normed rows before their factor of each row: ``x`` is bf16(r * gamma) of the residual stream r, ``ssq`` holds the
+    sums of r * r of every 16 columns, [columns / 16, 16], which the product behind makes the factors of."""
+
+    __slots__ = ("x", "ssq", "eps")
+
+    def __init__(self, x, ssq, eps):
+        self.x, self.ssq, self.eps = x, ssq, eps
+
+
+def scaled_rows_ok(M):
+    """May steps of M rows go through ``norm_linear`` and ``scaled_linear``? Where the skinny kernel takes them and nothing could
+    want a record of the separate operations."""
+    return (SKINNY and max(2, SKINNY_MIN_M) <= M <= MAX_ROWS and not torch.is_grad_enabled()
+            and torch._C._get_tracing_state() is None and not torch.compiler.is_compiling() and not _dispatch_modes()
+            and not (_function_modes() and _watched()) and not torch.is_autocast_enabled())
+
+
+def scaled_weight_ok(w, into=False):
+    """Is ``w`` [out, in] one that ``scaled_linear`` takes, or (``into``) ``norm_linear``?"""
+    return (torch.is_tensor(w) and w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2 and w.is_contiguous()
+            and w.data_ptr() % 16 == 0 and w.shape[1] % 128 == 0 and (not into or w.shape[0] % 16 == 0))
+
+
+def norm_linear(x, w, res, gamma, eps):
+    """(``ScaledRows`` of RMSNorm(x . w^T + res) * gamma, the new residual stream). x [M, K], res [M, N] contiguous bf16; the
+    product and the sum are rounded as ``linear`` and the norm's kernel round them."""
+    M, K = x.shape
+    N = w.shape[0]
+    assert x.is_contiguous() and res.is_contiguous() and res.shape == (M, N) and gamma.is_contiguous() and gamma.numel() == N
+    assert x.dtype == res.dtype == gamma.dtype == torch.bfloat16 and w.shape[1] == K
+    y, r = torch.empty_like(res), torch.empty_like(res)
+    ssq = torch.empty(N // 16, 16, dtype=torch.float32, device=x.device)
+    native.check(native.kernels().hds_skinny_norm_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), None, 0.0, res.data_ptr(),
+                                                       gamma.data_ptr(), r.data_ptr(), ssq.data_ptr(), M, N, K, 0,
+                                                       native.stream()), "skinny_norm_bf16")
+    return ScaledRows(y, ssq, float(eps)), r
+
+
+def scaled_linear(rows, w, act=None):
+    """The normed rows times w^T, or with ``act`` the gated unit of w = [gate; up]."""
+    x, glu = rows.x, 0 if act is None else 1 + _GATHER_ACTS[act]
+    M, K = x.shape
+    N = w.shape[0] // 2 if glu else w.shape[0]
+    assert w.shape[1] == K == 16 * rows.ssq.shape[0]
+    y = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    plan = _plan(M, N, K, 1 if glu else 0) if M > 8 else 0
+    lib = native.kernels()
+    if 0 < plan < 32 and plan % 16 < 2:
+        native.check(lib.hds_linear_scaled_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), rows.ssq.data_ptr(), rows.eps, M, N, K,
+                                                glu, plan, native.stream()), "linear_scaled_bf16")
+    else:
+        native.check(lib.hds_skinny_norm_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), rows.ssq.data_ptr(), rows.eps, None,
+                                              None, None, None, M, N, K, glu, native.stream()), "skinny_norm_bf16")
+    return y
+
+
 def _needs_grad(*tensors):
     """The kernels have no backward, and a trace would hold the allocation of their result only: with gradients wanted, or a
     trace in progress, the products are torch's."""

@@ -125,7 +125,9 @@ _KERNEL_SIGS = {
     "hds_packed_rows": "pppppp" + "iiiiiiii" + "s",
     "hds_linear_plan": "iiii",
     "hds_linear_bf16": "plppplp" + "iiiii" + "s",
+    "hds_linear_scaled_bf16": "pppp" + "f" + "iiiii" + "s",
     "hds_skinny_gemm_bf16": "pppp" + "iii" + "ll" + "i" + "s",
+    "hds_skinny_norm_bf16": "pppp" + "f" + "pppp" + "iiii" + "s",
     "hds_wmix_splits": "iii",
     "hds_wmix_supported": "iiii",
     "hds_wmix_resident": "iii",

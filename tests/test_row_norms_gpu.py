@@ -1,0 +1,111 @@
+"""Norms of decode rows inside the products around them (ops/gemv.py ``norm_linear``, ``scaled_linear``), against the separate
+operations and float64."""
+import pytest
+import torch
+
+from hcache_deepspeed_amd.ops import gemv
+from hcache_deepspeed_amd.ops.activations import glu
+from hcache_deepspeed_amd.ops.norm import rms_norm
+
+EPS = 1e-5
+
+
+def _rows(g, *shape, scale=1.0):
+    return (torch.randn(*shape, device="cuda", generator=g) * scale).bfloat16()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N,out,act", [
+    (2, 128, 128, 24, None), (3, 256, 2048, 3072, None), (8, 1024, 128, 40, "relu"), (9, 5632, 2048, 1000, "gelu_tanh"),
+    (13, 512, 4096, 6144, None), (16, 4096, 4096, 14336, "silu"), (16, 256, 4096, 32000, None), (16, 256, 8320, 512, "silu"),
+    (5, 256, 9216, 264, None)])
+def test_norm_between_products(cuda, M, K, N, out, act):
+    """One row block and the last row of it, widths of one and several parts a thread (and beyond four of them), the skinny
+    kernel with four and eight waves and the tiled one (16 rows of large weights), gated units of odd halves."""
+    g = torch.Generator(device="cuda").manual_seed(M * N + out)
+    x, w = _rows(g, M, K), _rows(g, N, K, scale=K**-0.5)
+    res, gamma = _rows(g, M, N), (1 + 0.1 * torch.randn(N, device="cuda", generator=g)).bfloat16()
+    w2 = _rows(g, out * (1 if act is None else 2), N, scale=N**-0.5)
+    with torch.no_grad():
+        assert gemv.scaled_rows_ok(M) and gemv.scaled_weight_ok(w, True) and gemv.scaled_weight_ok(w2)
+        rows, r = gemv.norm_linear(x, w, res, gamma, EPS)
+        y = gemv.scaled_linear(rows, w2, act)
+        _, want_r = rms_norm(gemv.skinny(x, w), gamma, EPS, res)
+        assert torch.equal(r, want_r)  # the same sums, rounded at the same places
+        d = r.double()
+        assert torch.equal(rows.x, (r.float() * gamma.float()).bfloat16())
+        ssq = rows.ssq.double().sum(0)[:M]
+        assert ((ssq - d.square().sum(1)).abs() <= N * 2**-24 * d.square().sum(1)).all()
+        z = rows.x.double() * torch.rsqrt(d.square().mean(1, keepdim=True) + EPS) @ w2.double().T
+        if act is not None:
+            h, u = z.chunk(2, 1)
+            f = {"silu": torch.nn.functional.silu, "relu": torch.relu, "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh")}[act]
+            z = f(h) * u
+        # the result is rounded to bf16 (2^-9 each, a gated unit's two inputs as well)
+        assert (y.double() - z).norm() <= (2 if act else 1) * 2**-8 * z.norm()
+        assert torch.equal(y, gemv.scaled_linear(rows, w2, act))
+
+
+@pytest.mark.gpu
+def test_norm_rows_out_of_range(cuda):
+    """Rows with an infinity or a NaN become NaN, as a norm's do; others beside them do not; an all-zero row stays zero."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x, w, w2 = _rows(g, 4, 256), _rows(g, 512, 256, scale=1 / 16), _rows(g, 48, 512, scale=0.05)
+    res, gamma = _rows(g, 4, 512), torch.ones(512, device="cuda", dtype=torch.bfloat16)
+    res[1, 3], res[2, 5], x[3], res[3] = float("inf"), float("nan"), 0, 0
+    with torch.no_grad():
+        rows, r = gemv.norm_linear(x, w, res, gamma, EPS)
+        y = gemv.scaled_linear(rows, w2)
+    assert torch.isfinite(y[0]).all() and y[1].isnan().all() and y[2].isnan().all() and not y[3].any()
+
+
+@pytest.mark.gpu
+def test_scaled_steps_are_asked_for(cuda, monkeypatch):
+    """Where nothing may watch the separate operations, and where the switches leave the rows to the skinny kernel."""
+    with torch.no_grad():
+        assert [gemv.scaled_rows_ok(m) for m in (1, 2, 16, 17)] == [False, True, True, False]
+        with torch.autocast("cuda"):
+            assert not gemv.scaled_rows_ok(4)
+        monkeypatch.setattr(gemv, "SKINNY", False)
+        assert not gemv.scaled_rows_ok(4)
+    assert not gemv.scaled_rows_ok(4)
+    w = torch.zeros(32, 256, device="cuda", dtype=torch.bfloat16)
+    assert gemv.scaled_weight_ok(w, True) and not gemv.scaled_weight_ok(w[:, :192]) and not gemv.scaled_weight_ok(w.float())
+    assert not gemv.scaled_weight_ok(w[:24], True) and gemv.scaled_weight_ok(w[:24]) and not gemv.scaled_weight_ok(w.t())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seqs,vocab", [(2, 512), (7, 500), (16, 512)])
+def test_decode_steps_without_norm_launches(cuda, monkeypatch, seqs, vocab):
+    """Decode steps, first eager, then replayed, give the same logits as with the norms' own launches, to bf16 through the
+    layers (0.3 to 0.7 % from 64 bits either)."""
+    from hcache_deepspeed_amd.inference.v2 import model as v2
+    from hcache_deepspeed_amd.inference.v2.arch import ArchSpec
+    from hcache_deepspeed_amd.inference.v2.engine import InferenceEngineV2, RaggedInferenceEngineConfig
+    W, ff, nq, nkv = 256, 384, 2, 1
+    g = torch.Generator(device="cuda").manual_seed(seqs)
+    layers = [{"ln1.w": 1 + _rows(g, W, scale=0.1), "ln2.w": 1 + _rows(g, W, scale=0.1), "qkv.w": _rows(g, (nq + 2 * nkv) * 128, W, scale=1 / 16),
+               "o.w": _rows(g, W, nq * 128, scale=1 / 16), "up.w": _rows(g, 2 * ff, W, scale=1 / 16), "down.w": _rows(g, W, ff, scale=0.05)}
+              for _ in range(3)]
+    sd = {"embed": _rows(g, vocab, W), "final.w": 1 + _rows(g, W, scale=0.1), "lm_head.w": _rows(g, vocab, W, scale=1 / 16), "layers": layers}
+    spec = ArchSpec("llama", vocab, W, 3, nq, nkv, 128, ff, norm_eps=EPS, rope_theta=10000.0, max_position_embeddings=512)
+    conf = RaggedInferenceEngineConfig.from_dict(dict(dtype="bf16", state_manager=dict(
+        max_context=256, max_ragged_batch_size=1024, max_tracked_sequences=16, kv_block_size=64)))
+    calls, sides = [], []
+    plain = v2.norm_linear
+    monkeypatch.setattr(v2, "norm_linear", lambda *a: calls.append(1) or plain(*a))
+    for on in (True, False):
+        if not on:
+            monkeypatch.setattr(v2, "scaled_rows_ok", lambda m: False)
+        eng = InferenceEngineV2(spec, sd, conf, device=torch.device("cuda", 0), num_kv_blocks=4 * seqs)
+        uids = list(range(seqs))
+        gen = torch.Generator().manual_seed(3)
+        out = [eng.put(uids, [torch.randint(0, vocab, (5 + 3 * u, ), generator=gen) for u in uids], capture_latents=False)[0].clone()]
+        for _ in range(4):
+            out.append(eng.put(uids, [torch.randint(0, vocab, (1, ), generator=gen) for u in uids], capture_latents=False)[0].clone())
+        sides.append(out)
+        assert bool(calls) == on
+        calls.clear()
+    assert torch.equal(sides[0][0], sides[1][0])
+    for a, b in zip(*(s[1:] for s in sides)):
+        assert (a.double() - b.double()).norm() <= 0.02 * b.double().norm()
