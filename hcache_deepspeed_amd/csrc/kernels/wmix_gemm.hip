@@ -20,6 +20,7 @@
 // and ran at 0.2-0.8x the bf16 GEMM. The next chunk's weights and A are loaded before the current chunk's MFMAs.
 // K splits (grid.z) write fp32 partials reduced by wmix_reduce_kernel.
 #include "packed_codes.h"
+#include "row_norm.h"
 
 namespace {
 using namespace hds;
@@ -245,22 +246,43 @@ __device__ __forceinline__ float wmix_act(float v, int act) {  // codes of act.h
   return v * __builtin_amdgcn_rcpf(1.f + __expf(-v));
 }
 
+struct WmixOut {
+  const bf16* bias;
+  bf16* C;  // [M, N]
+  int M, N, act;
+  RowScale scale;  // A's rows are still to be scaled (row_norm.h); M <= 16
+  RowNorm norm;    // what becomes of the sums is a stream to be scaled; M <= 16, N % 16 == 0, no gated unit, no bias
+};
+
+// what a tile's norm reads beside its sums
+struct NormIn {
+  bf16x4 res, gamma;
+  __device__ __forceinline__ void load(const WmixOut& o, int tile, int row, int g) {
+    if (o.norm.res == nullptr) return;
+    const int n = tile * 16 + 4 * g;
+    res = *reinterpret_cast<const bf16x4*>(o.norm.res + (int64_t)min(row, o.M - 1) * o.N + n);
+    gamma = *reinterpret_cast<const bf16x4*>(o.norm.gamma + n);
+  }
+};
+
 // a tile's sums: lane = A row r | 16 g, weight rows 4 g .. 4 g + 3
 template <bool GLU>
-__device__ __forceinline__ void wmix_store(f32x4 s, int tile, int row, int g, int lane, const bf16* bias, bf16* C, int M,
-                                           int N, int act) {
+__device__ __forceinline__ void wmix_store(f32x4 s, int tile, int row, int g, int lane, const WmixOut& o, const NormIn& in) {
   if constexpr (GLU) {  // lanes of the upper half hold the up rows of those 32 below
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int n = tile * 8 + 4 * (g & 1) + i;
       const float up = __shfl_down(s[i], 32, 64);
-      if (lane < 32 && row < M && n < N) C[(int64_t)row * N + n] = (bf16)(wmix_act((float)(bf16)s[i], act) * (float)(bf16)up);
+      if (lane < 32 && row < o.M && n < o.N)
+        o.C[(int64_t)row * o.N + n] = (bf16)(wmix_act((float)(bf16)s[i], o.act) * (float)(bf16)up);
     }
-  } else if (row < M) {
+  } else if (o.norm.res != nullptr) {
+    store_normed(o.norm, o.C, (int64_t)row * o.N + tile * 16 + 4 * g, s, in.res, in.gamma, tile, lane, row < o.M);
+  } else if (row < o.M) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int n = tile * 16 + 4 * g + i;
-      if (n < N) C[(int64_t)row * N + n] = (bf16)(s[i] + (bias ? (float)bias[n] : 0.f));
+      if (n < o.N) o.C[(int64_t)row * o.N + n] = (bf16)(s[i] + (o.bias ? (float)o.bias[n] : 0.f));
     }
   }
 }
@@ -269,10 +291,13 @@ __device__ __forceinline__ void wmix_store(f32x4 s, int tile, int row, int g, in
 template <int FMT, int E, int NT, int MT, int NW, int MW, bool GLU>
 __global__ __launch_bounds__(64 * NW, MW) void wmix_skinny_kernel(const bf16* __restrict__ A,
                                                                   const uint8_t* __restrict__ W,
-                                                                  const float* __restrict__ scales,
-                                                                  const bf16* __restrict__ bias, bf16* __restrict__ C,
-                                                                  int M, int N, int K, int G, int act) {
+                                                                  const float* __restrict__ scales, WmixOut out,
+                                                                  int K, int G) {
   __shared__ f32x4 red[NW - 1][NT][MT][64];
+  __shared__ __attribute__((aligned(16))) float rows[NW * 16];
+  const int M = out.M, N = out.N;
+  RowSums<64 * NW> sums;
+  if (out.scale.ssq != nullptr) sums.load(out.scale);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
   const int tile0 = blockIdx.x * NT, groups = K / G;
   f32x4 acc[NT][MT];
@@ -335,15 +360,19 @@ __global__ __launch_bounds__(64 * NW, MW) void wmix_skinny_kernel(const bf16* __
 #pragma unroll
       for (int m = 0; m < MT; ++m) red[wid - 1][t][m][lane] = acc[t][m];
   }
+  if (out.scale.ssq != nullptr) sums.add(out.scale, rows);
   __syncthreads();
   if (wid > 0) return;
+  const float rstd = out.scale.ssq != nullptr ? RowSums<64 * NW>::rstd(out.scale, rows, r) : 1.f;
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
 #pragma unroll
       for (int v = 0; v < NW - 1; ++v) acc[t][m] += red[v][t][m][lane];
-      wmix_store<GLU>(acc[t][m], tile0 + t, 16 * m + r, g, lane, bias, C, M, N, act);
+      NormIn in{};
+      if constexpr (!GLU) in.load(out, tile0 + t, 16 * m + r, g);
+      wmix_store<GLU>(acc[t][m] * rstd, tile0 + t, 16 * m + r, g, lane, out, in);
     }
 }
 
@@ -390,12 +419,17 @@ __device__ __forceinline__ f32x4 run_scales(const float* s, int run, int K, int 
 // Up to MR (8 or 16) rows: A in the same way, 1 KB of each row a run; the next run's loads are on their way meanwhile.
 template <int FMT, int E, int MR, int NW, bool GLU>
 __global__ __launch_bounds__(64 * NW) void wmix_lines_kernel(const bf16* __restrict__ A, const uint8_t* __restrict__ W,
-                                                             const float* __restrict__ scales,
-                                                             const bf16* __restrict__ bias, bf16* __restrict__ C, int M,
-                                                             int N, int K, int G, int act) {
+                                                             const float* __restrict__ scales, WmixOut out, int K, int G) {
   using L = Lines<FMT>;
   __shared__ __attribute__((aligned(16))) char buf[NW][L::WB + 1024 * MR];
+  __shared__ __attribute__((aligned(16))) float rows[NW * 16];
+  const int M = out.M, N = out.N;
+  RowSums<64 * NW> sums;
+  if (out.scale.ssq != nullptr) sums.load(out.scale);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, r = lane & 15, g = lane >> 4, groups = K / G;
+  NormIn in{};
+  if constexpr (!GLU)
+    if (wid == 0) in.load(out, blockIdx.x, r, g);
   const int row_bytes = K / 512 * L::RB + K % 512 * L::RB / 512, runs = (K + 511) / 512;
   char *wl = buf[wid], *al = wl + L::WB;
   const uint8_t* wp[L::NL];
@@ -446,11 +480,13 @@ __global__ __launch_bounds__(64 * NW) void wmix_lines_kernel(const bf16* __restr
     }
   }
   reinterpret_cast<f32x4*>(wl)[lane] = acc;
+  if (out.scale.ssq != nullptr) sums.add(out.scale, rows);
   __syncthreads();
   if (wid > 0) return;
 #pragma unroll
   for (int v = 1; v < NW; ++v) acc += reinterpret_cast<const f32x4*>(buf[v])[lane];
-  wmix_store<GLU>(acc, blockIdx.x, r, g, lane, bias, C, M, N, act);
+  if (out.scale.ssq != nullptr) acc *= RowSums<64 * NW>::rstd(out.scale, rows, r);
+  wmix_store<GLU>(acc, blockIdx.x, r, g, lane, out, in);
 }
 
 // Many weight rows of up to 4,096 k: workgroups that stay on their CU. Wave w of RW holds run w of A in registers, in the
@@ -460,11 +496,10 @@ constexpr int kResWaves = 8;
 template <int FMT, int E, int RW, bool GLU>
 __global__ __launch_bounds__(64 * kResWaves, 2) void wmix_resident_kernel(const bf16* __restrict__ A,
                                                                           const uint8_t* __restrict__ W,
-                                                                          const float* __restrict__ scales,
-                                                                          const bf16* __restrict__ bias,
-                                                                          bf16* __restrict__ C, int M, int N, int K, int G,
-                                                                          int act, int tiles) {
+                                                                          const float* __restrict__ scales, WmixOut out, int K,
+                                                                          int G, int tiles) {
   constexpr int TG = kResWaves / RW;
+  const int M = out.M, N = out.N;
   using L = Lines<FMT>;
   __shared__ __attribute__((aligned(16))) char buf[kResWaves][L::WB];
   __shared__ f32x4 red[2][4][kResWaves][64];
@@ -493,7 +528,16 @@ __global__ __launch_bounds__(64 * kResWaves, 2) void wmix_resident_kernel(const 
     for (int i = 0; i < 4; ++i)
       n.sc[i] = run_scales(scales + (int64_t)wmix_row<GLU>(t, 4 * g + i, N) * groups, wr, K, G, groups);
   };
+  RowSums<64 * kResWaves> sums;
+  if (out.scale.ssq != nullptr) sums.load(out.scale);
   load(t0, ahead);
+  float rstd = 1.f;
+  if (out.scale.ssq != nullptr) {  // (before the tiles: what its loads were ahead of is still on its way)
+    float* rows = reinterpret_cast<float*>(red[1]);
+    sums.add(out.scale, rows);
+    __syncthreads();
+    rstd = RowSums<64 * kResWaves>::rstd(out.scale, rows, r);
+  }
   bf16x8 x[4][4];
 #pragma unroll
   for (int c = 0; c < 4; ++c)
@@ -537,7 +581,9 @@ __global__ __launch_bounds__(64 * kResWaves, 2) void wmix_resident_kernel(const 
       f32x4 s = rb[i][tg * RW][lane];
 #pragma unroll
       for (int v = 1; v < RW; ++v) s += rb[i][tg * RW + v][lane];
-      wmix_store<GLU>(s, t, r, g, lane, bias, C, M, N, act);
+      NormIn in{};
+      if constexpr (!GLU) in.load(out, t, r, g);
+      wmix_store<GLU>(s * rstd, t, r, g, lane, out, in);
     }
   }
 }
@@ -613,21 +659,23 @@ HDS_EXPORT int hds_wmix_resident(int M, int N, int K) {
 // The same product for few rows as a stream of packed weights (wmix_skinny_kernel, wmix_lines_kernel,
 // wmix_resident_kernel): 1 <= M <= 16, fp6 up to 32. K and G multiples of 128, A 16-byte aligned. glu: 0, or 1 + activation code (0 silu, 1 gelu_tanh, 2 relu) for
 // W = [gate; up] of 2 N rows (M <= 16, no bias).
-HDS_EXPORT int hds_wmix_skinny(const void* A, const void* W, const float* scales, const void* bias, void* C, int M, int N,
-                               int K, int G, int fmt, int ebits, int glu, hipStream_t st) {
+static int wmix_skinny(const void* A, const void* W, const float* scales, const WmixOut& o, int K, int G, int fmt, int ebits,
+                       int glu, hipStream_t st) {
+  const int M = o.M, N = o.N;
+  const bf16* bias = o.bias;
   if (M < 1 || M > (fmt == 2 && !glu ? 32 : 16) || N < 1 || K < 128 || K % 128 || G < 128 || G % 128 || K % G || glu < 0 ||
       glu > 3 || (glu && bias) || (glu && N > (1 << 29)))
     return hipErrorInvalidValue;
   const int tiles = (N + (glu ? 7 : 15)) / (glu ? 8 : 16);
   auto launch = [&](auto kern, int nt, int waves) {
     hipLaunchKernelGGL(kern, dim3((tiles + nt - 1) / nt), dim3(64 * waves), 0, st, (const bf16*)A, (const uint8_t*)W,
-                       scales, (const bf16*)bias, (bf16*)C, M, N, K, G, glu - 1);
+                       scales, o, K, G);
     return hipGetLastError();
   };
   auto resident = [&](auto kern, int rw) {
     const int wg = (tiles + kResWaves / rw - 1) / (kResWaves / rw);
     hipLaunchKernelGGL(kern, dim3(wg < 256 ? wg : 256), dim3(64 * kResWaves), 0, st, (const bf16*)A, (const uint8_t*)W,
-                       scales, (const bf16*)bias, (bf16*)C, M, N, K, G, glu - 1, tiles);
+                       scales, o, K, G, tiles);
     return hipGetLastError();
   };
   const bool res = hds_wmix_resident(M, glu ? 2 * N : N, K);
@@ -674,4 +722,19 @@ HDS_EXPORT int hds_wmix_skinny(const void* A, const void* W, const float* scales
 #undef HDS_WSG
 #undef HDS_WS
   return hipErrorInvalidValue;
+}
+
+HDS_EXPORT int hds_wmix_skinny(const void* A, const void* W, const float* scales, const void* bias, void* C, int M, int N,
+                               int K, int G, int fmt, int ebits, int glu, hipStream_t st) {
+  return wmix_skinny(A, W, scales, WmixOut{(const bf16*)bias, (bf16*)C, M, N, glu - 1, {}, {}}, K, G, fmt, ebits, glu, st);
+}
+
+// The same of up to 16 rows with a norm on either side, as hds_skinny_norm_bf16 (gemv.hip)
+HDS_EXPORT int hds_wmix_norm(const void* A, const void* W, const float* scales, void* C, const float* ssq, float eps,
+                             const void* res, const void* gamma, void* r, float* ssq_out, int M, int N, int K, int G, int fmt,
+                             int ebits, int glu, hipStream_t st) {
+  if (M > 16 || (ssq == nullptr) == (res == nullptr) || (res != nullptr && (glu || N % 16 || !gamma || !r || !ssq_out)))
+    return hipErrorInvalidValue;
+  return wmix_skinny(A, W, scales, WmixOut{nullptr, (bf16*)C, M, N, glu - 1, {ssq, K / 16, eps},
+                                           {(const bf16*)res, (const bf16*)gamma, (bf16*)r, ssq_out}}, K, G, fmt, ebits, glu, st);
 }

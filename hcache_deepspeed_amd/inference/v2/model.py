@@ -40,7 +40,7 @@ from ... import comm as dist
 from ...ops import native
 from ...ops.activations import glu
 from ...ops.experts import ExpertSum
-from ...ops.gemv import ScaledRows, norm_linear, scaled_linear, scaled_rows_ok, scaled_weight_ok
+from ...ops.gemv import ScaledRows, scaled_rows_ok, scaled_weight_ok
 from ...ops.norm import layer_norm, rms_norm
 from ...ops.output_norm import experts_pre_norm
 from ...ops.paged import build_atoms, kv_rope_scatter
@@ -359,29 +359,34 @@ class RaggedTransformer:
         return ok and T == 1
 
     def _scaled_rows_ok(self, batch, T, capture):
-        """Decode steps of 2 to 16 sequences of a plain pre-RMSNorm, gated dense model on the bf16 BLAS linears, whose normed
-        rows nobody else reads: the products add the residual and make the norms' sums (ops/gemv.py ``norm_linear``,
-        ``scaled_linear``), so that a layer launches no norm. Registered modules that derive from the stock ones may compute
-        something else."""
+        """Decode steps of 2 to 16 sequences of a plain pre-RMSNorm, gated dense model whose normed rows nobody else reads: the
+        products add the residual and make the norms' sums (ops/gemv.py ``ScaledRows``), so that a layer launches no norm.
+        Registered modules that derive from the stock ones may compute something else."""
         if not scaled_rows_ok(T) or (capture and self.latent_mode != "kv"):
             return False
-        ok = getattr(self, "_scaled_static", None)
+        known = getattr(self, "_scaled_sizes", None)
+        if known is None:
+            known = self._scaled_sizes = {}
+        ok = known.get(T)
         if ok is None:
-            from .modules.implementations import BlasFPLinear, DSPreRMSNorm, RaggedUnembed
-            lins = (self.qkv_lin, self.o_lin, self.up_lin, self.down_lin) if self.layers and self.spec.moe is None else (None, )
-            ok = (self.device.type == "cuda" and self.dtype == torch.bfloat16 and self.tp == 1 and self.spec.gated
-                  and self.spec.parallel not in ("shared_ln", "two_ln") and self._act_name() in ("silu", "gelu_tanh", "relu")
+            from .modules.implementations import (BlasFPLinear, DSPreRMSNorm, QuantizedIntLinear, QuantizedWf6Af16Linear,
+                                                  RaggedUnembed)
+            ok = (bool(self.layers) and self.spec.moe is None and self.device.type == "cuda" and self.dtype == torch.bfloat16
+                  and self.tp == 1 and self.spec.gated and self.spec.parallel not in ("shared_ln", "two_ln")
+                  and self._act_name() in ("silu", "gelu_tanh", "relu")
                   and type(self.norm_mod) is DSPreRMSNorm and type(self.unembed_mod) is RaggedUnembed
-                  and all(type(m) is BlasFPLinear for m in lins)
+                  and all(type(m) in (BlasFPLinear, QuantizedIntLinear, QuantizedWf6Af16Linear)
+                          for m in (self.qkv_lin, self.o_lin, self.up_lin, self.down_lin))
                   and all(L[k] is None for L in self.layers for k in ("ln1.b", "ln2.b", "qkv.b", "o.b", "up.b", "down.b"))
-                  and all(scaled_weight_ok(L[k], k in ("o.w", "down.w"))
-                          for L in self.layers for k in ("qkv.w", "o.w", "up.w", "down.w"))
+                  and all(self.qkv_lin.rows_ok(T, L["qkv.w"]) and self.o_lin.rows_ok(T, L["o.w"], True)
+                          and self.up_lin.rows_ok(T, L["up.w"]) and self.down_lin.rows_ok(T, L["down.w"], True) for L in self.layers)
                   and scaled_weight_ok(self.lm_head) and self.lm_head_b is None and self.final_b is None
                   and all(torch.is_tensor(g) and g.dtype == torch.bfloat16 and g.is_contiguous()
                           for g in [self.final_w] + [L[k] for L in self.layers for k in ("ln1.w", "ln2.w")]))
-            self._scaled_static = ok
+            known[T] = ok
         return (ok and getattr(batch, "logits_of_last_tokens", False) and getattr(batch, "max_new", 0) == 1
-                and T == batch.current_sequences == batch.last_token_idx.shape[0] and torch.cuda.current_device() == self.lm_head.get_device())
+                and T == batch.current_sequences == batch.last_token_idx.shape[0]
+                and torch.cuda.current_device() == self.lm_head.get_device())
 
     # ------------------------------------------------------------------------------------------
     def decode_graph_eligible(self, batch, capture_latents):
@@ -504,12 +509,12 @@ class RaggedTransformer:
             elif capture_latents and self.latent_mode == "hidden_int8":
                 emit(i, self._pack_int8(x))
             if scaled:
-                qkv = scaled_linear(x, L["qkv.w"]) if isinstance(x, ScaledRows) else None
+                qkv = self.qkv_lin.scaled_rows(x, L["qkv.w"]) if isinstance(x, ScaledRows) else None
                 a = self._attend(i, L, x, batch, T, capture_latents, lat, events, sink, qkv).view(T, -1)
-                x, residual = norm_linear(a, L["o.w"], residual, L["ln2.w"], spec.norm_eps)
+                x, residual = self.o_lin.norm_rows(a, L["o.w"], residual, L["ln2.w"], spec.norm_eps)
                 behind = self.layers[i + 1]["ln1.w"] if i + 1 < len(self.layers) else self.final_w
-                h, residual = norm_linear(scaled_linear(x, L["up.w"], self._act_name()), L["down.w"], residual, behind,
-                                          spec.norm_eps)
+                h, residual = self.down_lin.norm_rows(self.up_lin.scaled_rows(x, L["up.w"]), L["down.w"], residual, behind,
+                                                      spec.norm_eps)
                 continue
             a = self._attn(i, L, x, batch, T, capture_latents, lat, events, sink)
             if spec.parallel == "shared_ln":

@@ -18,7 +18,8 @@ from ....ops.delta_rule import DeltaShape, delta_rule, make_delta_plan, step_ok
 from ....ops.embedding import lookup_rows
 from ....ops.experts import PAD, ExpertSum, RouterShape, routed_experts
 from ....ops.gated_scan import gated_scan, recur_step, recur_step_ok
-from ....ops.gemv import ScaledRows, glu_gemv, glu_linear, linear, scaled_linear  # decode-sized steps on the HIP kernels
+from ....ops.gemv import (ScaledRows, glu_gemv, glu_linear, linear, norm_linear, scaled_linear,
+                          scaled_weight_ok)  # decode-sized steps on the HIP kernels
 from ....ops.grouped_gemm import moe_ffn_dropless
 from ....ops.head_prep import HeadPrep
 from ....ops.input_norm import input_norm
@@ -32,7 +33,8 @@ from ....ops.output_norm import (PairSum, embed_rows, experts_pre_norm, padded, 
 from ....ops.paged import (HeadShape, decode_qkv_ok, head_attention, head_blocks_ok, kv_rope_scatter, make_head_plan,
                            paged_attention, paged_decode_qkv)
 from ....ops.paged_prefill import paged_attention_portions, portions_ok
-from ....ops.quantizer import fp6_linear, int_linear, packed_glu, quantize, quantize_minifloat
+from ....ops.quantizer import (fp6_linear, int_linear, packed_glu, packed_norm_linear, packed_norm_ok, packed_scaled_linear,
+                               quantize, quantize_minifloat)
 from ....ops.rope import rope_tables
 from .interfaces import (DSEmbeddingBase, DSEmbeddingRegistry, DSExpertLayerBase, DSExpertLayerRegistry, DSGatedMLPBase,
                          DSGatedMLPRegistry, DSInputNormBase, DSInputNormRegistry, DSLinearBase, DSLinearRegistry,
@@ -113,6 +115,16 @@ class BlasFPLinear(DSLinearBase):
             return linear(x, w, b)
         return bias_act(linear(x, w), b, a)
 
+    # decode steps with the norms inside the products (ops/gemv.py ``ScaledRows``)
+    def rows_ok(self, M, w, into=False):
+        return scaled_weight_ok(w, into)
+
+    def norm_rows(self, x, w, res, gamma, eps):
+        return norm_linear(x, w, res, gamma, eps)
+
+    def scaled_rows(self, rows, w):
+        return scaled_linear(rows, w, _glu_act(self._config))
+
 
 class _PackedWeight:
     """Weight-only quantized [out, in] matrix (groups along ``in``)."""
@@ -124,6 +136,28 @@ class _PackedWeight:
 
     def nbytes(self):
         return self.q.numel() * self.q.element_size() + self.scales.numel() * 4
+
+
+def _glu_act(c):
+    """The activation of a gated projection, else None."""
+    return c.activation[:-4] if c.activation.endswith("_glu") else None
+
+
+class _PackedRows:
+    """What ``BlasFPLinear`` has for decode steps with the norms inside the products, on packed weights of ``_fmt()``."""
+
+    def rows_ok(self, M, w, into=False):
+        glu = _glu_act(self._config) is not None
+        return (isinstance(w, _PackedWeight) and (not into or w.out_features % 16 == 0) and w.q.is_cuda and packed_norm_ok(
+            M, w.out_features // (2 if glu else 1), w.in_features, w.group_size, self._fmt(), 1 if glu else 0))
+
+    def norm_rows(self, x, w, res, gamma, eps):
+        return packed_norm_linear(x, w.q, w.scales, w.out_features, w.in_features, w.group_size, self._fmt(), res, gamma, eps)
+
+    def scaled_rows(self, rows, w):
+        act = _glu_act(self._config)
+        return packed_scaled_linear(rows, w.q, w.scales, w.out_features // (1 if act is None else 2), w.in_features, w.group_size,
+                                    self._fmt(), act)
 
 
 def _packed_glu(c, x, w, b, fmt):
@@ -141,7 +175,7 @@ def _group(c, in_features):
 
 
 @DSLinearRegistry.register_module
-class QuantizedWf6Af16Linear(DSLinearBase):
+class QuantizedWf6Af16Linear(_PackedRows, DSLinearBase):
     """FP6 (e3m2) weights, bf16 activations: the reference's ``quantized_wf6af16_linear``."""
 
     @staticmethod
@@ -151,6 +185,9 @@ class QuantizedWf6Af16Linear(DSLinearBase):
     @staticmethod
     def supports_config(c):
         return c.quantization_mode == "wf6af16" and _supports_act(c.activation) and c.in_channels % 16 == 0
+
+    def _fmt(self):
+        return "fp6"
 
     def transform_param(self, w):
         if isinstance(w, _PackedWeight) or w is None:
@@ -169,7 +206,7 @@ class QuantizedWf6Af16Linear(DSLinearBase):
 
 
 @DSLinearRegistry.register_module
-class QuantizedIntLinear(DSLinearBase):
+class QuantizedIntLinear(_PackedRows, DSLinearBase):
     """Symmetric group-wise INT8 / INT4 weights, bf16 activations (inference v1's int8 weight path in v2)."""
 
     @staticmethod
@@ -182,6 +219,9 @@ class QuantizedIntLinear(DSLinearBase):
 
     def _bits(self):
         return 8 if self._config.quantization_mode == "int8" else 4
+
+    def _fmt(self):
+        return self._config.quantization_mode
 
     def transform_param(self, w):
         if isinstance(w, _PackedWeight) or w is None:

@@ -133,6 +133,7 @@ _KERNEL_SIGS = {
     "hds_wmix_resident": "iii",
     "hds_paged_prefill": "pl" + "p" + "pl" + "pi" + "pp" + "iiii" + "f" + "ii" + "s",
     "hds_wmix_skinny": "ppppp" + "iiiiiii" + "s",
+    "hds_wmix_norm": "ppppp" + "f" + "pppp" + "iiiiiii" + "s",
     "hds_wmix_gemm": "pppppp" + "iiiiii" + "s",
     "hds_token_gather": "i" + "ppp" + "iiii" + "s",
     "hds_token_scatter": "i" + "ppp" + "iiii" + "s",

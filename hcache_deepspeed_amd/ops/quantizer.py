@@ -11,6 +11,7 @@ import os
 import torch
 
 from . import native
+from .gemv import ScaledRows
 
 _FP8_MAX = {"e4m3": 448.0, "e5m2": 57344.0}
 
@@ -259,6 +260,37 @@ def _wmix_skinny(x2, q_weight, scales, out_features, in_features, group_size, fm
                                                   native.ptr(bias), y.data_ptr(), M, out_features, in_features,
                                                   group_size, _FMTS[fmt], int(ebits), int(glu),
                                                   native.stream()), "wmix_skinny")
+    return y
+
+
+def packed_norm_ok(M, out_features, in_features, group_size, fmt, glu=0, ebits=3):
+    """May ``packed_norm_linear`` and ``packed_scaled_linear`` take M rows? Where ``_wmix_skinny`` takes them on its stream."""
+    return (1 < M <= 16 and in_features % 128 == 0 and group_size % 128 == 0 and in_features % group_size == 0
+            and (fmt != "fp6" or ebits in (2, 3)) and not _packed_plan(M, out_features, in_features, group_size, fmt, 1 if glu else 0)
+            and (glu or not _gemv_wins(M, out_features, in_features, fmt)))
+
+
+def packed_norm_linear(x, q_weight, scales, out_features, in_features, group_size, fmt, res, gamma, eps, ebits=3):
+    """ops/gemv.py ``norm_linear`` on packed weights."""
+    M, N = x.shape[0], out_features
+    assert x.shape == (M, in_features) and res.shape == (M, N) and gamma.numel() == N and N % 16 == 0 and scales.numel() * group_size == N * in_features
+    assert all(t.is_contiguous() and t.dtype == torch.bfloat16 for t in (x, res, gamma)) and x.data_ptr() % 16 == 0
+    y, r = torch.empty_like(res), torch.empty_like(res)
+    ssq = torch.empty(N // 16, 16, dtype=torch.float32, device=x.device)
+    native.check(native.kernels().hds_wmix_norm(x.data_ptr(), q_weight.data_ptr(), scales.data_ptr(), y.data_ptr(), None, 0.0,
+                                                res.data_ptr(), gamma.data_ptr(), r.data_ptr(), ssq.data_ptr(), M, N, in_features,
+                                                group_size, _FMTS[fmt], int(ebits), 0, native.stream()), "wmix_norm")
+    return ScaledRows(y, ssq, float(eps)), r
+
+
+def packed_scaled_linear(rows, q_weight, scales, out_features, in_features, group_size, fmt, act=None, ebits=3):
+    """ops/gemv.py ``scaled_linear`` on packed weights; ``out_features``: of the result."""
+    x, glu = rows.x, 0 if act is None else _GLU_ACTS[act]
+    assert in_features == x.shape[1] == 16 * rows.ssq.shape[0] and scales.numel() * group_size == (2 if glu else 1) * out_features * in_features
+    y = torch.empty(x.shape[0], out_features, dtype=torch.bfloat16, device=x.device)
+    native.check(native.kernels().hds_wmix_norm(x.data_ptr(), q_weight.data_ptr(), scales.data_ptr(), y.data_ptr(),
+                                                rows.ssq.data_ptr(), rows.eps, None, None, None, None, x.shape[0], out_features,
+                                                in_features, group_size, _FMTS[fmt], int(ebits), glu, native.stream()), "wmix_norm")
     return y
 
 

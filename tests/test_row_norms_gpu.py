@@ -3,8 +3,7 @@ operations and float64."""
 import pytest
 import torch
 
-from hcache_deepspeed_amd.ops import gemv
-from hcache_deepspeed_amd.ops.activations import glu
+from hcache_deepspeed_amd.ops import gemv, native
 from hcache_deepspeed_amd.ops.norm import rms_norm
 
 EPS = 1e-5
@@ -47,6 +46,39 @@ def test_norm_between_products(cuda, M, K, N, out, act):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["fp6", "int8", "int4"])
+@pytest.mark.parametrize("M,K,N,out,act", [(2, 256, 2048, 3072, None), (8, 4096, 4096, 6144, None), (3, 5632, 2048, 8192, "silu"),
+                                           (8, 128, 4096, 8192, "relu"), (16, 8192, 4096, 4096, "gelu_tanh"), (13, 2048, 1024, 1536, None)])
+def test_norm_between_packed_products(cuda, fmt, M, K, N, out, act):
+    """The same on packed weights, through each of the stream's kernels: whole lines, resident rows, one and two tiles."""
+    from hcache_deepspeed_amd.ops import quantizer as q
+    g = torch.Generator(device="cuda").manual_seed(M * N + out)
+    res, gamma = _rows(g, M, N), (1 + 0.1 * torch.randn(N, device="cuda", generator=g)).bfloat16()
+    x, w, w2 = _rows(g, M, K), _rows(g, N, K, scale=K**-0.5), _rows(g, out * (1 if act is None else 2), N, scale=N**-0.5)
+
+    def pack(w):
+        return q.quantize_minifloat(w, 128, 6, 2)[:2] if fmt == "fp6" else q.quantize(w, 128, int(fmt[3:]), True)[:2]
+    with torch.no_grad():
+        a, b = pack(w), pack(w2)
+        rows, r = q.packed_norm_linear(x, *a, N, K, 128, fmt, res, gamma, EPS)
+        y = q.packed_scaled_linear(rows, *b, out, N, 128, fmt, act)
+        plain = torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
+        native.check(native.kernels().hds_wmix_skinny(x.data_ptr(), a[0].data_ptr(), a[1].data_ptr(), None, plain.data_ptr(), M, N, K,
+                                                      128, q._FMTS[fmt], 3, 0, native.stream()), "wmix_skinny")
+        _, want_r = rms_norm(plain, gamma, EPS, res)
+        assert torch.equal(r, want_r) and torch.equal(rows.x, (r.float() * gamma.float()).bfloat16())
+        # the same weights against rows that are normed beforehand: both round the rows, the sums' factor and the result once
+        xn = (rows.x.double() * torch.rsqrt(r.double().square().mean(1, keepdim=True) + EPS))
+        stored = q.dequantize_minifloat(*b, 128, 6, 2, torch.float32) if fmt == "fp6" else q.dequantize(*b, None, 128, int(fmt[3:]), True, torch.float32)
+        z = xn @ stored.double().view(w2.shape).T
+        if act is not None:
+            h, u = z.chunk(2, 1)
+            f = {"silu": torch.nn.functional.silu, "relu": torch.relu, "gelu_tanh": lambda t: torch.nn.functional.gelu(t, approximate="tanh")}[act]
+            z = f(h) * u
+        assert (y.double() - z).norm() <= (2 if act else 1) * 2**-8 * z.norm()
+
+
+@pytest.mark.gpu
 def test_norm_rows_out_of_range(cuda):
     """Rows with an infinity or a NaN become NaN, as a norm's do; others beside them do not; an all-zero row stays zero."""
     g = torch.Generator(device="cuda").manual_seed(1)
@@ -75,8 +107,8 @@ def test_scaled_steps_are_asked_for(cuda, monkeypatch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("seqs,vocab", [(2, 512), (7, 500), (16, 512)])
-def test_decode_steps_without_norm_launches(cuda, monkeypatch, seqs, vocab):
+@pytest.mark.parametrize("seqs,vocab,quant", [(2, 512, ""), (7, 500, ""), (16, 512, ""), (5, 512, "wf6af16"), (3, 512, "int8"), (4, 512, "int4")])
+def test_decode_steps_without_norm_launches(cuda, monkeypatch, seqs, vocab, quant):
     """Decode steps, first eager, then replayed, give the same logits as with the norms' own launches, to bf16 through the
     layers (0.3 to 0.7 % from 64 bits either)."""
     from hcache_deepspeed_amd.inference.v2 import model as v2
@@ -89,11 +121,13 @@ def test_decode_steps_without_norm_launches(cuda, monkeypatch, seqs, vocab):
               for _ in range(3)]
     sd = {"embed": _rows(g, vocab, W), "final.w": 1 + _rows(g, W, scale=0.1), "lm_head.w": _rows(g, vocab, W, scale=1 / 16), "layers": layers}
     spec = ArchSpec("llama", vocab, W, 3, nq, nkv, 128, ff, norm_eps=EPS, rope_theta=10000.0, max_position_embeddings=512)
-    conf = RaggedInferenceEngineConfig.from_dict(dict(dtype="bf16", state_manager=dict(
+    conf = RaggedInferenceEngineConfig.from_dict(dict(dtype="bf16", quantization={"quantization_mode": quant} if quant else {}, state_manager=dict(
         max_context=256, max_ragged_batch_size=1024, max_tracked_sequences=16, kv_block_size=64)))
     calls, sides = [], []
-    plain = v2.norm_linear
-    monkeypatch.setattr(v2, "norm_linear", lambda *a: calls.append(1) or plain(*a))
+    from hcache_deepspeed_amd.inference.v2.modules import implementations as m
+    name = "packed_norm_linear" if quant else "norm_linear"
+    plain = getattr(m, name)
+    monkeypatch.setattr(m, name, lambda *a: calls.append(1) or plain(*a))
     for on in (True, False):
         if not on:
             monkeypatch.setattr(v2, "scaled_rows_ok", lambda m: False)
