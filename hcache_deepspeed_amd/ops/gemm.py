@@ -9,6 +9,7 @@ import os
 import torch
 
 from . import native
+from .gemv import _plan, rows_linear
 
 
 def _native_ok(a, b, out):
@@ -274,6 +275,33 @@ _DGRAD_LAYOUT = os.environ.get("HDS_DGRAD_LAYOUT", "auto")  # auto | direct | nt
 _DGRAD_CHOICE = {}
 
 
+def _dgrad_sliced(T, N, K):
+    """Is dX[T, K] = dY[T, N] W[N, K] one for csrc/kernels/linear.hip on W^T? Long reductions into few columns (an LM head's),
+    which leave the library a part of the CUs: 73 workgroups at 1,018 rows of [32000, 2048]. us, the faster of the library's two
+    layouts -> sliced, transposes included, at 40 / 128 / 509 / 1,018 rows: [32000, 768] 107 / 109 / 142 / 193 -> 46 / 55 / 82 /
+    104; [32000, 2048] 149 / 156 / 218 / 310 -> 108 / 120 / 162 / 210; [128256, 2048] 408 / 384 / 643 / 981 -> 357 / 386 / 502 /
+    695. Up to 4,096 columns only between the few rows that read the weight once and those that fill the chip: [32000, 4096] at
+    192 / 256 / 509 / 700 / 900 rows 204 / 243 / 322 / 330 / 346 -> 209 / 217 / 269 / 317 / 359, [28672, 4096] 188 / 229 / 303 /
+    306 / 333 -> 183 / 191 / 246 / 290 / 314. With a shorter or a longer reduction the transpose costs as much as the slices
+    give: 509 rows of [11264, 2048] 66 -> 70, [8192, 4096] 77 -> 82, [128256, 4096] 885 -> 919."""
+    if K <= 2048:
+        return 40 <= T <= 1100 and N >= 12 * K and bool(_plan(T, K, N))
+    return 256 <= T <= 640 and K <= 4096 and 6 * K <= N <= 8 * K and bool(_plan(T, K, N))
+
+
+def _dgrad_slices(dy2, w, out, cache):
+    """The sliced product, None where it does not take the call or its transpose does not fit."""
+    if not native.plain(dy2, w) or torch.is_autocast_enabled():
+        return None
+    try:
+        wt = transpose2d(w) if cache is None or "wt" not in cache else cache["wt"].t()
+        if cache is not None:
+            cache["wt"] = wt.t()
+        return rows_linear(dy2, wt, out=out)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def _dgrad_run(layout, dy2, w, out, cache=None):
     if layout == "nt":  # nt: dY @ (W^T)^T, hipBLASLt's NT form
         b = cache.get("wt") if cache is not None else None
@@ -299,6 +327,10 @@ def dgrad(dy2, w, out=None, cache=None):
                 and w.stride(1) == 1):
             layout = "direct"
         else:
+            if _dgrad_sliced(dy2.shape[0], *w.shape):
+                dx = _dgrad_slices(dy2, w, out, cache)
+                if dx is not None:
+                    return dx
             key = (_rows_bucket(dy2.shape[0]), dy2.shape[1], tuple(w.shape))
             layout = _DGRAD_CHOICE.get(key)
             if layout is None:

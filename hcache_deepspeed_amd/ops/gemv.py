@@ -99,9 +99,9 @@ def _watched():
     return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(_function_modes()))
 
 
-def rows_linear(x, w, b=None, glu=0):
-    """``F.linear(x, w, b)`` of 9 rows and more, or with ``glu`` = 1 + activation code the gated unit of w = [gate; up]; None
-    where the kernel does not take the call, as where anything could want a record of it (``native.plain``, torch.compile, a
+def rows_linear(x, w, b=None, glu=0, out=None):
+    """``F.linear(x, w, b)`` of 9 rows and more, or with ``glu`` = 1 + activation code the gated unit of w = [gate; up],
+    written to ``out`` (contiguous, x's type) where given; None where the kernel does not take the call, as where anything could want a record of it (``native.plain``, torch.compile, a
     dispatch or function mode: a trace by make_fx, a counter, fake tensors would find the allocation of the result only)."""
     if torch.compiler.is_compiling():
         return None
@@ -132,7 +132,10 @@ def rows_linear(x, w, b=None, glu=0):
     if b is not None and (b.dtype != torch.bfloat16 or not b.is_contiguous() or b.shape != w.shape[:1] or
                           b.get_device() != x.get_device()):
         return None
-    y = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
+    if out is not None and (out.dtype != torch.bfloat16 or out.device != x.device or not out.is_contiguous()
+                            or out.shape != (M, N) or out.data_ptr() % 8):
+        return None
+    y = torch.empty(M, N, dtype=torch.bfloat16, device=x.device) if out is None else out
     part = torch.empty(plan // 16, M, rows, dtype=torch.float32, device=x.device) if plan >= 32 else None
     native.check(native.kernels().hds_linear_bf16(px, ld, pw, native.ptr(b), y.data_ptr(), N, native.ptr(part), M, N, K, glu,
                                                   plan, native.stream()), "linear_bf16")

@@ -159,3 +159,34 @@ def test_one_operand_that_does_not_pad(monkeypatch):
     gemm._wgrad_run("nt", dy, x, out, False)
     ref, mag = dy.double().t() @ x.double(), dy.double().abs().t() @ x.double().abs()
     assert not made and ((out.double() - ref).abs() <= 2**-8 * ref.abs() + 2**-20 * mag).all()
+
+
+# one and several row tiles, rows behind the last tile, both rules, a last chunk that shares the transposed weight
+@pytest.mark.parametrize("T,N,K", [(40, 8192, 512), (129, 12352, 1024), (509, 32000, 2048), (1100, 32000, 768),
+                                   (257, 28672, 4096)])
+@pytest.mark.parametrize("kept", [False, True])
+def test_sliced_input_gradients_match_64_bits(T, N, K, kept):
+    from hcache_deepspeed_amd.ops import gemm
+    g = torch.Generator(device="cuda").manual_seed(T + N)
+    w = (torch.randn(N, K, device="cuda", generator=g) * N**-0.5).to(torch.bfloat16)
+    dy = torch.randn(T, N, device="cuda", generator=g).to(torch.bfloat16)
+    dy[-1, -64:] = 100
+    assert gemm._dgrad_sliced(T, N, K)
+    cache, out = {} if kept else None, torch.full((T, K), float("nan"), dtype=torch.bfloat16, device="cuda")
+    with torch.no_grad():
+        y = gemm.dgrad(dy, w, out=out, cache=cache)
+        again = gemm.dgrad(dy, w, cache=cache)
+        assert gemm._dgrad_slices(dy, w, None, None) is not None
+    recorded = gemm.dgrad(dy, w)  # gradients are being recorded: the library's
+    ref = dy.double() @ w.double()
+    # 32-bit sums of N products, then one rounding
+    bound = 2**-8 * ref.abs() + 2**-24 * N**0.5 * 8 * (dy.double().abs() @ w.double().abs()) + 1e-6
+    assert y.data_ptr() == out.data_ptr() and ((y.double() - ref).abs() <= bound).all() and torch.equal(y, again)
+    assert ((recorded.double() - ref).abs() <= bound).all()
+
+
+def test_sliced_input_gradients_stay_where_they_gain():
+    from hcache_deepspeed_amd.ops import gemm
+    for T, N, K in ((39, 32000, 2048), (1101, 32000, 2048), (509, 11264, 2048), (255, 32000, 4096), (641, 32000, 4096),
+                    (509, 128256, 4096), (509, 8192, 4096), (509, 57344, 8192)):
+        assert not gemm._dgrad_sliced(T, N, K)
