@@ -28,16 +28,25 @@ constexpr int kFewRows = 64;
 // ---------------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------------
-// PICK: with pick, output row i is made from rows pick[i] of x and res, of which there are n_in; negative ones count from
+// PICK 1: with pick, output row i is made from rows pick[i] of x and res, of which there are n_in; negative ones count from
 // the end, and a row outside them gives NaN. (Without PICK nothing asks at run time, which cost norms of one wave a row 0.1 us, 3 to
 // 5 % of 256 rows of 512 to 2,048.) A serving step normalises only the rows whose logits are wanted: gathering
 // them first took four launches (two index conversions, two gathers; 18 us of a 490 us decode step of 16 sequences).
+// PICK 2: pick holds 64-bit ids and x is an embedding: its rows are copied to res_out beside their norm, an id outside it gives
+// NaN in both. A step's lookup and first norm in one launch: a chain of kernels waits 2 to 4 us for each, and a long prompt's rows are
+// read once less (in a graph, lookup and norm apart -> here: 4 rows of 2,048 3.6 -> 2.2 us, 16 of 4,096 3.8 -> 2.4, 2,048 of 4,096
+// 16.0 -> 9.4, 16,000 of 2,048 40.8 -> 30.0).
 struct PickedRow {
   int row;
   bool ok;
 };
-template <bool PICK>
+template <int PICK>
 __device__ __forceinline__ PickedRow picked_row(const int* pick, int row, int n_in) {
+  if constexpr (PICK == 2) {
+    const int64_t id = reinterpret_cast<const int64_t*>(pick)[row];
+    const bool ok = id >= 0 && id < n_in;
+    return {ok ? (int)id : 0, ok};
+  }
   if (!PICK || pick == nullptr) return {row, true};
   int r = pick[row];
   if (r < 0) r += n_in;
@@ -61,7 +70,7 @@ __device__ __forceinline__ float row_sum(float v, float* red) {
 
 // WPR waves take a row. The few rows of a decode step would leave the latencies of a whole row's loads and stores to one wave
 // each: with a residual, 16 rows of 2048 / 4096 / 8192 2.6 / 3.4 / 5.1 us, with four waves a row 2.1 / 2.4 / 2.7.
-template <typename T, typename WT, int NV, bool LN, int WPR, bool PICK>
+template <typename T, typename WT, int NV, bool LN, int WPR, int PICK>
 __global__ __launch_bounds__(256) void norm_fwd_kernel(const T* __restrict__ x, const T* __restrict__ res,
                                                        T* __restrict__ res_out, const WT* __restrict__ w,
                                                        const WT* __restrict__ b, T* __restrict__ y,
@@ -92,11 +101,18 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const T* __restrict__ x, 
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[i][j] = to_f(from_f<T>(v[i][j] + r[j]));  // round like the unfused add
     }
-    if (res_out != nullptr && live) {
-      T* ro = res_out + (int64_t)row * cols;
+  }
+  if constexpr (PICK == 2) {
+    if (!in.ok)
 #pragma unroll
-      for (int i = 0; i < V; ++i) Vec8<T>::store(ro + c0 + i * 512, v[i]);
-    }
+      for (int i = 0; i < V; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[i][j] = NAN;
+  }
+  if ((PICK == 2 || res != nullptr) && res_out != nullptr && live) {
+    T* ro = res_out + (int64_t)row * cols;
+#pragma unroll
+    for (int i = 0; i < V; ++i) Vec8<T>::store(ro + c0 + i * 512, v[i]);
   }
   if constexpr (WPR > 1) {  // in front of the barriers; with whole rows a wave the registers are worth more
 #pragma unroll
@@ -139,14 +155,14 @@ __global__ __launch_bounds__(256) void norm_fwd_kernel(const T* __restrict__ x, 
     }
     Vec8<T>::store(yr + c, o);
   }
-  if (lane == 0 && wid % WPR == 0) {
+  if (PICK != 2 && lane == 0 && wid % WPR == 0) {
     stat_rstd[row] = rstd;
     if constexpr (LN) stat_mean[row] = mean;
   }
 }
 
 // Generic-width forward (cols % 8 == 0, any cols): two passes over the row (second hits L1/L2).
-template <typename T, typename WT, bool LN, bool PICK>
+template <typename T, typename WT, bool LN, int PICK>
 __global__ __launch_bounds__(256) void norm_fwd_generic(const T* __restrict__ x, const T* __restrict__ res,
                                                         T* __restrict__ res_out, const WT* __restrict__ w,
                                                         const WT* __restrict__ b, T* __restrict__ y,
@@ -169,8 +185,13 @@ __global__ __launch_bounds__(256) void norm_fwd_generic(const T* __restrict__ x,
       Vec8<T>::load(rr + c, r);
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = to_f(from_f<T>(v[j] + r[j]));
-      if (ro) Vec8<T>::store(ro + c, v);
     }
+    if constexpr (PICK == 2) {
+      if (!in.ok)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = NAN;
+    }
+    if (ro && (PICK == 2 || rr)) Vec8<T>::store(ro + c, v);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       s += v[j];
@@ -199,7 +220,7 @@ __global__ __launch_bounds__(256) void norm_fwd_generic(const T* __restrict__ x,
     for (int j = 0; j < 8; ++j) o[j] = (v[j] - mean) * rstd * wv[j] + bv[j];
     Vec8<T>::store(yr + c, o);
   }
-  if (lane == 0) {
+  if (PICK != 2 && lane == 0) {
     stat_rstd[row] = rstd;
     if (LN) stat_mean[row] = mean;
   }
@@ -389,7 +410,7 @@ __global__ __launch_bounds__(1024) void reduce_parts_kernel(const float* __restr
   out[c] = from_f<WT>(t);
 }
 
-template <typename T, typename WT, bool LN, bool PICK>
+template <typename T, typename WT, bool LN, int PICK>
 hipError_t launch_fwd_rows(const void* x, const void* res, void* res_out, const void* w, const void* b, void* y,
                            float* mean, float* rstd, int rows, int cols, float eps, const int* pick, int n_in,
                            hipStream_t st) {
@@ -401,7 +422,7 @@ hipError_t launch_fwd_rows(const void* x, const void* res, void* res_out, const 
   // 93): longer steps, the training ones among them, keep the sums of one wave in their order.
 #define HDS_NF(COLS, NV, WPR)                                              \
   case COLS:                                                               \
-    if (rows <= kFewRows) args(norm_fwd_kernel<T, WT, NV, LN, WPR, true>, WPR); \
+    if (rows <= kFewRows) args(norm_fwd_kernel<T, WT, NV, LN, WPR, PICK == 2 ? 2 : 1>, WPR); \
     else args(norm_fwd_kernel<T, WT, NV, LN, 1, PICK>, 1);                 \
     break
   switch (cols) {
@@ -424,8 +445,8 @@ hipError_t launch_fwd(const void* x, const void* res, void* res_out, const void*
                       float* mean, float* rstd, int rows, int cols, float eps, const int* pick, int n_in,
                       hipStream_t st) {
   if (pick != nullptr)
-    return launch_fwd_rows<T, WT, LN, true>(x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, pick, n_in, st);
-  return launch_fwd_rows<T, WT, LN, false>(x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, pick, n_in, st);
+    return launch_fwd_rows<T, WT, LN, 1>(x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, pick, n_in, st);
+  return launch_fwd_rows<T, WT, LN, 0>(x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, pick, n_in, st);
 }
 
 template <typename T, typename WT, bool LN>
@@ -474,6 +495,22 @@ HDS_EXPORT int hds_norm_fwd(int is_ln, int dtype, int wdtype, const void* x, con
   if (is_ln)
     HDS_DISPATCH2(dtype, wdtype, true, launch_fwd, x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, pick, n_in, st);
   HDS_DISPATCH2(dtype, wdtype, false, launch_fwd, x, res, res_out, w, b, y, mean, rstd, rows, cols, eps, pick, n_in, st);
+}
+
+// y[i] = RMSNorm(table[ids[i]]) * w and h[i] = table[ids[i]]; table [n_rows, cols]
+HDS_EXPORT int hds_embed_norm(int dtype, const void* table, const int64_t* ids, const void* w, void* h, void* y, int n,
+                              int cols, int n_rows, float eps, hipStream_t st) {
+  if (n < 0 || cols < 8 || cols % 8 || n_rows < 1) return hipErrorInvalidValue;
+  if (n == 0) return hipSuccess;
+  auto go = [&](auto t) {
+    using T = decltype(t);
+    return launch_fwd_rows<T, T, false, 2>(table, nullptr, h, w, nullptr, y, nullptr, nullptr, n, cols, eps, (const int*)ids,
+                                           n_rows, st);
+  };
+  if (dtype == kBF16) return go(bf16{});
+  if (dtype == kF32) return go(0.f);
+  if (dtype == kF16) return go((_Float16)0.f);
+  return hipErrorInvalidValue;
 }
 
 static int g_norm_bwd_max_parts = 512;

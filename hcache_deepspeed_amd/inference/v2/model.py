@@ -39,6 +39,7 @@ import torch.nn.functional as F
 from ... import comm as dist
 from ...ops import native
 from ...ops.activations import glu
+from ...ops.embedding import norm_rows
 from ...ops.experts import ExpertSum
 from ...ops.gemv import ScaledRows, scaled_rows_ok, scaled_weight_ok
 from ...ops.norm import layer_norm, rms_norm
@@ -48,7 +49,7 @@ from ...ops.rope import rope_tables
 from .modules import (DSEmbeddingsConfig, DSLinearConfig, DSMoEConfig, DSNormConfig, DSSelfAttentionConfig,
                       DSUnembedConfig, instantiate_attention, instantiate_embed, instantiate_linear, instantiate_moe,
                       instantiate_pre_norm, instantiate_unembed)
-from .modules.implementations import DSPreRMSNorm, GroupedGemmMoE, RaggedUnembed, _PackedWeight
+from .modules.implementations import DSPreRMSNorm, GroupedGemmMoE, RaggedEmbedding, RaggedUnembed, _PackedWeight
 
 
 class _Layer:
@@ -324,6 +325,16 @@ class RaggedTransformer:
     def _embed(self, batch):
         return self.embed_mod(batch, self.embed, self.pos_embed)
 
+    def _embed_norm(self, batch, T):
+        """The embedded rows and the first layer's norm of them, or None: a registered module that derives from the stock one may
+        compute something else, and one row is normed by the product behind it."""
+        if (self.pos_embed is not None or not self.layers or type(self.embed_mod) is not RaggedEmbedding
+                or type(self.norm_mod) is not DSPreRMSNorm or self.layers[0]["ln1.b"] is not None
+                or self.layers[0]["ln1.w"] is None or self._fused_decode_ok(T)
+                or type(self)._embed is not RaggedTransformer._embed or type(self)._norm is not RaggedTransformer._norm):
+            return None
+        return norm_rows(self.embed, batch.input_ids, self.layers[0]["ln1.w"], self.spec.norm_eps)
+
     def _attn(self, i, L, x, batch, T, capture, lat, events, sink=None, qkv=None):
         return self.o_lin(self._attend(i, L, x, batch, T, capture, lat, events, sink, qkv), L["o.w"], L["o.b"])
 
@@ -457,7 +468,8 @@ class RaggedTransformer:
         spec = self.spec
         self._prep(batch)
         T = batch.current_tokens
-        h = self._embed(batch)
+        first = self._embed_norm(batch, T)  # rows and their first norm by one kernel
+        h = self._embed(batch) if first is None else first[0]
         residual = None
         lat = None
         events = []
@@ -494,7 +506,7 @@ class RaggedTransformer:
         scaled = self._scaled_rows_ok(batch, T, capture_latents)
         for i, L in (enumerate(self.layers) if not self._fused_decode_ok(T) else ()):
             if residual is None:
-                x = self._norm(h, L["ln1.w"], L["ln1.b"])
+                x = self._norm(h, L["ln1.w"], L["ln1.b"]) if first is None else first[1]
                 residual = h
             elif scaled:
                 x = h

@@ -16,6 +16,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import native
+from ..offload import act_plan as _ap
 
 
 def embedding_grad_add_(grad, ids, dy, padding_idx=None):
@@ -52,6 +53,26 @@ def lookup_rows(table, ids):
                                                       table.shape[0], native.stream()), "gather_rows")
         return out
     return F.embedding(ids, table)
+
+
+def norm_rows(table, ids, weight, eps):
+    """(``lookup_rows(table, ids)``, the RMS norm of those rows) by one kernel, or None where it does not take the call."""
+    if not (native.use_native(table) and native.plain(table, ids, weight) and not _ap.tracking()):
+        return None
+    if not (table.dim() == 2 and ids.dim() == weight.dim() == 1 and ids.dtype == torch.int64
+            and table.device == ids.device == weight.device and weight.dtype == table.dtype
+            and table.dtype in (torch.float32, torch.bfloat16, torch.float16)
+            and 0 < ids.numel() < 1 << 28 and 0 < table.shape[0] < 1 << 31 and table.shape[1] == weight.shape[0] < 1 << 20
+            and table.shape[1] % 8 == 0 and table.shape[1] > 0
+            and table.is_contiguous() and ids.is_contiguous() and weight.is_contiguous()
+            and table.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0):
+        return None
+    h = torch.empty(ids.numel(), table.shape[1], dtype=table.dtype, device=table.device)
+    y = torch.empty_like(h)
+    native.check(native.kernels().hds_embed_norm(native.dt(table), table.data_ptr(), ids.data_ptr(), weight.data_ptr(),
+                                                 h.data_ptr(), y.data_ptr(), ids.numel(), table.shape[1], table.shape[0],
+                                                 float(eps), native.stream()), "embed_norm")
+    return h, y
 
 
 class EmbeddingFunction(torch.autograd.Function):

@@ -21,6 +21,7 @@ _hlib = None
 _KERNEL_SIGS = {
     "hds_norm_fwd": "iii" + "p" * 8 + "ii" + "f" + "pi" + "s",
     "hds_gather_rows": "ppp" + "ill" + "s",
+    "hds_embed_norm": "i" + "p" * 5 + "iiif" + "s",
     "hds_norm_bwd_nparts": "i",
     "hds_norm_bwd_set_max_parts": "i",
     "hds_norm_bwd": "iii" + "p" * 9 + "i" + "pp" + "iii" + "s",
