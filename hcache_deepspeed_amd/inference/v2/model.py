@@ -418,7 +418,7 @@ class RaggedTransformer:
     def forward_decode_graph(self, batch, capture_latents=False):
         """Replay the decode step for ``batch.current_sequences`` sequences: the graph reads the step's token ids and
         metadata from the batch's device buffer (``RaggedBatchWrapper.finalize``), replays every layer's kernels with
-        one launch, and the logits are copied out. A graph of before that buffer grew keeps the old one, into which
+        one launch, and the LM head behind it writes the logits to memory of their own (``_DecodeGraph.result``). A graph of before that buffer grew keeps the old one, into which
         they are copied. The first step of a batch size runs the forward eagerly over the same buffers, for a size may
         come once; the second captures it.
 
@@ -442,7 +442,7 @@ class RaggedTransformer:
             if g.graph is None:
                 g.capture(self)
             g.graph.replay()
-            out = g.out.clone()
+            out = g.result(self)
         if g.ring is not None:
             g.ring.end_step()
         return out, view
@@ -460,11 +460,12 @@ class RaggedTransformer:
         return ev
 
     @torch.no_grad()
-    def forward(self, batch, capture_latents=True, sync_latents=True, sink=None):
+    def forward(self, batch, capture_latents=True, sync_latents=True, sink=None, head=True):
         """Returns (logits [n_seqs, V], latents host [L, T, H] or [L, T, 2*n_kv*D] or None). With
         ``sync_latents=False`` the host does not wait for the latent D2H copies: ``self.latent_event`` (HIP event on
         the copy stream) marks when the returned host tensor is complete. ``sink(layer, rows)``: latents go to it
-        instead of to host memory (the decode graph's device ring)."""
+        instead of to host memory (the decode graph's device ring). ``head`` False: in the place of the logits what the stock
+        unembedding's ``project`` makes them of."""
         spec = self.spec
         self._prep(batch)
         T = batch.current_tokens
@@ -539,7 +540,9 @@ class RaggedTransformer:
                 h = self._expert_parts(L, x2)
                 if h is None:
                     h = self._allreduce(self._mlp(L, x2))
-        if scaled:
+        if not head:
+            logits = h if scaled else self.unembed_mod.rows(h, residual, batch, self.final_w, self.final_b, spec.norm_eps)
+        elif scaled:
             logits = self.unembed_mod.project(h, self.lm_head, None, self.tp_group, self.vocab)
         else:
             logits = self.unembed_mod(h, residual, batch, self.lm_head, self.lm_head_b, self.final_w, self.final_b,
@@ -851,11 +854,20 @@ class _DecodeGraph:
         self.seen = False
         self.graph = None
         self.out = None
+        # The stock LM head is not in the graph, whose every step writes the same memory: the logits would be copied out of it
+        # (a launch, 3 to 4.5 us behind a chain of kernels)
+        self.whole = type(model).forward is not RaggedTransformer.forward or type(model.unembed_mod) is not RaggedUnembed
 
-    def forward(self, model):
+    def result(self, model):
+        """Logits of the step replayed last."""
+        if self.whole:
+            return self.out.clone()
+        return model.unembed_mod.project(self.out, model.lm_head, model.lm_head_b, model.tp_group, model.vocab)
+
+    def forward(self, model, **kw):
         """The step over the static inputs, launch by launch; its latents go to the ring's slot, which moves on."""
         cap = self.ring is not None
-        out, _ = model.forward(self.batch, capture_latents=cap, sink=self.ring.sink if cap else None)
+        out, _ = model.forward(self.batch, capture_latents=cap, sink=self.ring.sink if cap else None, **kw)
         if cap:
             self.ring.advance()
         return out
@@ -893,7 +905,7 @@ class _DecodeGraph:
             with torch.cuda.stream(side):
                 g.capture_begin(pool=model._graph_pool)
                 try:
-                    self.out = self.forward(model)
+                    self.out = self.forward(model, **({} if self.whole else {"head": False}))
                 finally:
                     g.capture_end()
         finally:

@@ -384,12 +384,15 @@ class RaggedUnembed(DSUnembedBase):
 
     def forward(self, hidden, residual, batch, lm_head, lm_head_b, final_w, final_b, norm_eps=1e-5, tp_group=None,
                 vocab=None):
+        return self.project(self.rows(hidden, residual, batch, final_w, final_b, norm_eps), lm_head, lm_head_b, tp_group, vocab)
+
+    def rows(self, hidden, residual, batch, final_w, final_b, norm_eps=1e-5):
+        """Each sequence's last token, normed."""
         idx = batch.last_token_idx
         is_ln = self._config.norm_type != "rms"
         if isinstance(hidden, ExpertSum):
             if final_w is not None and not is_ln and self._every_row(batch, residual):
-                hl, _ = experts_pre_norm(hidden, residual, final_w, norm_eps)
-                return self.project(hl, lm_head, lm_head_b, tp_group, vocab)
+                return experts_pre_norm(hidden, residual, final_w, norm_eps)[0]
             hidden = sum_experts(residual, hidden, residual.dtype)
         if self._every_row(batch, hidden):  # nothing to gather
             if final_w is None:
@@ -406,7 +409,7 @@ class RaggedUnembed(DSUnembedBase):
             hl, _ = layer_norm(hidden[idx], final_w, final_b, norm_eps, residual[idx])
         else:
             hl, _ = rms_norm(hidden[idx], final_w, norm_eps, residual[idx])
-        return self.project(hl, lm_head, lm_head_b, tp_group, vocab)
+        return hl
 
     @staticmethod
     def _every_row(batch, hidden):
