@@ -5,7 +5,8 @@ V=128256). Here :func:`fused_linear_cross_entropy` runs the LM-head GEMM in row 
 chunk the HIP kernel (csrc/kernels/xent.hip) computes loss + LSE and overwrites the logits with
 d(loss)/d(logits), then two GEMMs produce d(hidden) for the chunk and accumulate d(W) in fp32.
 The backward only scales those by the incoming grad -- the logits are never stored and never
-recomputed.
+recomputed. Of one short chunk the forward keeps d(logits) and hidden, transposed, and the backward makes
+d(W) from them with the factor in the product's epilogue (ops/gemm.py ``scaled_wgrad``).
 """
 import torch
 import torch.nn.functional as F
@@ -133,6 +134,7 @@ class _FusedLinearCEFn(torch.autograd.Function):
         want_dw = need_grad and weight.requires_grad
         dw = None  # fp32 accumulator: the first chunk's GEMM writes it (beta = 0), no zero-fill pass
         native_path = native.use_native(hidden)
+        ops = None  # of a weight gradient that the backward makes and scales in one
         wcache = {}  # the LM-head weight transposed once for every chunk's dgrad (NT layout)
         for s in range(0, T, chunk_rows):
             e = min(T, s + chunk_rows)
@@ -159,7 +161,12 @@ class _FusedLinearCEFn(torch.autograd.Function):
                     else:
                         torch.mm(dl, weight, out=dh[s:e])
                 if want_dw:
-                    if dl.is_cuda and _ADDMM_OUT_DTYPE[0] is not False and (
+                    if native_path and s == 0 and e == T and weight.dtype == torch.bfloat16:
+                        from .gemm import scaled_wgrad_operands
+                        ops = scaled_wgrad_operands(dl, hc)
+                    if ops is not None:
+                        pass
+                    elif dl.is_cuda and _ADDMM_OUT_DTYPE[0] is not False and (
                             _ADDMM_OUT_DTYPE[0] or _probe_addmm_out_dtype(dl.device)):
                         from .gemm import wgrad  # fp32 accumulator, layout chosen per shape (TN or NT)
                         if dw is None:
@@ -171,7 +178,7 @@ class _FusedLinearCEFn(torch.autograd.Function):
                         _addmm_f32_(dw, dl.t(), hc)
             del logits
         del wcache
-        ctx.save_for_backward(dh, dw)
+        ctx.save_for_backward(dh, dw, *(ops or (None, None)))
         ctx.wdtype = weight.dtype
         ctx.weight = weight  # the Parameter object: its gradient may be written in place (ZeRO)
         ctx.mark_non_differentiable(losses)
@@ -181,18 +188,25 @@ class _FusedLinearCEFn(torch.autograd.Function):
     def backward(ctx, dsum, _dlosses):
         # the loss is returned already summed, so the upstream gradient is one scalar that scales
         # the eagerly computed d(hidden) and d(W)
-        dh, dw = ctx.saved_tensors
+        dh, dw, dlt, ht = ctx.saved_tensors
         gh = (dh * dsum.to(dh.dtype)) if dh is not None else None
         gw = None
-        if dw is not None:
+        if dw is not None or dlt is not None:
             from ..runtime.zero.linear import write_weight_grad
             scale = dsum.float()
 
-            def put(out, accumulate):  # fp32 accumulator -> the bf16 gradient buffer (one pass)
-                _scaled_grad_(out, dw, scale, accumulate)
+            def put(out, accumulate):
+                if dw is not None:  # fp32 accumulator -> the bf16 gradient buffer (one pass)
+                    _scaled_grad_(out, dw, scale, accumulate)
+                    return
+                from .gemm import scaled_wgrad
+                if not scaled_wgrad(dlt, ht, scale, out, accumulate):
+                    _scaled_grad_(out, _mm_f32(dlt, ht.t()), scale, accumulate)
 
             if not write_weight_grad(ctx.weight, put):
-                gw = _scaled_grad_(torch.empty(dw.shape, dtype=ctx.wdtype, device=dw.device), dw, scale, False)
+                shape = dw.shape if dw is not None else (dlt.shape[0], ht.shape[0])
+                gw = torch.empty(shape, dtype=ctx.wdtype, device=dsum.device)
+                put(gw, False)
         return gh, gw, None, None, None, None
 
 

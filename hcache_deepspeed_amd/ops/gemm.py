@@ -83,18 +83,53 @@ def _pads(x):
             and x.data_ptr() % 16 == 0 and x.shape[0] > 0 and x.shape[1] > 0)
 
 
-def transpose2d_padded(x):
-    """[R, C] (unit last stride) -> [C, R rounded up to a multiple of 64], zeros behind the R columns, by the HIP kernel; None
+def transpose2d_padded(x, unit=64):
+    """[R, C] (unit last stride) -> [C, R rounded up to a multiple of ``unit``, 64 or a multiple of it], zeros behind the R columns, by the HIP kernel; None
     where it does not apply. Rows of a transpose that are no multiple of 16 bytes cost the GEMM its fast loads."""
     R, C = x.shape
     if not _pads(x):
         return None
-    out = torch.empty(C, -(-R // 64) * 64, dtype=x.dtype, device=x.device)
+    out = torch.empty(C, -(-R // unit) * unit, dtype=x.dtype, device=x.device)
     if out.data_ptr() % 128:
         return None
     native.check(native.kernels().hds_transpose_bf16_pad(x.data_ptr(), out.data_ptr(), R, C, x.stride(0), out.shape[1],
                                                          native.stream()), "transpose_bf16_pad")
     return out
+
+
+def scaled_wgrad_operands(dy, x):
+    """The operands (dy^T, x^T) with which ``scaled_wgrad`` makes scale * dy^T . x for a scale known later, or None: for wide
+    results and a short reduction. There the time is that of the results, which it writes once, in bf16; a library product into
+    32 bits, scaled by a pass of its own, moves five times the bytes. us, that -> here, transposes included, from 64 / 300 / 1,018 /
+    2,046 / 3,000 rows: [32000, 2048] 126 / 170 / 250 / 366 / 470 -> 70 / 106 / 185 / 317 / 446 (4,096 rows 580 / 581), [32000,
+    4096] 248 / 325 / 456 / 657 / 911 -> 122 / 177 / 319 / 547 / 760, [128256, 4096] 928 / 1,234 / 1,769 / 2,552 / 3,596 -> 445 /
+    676 / 1,217 / 2,096 / 2,927, [8192, 2048] 39 / 50 / 73 / 101 / 126 -> 28 / 37 / 55 / 89 / 122; into fewer columns the transposes
+    are a larger part: [32000, 768] 56 / 86 / 127 / 192 / 226 -> 43 / 62 / 115 / 200 / 272, [16384, 1024] 39 / 50 / 71 / 98 / 123
+    -> 28 / 39 / 63 / 116 / 153."""
+    if not (_pads(dy) and _pads(x) and dy.dim() == x.dim() == 2 and dy.shape[0] == x.shape[0] and dy.device == x.device):
+        return None
+    (T, N), K = dy.shape, x.shape[1]
+    if T > (SCALED_WGRAD_ROWS if K >= 2048 else 1100) or N % 256 or K % 256 or N * K < 1 << 24 or N > 1 << 24 or K > 1 << 20:
+        return None
+    a = transpose2d_padded(dy, 128)
+    b = transpose2d_padded(x, 128) if a is not None else None
+    return None if b is None else (a, b)
+
+
+SCALED_WGRAD_ROWS = 3000
+
+
+def scaled_wgrad(a, b, scale, out, accumulate=False):
+    """out (+)= scale * a . b^T for operands of ``scaled_wgrad_operands`` and ``scale`` a float32 scalar on the device. False, with
+    nothing written, for an ``out`` that the kernel does not take."""
+    (M, P), N = a.shape, b.shape[0]
+    if not (out.dtype == torch.bfloat16 and out.is_contiguous() and out.shape == (M, N) and out.data_ptr() % 8 == 0
+            and out.device == a.device == b.device == scale.device and scale.dtype == torch.float32 and scale.numel() == 1
+            and a.is_contiguous() and b.is_contiguous()):
+        return False
+    native.check(native.kernels().hds_gemm_nt_scaled(a.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, P, P, P, N,
+                                                     scale.data_ptr(), int(bool(accumulate)), native.stream()), "gemm_nt_scaled")
+    return True
 
 
 _WGRAD_LAYOUT = os.environ.get("HDS_WGRAD_LAYOUT", "auto")  # auto | direct | nt | direct_sk2 | nt_sk2

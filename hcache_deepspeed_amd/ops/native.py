@@ -141,6 +141,7 @@ _KERNEL_SIGS = {
     "hds_token_sort": "p" + "ii" + "s",
     "hds_gemm_nt_supported": "iiiiii",
     "hds_gemm_nt": "ppp" + "iiiiii" + "f" + "ii" + "s",
+    "hds_gemm_nt_scaled": "ppp" + "iiiiii" + "p" + "i" + "s",
     "hds_gemm_mxfp8_supported": "iiiiii",
     "hds_gemm_mxfp8": "ppppp" + "iiiiii" + "f" + "i" + "s",
     "hds_mx_quant": "ppp" + "l" + "i" + "l" + "s",
