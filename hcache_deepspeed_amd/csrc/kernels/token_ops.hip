@@ -162,6 +162,46 @@ __global__ __launch_bounds__(256) void embed_bwd_kernel(const T* __restrict__ dy
   }
 }
 
+// The same without sorting, for few ids: the workgroup of every position compares its id with all of them, 64 a wave, and goes on
+// where no earlier one is the same. What bounds short steps' sorts is their launches and a workgroup's passes over the digits.
+// Sort and kernel above -> this, rows of 2,048, launch by launch: 64 / 1,018 / 2,046 / 3,000 / 4,096 ids 29.9 / 35.3 / 40.2 /
+// 54.3 / 56.2 -> 11.0 / 8.8 / 9.5 / 17.0 / 26.6 us; beyond, the comparisons grow with the square.
+constexpr int kFewIds = 4096;
+
+template <typename T>
+__global__ __launch_bounds__(256) void embed_bwd_few_kernel(const T* __restrict__ dy, const int64_t* __restrict__ ids,
+                                                            T* __restrict__ grad, int n, int D, int64_t V, int64_t pad_idx) {
+  __shared__ uint64_t same[kFewIds / 64];
+  const int i = blockIdx.x, words = (n + 63) / 64, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t id = ids[i];
+  if (id == pad_idx || id < 0 || id >= V) return;
+#pragma unroll 4
+  for (int k = w; k < words; k += 4) {
+    const int j = 64 * k + lane;
+    const uint64_t m = __ballot(j < n && ids[min(j, n - 1)] == id);
+    if (lane == 0) same[k] = m;
+  }
+  __syncthreads();
+  for (int k = 0; k < i / 64; ++k)
+    if (same[k] != 0) return;
+  if (same[i / 64] & ((1ull << (i % 64)) - 1)) return;
+  T* g = grad + id * (int64_t)D;
+  for (int c = threadIdx.x * 8; c < D; c += 256 * 8) {
+    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, old[8];
+    Vec8<T>::load(g + c, old);
+    for (int k = i / 64; k < words; ++k)
+      for (uint64_t m = same[k]; m != 0; m &= m - 1) {
+        float v[8];
+        Vec8<T>::load(dy + (64 * k + __builtin_ctzll(m)) * (int64_t)D + c, v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] += v[e];
+      }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) old[e] += acc[e];
+    Vec8<T>::store(g + c, old);
+  }
+}
+
 #define HDS_TOK_DISPATCH(dtype, ...)                  \
   switch (dtype) {                                    \
     case kF32: { typedef float T; __VA_ARGS__; break; }    \
@@ -236,3 +276,15 @@ HDS_EXPORT int hds_embed_bwd(int dtype, const void* dy, const int64_t* sorted, c
                                              sorted, perm, (T*)grad, n, D, V, pad_idx));
   return (int)hipGetLastError();
 }
+
+// ids [n] as they come, of at most hds_embed_bwd_few_max()
+HDS_EXPORT int hds_embed_bwd_few(int dtype, const void* dy, const int64_t* ids, void* grad, int n, int D, int64_t V,
+                                 int64_t pad_idx, hipStream_t st) {
+  if (n <= 0) return 0;
+  if (D % 8 || n > kFewIds) return (int)hipErrorInvalidValue;
+  HDS_TOK_DISPATCH(dtype, hipLaunchKernelGGL(embed_bwd_few_kernel<T>, dim3(n), dim3(256), 0, st, (const T*)dy, ids, (T*)grad,
+                                             n, D, V, pad_idx));
+  return (int)hipGetLastError();
+}
+
+HDS_EXPORT int hds_embed_bwd_few_max() { return kFewIds; }

@@ -3,7 +3,7 @@
 The framework's default ``nn.Embedding`` backward sorts the ids, reduces duplicates into a DENSE [V, D]
 gradient (fill + compute_grad_weight + sum_and_scatter) and AccumulateGrad then adds that whole tensor into
 ``.grad`` -- for Llama-3 (V=128256, D=4096) three passes over 1 GB per micro-step. Here the ids are sorted
-once and one HIP workgroup per distinct id adds its tokens' rows straight into the parameter's gradient
+once (4,096 and fewer are compared with each other instead) and one HIP workgroup per distinct id adds its tokens' rows straight into the parameter's gradient
 buffer (the flat ZeRO buffer), touching only the rows that occur. Reference counterpart: the embedding of
 every model trained through ``deepspeed.initialize`` (the reference uses the framework kernel).
 
@@ -27,11 +27,16 @@ def embedding_grad_add_(grad, ids, dy, padding_idx=None):
     if native.use_native(grad) and D % 8 == 0 and dy.dtype == grad.dtype and \
             grad.dtype in (torch.float32, torch.bfloat16, torch.float16) and grad.is_contiguous():
         dy = dy.contiguous()
-        srt, perm = torch.sort(ids.to(torch.int64), stable=True)
         pad = -1 if padding_idx is None else int(padding_idx) % V
-        native.check(native.kernels().hds_embed_bwd(native.dt(grad), dy.data_ptr(), srt.data_ptr(), perm.data_ptr(),
-                                                    grad.data_ptr(), ids.numel(), D, V, pad, native.stream()),
-                     "embed_bwd")
+        lib = native.kernels()
+        if ids.numel() <= lib.hds_embed_bwd_few_max():
+            ids = ids.to(torch.int64).contiguous()
+            native.check(lib.hds_embed_bwd_few(native.dt(grad), dy.data_ptr(), ids.data_ptr(), grad.data_ptr(), ids.numel(), D,
+                                               V, pad, native.stream()), "embed_bwd_few")
+            return grad
+        srt, perm = torch.sort(ids.to(torch.int64), stable=True)
+        native.check(lib.hds_embed_bwd(native.dt(grad), dy.data_ptr(), srt.data_ptr(), perm.data_ptr(), grad.data_ptr(),
+                                       ids.numel(), D, V, pad, native.stream()), "embed_bwd")
         return grad
     if padding_idx is not None:
         keep = ids != (int(padding_idx) % V)

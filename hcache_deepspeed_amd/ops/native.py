@@ -153,6 +153,8 @@ _KERNEL_SIGS = {
     "hds_evoformer_bwd": "p" * 10 + "pp" + "i" + "ppp" + "iiiii" + "f" + "s",
     "hds_evoformer_pair_chunks": "iiii",
     "hds_evoformer_pair_staged": "iiiiii",
+    "hds_embed_bwd_few": "i" + "ppp" + "ii" + "ll" + "s",
+    "hds_embed_bwd_few_max": "",
     "hds_embed_bwd": "i" + "pppp" + "l" + "i" + "ll" + "s",
     "hds_slice_mask": "i" + "ppp" + "iiiii" + "s",
     "hds_grouped_gemm_max_tiles": "ii",
