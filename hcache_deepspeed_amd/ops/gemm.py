@@ -125,7 +125,7 @@ def scaled_wgrad(a, b, scale, out, accumulate=False):
     (M, P), N = a.shape, b.shape[0]
     if not (out.dtype == torch.bfloat16 and out.is_contiguous() and out.shape == (M, N) and out.data_ptr() % 8 == 0
             and out.device == a.device == b.device == scale.device and scale.dtype == torch.float32 and scale.numel() == 1
-            and a.is_contiguous() and b.is_contiguous()):
+            and a.is_contiguous() and b.is_contiguous() and (a.data_ptr() | b.data_ptr()) % 16 == 0):
         return False
     native.check(native.kernels().hds_gemm_nt_scaled(a.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, P, P, P, N,
                                                      scale.data_ptr(), int(bool(accumulate)), native.stream()), "gemm_nt_scaled")
