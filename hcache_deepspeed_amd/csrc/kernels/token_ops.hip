@@ -164,14 +164,17 @@ __global__ __launch_bounds__(256) void embed_bwd_kernel(const T* __restrict__ dy
 
 // The same without sorting, for few ids: the workgroup of every position compares its id with all of them, 64 a wave, and goes on
 // where no earlier one is the same. What bounds short steps' sorts is their launches and a workgroup's passes over the digits.
-// Sort and kernel above -> this, rows of 2,048, launch by launch: 64 / 1,018 / 2,046 / 3,000 / 4,096 ids 29.9 / 35.3 / 40.2 /
-// 54.3 / 56.2 -> 11.0 / 8.8 / 9.5 / 17.0 / 26.6 us; beyond, the comparisons grow with the square.
-constexpr int kFewIds = 4096;
+// Sort and kernel above -> this, rows of 2,048, launch by launch: 64 / 1,018 / 2,046 / 3,000 / 4,096 ids 30.0 / 35.1 / 41.1 /
+// 53.6 / 56.2 -> 8.6 / 9.6 / 9.2 / 13.6 / 21.0 us; beyond, the comparisons grow with the square. Rows of one id are added in their order,
+// kAtOnce of them on their way: 4,096 ids, half of them one 867 -> 279 (row by row 606), 1,018, three in ten 105 -> 30 (52).
+constexpr int kFewIds = 4096;  // (a lane for each 64)
+constexpr int kAtOnce = 8;     // rows on their way: an id of padding may be half of all
 
 template <typename T>
 __global__ __launch_bounds__(256) void embed_bwd_few_kernel(const T* __restrict__ dy, const int64_t* __restrict__ ids,
                                                             T* __restrict__ grad, int n, int D, int64_t V, int64_t pad_idx) {
   __shared__ uint64_t same[kFewIds / 64];
+  __shared__ uint16_t list[kFewIds];
   const int i = blockIdx.x, words = (n + 63) / 64, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t id = ids[i];
   if (id == pad_idx || id < 0 || id >= V) return;
@@ -182,20 +185,39 @@ __global__ __launch_bounds__(256) void embed_bwd_few_kernel(const T* __restrict_
     if (lane == 0) same[k] = m;
   }
   __syncthreads();
-  for (int k = 0; k < i / 64; ++k)
-    if (same[k] != 0) return;
-  if (same[i / 64] & ((1ull << (i % 64)) - 1)) return;
+  // every wave for itself, a lane a word: is an earlier position's id the same, how many are
+  uint64_t m = lane < words ? same[lane] : 0;
+  const uint64_t earlier = lane < i / 64 ? m : lane == i / 64 ? m & ((1ull << (i % 64)) - 1) : 0;
+  if (__any(earlier != 0)) return;
+  int upto = __popcll(m);
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(upto, o, 64);
+    if (lane >= o) upto += v;
+  }
+  const int count = __shfl(upto, 63, 64);
+  if (count > 1) {
+    if (w == 0)
+      for (int p = upto - __popcll(m); m != 0; m &= m - 1) list[p++] = (uint16_t)(64 * lane + __builtin_ctzll(m));
+    __syncthreads();
+  }
   T* g = grad + id * (int64_t)D;
   for (int c = threadIdx.x * 8; c < D; c += 256 * 8) {
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, old[8];
+    float acc[8], old[8];
     Vec8<T>::load(g + c, old);
-    for (int k = i / 64; k < words; ++k)
-      for (uint64_t m = same[k]; m != 0; m &= m - 1) {
-        float v[8];
-        Vec8<T>::load(dy + (64 * k + __builtin_ctzll(m)) * (int64_t)D + c, v);
+    Vec8<T>::load(dy + i * (int64_t)D + c, acc);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] += v[e];
-      }
+    for (int e = 0; e < 8; ++e) acc[e] += 0.f;
+    for (int p = 1; p < count; p += kAtOnce) {
+      float v[kAtOnce][8];
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u) Vec8<T>::load(dy + list[min(p + u, count - 1)] * (int64_t)D + c, v[u]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < kAtOnce; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] = p + u < count ? acc[e] + v[u][e] : acc[e];
+    }
 #pragma unroll
     for (int e = 0; e < 8; ++e) old[e] += acc[e];
     Vec8<T>::store(g + c, old);
