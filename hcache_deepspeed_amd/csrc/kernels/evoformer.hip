@@ -109,7 +109,7 @@ template <int D>
 struct Stager {
   using T = Tile<D>;
   static constexpr int PER = 1024 / T::RB;
-  uint32_t first, even, odd;  // of a lane: of the wave's first instruction; without its number, by the parity of the wave instruction's number: a tile's swizzle looks as far
+  uint32_t even, odd;  // of a lane, without the wave instruction's number, by that number's parity: a tile's swizzle looks as far
   int w, count, step;
   uint32_t bytes, stride;
   __device__ __forceinline__ Stager(int row0, int nt, int nw, int64_t ld, int L) {
@@ -121,20 +121,17 @@ struct Stager {
     bytes = (uint32_t)(L - 1) * 2 * (uint32_t)ld + 2 * D;
     even = 2 * (uint32_t)ld * (row0 + row) + 16 * ((lane % T::CH) ^ T::mix(row));
     odd = 2 * (uint32_t)ld * (row0 + row) + 16 * ((lane % T::CH) ^ T::mix(PER + row));
-    first = (w & 1 ? odd : even) + w * stride;
   }
+  // The whole distance goes into the vector offset: only that is held against the range, so that positions past the end are.
   // (one: of whole workgroups that move 1 KB a wave)
   __device__ __forceinline__ void stage(char* lds, const bf16* m, bool one) const {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)m, (short)0, bytes, 0x00020000);
     const uint32_t at[2] = {even, odd};
-    if (one) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(lds + w * 1024), 16, first, 0, 0, 0);
-      return;
-    }
     for (int i = w; i < count; i += step) {
       uint32_t voff = at[0];
       if (i & 1) voff = at[1];
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(lds + i * 1024), 16, voff, i * stride, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(lds + i * 1024), 16, voff + i * stride, 0, 0, 0);
+      if (one) break;
     }
   }
 };

@@ -286,3 +286,29 @@ def test_evoformer_walked_rows(cuda, B, N, L, H):
             (slice(None), slice(None), i, h) for i, h in ((5, 0), (6, 0), (7, 0), (8, H - 1))]:
         assert (x[part] - y[part]).norm() <= 4 * 2**-8 * y[part].norm()
     assert not x[:, 3].any() and not y[:, 3].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,L,H", [(520, 17, 8), (190, 97, 8), (66, 200, 8), (130, 240, 4), (66, 161, 8)])
+def test_evoformer_positions_past_the_end_are_not_read(cuda, N, L, H):
+    """Rows whose last tile of 32 is partial, with NaN in the rows behind: nothing of a neighbour comes into a row, and nothing
+    of what lies behind the last one into the pair bias' gradient."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    q, k, v, do = whole = [rnd(1, N + 1, L, H, 32).bfloat16() for _ in range(4)]
+    b1, b2 = torch.zeros(1, N, 1, 1, L, dtype=torch.bfloat16, device="cuda"), rnd(1, 1, H, L, L).bfloat16()
+
+    def call(rows):
+        q, k, v, do = (t[:, :N].detach() for t in rows)
+        assert q.is_contiguous()
+        leaves = [t.requires_grad_() for t in (q, k, v, b2.detach())]
+        out = DS4Sci_EvoformerAttention(*leaves[:3], [b1, leaves[3]])
+        return [out.detach()] + list(torch.autograd.grad(out, leaves, do))
+    clean = call(whole)
+    for t in whole:
+        t[:, N:] = math.nan
+    assert all(torch.equal(a, b) for a, b in zip(call(whole), clean))
+    for t in whole:
+        t[:, 1::2] = math.nan
+    for a, b in zip(call(whole)[:4], clean):
+        assert torch.equal(a[:, ::2], b[:, ::2])
