@@ -1459,7 +1459,7 @@ HDS_EXPORT int hds_evoformer_fwd(const void* q, const void* k, const void* v, co
   const int nt = (L + 31) / 32;
   const int64_t rows = (int64_t)B * N * H, slots = 256 * (8 / std::max(1, std::min(nt, 8)));
   if (bias_dtype == kBF16 && D == 32 && nt <= 8 && rows > 2 * slots && rows <= 64 * slots &&
-      (int64_t)L * H * D < (1 << 30)) {  // (offsets in 32 bits)
+      ((int64_t)L + 31) * H * D < (int64_t)1 << 31) {  // (Stager: offsets in 32 bits, of whole tiles)
     const int per = (int)((rows + slots - 1) / slots);  // workgroups that fill the chip once
     const dim3 grid(B * H * ((N + per - 1) / per)), threads(64 * nt);
     if (nt == 1) hipLaunchKernelGGL(evo_fwd_rows_kernel<1>, grid, threads, 0, st, p, per);
@@ -1497,7 +1497,7 @@ HDS_EXPORT int hds_evoformer_pair_chunks(int B, int N, int L, int H) {
 // heads 16.6 / 20.0, 64 x 128 19.4 / 18.3, 512 x 80, 8 heads 102 / 71, 512 x 160 232 / 213; 32-bit biases, D = 32, 512 x 192 264 /
 // 349, 512 x 256 333 / 294, D = 64, 418 / 440 and 524 / 330.
 HDS_EXPORT int hds_evoformer_pair_staged(int B, int N, int L, int H, int D, int bias_dtype) {
-  if (D == 128 || L <= 32 * kPairTiles) return 0;
+  if (D == 128 || L <= 32 * kPairTiles || ((int64_t)L + 127) * H * D >= (int64_t)1 << 31) return 0;  // (Stager: 32 bits, 128 rows)
   const int64_t q32 = (L + 31) / 32, k64 = (L + 32 * kPairTiles - 1) / (32 * kPairTiles);
   const int64_t waves = (int64_t)hds_evoformer_pair_chunks(B, N, L, H) * B * H * q32 * k64;
   if (bias_dtype != kBF16) return waves > 1024 && L % (64 * kPairTiles) == 0;

@@ -312,3 +312,12 @@ def test_evoformer_positions_past_the_end_are_not_read(cuda, N, L, H):
         t[:, 1::2] = math.nan
     for a, b in zip(call(whole)[:4], clean):
         assert torch.equal(a[:, ::2], b[:, ::2])
+
+
+@pytest.mark.parametrize("L,H,D,want", [(65, 174000, 64, 1), (65, 175000, 64, 0), (128, 263000, 32, 1), (128, 264000, 32, 0),
+                                        (300, 78000, 64, 1), (300, 79000, 64, 0), (100, 1 << 25, 64, 0)])
+def test_evoformer_staged_rows_have_offsets_in_32_bits(L, H, D, want):
+    """The pair bias' gradient by staged rows, whose distances are 32 bits, only where (L + 127) rows of H heads fit."""
+    from hcache_deepspeed_amd.ops import native
+    assert native.kernels().hds_evoformer_pair_staged(1, 4, L, H, D, 1) == want
+    assert want == (2 * (L + 127) * H * D < 1 << 32)
