@@ -606,6 +606,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
     const char* sk = smem + (n & 1) * W::kRow;
     const char* sv = sk + W::M;
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");  // (the barrier alone orders no access of the compiler's)
     bf16x8 qf[2] = {qn[0], qn[1]};
     if (n + 1 < n1) load(n + 1);
 
@@ -684,6 +685,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
     load(n);
     arrived();
     __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
     if (!(again >> (n - n0) & 1)) continue;
     const char* sk = smem + (n & 1) * W::kRow;
     bf16x8 qf[2] = {qn[0], qn[1]};
