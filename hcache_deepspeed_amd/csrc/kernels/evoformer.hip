@@ -509,7 +509,8 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_fwd_kernel(EvoParams p, in
 // keeps its 32 queries' as what the scores start from, in 32 bits (128 registers), instead of multiplying it in again. Scores
 // are q . k + bias / scale, a running maximum is raised only where a score exceeds it by 2^8, and exponents take one fused
 // operation (see far_off): 90 instructions a tile of 32 x 32, which is what bounds two waves a SIMD (about five cycles each,
-// whatever they are). Rows that this does not hold for are computed again as above.
+// whatever they are). Rows that this does not hold for are computed again as above: where one of the maxima met is far off, where no
+// key is visible, and where the sum is no number (biases of opposite signs that overflow over the whole scale).
 template <int NT>
 struct RowRing {
   static constexpr int M = 32 * NT * 64, kMask = 256 * ((NT + 1) / 2);  // bytes of K or V, of the mask (4 a key)
@@ -611,6 +612,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
     if (n + 1 < n1) load(n + 1);
 
     float m = -INFINITY, l = 0.f, ref = 0.f;
+    bool good = true;  // no reference so far is far off: beside one, keys seen later would count as anything
     f32x16 acc[1] = {};
     // C tiles at a time: their products, and what follows of each, lie in the other's shadow
     auto tiles = [&](auto count, int t0) {
@@ -644,6 +646,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
           const float alpha = fast_exp2((m - top) * mul);
           m = top;
           ref = m * mul;
+          good &= fabsf(ref) <= 256.f;
           l *= alpha;
           acc[0] *= alpha;
         }
@@ -668,7 +671,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
       if (t + 1 < NT && t + 1 < nt) tiles(std::integral_constant<int, (NT > 1 ? 2 : 1)>{}, t);
       else tiles(std::integral_constant<int, 1>{}, t);
     }
-    if (!__all(fabsf(ref) <= 256.f && m > -INFINITY)) again |= 1ull << (n - n0);
+    if (!__all(good && m > -INFINITY && l < INFINITY)) again |= 1ull << (n - n0);
     arrived();  // the next row's; what is stored here is on its way while that one is computed
     store(n, acc[0], ref, l);
   }

@@ -321,3 +321,83 @@ def test_evoformer_staged_rows_have_offsets_in_32_bits(L, H, D, want):
     from hcache_deepspeed_amd.ops import native
     assert native.kernels().hds_evoformer_pair_staged(1, 4, L, H, D, 1) == want
     assert want == (2 * (L + 127) * H * D < 1 << 32)
+
+
+def _walked(cuda, N, L, H, b1, b2, g):
+    """Inputs, result, normalisers and gradients of a call, against float64 in blocks of rows."""
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    q, k, v, do = (rnd(1, N, L, H, 32).bfloat16() for _ in range(4))
+    leaves = [t.requires_grad_() for t in (q, k, v, b2)]
+    out = DS4Sci_EvoformerAttention(q, k, v, [b1, b2])
+    got = [out] + list(torch.autograd.grad(out, leaves, do))
+    want = [torch.empty(t.shape, dtype=torch.float64, device=cuda) for t in got]
+    want[4].zero_()
+    for n in range(N):
+        qh, kh, vh = one = [t[:, n:n + 1].detach().double().requires_grad_() for t in (q, k, v)]
+        pair = b2.detach().double().requires_grad_()
+        s = qh.transpose(-2, -3) @ kh.transpose(-2, -3).transpose(-1, -2) / math.sqrt(32) + b1[:, n:n + 1].double() + pair
+        top = s.detach().amax(-1, keepdim=True)
+        p = torch.exp(s - torch.where(top.isinf(), 0., top))
+        ref = (p / p.sum(-1, keepdim=True).clamp_min(1e-300) @ vh.transpose(-2, -3)).transpose(-2, -3)
+        grads = torch.autograd.grad(ref, one + [pair], do[:, n:n + 1].double())
+        for w, x in zip(want, (ref, ) + grads[:3]):
+            w[:, n:n + 1] = x.detach()
+        want[4] += grads[3]
+    return got, want
+
+
+_LOWS = (-1e9, -2e10, -1e12, -1e15, -1e30, -1e35, -1e37, -3e37, -math.inf, torch.finfo(torch.bfloat16).min)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,L,H,where", [(66, 200, 8, "mask"), (66, 256, 8, "pair"), (190, 97, 8, "mask"), (190, 128, 8, "pair"),
+                                         (130, 161, 4, "mask"), (260, 64, 8, "mask"), (260, 40, 8, "pair")])
+def test_evoformer_walked_rows_leading_keys(cuda, N, L, H, where):
+    """Rows whose first one, two or four tiles of keys have a large negative bias of any size, in walking workgroups: later keys
+    have the weight. Against float64, with the bound of the edge tests, and each such row by itself."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    b1 = torch.zeros(1, N, 1, 1, L, dtype=torch.bfloat16, device="cuda")
+    b2 = torch.randn(1, 1, H, L, L, device="cuda", generator=g).bfloat16()
+    firsts = [f for f in (32, 64, 128) if f < L]
+    if where == "mask":
+        for i, low in enumerate(_LOWS):
+            for j, first in enumerate(firsts):
+                b1[:, 3 * i + j, ..., :first] = low
+    else:
+        for i, low in enumerate(_LOWS):
+            for j, first in enumerate(firsts):
+                b2[:, :, i % H, 3 * i + j, :first] = low
+    got, want = _walked(cuda, N, L, H, b1, b2, g)
+    for x, y in zip(got, want):
+        assert torch.isfinite(x).all()
+        assert (x.double() - y).norm() <= 4 * 2**-8 * y.norm() + 1e-6
+    x, y = got[0].double(), want[0]
+    rows = (range(3 * len(_LOWS)) if where == "mask" else [])
+    for part in [(slice(None), n) for n in rows] + [(slice(None), slice(None), n) for n in range(min(L, 3 * len(_LOWS)))]:
+        assert (x[part] - y[part]).norm() <= 4 * 2**-8 * y[part].norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [0.125, 0.249, 1.0, 3.0])
+@pytest.mark.parametrize("N,L,H", [(66, 200, 8), (190, 97, 8), (260, 64, 8)])
+def test_evoformer_walked_rows_of_a_scale(cuda, N, L, H, scale):
+    """The same of other scales than D^-0.5 through the kernels' entry: with scales of one and more the lowest value stays finite
+    over them. 32-bit scores of up to 20 (lse), the result rounded to bf16."""
+    from hcache_deepspeed_amd.ops import native
+    g = torch.Generator(device="cuda").manual_seed(L)
+    q, k, v = (torch.randn(1, N, L, H, 32, device="cuda", generator=g).bfloat16() for _ in range(3))
+    q /= 32**0.5 * scale
+    b1 = torch.zeros(1, N, 1, 1, L, device=cuda, dtype=torch.bfloat16)
+    for i, low in enumerate(_LOWS):
+        b1[:, 2 * i, ..., :32], b1[:, 2 * i + 1, ..., :L // 2] = low, low
+    b2 = torch.randn(1, 1, H, L, L, device=cuda, generator=g).bfloat16()
+    o, lse = torch.empty_like(q), torch.empty(1, N, H, L, device=cuda)
+    native.check(native.kernels().hds_evoformer_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), b1.data_ptr(), b2.data_ptr(), 1,
+                                                    o.data_ptr(), lse.data_ptr(), 1, N, L, H, 32, scale, native.stream()), "fwd")
+    scale = torch.tensor(scale, dtype=torch.float32).double().item()
+    for n in range(N):
+        a, b, e = (t[0, n].double().transpose(0, 1) for t in (q, k, v))
+        s = a @ b.transpose(1, 2) * scale + b1[0, n].double() + b2[0, 0].double()
+        ref = (torch.softmax(s, -1) @ e).transpose(0, 1)
+        assert (o[0, n].double() - ref).norm() <= 2 * 2**-8 * ref.norm()
+        assert (lse[0, n].double() - torch.logsumexp(s, -1)).abs().max() <= 1e-4
