@@ -401,3 +401,23 @@ def test_evoformer_walked_rows_of_a_scale(cuda, N, L, H, scale):
         ref = (torch.softmax(s, -1) @ e).transpose(0, 1)
         assert (o[0, n].double() - ref).norm() <= 2 * 2**-8 * ref.norm()
         assert (lse[0, n].double() - torch.logsumexp(s, -1)).abs().max() <= 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,L,H", [(128, 256, 8), (66, 200, 8), (190, 97, 8), (260, 64, 8), (520, 17, 8)])
+def test_evoformer_walked_rows_round_as_single_ones(cuda, N, L, H):
+    """The walking workgroups raise a row's maximum with every tile of 32 keys, as the general kernel does, so that the weights
+    are rounded alike: of its values (as those rows give them in calls of one row each) but for the rounding of 32-bit sums,
+    which turns few of the results' last bits."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    q, k, v = (torch.randn(1, N, L, H, 32, device="cuda", generator=g).bfloat16() for _ in range(3))
+    b1 = torch.where(torch.rand(1, N, 1, 1, L, device="cuda", generator=g) < 0.1, -1e9, 0.).bfloat16()
+    b2 = torch.randn(1, 1, H, L, L, device="cuda", generator=g).bfloat16()
+    with torch.no_grad():
+        out = DS4Sci_EvoformerAttention(q, k, v, [b1, b2])
+        for n in range(0, N, 7):
+            one = DS4Sci_EvoformerAttention(*(t[:, n:n + 1].contiguous() for t in (q, k, v, )), [b1[:, n:n + 1].contiguous(), b2])
+            a, b = out[:, n].double(), one[:, 0].double()
+            # a weight near the middle of two bf16 values may fall either way: 2^-8 of it. One in a hundred does (2^-24 of a
+            # sum's rounding against 2^-8 would be one in thousands); with a maximum raised less often all of them may
+            assert (a - b).norm() <= 0.1 * 2**-8 * b.norm()
