@@ -361,6 +361,18 @@ struct QueryBias<D, float> {
 // that factor could be anything, and the difference is taken first.
 __device__ __forceinline__ bool far_off(float ref) { return fabsf(ref) > 256.f && fabsf(ref) < INFINITY; }
 constexpr float kNone = -3e38f;  // the maximum of a row without a visible key so far, minus infinity but for its differences
+// A large positive bias (or a NaN) beside a large negative one may give a score near zero, which then depends on the order of
+// the sums, and overflow by itself over the whole scale: such ones, too, go the way of the rows far off
+constexpr int16_t kLarge = 0x4380;  // 256 in bf16
+__device__ __forceinline__ bool any_large(const u32x4& f) {
+  typedef int16_t s16x8 __attribute__((ext_vector_type(8)));
+  const s16x8 v = __builtin_bit_cast(s16x8, f);
+  bool large = false;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) large |= v[i] > kLarge;
+  return large;
+}
+__device__ __forceinline__ bool is_large(bf16 v) { return __builtin_bit_cast(int16_t, v) > kLarge; }
 
 struct EvoParams {
   const bf16 *q, *k, *v, *o, *dout;
@@ -511,8 +523,7 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_fwd_kernel(EvoParams p, in
 // are q . k + bias / scale, and exponents take one fused operation (see far_off). The maximum is raised with every tile, as above:
 // raised only where a score exceeds it by 2^8, the largest weight, too, is rounded to bf16 (error against 64 bits 0.00225 instead of
 // 0.00198; with every second tile 0.00200 and 2 us of 36 less). Rows that this does not hold for are computed again as above:
-// where one of the maxima met is far off, where no key is visible, and where the sum is no number (biases of opposite signs that
-// overflow over the whole scale).
+// where one of the maxima met is far off, where no key is visible or the sum is no number, and where a bias is large.
 template <int NT>
 struct RowRing {
   static constexpr int M = 32 * NT * 64, kMask = 256 * ((NT + 1) / 2);  // bytes of K or V, of the mask (4 a key)
@@ -565,6 +576,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
   bf16x8 inv = pieces<D>(Inverse<D>(p.rest));
   times<16>(inv, 1.f / p.power);
   QueryBias<D, bf16> bias = biases(n0);
+  bool fine = true;
   u32x4 pair[NT][2] = {};  // (all on their way at once)
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -578,6 +590,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
     if (t < nt) {
       if (p.b2 != nullptr) {
         bias.watch(pair[t]);
+        fine &= !any_large(pair[t][0]) && !any_large(pair[t][1]);
         pair[t][0] = finite(pair[t][0]);
         pair[t][1] = finite(pair[t][1]);
         start[t] = bias.add_pair(pair[t], start[t]) * (1.f / p.power);
@@ -614,7 +627,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
     if (n + 1 < n1) load(n + 1);
 
     float ref = kNone, l = 0.f;
-    bool good = true;  // no maximum so far is far off: beside one, keys seen later would count as anything
+    bool good = fine;  // no bias is large, no maximum so far is far off: beside one, keys seen later would count as anything
     f32x16 acc[1] = {};
     // C tiles at a time: their products, and what follows of each, lie in the other's shadow
     auto tiles = [&](auto count, int t0) {
@@ -625,6 +638,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
       for (int i = 0; i < C; ++i) {
         const bf16 v = p.b1 != nullptr ? *reinterpret_cast<const bf16*>(sv + W::M + 4 * (32 * (t0 + i) + j)) : (bf16)0.f;
         x[i] = mfma(spread<D>(v), inv, start[t0 + i]);
+        good &= !is_large(v);
       }
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks)
@@ -1241,7 +1255,7 @@ __global__ __launch_bounds__(512, 2) void evo_dpair_rows_kernel(EvoParams p, int
 #pragma unroll
     for (int r = 0; r < 16; ++r) sum[t][r] = 0.f;
 
-  // the pair bias and the rows' normalisers, on their way together
+  // the pair bias, the rows' normalisers and masks, on their way together
   u32x4 pair[kPairTiles][2] = {};
   if constexpr (sizeof(TB) == 2) {
 #pragma unroll
@@ -1257,15 +1271,25 @@ __global__ __launch_bounds__(512, 2) void evo_dpair_rows_kernel(EvoParams p, int
     for (int i = 0; i < 8; ++i) v[i] = (p.lse + (((int64_t)b * p.N + min(n + i, n1 - 1)) * p.H + h) * L)[(uint32_t)qc];
 #pragma unroll
     for (int i = 0; i < 8; ++i) far |= far_off(v[i] * kLog2e);
+    if constexpr (sizeof(TB) == 2)
+      if (p.b1 != nullptr) {
+        bf16 m[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          m[i] = ((const bf16*)p.b1 + ((int64_t)b * p.N + min(n + i, n1 - 1)) * L)[(uint32_t)min(kk0 + lane, L - 1)];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) far |= is_large(m[i]);
+      }
   }
-  far = __any(far);
   if constexpr (sizeof(TB) == 2) {
 #pragma unroll
     for (int t = 0; t < kPairTiles; ++t) {
+      far |= any_large(pair[t][0]) || any_large(pair[t][1]);
       pair[t][0] = finite(pair[t][0]);
       pair[t][1] = finite(pair[t][1]);
     }
   }
+  far = __any(far);
   auto walk = [&](auto tail, auto is_far) {
     constexpr bool TAIL = decltype(tail)::value, FAR = decltype(is_far)::value;
     // Near rows: scores are q . k + bias / scale, and a bias that overflows is one whose weight is zero. Far ones as elsewhere

@@ -421,3 +421,35 @@ def test_evoformer_walked_rows_round_as_single_ones(cuda, N, L, H):
             # a weight near the middle of two bf16 values may fall either way: 2^-8 of it. One in a hundred does (2^-24 of a
             # sum's rounding against 2^-8 would be one in thousands); with a maximum raised less often all of them may
             assert (a - b).norm() <= 0.1 * 2**-8 * b.norm()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,L,H", [(66, 200, 8), (190, 97, 8), (130, 256, 8), (260, 64, 8)])
+def test_evoformer_biases_of_opposite_signs(cuda, N, L, H):
+    """Large biases that take each other back to the scores' range. What the scores are then depends on the order of the sums, but
+    it is one order: a query's weights add up to one in the result, in dV and (dS to zero) in the pair bias' gradient."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    q, k, v, do = (rnd(1, N, L, H, 32).bfloat16() for _ in range(4))
+    b1, b2 = torch.zeros(1, N, 1, 1, L, dtype=torch.bfloat16, device="cuda"), rnd(1, 1, H, L, L).bfloat16()
+    sides = ((-1e9, 1e9), (-1e38, 1e38), (-2e37, 2e37), (1e9, -1e9), (1e38, -1e38), (5e4, -5e4), (-300, 300), (1e38, -math.inf))
+    for i, (mask, pair) in enumerate(sides):  # 32 queries of a head each, so that nothing else decides about them
+        b1[:, i, ..., 4:14] = mask
+        b2[:, :, i, :32, 4:14] = pair
+    keep = [do[0, i, :32, i].clone() for i in range(8)]
+    do.zero_()
+    for i in range(8):
+        do[0, i, :32, i] = keep[i]
+    leaves = [t.requires_grad_() for t in (q, k, v, b2)]
+    with torch.no_grad():
+        total = DS4Sci_EvoformerAttention(q, k, torch.ones_like(v), [b1, b2])
+    assert (total.double() - 1).abs().max() <= 2**-6  # (p and the result are rounded to bf16)
+    out = DS4Sci_EvoformerAttention(q, k, v, [b1, b2])
+    grads = torch.autograd.grad(out, leaves, do)
+    assert all(torch.isfinite(t).all() for t in (out, ) + grads)
+    for i, (mask, pair) in enumerate(sides):
+        # p and dV are rounded to bf16; from 1e37 on, in units of 1e30, the order of a product's own sums counts
+        dv, want = grads[2][0, i, :, i].double().sum(0), keep[i].double().sum(0)
+        assert pair > 1e10 or (dv - want).norm() <= 2 * 2**-8 * keep[i].double().norm(), (i, (dv - want).norm() / want.norm())
+        ds = grads[3][0, 0, i, :32].double()
+        assert (ds.sum(-1).abs() <= 2**-6 * ds.abs().sum(-1)).all()
