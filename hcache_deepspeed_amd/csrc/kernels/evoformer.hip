@@ -524,6 +524,8 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_fwd_kernel(EvoParams p, in
 // raised only where a score exceeds it by 2^8, the largest weight, too, is rounded to bf16 (error against 64 bits 0.00225 instead of
 // 0.00198; with every second tile 0.00200 and 2 us of 36 less). Rows that this does not hold for are computed again as above:
 // where one of the maxima met is far off, where no key is visible or the sum is no number, and where a bias is large.
+// A kernel for each count of tiles: in one for several, the way of a last single tile lay between those of the pairs (34 KB of
+// code instead of 20, and 13 registers in scratch memory).
 template <int NT>
 struct RowRing {
   static constexpr int M = 32 * NT * 64, kMask = 256 * ((NT + 1) / 2);  // bytes of K or V, of the mask (4 a key)
@@ -555,7 +557,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
                               p.b2 != nullptr ? (const bf16*)p.b2 + ((int64_t)(b * p.H + h) * L + q) * L : nullptr, rest);
   };
 
-  Stager<D> of_k(0, nt, nt, ld, L);
+  Stager<D> of_k(0, NT, NT, ld, L);
   const uint32_t mask_at = 2 * threadIdx.x, q_at = 2 * (qc * ld + 8 * hf);
   bf16x8 qn[2];
   auto load = [&](int n) {
@@ -565,7 +567,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
     for (int ks = 0; ks < 2; ++ks) qn[ks] = *reinterpret_cast<const bf16x8*>((const char*)(p.q + base) + (q_at + 32 * ks));
     of_k.stage(s, p.k + base, false);
     of_k.stage(s + W::M, p.v + base, false);
-    if (p.b1 != nullptr && w < (nt + 1) / 2)
+    if (p.b1 != nullptr && w < (NT + 1) / 2)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           __builtin_amdgcn_make_buffer_rsrc((void*)((const bf16*)p.b1 + bn * L), (short)0, 2 * L, 0x00020000),
           (lds_void*)(s + 2 * W::M + 256 * w), 2, mask_at, 0, 0, 0);
@@ -580,26 +582,25 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
   u32x4 pair[NT][2] = {};  // (all on their way at once)
 #pragma unroll
   for (int t = 0; t < NT; ++t)
-    if (t < nt && p.b2 != nullptr) {
-      if (32 * t + 32 <= L) bias.template load_pair<false>(32 * t, L, pair[t]);
+    if (p.b2 != nullptr) {
+      if (t + 1 < NT || 32 * NT == L) bias.template load_pair<false>(32 * t, L, pair[t]);
       else bias.template load_pair<true>(32 * t, L, pair[t]);
     }
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
+    __builtin_amdgcn_sched_barrier(0);  // (tile by tile, here and below: the scheduler would spill)
     start[t] = f32x16{};
-    if (t < nt) {
-      if (p.b2 != nullptr) {
-        bias.watch(pair[t]);
-        fine &= !any_large(pair[t][0]) && !any_large(pair[t][1]);
-        pair[t][0] = finite(pair[t][0]);
-        pair[t][1] = finite(pair[t][1]);
-        start[t] = bias.add_pair(pair[t], start[t]) * (1.f / p.power);
-      }
-      if (32 * t + 32 > L) {
+    if (p.b2 != nullptr) {
+      bias.watch(pair[t]);
+      fine &= !any_large(pair[t][0]) && !any_large(pair[t][1]);
+      pair[t][0] = finite(pair[t][0]);
+      pair[t][1] = finite(pair[t][1]);
+      start[t] = bias.add_pair(pair[t], start[t]) * (1.f / p.power);
+    }
+    if (t + 1 == NT) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r)
-          if (32 * t + acc_row(r, hf) >= L) start[t][r] = -INFINITY;
-      }
+      for (int r = 0; r < 16; ++r)
+        if (32 * t + acc_row(r, hf) >= L) start[t][r] = -INFINITY;
     }
   }
   const bool nan = bias.nan();
@@ -634,6 +635,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
       constexpr int C = decltype(count)::value;
       f32x16 x[C];
       bf16x8 vt[C][2];
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < C; ++i) {
         const bf16 v = p.b1 != nullptr ? *reinterpret_cast<const bf16*>(sv + W::M + 4 * (32 * (t0 + i) + j)) : (bf16)0.f;
@@ -674,8 +676,9 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
 #pragma unroll
     for (int t = 0; t < NT; t += 2) {
       if (t >= nt) break;
-      if (t + 1 < NT && t + 1 < nt) tiles(std::integral_constant<int, (NT > 1 ? 2 : 1)>{}, t);
-      else tiles(std::integral_constant<int, 1>{}, t);
+      if constexpr (NT > 1)
+        if (t + 1 < NT) tiles(std::integral_constant<int, 2>{}, t);
+      if (t + 1 == NT) tiles(std::integral_constant<int, 1>{}, t);
     }
     if (!__all(good && fabsf(ref) <= 256.f && l < INFINITY)) again |= 1ull << (n - n0);
     arrived();  // the next row's; what is stored here is on its way while that one is computed
@@ -687,7 +690,7 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
   if (lane == 0) s_again[w] = again;
   __syncthreads();
   uint64_t all = 0;
-  for (int i = 0; i < nt; ++i) all |= s_again[i];
+  for (int i = 0; i < NT; ++i) all |= s_again[i];
   for (int n = n0; n < n1; ++n) {
     if (!(all >> (n - n0) & 1)) continue;  // (the same for all waves)
     __syncthreads();
@@ -702,7 +705,8 @@ __global__ __launch_bounds__(64 * NT, 2) void evo_fwd_rows_kernel(EvoParams p, i
     float m = -INFINITY, l = 0.f;
     f32x16 acc[1] = {};
     QueryBias<D, bf16> rows = biases(n);
-    for (int t = 0; t < nt; ++t) evo_tile<D, true>(rows, sk, sk + W::M, 32 * t, 32 * t, hf, L, c, qf, acc, m, l);
+#pragma unroll 1
+    for (int t = 0; t < NT; ++t) evo_tile<D, true>(rows, sk, sk + W::M, 32 * t, 32 * t, hf, L, c, qf, acc, m, l);
     store(n, acc[0], m * c, l);
   }
 }
@@ -1290,8 +1294,9 @@ __global__ __launch_bounds__(512, 2) void evo_dpair_rows_kernel(EvoParams p, int
     }
   }
   far = __any(far);
-  auto walk = [&](auto tail, auto is_far) {
-    constexpr bool TAIL = decltype(tail)::value, FAR = decltype(is_far)::value;
+  auto walk = [&](auto is_far) {
+    // (32-bit biases: whole workgroups only. The others' tail is a choice a tile)
+    constexpr bool TAIL = sizeof(TB) == 2, FAR = decltype(is_far)::value;
     // Near rows: scores are q . k + bias / scale, and a bias that overflows is one whose weight is zero. Far ones as elsewhere
     constexpr bool kPlain = sizeof(TB) == 2 && !FAR;
     const float mul = kPlain ? p.scale * kLog2e : c;
@@ -1394,12 +1399,7 @@ __global__ __launch_bounds__(512, 2) void evo_dpair_rows_kernel(EvoParams p, int
       }
     }
   };
-  // the workgroup's tail is every wave's: they meet at barriers (with 32-bit biases there is none)
-  const bool whole = sizeof(TB) == 4 || ks0 + 32 * kPairTiles * nwk <= L;
-  if (whole && !far) walk(std::false_type{}, std::false_type{});
-  else if (whole) walk(std::false_type{}, std::true_type{});
-  else if (!far) walk(std::true_type{}, std::false_type{});
-  else walk(std::true_type{}, std::true_type{});
+  if (!far) walk(std::false_type{}); else walk(std::true_type{});  // (waves of either kind meet at the barriers, as many in both)
   if (!live || myq >= L) return;
   store_pair_sums(p.part + (((int64_t)chunk * p.B + b) * p.H + h) * L * L + (int64_t)myq * L, sum, kk0, hf, L);
 }
@@ -1483,10 +1483,19 @@ HDS_EXPORT int hds_evoformer_fwd(const void* q, const void* k, const void* v, co
       ((int64_t)L + 31) * H * D < (int64_t)1 << 31) {  // (Stager: offsets in 32 bits, of whole tiles)
     const int per = (int)((rows + slots - 1) / slots);  // workgroups that fill the chip once
     const dim3 grid(B * H * ((N + per - 1) / per)), threads(64 * nt);
-    if (nt == 1) hipLaunchKernelGGL(evo_fwd_rows_kernel<1>, grid, threads, 0, st, p, per);
-    else if (nt == 2) hipLaunchKernelGGL(evo_fwd_rows_kernel<2>, grid, threads, 0, st, p, per);
-    else if (nt <= 4) hipLaunchKernelGGL(evo_fwd_rows_kernel<4>, grid, threads, 0, st, p, per);
-    else hipLaunchKernelGGL(evo_fwd_rows_kernel<8>, grid, threads, 0, st, p, per);
+    switch (nt) {
+#define HDS_EVO_ROWS(NT) \
+  case NT: hipLaunchKernelGGL(evo_fwd_rows_kernel<NT>, grid, threads, 0, st, p, per); break
+      HDS_EVO_ROWS(1);
+      HDS_EVO_ROWS(2);
+      HDS_EVO_ROWS(3);
+      HDS_EVO_ROWS(4);
+      HDS_EVO_ROWS(5);
+      HDS_EVO_ROWS(6);
+      HDS_EVO_ROWS(7);
+      HDS_EVO_ROWS(8);
+#undef HDS_EVO_ROWS
+    }
     return hipGetLastError();
   }
   const int nw = waves_of(L, D == 128 ? kWaves<128> : kWaves<32>), blocks = (L + 32 * nw - 1) / (32 * nw);
