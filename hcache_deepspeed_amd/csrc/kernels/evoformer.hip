@@ -1461,6 +1461,32 @@ int waves_of(int L, int most) {
     if (D == 32) CALL(32, float); else if (D == 64) CALL(64, float); else CALL(128, float);                         \
   }
 
+// Rows that a forward workgroup of heads of 32 with bf16 biases walks over (evo_fwd_rows_kernel), 0: a workgroup a row. Where
+// there are more than two rows for each workgroup that the chip holds at once (slots) and an estimate is for it. A walk is one
+// batch b, so that few rows n make many short ones. In units of a row that is walked over: a workgroup costs its rows and 1 to 1.25 for
+// the pair bias, in whole rounds where one fills a CU; a workgroup a row costs 1.45 (1.35 with five tiles) a row and slot. Up to
+// 64 positions walking is the faster one throughout. us, a workgroup a row / walking, 8 heads, B x N: 256 positions 1 x 65 27.7 /
+// 26.6, 1 x 128 38.6 / 34.0, 1 x 256 70 / 56, 192 x 1 78.8 / 100.9, 96 x 2 58.2 / 65.4, 64 x 3 56.4 / 55.6, 48 x 4 55.3 / 63.0, 32 x 6 55.7 / 45.5,
+// 24 x 8 54.1 / 62.5; 128 positions 1 x 131 16.1 / 17.2, 1 x 192 19.8 / 18.8, 1 x 512 43.5 / 34.7, 384 x 1 38.1 / 47.1, 192 x 2 35.6 /
+// 37.1, 96 x 4 34.7 / 31.6; 154 positions 1 x 128 27.8 / 22.8; 64 positions 1 x 261 14.5 / 12.4, 768 x 1 35.1 / 28.1; 32, 1536 x 1 41.5 / 22.2.
+// (A row's bit in one word: no more than 64.)
+HDS_EXPORT int hds_evoformer_walk(int B, int N, int L, int H) {
+  const int64_t nt = (L + 31) / 32, heads = (int64_t)B * H, rows = heads * N;
+  if (B <= 0 || N <= 0 || L <= 0 || H <= 0 || nt > 8 || (L + 31) * (int64_t)H * 32 >= (int64_t)1 << 31)  // (Stager: 32 bits, whole tiles)
+    return 0;
+  const int64_t slots = 256 * (8 / nt), even = std::min<int64_t>(N, (rows + slots - 1) / slots);
+  if (rows <= 2 * slots || even > 64) return 0;
+  if (nt <= 2) return (int)even;
+  auto cost = [&](int64_t per) {
+    const float rounds = (float)(heads * ((N + per - 1) / per)) / (float)slots;
+    return std::max(1.f, nt > 4 ? std::ceil(rounds) : rounds) * ((float)per + (nt > 4 ? 1.25f : 1.f));
+  };
+  const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(N, slots / heads)), once = (N + chunks - 1) / chunks;
+  const int64_t per = once <= 64 && cost(once) < cost(even) ? once : even;
+  const float each = (float)rows / (float)slots;
+  return cost(per) < (nt == 5 ? 1.35f : 1.45f) * (nt > 4 ? std::ceil(each) : each) ? (int)per : 0;
+}
+
 // q/k/v/o [B, N, L, H, D] bf16, 16-byte aligned; b1 [B, N, 1, 1, L] or null; b2 [B, 1, H, L, L] or null (bias dtype: 1 =
 // bf16, 0 = fp32); lse [B, N, H, L] fp32 (natural log of the softmax normaliser of the scaled + biased scores). A query whose keys
 // are all masked by minus infinity gives zeros (and no gradients); its lse is plus infinity. scale > 0; with D = 64 and
@@ -1474,14 +1500,8 @@ HDS_EXPORT int hds_evoformer_fwd(const void* q, const void* k, const void* v, co
   p.q = (const bf16*)q; p.k = (const bf16*)k; p.v = (const bf16*)v; p.b1 = b1; p.b2 = b2; p.out = (bf16*)o; p.lse = lse;
   p.B = B; p.N = N; p.L = L; p.H = H;
   if (!set_scale(p, scale, bias_dtype, D)) return hipErrorInvalidValue;
-  // Workgroups that walk over three rows and more: us, a workgroup a row / walking, 8 heads: 256 positions, 48 / 65 / 112 / 128
-  // rows n 22.0 / 30.0 / 37.2 / 40.0 -> 22.9 / 28.3 / 35.0 / 36.3, 512 of 250 147 -> 111; of 128 positions, 130 / 256 16.7 / 25.5
-  // -> 16.5 / 21.8; 512 of 64 25.2 -> 17.8. (A row's bit in one word: no more than 64.)
-  const int nt = (L + 31) / 32;
-  const int64_t rows = (int64_t)B * N * H, slots = 256 * (8 / std::max(1, std::min(nt, 8)));
-  if (bias_dtype == kBF16 && D == 32 && nt <= 8 && rows > 2 * slots && rows <= 64 * slots &&
-      ((int64_t)L + 31) * H * D < (int64_t)1 << 31) {  // (Stager: offsets in 32 bits, of whole tiles)
-    const int per = (int)((rows + slots - 1) / slots);  // workgroups that fill the chip once
+  if (const int per = bias_dtype == kBF16 && D == 32 ? hds_evoformer_walk(B, N, L, H) : 0; per > 0) {
+    const int nt = (L + 31) / 32;
     const dim3 grid(B * H * ((N + per - 1) / per)), threads(64 * nt);
     switch (nt) {
 #define HDS_EVO_ROWS(NT) \

@@ -153,6 +153,7 @@ _KERNEL_SIGS = {
     "hds_evoformer_bwd": "p" * 10 + "pp" + "i" + "ppp" + "iiiii" + "f" + "s",
     "hds_evoformer_pair_chunks": "iiii",
     "hds_evoformer_pair_staged": "iiiiii",
+    "hds_evoformer_walk": "iiii",
     "hds_embed_bwd_few": "i" + "ppp" + "ii" + "ll" + "s",
     "hds_embed_bwd_few_max": "",
     "hds_embed_bwd": "i" + "pppp" + "l" + "i" + "ll" + "s",

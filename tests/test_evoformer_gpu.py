@@ -453,3 +453,40 @@ def test_evoformer_biases_of_opposite_signs(cuda, N, L, H):
         assert pair > 1e10 or (dv - want).norm() <= 2 * 2**-8 * keep[i].double().norm(), (i, (dv - want).norm() / want.norm())
         ds = grads[3][0, 0, i, :32].double()
         assert (ds.sum(-1).abs() <= 2**-6 * ds.abs().sum(-1)).all()
+
+
+@pytest.mark.parametrize("B,N,L,H,want", [
+    (1, 64, 256, 8, 0), (1, 65, 256, 8, 3), (1, 128, 256, 8, 4), (1, 2048, 256, 8, 64), (1, 2049, 256, 8, 0), (1, 128, 257, 8, 0),
+    (192, 1, 256, 8, 0), (96, 2, 200, 8, 0), (48, 4, 256, 8, 0), (24, 8, 256, 8, 0), (32, 6, 256, 8, 6), (16, 12, 250, 8, 6),
+    (1, 257, 256, 3, 4), (1, 512, 256, 3, 7), (384, 1, 128, 8, 0), (192, 2, 128, 8, 0), (96, 4, 128, 8, 4), (24, 16, 100, 8, 6),
+    (1, 131, 128, 8, 0), (1, 192, 128, 8, 3), (768, 1, 64, 8, 1), (1, 256, 64, 8, 0), (1, 257, 64, 8, 3), (1536, 1, 17, 8, 1)])
+def test_evoformer_rows_of_a_walk(B, N, L, H, want):
+    """Rows of a forward workgroup: as many as let the launch run in one round, and a workgroup a row where walks would be short
+    or a second round mostly empty."""
+    from hcache_deepspeed_amd.ops import native
+    assert native.kernels().hds_evoformer_walk(B, N, L, H) == want
+
+
+def test_evoformer_sizes_above_walk():
+    """The sizes of the tests of walking workgroups are theirs."""
+    from hcache_deepspeed_amd.ops import native
+    for N, L, H in [(66, 200, 8), (66, 256, 8), (66, 161, 8), (128, 256, 8), (130, 256, 8), (130, 240, 4), (130, 161, 4), (190, 97, 8),
+                    (190, 128, 8), (260, 64, 8), (260, 40, 8), (520, 17, 8)]:
+        assert native.kernels().hds_evoformer_walk(1, N, L, H) >= 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,N,L,H", [(40, 8, 250, 3), (32, 6, 200, 8), (700, 3, 40, 2), (96, 4, 100, 8), (2100, 1, 20, 2)])
+def test_evoformer_walks_in_many_batches(cuda, B, N, L, H):
+    """Walks that end with a batch, against the rows of some batches in calls of their own."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()  # noqa: E731
+    q, k, v = (rnd(B, N, L, H, 32) for _ in range(3))
+    b1 = torch.where(torch.rand(B, N, 1, 1, L, device="cuda", generator=g) < 0.1, -1e9, 0.).bfloat16()
+    b2 = rnd(B, 1, H, L, L)
+    with torch.no_grad():
+        out = DS4Sci_EvoformerAttention(q, k, v, [b1, b2])
+        for b in sorted({0, 1, B // 2, B - 1}):
+            one = DS4Sci_EvoformerAttention(*(t[b:b + 1] for t in (q, k, v)), [b1[b:b + 1], b2[b:b + 1]])
+            x, y = out[b].double(), one[0].double()
+            assert (x - y).norm() <= 0.1 * 2**-8 * y.norm()  # (as rows by themselves above)
