@@ -258,8 +258,8 @@ struct WmixOut {
 struct NormIn {
   bf16x4 res, gamma;
   __device__ __forceinline__ void load(const WmixOut& o, int tile, int row, int g) {
-    if (o.norm.res == nullptr) return;
     const int n = tile * 16 + 4 * g;
+    if (o.norm.res == nullptr || n >= o.N) return;  // (with two tiles a workgroup the last may not be there)
     res = *reinterpret_cast<const bf16x4*>(o.norm.res + (int64_t)min(row, o.M - 1) * o.N + n);
     gamma = *reinterpret_cast<const bf16x4*>(o.norm.gamma + n);
   }
@@ -277,7 +277,8 @@ __device__ __forceinline__ void wmix_store(f32x4 s, int tile, int row, int g, in
         o.C[(int64_t)row * o.N + n] = (bf16)(wmix_act((float)(bf16)s[i], o.act) * (float)(bf16)up);
     }
   } else if (o.norm.res != nullptr) {
-    store_normed(o.norm, o.C, (int64_t)row * o.N + tile * 16 + 4 * g, s, in.res, in.gamma, tile, lane, row < o.M);
+    if (tile * 16 < o.N)  // (whole tiles)
+      store_normed(o.norm, o.C, (int64_t)row * o.N + tile * 16 + 4 * g, s, in.res, in.gamma, tile, lane, row < o.M);
   } else if (row < o.M) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

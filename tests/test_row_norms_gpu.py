@@ -79,6 +79,30 @@ def test_norm_between_packed_products(cuda, fmt, M, K, N, out, act):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["fp6", "int8", "int4"])
+@pytest.mark.parametrize("M,K,N", [(9, 2048, 16384), (12, 2048, 16400), (16, 512, 16400), (16, 8320, 16400), (5, 4096, 16400), (16, 2048, 32784)])
+def test_norm_behind_packed_products_of_many_columns(cuda, fmt, M, K, N):
+    """Two tiles a workgroup, the last of them with one, whole lines and resident rows: every column once, nothing behind."""
+    from hcache_deepspeed_amd.ops import quantizer as q
+    g = torch.Generator(device="cuda").manual_seed(M * N)
+    res, gamma = _rows(g, M, N), (1 + 0.1 * torch.randn(N, device="cuda", generator=g)).bfloat16()
+    x, w = _rows(g, M, K), _rows(g, N, K, scale=K**-0.5)
+    packed, scales = q.quantize_minifloat(w, 128, 6, 2)[:2] if fmt == "fp6" else q.quantize(w, 128, int(fmt[3:]), True)[:2]
+    y, r = (torch.full((M + 1, N), 7.0, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    ssq = torch.full((N // 16 + 4, 16), 7.0, device="cuda")
+    plain = torch.empty(M, N, device="cuda", dtype=torch.bfloat16)
+    lib, end = native.kernels(), (K, 128, q._FMTS[fmt], 3, 0, native.stream())
+    native.check(lib.hds_wmix_norm(x.data_ptr(), packed.data_ptr(), scales.data_ptr(), y.data_ptr(), None, 0.0, res.data_ptr(),
+                                   gamma.data_ptr(), r.data_ptr(), ssq.data_ptr(), M, N, *end), "wmix_norm")
+    native.check(lib.hds_wmix_skinny(x.data_ptr(), packed.data_ptr(), scales.data_ptr(), None, plain.data_ptr(), M, N, *end), "wmix_skinny")
+    _, want = rms_norm(plain, gamma, EPS, res)
+    assert torch.equal(r[:M], want) and torch.equal(y[:M], (want.float() * gamma.float()).bfloat16())
+    parts = want.double().square().view(M, N // 16, 16).sum(-1).T
+    assert ((ssq[:N // 16, :M].double() - parts).abs() <= 16 * 2**-24 * parts).all()
+    assert (y[M] == 7).all() and (r[M] == 7).all() and (ssq[N // 16:] == 7).all()
+
+
+@pytest.mark.gpu
 def test_norm_rows_out_of_range(cuda):
     """Rows with an infinity or a NaN become NaN, as a norm's do; others beside them do not; an all-zero row stays zero."""
     g = torch.Generator(device="cuda").manual_seed(1)
