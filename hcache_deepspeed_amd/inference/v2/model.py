@@ -52,6 +52,12 @@ from .modules import (DSEmbeddingsConfig, DSLinearConfig, DSMoEConfig, DSNormCon
 from .modules.implementations import DSPreRMSNorm, GroupedGemmMoE, RaggedEmbedding, RaggedUnembed, _PackedWeight
 
 
+def _stock_module(m, *types):
+    """Is the module one of these types itself, with the type's own ``forward``? Registered ones that derive from it, and objects
+    that were given another, may compute something else."""
+    return type(m) in types and "forward" not in vars(m)
+
+
 class _Layer:
 
     def __init__(self):
@@ -325,13 +331,16 @@ class RaggedTransformer:
     def _embed(self, batch):
         return self.embed_mod(batch, self.embed, self.pos_embed)
 
+    def _stock(self, *names):
+        """Are these methods the ones of this class, neither a derived class's nor the object's own?"""
+        return all(getattr(getattr(self, n), "__func__", None) is getattr(RaggedTransformer, n) for n in names)
+
     def _embed_norm(self, batch, T):
         """The embedded rows and the first layer's norm of them, or None: a registered module that derives from the stock one may
         compute something else, and one row is normed by the product behind it."""
-        if (self.pos_embed is not None or not self.layers or type(self.embed_mod) is not RaggedEmbedding
-                or type(self.norm_mod) is not DSPreRMSNorm or self.layers[0]["ln1.b"] is not None
-                or self.layers[0]["ln1.w"] is None or self._fused_decode_ok(T)
-                or type(self)._embed is not RaggedTransformer._embed or type(self)._norm is not RaggedTransformer._norm):
+        if (self.pos_embed is not None or not self.layers or not _stock_module(self.embed_mod, RaggedEmbedding)
+                or not _stock_module(self.norm_mod, DSPreRMSNorm) or self.layers[0]["ln1.b"] is not None
+                or self.layers[0]["ln1.w"] is None or self._fused_decode_ok(T) or not self._stock("_embed", "_norm")):
             return None
         return norm_rows(self.embed, batch.input_ids, self.layers[0]["ln1.w"], self.spec.norm_eps)
 
@@ -372,22 +381,25 @@ class RaggedTransformer:
     def _scaled_rows_ok(self, batch, T, capture):
         """Decode steps of 2 to 16 sequences of a plain pre-RMSNorm, gated dense model whose normed rows nobody else reads: the
         products add the residual and make the norms' sums (ops/gemv.py ``ScaledRows``), so that a layer launches no norm.
-        Registered modules that derive from the stock ones may compute something else."""
+        Modules and models that derive from the stock ones may compute something else."""
         if not scaled_rows_ok(T) or (capture and self.latent_mode != "kv"):
+            return False
+        from .modules.implementations import (BlasFPLinear, DSDenseBlockedAttention, QuantizedIntLinear, QuantizedWf6Af16Linear,
+                                              RaggedUnembed)
+        if not (self._stock("_attn", "_attend", "_mlp", "_norm", "_allreduce", "_expert_parts")
+                and _stock_module(self.norm_mod, DSPreRMSNorm) and _stock_module(self.unembed_mod, RaggedUnembed)
+                and _stock_module(self.attn_mod, DSDenseBlockedAttention)
+                and all(_stock_module(m, BlasFPLinear, QuantizedIntLinear, QuantizedWf6Af16Linear)
+                        for m in (self.qkv_lin, self.o_lin) + ((self.up_lin, self.down_lin) if self.spec.moe is None else ()))):
             return False
         known = getattr(self, "_scaled_sizes", None)
         if known is None:
             known = self._scaled_sizes = {}
         ok = known.get(T)
         if ok is None:
-            from .modules.implementations import (BlasFPLinear, DSPreRMSNorm, QuantizedIntLinear, QuantizedWf6Af16Linear,
-                                                  RaggedUnembed)
             ok = (bool(self.layers) and self.spec.moe is None and self.device.type == "cuda" and self.dtype == torch.bfloat16
                   and self.tp == 1 and self.spec.gated and self.spec.parallel not in ("shared_ln", "two_ln")
                   and self._act_name() in ("silu", "gelu_tanh", "relu")
-                  and type(self.norm_mod) is DSPreRMSNorm and type(self.unembed_mod) is RaggedUnembed
-                  and all(type(m) in (BlasFPLinear, QuantizedIntLinear, QuantizedWf6Af16Linear)
-                          for m in (self.qkv_lin, self.o_lin, self.up_lin, self.down_lin))
                   and all(L[k] is None for L in self.layers for k in ("ln1.b", "ln2.b", "qkv.b", "o.b", "up.b", "down.b"))
                   and all(self.qkv_lin.rows_ok(T, L["qkv.w"]) and self.o_lin.rows_ok(T, L["o.w"], True)
                           and self.up_lin.rows_ok(T, L["up.w"]) and self.down_lin.rows_ok(T, L["down.w"], True) for L in self.layers)
@@ -856,7 +868,7 @@ class _DecodeGraph:
         self.out = None
         # The stock LM head is not in the graph, whose every step writes the same memory: the logits would be copied out of it
         # (a launch, 3 to 4.5 us behind a chain of kernels)
-        self.whole = type(model).forward is not RaggedTransformer.forward or type(model.unembed_mod) is not RaggedUnembed
+        self.whole = not (model._stock("forward") and _stock_module(model.unembed_mod, RaggedUnembed))
 
     def result(self, model):
         """Logits of the step replayed last."""

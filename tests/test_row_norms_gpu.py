@@ -167,3 +167,60 @@ def test_decode_steps_without_norm_launches(cuda, monkeypatch, seqs, vocab, quan
     assert torch.equal(sides[0][0], sides[1][0])
     for a, b in zip(*(s[1:] for s in sides)):
         assert (a.double() - b.double()).norm() <= 0.02 * b.double().norm()
+
+
+def _small_engine(g, layers=2):
+    from hcache_deepspeed_amd.inference.v2.arch import ArchSpec
+    from hcache_deepspeed_amd.inference.v2.engine import InferenceEngineV2, RaggedInferenceEngineConfig
+    W, ff, nq, nkv, vocab = 256, 384, 2, 1, 512
+    sd = {"embed": _rows(g, vocab, W), "final.w": 1 + _rows(g, W, scale=0.1), "lm_head.w": _rows(g, vocab, W, scale=1 / 16), "layers": [
+        {"ln1.w": 1 + _rows(g, W, scale=0.1), "ln2.w": 1 + _rows(g, W, scale=0.1), "qkv.w": _rows(g, (nq + 2 * nkv) * 128, W, scale=1 / 16),
+         "o.w": _rows(g, W, nq * 128, scale=1 / 16), "up.w": _rows(g, 2 * ff, W, scale=1 / 16), "down.w": _rows(g, W, ff, scale=0.05)}
+        for _ in range(layers)]}
+    spec = ArchSpec("llama", vocab, W, layers, nq, nkv, 128, ff, norm_eps=EPS, rope_theta=10000.0, max_position_embeddings=512)
+    conf = RaggedInferenceEngineConfig.from_dict(dict(dtype="bf16", state_manager=dict(
+        max_context=256, max_ragged_batch_size=1024, max_tracked_sequences=16, kv_block_size=64)))
+    return InferenceEngineV2(spec, sd, conf, device=torch.device("cuda", 0), num_kv_blocks=32)
+
+
+def _steps(eng, seqs, first=0, steps=3):
+    """Logits of a prompt each and some decode steps: launched, captured and replayed ones."""
+    gen = torch.Generator().manual_seed(3)
+    uids = list(range(first, first + seqs))
+    out = [eng.put(uids, [torch.randint(0, 512, (5 + 3 * u, ), generator=gen) for u in range(seqs)], capture_latents=False)[0].clone()]
+    for _ in range(steps):
+        out.append(eng.put(uids, [torch.randint(0, 512, (1, ), generator=gen) for _ in uids], capture_latents=False)[0].clone())
+    return torch.stack(out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what", ["_mlp", "_attn", "_norm", "_allreduce", "own", "attention", "norm", "head"])
+def test_decode_steps_of_models_of_their_own(cuda, monkeypatch, what):
+    """What a derived model, an object or a registered attention has in the place of a stock part is what decode steps compute."""
+    from hcache_deepspeed_amd.inference.v2 import model as v2
+    from hcache_deepspeed_amd.inference.v2.modules.implementations import DSDenseBlockedAttention
+    sides = []
+    for off in (False, True):
+        if off:
+            monkeypatch.setattr(v2, "scaled_rows_ok", lambda m: False)
+        eng = _small_engine(torch.Generator(device="cuda").manual_seed(5))
+        m = eng._model
+        if what == "attention":
+            class Spread(DSDenseBlockedAttention):  # rows that are no plain matrix
+                def forward(self, *a):
+                    return torch.cat([super().forward(*a)] * 2, 1)[:, ::2].mul(2)
+            m.attn_mod = Spread(m.attn_mod._config)
+        elif what == "own":
+            plain = m._mlp
+            m._mlp = lambda L, x: plain(L, x) * 2
+        elif what in ("norm", "head"):  # an object's own
+            mod = m.norm_mod if what == "norm" else m.unembed_mod
+            plain = mod.forward
+            mod.forward = (lambda *a: tuple(t * 2 for t in plain(*a))) if what == "norm" else (lambda *a: plain(*a) + 1)
+        else:
+            def double(self, *a, **kw):
+                y = getattr(v2.RaggedTransformer, what)(self, *a, **kw)
+                return (y[0] * 2, y[1]) if isinstance(y, tuple) else y * 2
+            m.__class__ = type("Own", (v2.RaggedTransformer, ), {what: double})
+        sides.append(_steps(eng, 3))
+    assert torch.equal(*sides)
