@@ -378,38 +378,42 @@ class RaggedTransformer:
         # slower than the separate RMSNorm kernel (732 vs 773 tok/s); at B = 1: 247 vs 234 (profiles/r6/fused_decode/)
         return ok and T == 1
 
-    def _scaled_rows_ok(self, batch, T, capture):
+    def _scaled_rows_ok(self, batch, T, capture, rows):
         """Decode steps of 2 to 16 sequences of a plain pre-RMSNorm, gated dense model whose normed rows nobody else reads: the
         products add the residual and make the norms' sums (ops/gemv.py ``ScaledRows``), so that a layer launches no norm.
-        Modules and models that derive from the stock ones may compute something else."""
+        Modules and models that derive from the stock ones may compute something else. ``rows``: the embedded ones.
+        Asked of the weights as they are, at every step that is launched (a replayed one was asked when it was captured)."""
         if not scaled_rows_ok(T) or (capture and self.latent_mode != "kv"):
             return False
         from .modules.implementations import (BlasFPLinear, DSDenseBlockedAttention, QuantizedIntLinear, QuantizedWf6Af16Linear,
                                               RaggedUnembed)
-        if not (self._stock("_attn", "_attend", "_mlp", "_norm", "_allreduce", "_expert_parts")
+        spec, head = self.spec, self.lm_head
+        if not (self.device.type == "cuda" and self.dtype == torch.bfloat16 and self.tp == 1 and spec.moe is None and spec.gated
+                and spec.parallel not in ("shared_ln", "two_ln") and self._act_name() in ("silu", "gelu_tanh", "relu")
+                and self.layers and self._stock("_attn", "_attend", "_mlp", "_norm", "_allreduce", "_expert_parts")
                 and _stock_module(self.norm_mod, DSPreRMSNorm) and _stock_module(self.unembed_mod, RaggedUnembed)
                 and _stock_module(self.attn_mod, DSDenseBlockedAttention)
                 and all(_stock_module(m, BlasFPLinear, QuantizedIntLinear, QuantizedWf6Af16Linear)
-                        for m in (self.qkv_lin, self.o_lin) + ((self.up_lin, self.down_lin) if self.spec.moe is None else ()))):
+                        for m in (self.qkv_lin, self.o_lin, self.up_lin, self.down_lin))):
             return False
-        known = getattr(self, "_scaled_sizes", None)
-        if known is None:
-            known = self._scaled_sizes = {}
-        ok = known.get(T)
-        if ok is None:
-            ok = (bool(self.layers) and self.spec.moe is None and self.device.type == "cuda" and self.dtype == torch.bfloat16
-                  and self.tp == 1 and self.spec.gated and self.spec.parallel not in ("shared_ln", "two_ln")
-                  and self._act_name() in ("silu", "gelu_tanh", "relu")
-                  and all(L[k] is None for L in self.layers for k in ("ln1.b", "ln2.b", "qkv.b", "o.b", "up.b", "down.b"))
-                  and all(self.qkv_lin.rows_ok(T, L["qkv.w"]) and self.o_lin.rows_ok(T, L["o.w"], True)
-                          and self.up_lin.rows_ok(T, L["up.w"]) and self.down_lin.rows_ok(T, L["down.w"], True) for L in self.layers)
-                  and scaled_weight_ok(self.lm_head) and self.lm_head_b is None and self.final_b is None
-                  and all(torch.is_tensor(g) and g.dtype == torch.bfloat16 and g.is_contiguous()
-                          for g in [self.final_w] + [L[k] for L in self.layers for k in ("ln1.w", "ln2.w")]))
-            known[T] = ok
-        return (ok and getattr(batch, "logits_of_last_tokens", False) and getattr(batch, "max_new", 0) == 1
-                and T == batch.current_sequences == batch.last_token_idx.shape[0]
-                and torch.cuda.current_device() == self.lm_head.get_device())
+        if not (getattr(batch, "logits_of_last_tokens", False) and getattr(batch, "max_new", 0) == 1
+                and T == batch.current_sequences == batch.last_token_idx.shape[0] and scaled_weight_ok(head)
+                and self.lm_head_b is None and self.final_b is None and torch.cuda.current_device() == head.get_device()):
+            return False
+        W = head.shape[1]
+
+        def plain(t, *shape):  # contiguous rows that 16-byte reads may begin
+            return (torch.is_tensor(t) and t.dtype == torch.bfloat16 and t.shape == shape and t.device == head.device
+                    and t.is_contiguous() and t.data_ptr() % 16 == 0)
+        if not (plain(rows, T, W) and plain(self.final_w, W)):
+            return False
+        for L in self.layers:
+            if not (all(L[k] is None for k in ("ln1.b", "ln2.b", "qkv.b", "o.b", "up.b", "down.b"))
+                    and plain(L["ln1.w"], W) and plain(L["ln2.w"], W)
+                    and self.qkv_lin.rows_ok(T, L["qkv.w"]) and self.o_lin.rows_ok(T, L["o.w"], True)
+                    and self.up_lin.rows_ok(T, L["up.w"]) and self.down_lin.rows_ok(T, L["down.w"], True)):
+                return False
+        return True
 
     # ------------------------------------------------------------------------------------------
     def decode_graph_eligible(self, batch, capture_latents):
@@ -516,7 +520,7 @@ class RaggedTransformer:
                 h = self.down_lin(g, L["down.w"], L["down.b"])
             if stage is not None:
                 ring.flush_stage()  # every layer's latent rows into the ring slot, one store
-        scaled = self._scaled_rows_ok(batch, T, capture_latents)
+        scaled = self._scaled_rows_ok(batch, T, capture_latents, h)
         for i, L in (enumerate(self.layers) if not self._fused_decode_ok(T) else ()):
             if residual is None:
                 x = self._norm(h, L["ln1.w"], L["ln1.b"]) if first is None else first[1]

@@ -224,3 +224,23 @@ def test_decode_steps_of_models_of_their_own(cuda, monkeypatch, what):
             m.__class__ = type("Own", (v2.RaggedTransformer, ), {what: double})
         sides.append(_steps(eng, 3))
     assert torch.equal(*sides)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("key", ["qkv.w", "o.w", "up.w", "down.w", "ln2.w"])
+def test_decode_steps_after_an_exchange_of_weights(cuda, key):
+    """Weights of another layout or alignment that come in the place of others, for a batch size that has decoded before too: the
+    same values, the same logits to the rounding of bf16 layers."""
+    eng = _small_engine(torch.Generator(device="cuda").manual_seed(5))
+    eng._model.decode_graph_max_batch = 0  # (a graph keeps the weights that it was captured with)
+    want = _steps(eng, 3)
+    for u in range(3):
+        eng.flush(u)
+    for L in eng._model.layers:
+        w = L.w[key]
+        if w.dim() == 2:
+            L.w[key] = w.t().contiguous().t()
+        else:  # two bytes from where rows of 16 begin
+            L.w[key] = torch.cat([w[:1], w])[1:]
+    got = _steps(eng, 3)
+    assert (got.double() - want.double()).norm() <= 0.02 * want.double().norm()
