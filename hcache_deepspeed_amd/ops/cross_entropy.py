@@ -162,8 +162,8 @@ class _FusedLinearCEFn(torch.autograd.Function):
                         torch.mm(dl, weight, out=dh[s:e])
                 if want_dw:
                     if native_path and s == 0 and e == T and weight.dtype == torch.bfloat16:
-                        from .gemm import scaled_wgrad_operands
-                        ops = scaled_wgrad_operands(dl, hc)
+                        from .gemm import scaled_wgrad_gains, scaled_wgrad_operands
+                        ops = scaled_wgrad_operands(dl, hc) if scaled_wgrad_gains(T, H) else None
                     if ops is not None:
                         pass
                     elif dl.is_cuda and _ADDMM_OUT_DTYPE[0] is not False and (

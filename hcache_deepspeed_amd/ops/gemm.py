@@ -103,9 +103,8 @@ def scaled_wgrad_operands(dy, x):
     32 bits, scaled by a pass of its own, moves five times the bytes. us, that -> here, transposes included, from 64 / 300 / 1,018 /
     2,046 / 3,000 rows: [32000, 2048] 126 / 170 / 250 / 366 / 470 -> 70 / 106 / 185 / 317 / 446 (4,096 rows 580 / 581), [32000,
     4096] 248 / 325 / 456 / 657 / 911 -> 122 / 177 / 319 / 547 / 760, [128256, 4096] 928 / 1,234 / 1,769 / 2,552 / 3,596 -> 445 /
-    676 / 1,217 / 2,096 / 2,927, [8192, 2048] 39 / 50 / 73 / 101 / 126 -> 28 / 37 / 55 / 89 / 122; into fewer columns the transposes
-    are a larger part: [32000, 768] 56 / 86 / 127 / 192 / 226 -> 43 / 62 / 115 / 200 / 272, [16384, 1024] 39 / 50 / 71 / 98 / 123
-    -> 28 / 39 / 63 / 116 / 153."""
+    676 / 1,217 / 2,096 / 2,927, [8192, 2048] 39 / 50 / 73 / 101 / 126 -> 28 / 37 / 55 / 89 / 122. ``scaled_wgrad_gains`` says where
+    it is the faster way."""
     if not (_pads(dy) and _pads(x) and dy.dim() == x.dim() == 2 and dy.shape[0] == x.shape[0] and dy.device == x.device):
         return None
     (T, N), K = dy.shape, x.shape[1]
@@ -117,6 +116,14 @@ def scaled_wgrad_operands(dy, x):
 
 
 SCALED_WGRAD_ROWS = 3000
+
+
+def scaled_wgrad_gains(T, K):
+    """Is ``scaled_wgrad`` the faster way for a product of T rows with K columns? Into few columns the transposes are a larger part:
+    us, product and scaling apart -> here, 200 / 509 / 800 / 1,018 rows: [65536, 256] 44 / 55 / 58 / 70 -> 39 / 62 / 90 / 102,
+    [32768, 512] 45 / 53 / 56 / 67 -> 36 / 41 / 63 / 73, [32000, 768] 76 / 85 / 83 / 109 -> 49 / 63 / 92 / 103, [16384, 1024] 44 /
+    53 / 54 / 65 -> 30 / 40 / 48 / 52 (2,046 98 / 116), [32000, 1536] 110 / 144 / 150 / 185 -> 69 / 95 / 131 / 143."""
+    return T <= (SCALED_WGRAD_ROWS if K >= 2048 else 1100 if K >= 1024 else 640 if K >= 512 else 256)
 
 
 def scaled_wgrad(a, b, scale, out, accumulate=False):

@@ -72,3 +72,24 @@ def test_loss_and_gradients(T):
     # both from the same rounded logits and their gradients (2^-9 each), once rounded
     assert e[0] < 0.01 and e[0] < 1.05 * e[1], e
     assert torch.allclose(one[0], two[0], rtol=1e-5) and (one[1].float() - two[1].float()).norm() < 0.01 * two[1].float().norm()
+
+
+@pytest.mark.parametrize("T,V,H,want", [(200, 65536, 256, True), (257, 65536, 256, False), (640, 32768, 512, True), (641, 32768, 512, False),
+                                        (1100, 16384, 1024, True), (1101, 16384, 1024, False), (1101, 8192, 2048, True)])
+def test_short_heads_are_left_where_their_transposes_cost_more(cuda, monkeypatch, T, V, H, want):
+    """Which way the LM head's gradient is made, by its columns; the same gradient either way."""
+    from hcache_deepspeed_amd.ops import gemm
+    g = torch.Generator(device="cuda").manual_seed(T)
+    h = torch.randn(T, H, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(V, H, device="cuda", generator=g) * H**-0.5).bfloat16().requires_grad_()
+    ids = torch.randint(0, V, (T, ), device="cuda", generator=g)
+    calls, plain, grads = [], gemm.scaled_wgrad, []
+    monkeypatch.setattr(gemm, "scaled_wgrad", lambda *a: calls.append(1) or plain(*a))
+    for off in (False, True):
+        if off:
+            monkeypatch.setattr(gemm, "scaled_wgrad_operands", lambda *a: None)
+        loss = fused_linear_cross_entropy(h, w, ids)
+        grads.append(torch.autograd.grad(loss, w)[0].double())
+        assert bool(calls) == (want and not off)
+        calls.clear()
+    assert (grads[0] - grads[1]).norm() <= 2**-8 * grads[1].norm()
