@@ -109,7 +109,7 @@ template <int D>
 struct Stager {
   using T = Tile<D>;
   static constexpr int PER = 1024 / T::RB;
-  uint32_t even, odd;  // of a lane, without the wave instruction's number, by that number's parity: a tile's swizzle looks as far
+  uint32_t first, even, odd;  // of a lane: of the wave's first instruction; without its number, by that number's parity: a tile's swizzle looks as far
   int w, count, step;
   uint32_t bytes, stride;
   __device__ __forceinline__ Stager(int row0, int nt, int nw, int64_t ld, int L) {
@@ -121,17 +121,21 @@ struct Stager {
     bytes = (uint32_t)(L - 1) * 2 * (uint32_t)ld + 2 * D;
     even = 2 * (uint32_t)ld * (row0 + row) + 16 * ((lane % T::CH) ^ T::mix(row));
     odd = 2 * (uint32_t)ld * (row0 + row) + 16 * ((lane % T::CH) ^ T::mix(PER + row));
+    first = (w & 1 ? odd : even) + w * stride;
   }
   // The whole distance goes into the vector offset: only that is held against the range, so that positions past the end are.
   // (one: of whole workgroups that move 1 KB a wave)
   __device__ __forceinline__ void stage(char* lds, const bf16* m, bool one) const {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)m, (short)0, bytes, 0x00020000);
     const uint32_t at[2] = {even, odd};
+    if (one) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(lds + w * 1024), 16, first, 0, 0, 0);
+      return;
+    }
     for (int i = w; i < count; i += step) {
       uint32_t voff = at[0];
       if (i & 1) voff = at[1];
       __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(lds + i * 1024), 16, voff + i * stride, 0, 0, 0);
-      if (one) break;
     }
   }
 };
@@ -1269,21 +1273,19 @@ __global__ __launch_bounds__(512, 2) void evo_dpair_rows_kernel(EvoParams p, int
     }
   }
   bool far = false;
-  for (int n = n0; n < n1; n += 8) {
-    float v[8];
+  const bool masked = sizeof(TB) == 2 && p.b1 != nullptr;
+  const int mk = min(kk0 + lane, L - 1);
+  for (int n = n0; n < n1; n += 16) {
+    float v[16];
+    bf16 m[16];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = (p.lse + (((int64_t)b * p.N + min(n + i, n1 - 1)) * p.H + h) * L)[(uint32_t)qc];
+    for (int i = 0; i < 16; ++i) {
+      const int64_t bn = (int64_t)b * p.N + min(n + i, n1 - 1);
+      v[i] = (p.lse + (bn * p.H + h) * L)[(uint32_t)qc];
+      m[i] = *(masked ? (const bf16*)p.b1 + bn * L + mk : p.q);  // (a branch would have every row wait for the one before)
+    }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) far |= far_off(v[i] * kLog2e);
-    if constexpr (sizeof(TB) == 2)
-      if (p.b1 != nullptr) {
-        bf16 m[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          m[i] = ((const bf16*)p.b1 + ((int64_t)b * p.N + min(n + i, n1 - 1)) * L)[(uint32_t)min(kk0 + lane, L - 1)];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) far |= is_large(m[i]);
-      }
+    for (int i = 0; i < 16; ++i) far = far | far_off(v[i] * kLog2e) | (masked & is_large(m[i]));
   }
   if constexpr (sizeof(TB) == 2) {
 #pragma unroll
