@@ -16,10 +16,10 @@
 //   * pair-bias gradient: the sum of dS over the N rows stays in registers. A wave owns 32 queries x 64 keys of one
 //     (b, h) and walks over a chunk of the rows, recomputing the two products that dS needs; chunks are added by a second
 //     kernel that also rounds. No atomics, the same result every time.
-// Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): a forward and backward 136 us (with a forward workgroup a
+// Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): a forward and backward 137 us (with a forward workgroup a
 // row and the pair bias through the matrix cores in every row 147; with dQ and dK / dV apart and the pair gradient's rows
-// loaded by wave 199); in a kernel trace, where launches do not overlap, forward 34 us (a workgroup a row 42), dQ + dK + dV 67
-// (apart 52 + 51), pair gradient 32 + 4 (bias through the matrix cores 43 + 4, rows by wave 56 + 4)
+// loaded by wave 199); in a kernel trace, where launches do not overlap, forward 38 us (a workgroup a row 42 to 45), dQ + dK +
+// dV 68 (apart 52 + 51), pair gradient 33 + 4 (bias through the matrix cores 43 + 4, rows by wave 56 + 4)
 // (before: one wave a workgroup with operands from global memory and 2-byte reads of V 169 us; the FlashAttention
 // backward kernels with 32-bit atomics into the pair gradient 271 + 1,585 us).
 #include <algorithm>
@@ -530,6 +530,9 @@ __global__ __launch_bounds__(64 * kWaves<D>) void evo_fwd_kernel(EvoParams p, in
 // where one of the maxima met is far off, where no key is visible or the sum is no number, and where a bias is large.
 // A kernel for each count of tiles: in one for several, the way of a last single tile lay between those of the pairs (34 KB of
 // code instead of 20, and 13 registers in scratch memory).
+// Its time, by counters at 128 x 256 positions, 8 heads: 73,500 cycles a wave, of which a SIMD's two waves issue vector
+// instructions (4,800 each, for the pair bias and four rows) for 60 % and products for 18 %; a wave waits for 38 %, for the
+// pair bias and the first row and at the four rows' barriers.
 template <int NT>
 struct RowRing {
   static constexpr int M = 32 * NT * 64, kMask = 256 * ((NT + 1) / 2);  // bytes of K or V, of the mask (4 a key)
@@ -1223,9 +1226,9 @@ __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblo
 // hds_evoformer_pair_staged says so: a workgroup of up to 4 x 2 waves stages the queries and the keys that its waves share, a
 // row ahead (three rows ahead is level). In the kernel above each wave loads its own, between them almost three times the bytes, in pieces of 16
 // bytes a row, and waits for them: 128 rows of 256, 8 heads, D = 32 58 -> 42 us; a training pass with D = 64 296 -> 251 us.
-// What bounds it is how many instructions a wave has, about five cycles each with two waves a SIMD: with the pair bias as what
-// the scores start from (of near rows, see far_off) instead of six products a tile, one operation for the exponent's argument
-// and the distances of a row's loads made once, 170 instead of 380 a row and 42 -> 32 us.
+// The pair bias is what the scores start from (of near rows, see far_off) instead of six products a tile, the exponent's argument
+// takes one operation, and the distances of a row's loads are made once: 42 -> 33 us. By counters, of 64,600 cycles a wave a SIMD's
+// two waves issue vector instructions for 45 % and products for 17 %; a wave waits for 36 %, at the start and for each row.
 template <int D>
 struct PairRows {
   static constexpr int M = 128 * Tile<D>::RB;    // bytes of a matrix: 128 rows

@@ -324,7 +324,8 @@ def _dgrad_sliced(T, N, K):
     104; [32000, 2048] 149 / 156 / 218 / 310 -> 108 / 120 / 162 / 210; [128256, 2048] 408 / 384 / 643 / 981 -> 357 / 386 / 502 /
     695. Up to 4,096 columns only between the few rows that read the weight once and those that fill the chip: [32000, 4096] at
     192 / 256 / 509 / 700 / 900 rows 204 / 243 / 322 / 330 / 346 -> 209 / 217 / 269 / 317 / 359, [28672, 4096] 188 / 229 / 303 /
-    306 / 333 -> 183 / 191 / 246 / 290 / 314. With a shorter or a longer reduction the transpose costs as much as the slices
+    306 / 333 -> 183 / 191 / 246 / 290 / 314, and so between: at 256 / 509 / 640 rows [16384, 2560] 93 / 123 / 134 -> 69 / 90 / 107,
+    [22016, 3072] 165 / 232 / 231 -> 114 / 146 / 167, [28672, 3584] 199 / 272 / 241 -> 151 / 199 / 223. With a shorter or a longer reduction the transpose costs as much as the slices
     give: 509 rows of [11264, 2048] 66 -> 70, [8192, 4096] 77 -> 82, [128256, 4096] 885 -> 919."""
     if K <= 2048:
         return 40 <= T <= 1100 and N >= 12 * K and bool(_plan(T, K, N))
