@@ -19,7 +19,7 @@
 // Measured (B = 1, N = 128, L = 256, H = 8, D = 32, both biases bf16): a forward and backward 137 us (with a forward workgroup a
 // row and the pair bias through the matrix cores in every row 147; with dQ and dK / dV apart and the pair gradient's rows
 // loaded by wave 199); in a kernel trace, where launches do not overlap, forward 38 us (a workgroup a row 42 to 45), dQ + dK +
-// dV 68 (apart 52 + 51), pair gradient 33 + 4 (bias through the matrix cores 43 + 4, rows by wave 56 + 4)
+// dV 68 (apart 52 + 51), pair gradient 34 + 4 (bias through the matrix cores 43 + 4, rows by wave 56 + 4)
 // (before: one wave a workgroup with operands from global memory and 2-byte reads of V 169 us; the FlashAttention
 // backward kernels with 32-bit atomics into the pair gradient 271 + 1,585 us).
 #include <algorithm>
@@ -1227,7 +1227,7 @@ __global__ __launch_bounds__(256, 2) void evo_dpair_kernel(EvoParams p, int qblo
 // row ahead (three rows ahead is level). In the kernel above each wave loads its own, between them almost three times the bytes, in pieces of 16
 // bytes a row, and waits for them: 128 rows of 256, 8 heads, D = 32 58 -> 42 us; a training pass with D = 64 296 -> 251 us.
 // The pair bias is what the scores start from (of near rows, see far_off) instead of six products a tile, the exponent's argument
-// takes one operation, and the distances of a row's loads are made once: 42 -> 33 us. By counters, of 64,600 cycles a wave a SIMD's
+// takes one operation, and the distances of a row's loads are made once: 42 -> 34 us. By counters, of 64,600 cycles a wave a SIMD's
 // two waves issue vector instructions for 45 % and products for 17 %; a wave waits for 36 %, at the start and for each row.
 template <int D>
 struct PairRows {

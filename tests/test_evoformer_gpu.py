@@ -490,3 +490,23 @@ def test_evoformer_walks_in_many_batches(cuda, B, N, L, H):
             one = DS4Sci_EvoformerAttention(*(t[b:b + 1] for t in (q, k, v)), [b1[b:b + 1], b2[b:b + 1]])
             x, y = out[b].double(), one[0].double()
             assert (x - y).norm() <= 0.1 * 2**-8 * y.norm()  # (as rows by themselves above)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", ["none", "mask", "pair"])
+@pytest.mark.parametrize("N,L,H", [(66, 200, 8), (190, 97, 8), (520, 17, 8)])
+def test_evoformer_walks_with_fewer_biases(cuda, N, L, H, which):
+    """Walking workgroups without the mask, the pair bias or both, with the bound of the edge tests."""
+    if which != "none":
+        test_evoformer_edges_hip(cuda, 1, N, L, H, 32, which, torch.bfloat16)
+        return
+    g = torch.Generator(device="cuda").manual_seed(L)
+    q, k, v, do = (torch.randn(1, N, L, H, 32, device="cuda", generator=g).bfloat16() for _ in range(4))
+    leaves = [t.requires_grad_() for t in (q, k, v)]
+    out = DS4Sci_EvoformerAttention(*leaves, [])
+    got = [out] + list(torch.autograd.grad(out, leaves, do))
+    exact = [t.detach().double().requires_grad_() for t in leaves]
+    qh, kh, vh = (t.transpose(-2, -3) for t in exact)
+    ref = (torch.softmax(qh @ kh.transpose(-1, -2) / math.sqrt(32), -1) @ vh).transpose(-2, -3)
+    for x, y in zip(got, [ref] + list(torch.autograd.grad(ref, exact, do.double()))):
+        assert (x.double() - y).norm() <= 4 * 2**-8 * y.norm()
